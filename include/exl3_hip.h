@@ -429,7 +429,7 @@ int exl3_unpack_trellis(const uint16_t *trellis, long long n_tiles, int K, uint1
  *   q_tiles   fp32 [n_tiles][256]   decoded value of the chosen codeword
  *   indices   u16  [n_tiles][256]   full 16-bit codewords; indices & (2^K - 1) are
  *                                   the symbols exl3_pack_trellis takes
- *   workspace backpointer slots, exl3_quantize_slot_bytes(K) each. At least one
+ *   workspace path-cost slots, exl3_quantize_slot_bytes(K) each. At least one
  *             slot is required (EXL3_E_WORKSPACE); exl3_quantize_workspace_bytes()
  *             is what keeps every CU busy; more than that is not used. A tile
  *             batch larger than the slot count is walked by the same launch.

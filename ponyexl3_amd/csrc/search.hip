@@ -10,14 +10,14 @@
 // runs once around the tile and backtracks to the state in front of position 0;
 // pass 1 starts at position 0 pinned to that state and has to end in it.
 //
-// One workgroup of 256 lanes owns a tile; both cost rows live in LDS
-// (2 * 2^(16-K) halfs: 64 KiB at K=2, 512 B at K=8), the backpointers (256 steps x
-// 2^(16-K) uint16) in the caller's workspace, one slot per resident workgroup; a
-// workgroup walks over tiles blockIdx.x, blockIdx.x + gridDim.x, .. reusing its
-// slot. Every step evaluates all 65536 codewords, five VALU instructions each, so
-// a tile costs about 2 * 256 * 65536 * 5 lane-operations whatever K is; the serial
-// backtrack (256 dependent loads by one lane) overlaps with the other workgroup
-// of the CU.
+// One workgroup of 1024 lanes per CU evaluates all 65536 codewords of a step, 64 per
+// lane, and keeps only the minimum per state: which fresh value won matters for the 256
+// states on the final path alone, so the backtrack works it out again for those from the
+// cost rows of the pass (kept in the caller's workspace, 256 x 2^(16-K) halfs per tile)
+// instead of every state paying for a select per candidate. A candidate then costs a
+// subtraction, an fma and half of a three-operand minimum. The backtrack of one tile is a
+// chain of 256 dependent loads; a workgroup keeps two tiles in flight and one of its waves
+// walks the chain of one tile while all of them run the forward steps of the other.
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 
@@ -57,252 +57,341 @@ __device__ __forceinline__ void take_if_less(float err, float& best, uint32_t& b
         : "vcc");
 }
 
-// Lane <-> state assignment. With L = tid & (2^K - 1) and hi = tid >> K a lane owns
-// the PER_LANE = 2^(8-K) compressed states e(j) = L | ((hi*PER_LANE + j) << K).
-// Their predecessors for one fresh value f, (f << (16-2K)) | (hi*PER_LANE + j), are
-// consecutive in j, so a lane fetches the previous costs of up to eight of its
-// states with one LDS read. The 256 codewords (f, j) a lane ever evaluates do
-// not depend on the step: their decoded fp16 values stay in 128 registers for the
-// whole launch, and a candidate costs five VALU instructions: two mixed-precision
-// fmas (value - target; dh*dh + previous cost, both reading their fp16 operand
-// directly), one compare and two selects.
-template <int K, int CB>
-__global__ __launch_bounds__(256, 2) void quantize_tiles_kernel(const float* __restrict__ tiles,
-                                                             float* __restrict__ q_tiles,
-                                                             uint16_t* __restrict__ indices,
-                                                             uint16_t* back_ws, int n_tiles,
-                                                             float one) {
-    constexpr int KR = 16 - K, EDGES = 1 << KR, KK = 1 << K;
-    constexpr int PER_LANE = EDGES / 256;             // states per lane
-    constexpr int CH = PER_LANE < 8 ? PER_LANE : 8;   // states per LDS read
-    // A cost row is stored in blocks of 256 states with PAD halfs between blocks:
-    // the lanes of a wave write the states of 64 / 2^K different blocks at the same
-    // offset, and unpadded those would all fall into the same LDS banks.
-    constexpr int PAD = KK > 8 ? KK : 8;
-    constexpr int ROW = EDGES + (EDGES / 256) * PAD;
-    auto row_index = [](uint32_t e) { return e + (e >> 8) * PAD; };
-    // Backpointers of one step are stored as [j][lane] (lane = owner of the state,
-    // j = its index among the lane's states): wave-wide contiguous stores.
-    auto back_index = [](uint32_t e) {
-        const uint32_t pj = e >> K;
-        const uint32_t owner = ((pj / PER_LANE) << K) | (e & (KK - 1));
-        return (pj % PER_LANE) * 256 + owner;
-    };
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-    half_t* costs = reinterpret_cast<half_t*>(lds_raw);  // [2][EDGES]
-    __shared__ float target_s[256];
-    __shared__ uint32_t red_key[4];
-    __shared__ uint32_t sh_pin;
-    const int tid = threadIdx.x;
-    const uint32_t low = (uint32_t)tid & (KK - 1);
-    const uint32_t base = ((uint32_t)tid >> K) * PER_LANE;  // e(j) >> K = base + j
-    uint16_t* back = back_ws + (size_t)blockIdx.x * 256 * EDGES;
-    // lane parts of the cost-row addresses (see unit_addr and the store below)
-    const uint32_t lane_rd0 = KR - K >= 8 ? base + (base >> 8) * PAD : base;
-    const uint32_t lane_wr0 = row_index((base << K) | low);
-
-    // decoded values of the lane's codewords, index c = f*PER_LANE + j, two per register
-    half2_t lut[128];
-#pragma unroll
-    for (int c = 0; c < 256; c += 4) {
-        uint32_t cw[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t f = (uint32_t)(c + i) / PER_LANE, j = (uint32_t)(c + i) % PER_LANE;
-            cw[i] = (f << KR) | ((base + j) << K) | low;
-        }
-        decode_pair2<CB>(cw[0], cw[1], cw[2], cw[3], lut[c / 2], lut[c / 2 + 1]);
+// Where things sit for one K. A compressed state e (16-K bits) splits in two ways:
+//   as the target of a step   e = p << K | l      (p: 16-2K bits, l: K bits)
+//   as its source             e = f << P | p      (f: the K bits above, P = 16-2K)
+// The 2^K candidates of a target (p, l) are the sources (f, p), f = 0 .. 2^K - 1, and all
+// 2^K targets of one p share them. A cost row is therefore stored as [p][f]: the costs a
+// lane needs for one p are one consecutive run of LDS words.
+// A lane owns 2^G source groups p (the ones that differ in the low bits of the top K bits
+// of their targets, so that the 2^G costs it produces for one l are neighbours in the next
+// row: one store) times 2^S targets l of each; from K = 6 on one target, whose candidates
+// are shared among FS lanes at K = 7 and 8.
+template <int K>
+struct SearchMap {
+    static constexpr int KR = 16 - K, P = 16 - 2 * K, KK = 1 << K, EDGES = 1 << KR;
+    static constexpr int G = K == 2 || K == 3 ? 2 : K == 4 ? 1 : 0;
+    static constexpr int S = K <= 6 ? 6 - K - G : 0;
+    static constexpr int FS = K <= 6 ? 1 : 1 << (K - 6);
+    static constexpr int NG = 1 << G, NS = 1 << S, NF = KK / FS;  // NG * NS * NF = 64
+    static constexpr int ROW_BYTES = 2 * EDGES;
+    // Byte offset of source (f, p) in a cost row. Rows of one p are 2^(K+1) bytes; the
+    // 16-byte units (8-byte at K = 2) are permuted by exclusive-or so that the lanes of a
+    // wave hit different LDS banks in both directions: consecutive p when they read, p
+    // that differ in bits K and up when they write.
+    static __device__ __forceinline__ uint32_t at(uint32_t p, uint32_t f) {
+        if constexpr (K == 2) return ((p ^ ((p >> 4) & 3)) << 3) + 2 * f;
+        else if constexpr (K == 3) return ((p ^ ((p >> 3) & 7)) << 4) + 2 * f;
+        else if constexpr (K == 4) return (((2 * p + (f >> 3)) ^ ((p >> 4) & 7)) << 4) + 2 * (f & 7);
+        else if constexpr (K == 5) return (((4 * p + (f >> 3)) ^ ((p >> 1) & 3)) << 4) + 2 * (f & 7);
+        else if constexpr (K == 6) return (((8 * p + (f >> 3)) ^ (p & 7)) << 4) + 2 * (f & 7);
+        else return (p << (K + 1)) + 2 * f;
     }
+    // p of group g, l of target s and first fresh value of lane `tid`
+    static __device__ __forceinline__ uint32_t lane_p(uint32_t tid, int g) {
+        if constexpr (K <= 5) {
+            constexpr int PL = P - K;  // bits of p below the top K
+            const uint32_t plow = tid & ((1u << PL) - 1), phigh = (tid >> PL) & ((1u << (K - G)) - 1);
+            return (((phigh << G) | (uint32_t)g) << PL) | plow;
+        } else {
+            return (tid / FS) >> K;
+        }
+    }
+    static __device__ __forceinline__ uint32_t lane_l(uint32_t tid, int s) {
+        if constexpr (K <= 5) return ((tid >> (P - G)) << S) | (uint32_t)s;
+        else return (tid / FS) & (KK - 1);
+    }
+    static __device__ __forceinline__ uint32_t lane_f(uint32_t tid) { return (tid & (FS - 1)) * NF; }
+};
 
-    for (int tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        __syncthreads();  // the previous tile's backtrack has finished with target_s / back
-        target_s[tid] = tiles[(size_t)tile * 256 + tid];
-        uint32_t pin = 0;
-        for (int pass = 0; pass < 2; pass++) {
-            const int roll = pass == 0 ? 128 : 0;
+constexpr int kSearchThreads = 1024;
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t min_dpp(uint32_t v) {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+    return o < v ? o : v;
+}
+
+// Minimum over the wave of values that repeat every 2^K lanes.
+template <int K>
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+    v = min_dpp<0xB1>(v);                               // lanes 1 apart
+    v = min_dpp<0x4E>(v);                               // 2 apart
+    if constexpr (K > 2) v = min_dpp<0x141>(v);         // half-row mirror: 4 apart
+    if constexpr (K > 3) v = min_dpp<0x140>(v);         // row mirror: 8 apart
+    if constexpr (K > 4) {
+        float a = __builtin_bit_cast(float, v), b = a;  // 16 apart
+        swap_rows16(a, b);
+        const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        v = x < y ? x : y;
+    }
+    if constexpr (K > 5) {
+        float a = __builtin_bit_cast(float, v), b = a;  // 32 apart
+        swap_halves32(a, b);
+        const uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        v = x < y ? x : y;
+    }
+    return v;
+}
+
+// One step of the backtrack: the predecessor of state `edge` given the costs before the
+// step (cost[j] = that of fresh value lane + 64 j, repeating if there are fewer than 64).
+// The first fresh value that attains the minimum wins; 0 if no candidate stays under the
+// bound, as in the reference. Errors are non-negative, so their bits order like they do.
+template <int K, int CB>
+__device__ __forceinline__ uint32_t search_predecessor(const half_t (&cost)[K > 6 ? 1 << (K - 6) : 1],
+                                                       uint32_t edge, float target, int lane) {
+    using M = SearchMap<K>;
+    constexpr int NB = K > 6 ? 1 << (K - 6) : 1;
+    uint32_t err[NB], best = __builtin_bit_cast(uint32_t, kCostInf);
+    const uint32_t bound = best;
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        const uint32_t f = (uint32_t)(lane + 64 * j) & (M::KK - 1);
+        const float dh = decode1_f32<CB>((f << M::KR) | edge) - target;
+        err[j] = __builtin_bit_cast(uint32_t, __builtin_fmaf(dh, dh, (float)cost[j]));
+        best = err[j] < best ? err[j] : best;
+    }
+    best = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_min<K>(best));
+    uint32_t f = 0;
+#pragma unroll
+    for (int j = NB - 1; j >= 0; j--) {
+        const unsigned long long hit = __ballot(err[j] == best);
+        if (hit) f = (uint32_t)(64 * j + __builtin_ctzll(hit));
+    }
+    return best < bound ? (f << M::P) | (edge >> K) : 0u;
+}
+
+// Workgroup b walks over tiles b, b + gridDim.x, .. in phases of 256 steps. With two
+// cost-history slots (b + gridDim.x < n_slots) phase n runs the forward steps of slot n & 1
+// (warm-up pass, two phases later the pinned pass) and the backtrack of what slot ~n & 1 did
+// in phase n - 1; with one slot the odd phases only backtrack. (A tile
+// alone on its CU takes 0.80 ms, of which the forward steps are 0.70.)
+//
+// The kernel is bound by VALU issue: 64 candidates per lane and step are 64 subtractions,
+// 64 mixed-precision fmas (the previous cost is read as fp16) and 32 v_min3; the lane's 64
+// decoded values stay in registers as fp32 for the whole launch. 16 waves of at most 128
+// registers fill the CU, so the whole of a step hides its own LDS latency; one barrier per
+// step. Rows are copied to the history in 16-byte stores from the finished LDS row of the
+// step before, by the upper eight waves: the wave that backtracks (0) has no stores in
+// flight that its loads would have to wait for.
+// Measured on 4096 tiles: 1.36 us per step (about 2600 of its 2900 cycles are issue slots),
+// 303 k (K = 2), 361 k (3), 364-368 k (4..6), 345 k tiles/s (7, 8) and 0.8 ms for up to 256
+// tiles at once. With a compare and two selects per candidate for the backpointer, 256 lanes
+// per tile and the backtrack at the end of each pass it was 141 k, 172 k, 189-225 k, 195-217 k
+// and 1.6-2.5 ms.
+template <int K, int CB>
+__global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
+    const float* __restrict__ tiles, float* __restrict__ q_tiles, uint16_t* __restrict__ indices,
+    unsigned char* history, int n_tiles, int n_slots) {
+    using M = SearchMap<K>;
+    constexpr int EDGES = M::EDGES, KK = M::KK, NG = M::NG, NS = M::NS, NF = M::NF, FS = M::FS;
+    constexpr int NB = K > 6 ? 1 << (K - 6) : 1;
+    constexpr size_t kSlotBytes = (size_t)256 * M::ROW_BYTES;
+    extern __shared__ __attribute__((aligned(16))) unsigned char rows_s[];  // [2][ROW_BYTES]
+    __shared__ float target_s[2][256];
+    __shared__ uint16_t state_s[256];
+    __shared__ uint32_t red_key[16];
+    __shared__ uint32_t pin_s[2];
+    uint32_t tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(tid >> 6));
+
+    const bool two = (int)(blockIdx.x + gridDim.x) < n_slots;
+    auto phase_tile = [&](int n) -> long long {  // tile of forward phase n, -1 if it has none
+        if (n < 0 || (!two && (n & 1))) return -1;
+        const int j = two ? 2 * (n >> 2) + (n & 1) : n >> 2;
+        const long long t = blockIdx.x + (long long)gridDim.x * j;
+        return t < n_tiles ? t : -1;
+    };
+    uint32_t back_edge = 0;  // state the pending backtrack starts from
+    for (int n = 0;; n++) {
+        const long long tile = phase_tile(n), back_tile = phase_tile(n - 1);
+        if (tile < 0 && back_tile < 0 && phase_tile(n + 1) < 0 && phase_tile(n + 2) < 0 &&
+            phase_tile(n + 3) < 0)
+            break;
+        // the lane's addresses are derived anew in every phase: held across the phases
+        // they would take registers that the step loop needs
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63;
+        const int slot = n & 1, pass = (n >> 1) & 1, back_pass = ((n - 1) >> 1) & 1;
+        unsigned char* hist = history + kSlotBytes * (blockIdx.x + (size_t)slot * gridDim.x);
+        const unsigned char* back_hist = history + kSlotBytes * (blockIdx.x + (size_t)(slot ^ 1) * gridDim.x);
+        // the warm-up pass starts at position 128 and is walked back to position 0 only
+        const int roll = pass == 0 ? 128 : 0, back_roll = back_pass == 0 ? 128 : 0;
+        const int back_end = back_pass == 0 ? 128 : 0;
+        const bool backs = back_tile >= 0 && wave == 0;
+        const uint32_t back_pin = back_pass == 1 ? pin_s[slot ^ 1] : 0;
+        uint32_t edge = __builtin_amdgcn_readfirstlane((int)back_edge);
+
+        // one step of the pending backtrack in two halves: request the costs in front of
+        // it, later pick the predecessor
+        half_t cost[NB];
+        auto back_request = [&](int step) {
+            const uint32_t p = edge >> K;
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const uint32_t f = (uint32_t)(lane + 64 * j) & (KK - 1);
+                if (step > 0) {
+                    cost[j] = *reinterpret_cast<const half_t*>(
+                        back_hist + (size_t)(step - 1) * M::ROW_BYTES + M::at(p, f));
+                } else {  // in front of the pinned pass: nothing but the pin
+                    cost[j] = ((f << M::P) | p) == back_pin ? (half_t)0.0f : bits_to_half(0x7C00);
+                }
+            }
+        };
+        auto back_take = [&](int step) {
+            const int ri = (step + back_roll) & 255;
+            const uint32_t prev = search_predecessor<K, CB>(cost, edge, target_s[slot ^ 1][ri], lane);
+            if (lane == 0) state_s[ri] = (uint16_t)((prev << K) | edge);
+            edge = prev;
+        };
+
+        if (tile < 0) {
+            if (backs)
+                for (int step = 255; step >= back_end; step--) {
+                    back_request(step);
+                    back_take(step);
+                }
+        } else {
+            const uint32_t pin = pin_s[slot];  // (pass 0: not used)
+            if (pass == 0 && tid < 256) target_s[slot][tid] = tiles[(size_t)tile * 256 + tid];
             // Step 0 has no predecessor costs: a row of zeros stands in for them
             // (fma(dh, dh, 0) is the rounded square), and in the pinned pass +inf
             // everywhere but at the pin keeps every other predecessor from winning.
-            {
+#pragma unroll 1
+            for (uint32_t e = tid; e < (uint32_t)EDGES; e += kSearchThreads) {
                 const half_t open = pass == 0 ? (half_t)0.0f : bits_to_half(0x7C00);
-                for (int i = 0; i < PER_LANE; i++) {
-                    const uint32_t e = (uint32_t)(tid + 256 * i);
-                    costs[ROW + row_index(e)] = (pass == 1 && e == pin) ? (half_t)0.0f : open;
-                }
+                *reinterpret_cast<half_t*>(rows_s + M::ROW_BYTES + M::at(e & ((1u << M::P) - 1), e >> M::P)) =
+                    pass == 1 && e == pin ? (half_t)0.0f : open;
             }
+            // decoded values of the lane's codewords (f, p, l), f << KR | p << K | l, for the
+            // steps of this phase (kept across phases they would be live next to the
+            // backtrack's own code and spill)
+            float val[NG][NS][NF];
+#pragma unroll
+            for (int g = 0; g < NG; g++)
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    const uint32_t e = (M::lane_p(tid, g) << K) | M::lane_l(tid, s);
+#pragma unroll
+                    for (int f = 0; f < NF; f += 4) {
+                        const uint32_t c = ((M::lane_f(tid) + f) << M::KR) | e;
+                        float v[4];
+                        decode4_f32<CB>(c, c + EDGES, c + 2 * EDGES, c + 3 * EDGES, v);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            asm volatile("" : "+v"(v[i]));  // decoded here, not again in every step
+                            val[g][s][f + i] = v[i];
+                        }
+                    }
+                }
             __syncthreads();
 #pragma unroll 1
             for (int step = 0; step < 256; step++) {
-                const int ri = (step + roll) & 255;
-                const half_t* cprev = costs + ((step & 1) ^ 1) * ROW;
-                half_t* ccurr = costs + (step & 1) * ROW;
-                const float negt = -target_s[ri];
-                // The table is the same in every step; without this the compiler hoists
-                // its 256 fp16 -> fp32 conversions out of the loop and runs out of registers.
+                const unsigned char* prev_row = rows_s + ((step & 1) ^ 1) * M::ROW_BYTES;
+                unsigned char* row = rows_s + (step & 1) * M::ROW_BYTES;
+                const float target = target_s[slot][(step + roll) & 255];
+                const int back_step = 255 - step;
+                const bool back_now = backs && back_step >= back_end;
+                if (back_now) back_request(back_step);
+                // the row before this one goes to the history (what the backtrack of the
+                // warm-up pass never reads is left out)
+                if (step > (pass == 0 ? 127 : 0)) {
+                    unsigned char* dst = hist + (size_t)(step - 1) * M::ROW_BYTES;
+                    if (tid >= kSearchThreads / 2)
+                        for (uint32_t o = (tid - kSearchThreads / 2) * 16; o < (uint32_t)M::ROW_BYTES;
+                             o += 8 * kSearchThreads)
+                            *reinterpret_cast<uint4_t*>(dst + o) = *reinterpret_cast<const uint4_t*>(prev_row + o);
+                }
+                half_t out[NG][NS];
 #pragma unroll
-                for (int i = 0; i < 128; i++) asm volatile("" : "+v"(lut[i]));
-
-                // Read units: UNIT previous costs from consecutive LDS addresses. For
-                // K <= 7 a unit is one fresh value f and CH consecutive states of the
-                // lane; at K = 8 a lane has one state whose predecessors are the fresh
-                // values themselves, eight to a unit. One unit is fetched ahead.
-                constexpr bool ALONG_F = PER_LANE == 1;
-                constexpr int UNIT = ALONG_F ? 8 : CH;
-                constexpr int N_UNITS = 256 / UNIT;
-                // Address = lane part (computed once) + a compile-time part that fits the
-                // immediate offset of the LDS instruction. The split is exact: the fresh
-                // value contributes whole 256-state blocks (K <= 4) or decides the block
-                // on its own (K > 4), and a lane's states never cross a block.
-                auto unit_addr = [&](int u) -> const half_t* {
-                    if constexpr (ALONG_F) {
-                        return cprev + u * 8;  // base = 0: predecessor = fresh
-                    } else {
-                        const int ch = u / KK, f = u % KK;
-                        const int fpart = f << (KR - K);
-                        const int blocks = KR - K >= 8 ? fpart >> 8 : f >> (8 - (KR - K));
-                        return cprev + lane_rd0 + (fpart + ch * CH + blocks * PAD);
-                    }
-                };
-                auto fetch = [&](int u) {
-                    uint4_t v = {0u, 0u, 0u, 0u};
-                    const half_t* src = unit_addr(u);
-                    if constexpr (UNIT == 8) {
-                        v = *reinterpret_cast<const uint4_t*>(src);
-                    } else if constexpr (UNIT == 4) {
-                        const uint2_t t = *reinterpret_cast<const uint2_t*>(src);
-                        v.x = t.x;
-                        v.y = t.y;
-                    } else {
-                        v.x = *reinterpret_cast<const uint32_t*>(src);
-                    }
-                    return v;
-                };
-                // Fresh values are walked in blocks of 64 so that the index a select
-                // writes is an inline constant; blocks after the first are merged into
-                // the running minimum with a strict <, which keeps the first minimum.
-                constexpr int NB = ALONG_F ? 1 : CH;  // running minima held at a time
-                constexpr uint32_t kNone = 64;        // block-local "nothing beat the bound"
-                constexpr uint32_t kNoneAll = KK > 64 ? KK : 64;  // the same for the whole walk
-                float best[NB], blk_best[NB];
-                uint32_t best_f[NB], blk_f[NB];
-                uint4_t cur = fetch(0);
-                static_for<0, N_UNITS>([&](auto uc) {
-                    constexpr int u = uc.value;
-                    const uint4_t nxt = fetch(u + 1 < N_UNITS ? u + 1 : u);
-                    constexpr int ch = ALONG_F ? 0 : u / KK;
-                    constexpr int f0 = ALONG_F ? u * 8 : u % KK;
-                    if constexpr ((f0 & 63) == 0) {
+                for (int g = 0; g < NG; g++) {
+                    const uint32_t p = M::lane_p(tid, g), f0 = M::lane_f(tid);
+                    float best[NS];
 #pragma unroll
-                        for (int b = 0; b < NB; b++) {
-                            if (f0 == 0) {
-                                best[b] = kCostInf;
-                                best_f[b] = kNoneAll;
+                    for (int s = 0; s < NS; s++) best[s] = kCostInf;
+#pragma unroll
+                    for (int fc = 0; fc < NF; fc += 8) {
+                        constexpr int CH = NF < 8 ? NF : 8;
+                        uint32_t w[4];
+                        if constexpr (CH == 8) {
+                            const uint4_t q = *reinterpret_cast<const uint4_t*>(prev_row + M::at(p, f0 + fc));
+                            w[0] = q.x, w[1] = q.y, w[2] = q.z, w[3] = q.w;
+                        } else {
+                            const uint2_t q = *reinterpret_cast<const uint2_t*>(prev_row + M::at(p, f0 + fc));
+                            w[0] = q.x, w[1] = q.y, w[2] = w[3] = 0;
+                        }
+#pragma unroll
+                        for (int s = 0; s < NS; s++)
+#pragma unroll
+                            for (int i = 0; i < CH; i += 2) {
+                                const half2_t pc = bits_to_half2(w[i >> 1]);
+                                const float d0 = val[g][s][fc + i] - target, d1 = val[g][s][fc + i + 1] - target;
+                                const float e0 = __builtin_fmaf(d0, d0, (float)pc.x);
+                                const float e1 = __builtin_fmaf(d1, d1, (float)pc.y);
+                                // an error at or above the bound never wins, which is all the
+                                // reference's clamp to 65504 achieves
+                                best[s] = __builtin_fminf(__builtin_fminf(best[s], e0), e1);
                             }
-                            blk_best[b] = kCostInf;
-                            blk_f[b] = kNone;
-                        }
                     }
-                    const uint32_t words[4] = {cur.x, cur.y, cur.z, cur.w};
-                    static_for<0, UNIT>([&](auto ic) {
-                        constexpr int i = ic.value;
-                        constexpr int f = ALONG_F ? f0 + i : f0;
-                        constexpr int b = ALONG_F ? 0 : i;
-                        constexpr int c = ALONG_F ? f : f * PER_LANE + ch * CH + i;
-                        const half_t val = (c & 1) ? lut[c >> 1].y : lut[c >> 1].x;
-                        const half2_t pp = bits_to_half2(words[i >> 1]);
-                        const half_t pc = (i & 1) ? pp.y : pp.x;
-                        // `one` is 1.0f passed as a kernel argument, so both fmas keep an
-                        // fp16 operand and are converted inside the instruction
-                        const float dh = __builtin_fmaf((float)val, one, negt);
-                        const float err = __builtin_fmaf(dh, dh, (float)pc);
-                        // an error at or above the bound never wins, which is all the
-                        // reference's clamp to 65504 achieves
-                        if constexpr (KK <= 64)
-                            take_if_less<f>(err, best[b], best_f[b]);
-                        else
-                            take_if_less<(f & 63)>(err, blk_best[b], blk_f[b]);
-                    });
-                    constexpr int f_last = ALONG_F ? f0 + 7 : f0;
-                    if constexpr (KK > 64 && (f_last & 63) == 63) {
 #pragma unroll
-                        for (int b = 0; b < NB; b++) {
-                            if (blk_best[b] < best[b]) {
-                                best[b] = blk_best[b];
-                                best_f[b] = blk_f[b] + (uint32_t)(f_last & ~63);
-                            }
-                        }
+                    for (int s = 0; s < NS; s++) {
+                        if constexpr (FS >= 2) best[s] = __builtin_fminf(best[s], dpp_move<0xB1>(best[s]));
+                        if constexpr (FS >= 4) best[s] = __builtin_fminf(best[s], dpp_move<0x4E>(best[s]));
+                        out[g][s] = (half_t)best[s];
                     }
-                    if constexpr (f_last == KK - 1) {
-                        // one scalar base per chunk; the stores below differ only in their
-                        // immediate offsets and share the lane offset (otherwise the compiler
-                        // keeps a separate offset register per store, 64 of them at K = 2)
-                        size_t row_off = (size_t)ri * EDGES + (ch * CH) * 256;
-                        asm volatile("" : "+s"(row_off));
-                        uint16_t* rowbase = back + row_off;
+                }
 #pragma unroll
-                        for (int b = 0; b < NB; b++) {
-                            const uint32_t pj = base + ch * CH + b;
-                            // state (pj << K) | low: all states of a lane lie in one block
-                            ccurr[lane_wr0 + ((ch * CH + b) << K)] = (half_t)best[b];
-                            // The reference leaves the backpointer at 0 when nothing beat the
-                            // bound. It skips the store for positions 128..255 of the warm-up
-                            // pass, which nobody reads; storing them anyway (the pinned pass
-                            // rewrites every row before it is walked) keeps the loop free of
-                            // branches.
-                            const uint32_t bp =
-                                best_f[b] == kNoneAll ? 0u : (best_f[b] << (KR - K)) | pj;
-                            rowbase[b * 256 + tid] = (uint16_t)bp;
-                        }
+                for (int s = 0; s < NS; s++) {
+                    const uint32_t e = (M::lane_p(tid, 0) << K) | M::lane_l(tid, s);
+                    unsigned char* dst = row + M::at(e & ((1u << M::P) - 1), e >> M::P);
+                    if constexpr (NG == 4) {
+                        const half4_t o = {out[0][s], out[1][s], out[2][s], out[3][s]};
+                        *reinterpret_cast<half4_t*>(dst) = o;
+                    } else if constexpr (NG == 2) {
+                        const half2_t o = {out[0][s], out[1][s]};
+                        *reinterpret_cast<half2_t*>(dst) = o;
+                    } else {
+                        if (FS == 1 || (tid & (FS - 1)) == 0) *reinterpret_cast<half_t*>(dst) = out[0][s];
                     }
-                    cur = nxt;
-                    __builtin_amdgcn_sched_barrier(0);
-                });
+                }
+                if (back_now) back_take(back_step);
                 __syncthreads();
             }
-
-            // first minimum of the final costs (pass 0): key = cost bits : state
-            if (pass == 0) {
-                uint32_t key = 0xFFFFFFFFu;
-                const half_t* cfin = costs + ROW;  // step 255 wrote row 1
-                for (int i = 0; i < PER_LANE; i++) {
-                    const uint32_t e = (uint32_t)(tid + 256 * i);
-                    const uint32_t kbits = (uint32_t)half_to_bits(cfin[row_index(e)]);
-                    const uint32_t cand = (kbits << 16) | e;
-                    key = cand < key ? cand : key;
-                }
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) {
-                    const uint32_t o = (uint32_t)__shfl_xor((int)key, off, kWave);
-                    key = o < key ? o : key;
-                }
-                if ((tid & 63) == 0) red_key[tid >> 6] = key;
-            }
-            __syncthreads();
-            if (tid == 0) {
-                uint32_t edge = pin;
-                if (pass == 0) {
-                    uint32_t key = red_key[0];
-                    for (int w = 1; w < 4; w++) key = red_key[w] < key ? red_key[w] : key;
-                    // a cost that never dropped below the bound selects state 0
-                    edge = (key >> 16) >= 0x7BFFu ? 0u : (key & 0xFFFFu);
-                }
-                for (int step_i = 255; step_i >= 0; step_i--) {
-                    const int ri = (step_i + roll) & 255;
-                    const uint32_t prev = back[(size_t)ri * EDGES + back_index(edge)];
-                    const uint32_t state = ((prev << K) | edge) & 0xFFFFu;
-                    edge = prev;
-                    if (pass == 1) {
-                        indices[(size_t)tile * 256 + ri] = (uint16_t)state;
-                        q_tiles[(size_t)tile * 256 + ri] = decode1_f32<CB>(state);
-                    } else if (ri == 0) {
-                        break;
-                    }
-                }
-                sh_pin = edge;
-            }
-            __syncthreads();
-            pin = sh_pin;
         }
+        if (backs && lane == 0 && back_pass == 0) pin_s[slot ^ 1] = edge;  // state in front of position 0
+        if (tile >= 0 && pass == 0) {
+            // first minimum of the final costs: key = cost bits : state (step 255 wrote row 1)
+            uint32_t key = 0xFFFFFFFFu;
+#pragma unroll 1
+            for (uint32_t e = tid; e < (uint32_t)EDGES; e += kSearchThreads) {
+                const uint32_t bits = *reinterpret_cast<const uint16_t*>(
+                    rows_s + M::ROW_BYTES + M::at(e & ((1u << M::P) - 1), e >> M::P));
+                const uint32_t cand = (bits << 16) | e;
+                key = cand < key ? cand : key;
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                const uint32_t o = (uint32_t)__shfl_xor((int)key, off, kWave);
+                key = o < key ? o : key;
+            }
+            if (lane == 0) red_key[wave] = key;
+        }
+        __syncthreads();
+        if (back_tile >= 0 && back_pass == 1 && tid < 256) {
+            const uint32_t state = state_s[tid];
+            indices[(size_t)back_tile * 256 + tid] = (uint16_t)state;
+            q_tiles[(size_t)back_tile * 256 + tid] = decode1_f32<CB>(state);
+        }
+        if (tile >= 0 && pass == 0) {
+            uint32_t key = red_key[0];
+            for (int w = 1; w < 16; w++) key = red_key[w] < key ? red_key[w] : key;
+            // a cost that never dropped below the bound selects state 0
+            back_edge = (key >> 16) >= 0x7BFFu ? 0u : (key & 0xFFFFu);
+        } else {
+            back_edge = pin_s[slot];  // the pinned pass has to end where it began
+        }
+        __syncthreads();
     }
 }
 
@@ -329,17 +418,16 @@ __global__ __launch_bounds__(256) void pack_trellis_kernel(const uint16_t* __res
     packed[gid] = word;
 }
 
-// Workgroups the search keeps resident: the kernel holds its decode table in
-// registers; its register count leaves room for two waves per SIMD, i.e. two
-// workgroups per CU (three from K = 6 on, where fewer address registers are live).
-static int quantize_slots_wanted(int K) {
-    hipDeviceProp_t prop;
-    int dev = 0;
-    int cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-        cus = prop.multiProcessorCount;
-    return cus * (K >= 6 ? 3 : 2);
+static int quantize_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    return cus;
 }
+
+// Cost-history slots worth having: two tiles in flight on every CU.
+static int quantize_slots_wanted() { return 2 * quantize_cus(); }
 
 }  // namespace exl3
 
@@ -350,7 +438,7 @@ EXL3_EXPORT size_t exl3_quantize_slot_bytes(int K) {
 
 EXL3_EXPORT size_t exl3_quantize_workspace_bytes(int n_tiles, int K) {
     if (K < 2 || K > 8 || n_tiles < 1) return 0;
-    const int want = exl3::quantize_slots_wanted(K);
+    const int want = exl3::quantize_slots_wanted();
     return exl3_quantize_slot_bytes(K) * (size_t)(n_tiles < want ? n_tiles : want);
 }
 
@@ -366,12 +454,13 @@ EXL3_EXPORT int exl3_quantize_tiles(const float* tiles, int n_tiles, int K, int 
     const size_t slot = exl3_quantize_slot_bytes(K);
     size_t slots = workspace_bytes / slot;
     if (slots < 1) return EXL3_E_WORKSPACE;
-    const size_t want = (size_t)quantize_slots_wanted(K);
+    const size_t want = (size_t)quantize_slots_wanted();
     if (slots > want) slots = want;
     if (slots > (size_t)n_tiles) slots = (size_t)n_tiles;
-    const size_t edges = (size_t)1 << (16 - K);
-    const size_t pad = (size_t)((1 << K) > 8 ? (1 << K) : 8);
-    const size_t lds = 2 * sizeof(uint16_t) * (edges + edges / 256 * pad);  // two padded cost rows
+    // one workgroup per CU; slots beyond the grid are the workgroups' second ones
+    const size_t cus = (size_t)quantize_cus();
+    const size_t grid = slots < cus ? slots : cus;
+    const size_t lds = 2 * (sizeof(uint16_t) << (16 - K));  // two cost rows
     return dispatch_k_cb(K, cb, [&](auto k, auto c) {
         if constexpr (k.value < 2) {
             return (int)EXL3_E_BAD_K;
@@ -381,8 +470,9 @@ EXL3_EXPORT int exl3_quantize_tiles(const float* tiles, int n_tiles, int K, int 
                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
                 return (int)EXL3_E_LAUNCH;
             quantize_tiles_kernel<k.value, c.value>
-                <<<dim3((unsigned)slots), dim3(256), lds, as_stream(stream)>>>(
-                    tiles, q_tiles, indices, reinterpret_cast<uint16_t*>(workspace), n_tiles, 1.0f);
+                <<<dim3((unsigned)grid), dim3(kSearchThreads), lds, as_stream(stream)>>>(
+                    tiles, q_tiles, indices, reinterpret_cast<unsigned char*>(workspace), n_tiles,
+                    (int)slots);
             return launch_status();
         }
     });

@@ -18,16 +18,17 @@ from . import _lib
 from .layer import tensor_core_perm, tensor_core_perm_inverse
 from .ops import _check_cuda, _ptr, _stream
 
-# Bound on the backpointer scratch of one launch. The reference's default is
+# Bound on the path-cost scratch of one launch. The reference's default is
 # 256 MiB; here the default is what keeps every CU of the device busy (about
-# 2 GiB at K = 4), because a launch walks over any number of tiles with the slots
-# it has.
+# 1 GiB at K = 4, 4 GiB at K = 2), because a launch walks over any number of tiles
+# with the slots it has.
 DEFAULT_MAX_SCRATCH_BYTES = 4 << 30
 
 
 def scratch_bytes_per_tile(k: int) -> int:
-    """Backpointer bytes one resident tile needs (``_scratch_bytes_per_tile``,
-    metal_search.py:206-210; the two cost rows live in LDS here)."""
+    """Scratch bytes one resident tile needs (``_scratch_bytes_per_tile``,
+    metal_search.py:206-210): the cost rows of a pass, from which the backtrack works
+    out the predecessors on its path."""
     return int(_lib.load().exl3_quantize_slot_bytes(int(k)))
 
 

@@ -79,6 +79,23 @@ def test_small_scratch_budget_walks_the_batch_with_few_slots(cuda, oracle):
     np.testing.assert_array_equal(idx1, idx_all)
 
 
+@pytest.mark.parametrize("k,n", [(2, 1), (5, 255), (6, 257), (8, 511), (7, 515), (8, 1030)])
+def test_tile_counts_around_the_resident_slots(cuda, oracle, k, n):
+    """One tile per workgroup, a second one in flight on some or all of them, several
+    rounds with a ragged last one: every tile gets the oracle's path whatever its
+    place, and so it does with memory for 300 tiles in flight."""
+    from ponyexl3_amd import search
+
+    base = _tiles(900 + k, 3, 1.2)
+    q_ref, idx_ref = oracle.quantize_tiles_search(base, k, MCG)
+    at = np.arange(n) % 3
+    print(f"search k={k} n={n}", flush=True)
+    for budget in (search.DEFAULT_MAX_SCRATCH_BYTES, 300 * search.scratch_bytes_per_tile(k)):
+        q, idx = search.quantize_tiles_np(base[at], k, MCG, device=cuda, max_scratch_bytes=budget)
+        np.testing.assert_array_equal(idx, idx_ref[at])
+        np.testing.assert_array_equal(q, q_ref[at])
+
+
 def test_argument_errors(cuda):
     from ponyexl3_amd import search
 
