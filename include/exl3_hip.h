@@ -84,6 +84,19 @@ int exl3_decode_full_t(const uint16_t *trellis, int in_tiles, int out_tiles, int
                        int tn_offset, int tn_count, uint16_t *w_out_t, void *stream);
 
 /*
+ * Public weight diag(suh) . H128 . W_inner . H128 . diag(svh) of a slice of tile columns in
+ * one pass over the packed trellis, with the cast points of the runtime forward (the layer
+ * applied to an fp16 identity): replaces the identity-through-the-prefill-path fold of
+ * ponyexl3/mlx/native.py:49-85. in_tiles and tn_count are multiples of 8.
+ *   suh     fp16 [16*in_tiles] or NULL     svh  fp16 [16*tn_count] (of the slice) or NULL
+ *   w_out   fp16, 16-byte aligned: [16*in_tiles][16*tn_count], or transposed != 0:
+ *           [16*tn_count][16*in_tiles]
+ */
+int exl3_public_weight(const uint16_t *trellis, int in_tiles, int out_tiles, int K, int cb,
+                       const uint16_t *suh, const uint16_t *svh, int tn_offset, int tn_count,
+                       int transposed, uint16_t *w_out, void *stream);
+
+/*
  * Input-side Hadamard-128 with per-channel multipliers, fp32 butterflies:
  *   xh[r][s][:] = fp16( H128/sqrt(128) applied per 128-block to (x[r][:] * suh[s][:]) )
  * Replaces EXL3LayerRuntime.prepare_xh (ponyexl3/mlx/layer_state.py:133-136),

@@ -48,6 +48,7 @@ PROTOTYPES = {
     "exl3_pack_trellis": (_i, [_vp, ctypes.c_longlong, _i, _vp, _vp]),
     "exl3_decode_full_eg": (_i, [_vp, _i, _i, _i, _i, _i, _vp, _vp]),
     "exl3_decode_full_t": (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp]),
+    "exl3_public_weight": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i, _i, _i, _vp, _vp]),
     "exl3_had128_pre": (_i, [_vp, _i, _i, _vp, _i, _vp, _vp]),
     "exl3_had128_post": (_i, [_vp, _i, _i, _sz, _i, _i, _vp, _vp, _vp, _vp]),
     "exl3_gemv": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _sz, _vp]),

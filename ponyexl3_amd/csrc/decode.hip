@@ -9,6 +9,9 @@
 //
 // Transposed (out, in): one wavefront decodes the 8 tiles (tk0..tk0+7, tn), so
 // that each of the tile column's 16 output rows receives 128 contiguous halfs.
+//
+// exl3_public_weight: the same decode with both Hadamard transforms and scale vectors
+// applied on the way out (public_weight_kernel).
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 
@@ -116,6 +119,170 @@ __global__ __launch_bounds__(256) void decode_full_t_kernel(const uint32_t* __re
     }
 }
 
+// Public weight W_pub = diag(suh) . H . W_inner . H . diag(svh) of one 128 x 128 block per
+// workgroup, in (in, out) or (T) transposed (out, in) order, with the runtime's cast points:
+// the result of pushing an fp16 identity through rotation, GEMM and output transform
+// (ponyexl3/mlx/native.py:49-70) without the identity. Row i of the rotated identity is
+// q_i * sign(H[i][:]) with q_i = fp16(suh_i / sqrt(128)), so the GEMM is a Hadamard product
+// over the rows of the block:
+//   Y[i][n] = fp16(sum_j +-q_i W[j][n]),   Z[i][m] = fp16(sum_n +-Y[i][n] / sqrt(128) * svh_m)
+// Both run on the matrix pipe (v_mfma_f32_16x16x32_f16, fp32 sums in the order of the
+// prefill GEMM), the fragments of H made from sign words each lane holds. 512 MFMAs
+// per block = 21 us for 5120 x 17408 and the decode 9 us, so the kernel is bound by writing
+// the result; it goes out through LDS in 256-byte row pieces, non-temporal (nobody reads it
+// soon; 65 -> 62 us). One 34 KiB LDS tile serves all three stages (each stage reads its
+// operands into registers before the next one writes), so several workgroups share a CU and
+// their phases overlap; four instead of three per CU (128 registers) is no faster.
+// Measured, 5120 x 17408 at K = 4, transposed: 62 us (3.6 TB/s of trellis and result); the
+// identity through the prefill kernels, the concatenation of its column stripes and the
+// transposed copy took 1.42 ms.
+constexpr int kPubLd = 128 + kDecPad;  // halfs per row: 16-byte reads of 16 rows hit all banks
+
+// Signs of a fragment of H128 for rows / columns 16 nt + fr and k = 32 ks + 8 q + 0..7: entry
+// (k, n) has sign parity(k & n), which splits into a part the lane knows (fr, q and the k
+// inside the fragment), a part that needs nt & 1, and one that is the same for every lane
+// (nt >> 1 and ks). get() is the fragment times `mag`, an fp16 value in both halves.
+struct HadamardFragments {
+    uint4_t base, odd;  // sign bits for nt even, nt odd
+    __device__ __forceinline__ HadamardFragments(int lane) {
+        const int fr = lane & 15, q = lane >> 4;
+        const uint32_t flip = ((fr >> 3) & q & 1) ? 0x80008000u : 0u;
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t lo = __builtin_popcount(fr & 7 & (2 * i)) & 1;
+            const uint32_t hi = __builtin_popcount(fr & 7 & (2 * i + 1)) & 1;
+            w[i] = (lo << 15) ^ (hi << 31) ^ flip;
+        }
+        base = uint4_t{w[0], w[1], w[2], w[3]};
+        odd = base ^ ((q >> 1) ? 0x80008000u : 0u);
+    }
+    template <int NT, int KS>
+    __device__ __forceinline__ half8_t get(uint32_t mag) const {
+        constexpr bool neg = (((NT >> 1) & KS & 1) ^ ((NT >> 2) & (KS >> 1) & 1)) != 0;
+        return __builtin_bit_cast(half8_t, ((NT & 1) ? odd : base) ^ (neg ? mag ^ 0x80008000u : mag));
+    }
+};
+
+template <int K, int CB, bool T>
+__global__ __launch_bounds__(256, 3) void public_weight_kernel(
+    const uint32_t* __restrict__ trellis, const half_t* __restrict__ suh,
+    const half_t* __restrict__ svh, half_t* __restrict__ w_out, int out_tiles, int tn_offset,
+    int blocks_fast, size_t ldw) {
+    constexpr float kScale = 0.088388347648318440550f;  // 1/sqrt(128)
+    __shared__ __attribute__((aligned(16))) half_t tile[128 * kPubLd];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int fr = lane & 15, q = lane >> 4;
+    // consecutive workgroups write consecutive pieces of the same output rows
+    const int fast = blockIdx.x % blocks_fast, slow = blockIdx.x / blocks_fast;
+    const int bi = T ? fast : slow, bn = T ? slow : fast;
+
+    // decode: wave w takes tile rows 2w, 2w + 1; a lane's two columns go to tile[n][j], 16
+    // consecutive j (pairs {2cs + hh + 4t, t = 0..3} are rows 8hh..8hh+7 of column cs)
+    {
+        uint32_t own[2][K];
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const uint32_t* p = trellis + ((size_t)(bi * 8 + 2 * wave + r) * out_tiles + tn_offset + bn * 8) * (8 * K) +
+                                lane * K;
+#pragma unroll
+            for (int i = 0; i < K; i++) own[r][i] = __builtin_nontemporal_load(p + i);
+        }
+        const int n0 = (lane >> 3) * 16 + (lane & 7);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const LaneWords<K> lw = finish_lane_words<K>(own[r], lane);
+            half2_t wp[16];
+            decode_lane<K, CB>(lw, wp);
+#pragma unroll
+            for (int cs = 0; cs < 2; cs++)
+#pragma unroll
+                for (int hh = 0; hh < 2; hh++) {
+                    const half2_t* c = wp + 8 * cs + 4 * hh;
+                    *reinterpret_cast<uint4_t*>(tile + (n0 + 8 * cs) * kPubLd + (2 * wave + r) * 16 + 8 * hh) =
+                        uint4_t{half2_to_bits(c[0]), half2_to_bits(c[1]), half2_to_bits(c[2]), half2_to_bits(c[3])};
+                }
+        }
+    }
+    __syncthreads();
+    const HadamardFragments had(lane);
+    half8_t op[2][4];
+    float4_t acc[2][8];
+    auto read_operands = [&] {  // rows 32 wave .. + 31 of the tile, all 128 k
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++)
+                op[rt][ks] = *reinterpret_cast<const half8_t*>(tile + (wave * 32 + rt * 16 + fr) * kPubLd + ks * 32 + q * 8);
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+            for (int nt = 0; nt < 8; nt++) acc[rt][nt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    };
+
+    // Y^T[n][i] = sum_j W^T[n][j] H[j][i]: a lane gets four consecutive n of one i
+    read_operands();
+    __syncthreads();
+    static_for<0, 8>([&](auto nt) {
+        const float su = suh ? (float)suh[bi * 128 + nt.value * 16 + fr] : 1.0f;
+        const uint32_t qi = half_to_bits((half_t)__fmul_rn(su, kScale)) * 0x10001u;
+        static_for<0, 4>([&](auto ks) {
+            const half8_t h = had.template get<nt.value, ks.value>(qi);
+#pragma unroll
+            for (int rt = 0; rt < 2; rt++)
+                acc[rt][nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[rt][ks.value], h,
+                                                                           acc[rt][nt.value], 0, 0, 0);
+        });
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++) {
+            half4_t o;
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] = (half_t)acc[rt][nt.value][c];
+            *reinterpret_cast<half4_t*>(tile + (nt.value * 16 + fr) * kPubLd + wave * 32 + rt * 16 + q * 4) = o;
+        }
+    });
+    __syncthreads();
+
+    // Z: a lane gets four consecutive i of one m (T) or four consecutive m of one i
+    read_operands();
+    __syncthreads();
+    static_for<0, 4>([&](auto ks) {
+        static_for<0, 8>([&](auto nt) {
+            const half8_t h = had.template get<nt.value, ks.value>(0x3C003C00u);
+#pragma unroll
+            for (int rt = 0; rt < 2; rt++)
+                acc[rt][nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    T ? op[rt][ks.value] : h, T ? h : op[rt][ks.value], acc[rt][nt.value], 0, 0, 0);
+        });
+    });
+    const half_t* sv = svh ? svh + bn * 128 : nullptr;
+#pragma unroll
+    for (int nt = 0; nt < 8; nt++) {
+        float s[4] = {1.f, 1.f, 1.f, 1.f};
+        if (sv) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) s[c] = (float)(T ? sv[nt * 16 + fr] : sv[nt * 16 + q * 4 + c]);
+        }
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++) {
+            half4_t o;
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] = (half_t)__fmul_rn(__fmul_rn(acc[rt][nt][c], kScale), s[c]);
+            half_t* dst = T ? tile + (nt * 16 + fr) * kPubLd + wave * 32 + rt * 16 + q * 4
+                            : tile + (wave * 32 + rt * 16 + fr) * kPubLd + nt * 16 + q * 4;
+            *reinterpret_cast<half4_t*>(dst) = o;
+        }
+    }
+    __syncthreads();
+    half_t* out = w_out + (size_t)(T ? bn : bi) * 128 * ldw + (size_t)(T ? bi : bn) * 128;
+#pragma unroll
+    for (int it = 0; it < 8; it++) {
+        const int row = it * 16 + (threadIdx.x >> 4), c = (threadIdx.x & 15) * 8;
+        __builtin_nontemporal_store(*reinterpret_cast<const uint4_t*>(tile + row * kPubLd + c),
+                                    reinterpret_cast<uint4_t*>(out + (size_t)row * ldw + c));
+    }
+}
+
 // Packed tiles -> their 256 16-bit codewords in kernel (stream) order
 // (unpack_trellis, ponyexl3/ref/trellis.py:153-214). Lanes 8t..8t+7 of a wave own
 // tile t of eight consecutive tiles; lane u extracts codewords 32u..32u+31 and
@@ -204,6 +371,33 @@ EXL3_EXPORT int exl3_decode_full_t(const uint16_t* trellis, int in_tiles, int ou
             <<<dim3((unsigned)grid), dim3(256), 0, as_stream(stream)>>>(
                 reinterpret_cast<const uint32_t*>(trellis), reinterpret_cast<half_t*>(w_out_t),
                 in_tiles, out_tiles, tn_offset, tn_count);
+        return launch_status();
+    });
+}
+
+EXL3_EXPORT int exl3_public_weight(const uint16_t* trellis, int in_tiles, int out_tiles, int K,
+                                   int cb, const uint16_t* suh, const uint16_t* svh, int tn_offset,
+                                   int tn_count, int transposed, uint16_t* w_out, void* stream) {
+    using namespace exl3;
+    if (int rc = check_k_cb(K, cb)) return rc;
+    if (!trellis || !w_out) return EXL3_E_NULL_POINTER;
+    if (in_tiles < 0 || out_tiles < 0 || tn_offset < 0 || tn_count < 0 || in_tiles % 8 ||
+        tn_count % 8 || tn_offset + tn_count > out_tiles)
+        return EXL3_E_BAD_SHAPE;
+    if (in_tiles == 0 || tn_count == 0) return EXL3_OK;
+    if ((reinterpret_cast<uintptr_t>(w_out) & 15) || (reinterpret_cast<uintptr_t>(trellis) & 3))
+        return EXL3_E_BAD_SHAPE;
+    const int blocks_in = in_tiles / 8, blocks_out = tn_count / 8;
+    const long long grid = (long long)blocks_in * blocks_out;
+    if (grid > 0x7FFFFFFFLL) return EXL3_E_BAD_SHAPE;
+    return dispatch_k_cb(K, cb, [&](auto k, auto c) {
+        auto kernel = transposed ? public_weight_kernel<k.value, c.value, true>
+                                 : public_weight_kernel<k.value, c.value, false>;
+        kernel<<<dim3((unsigned)grid), dim3(256), 0, as_stream(stream)>>>(
+            reinterpret_cast<const uint32_t*>(trellis), reinterpret_cast<const half_t*>(suh),
+            reinterpret_cast<const half_t*>(svh), reinterpret_cast<half_t*>(w_out), out_tiles,
+            tn_offset, transposed ? blocks_in : blocks_out,
+            (size_t)(transposed ? in_tiles : tn_count) * 16);
         return launch_status();
     });
 }

@@ -46,6 +46,29 @@ def test_public_weight_equals_identity_through_the_module(cuda):
     assert float((fold != module).float().mean()) < 0.01
 
 
+@pytest.mark.parametrize("k,cb,n_in,n_out", [(1, 0, 128, 128), (2, 1, 384, 1152), (5, 2, 128, 256),
+                                             (7, 0, 640, 128), (8, 1, 256, 384)])
+def test_public_weight_slices_and_transpose(cuda, oracle, k, cb, n_in, n_out):
+    """One block, one block row, one block column, general scale vectors and none:
+    against the oracle; a slice and the transposed form hold the same bits."""
+    from ponyexl3_amd import ops
+
+    rng = np.random.default_rng(40 + k)
+    tr = rng.integers(0, 65536, size=(n_in // 16, n_out // 16, 16 * k), dtype=np.uint16)
+    suh = (rng.standard_normal(n_in) * 0.7).astype(np.float16)
+    svh = (rng.standard_normal(n_out) * 0.02).astype(np.float16)
+    trt, s, v = ops.as_trellis_tensor(tr, cuda), torch.from_numpy(suh).to(cuda), torch.from_numpy(svh).to(cuda)
+    print(f"public weight k={k} cb={cb} {n_in}x{n_out}", flush=True)
+    w = ops.public_weight(trt, k, cb, s, v)
+    assert rel_l2(w.cpu().numpy(), oracle.reconstruct_public_weights(tr, suh, svh, k, cb)) < 1e-3
+    assert torch.equal(ops.public_weight(trt, k, cb, s, v, transposed=True), w.T)
+    last = ops.public_weight(trt, k, cb, s, v[-128:].contiguous(), tn_offset=n_out // 16 - 8)
+    assert torch.equal(last, w[:, -128:])
+    one_in, one_out = np.ones(n_in, np.float16), np.ones(n_out, np.float16)
+    plain = ops.public_weight(trt, k, cb)
+    assert rel_l2(plain.cpu().numpy(), oracle.reconstruct_public_weights(tr, one_in, one_out, k, cb)) < 1e-3
+
+
 @pytest.mark.parametrize("bias", [False, True])
 def test_folded_linear_tracks_exact_layer(cuda, oracle, bias):
     from ponyexl3_amd import make_exl3_layer, native
