@@ -12,6 +12,7 @@ import os
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libexl3_hip.so")
+HOST_LIB_PATH = os.path.join(_PKG_DIR, "_exl3_host.so")
 DIAG_LIB_PATH = os.path.join(_PKG_DIR, "libexl3_diag.so")
 
 EXL3_OK = 0
@@ -89,6 +90,7 @@ DIAG_PROTOTYPES = {
 
 _lib = None
 _diag = None
+_host = None
 
 
 def load() -> ctypes.CDLL:
@@ -109,6 +111,20 @@ def load() -> ctypes.CDLL:
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+def host():
+    """The native host path of the modules (``_exl3_host.so``, built from
+    csrc/torch_host.cpp over the C ABI of libexl3_hip.so)."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_LIB_PATH):
+            raise RuntimeError(f"{HOST_LIB_PATH} is missing: run `python -m ponyexl3_amd.build`")
+        from . import _exl3_host
+
+        _host = _exl3_host
+    return _host
 
 
 def load_diag() -> ctypes.CDLL:

@@ -4,7 +4,8 @@
 file is one translation unit compiled in parallel; the objects are linked into
 ``ponyexl3_amd/libexl3_hip.so``, the C-ABI library declared in
 ``include/exl3_hip.h``, and (``diag.hip`` alone) ``ponyexl3_amd/libexl3_diag.so``,
-the measurement probes declared in ``include/exl3_diag.h``.
+the measurement probes declared in ``include/exl3_diag.h``. ``torch_host.cpp``, the
+modules' host path over that library, becomes ``ponyexl3_amd/_exl3_host.so``.
 """
 
 from __future__ import annotations
@@ -14,6 +15,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
@@ -24,6 +26,9 @@ SOURCES = ["decode.hip", "hadamard.hip", "gemv.hip", "linear_mid.hip", "gemm.hip
 # measurement probes (include/exl3_diag.h): a library of their own, kept out of the product ABI
 DIAG_SOURCES = ["diag.hip"]
 DIAG_LIB_PATH = os.path.join(PKG_DIR, "libexl3_diag.so")
+
+HOST_SOURCE = "torch_host.cpp"
+HOST_LIB_PATH = os.path.join(PKG_DIR, "_exl3_host.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -58,12 +63,45 @@ def _compile(src: str, extra: list[str]) -> str:
     return obj
 
 
+def _compile_host() -> str:
+    """The CPython extension against this interpreter's torch; returns its object file."""
+    import torch
+
+    inc = os.path.join(os.path.dirname(torch.__file__), "include")
+    obj = os.path.join(OBJ_DIR, "torch_host.o")
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+           "-isystem", inc, "-isystem", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+           "-isystem", sysconfig.get_paths()["include"],
+           "-c", os.path.join(CSRC, HOST_SOURCE), "-o", obj]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {HOST_SOURCE}:\n{proc.stderr[-8000:]}")
+    if proc.stderr.strip():
+        sys.stderr.write(proc.stderr)
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    import torch
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [shutil.which("g++") or "c++", "-shared", "-o", HOST_LIB_PATH, obj, f"-L{lib}", f"-L{PKG_DIR}",
+           "-lexl3_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link failed:\n{proc.stderr[-4000:]}")
+
+
 def build(verbose: bool = False, jobs: int | None = None, extra_flags: list[str] | None = None) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     extra = list(extra_flags or [])
     every = SOURCES + DIAG_SOURCES
-    jobs = jobs or min(len(every), int(os.environ.get("MAX_JOBS", "8")))
+    jobs = jobs or min(len(every) + 1, int(os.environ.get("MAX_JOBS", "8")))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host)
         objs = list(pool.map(lambda s: _compile(s, extra), every))
     for path, group in ((LIB_PATH, objs[: len(SOURCES)]), (DIAG_LIB_PATH, objs[len(SOURCES):])):
         cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", path, *group]
@@ -72,6 +110,9 @@ def build(verbose: bool = False, jobs: int | None = None, extra_flags: list[str]
             raise RuntimeError(f"link failed:\n{proc.stderr[-4000:]}")
         if verbose:
             print(f"built {path} ({os.path.getsize(path)} bytes)")
+    _link_host(host.result())
+    if verbose:
+        print(f"built {HOST_LIB_PATH} ({os.path.getsize(HOST_LIB_PATH)} bytes)")
     return LIB_PATH
 
 

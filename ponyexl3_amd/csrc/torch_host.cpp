@@ -1,0 +1,326 @@
+// Host path of the torch modules in native code: one call per layer forward that checks the
+// activations, allocates the output, finds the stream's scratch and launches through the C
+// ABI of libexl3_hip.so. The same steps in Python (tensor methods, three size queries and a
+// ctypes call with 18 arguments) took 22 us per call, nearly four times the GPU time of a
+// small layer (5120 -> 1024, one row: 5.8 us); calls now follow each other at 6.8 us.
+//
+// The module also owns the scratch buffers and counters of every (device, stream).
+// Everything runs under the GIL.
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cstdint>
+#include <map>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "../../include/exl3_hip.h"
+
+namespace {
+
+// Raises what ponyexl3_amd._lib.check raises for a status code.
+void check_status(int rc, const char* what) {
+    if (rc == EXL3_OK) return;
+    PyObject* mod = PyImport_ImportModule("ponyexl3_amd._lib");
+    PyObject* r = mod ? PyObject_CallMethod(mod, "check", "is", rc, what) : nullptr;
+    Py_XDECREF(mod);
+    Py_XDECREF(r);
+    throw python_error();
+}
+
+[[noreturn]] void value_error(const std::string& msg) {
+    PyErr_SetString(PyExc_ValueError, msg.c_str());
+    throw python_error();
+}
+
+const uint16_t* half_ptr(const at::Tensor& t) {
+    return t.defined() ? static_cast<const uint16_t*>(t.const_data_ptr()) : nullptr;
+}
+const int32_t* int_ptr(const at::Tensor& t) {
+    return t.defined() ? static_cast<const int32_t*>(t.const_data_ptr()) : nullptr;
+}
+uint16_t* half_out(const at::Tensor& t) { return static_cast<uint16_t*>(t.mutable_data_ptr()); }
+
+at::Tensor tensor_or_none(PyObject* o, const char* name) {
+    if (o == Py_None) return {};
+    if (!THPVariable_Check(o)) value_error(std::string(name) + " must be a torch.Tensor");
+    return THPVariable_Unpack(o);
+}
+
+// ---------------------------------------------------------------------------
+// Scratch of one (device, stream): launches on one stream are ordered, so they can share
+// buffers; two streams of a device running EXL3 layers at the same time must not (the
+// counters and partial rows of one launch would be read by the other). A buffer that is
+// replaced by a larger one stays allocated: a HIP graph captured earlier still replays
+// launches that point into it. Buffers grow by half at least, which bounds what is kept.
+struct Scratch {
+    at::Tensor buf[3];
+};
+enum { kWorkspace = 0, kGemmWorkspace = 1, kCounters = 2 };
+
+std::map<std::pair<int, void*>, Scratch>& scratch_map() {
+    static auto* m = new std::map<std::pair<int, void*>, Scratch>;  // never destroyed: outlives the HIP runtime
+    return *m;
+}
+std::vector<at::Tensor>& retired() {
+    static auto* v = new std::vector<at::Tensor>;
+    return *v;
+}
+
+struct StreamContext {
+    int device;
+    void* stream;
+    Scratch& scratch;
+    explicit StreamContext(int dev)
+        : device(dev),
+          stream(c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(dev)).stream()),
+          scratch(scratch_map()[{dev, stream}]) {}
+
+    // `n` bytes of scratch, or an int32 array of at least n zeroed when created (the kernels
+    // leave it zero)
+    const at::Tensor& get(int kind, size_t n) {
+        at::Tensor& t = scratch.buf[kind];
+        if (!t.defined() || static_cast<size_t>(t.numel()) < n) {
+            size_t want = std::max(n, t.defined() ? static_cast<size_t>(t.numel()) * 3 / 2 : 0);
+            want = std::max<size_t>(want, kind == kCounters ? 4096 : size_t(1) << 20);
+            if (t.defined()) retired().push_back(t);
+            const auto opt = at::TensorOptions()
+                                 .device(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device)))
+                                 .dtype(kind == kCounters ? at::kInt : at::kByte);
+            t = kind == kCounters ? at::zeros({static_cast<int64_t>(want)}, opt)
+                                  : at::empty({static_cast<int64_t>(want)}, opt);
+        }
+        return t;
+    }
+};
+
+// scratch(kind, device index, n) -> tensor of the device's current stream, or None where
+// there is none yet and n < 0
+PyObject* py_scratch(PyObject*, PyObject* args) {
+    HANDLE_TH_ERRORS
+    int kind, device;
+    long long n;
+    if (!PyArg_ParseTuple(args, "iiL", &kind, &device, &n)) throw python_error();
+    if (kind < 0 || kind > 2) value_error("unknown scratch kind");
+    StreamContext ctx(device);
+    if (n < 0) {
+        if (!ctx.scratch.buf[kind].defined()) Py_RETURN_NONE;
+        return THPVariable_Wrap(ctx.scratch.buf[kind]);
+    }
+    return THPVariable_Wrap(ctx.get(kind, static_cast<size_t>(n)));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---------------------------------------------------------------------------
+// A linear layer or a sibling-fused group.
+struct LinearLayer {
+    at::Tensor trellis, suh, svh, bias, group_sub, block_sub;
+    std::vector<int64_t> member_out;  // out_features of each sibling; empty = one linear
+    int k = 0, cb = 0, in_tiles = 0, out_tiles = 0, n_sub = 1;
+    int64_t in_features() const { return int64_t(in_tiles) * 16; }
+    int64_t out_features() const { return int64_t(out_tiles) * 16; }
+};
+
+// x: contiguous fp16 (rows, in) on the layer's device, y: (rows, out)
+void linear_run(const LinearLayer& l, const at::Tensor& x, int64_t rows64, const at::Tensor& y, bool fused) {
+    if (rows64 == 0) return;
+    if (rows64 > INT32_MAX) value_error("too many rows");
+    const int rows = static_cast<int>(rows64);
+    const int n_in = l.in_tiles * 16, n_out = l.out_tiles * 16;
+    const int small_rows = exl3_gemv_max_rows();
+    StreamContext ctx(x.device().index());
+    const uint16_t* xp = half_ptr(x);
+    uint16_t* yp = half_out(y);
+    const uint16_t* tr = half_ptr(l.trellis);
+    if (l.n_sub > 1 && rows > (fused ? exl3_linear_small_max_rows() : small_rows)) {
+        bool one_launch = true;  // members end on 256-column blocks
+        int64_t total = 0;
+        for (int64_t n : l.member_out) {
+            one_launch = one_launch && n % 256 == 0;
+            total += n;
+        }
+        if (l.member_out.size() != static_cast<size_t>(l.n_sub) || total != n_out)
+            value_error("member_out must list the out_features of the stacked members");
+        const at::Tensor xh = at::empty({rows64, l.n_sub, n_in}, x.options());
+        check_status(exl3_had128_pre(xp, rows, n_in, half_ptr(l.suh), l.n_sub, half_out(xh), ctx.stream),
+                     "exl3_had128_pre");
+        if (one_launch) {
+            // one GEMM launch over all members, each block reading its member's rotation, then
+            // the output transform
+            const at::Tensor block_sub =
+                l.block_sub.defined() ? l.block_sub : l.group_sub.slice(0, 0, l.group_sub.numel(), 2).contiguous();
+            const size_t bytes = exl3_linear_prefill_workspace_bytes(rows, n_in, n_out);
+            const at::Tensor& ws = ctx.get(kWorkspace, bytes);
+            check_status(exl3_linear_prefill(half_ptr(xh), rows, l.n_sub, tr, l.in_tiles, l.out_tiles, l.k, l.cb,
+                                             int_ptr(block_sub), half_ptr(l.svh), half_ptr(l.bias), yp,
+                                             ws.mutable_data_ptr(), ws.numel(), ctx.stream),
+                         "exl3_linear_prefill");
+            return;
+        }
+        int tn0 = 0;
+        for (size_t i = 0; i < l.member_out.size(); i++) {
+            if (l.member_out[i] % 128) value_error("member out_features must be multiples of 128");
+            const int tn = static_cast<int>(l.member_out[i] / 16);
+            const size_t bytes = exl3_gemm_workspace_bytes(rows, l.in_tiles, tn);
+            void* ws = bytes ? ctx.get(kGemmWorkspace, bytes).mutable_data_ptr() : nullptr;
+            check_status(exl3_gemm(half_ptr(xh) + i * n_in, rows, size_t(l.n_sub) * n_in, tr, l.in_tiles, l.out_tiles,
+                                   l.k, l.cb, tn0, tn, yp + size_t(16) * tn0, n_out, ws, bytes, ctx.stream),
+                         "exl3_gemm");
+            tn0 += tn;
+        }
+        check_status(exl3_had128_post(yp, 0, 1, size_t(rows) * n_out, rows, n_out, half_ptr(l.svh), half_ptr(l.bias),
+                                      yp, ctx.stream),
+                     "exl3_had128_post");
+        return;
+    }
+    const size_t bytes = exl3_linear_workspace_bytes(rows, n_in, n_out, l.n_sub);
+    const at::Tensor& ws = ctx.get(kWorkspace, bytes);
+    int32_t* cnt = nullptr;
+    size_t cnt_len = 0;
+    if (fused) {
+        // one-launch kernel: a 64-bit accumulator per (row, output column) = two ints each;
+        // medium-batch kernel: one counter per 128-column group. Two more for the status word.
+        const size_t n = rows <= small_rows ? size_t(2) * rows * n_out : n_out / 128;
+        const at::Tensor& c = ctx.get(kCounters, n + 2);
+        cnt = static_cast<int32_t*>(c.mutable_data_ptr());
+        cnt_len = c.numel();
+    }
+    check_status(exl3_linear_forward(xp, rows, tr, l.in_tiles, l.out_tiles, l.k, l.cb, half_ptr(l.suh), l.n_sub,
+                                     int_ptr(l.group_sub), half_ptr(l.svh), half_ptr(l.bias), yp,
+                                     ws.mutable_data_ptr(), ws.numel(), cnt, cnt_len, ctx.stream),
+                 "exl3_linear_forward");
+}
+
+// Activations as the kernels take them: fp16, contiguous, last dimension `features`.
+at::Tensor activations(PyObject* arg, int64_t features) {
+    if (!THPVariable_Check(arg)) value_error("x must be a torch.Tensor");
+    at::Tensor x = THPVariable_Unpack(arg);
+    if (x.dim() < 1 || x.size(-1) != features)
+        value_error("expected last dim " + std::to_string(features) + ", got " +
+                    (x.dim() < 1 ? std::string("a scalar") : std::to_string(x.size(-1))));
+    if (!x.is_cuda()) value_error("x must live on the GPU (got device " + x.device().str() + ")");
+    if (x.scalar_type() != at::kHalf) x = x.to(at::kHalf);
+    return x.is_contiguous() ? x : x.contiguous();
+}
+
+struct PyLinear {
+    PyObject_HEAD
+    LinearLayer* layer;
+};
+
+int linear_init(PyObject* self, PyObject* args, PyObject*) {
+    try {
+        PyObject *trellis, *suh, *svh, *bias, *group_sub, *block_sub, *members;
+        int k, cb;
+        if (!PyArg_ParseTuple(args, "OiiOOOOOO", &trellis, &k, &cb, &suh, &svh, &bias, &group_sub, &block_sub, &members))
+            return -1;
+        auto l = std::make_unique<LinearLayer>();
+        l->trellis = tensor_or_none(trellis, "trellis");
+        if (!l->trellis.defined() || l->trellis.dim() != 3) value_error("trellis must be 3D (in_tiles, out_tiles, 16*K)");
+        l->suh = tensor_or_none(suh, "suh");
+        l->svh = tensor_or_none(svh, "svh");
+        l->bias = tensor_or_none(bias, "bias");
+        l->group_sub = tensor_or_none(group_sub, "group_sub");
+        l->block_sub = tensor_or_none(block_sub, "block_sub");
+        l->k = k;
+        l->cb = cb;
+        l->in_tiles = static_cast<int>(l->trellis.size(0));
+        l->out_tiles = static_cast<int>(l->trellis.size(1));
+        l->n_sub = l->suh.defined() && l->suh.dim() == 2 ? static_cast<int>(l->suh.size(0)) : 1;
+        if (members != Py_None) {
+            PyObject* seq = PySequence_Fast(members, "member_out must be a sequence");
+            if (!seq) return -1;
+            for (Py_ssize_t i = 0; i < PySequence_Fast_GET_SIZE(seq); i++)
+                l->member_out.push_back(PyLong_AsLongLong(PySequence_Fast_GET_ITEM(seq, i)));
+            Py_DECREF(seq);
+            if (PyErr_Occurred()) return -1;
+        }
+        delete reinterpret_cast<PyLinear*>(self)->layer;
+        reinterpret_cast<PyLinear*>(self)->layer = l.release();
+        return 0;
+    } catch (python_error& e) {
+        e.restore();
+        return -1;
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return -1;
+    }
+}
+
+void linear_dealloc(PyObject* self) {
+    delete reinterpret_cast<PyLinear*>(self)->layer;
+    Py_TYPE(self)->tp_free(self);
+}
+
+// layer(x): (..., in) -> (..., out) fp16, or for a group a tuple of its members' outputs
+// (views of one buffer)
+PyObject* linear_call(PyObject* self, PyObject* args, PyObject* kwargs) {
+    HANDLE_TH_ERRORS
+    const LinearLayer* l = reinterpret_cast<PyLinear*>(self)->layer;
+    if (!l || PyTuple_GET_SIZE(args) != 1 || kwargs) value_error("a layer takes one positional argument");
+    const at::Tensor x = activations(PyTuple_GET_ITEM(args, 0), l->in_features());
+    c10::OptionalDeviceGuard guard(x.device());
+    at::DimVector shape(x.sizes());
+    shape.back() = l->out_features();
+    at::Tensor y = at::empty(shape, x.options());
+    linear_run(*l, x, x.numel() / l->in_features(), y, true);
+    if (l->member_out.empty()) return THPVariable_Wrap(std::move(y));
+    PyObject* out = PyTuple_New(static_cast<Py_ssize_t>(l->member_out.size()));
+    if (!out) throw python_error();
+    int64_t at_col = 0;
+    for (size_t i = 0; i < l->member_out.size(); i++) {
+        PyTuple_SET_ITEM(out, static_cast<Py_ssize_t>(i), THPVariable_Wrap(y.narrow(-1, at_col, l->member_out[i])));
+        at_col += l->member_out[i];
+    }
+    return out;
+    END_HANDLE_TH_ERRORS
+}
+
+// layer.rows(x2d, fused): operator form, x checked by the caller
+PyObject* linear_rows(PyObject* self, PyObject* args) {
+    HANDLE_TH_ERRORS
+    PyObject* x_arg;
+    int fused;
+    if (!PyArg_ParseTuple(args, "Op", &x_arg, &fused)) throw python_error();
+    const LinearLayer* l = reinterpret_cast<PyLinear*>(self)->layer;
+    if (!l) value_error("not initialised");
+    const at::Tensor x = activations(x_arg, l->in_features());
+    c10::OptionalDeviceGuard guard(x.device());
+    const int64_t rows = x.numel() / l->in_features();
+    at::Tensor y = at::empty({rows, l->out_features()}, x.options());
+    linear_run(*l, x, rows, y, fused != 0);
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef linear_methods[] = {{"rows", linear_rows, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+
+PyTypeObject linear_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyMethodDef module_methods[] = {{"scratch", py_scratch, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_exl3_host", nullptr, -1, module_methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__exl3_host() {
+    linear_type.tp_name = "ponyexl3_amd._exl3_host.Linear";
+    linear_type.tp_basicsize = sizeof(PyLinear);
+    linear_type.tp_flags = Py_TPFLAGS_DEFAULT;
+    linear_type.tp_new = PyType_GenericNew;
+    linear_type.tp_init = linear_init;
+    linear_type.tp_dealloc = linear_dealloc;
+    linear_type.tp_call = linear_call;
+    linear_type.tp_methods = linear_methods;
+    if (PyType_Ready(&linear_type) < 0) return nullptr;
+    PyObject* m = PyModule_Create(&module_def);
+    if (!m) return nullptr;
+    Py_INCREF(&linear_type);
+    if (PyModule_AddObject(m, "Linear", reinterpret_cast<PyObject*>(&linear_type)) < 0) return nullptr;
+    return m;
+}

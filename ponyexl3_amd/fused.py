@@ -15,7 +15,7 @@ import weakref
 import numpy as np
 import torch
 
-from . import ops
+from . import _lib, ops
 from .layer import EXL3Layer, codebook_mode_from_flags, unpack_signs_or_pass
 
 
@@ -66,19 +66,22 @@ class FusedEXL3Group(torch.nn.Module):
         self._cache_key = None
         self._cache_out = None
         self._cache_served: set = set()
+        self._native = None
+
+    def __getstate__(self):
+        # the native handle is made again on the first call of a copy
+        return {**self.__dict__, "_native": None}
 
     def extra_repr(self) -> str:
         return f"members={self._keys}, k={self._k}"
 
     def forward_all(self, x: torch.Tensor) -> tuple[torch.Tensor, ...]:
-        lead = tuple(x.shape[:-1])
-        x2d = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
-        y = ops.linear_forward(
-            x2d, self._trellis, self._k, self._cb, self._suh_stack, self._svh_cat, None,
-            self._group_sub, member_out=self._out_features, block_sub=self._block_sub,
-        )
-        outs = torch.split(y, self._out_features, dim=-1)
-        return tuple(o.reshape(lead + (n,)) for o, n in zip(outs, self._out_features))
+        native = self._native
+        if native is None:
+            native = self._native = _lib.host().Linear(
+                self._trellis, self._k, self._cb, self._suh_stack, self._svh_cat, None, self._group_sub,
+                self._block_sub, self._out_features)
+        return native(x)
 
     def _same_input(self, x: torch.Tensor, idx: int | None = None) -> bool:
         """Whether x is the input the cached outputs were computed from. The reference

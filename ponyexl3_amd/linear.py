@@ -15,7 +15,7 @@ from typing import Any
 import numpy as np
 import torch
 
-from . import ops
+from . import _lib, ops
 from .layer import EXL3Layer, codebook_mode_from_flags, unpack_signs_or_pass
 
 
@@ -91,6 +91,7 @@ class EXL3Linear(torch.nn.Module):
         self._rt = layer_runtime(layer, device)
         self.in_features = layer.in_features
         self.out_features = layer.out_features
+        self._native = None
 
     def extra_repr(self) -> str:
         return f"in={self.in_features}, out={self.out_features}, k={self._exl3.k}"
@@ -103,10 +104,14 @@ class EXL3Linear(torch.nn.Module):
         self._exl3.trellis = None
         return self
 
+    def __getstate__(self):
+        # the native handle is made again on the first call of a copy
+        return {**self.__dict__, "_native": None}
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        rt = self._rt
-        if x.shape[-1] != self.in_features:
-            raise ValueError(f"expected last dim {self.in_features}, got {x.shape[-1]}")
-        x2d = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
-        y = ops.linear_forward(x2d, rt.trellis, rt.k, rt.cb, rt.suh, rt.svh, rt.bias)
-        return y.reshape(tuple(x.shape[:-1]) + (self.out_features,))
+        native = self._native
+        if native is None:
+            rt = self._rt
+            native = self._native = _lib.host().Linear(rt.trellis, rt.k, rt.cb, rt.suh, rt.svh, rt.bias, None, None,
+                                                       None)
+        return native(x)

@@ -17,12 +17,6 @@ import torch
 
 from . import _lib
 
-_workspaces: dict = {}
-# Buffers that were replaced by larger ones stay allocated: a HIP graph captured
-# earlier still replays launches that point into them.
-_retired: list = []
-
-
 def _check_cuda(t: torch.Tensor, name: str) -> None:
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch.Tensor")
@@ -40,28 +34,18 @@ def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-def _buffer_key(device):
-    """Scratch buffers and counters belong to one (device, stream) pair: launches on
-    one stream are ordered, so they can share a buffer; two streams of a device
-    running EXL3 layers at the same time must not (the group counters and partial
-    rows of one launch would be read by the other)."""
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    return (device.type, index, torch.cuda.current_stream(index).cuda_stream)
+# Scratch buffers and counters belong to one (device, stream) pair and live in the native
+# host module, which the layer modules use directly (csrc/torch_host.cpp).
+_WORKSPACE, _GEMM_WORKSPACE, _COUNTERS = 0, 1, 2
+
+
+def _device_index(device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
 
 
 def workspace(device, nbytes: int) -> torch.Tensor:
     """Scratch buffer of the current (device, stream), grown on demand."""
-    key = _buffer_key(device)
-    buf = _workspaces.get(key)
-    if buf is None or buf.numel() < nbytes:
-        if buf is not None:
-            _retired.append(buf)
-        buf = torch.empty(max(int(nbytes), 1 << 20), dtype=torch.uint8, device=device)
-        _workspaces[key] = buf
-    return buf
-
-
-_gemm_workspaces: dict = {}
+    return _lib.host().scratch(_WORKSPACE, _device_index(device), max(int(nbytes), 0))
 
 
 def gemm_workspace(device, nbytes: int):
@@ -70,17 +54,7 @@ def gemm_workspace(device, nbytes: int):
     layer forward)."""
     if nbytes <= 0:
         return None
-    key = _buffer_key(device)
-    buf = _gemm_workspaces.get(key)
-    if buf is None or buf.numel() < nbytes:
-        if buf is not None:
-            _retired.append(buf)
-        buf = torch.empty(int(nbytes), dtype=torch.uint8, device=device)
-        _gemm_workspaces[key] = buf
-    return buf
-
-
-_counters: dict = {}
+    return _lib.host().scratch(_GEMM_WORKSPACE, _device_index(device), int(nbytes))
 
 
 def sync_counters(device, n: int) -> torch.Tensor:
@@ -89,14 +63,7 @@ def sync_counters(device, n: int) -> torch.Tensor:
     created; the kernels leave it zero, so it is reused as is. Its last int is the
     status word the library sets when a split reduction gives up
     (``check_counters`` reads it)."""
-    key = _buffer_key(device)
-    buf = _counters.get(key)
-    if buf is None or buf.numel() < n + 2:
-        if buf is not None:
-            _retired.append(buf)
-        buf = torch.zeros(max(int(n) + 2, 4096), dtype=torch.int32, device=device)
-        _counters[key] = buf
-    return buf
+    return _lib.host().scratch(_COUNTERS, _device_index(device), int(n) + 2)
 
 
 def check_counters(device) -> None:
@@ -105,7 +72,7 @@ def check_counters(device) -> None:
     calls overlapped on it; the affected outputs are NaN) or if the array is not all zero
     as every finished launch leaves it. Either way the array is zeroed again, so the
     next call starts clean. A synchronisation: for tests and debugging, not the hot path."""
-    buf = _counters.get(_buffer_key(device))
+    buf = _lib.host().scratch(_COUNTERS, _device_index(device), -1)
     if buf is None:
         return
     rc = _lib.load().exl3_counters_status(_ptr(buf), buf.numel(), _stream())
@@ -621,7 +588,6 @@ def linear_forward(x2d, trellis, k, cb, suh=None, svh=None, bias=None, group_sub
     _half(x2d, "x")
     if x2d.dim() != 2 or x2d.shape[1] != in_tiles * 16:
         raise ValueError(f"x must be (rows, {in_tiles * 16})")
-    rows = x2d.shape[0]
     n_in, n_out = in_tiles * 16, out_tiles * 16
     if n_in % 128 or n_out % 128:
         raise ValueError("in/out features must be multiples of 128 for the Hadamard transform")
@@ -642,48 +608,8 @@ def linear_forward(x2d, trellis, k, cb, suh=None, svh=None, bias=None, group_sub
             raise ValueError("group_sub must be int32 with out_features/128 entries")
     elif n_sub > 1:
         raise ValueError("group_sub is required with stacked suh")
-    y = torch.empty((rows, n_out), dtype=torch.float16, device=x2d.device)
-    if rows == 0:
-        return y
-    if n_sub > 1 and rows > (linear_small_max_rows() if fused else gemv_max_rows()):
-        if member_out is None or len(member_out) != n_sub or sum(member_out) != n_out:
-            raise ValueError("member_out must list the out_features of the stacked members")
-        xh = had128_pre(x2d, suh)  # (rows, n_sub, in)
-        if all(n % 256 == 0 for n in member_out):
-            # members end on 256-column blocks: one GEMM launch over all of them, each
-            # block reading its member's rotation, then the output transform
-            if block_sub is None:
-                block_sub = group_sub[::2].contiguous()
-            lib = _lib.load()
-            ws_bytes = int(lib.exl3_linear_prefill_workspace_bytes(rows, n_in, n_out))
-            ws = workspace(x2d.device, ws_bytes)
-            rc = lib.exl3_linear_prefill(
-                _ptr(xh), rows, n_sub, _ptr(trellis), in_tiles, out_tiles, int(k), int(cb),
-                _ptr(block_sub), _ptr(svh), _ptr(bias), _ptr(y), _ptr(ws), ws.numel(), _stream())
-            _lib.check(rc, "exl3_linear_prefill")
-            return y
-        tn0 = 0
-        for i, n in enumerate(member_out):
-            if n % 128:
-                raise ValueError("member out_features must be multiples of 128")
-            gemm_into(xh.data_ptr() + 2 * i * n_in, rows, n_sub * n_in, trellis, k, cb, tn0, n // 16,
-                      y.data_ptr() + 2 * 16 * tn0, n_out, x2d.device)
-            tn0 += n // 16
-        return had128_post(y, svh, bias)
-    lib = _lib.load()
-    ws_bytes = int(lib.exl3_linear_workspace_bytes(rows, n_in, n_out, n_sub))
-    ws = workspace(x2d.device, ws_bytes)
-    # one-launch kernel: a 64-bit accumulator per (row, output column) = two ints each;
-    # medium-batch kernel: one counter per 128-column group
-    n_cnt = 2 * rows * n_out if rows <= gemv_max_rows() else n_out // 128
-    cnt = sync_counters(x2d.device, n_cnt) if fused else None
-    rc = lib.exl3_linear_forward(
-        _ptr(x2d), rows, _ptr(trellis), in_tiles, out_tiles, int(k), int(cb), _ptr(suh), n_sub,
-        _ptr(group_sub), _ptr(svh), _ptr(bias), _ptr(y), _ptr(ws), ws.numel(), _ptr(cnt),
-        0 if cnt is None else cnt.numel(), _stream(),
-    )
-    _lib.check(rc, "exl3_linear_forward")
-    return y
+    return _lib.host().Linear(trellis, int(k), int(cb), suh, svh, bias, group_sub, block_sub,
+                              member_out).rows(x2d, bool(fused))
 
 
 def moe_forward(x2d, indices, gu_trellis, gu_suh, gu_svh, dn_trellis, dn_suh, dn_svh, k, cb,
