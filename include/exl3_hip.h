@@ -422,6 +422,40 @@ int exl3_moe_glu_rows(const uint16_t *g, const uint16_t *u, int n_rows, int H, c
                       int activation, uint16_t *xh_dn, void *stream);
 
 /*
+ * The whole prefill chain of EXL3SwitchGLU._prefill (ponyexl3/mlx/exl3_moe.py:684-768): sort
+ * by expert, rotations, segmented GEMMs, GLU, down projection, output transform. Arguments
+ * as exl3_moe_forward; no limit of 4096 pairs, num_experts <= 1024.
+ *   scores  fp16 [tokens][top_k]: y is fp16 [tokens][D], the weighted sum of a token's
+ *           slots (exl3_moe.py:838-839); NULL: y is fp16 [tokens][top_k][D]
+ *   workspace  at least exl3_moe_prefill_workspace_bytes(), 16-byte aligned
+ */
+size_t exl3_moe_prefill_workspace_bytes(int tokens, int top_k, int n_experts, int D, int H);
+int exl3_moe_prefill(const uint16_t *x, int tokens, const int32_t *indices, int top_k,
+                     const uint16_t *gu_trellis, const uint16_t *gu_suh, const uint16_t *gu_svh,
+                     const uint16_t *dn_trellis, const uint16_t *dn_suh, const uint16_t *dn_svh,
+                     int num_experts, int D, int H, int K, int cb, int activation,
+                     const uint16_t *scores, uint16_t *y, void *workspace, size_t workspace_bytes,
+                     void *stream);
+
+/*
+ * exl3_moe_route: the router of EXL3MoEBlock behind its matrix product
+ * (ponyexl3/mlx/exl3_moe.py:817-836): fp32 softmax over n_experts logits, the top_k
+ * largest (ties: lowest expert) in descending order, renormalised to sum 1 if `norm`.
+ *   logits  fp16 or (logits_fp32) fp32 [tokens][n_experts]
+ *   shared_logits  NULL, or [tokens] of the same type: every token also gets expert
+ *           n_experts with weight sigmoid(shared logit), behind its top_k
+ *   indices i32, scores fp16 [tokens][top_k + (shared_logits != NULL)]
+ * n_experts <= 1024 and top_k <= 64 (EXL3_E_UNSUPPORTED above that).
+ * exl3_moe_combine: out[t] = sum_j y[t][j] * scores[t][j] (exl3_moe.py:838-839);
+ *   y fp16 [tokens][slots][D], out fp16 [tokens][D], both 16-byte aligned, D % 8 == 0.
+ */
+int exl3_moe_route(const void *logits, int logits_fp32, const void *shared_logits, int tokens,
+                   int n_experts, int top_k, int norm, int32_t *indices, uint16_t *scores,
+                   void *stream);
+int exl3_moe_combine(const uint16_t *y, const uint16_t *scores, int tokens, int slots, int D,
+                     uint16_t *out, void *stream);
+
+/*
  * Packed tiles -> their 256 sliding-window codewords per tile, kernel order.
  * Replaces unpack_trellis (ponyexl3/ref/trellis.py:153-214); the inverse of
  * exl3_pack_trellis on the low K bits. K in 1..8.

@@ -42,6 +42,12 @@ PROTOTYPES = {
     "exl3_linear_prefill": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "exl3_moe_sort": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),
     "exl3_moe_glu_rows": (_i, [_vp, _vp, _i, _i, _vp, _vp, _vp, _i, _i, _vp, _vp]),
+    "exl3_moe_prefill_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "exl3_moe_prefill": (
+        _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _sz, _vp],
+    ),
+    "exl3_moe_route": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),
+    "exl3_moe_combine": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp]),
     "exl3_quantize_slot_bytes": (_sz, [_i]),
     "exl3_quantize_workspace_bytes": (_sz, [_i, _i]),
     "exl3_quantize_tiles": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _sz, _vp]),

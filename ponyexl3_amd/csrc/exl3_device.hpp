@@ -305,6 +305,37 @@ __device__ __forceinline__ void wht128_lanes(float& a, float& b, int lane) {
     swap_rows16(a, b);
 }
 
+// v[j] = element 8*(lane & 15) + j of the lane group's block, unnormalised WHT in place.
+__device__ __forceinline__ void wht128_wide(float (&v)[8], int lane) {
+#pragma unroll
+    for (int h = 1; h < 8; h <<= 1) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if ((j & h) == 0) {
+                const float lo = v[j], hi = v[j + h];
+                v[j] = __fadd_rn(lo, hi);
+                v[j + h] = __fsub_rn(lo, hi);
+            }
+        }
+    }
+    // lanes 1, 2, 4, 8 apart: DPP operands, no LDS
+    static_for<0, 4>([&](auto bit) {
+        const uint32_t sign = lane_sign_mask(lane, bit.value);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = butterfly_dpp<bit.value>(v[j], sign);
+    });
+}
+
+__device__ __forceinline__ void halfs_to_floats(uint4_t q, float (&v)[8]) {
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const half2_t h = bits_to_half2(w[i]);
+        v[2 * i] = (float)h.x;
+        v[2 * i + 1] = (float)h.y;
+    }
+}
+
 __device__ __forceinline__ float dot2(half2_t a, half2_t b, float c) {
     return __builtin_amdgcn_fdot2(a, b, c, false);
 }

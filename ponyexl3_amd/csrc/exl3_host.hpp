@@ -164,6 +164,10 @@ int launch_had_rows(const uint16_t* x, int n_in_rows, int rows, int n, const int
                     size_t scale_ld, int post, uint16_t* out, int n_out_rows,
                     const int32_t* out_index, hipStream_t stream);
 
+int launch_moe_combine_rows(const uint16_t* y, const int32_t* position, const int32_t* indices,
+                            const uint16_t* svh, const uint16_t* scores, int tokens, int slots,
+                            int n_experts, int D, uint16_t* out, hipStream_t stream);
+
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Integer tuning knob from the environment, clamped to [lo, hi].

@@ -48,37 +48,6 @@ struct RowMap {
     }
 };
 
-// v[j] = element 8*(lane & 15) + j of the lane group's block, unnormalised WHT in place.
-__device__ __forceinline__ void wht128_wide(float (&v)[8], int lane) {
-#pragma unroll
-    for (int h = 1; h < 8; h <<= 1) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if ((j & h) == 0) {
-                const float lo = v[j], hi = v[j + h];
-                v[j] = lo + hi;
-                v[j + h] = lo - hi;
-            }
-        }
-    }
-    // lanes 1, 2, 4, 8 apart: DPP operands, no LDS
-    static_for<0, 4>([&](auto bit) {
-        const uint32_t sign = lane_sign_mask(lane, bit.value);
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = butterfly_dpp<bit.value>(v[j], sign);
-    });
-}
-
-__device__ __forceinline__ void halfs_to_floats(uint4_t q, float (&v)[8]) {
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const half2_t h = bits_to_half2(w[i]);
-        v[2 * i] = (float)h.x;
-        v[2 * i + 1] = (float)h.y;
-    }
-}
-
 // Wide forms: grid.x = number of output rows ((row, sub) pairs for the input side);
 // the four waves of a workgroup take consecutive 512-element chunks of the row,
 // and grid.y workgroups share a row when there are too few rows to fill the chip.

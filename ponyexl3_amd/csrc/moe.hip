@@ -819,12 +819,12 @@ constexpr int kSortMaxExperts = 1024;
 
 // Stable counting sort by expert id. Outputs, all indexed by sorted position:
 //   order[pos] = pair index (token * top_k + slot), tok[pos] = token,
-//   sidx[pos] = expert; table[b] = {expert, first row, end row of the expert, 0}
+//   sidx[pos] = expert; position[pair] = pos unless NULL; table[b] = {expert, first row, end row of the expert, 0}
 // for every block of block_rows rows, unused entries {E-1, N, N, 0} (empty).
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int* __restrict__ indices, int n_pairs, int top_k, int E, int block_rows,
     int* __restrict__ order, int* __restrict__ tok, int* __restrict__ sidx,
-    int4* __restrict__ table, int table_len) {
+    int* __restrict__ position, int4* __restrict__ table, int table_len) {
     __shared__ int count[kSortMaxExperts];  // pairs per expert, later the scatter cursor
     __shared__ unsigned short wave_count[kSortThreads / 64][kSortMaxExperts];  // <= 64 each
     __shared__ int scan_tmp[2][kSortThreads / 64];
@@ -895,6 +895,7 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
             order[pos] = i;
             tok[pos] = i / top_k;
             sidx[pos] = e;
+            if (position) position[i] = pos;
         }
         __syncthreads();
         for (int ee = tid; ee < E; ee += kSortThreads) {
@@ -1119,9 +1120,104 @@ EXL3_EXPORT int exl3_moe_sort(const int32_t* indices, int n_pairs, int top_k, in
     if (n_experts > kSortMaxExperts) return EXL3_E_UNSUPPORTED;
     if (reinterpret_cast<uintptr_t>(table) & 15) return EXL3_E_BAD_SHAPE;
     moe_sort_kernel<<<dim3(1), dim3(kSortThreads), 0, as_stream(stream)>>>(
-        indices, n_pairs, top_k, n_experts, block_rows, order, tok, sidx,
+        indices, n_pairs, top_k, n_experts, block_rows, order, tok, sidx, nullptr,
         reinterpret_cast<int4*>(table), table_len);
     return launch_status();
+}
+
+namespace exl3 {
+
+// Many tokens: the pairs sorted by expert, every expert's rows through the segmented GEMM.
+// Row blocks of the GEMM: the smallest that holds an average expert's rows, so that its
+// weights are decoded once.
+static int moe_prefill_block_rows(long long pairs, int n_experts) {
+    const double per_expert = (double)pairs / n_experts;
+    return per_expert <= 48 ? 64 : per_expert <= 112 ? 128 : 256;
+}
+
+struct MoePrefillWorkspace {
+    size_t o_tables, o_table, o_xg, o_xu, o_g, o_u, o_xd, total;
+    int block_rows, table_len;
+};
+
+static MoePrefillWorkspace moe_prefill_workspace(long long pairs, int E, int D, int H) {
+    MoePrefillWorkspace w{};
+    w.block_rows = moe_prefill_block_rows(pairs, E);
+    w.table_len = (int)(pairs / w.block_rows + E);
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t o = at;
+        at += align_up(bytes, 256);
+        return o;
+    };
+    w.o_tables = take((size_t)pairs * 4 * sizeof(int));  // order, tok, sidx, position
+    w.o_table = take((size_t)w.table_len * sizeof(int4));
+    w.o_xg = take((size_t)pairs * D * 2);  // later the down projection's output
+    w.o_xu = take((size_t)pairs * D * 2);
+    w.o_g = take((size_t)pairs * H * 2);
+    w.o_u = take((size_t)pairs * H * 2);
+    w.o_xd = take((size_t)pairs * H * 2);
+    w.total = at;
+    return w;
+}
+
+}  // namespace exl3
+
+EXL3_EXPORT size_t exl3_moe_prefill_workspace_bytes(int tokens, int top_k, int n_experts, int D, int H) {
+    if (tokens < 1 || top_k < 1 || n_experts < 1 || D < 128 || H < 128 || D % 128 || H % 128) return 0;
+    return exl3::moe_prefill_workspace((long long)tokens * top_k, n_experts, D, H).total;
+}
+
+EXL3_EXPORT int exl3_moe_prefill(const uint16_t* x, int tokens, const int32_t* indices, int top_k,
+                                 const uint16_t* gu_trellis, const uint16_t* gu_suh,
+                                 const uint16_t* gu_svh, const uint16_t* dn_trellis,
+                                 const uint16_t* dn_suh, const uint16_t* dn_svh, int num_experts,
+                                 int D, int H, int K, int cb, int activation,
+                                 const uint16_t* scores, uint16_t* y, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+    using namespace exl3;
+    if (int rc = check_k_cb(K, cb)) return rc;
+    if (!x || !indices || !gu_trellis || !gu_suh || !gu_svh || !dn_trellis || !dn_suh || !dn_svh || !y ||
+        !workspace)
+        return EXL3_E_NULL_POINTER;
+    if (tokens < 1 || top_k < 1 || num_experts < 1 || D < 128 || H < 128 || D % 128 || H % 128 ||
+        (long long)tokens * top_k > (1 << 28))
+        return EXL3_E_BAD_SHAPE;
+    if (activation != 0 && activation != 1) return EXL3_E_UNSUPPORTED;
+    if (num_experts > kSortMaxExperts) return EXL3_E_UNSUPPORTED;
+    const int N = tokens * top_k, E = num_experts;
+    const MoePrefillWorkspace w = moe_prefill_workspace(N, E, D, H);
+    if (workspace_bytes < w.total) return EXL3_E_WORKSPACE;
+    if (reinterpret_cast<uintptr_t>(workspace) & 15) return EXL3_E_BAD_SHAPE;
+    char* base = static_cast<char*>(workspace);
+    int* order = reinterpret_cast<int*>(base + w.o_tables);
+    int *tok = order + N, *sidx = tok + N, *position = sidx + N;
+    int* table = reinterpret_cast<int*>(base + w.o_table);
+    auto buf = [&](size_t o) { return reinterpret_cast<uint16_t*>(base + o); };
+    uint16_t *xg = buf(w.o_xg), *xu = buf(w.o_xu), *g = buf(w.o_g), *u = buf(w.o_u), *xd = buf(w.o_xd);
+    hipStream_t s = as_stream(stream);
+    moe_sort_kernel<<<dim3(1), dim3(kSortThreads), 0, s>>>(indices, N, top_k, E, w.block_rows, order, tok, sidx,
+                                                           position, reinterpret_cast<int4*>(table), w.table_len);
+    if (int rc = launch_status()) return rc;
+    // rotations read x through the token table and the signs through the expert table
+    if (int rc = launch_had_rows(x, tokens, N, D, tok, gu_suh, E, sidx, (size_t)2 * D, 0, xg, N, nullptr, s)) return rc;
+    if (int rc = launch_had_rows(x, tokens, N, D, tok, gu_suh + D, E, sidx, (size_t)2 * D, 0, xu, N, nullptr, s))
+        return rc;
+    const int gt = H / 16, dt = D / 16;
+    if (int rc = launch_gemm_grouped(xg, N, D, gu_trellis, D / 16, E * 2 * gt, K, cb, 0, gt, E, table, w.table_len,
+                                     w.block_rows, g, H, s))
+        return rc;
+    if (int rc = launch_gemm_grouped(xu, N, D, gu_trellis, D / 16, E * 2 * gt, K, cb, E * gt, gt, E, table,
+                                     w.table_len, w.block_rows, u, H, s))
+        return rc;
+    // finish gate and up, GLU, rotate for the down projection: one launch
+    if (int rc = exl3_moe_glu_rows(g, u, N, H, sidx, gu_svh, dn_suh, E, activation, xd, stream)) return rc;
+    if (int rc = launch_gemm_grouped(xd, N, H, dn_trellis, H / 16, E * dt, K, cb, 0, dt, E, table, w.table_len,
+                                     w.block_rows, xg, D, s))
+        return rc;
+    // output transform and either the weighted sum per token or the (token, slot) order
+    if (scores) return launch_moe_combine_rows(xg, position, indices, dn_svh, scores, tokens, top_k, E, D, y, s);
+    return launch_had_rows(xg, N, N, D, nullptr, dn_svh, E, sidx, (size_t)D, 1, y, N, order, s);
 }
 
 EXL3_EXPORT int exl3_moe_glu_rows(const uint16_t* g, const uint16_t* u, int n_rows, int H,

@@ -1,0 +1,266 @@
+// Router and weighted sum around the routed experts: what EXL3MoEBlock does between the
+// router's matrix product and its output (ponyexl3/mlx/exl3_moe.py:817-839).
+//
+// Both are bound by latency at decode sizes: as tensor operations they were twelve launches
+// of 1.5-12 us each (57 us of GPU time and 120 us of host time per decoded token), here they
+// are one launch before the experts and one behind them.
+#include "exl3_device.hpp"
+#include "exl3_host.hpp"
+
+namespace exl3 {
+
+constexpr int kRouteMaxExperts = 1024;  // 16 per lane
+constexpr int kRouteMaxTopK = 64;       // one per lane
+
+template <int CTRL>
+__device__ __forceinline__ int dpp_i32(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+}
+__device__ __forceinline__ void swap16_i32(int& a, int& b) {
+    float x = __builtin_bit_cast(float, a), y = __builtin_bit_cast(float, b);
+    swap_rows16(x, y);
+    a = __builtin_bit_cast(int, x);
+    b = __builtin_bit_cast(int, y);
+}
+__device__ __forceinline__ void swap32_i32(int& a, int& b) {
+    float x = __builtin_bit_cast(float, a), y = __builtin_bit_cast(float, b);
+    swap_halves32(x, y);
+    a = __builtin_bit_cast(int, x);
+    b = __builtin_bit_cast(int, y);
+}
+// op over the wave, the result in every lane: lanes 1, 2, 4, 8 apart through DPP operands
+// (quad permutations, mirrors), 16 and 32 apart by swapping registers
+template <typename Op>
+__device__ __forceinline__ int wave_all(int v, Op op) {
+    v = op(v, dpp_i32<0xB1>(v));
+    v = op(v, dpp_i32<0x4E>(v));
+    v = op(v, dpp_i32<0x141>(v));
+    v = op(v, dpp_i32<0x140>(v));
+    int a = v, b = v;
+    swap16_i32(a, b);
+    v = op(a, b);
+    a = v, b = v;
+    swap32_i32(a, b);
+    return op(a, b);
+}
+__device__ __forceinline__ int wave_max_i32(int v) {
+    return wave_all(v, [](int a, int b) { return a > b ? a : b; });
+}
+__device__ __forceinline__ float wave_max_f32(float v) {
+    return __builtin_bit_cast(float, wave_all(__builtin_bit_cast(int, v), [](int a, int b) {
+                                  return __builtin_bit_cast(int, __builtin_fmaxf(__builtin_bit_cast(float, a),
+                                                                                 __builtin_bit_cast(float, b)));
+                              }));
+}
+__device__ __forceinline__ float wave_sum_f32(float v) {
+    return __builtin_bit_cast(float, wave_all(__builtin_bit_cast(int, v), [](int a, int b) {
+                                  return __builtin_bit_cast(int, __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b));
+                              }));
+}
+
+// One wave per token; lane l holds experts l, l + 64, ..: softmax in fp32, then top_k rounds
+// of "largest probability, lowest expert among equals" (probabilities are non-negative, so
+// their bits order like they do; a taken or absent expert is -1). Lane j keeps choice j.
+// With a shared expert its index n_experts and sigmoid(shared logit) follow the top_k.
+template <typename T, int EPL>
+__global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ logits,
+                                                        const T* __restrict__ shared_logits, int tokens,
+                                                        int n_experts, int top_k, int norm,
+                                                        int* __restrict__ indices, half_t* __restrict__ scores) {
+    const int lane = threadIdx.x & 63;
+    const long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= tokens) return;
+    const T* row = logits + t * n_experts;
+    float v[EPL], m = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < EPL; i++) {
+        v[i] = i * 64 + lane < n_experts ? (float)row[i * 64 + lane] : -__builtin_inff();
+        m = __builtin_fmaxf(m, v[i]);
+    }
+    m = wave_max_f32(m);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < EPL; i++) {
+        v[i] = expf(v[i] - m);  // 0 where there is no expert
+        sum += v[i];
+    }
+    sum = wave_sum_f32(sum);
+    int key[EPL];
+#pragma unroll
+    for (int i = 0; i < EPL; i++)
+        key[i] = i * 64 + lane < n_experts ? __builtin_bit_cast(int, v[i] / sum) & 0x7FFFFFFF : -1;
+    float chosen = 0.f;
+    int chosen_e = 0;
+    for (int j = 0; j < top_k; j++) {
+        int best = key[0];
+#pragma unroll
+        for (int i = 1; i < EPL; i++) best = key[i] > best ? key[i] : best;
+        best = __builtin_amdgcn_readfirstlane(wave_max_i32(best));
+        int e = 0;
+#pragma unroll
+        for (int i = EPL - 1; i >= 0; i--) {
+            const unsigned long long hit = __ballot(key[i] == best);
+            if (hit) e = i * 64 + (int)__builtin_ctzll(hit);
+        }
+#pragma unroll
+        for (int i = 0; i < EPL; i++)
+            if (e == i * 64 + lane) key[i] = -1;
+        if (lane == j) {
+            chosen = __builtin_bit_cast(float, best);
+            chosen_e = e;
+        }
+    }
+    if (norm) chosen = chosen / wave_sum_f32(chosen);
+    const int slots = top_k + (shared_logits != nullptr);
+    if (lane < top_k) {
+        indices[t * slots + lane] = chosen_e;
+        scores[t * slots + lane] = (half_t)chosen;
+    }
+    if (shared_logits && lane == 0) {
+        const float s = (float)shared_logits[t];
+        indices[t * slots + top_k] = n_experts;
+        scores[t * slots + top_k] = (half_t)(float)(T)(1.0f / (1.0f + expf(-s)));
+    }
+}
+
+// out[t][:] = fp16(sum_j y[t][j][:] * scores[t][j]), fp32 products and sum in slot order;
+// eight columns per lane, four slots' rows in flight.
+__global__ __launch_bounds__(256) void moe_combine_kernel(const half_t* __restrict__ y,
+                                                          const half_t* __restrict__ scores, long long n_chunks,
+                                                          int slots, int D, half_t* __restrict__ out) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n_chunks) return;
+    const int chunks = D >> 3;
+    const long long t = i / chunks;
+    const int c = (int)(i % chunks) * 8;
+    const half_t* yt = y + t * slots * D + c;
+    const half_t* st = scores + t * slots;
+    float acc[8] = {};
+    for (int j0 = 0; j0 < slots; j0 += 4) {
+        uint4_t q[4];
+        float s[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int jj = j0 + j < slots ? j0 + j : slots - 1;
+            q[j] = *reinterpret_cast<const uint4_t*>(yt + (size_t)jj * D);
+            s[j] = (float)st[jj];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j0 + j < slots) {
+                float v[8];
+                halfs_to_floats(q[j], v);
+#pragma unroll
+                for (int k = 0; k < 8; k++) acc[k] = __builtin_fmaf(v[k], s[j], acc[k]);
+            }
+        }
+    }
+    half8_t o;
+#pragma unroll
+    for (int k = 0; k < 8; k++) o[k] = (half_t)acc[k];
+    *reinterpret_cast<half8_t*>(out + t * D + c) = o;
+}
+
+// The same sum over rows that the segmented GEMM left sorted by expert and untransformed:
+// row position[t * slots + j] of y belongs to slot j. Applies the output Hadamard and the
+// expert's svh to every row on the way (rounded to fp16 as the per-slot outputs are), so the
+// per-slot outputs are never written. One workgroup per token and 2048 columns.
+__global__ __launch_bounds__(256) void moe_combine_rows_kernel(
+    const half_t* __restrict__ y, const int* __restrict__ position, const int* __restrict__ indices,
+    const half_t* __restrict__ svh, const half_t* __restrict__ scores, int slots, int n_experts, int D,
+    half_t* __restrict__ out) {
+    constexpr float kScale = 0.088388347648318440550f;  // 1/sqrt(128)
+    const int lane = threadIdx.x & 63;
+    const size_t t = blockIdx.x;
+    const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
+    if (c >= D) return;  // whole 16-lane groups: D is a multiple of 128
+    float acc[8] = {};
+    for (int j0 = 0; j0 < slots; j0 += 4) {
+        uint4_t q[4], sq[4];
+        float s[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const size_t at = t * slots + (j0 + j < slots ? j0 + j : slots - 1);
+            int e = indices[at];
+            e = e < 0 ? 0 : (e >= n_experts ? n_experts - 1 : e);
+            q[j] = *reinterpret_cast<const uint4_t*>(y + (size_t)position[at] * D + c);
+            sq[j] = *reinterpret_cast<const uint4_t*>(svh + (size_t)e * D + c);
+            s[j] = (float)scores[at];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j0 + j < slots) {
+                float v[8], sv[8];
+                halfs_to_floats(q[j], v);
+                halfs_to_floats(sq[j], sv);
+                wht128_wide(v, lane);
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const half_t h = (half_t)__fmul_rn(__fmul_rn(v[k], kScale), sv[k]);
+                    acc[k] = __builtin_fmaf((float)h, s[j], acc[k]);
+                }
+            }
+        }
+    }
+    half8_t o;
+#pragma unroll
+    for (int k = 0; k < 8; k++) o[k] = (half_t)acc[k];
+    *reinterpret_cast<half8_t*>(out + t * D + c) = o;
+}
+
+int launch_moe_combine_rows(const uint16_t* y, const int32_t* position, const int32_t* indices,
+                            const uint16_t* svh, const uint16_t* scores, int tokens, int slots,
+                            int n_experts, int D, uint16_t* out, hipStream_t stream) {
+    moe_combine_rows_kernel<<<dim3((unsigned)tokens, (unsigned)((D + 2047) / 2048)), dim3(256), 0, stream>>>(
+        reinterpret_cast<const half_t*>(y), position, indices, reinterpret_cast<const half_t*>(svh),
+        reinterpret_cast<const half_t*>(scores), slots, n_experts, D, reinterpret_cast<half_t*>(out));
+    return launch_status();
+}
+
+template <typename T>
+static int launch_route(const void* logits, const void* shared_logits, int tokens, int n_experts, int top_k,
+                        int norm, int32_t* indices, uint16_t* scores, hipStream_t stream) {
+    auto go = [&](auto epl) {
+        moe_route_kernel<T, epl.value><<<dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, stream>>>(
+            static_cast<const T*>(logits), static_cast<const T*>(shared_logits), tokens, n_experts, top_k, norm,
+            indices, reinterpret_cast<half_t*>(scores));
+        return launch_status();
+    };
+    if (n_experts <= 64) return go(std::integral_constant<int, 1>{});
+    if (n_experts <= 128) return go(std::integral_constant<int, 2>{});
+    if (n_experts <= 256) return go(std::integral_constant<int, 4>{});
+    if (n_experts <= 512) return go(std::integral_constant<int, 8>{});
+    return go(std::integral_constant<int, 16>{});
+}
+
+}  // namespace exl3
+
+EXL3_EXPORT int exl3_moe_route(const void* logits, int logits_fp32, const void* shared_logits, int tokens,
+                               int n_experts, int top_k, int norm, int32_t* indices, uint16_t* scores,
+                               void* stream) {
+    using namespace exl3;
+    if (!logits || !indices || !scores) return EXL3_E_NULL_POINTER;
+    if (tokens < 0 || n_experts < 1 || top_k < 1 || top_k > n_experts) return EXL3_E_BAD_SHAPE;
+    if (n_experts > kRouteMaxExperts || top_k > kRouteMaxTopK) return EXL3_E_UNSUPPORTED;
+    if (tokens == 0) return EXL3_OK;
+    return logits_fp32 ? launch_route<float>(logits, shared_logits, tokens, n_experts, top_k, norm, indices,
+                                             scores, as_stream(stream))
+                       : launch_route<half_t>(logits, shared_logits, tokens, n_experts, top_k, norm, indices,
+                                              scores, as_stream(stream));
+}
+
+EXL3_EXPORT int exl3_moe_combine(const uint16_t* y, const uint16_t* scores, int tokens, int slots, int D,
+                                 uint16_t* out, void* stream) {
+    using namespace exl3;
+    if (!y || !scores || !out) return EXL3_E_NULL_POINTER;
+    if (tokens < 0 || slots < 1 || D < 8 || D % 8) return EXL3_E_BAD_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(y) & 15) || (reinterpret_cast<uintptr_t>(out) & 15)) return EXL3_E_BAD_SHAPE;
+    if (tokens == 0) return EXL3_OK;
+    const long long n = (long long)tokens * (D / 8);
+    const long long grid = (n + 255) / 256;
+    if (grid > 0x7FFFFFFFLL) return EXL3_E_BAD_SHAPE;
+    moe_combine_kernel<<<dim3((unsigned)grid), dim3(256), 0, as_stream(stream)>>>(
+        reinterpret_cast<const half_t*>(y), reinterpret_cast<const half_t*>(scores), n, slots, D,
+        reinterpret_cast<half_t*>(out));
+    return launch_status();
+}

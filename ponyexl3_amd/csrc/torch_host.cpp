@@ -13,8 +13,10 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <string>
 #include <utility>
 #include <vector>
@@ -302,6 +304,170 @@ PyMethodDef linear_methods[] = {{"rows", linear_rows, METH_VARARGS, nullptr}, {n
 
 PyTypeObject linear_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// ---------------------------------------------------------------------------
+// Routed experts of a MoE block (stacked trellises).
+struct ExpertStack {
+    at::Tensor gu_trellis, gu_suh, gu_svh, dn_trellis, dn_suh, dn_svh;
+    int k = 0, cb = 0, activation = 0;
+    int experts() const { return static_cast<int>(gu_suh.size(0)); }
+    int dim() const { return static_cast<int>(gu_suh.size(2)); }
+    int hidden() const { return static_cast<int>(dn_suh.size(1)); }
+};
+
+// x (tokens, D) fp16, indices (tokens, top_k) int32, both contiguous -> y: (tokens, top_k, D),
+// or with scores (fp16, like indices) the weighted sums (tokens, D).
+void experts_run(const ExpertStack& m, const at::Tensor& x, const at::Tensor& indices, const at::Tensor& scores,
+                 bool prefill, const at::Tensor& y) {
+    const int64_t tokens = indices.size(0), top_k = indices.size(1);
+    if (tokens == 0 || top_k == 0) return;
+    if (tokens * top_k > INT32_MAX) value_error("too many (token, slot) pairs");
+    const int E = m.experts(), D = m.dim(), H = m.hidden(), kk = static_cast<int>(top_k);
+    StreamContext ctx(x.device().index());
+    if (prefill) {
+        const int t = static_cast<int>(tokens);
+        const at::Tensor& ws = ctx.get(kWorkspace, exl3_moe_prefill_workspace_bytes(t, kk, E, D, H));
+        check_status(exl3_moe_prefill(half_ptr(x), t, int_ptr(indices), kk, half_ptr(m.gu_trellis), half_ptr(m.gu_suh),
+                                      half_ptr(m.gu_svh), half_ptr(m.dn_trellis), half_ptr(m.dn_suh),
+                                      half_ptr(m.dn_svh), E, D, H, m.k, m.cb, m.activation, half_ptr(scores),
+                                      half_out(y), ws.mutable_data_ptr(), ws.numel(), ctx.stream),
+                     "exl3_moe_prefill");
+        return;
+    }
+    const at::Tensor slots = scores.defined() ? at::empty({tokens, top_k, D}, x.options()) : y;
+    const int64_t chunk = std::max<int64_t>(1, 4096 / top_k);
+    for (int64_t t0 = 0; t0 < tokens; t0 += chunk) {
+        const int t = static_cast<int>(std::min(chunk, tokens - t0));
+        const at::Tensor& ws = ctx.get(kWorkspace, exl3_moe_workspace_bytes(t, kk, D, H));
+        // counter memory for the gate/up reduction through accumulators; the length tells the
+        // library so. Two more ints make the last one the status word.
+        const size_t n_cnt = size_t(t) * kk * (size_t(4) * H + D / 128) + 2;
+        const at::Tensor& cnt = ctx.get(kCounters, n_cnt);
+        check_status(exl3_moe_forward(half_ptr(x) + t0 * D, t, int_ptr(indices) + t0 * top_k, kk,
+                                      half_ptr(m.gu_trellis), half_ptr(m.gu_suh), half_ptr(m.gu_svh),
+                                      half_ptr(m.dn_trellis), half_ptr(m.dn_suh), half_ptr(m.dn_svh), E, D, H, m.k,
+                                      m.cb, m.activation, half_out(slots) + t0 * top_k * D, ws.mutable_data_ptr(),
+                                      ws.numel(), static_cast<int32_t*>(cnt.mutable_data_ptr()), n_cnt, ctx.stream),
+                     "exl3_moe_forward");
+    }
+    if (scores.defined())
+        check_status(exl3_moe_combine(half_ptr(slots), half_ptr(scores), static_cast<int>(tokens), kk, D, half_out(y),
+                                      ctx.stream),
+                     "exl3_moe_combine");
+}
+
+struct PyExperts {
+    PyObject_HEAD
+    ExpertStack* stack;
+};
+
+int experts_init(PyObject* self, PyObject* args, PyObject*) {
+    try {
+        PyObject* t[6];
+        int k, cb, activation;
+        if (!PyArg_ParseTuple(args, "OOOOOOiii", &t[0], &t[1], &t[2], &t[3], &t[4], &t[5], &k, &cb, &activation)) return -1;
+        auto m = std::make_unique<ExpertStack>();
+        at::Tensor* to[6] = {&m->gu_trellis, &m->gu_suh, &m->gu_svh, &m->dn_trellis, &m->dn_suh, &m->dn_svh};
+        for (int i = 0; i < 6; i++) {
+            *to[i] = tensor_or_none(t[i], "expert weights");
+            if (!to[i]->defined() || !to[i]->is_cuda() || !to[i]->is_contiguous())
+                value_error("expert weights must be contiguous tensors on the GPU");
+        }
+        m->k = k;
+        m->cb = cb;
+        m->activation = activation;
+        delete reinterpret_cast<PyExperts*>(self)->stack;
+        reinterpret_cast<PyExperts*>(self)->stack = m.release();
+        return 0;
+    } catch (python_error& e) {
+        e.restore();
+        return -1;
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return -1;
+    }
+}
+
+void experts_dealloc(PyObject* self) {
+    delete reinterpret_cast<PyExperts*>(self)->stack;
+    Py_TYPE(self)->tp_free(self);
+}
+
+// experts.slots(x (B, S, D), indices (B, S, top_k), prefill) -> (B, S, top_k, D)
+PyObject* experts_slots(PyObject* self, PyObject* args) {
+    HANDLE_TH_ERRORS
+    PyObject *x_arg, *idx_arg;
+    int prefill;
+    if (!PyArg_ParseTuple(args, "OOp", &x_arg, &idx_arg, &prefill)) throw python_error();
+    const ExpertStack& m = *reinterpret_cast<PyExperts*>(self)->stack;
+    const at::Tensor x = activations(x_arg, m.dim());
+    c10::OptionalDeviceGuard guard(x.device());
+    if (!THPVariable_Check(idx_arg)) value_error("indices must be a torch.Tensor");
+    at::Tensor idx = THPVariable_Unpack(idx_arg);
+    if (idx.dim() != 3) value_error("indices must be (B, S, top_k)");
+    if (!idx.is_cuda()) value_error("indices must live on the GPU (got device " + idx.device().str() + ")");
+    const int64_t B = idx.size(0), S = idx.size(1), kk = idx.size(2);
+    if (x.numel() != B * S * m.dim()) value_error("x and indices disagree on the number of tokens");
+    if (idx.scalar_type() != at::kInt) idx = idx.to(at::kInt);
+    idx = idx.reshape({B * S, kk}).contiguous();
+    at::Tensor y = at::empty({B, S, kk, m.dim()}, x.options());
+    experts_run(m, x, idx, {}, prefill != 0, y);
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// experts.block(x (..., D), logits, shared_logits or None, top_k, norm, prefill) -> (..., D):
+// routing, experts and weighted sum. None where the native route does not apply (other types,
+// sizes beyond its kernel, logits that carry a gradient).
+PyObject* experts_block(PyObject* self, PyObject* args) {
+    HANDLE_TH_ERRORS
+    PyObject *x_arg, *logits_arg, *shared_arg;
+    int top_k, norm, prefill;
+    if (!PyArg_ParseTuple(args, "OOOipp", &x_arg, &logits_arg, &shared_arg, &top_k, &norm, &prefill))
+        throw python_error();
+    const ExpertStack& m = *reinterpret_cast<PyExperts*>(self)->stack;
+    if (!THPVariable_Check(x_arg) || !THPVariable_Check(logits_arg)) Py_RETURN_NONE;
+    at::Tensor x = THPVariable_Unpack(x_arg);
+    const at::Tensor& logits = THPVariable_Unpack(logits_arg);
+    const at::Tensor shared = tensor_or_none(shared_arg, "shared gate output");
+    const bool has_shared = shared.defined();
+    const int D = m.dim();
+    if (!x.is_cuda() || x.scalar_type() != at::kHalf || x.dim() < 1 || x.size(-1) != D || x.requires_grad() ||
+        !logits.is_cuda() || logits.requires_grad() || logits.dim() < 1 || !logits.is_contiguous() ||
+        (logits.scalar_type() != at::kHalf && logits.scalar_type() != at::kFloat))
+        Py_RETURN_NONE;
+    const int64_t tokens = x.numel() / D, n_experts = logits.size(-1);
+    if (logits.numel() != tokens * n_experts || n_experts + has_shared > m.experts() || n_experts > 1024 ||
+        (has_shared && n_experts != m.experts() - 1) || top_k < 1 || top_k > 64 || top_k > n_experts || tokens == 0 ||
+        (prefill && m.experts() > 1024))
+        Py_RETURN_NONE;
+    if (has_shared && (!shared.is_cuda() || shared.requires_grad() || shared.scalar_type() != logits.scalar_type() ||
+                       shared.numel() != tokens || !shared.is_contiguous()))
+        Py_RETURN_NONE;
+    c10::OptionalDeviceGuard guard(x.device());
+    if (!x.is_contiguous()) x = x.contiguous();
+    const int64_t kk = top_k + has_shared;
+    // indices and scores in one allocation
+    const at::Tensor routing = at::empty({tokens * kk * 6}, x.options().dtype(at::kByte));
+    const at::Tensor idx = routing.narrow(0, 0, tokens * kk * 4).view(at::kInt).view({tokens, kk});
+    const at::Tensor scores = routing.narrow(0, tokens * kk * 4, tokens * kk * 2).view(at::kHalf).view({tokens, kk});
+    StreamContext ctx(x.device().index());
+    check_status(exl3_moe_route(logits.const_data_ptr(), logits.scalar_type() == at::kFloat,
+                                has_shared ? shared.const_data_ptr() : nullptr, static_cast<int>(tokens),
+                                static_cast<int>(n_experts), top_k, norm, static_cast<int32_t*>(idx.mutable_data_ptr()),
+                                half_out(scores), ctx.stream),
+                 "exl3_moe_route");
+    at::Tensor y = at::empty(x.sizes(), x.options());
+    experts_run(m, x, idx, scores, prefill != 0, y);
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef experts_methods[] = {{"slots", experts_slots, METH_VARARGS, nullptr},
+                                 {"block", experts_block, METH_VARARGS, nullptr},
+                                 {nullptr, nullptr, 0, nullptr}};
+
+PyTypeObject experts_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
 PyMethodDef module_methods[] = {{"scratch", py_scratch, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_exl3_host", nullptr, -1, module_methods};
@@ -317,10 +483,19 @@ PyMODINIT_FUNC PyInit__exl3_host() {
     linear_type.tp_dealloc = linear_dealloc;
     linear_type.tp_call = linear_call;
     linear_type.tp_methods = linear_methods;
-    if (PyType_Ready(&linear_type) < 0) return nullptr;
+    experts_type.tp_name = "ponyexl3_amd._exl3_host.Experts";
+    experts_type.tp_basicsize = sizeof(PyExperts);
+    experts_type.tp_flags = Py_TPFLAGS_DEFAULT;
+    experts_type.tp_new = PyType_GenericNew;
+    experts_type.tp_init = experts_init;
+    experts_type.tp_dealloc = experts_dealloc;
+    experts_type.tp_methods = experts_methods;
+    if (PyType_Ready(&linear_type) < 0 || PyType_Ready(&experts_type) < 0) return nullptr;
     PyObject* m = PyModule_Create(&module_def);
     if (!m) return nullptr;
     Py_INCREF(&linear_type);
     if (PyModule_AddObject(m, "Linear", reinterpret_cast<PyObject*>(&linear_type)) < 0) return nullptr;
+    Py_INCREF(&experts_type);
+    if (PyModule_AddObject(m, "Experts", reinterpret_cast<PyObject*>(&experts_type)) < 0) return nullptr;
     return m;
 }

@@ -9,7 +9,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from . import ops
+from . import _lib, ops
 from .layer import EXL3Layer, codebook_mode_from_flags, unpack_signs_or_pass
 
 _MOE_ACTIVATIONS = {"silu": 0, "gelu": 1}
@@ -54,6 +54,18 @@ class EXL3SwitchGLU(torch.nn.Module):
             got = tuple(getattr(self, "_" + name).shape)
             if got != shape:
                 raise ValueError(f"{name} shape {got} != expected {shape}")
+        self._native = None
+
+    def __getstate__(self):
+        # the native handle is made again on the first call of a copy
+        return {**self.__dict__, "_native": None}
+
+    def native(self):
+        if self._native is None:
+            self._native = _lib.host().Experts(
+                self._gu_trellis, self._gu_suh, self._gu_svh, self._dn_trellis, self._dn_suh, self._dn_svh,
+                self._k, self._cb, _MOE_ACTIVATIONS[self._activation])
+        return self._native
 
     @classmethod
     def from_layers(cls, gate: list[EXL3Layer], up: list[EXL3Layer], down: list[EXL3Layer],
@@ -103,45 +115,32 @@ class EXL3SwitchGLU(torch.nn.Module):
         if indices.dim() != 3:
             raise ValueError("indices must be (B, S, top_k)")
         B, S, kk = indices.shape
-        R = B * S
-        D = self.input_dims
-        x2d = x.reshape(R, D).to(torch.float16).contiguous()
-        idx = indices.reshape(R, kk).to(torch.int32).contiguous()
-        if self._use_prefill(R, kk):
-            return self._prefill(x2d, idx).reshape(B, S, kk, D)
-        chunk = max(1, 4096 // kk)
-        outs = []
-        for r0 in range(0, R, chunk):
-            outs.append(
-                ops.moe_forward(
-                    x2d[r0 : r0 + chunk], idx[r0 : r0 + chunk], self._gu_trellis, self._gu_suh,
-                    self._gu_svh, self._dn_trellis, self._dn_suh, self._dn_svh, self._k, self._cb,
-                    _MOE_ACTIVATIONS[self._activation],
-                )
-            )
-        y = outs[0] if len(outs) == 1 else torch.cat(outs, dim=0)
-        return y.reshape(B, S, kk, D)
+        prefill = self._use_prefill(B * S, kk)
+        if prefill and self.num_experts > ops.MOE_SORT_MAX_EXPERTS:
+            x2d = x.reshape(B * S, self.input_dims).to(torch.float16).contiguous()
+            idx = indices.reshape(B * S, kk).to(torch.int32).contiguous()
+            return self._prefill_many_experts(x2d, idx).reshape(B, S, kk, self.input_dims)
+        return self.native().slots(x, indices, prefill)
 
-    def _prefill(self, x2d: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
+    def _prefill_many_experts(self, x2d: torch.Tensor, idx: torch.Tensor) -> torch.Tensor:
         """Many tokens: sort the (token, slot) pairs by expert so that every expert's
         weights are decoded once per block of its rows, rotate with per-row sign
         vectors, run the segmented MFMA GEMM, finish per row, unsort
         (``EXL3SwitchGLU._prefill``, ponyexl3/mlx/exl3_moe.py:684-768). No host
-        synchronisation: the block table is built on the device for the worst case."""
+        synchronisation: the block table is built on the device for the worst case.
+        ``exl3_moe_prefill`` runs this chain natively; this form, with the sort as torch
+        operations, is for more experts than its sort kernel takes."""
         E, D, H = self.num_experts, self.input_dims, self.hidden_dims
         R, kk = idx.shape
         N = R * kk
         per_expert = N / E
         block_rows = 64 if per_expert <= 48 else 128 if per_expert <= 112 else 256
-        if E <= ops.MOE_SORT_MAX_EXPERTS:
-            order32, tok32, sidx32, table = ops.moe_sort(idx, E, block_rows)  # one launch
-        else:
-            flat = idx.reshape(-1).long().clamp_(0, E - 1)
-            order = torch.argsort(flat, stable=True)
-            sidx = flat[order]
-            table = ops.segment_table(sidx, E, block_rows)
-            sidx32, order32 = sidx.int(), order.int()
-            tok32 = torch.div(order, kk, rounding_mode="floor").int()
+        flat = idx.reshape(-1).long().clamp_(0, E - 1)
+        order = torch.argsort(flat, stable=True)
+        sidx = flat[order]
+        table = ops.segment_table(sidx, E, block_rows)
+        sidx32, order32 = sidx.int(), order.int()
+        tok32 = torch.div(order, kk, rounding_mode="floor").int()
         k, cb = self._k, self._cb
         gt, dt = H // 16, D // 16
         # rotations read x through the token table and the signs through the expert table
@@ -191,10 +190,14 @@ class EXL3MoEBlock(torch.nn.Module):
         self._shared_idx = switch.num_experts - 1
 
     def route(self, x: torch.Tensor):
-        inds, scores = route_topk(self.gate(x), self.top_k, self.norm_topk_prob)
+        shared = None if self.shared_expert_gate is None else self.shared_expert_gate(x)
+        return self._select(x, self.gate(x), shared)
+
+    def _select(self, x, logits, shared_logits):
+        inds, scores = route_topk(logits, self.top_k, self.norm_topk_prob)
         scores = scores.to(x.dtype)
-        if self.shared_expert_gate is not None:
-            shared_w = torch.sigmoid(self.shared_expert_gate(x)).to(x.dtype)
+        if shared_logits is not None:
+            shared_w = torch.sigmoid(shared_logits).to(x.dtype)
             shared = torch.full(inds.shape[:-1] + (1,), self._shared_idx, dtype=inds.dtype,
                                 device=inds.device)
             inds = torch.cat([inds, shared], dim=-1)
@@ -204,6 +207,18 @@ class EXL3MoEBlock(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         lead = tuple(x.shape[:-1])
         x3 = x.reshape(1, -1, x.shape[-1])
-        inds, scores = self.route(x3)
-        y = self.switch_mlp(x3, inds)
+        switch = self.switch_mlp
+        if (type(self) is EXL3MoEBlock and type(switch) is EXL3SwitchGLU
+                and not (switch._forward_hooks or switch._forward_pre_hooks)):
+            # the gates are the caller's modules; routing, experts and sum are one native call
+            logits = self.gate(x3)
+            shared = None if self.shared_expert_gate is None else self.shared_expert_gate(x3)
+            prefill = switch._use_prefill(x3.shape[1], self.top_k + (shared is not None))
+            y = switch.native().block(x, logits, shared, self.top_k, self.norm_topk_prob, prefill)
+            if y is not None:
+                return y
+            inds, scores = self._select(x3, logits, shared)
+        else:
+            inds, scores = self.route(x3)
+        y = switch(x3, inds)
         return combine_experts(y, scores).reshape(lead + (x.shape[-1],))

@@ -443,3 +443,58 @@ def test_glu_rows_kernel_equals_separate_launches(cuda, act):
     assert float(diff) <= 4e-3 * float(ref.float().abs().max())
     with pytest.raises(ValueError):
         ops.moe_glu_rows(g, u[:, :256], sidx, gu_svh, dn_suh, act)
+
+
+@pytest.mark.parametrize("tokens,E,top_k,norm,fp32", [(1, 1, 1, True, False), (5, 63, 8, True, False),
+                                                      (3, 64, 64, False, True), (130, 65, 4, True, True),
+                                                      (7, 257, 6, False, False), (4, 1024, 16, True, False)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_route_kernel_against_torch(cuda, tokens, E, top_k, norm, fp32, shared):
+    """Softmax, top-k (ties: lowest expert first) and weights against torch in float64,
+    on coarse logits so that ties do occur, also at the k-th place."""
+    from ponyexl3_amd import _lib, ops
+
+    g = torch.Generator().manual_seed(E + top_k)
+    logits = (torch.randn((tokens, E), generator=g) * 4).round() / 4
+    sl = torch.randn((tokens, 1), generator=g)
+    dt = torch.float32 if fp32 else torch.float16
+    ld, sd = logits.to(dt).to(cuda), sl.to(dt).to(cuda)
+    slots = top_k + shared
+    idx = torch.full((tokens, slots), -1, dtype=torch.int32, device=cuda)
+    scores = torch.zeros((tokens, slots), dtype=torch.float16, device=cuda)
+    print(f"route tokens={tokens} E={E} k={top_k}", flush=True)
+    rc = _lib.load().exl3_moe_route(ops._ptr(ld), int(fp32), ops._ptr(sd) if shared else None, tokens, E, top_k,
+                                    int(norm), ops._ptr(idx), ops._ptr(scores), ops._stream())
+    _lib.check(rc, "exl3_moe_route")
+    order = torch.argsort(-logits, dim=-1, stable=True)[:, :top_k]
+    w = torch.gather(torch.softmax(logits.double(), dim=-1), 1, order)
+    if norm:
+        w = w / w.sum(dim=-1, keepdim=True)
+    assert torch.equal(idx[:, :top_k].cpu().long(), order)
+    torch.testing.assert_close(scores[:, :top_k].cpu().double(), w, rtol=1e-3, atol=1e-6)
+    if shared:
+        assert (idx[:, top_k] == E).all()
+        torch.testing.assert_close(scores[:, top_k].cpu().double(), torch.sigmoid(sd.cpu().double())[:, 0],
+                                   rtol=1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("tokens,shared", [(1, False), (9, True), (30, True), (67, False)])
+def test_moe_block_native_chain_equals_its_parts(cuda, tokens, shared):
+    """Slot kernels, slot kernels with shared passes and the sorted prefill chain with the
+    weighted sum in its last kernel: the block against route, experts and sum one by one."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+    from ponyexl3_amd.moe import combine_experts
+
+    E, D, H, kk = 9, 384, 128, 3
+    gate, up, down = _experts(E, D, H, 4, True, 4200)
+    switch = EXL3SwitchGLU.from_layers(gate, up, down)
+    g = torch.Generator().manual_seed(tokens)
+    lin = lambda n: torch.nn.Linear(D, n, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin(E - shared), lin(1) if shared else None, switch, kk)
+    x = (torch.randn((1, tokens, D), generator=g) * 0.2).half().to(cuda)
+    print(f"moe block tokens={tokens}", flush=True)
+    y = block(x)
+    inds, scores = block.route(x)
+    ref = combine_experts(switch(x, inds).float(), scores)
+    assert y.shape == x.shape and y.dtype == torch.float16
+    assert rel_l2(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
