@@ -438,6 +438,16 @@ int exl3_moe_prefill(const uint16_t *x, int tokens, const int32_t *indices, int 
                      void *stream);
 
 /*
+ * Router logits for a few tokens, fp16(x . w^T) with fp32 sums, the router's matrix product
+ * (ponyexl3/mlx/exl3_moe.py:817): x fp16 [tokens][D], w fp16 [n_experts][D], D % 32 == 0,
+ * logits fp16 [tokens][n_experts]; w_shared (or NULL) fp16 [D], the shared expert's gate,
+ * gives shared_logits fp16 [tokens]. x, w and w_shared 16-byte aligned.
+ */
+int exl3_moe_gate(const uint16_t *x, int tokens, int D, const uint16_t *w, int n_experts,
+                  const uint16_t *w_shared, uint16_t *logits, uint16_t *shared_logits,
+                  void *stream);
+
+/*
  * exl3_moe_route: the router of EXL3MoEBlock behind its matrix product
  * (ponyexl3/mlx/exl3_moe.py:817-836): fp32 softmax over n_experts logits, the top_k
  * largest (ties: lowest expert) in descending order, renormalised to sum 1 if `norm`.

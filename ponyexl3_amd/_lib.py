@@ -46,6 +46,7 @@ PROTOTYPES = {
     "exl3_moe_prefill": (
         _i, [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _sz, _vp],
     ),
+    "exl3_moe_gate": (_i, [_vp, _i, _i, _vp, _i, _vp, _vp, _vp, _vp]),
     "exl3_moe_route": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),
     "exl3_moe_combine": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp]),
     "exl3_quantize_slot_bytes": (_sz, [_i]),

@@ -8,8 +8,10 @@
 // Everything runs under the GIL.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <ATen/ATen.h>
+#include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -415,42 +417,119 @@ PyObject* experts_slots(PyObject* self, PyObject* args) {
     END_HANDLE_TH_ERRORS
 }
 
-// experts.block(x (..., D), logits, shared_logits or None, top_k, norm, prefill) -> (..., D):
-// routing, experts and weighted sum. None where the native route does not apply (other types,
-// sizes beyond its kernel, logits that carry a gradient).
+// Up to this many tokens the router's product runs in exl3_moe_gate, above it in the gate
+// module: its kernel is made for one round trip to memory, not for throughput.
+constexpr int64_t kGateMaxTokens = 32;
+
+// The weight of a plain bias-free fp16 torch.nn.Linear without hooks, as exl3_moe_gate
+// takes it; undefined if `gate` is anything else.
+at::Tensor plain_gate_weight(PyObject* gate, PyObject* linear_class, int D) {
+    if (reinterpret_cast<PyObject*>(Py_TYPE(gate)) != linear_class) return {};
+    PyObject** dict = _PyObject_GetDictPtr(gate);
+    if (!dict || !*dict) return {};
+    auto item = [&](const char* name) { return PyDict_GetItemString(*dict, name); };
+    for (const char* hooks : {"_forward_hooks", "_forward_pre_hooks"}) {
+        PyObject* h = item(hooks);
+        if (!h || PyObject_Size(h) != 0) return {};
+    }
+    if (item("forward")) return {};  // replaced on the instance
+    PyObject* params = item("_parameters");
+    if (!params || !PyDict_Check(params)) return {};
+    PyObject* bias = PyDict_GetItemString(params, "bias");
+    PyObject* weight = PyDict_GetItemString(params, "weight");
+    if ((bias && bias != Py_None) || !weight || !THPVariable_Check(weight)) return {};
+    const at::Tensor& w = THPVariable_Unpack(weight);
+    if (!w.is_cuda() || w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != D || !w.is_contiguous() ||
+        (reinterpret_cast<uintptr_t>(w.const_data_ptr()) & 15))
+        return {};
+    return w;
+}
+
+PyObject* linear_module_class() {
+    static PyObject* cls = [] {
+        PyObject* nn = PyImport_ImportModule("torch.nn");
+        PyObject* c = nn ? PyObject_GetAttrString(nn, "Linear") : nullptr;
+        Py_XDECREF(nn);
+        return c;
+    }();
+    if (!cls) throw python_error();
+    return cls;
+}
+
+// experts.block(x (..., D), gate, shared gate or None, top_k, norm, prefill) -> (..., D): the
+// router (the gates are modules of the caller's; called, or if they are plain Linears and
+// there are few tokens, computed here), experts and weighted sum. Where the native route does
+// not apply (other types, sizes beyond its kernels, values that carry a gradient) it returns
+// (logits, shared logits or None) if the gates have been called, None if not.
 PyObject* experts_block(PyObject* self, PyObject* args) {
     HANDLE_TH_ERRORS
-    PyObject *x_arg, *logits_arg, *shared_arg;
+    PyObject *x_arg, *gate, *shared_gate;
     int top_k, norm, prefill;
-    if (!PyArg_ParseTuple(args, "OOOipp", &x_arg, &logits_arg, &shared_arg, &top_k, &norm, &prefill))
-        throw python_error();
+    if (!PyArg_ParseTuple(args, "OOOipp", &x_arg, &gate, &shared_gate, &top_k, &norm, &prefill)) throw python_error();
     const ExpertStack& m = *reinterpret_cast<PyExperts*>(self)->stack;
-    if (!THPVariable_Check(x_arg) || !THPVariable_Check(logits_arg)) Py_RETURN_NONE;
+    if (!THPVariable_Check(x_arg)) Py_RETURN_NONE;
     at::Tensor x = THPVariable_Unpack(x_arg);
-    const at::Tensor& logits = THPVariable_Unpack(logits_arg);
-    const at::Tensor shared = tensor_or_none(shared_arg, "shared gate output");
-    const bool has_shared = shared.defined();
+    const bool has_shared = shared_gate != Py_None;
     const int D = m.dim();
     if (!x.is_cuda() || x.scalar_type() != at::kHalf || x.dim() < 1 || x.size(-1) != D || x.requires_grad() ||
-        !logits.is_cuda() || logits.requires_grad() || logits.dim() < 1 || !logits.is_contiguous() ||
-        (logits.scalar_type() != at::kHalf && logits.scalar_type() != at::kFloat))
+        x.numel() == 0 || top_k < 1 || top_k > 64 || (prefill && m.experts() > 1024))
         Py_RETURN_NONE;
-    const int64_t tokens = x.numel() / D, n_experts = logits.size(-1);
-    if (logits.numel() != tokens * n_experts || n_experts + has_shared > m.experts() || n_experts > 1024 ||
-        (has_shared && n_experts != m.experts() - 1) || top_k < 1 || top_k > 64 || top_k > n_experts || tokens == 0 ||
-        (prefill && m.experts() > 1024))
-        Py_RETURN_NONE;
-    if (has_shared && (!shared.is_cuda() || shared.requires_grad() || shared.scalar_type() != logits.scalar_type() ||
-                       shared.numel() != tokens || !shared.is_contiguous()))
-        Py_RETURN_NONE;
+    const int64_t tokens = x.numel() / D;
     c10::OptionalDeviceGuard guard(x.device());
     if (!x.is_contiguous()) x = x.contiguous();
+    StreamContext ctx(x.device().index());
+
+    at::Tensor logits, shared;
+    const bool grad = at::GradMode::is_enabled();
+    if (tokens <= kGateMaxTokens) {
+        const at::Tensor w = plain_gate_weight(gate, linear_module_class(), D);
+        const at::Tensor ws = has_shared ? plain_gate_weight(shared_gate, linear_module_class(), D) : at::Tensor();
+        if (w.defined() && !(grad && w.requires_grad()) &&
+            (!has_shared || (ws.defined() && ws.size(0) == 1 && !(grad && ws.requires_grad())))) {
+            const int64_t E = w.size(0);
+            const at::Tensor out = at::empty({tokens * (E + has_shared)}, x.options());
+            logits = out.narrow(0, 0, tokens * E).view({tokens, E});
+            if (has_shared) shared = out.narrow(0, tokens * E, tokens);
+            check_status(exl3_moe_gate(half_ptr(x), static_cast<int>(tokens), D, half_ptr(w), static_cast<int>(E),
+                                       half_ptr(ws), half_out(logits), has_shared ? half_out(shared) : nullptr,
+                                       ctx.stream),
+                         "exl3_moe_gate");
+        }
+    }
+    if (!logits.defined()) {
+        THPObjectPtr x3(THPVariable_Wrap(x.view({1, tokens, D})));
+        THPObjectPtr l(PyObject_CallFunctionObjArgs(gate, x3.get(), nullptr));
+        if (!l) throw python_error();
+        THPObjectPtr s;
+        if (has_shared) {
+            s = THPObjectPtr(PyObject_CallFunctionObjArgs(shared_gate, x3.get(), nullptr));
+            if (!s) throw python_error();
+        }
+        auto usable = [&](PyObject* o, int64_t numel_per_token) {
+            if (!THPVariable_Check(o)) return false;
+            const at::Tensor& t = THPVariable_Unpack(o);
+            return t.is_cuda() && !t.requires_grad() && t.dim() >= 1 && t.is_contiguous() &&
+                   (t.scalar_type() == at::kHalf || t.scalar_type() == at::kFloat) &&
+                   t.numel() == tokens * (numel_per_token ? numel_per_token : t.size(-1));
+        };
+        const bool ok = usable(l.get(), 0) && (!has_shared || (usable(s.get(), 1) && THPVariable_Unpack(s.get()).scalar_type() ==
+                                                                             THPVariable_Unpack(l.get()).scalar_type()));
+        if (!ok) return PyTuple_Pack(2, l.get(), has_shared ? s.get() : Py_None);
+        logits = THPVariable_Unpack(l.get());
+        if (has_shared) shared = THPVariable_Unpack(s.get());
+    }
+    const int64_t n_experts = logits.size(-1);
+    if (n_experts + has_shared > m.experts() || n_experts > 1024 || (has_shared && n_experts != m.experts() - 1) ||
+        top_k > n_experts) {
+        THPObjectPtr l(THPVariable_Wrap(logits.view({1, tokens, n_experts})));
+        THPObjectPtr s(has_shared ? THPVariable_Wrap(shared.view({1, tokens, 1})) : Py_NewRef(Py_None));
+        return PyTuple_Pack(2, l.get(), s.get());
+    }
     const int64_t kk = top_k + has_shared;
     // indices and scores in one allocation
     const at::Tensor routing = at::empty({tokens * kk * 6}, x.options().dtype(at::kByte));
     const at::Tensor idx = routing.narrow(0, 0, tokens * kk * 4).view(at::kInt).view({tokens, kk});
     const at::Tensor scores = routing.narrow(0, tokens * kk * 4, tokens * kk * 2).view(at::kHalf).view({tokens, kk});
-    StreamContext ctx(x.device().index());
     check_status(exl3_moe_route(logits.const_data_ptr(), logits.scalar_type() == at::kFloat,
                                 has_shared ? shared.const_data_ptr() : nullptr, static_cast<int>(tokens),
                                 static_cast<int>(n_experts), top_k, norm, static_cast<int32_t*>(idx.mutable_data_ptr()),

@@ -205,20 +205,21 @@ class EXL3MoEBlock(torch.nn.Module):
         return inds, scores
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = tuple(x.shape[:-1])
-        x3 = x.reshape(1, -1, x.shape[-1])
-        switch = self.switch_mlp
+        modules = self._modules  # plain dictionary: nn.Module's attribute lookup is slow
+        gate, switch = modules.get("gate") or self.gate, modules["switch_mlp"]
+        shared_gate = modules.get("shared_expert_gate")
+        got = None
         if (type(self) is EXL3MoEBlock and type(switch) is EXL3SwitchGLU
                 and not (switch._forward_hooks or switch._forward_pre_hooks)):
-            # the gates are the caller's modules; routing, experts and sum are one native call
-            logits = self.gate(x3)
-            shared = None if self.shared_expert_gate is None else self.shared_expert_gate(x3)
-            prefill = switch._use_prefill(x3.shape[1], self.top_k + (shared is not None))
-            y = switch.native().block(x, logits, shared, self.top_k, self.norm_topk_prob, prefill)
-            if y is not None:
-                return y
-            inds, scores = self._select(x3, logits, shared)
-        else:
-            inds, scores = self.route(x3)
+            # routing, experts and weighted sum in one native call
+            dim = x.shape[-1]
+            prefill = dim > 0 and switch._use_prefill(x.numel() // dim, self.top_k + (shared_gate is not None))
+            got = switch.native().block(x, gate, shared_gate, self.top_k, self.norm_topk_prob, prefill)
+            if isinstance(got, torch.Tensor):
+                return got
+        lead = tuple(x.shape[:-1])
+        x3 = x.reshape(1, -1, x.shape[-1])
+        # (the gates may have been called already)
+        inds, scores = self.route(x3) if got is None else self._select(x3, *got)
         y = switch(x3, inds)
         return combine_experts(y, scores).reshape(lead + (x.shape[-1],))

@@ -498,3 +498,27 @@ def test_moe_block_native_chain_equals_its_parts(cuda, tokens, shared):
     ref = combine_experts(switch(x, inds).float(), scores)
     assert y.shape == x.shape and y.dtype == torch.float16
     assert rel_l2(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
+
+
+@pytest.mark.parametrize("tokens,E,D", [(1, 1, 128), (1, 256, 2048), (3, 15, 384), (16, 16, 1152), (17, 257, 640),
+                                        (32, 33, 2176)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_gate_kernel_against_float64(cuda, tokens, E, D, shared):
+    """Router logits and the shared gate's: fp16 roundings of the exact products, up to
+    the fp32 sums."""
+    from ponyexl3_amd import _lib, ops
+
+    g = torch.Generator().manual_seed(D + E)
+    x = torch.randn((tokens, D), generator=g).half()
+    w = (torch.randn((E + 1, D), generator=g) / D ** 0.5).half()
+    xd, wd = x.to(cuda), w.to(cuda)
+    logits = torch.full((tokens, E), float("nan"), dtype=torch.float16, device=cuda)
+    sl = torch.full((tokens,), float("nan"), dtype=torch.float16, device=cuda)
+    print(f"gate tokens={tokens} E={E} D={D}", flush=True)
+    rc = _lib.load().exl3_moe_gate(ops._ptr(xd), tokens, D, ops._ptr(wd), E, ops._ptr(wd[E]) if shared else None,
+                                   ops._ptr(logits), ops._ptr(sl) if shared else None, ops._stream())
+    _lib.check(rc, "exl3_moe_gate")
+    ref = x.double() @ w.double().T
+    torch.testing.assert_close(logits.cpu().double(), ref[:, :E], rtol=6e-4, atol=1e-5)
+    if shared:
+        torch.testing.assert_close(sl.cpu().double(), ref[:, E], rtol=6e-4, atol=1e-5)
