@@ -111,6 +111,14 @@ int exl3_had128_pre(const uint16_t *x, int rows, int n, const uint16_t *suh, int
                     uint16_t *xh, void *stream);
 
 /*
+ * The same rotation as the layer forwards run it: from nine rows on the Hadamard products
+ * are on the matrix pipe (exact products, fp32 sums in another order, so single results can
+ * round differently from exl3_had128_pre's).
+ */
+int exl3_rotate(const uint16_t *x, int rows, int n, const uint16_t *suh, int n_sub, uint16_t *xh,
+                void *stream);
+
+/*
  * Hadamard-128 with one scale vector per row (rows routed to different experts),
  * with the row gathers and the final scatter of the sorted MoE prefill folded in:
  *   post == 0: out[o(r)] = fp16(had128(x[i(r)] * scale[s(r)]))  (_rows_prep,

@@ -58,6 +58,7 @@ PROTOTYPES = {
     "exl3_decode_full_t": (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp]),
     "exl3_public_weight": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i, _i, _i, _vp, _vp]),
     "exl3_had128_pre": (_i, [_vp, _i, _i, _vp, _i, _vp, _vp]),
+    "exl3_rotate": (_i, [_vp, _i, _i, _vp, _i, _vp, _vp]),
     "exl3_had128_post": (_i, [_vp, _i, _i, _sz, _i, _i, _vp, _vp, _vp, _vp]),
     "exl3_gemv": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp, _sz, _vp]),
     "exl3_gemv_workspace_bytes": (_sz, [_i, _i, _i]),

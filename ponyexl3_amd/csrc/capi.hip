@@ -113,7 +113,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
     }
 
     // Prefill: rotation kernel, MFMA GEMM, output transform.
-    if (int rc = launch_had_pre(x, rows, in_features, suh, n_sub, xh, s)) return rc;
+    if (int rc = launch_rotate_layer(x, rows, in_features, suh, n_sub, xh, s)) return rc;
     if (counters && rows <= linear_mid_max_rows()) {
         // a few dozen rows: the decode still sets the pace; every weight is decoded
         // once and goes from registers into 16x16x32 MFMA; split reduction and output

@@ -305,6 +305,30 @@ __device__ __forceinline__ void wht128_lanes(float& a, float& b, int lane) {
     swap_rows16(a, b);
 }
 
+// Direct load global -> LDS: lane l's 16 bytes at base + offset go to LDS byte lds + 16 l (lds
+// uniform). As inline assembly because the compiler's builtin marks the load as one that may
+// complete out of order with others, after which every wait it inserts for a register load
+// is for ALL memory operations; here it only sees its own loads and waits for those (too
+// strictly by the direct loads in between, never too weakly). The caller waits for the data
+// with s_waitcnt vmcnt. (m0 is reserved: the compiler sets it right where it needs it.)
+__device__ __forceinline__ void load_lds16(const void* base, uint32_t offset, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
+                 : "memory");
+}
+__device__ __forceinline__ uint32_t lds_byte_address(const void* p) {
+    return (uint32_t)(uintptr_t)(const void __attribute__((address_space(3)))*)p;
+}
+
+// Workgroup barrier behind which this wave's LDS accesses are complete and all but its last
+// VM vector memory operations; __syncthreads() waits for every one of those, prefetches
+// included.
+template <int VM>
+__device__ __forceinline__ void barrier_with_loads_in_flight() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VM) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // v[j] = element 8*(lane & 15) + j of the lane group's block, unnormalised WHT in place.
 __device__ __forceinline__ void wht128_wide(float (&v)[8], int lane) {
 #pragma unroll

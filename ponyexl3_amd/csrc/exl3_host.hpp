@@ -164,9 +164,19 @@ int launch_had_rows(const uint16_t* x, int n_in_rows, int rows, int n, const int
                     size_t scale_ld, int post, uint16_t* out, int n_out_rows,
                     const int32_t* out_index, hipStream_t stream);
 
-int launch_moe_combine_rows(const uint16_t* y, const int32_t* position, const int32_t* indices,
-                            const uint16_t* svh, const uint16_t* scores, int tokens, int slots,
-                            int n_experts, int D, uint16_t* out, hipStream_t stream);
+int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub, uint16_t* xh,
+                        hipStream_t stream);
+int launch_had_pre_pairs(const uint16_t* x, int tokens, int rows, int n, const int32_t* tok,
+                         const uint16_t* gu_suh, int n_experts, const int32_t* expert, uint16_t* xg,
+                         size_t sub_stride, hipStream_t stream);
+
+// Experts of rows sorted by expert (row-block table as exl3_moe_sort's, blocks of 32 or 64):
+// gate, up, GLU and rotation to xd [n_rows][H], down to out[order[r]] [..][D].
+int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const uint16_t* gu_trellis,
+                    const uint16_t* gu_svh, const uint16_t* dn_trellis, const uint16_t* dn_suh,
+                    const uint16_t* dn_svh, int E, int D, int H, int K, int cb, int activation,
+                    const int32_t* table, int n_blocks, int block_rows, const int32_t* order,
+                    uint16_t* xd, uint16_t* out, hipStream_t stream);
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 

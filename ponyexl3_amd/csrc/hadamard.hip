@@ -16,6 +16,7 @@
 // caller-visible casts of ponyexl3/ref/forward.py:34,41,42,45.
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
+#include "exl3_rows.hpp"
 
 #pragma clang fp contract(off)
 
@@ -107,6 +108,117 @@ __global__ __launch_bounds__(256) void had_pre_wide_kernel(const half_t* __restr
             }
         }
     }
+}
+
+// Input side on the matrix pipe: a wave rotates 16 rows x one 128-wide block, for
+// subs_per_wave of the stacked siblings from one read of x. The products x * suh have 22
+// significant bits; they enter the matrix instructions exactly as a high and a low fp16
+// part (the low parts of plain signs are all zero and then skipped) against entries +-1, with
+// fp32 sums, so the result is the fp32 butterfly's up to the order of the additions. 32 (or
+// 64) matrix instructions of 16 cycles and about 3 VALU instructions per element replace
+// about 18: the butterfly form was bound by VALU issue (23 us for 2048 x 5120 to two siblings,
+// 31 MB read and 42 MB written with the signs).
+// Row maps (MoE rows sorted by expert): source row in_index[r], scale row scale_index[r] of
+// scale_ld halfs; indices outside the buffers skip the row.
+// out + s * sub_stride + r * row_stride
+struct RotateArgs {
+    const half_t* x;
+    const half_t* suh;
+    half_t* out;
+    int rows, n, n_sub, subs_per_wave;
+    size_t sub_scale, sub_stride, row_stride;  // halfs from one sibling's scales / results to the next
+    const int32_t* in_index;
+    const int32_t* scale_index;
+    size_t scale_ld;
+    unsigned n_in, n_scale;
+};
+
+__global__ __launch_bounds__(256) void had_pre_mfma_kernel(RotateArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int fr = lane & 15, q = lane >> 4;
+    const int blocks = a.n >> 7;
+    const long long wid = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int row_tiles = (a.rows + 15) >> 4;
+    if (wid >= (long long)row_tiles * blocks) return;
+    // consecutive waves take consecutive blocks of the same rows
+    const int blk = (int)(wid % blocks), r = (int)(wid / blocks) * 16 + fr;
+    bool valid = r < a.rows;
+    unsigned src = valid ? (unsigned)r : 0u, scale_row = 0;
+    if (a.in_index) {
+        src = (unsigned)a.in_index[src];
+        valid = valid && src < a.n_in;
+    }
+    if (a.scale_index) {
+        scale_row = (unsigned)a.scale_index[valid ? r : 0];
+        valid = valid && scale_row < a.n_scale;
+    }
+    if (!valid) src = 0, scale_row = 0;
+    const size_t col = (size_t)blk * 128 + q * 8;
+    const half_t* xr = a.x + (size_t)src * a.n + col;
+    half8_t xv[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) xv[k] = *reinterpret_cast<const half8_t*>(xr + k * 32);
+    const HadamardColumns had(lane);
+    const int s_begin = blockIdx.y * a.subs_per_wave, s_end = min(s_begin + a.subs_per_wave, a.n_sub);
+    for (int s = s_begin; s < s_end; s++) {
+        half8_t hi[4], lo[4];
+        uint32_t low_bits = 0;
+        if (a.suh) {
+            const half_t* sr = a.suh + (size_t)scale_row * a.scale_ld + (size_t)s * a.sub_scale + col;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const half8_t sv = *reinterpret_cast<const half8_t*>(sr + k * 32);
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    half_t h, l;
+                    split_halves(__fmul_rn((float)xv[k][j], (float)sv[j]), h, l);
+                    hi[k][j] = h;
+                    lo[k][j] = l;
+                }
+                low_bits |= any_bits(lo[k]);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) hi[k] = xv[k];
+        }
+        float4_t z[8];
+#pragma unroll
+        for (int nt = 0; nt < 8; nt++) z[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
+        static_for<0, 4>([&](auto k) {
+            static_for<0, 8>([&](auto nt) {
+                z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(), hi[k.value],
+                                                                     z[nt.value], 0, 0, 0);
+            });
+        });
+        if (__ballot(low_bits != 0)) {
+            static_for<0, 4>([&](auto k) {
+                static_for<0, 8>([&](auto nt) {
+                    z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(),
+                                                                         lo[k.value], z[nt.value], 0, 0, 0);
+                });
+            });
+        }
+        if (valid) {
+            half_t* o = a.out + (size_t)s * a.sub_stride + (size_t)r * a.row_stride + col;
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                half8_t v;
+#pragma unroll
+                for (int c = 0; c < 8; c++) v[c] = (half_t)(z[2 * p + (c >> 2)][c & 3] * kHadScale);
+                *reinterpret_cast<half8_t*>(o + p * 32) = v;
+            }
+        }
+    }
+}
+
+static int launch_rotate(RotateArgs a, hipStream_t stream) {
+    const long long waves = (long long)((a.rows + 15) / 16) * (a.n / 128);
+    // few rows: the siblings in parallel; else one read of x for all of them
+    a.subs_per_wave = waves * a.n_sub <= 4096 ? 1 : a.n_sub;
+    const long long grid = (waves + 3) / 4, gy = (a.n_sub + a.subs_per_wave - 1) / a.subs_per_wave;
+    if (grid > 0x7FFFFFFFLL || gy > 65535) return EXL3_E_BAD_SHAPE;
+    had_pre_mfma_kernel<<<dim3((unsigned)grid, (unsigned)gy), dim3(256), 0, stream>>>(a);
+    return launch_status();
 }
 
 __global__ __launch_bounds__(256) void had_post_wide_kernel(const half_t* __restrict__ y,
@@ -344,6 +456,47 @@ int launch_had_rows(const uint16_t* x, int n_in_rows, int rows, int n, const int
     return launch_status();
 }
 
+// The rotation as the layer forwards use it: on the matrix pipe from nine rows on.
+int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub, uint16_t* xh,
+                        hipStream_t stream) {
+    if (rows < 9 || n < 128 || n % 128 || n_sub < 1 || (!suh && n_sub != 1) || !x || !xh || !aligned16(x) ||
+        !aligned16(xh) || (suh && !aligned16(suh)))
+        return launch_had_pre(x, rows, n, suh, n_sub, xh, stream);
+    RotateArgs a{};
+    a.x = reinterpret_cast<const half_t*>(x);
+    a.suh = reinterpret_cast<const half_t*>(suh);
+    a.out = reinterpret_cast<half_t*>(xh);
+    a.rows = rows;
+    a.n = n;
+    a.n_sub = n_sub;
+    a.sub_scale = a.sub_stride = (size_t)n;
+    a.row_stride = (size_t)n_sub * n;
+    return launch_rotate(a, stream);
+}
+
+// Rows sorted by expert: both rotations (gate and up signs of the row's expert, gu_suh
+// [E][2][n]) of token row tok[r], to xg[r] and, sub_stride halfs further, xu[r].
+int launch_had_pre_pairs(const uint16_t* x, int tokens, int rows, int n, const int32_t* tok, const uint16_t* gu_suh,
+                         int n_experts, const int32_t* expert, uint16_t* xg, size_t sub_stride, hipStream_t stream) {
+    if (!aligned16(x) || !aligned16(gu_suh) || !aligned16(xg) || sub_stride % 8) return EXL3_E_BAD_SHAPE;
+    RotateArgs a{};
+    a.x = reinterpret_cast<const half_t*>(x);
+    a.suh = reinterpret_cast<const half_t*>(gu_suh);
+    a.out = reinterpret_cast<half_t*>(xg);
+    a.rows = rows;
+    a.n = n;
+    a.n_sub = 2;
+    a.sub_scale = (size_t)n;
+    a.sub_stride = sub_stride;
+    a.row_stride = (size_t)n;
+    a.in_index = tok;
+    a.scale_index = expert;
+    a.scale_ld = (size_t)2 * n;
+    a.n_in = (unsigned)tokens;
+    a.n_scale = (unsigned)n_experts;
+    return launch_rotate(a, stream);
+}
+
 }  // namespace exl3
 
 EXL3_EXPORT int exl3_had128_rows(const uint16_t* x, int n_in_rows, int rows, int n,
@@ -359,6 +512,11 @@ EXL3_EXPORT int exl3_had128_rows(const uint16_t* x, int n_in_rows, int rows, int
 EXL3_EXPORT int exl3_had128_pre(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub,
                                 uint16_t* xh, void* stream) {
     return exl3::launch_had_pre(x, rows, n, suh, n_sub, xh, exl3::as_stream(stream));
+}
+
+EXL3_EXPORT int exl3_rotate(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub, uint16_t* xh,
+                            void* stream) {
+    return exl3::launch_rotate_layer(x, rows, n, suh, n_sub, xh, exl3::as_stream(stream));
 }
 
 EXL3_EXPORT int exl3_had128_post(const void* y, int y_is_fp32, int n_sum, size_t sum_stride,

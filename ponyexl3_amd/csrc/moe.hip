@@ -31,6 +31,7 @@
 // (ponyexl3/mlx/exl3_moe.py:345-422) are what this replaces.
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
+#include "exl3_glu.hpp"
 #include "exl3_small.hpp"
 
 #include <algorithm>
@@ -82,14 +83,6 @@ __global__ __launch_bounds__(256) void moe_prep_kernel(
     o.x = (half_t)(a * kHadScaleF);
     o.y = (half_t)(b * kHadScaleF);
     *reinterpret_cast<half2_t*>(xh_gu + (size_t)sp * D + blk * 128 + 2 * lane) = o;
-}
-
-__device__ __forceinline__ float glu_act(float g, float u, int activation) {
-    if (activation == 1) {
-        const float t = 0.797884560803f * (g + 0.044715f * g * g * g);
-        return 0.5f * g * (1.0f + tanhf(t)) * u;
-    }
-    return (g / (1.0f + expf(-g))) * u;
 }
 
 // One wave per (slot, 128-block of H): finishes gate and up, applies the GLU and
@@ -819,25 +812,36 @@ constexpr int kSortMaxExperts = 1024;
 
 // Stable counting sort by expert id. Outputs, all indexed by sorted position:
 //   order[pos] = pair index (token * top_k + slot), tok[pos] = token,
-//   sidx[pos] = expert; position[pair] = pos unless NULL; table[b] = {expert, first row, end row of the expert, 0}
+//   sidx[pos] = expert; table[b] = {expert, first row, end row of the expert, 0}
 // for every block of block_rows rows, unused entries {E-1, N, N, 0} (empty).
+//
+// Each of the 16 waves owns one contiguous segment of the pairs and a cursor per expert in
+// LDS: count, one scan over (expert, wave), then every wave places its segment 64 pairs at a
+// time without meeting the others. A pair's rank among equal experts of its 64 comes from
+// ballots over the bits of the expert id. Latency-bound: 13 833 pairs over 257 experts take
+// 11 us; walking the pairs 1024 at a time with counts exchanged across the waves took 41.
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int* __restrict__ indices, int n_pairs, int top_k, int E, int block_rows,
     int* __restrict__ order, int* __restrict__ tok, int* __restrict__ sidx,
-    int* __restrict__ position, int4* __restrict__ table, int table_len) {
-    __shared__ int count[kSortMaxExperts];  // pairs per expert, later the scatter cursor
-    __shared__ unsigned short wave_count[kSortThreads / 64][kSortMaxExperts];  // <= 64 each
-    __shared__ int scan_tmp[2][kSortThreads / 64];
+    int4* __restrict__ table, int table_len) {
+    constexpr int kWaves = kSortThreads / 64;
+    extern __shared__ int cursor[];  // [kWaves][E]
+    __shared__ int scan_tmp[2][kWaves];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < E; e += kSortThreads) count[e] = 0;
-    for (int i = tid; i < (kSortThreads / 64) * kSortMaxExperts; i += kSortThreads)
-        (&wave_count[0][0])[i] = 0;
+    for (int i = tid; i < kWaves * E; i += kSortThreads) cursor[i] = 0;
     __syncthreads();
-    for (int i = tid; i < n_pairs; i += kSortThreads) atomicAdd(&count[clamp_expert(indices[i], E)], 1);
+    const int per_wave = (n_pairs + 64 * kWaves - 1) / (64 * kWaves) * 64;
+    const int begin = wave * per_wave, end = min(begin + per_wave, n_pairs);
+    int* mine = cursor + wave * E;
+    for (int i = begin + lane; i < end; i += 64) atomicAdd(&mine[clamp_expert(indices[i], E)], 1);
     __syncthreads();
 
     // exclusive scans over the experts (E <= 1024 = one value per thread): rows and blocks
-    const int c = tid < E ? count[tid] : 0;
+    int c = 0;
+    if (tid < E) {
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) c += cursor[w * E + tid];
+    }
     const int nb = (c + block_rows - 1) / block_rows;
     int inc_rows = c, inc_blk = nb;
 #pragma unroll
@@ -854,7 +858,8 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     }
     __syncthreads();
     int base_rows = 0, base_blk = 0, total_blk = 0;
-    for (int w = 0; w < kSortThreads / 64; w++) {
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
         if (w < wave) {
             base_rows += scan_tmp[0][w];
             base_blk += scan_tmp[1][w];
@@ -863,9 +868,14 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     }
     const int row0 = base_rows + inc_rows - c;  // first sorted row of expert tid
     const int blk0 = base_blk + inc_blk - nb;
-    __syncthreads();
     if (tid < E) {
-        count[tid] = row0;  // scatter cursor
+        int at = row0;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const int n = cursor[w * E + tid];
+            cursor[w * E + tid] = at;
+            at += n;
+        }
         for (int b = 0; b < nb && blk0 + b < table_len; b++)
             table[blk0 + b] = int4{tid, row0 + b * block_rows, row0 + c, 0};
     }
@@ -873,41 +883,28 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
         table[b] = int4{E - 1, n_pairs, n_pairs, 0};
     __syncthreads();
 
-    // stable scatter, 1024 pairs at a time in pair order: rank inside the wave by
-    // matching expert ids bit by bit, then across the waves of the chunk
     int ebits = 0;
     while ((1 << ebits) < E) ebits++;
-    for (int i0 = 0; i0 < n_pairs; i0 += kSortThreads) {
-        const int i = i0 + tid;
-        const bool valid = i < n_pairs;
-        const int e = valid ? clamp_expert(indices[i], E) : 0;
+    int next = begin + lane < end ? indices[begin + lane] : 0;
+    for (int i0 = begin; i0 < end; i0 += 64) {
+        const int i = i0 + lane;
+        const bool valid = i < end;
+        const int e = valid ? clamp_expert(next, E) : 0;
+        if (i + 64 < end) next = indices[i + 64];
         unsigned long long same = __ballot(valid);
         for (int b = 0; b < ebits; b++) {
-            const unsigned long long m = __ballot(valid && ((e >> b) & 1));
+            const unsigned long long m = __ballot((e >> b) & 1);
             same &= ((e >> b) & 1) ? m : ~m;
         }
         const int rank = __popcll(same & ((1ull << lane) - 1ull));
-        if (valid && rank == 0) wave_count[wave][e] = (unsigned short)__popcll(same);
-        __syncthreads();
         if (valid) {
-            int pos = count[e] + rank;
-            for (int w = 0; w < wave; w++) pos += wave_count[w][e];
+            const int first = mine[e];
+            if (rank == 0) mine[e] = first + __popcll(same);  // behind the reads: LDS is in order
+            const int pos = first + rank;
             order[pos] = i;
             tok[pos] = i / top_k;
             sidx[pos] = e;
-            if (position) position[i] = pos;
         }
-        __syncthreads();
-        for (int ee = tid; ee < E; ee += kSortThreads) {
-            int add = 0;
-#pragma unroll
-            for (int w = 0; w < kSortThreads / 64; w++) {
-                add += wave_count[w][ee];
-                wave_count[w][ee] = 0;
-            }
-            count[ee] += add;
-        }
-        __syncthreads();
     }
 }
 
@@ -947,6 +944,19 @@ __global__ __launch_bounds__(256) void moe_glu_rows_kernel(
     o.x = (half_t)(a * kHadScaleF);
     o.y = (half_t)(b * kHadScaleF);
     *reinterpret_cast<half2_t*>(xh_dn + off) = o;
+}
+
+static int launch_moe_sort(const int32_t* indices, int n_pairs, int top_k, int n_experts, int block_rows,
+                           int32_t* order, int32_t* tok, int32_t* sidx, int32_t* table, int table_len,
+                           hipStream_t stream) {
+    const size_t lds = (size_t)(kSortThreads / 64) * n_experts * sizeof(int);
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_sort_kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return EXL3_E_LAUNCH;
+    moe_sort_kernel<<<dim3(1), dim3(kSortThreads), lds, stream>>>(indices, n_pairs, top_k, n_experts, block_rows,
+                                                                  order, tok, sidx, reinterpret_cast<int4*>(table),
+                                                                  table_len);
+    return launch_status();
 }
 
 }  // namespace exl3
@@ -1119,24 +1129,18 @@ EXL3_EXPORT int exl3_moe_sort(const int32_t* indices, int n_pairs, int top_k, in
         return EXL3_E_BAD_SHAPE;
     if (n_experts > kSortMaxExperts) return EXL3_E_UNSUPPORTED;
     if (reinterpret_cast<uintptr_t>(table) & 15) return EXL3_E_BAD_SHAPE;
-    moe_sort_kernel<<<dim3(1), dim3(kSortThreads), 0, as_stream(stream)>>>(
-        indices, n_pairs, top_k, n_experts, block_rows, order, tok, sidx, nullptr,
-        reinterpret_cast<int4*>(table), table_len);
-    return launch_status();
+    return launch_moe_sort(indices, n_pairs, top_k, n_experts, block_rows, order, tok, sidx, table, table_len,
+                           as_stream(stream));
 }
 
 namespace exl3 {
 
-// Many tokens: the pairs sorted by expert, every expert's rows through the segmented GEMM.
-// Row blocks of the GEMM: the smallest that holds an average expert's rows, so that its
-// weights are decoded once.
-static int moe_prefill_block_rows(long long pairs, int n_experts) {
-    const double per_expert = (double)pairs / n_experts;
-    return per_expert <= 48 ? 64 : per_expert <= 112 ? 128 : 256;
-}
+// Row blocks of the prefill kernels: 32 rows where an average expert's rows fit with room to
+// spare (half the matrix work and registers), else 64, decoded again for every further 64.
+static int moe_prefill_block_rows(long long pairs, int n_experts) { return pairs <= 24ll * n_experts ? 32 : 64; }
 
 struct MoePrefillWorkspace {
-    size_t o_tables, o_table, o_xg, o_xu, o_g, o_u, o_xd, total;
+    size_t o_tables, o_table, o_xg, o_xu, o_xd, total;
     int block_rows, table_len;
 };
 
@@ -1150,12 +1154,10 @@ static MoePrefillWorkspace moe_prefill_workspace(long long pairs, int E, int D, 
         at += align_up(bytes, 256);
         return o;
     };
-    w.o_tables = take((size_t)pairs * 4 * sizeof(int));  // order, tok, sidx, position
+    w.o_tables = take((size_t)pairs * 3 * sizeof(int));  // order, tok, sidx
     w.o_table = take((size_t)w.table_len * sizeof(int4));
-    w.o_xg = take((size_t)pairs * D * 2);  // later the down projection's output
+    w.o_xg = take((size_t)pairs * D * 2);  // later the slots' outputs
     w.o_xu = take((size_t)pairs * D * 2);
-    w.o_g = take((size_t)pairs * H * 2);
-    w.o_u = take((size_t)pairs * H * 2);
     w.o_xd = take((size_t)pairs * H * 2);
     w.total = at;
     return w;
@@ -1188,36 +1190,25 @@ EXL3_EXPORT int exl3_moe_prefill(const uint16_t* x, int tokens, const int32_t* i
     const int N = tokens * top_k, E = num_experts;
     const MoePrefillWorkspace w = moe_prefill_workspace(N, E, D, H);
     if (workspace_bytes < w.total) return EXL3_E_WORKSPACE;
-    if (reinterpret_cast<uintptr_t>(workspace) & 15) return EXL3_E_BAD_SHAPE;
+    for (const void* p : {(const void*)workspace, (const void*)y, (const void*)gu_svh, (const void*)dn_suh,
+                          (const void*)dn_svh, (const void*)x, (const void*)gu_suh})
+        if (reinterpret_cast<uintptr_t>(p) & 15) return EXL3_E_BAD_SHAPE;
     char* base = static_cast<char*>(workspace);
     int* order = reinterpret_cast<int*>(base + w.o_tables);
-    int *tok = order + N, *sidx = tok + N, *position = sidx + N;
+    int *tok = order + N, *sidx = tok + N;
     int* table = reinterpret_cast<int*>(base + w.o_table);
-    auto buf = [&](size_t o) { return reinterpret_cast<uint16_t*>(base + o); };
-    uint16_t *xg = buf(w.o_xg), *xu = buf(w.o_xu), *g = buf(w.o_g), *u = buf(w.o_u), *xd = buf(w.o_xd);
+    uint16_t* xg = reinterpret_cast<uint16_t*>(base + w.o_xg);
+    uint16_t* xd = reinterpret_cast<uint16_t*>(base + w.o_xd);
+    const size_t xu_offset = (w.o_xu - w.o_xg) / 2;
     hipStream_t s = as_stream(stream);
-    moe_sort_kernel<<<dim3(1), dim3(kSortThreads), 0, s>>>(indices, N, top_k, E, w.block_rows, order, tok, sidx,
-                                                           position, reinterpret_cast<int4*>(table), w.table_len);
-    if (int rc = launch_status()) return rc;
-    // rotations read x through the token table and the signs through the expert table
-    if (int rc = launch_had_rows(x, tokens, N, D, tok, gu_suh, E, sidx, (size_t)2 * D, 0, xg, N, nullptr, s)) return rc;
-    if (int rc = launch_had_rows(x, tokens, N, D, tok, gu_suh + D, E, sidx, (size_t)2 * D, 0, xu, N, nullptr, s))
+    if (int rc = launch_moe_sort(indices, N, top_k, E, w.block_rows, order, tok, sidx, table, w.table_len, s)) return rc;
+    if (int rc = launch_had_pre_pairs(x, tokens, N, D, tok, gu_suh, E, sidx, xg, xu_offset, s)) return rc;
+    // gate, up, GLU and rotation, then down with its output transform, back in pair order
+    uint16_t* slots = scores ? xg : y;
+    if (int rc = launch_moe_rows(xg, xg + xu_offset, N, gu_trellis, gu_svh, dn_trellis, dn_suh, dn_svh, E, D, H, K, cb,
+                                 activation, table, w.table_len, w.block_rows, order, xd, slots, s))
         return rc;
-    const int gt = H / 16, dt = D / 16;
-    if (int rc = launch_gemm_grouped(xg, N, D, gu_trellis, D / 16, E * 2 * gt, K, cb, 0, gt, E, table, w.table_len,
-                                     w.block_rows, g, H, s))
-        return rc;
-    if (int rc = launch_gemm_grouped(xu, N, D, gu_trellis, D / 16, E * 2 * gt, K, cb, E * gt, gt, E, table,
-                                     w.table_len, w.block_rows, u, H, s))
-        return rc;
-    // finish gate and up, GLU, rotate for the down projection: one launch
-    if (int rc = exl3_moe_glu_rows(g, u, N, H, sidx, gu_svh, dn_suh, E, activation, xd, stream)) return rc;
-    if (int rc = launch_gemm_grouped(xd, N, H, dn_trellis, H / 16, E * dt, K, cb, 0, dt, E, table, w.table_len,
-                                     w.block_rows, xg, D, s))
-        return rc;
-    // output transform and either the weighted sum per token or the (token, slot) order
-    if (scores) return launch_moe_combine_rows(xg, position, indices, dn_svh, scores, tokens, top_k, E, D, y, s);
-    return launch_had_rows(xg, N, N, D, nullptr, dn_svh, E, sidx, (size_t)D, 1, y, N, order, s);
+    return scores ? exl3_moe_combine(slots, scores, tokens, top_k, D, y, stream) : EXL3_OK;
 }
 
 EXL3_EXPORT int exl3_moe_glu_rows(const uint16_t* g, const uint16_t* u, int n_rows, int H,

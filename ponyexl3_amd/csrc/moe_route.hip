@@ -210,62 +210,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const half_t* __restri
     *reinterpret_cast<half8_t*>(out + t * D + c) = o;
 }
 
-// The same sum over rows that the segmented GEMM left sorted by expert and untransformed:
-// row position[t * slots + j] of y belongs to slot j. Applies the output Hadamard and the
-// expert's svh to every row on the way (rounded to fp16 as the per-slot outputs are), so the
-// per-slot outputs are never written. One workgroup per token and 2048 columns.
-__global__ __launch_bounds__(256) void moe_combine_rows_kernel(
-    const half_t* __restrict__ y, const int* __restrict__ position, const int* __restrict__ indices,
-    const half_t* __restrict__ svh, const half_t* __restrict__ scores, int slots, int n_experts, int D,
-    half_t* __restrict__ out) {
-    constexpr float kScale = 0.088388347648318440550f;  // 1/sqrt(128)
-    const int lane = threadIdx.x & 63;
-    const size_t t = blockIdx.x;
-    const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
-    if (c >= D) return;  // whole 16-lane groups: D is a multiple of 128
-    float acc[8] = {};
-    for (int j0 = 0; j0 < slots; j0 += 4) {
-        uint4_t q[4], sq[4];
-        float s[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const size_t at = t * slots + (j0 + j < slots ? j0 + j : slots - 1);
-            int e = indices[at];
-            e = e < 0 ? 0 : (e >= n_experts ? n_experts - 1 : e);
-            q[j] = *reinterpret_cast<const uint4_t*>(y + (size_t)position[at] * D + c);
-            sq[j] = *reinterpret_cast<const uint4_t*>(svh + (size_t)e * D + c);
-            s[j] = (float)scores[at];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (j0 + j < slots) {
-                float v[8], sv[8];
-                halfs_to_floats(q[j], v);
-                halfs_to_floats(sq[j], sv);
-                wht128_wide(v, lane);
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    const half_t h = (half_t)__fmul_rn(__fmul_rn(v[k], kScale), sv[k]);
-                    acc[k] = __builtin_fmaf((float)h, s[j], acc[k]);
-                }
-            }
-        }
-    }
-    half8_t o;
-#pragma unroll
-    for (int k = 0; k < 8; k++) o[k] = (half_t)acc[k];
-    *reinterpret_cast<half8_t*>(out + t * D + c) = o;
-}
-
-int launch_moe_combine_rows(const uint16_t* y, const int32_t* position, const int32_t* indices,
-                            const uint16_t* svh, const uint16_t* scores, int tokens, int slots,
-                            int n_experts, int D, uint16_t* out, hipStream_t stream) {
-    moe_combine_rows_kernel<<<dim3((unsigned)tokens, (unsigned)((D + 2047) / 2048)), dim3(256), 0, stream>>>(
-        reinterpret_cast<const half_t*>(y), position, indices, reinterpret_cast<const half_t*>(svh),
-        reinterpret_cast<const half_t*>(scores), slots, n_experts, D, reinterpret_cast<half_t*>(out));
-    return launch_status();
-}
-
 template <typename T>
 static int launch_route(const void* logits, const void* shared_logits, int tokens, int n_experts, int top_k,
                         int norm, int32_t* indices, uint16_t* scores, hipStream_t stream) {

@@ -1,0 +1,327 @@
+// Routed experts of a prefill chunk: the (token, slot) rows are sorted by expert, a
+// workgroup takes up to 64 rows of one expert through 128 columns of gate AND up or 256
+// columns of down (see exl3_rows.hpp for the contraction).
+//
+// moe_gateup_rows_kernel ends with everything that stands between the two products: output
+// transform of gate and up (ponyexl3/ref/forward.py:41-42), GLU, rotation for the down
+// projection - a Hadamard block of H is exactly one 128-column group - so gate and up never
+// reach memory. moe_down_rows_kernel applies its output transform and stores rows at their
+// (token, slot) place.
+#include "exl3_device.hpp"
+#include "exl3_host.hpp"
+#include "exl3_rows.hpp"
+#include "exl3_glu.hpp"
+
+#pragma clang fp contract(off)
+
+namespace exl3 {
+
+constexpr int kRowsThreads = 512;
+constexpr int kYPad = 8;  // halfs: 16-byte reads of 16 tile rows hit all banks
+
+// Sums of two k-slices: the wave of slice ks keeps columns cs = ks. `ex` holds MR*4 float4 per
+// lane and wave; every wave passes its other half to its partner (wave ^ 1).
+template <int MR>
+__device__ __forceinline__ void rows_add_slices2(float16_t (&acc)[MR][2], float4_t* ex, int wave, int lane,
+                                                 float16_t (&sum)[MR]) {
+    const bool second = wave & 1;
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float4_t v;
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = second ? acc[mr][0][4 * i + c] : acc[mr][1][4 * i + c];
+            ex[((wave ^ 1) * MR * 4 + mr * 4 + i) * 64 + lane] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4_t v = ex[(wave * MR * 4 + mr * 4 + i) * 64 + lane];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                sum[mr][4 * i + c] = __fadd_rn(second ? acc[mr][1][4 * i + c] : acc[mr][0][4 * i + c], v[c]);
+        }
+    __syncthreads();
+}
+
+// The fp16 casts of the sums to an LDS tile [BM][ld], first column `col` of the wave's strip.
+template <int MR>
+__device__ __forceinline__ void rows_store_half(const float16_t (&sum)[MR], half_t* tile, int ld, int col, int cs,
+                                                int lane) {
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            half4_t o;
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] = (half_t)sum[mr][4 * i + c];
+            *reinterpret_cast<half4_t*>(tile + (mr * 32 + (lane & 31)) * ld + col + 16 * i + 8 * cs +
+                                        4 * (lane >> 5)) = o;
+        }
+}
+
+// grid: unit = (row block b, 128-column block hg of H), dealt so that the units of a row block
+// land on one XCD (they read the same activations): b = 8 (u / (8 hblocks)) + u % 8.
+// table[b] = {expert, first row, end row of the expert, 0}, empty if first >= end.
+template <int K, int CB, int MR>
+__global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
+    const uint32_t* __restrict__ trellis, const half_t* __restrict__ xg, const half_t* __restrict__ xu,
+    const int4* __restrict__ table, int n_blocks, const half_t* __restrict__ gu_svh,
+    const half_t* __restrict__ dn_suh, half_t* __restrict__ xd, int n_rows, int E, int D, int H, int activation) {
+    using T = RowsTile<MR, 2>;
+    constexpr int kFillWaves = 4, LPW = T::FILLS / kFillWaves;
+    constexpr int kLd = 128 + kYPad;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int hblocks = H >> 7;
+    const int set = blockIdx.x / (8 * hblocks), in_set = blockIdx.x % (8 * hblocks);
+    const int b = set * 8 + (in_set & 7), hg = in_set >> 3;
+    if (b >= n_blocks) return;
+    const int4 blk = table[b];
+    const int e = blk.x, m0 = blk.y, end = min(blk.z, n_rows);
+    if (e < 0 || e >= E || m0 < 0 || m0 >= end) return;
+    const int valid = min(end - m0, T::BM);
+
+    const int proj = wave >> 2, cq = (wave >> 1) & 1, ks = wave & 1;
+    const size_t row_words = (size_t)E * 2 * (H >> 4) * (8 * K);
+    const uint32_t* w = trellis + (size_t)(2 * ks + (lane >> 5)) * row_words +
+                        ((size_t)(proj * E + e) * (H >> 4) + hg * 8 + cq * 4 + ((lane >> 3) & 3)) * (8 * K) +
+                        (lane & 7) * K;
+    half_t* stages = reinterpret_cast<half_t*>(lds) + proj * 3 * T::STAGE;
+    uint32_t a_off[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, 2>((wave & 3) * LPW + i, lane, valid - 1, D);
+    float16_t acc[MR][2];
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int cs = 0; cs < 2; cs++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
+    rows_main<K, CB, MR, 2, LPW>(w, 4 * row_words, reinterpret_cast<const char*>((proj ? xu : xg) + (size_t)m0 * D),
+                                 a_off, true, lds_byte_address(stages) + (wave & 3) * LPW * 1024,
+                                 stages, rows_read_base<MR, 2>(ks, lane), D >> 6, lane, acc);
+
+    float16_t sum[MR];
+    rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
+    half_t* tile = reinterpret_cast<half_t*>(lds);  // [gate | up][BM][kLd]
+    rows_store_half<MR>(sum, tile + proj * T::BM * kLd, kLd, cq * 64, ks, lane);
+    __syncthreads();
+
+    // Output transform, GLU and rotation: a wave takes a 16-row tile and MR of the four
+    // 32-column parts of the block.
+    const int rt = wave % (2 * MR), part = wave / (2 * MR);
+    const int fr = lane & 15, q = lane >> 4;
+    const HadamardColumns had(lane);
+    const half_t* yrow = tile + (rt * 16 + fr) * kLd + q * 8;
+    auto transform = [&](const half8_t (&y)[4], auto a_const, float (&z)[8]) {
+        float4_t t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        constexpr int a = decltype(a_const)::value;
+        static_for<0, 4>([&](auto k) {
+            t[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<2 * a, k.value>(), y[k.value], t[0], 0, 0, 0);
+            t[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<2 * a + 1, k.value>(), y[k.value], t[1], 0, 0, 0);
+        });
+#pragma unroll
+        for (int c = 0; c < 8; c++) z[c] = t[c >> 2][c & 3];
+    };
+    // f(a) for the wave's parts a, which are compile-time values in each branch
+    auto for_parts = [&](auto f) {
+        static_for<0, 4 / MR>([&](auto p) {
+            if (part == p.value)
+                static_for<0, MR>([&](auto i) { f(std::integral_constant<int, p.value * MR + i.value>{}, i); });
+        });
+    };
+    half8_t hi[MR], lo[MR];
+    {
+        half8_t yg[4], yu[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            yg[k] = *reinterpret_cast<const half8_t*>(yrow + k * 32);
+            yu[k] = *reinterpret_cast<const half8_t*>(yrow + T::BM * kLd + k * 32);
+        }
+        for_parts([&](auto a, auto i) {
+            const int col = hg * 128 + a.value * 32 + q * 8;
+            const half8_t sg = *reinterpret_cast<const half8_t*>(gu_svh + (size_t)e * 2 * H + col);
+            const half8_t su = *reinterpret_cast<const half8_t*>(gu_svh + (size_t)e * 2 * H + H + col);
+            const half8_t ds = *reinterpret_cast<const half8_t*>(dn_suh + (size_t)e * H + col);
+            float zg[8], zu[8], h[8];
+            transform(yg, a, zg);
+            transform(yu, a, zu);
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                zg[c] = (float)(half_t)(zg[c] * kHadNorm * (float)sg[c]);
+                zu[c] = (float)(half_t)(zu[c] * kHadNorm * (float)su[c]);
+            }
+            if (activation == 1) {
+#pragma unroll
+                for (int c = 0; c < 8; c++) h[c] = glu_act(zg[c], zu[c], 1);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 8; c++) h[c] = glu_act(zg[c], zu[c], 0);
+            }
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                half_t h0, h1;
+                split_halves((float)(half_t)h[c] * (float)ds[c], h0, h1);
+                hi[i.value][c] = h0;
+                lo[i.value][c] = h1;
+            }
+        });
+    }
+    __syncthreads();
+    for_parts([&](auto a, auto i) {
+        half_t* dst = tile + (rt * 16 + fr) * kLd + a.value * 32 + q * 8;
+        *reinterpret_cast<half8_t*>(dst) = hi[i.value];
+        *reinterpret_cast<half8_t*>(dst + T::BM * kLd) = lo[i.value];
+    });
+    __syncthreads();
+    half8_t yh[4], yl[4];
+    uint32_t low_bits = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        yh[k] = *reinterpret_cast<const half8_t*>(yrow + k * 32);
+        yl[k] = *reinterpret_cast<const half8_t*>(yrow + T::BM * kLd + k * 32);
+        low_bits |= any_bits(yl[k]);
+    }
+    const bool has_low = __ballot(low_bits != 0) != 0;  // never with plain signs: the product is exact
+    const bool store = rt * 16 + fr < valid;
+    half_t* out = xd + (size_t)(m0 + rt * 16 + fr) * H + hg * 128 + q * 8;
+    for_parts([&](auto a, auto) {
+        float z[8];
+        transform(yh, a, z);
+        if (has_low) {
+            float zl[8];
+            transform(yl, a, zl);
+#pragma unroll
+            for (int c = 0; c < 8; c++) z[c] = __fadd_rn(z[c], zl[c]);
+        }
+        half8_t o;
+#pragma unroll
+        for (int c = 0; c < 8; c++) o[c] = (half_t)(z[c] * kHadNorm);
+        if (store) *reinterpret_cast<half8_t*>(out + a.value * 32) = o;
+    });
+}
+
+// unit = (row block b, 256-column block g of D), XCD order as above; rows go to out[order[r]].
+template <int K, int CB, int MR>
+__global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
+    const uint32_t* __restrict__ trellis, const half_t* __restrict__ xd, const int4* __restrict__ table, int n_blocks,
+    const half_t* __restrict__ dn_svh, const int* __restrict__ order, half_t* __restrict__ out, int n_rows, int E,
+    int D, int H) {
+    using T = RowsTile<MR, 2>;
+    constexpr int LPW = (T::FILLS + 7) / 8;
+    constexpr int kLd = 256 + kYPad;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int gblocks = (D + 255) >> 8;
+    const int set = blockIdx.x / (8 * gblocks), in_set = blockIdx.x % (8 * gblocks);
+    const int b = set * 8 + (in_set & 7), g = in_set >> 3;
+    if (b >= n_blocks) return;
+    const int4 blk = table[b];
+    const int e = blk.x, m0 = blk.y, end = min(blk.z, n_rows);
+    if (e < 0 || e >= E || m0 < 0 || m0 >= end) return;
+    const int valid = min(end - m0, T::BM);
+    // a last block of 128 columns: its upper half repeats the lower half's and is not stored
+    const bool full = g * 256 + 128 < D;
+
+    const int cq = wave >> 1, ks = wave & 1;
+    const size_t row_words = (size_t)E * (D >> 4) * (8 * K);
+    const uint32_t* w = trellis + (size_t)(2 * ks + (lane >> 5)) * row_words +
+                        ((size_t)e * (D >> 4) + g * 16 + (full ? cq : cq & 1) * 4 + ((lane >> 3) & 3)) * (8 * K) +
+                        (lane & 7) * K;
+    half_t* stages = reinterpret_cast<half_t*>(lds);
+    uint32_t a_off[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, 2>(wave * LPW + i, lane, valid - 1, H);
+    float16_t acc[MR][2];
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int cs = 0; cs < 2; cs++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
+    rows_main<K, CB, MR, 2, LPW>(w, 4 * row_words, reinterpret_cast<const char*>(xd + (size_t)m0 * H), a_off,
+                                 wave * LPW < T::FILLS, lds_byte_address(stages) + wave * LPW * 1024,
+                                 stages, rows_read_base<MR, 2>(ks, lane), H >> 6, lane, acc);
+    float16_t sum[MR];
+    rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
+    half_t* tile = reinterpret_cast<half_t*>(lds);  // [BM][kLd]
+    rows_store_half<MR>(sum, tile, kLd, cq * 64, ks, lane);
+    __syncthreads();
+
+    // output transform: a wave takes a 16-row tile and 2 MR of the eight 32-column parts
+    const int rt = wave % (2 * MR), part = wave / (2 * MR);
+    const int fr = lane & 15, q = lane >> 4;
+    const HadamardColumns had(lane);
+    const int r = rt * 16 + fr;
+    const size_t dst_row = r < valid ? (size_t)order[m0 + r] : 0;
+    static_for<0, 4 / MR>([&](auto p) {
+        if (part != p.value) return;
+        static_for<0, 2 * MR>([&](auto i) {
+            constexpr int c = p.value * 2 * MR + i.value, half = c >> 2, a = c & 3;
+            if (half && !full) return;
+            const half_t* yrow = tile + (rt * 16 + fr) * kLd + half * 128 + q * 8;
+            float4_t t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+            static_for<0, 4>([&](auto k) {
+                const half8_t y = *reinterpret_cast<const half8_t*>(yrow + k.value * 32);
+                t[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<2 * a, k.value>(), y, t[0], 0, 0, 0);
+                t[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<2 * a + 1, k.value>(), y, t[1], 0, 0, 0);
+            });
+            const int col = g * 256 + half * 128 + a * 32 + q * 8;
+            const half8_t sv = *reinterpret_cast<const half8_t*>(dn_svh + (size_t)e * D + col);
+            half8_t o;
+#pragma unroll
+            for (int j = 0; j < 8; j++) o[j] = (half_t)(t[j >> 2][j & 3] * kHadNorm * (float)sv[j]);
+            if (r < valid) *reinterpret_cast<half8_t*>(out + dst_row * D + col) = o;
+        });
+    });
+}
+
+template <int MR>
+static constexpr size_t rows_lds_bytes(int tiles, int tile_cols) {
+    const size_t stages = (size_t)tiles * 3 * RowsTile<MR, 2>::STAGE * 2;
+    const size_t exchange = (size_t)8 * MR * 4 * 64 * 16;
+    const size_t y = (size_t)tiles * RowsTile<MR, 2>::BM * (tile_cols + kYPad) * 2;
+    return stages > exchange ? (stages > y ? stages : y) : (exchange > y ? exchange : y);
+}
+
+// block_rows: 32 or 64
+int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const uint16_t* gu_trellis,
+                    const uint16_t* gu_svh, const uint16_t* dn_trellis, const uint16_t* dn_suh,
+                    const uint16_t* dn_svh, int E, int D, int H, int K, int cb, int activation,
+                    const int32_t* table, int n_blocks, int block_rows, const int32_t* order, uint16_t* xd,
+                    uint16_t* out, hipStream_t stream) {
+    const long long sets = (n_blocks + 7) / 8;
+    const long long gu_grid = sets * 8 * (H / 128), dn_grid = sets * 8 * ((D + 255) / 256);
+    if (gu_grid > 0x7FFFFFFFLL || dn_grid > 0x7FFFFFFFLL) return EXL3_E_BAD_SHAPE;
+    auto H_ = [](const uint16_t* p) { return reinterpret_cast<const half_t*>(p); };
+    return dispatch_k_cb(K, cb, [&](auto k, auto c) {
+        auto go = [&](auto mrc) {
+            constexpr int MR = mrc.value;
+            constexpr size_t gu_lds = rows_lds_bytes<MR>(2, 128), dn_lds = rows_lds_bytes<MR>(1, 256);
+            auto gu = moe_gateup_rows_kernel<k.value, c.value, MR>;
+            auto dn = moe_down_rows_kernel<k.value, c.value, MR>;
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(gu), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)gu_lds) != hipSuccess ||
+                hipFuncSetAttribute(reinterpret_cast<const void*>(dn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)dn_lds) != hipSuccess)
+                return (int)EXL3_E_LAUNCH;
+            gu<<<dim3((unsigned)gu_grid), dim3(kRowsThreads), gu_lds, stream>>>(
+                reinterpret_cast<const uint32_t*>(gu_trellis), H_(xg), H_(xu), reinterpret_cast<const int4*>(table),
+                n_blocks, H_(gu_svh), H_(dn_suh), reinterpret_cast<half_t*>(xd), n_rows, E, D, H, activation);
+            if (int rc = launch_status()) return rc;
+            dn<<<dim3((unsigned)dn_grid), dim3(kRowsThreads), dn_lds, stream>>>(
+                reinterpret_cast<const uint32_t*>(dn_trellis), H_(xd), reinterpret_cast<const int4*>(table), n_blocks,
+                H_(dn_svh), order, reinterpret_cast<half_t*>(out), n_rows, E, D, H);
+            return launch_status();
+        };
+        return block_rows == 32 ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 2>{});
+    });
+}
+
+}  // namespace exl3
