@@ -166,8 +166,8 @@ int launch_had_rows(const uint16_t* x, int n_in_rows, int rows, int n, const int
 
 int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub, uint16_t* xh,
                         hipStream_t stream);
-int launch_had_pre_pairs(const uint16_t* x, int tokens, int rows, int n, const int32_t* tok,
-                         const uint16_t* gu_suh, int n_experts, const int32_t* expert, uint16_t* xg,
+int launch_had_pre_pairs(const uint16_t* x, int tokens, int top_k, int n, const int32_t* order,
+                         const int32_t* indices, const uint16_t* gu_suh, int n_experts, uint16_t* xg,
                          size_t sub_stride, hipStream_t stream);
 
 // Experts of rows sorted by expert (row-block table as exl3_moe_sort's, blocks of 32 or 64):

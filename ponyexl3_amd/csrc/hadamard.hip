@@ -111,29 +111,29 @@ __global__ __launch_bounds__(256) void had_pre_wide_kernel(const half_t* __restr
 }
 
 // Input side on the matrix pipe: a wave rotates 16 rows x one 128-wide block, for
-// subs_per_wave of the stacked siblings from one read of x. The products x * suh have 22
-// significant bits; they enter the matrix instructions exactly as a high and a low fp16
-// part (the low parts of plain signs are all zero and then skipped) against entries +-1, with
-// fp32 sums, so the result is the fp32 butterfly's up to the order of the additions. 32 (or
-// 64) matrix instructions of 16 cycles and about 3 VALU instructions per element replace
-// about 18: the butterfly form was bound by VALU issue (23 us for 2048 x 5120 to two siblings,
-// 31 MB read and 42 MB written with the signs).
-// Row maps (MoE rows sorted by expert): source row in_index[r], scale row scale_index[r] of
-// scale_ld halfs; indices outside the buffers skip the row.
-// out + s * sub_stride + r * row_stride
+// subs_per_wave of the stacked siblings from one read of x, against entries +-1 with fp32 sums
+// (the fp32 butterfly's result up to the order of the additions). Plain signs (packed sign
+// words, the usual case) are applied to the fp16 bits of x; general scale vectors give
+// products of 22 bits, which enter exactly as a high and a low fp16 part. 32 (64) matrix
+// instructions of 16 cycles and 2 (6) VALU instructions per element replace about 18: the
+// butterfly form is bound by VALU issue.
+// Row maps (MoE rows sorted by expert): row r is pair p = pair[r] of token p / top_k and
+// expert pair_expert[p], whose scales are scale_ld halfs from the next expert's; entries
+// outside the buffers are clamped.
+// Results: out + s * sub_stride + r * row_stride.
 struct RotateArgs {
     const half_t* x;
     const half_t* suh;
     half_t* out;
     int rows, n, n_sub, subs_per_wave;
     size_t sub_scale, sub_stride, row_stride;  // halfs from one sibling's scales / results to the next
-    const int32_t* in_index;
-    const int32_t* scale_index;
+    const int32_t* pair;
+    const int32_t* pair_expert;
+    int top_k, n_tokens, n_experts;
     size_t scale_ld;
-    unsigned n_in, n_scale;
 };
 
-__global__ __launch_bounds__(256) void had_pre_mfma_kernel(RotateArgs a) {
+__global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
     const int lane = threadIdx.x & 63;
     const int fr = lane & 15, q = lane >> 4;
     const int blocks = a.n >> 7;
@@ -142,60 +142,60 @@ __global__ __launch_bounds__(256) void had_pre_mfma_kernel(RotateArgs a) {
     if (wid >= (long long)row_tiles * blocks) return;
     // consecutive waves take consecutive blocks of the same rows
     const int blk = (int)(wid % blocks), r = (int)(wid / blocks) * 16 + fr;
-    bool valid = r < a.rows;
-    unsigned src = valid ? (unsigned)r : 0u, scale_row = 0;
-    if (a.in_index) {
-        src = (unsigned)a.in_index[src];
-        valid = valid && src < a.n_in;
+    const bool valid = r < a.rows;
+    int src = valid ? r : 0, scale_row = 0;
+    if (a.pair) {
+        const int p = min(max(a.pair[src], 0), a.n_tokens * a.top_k - 1);
+        scale_row = min(max(a.pair_expert[p], 0), a.n_experts - 1);
+        src = p / a.top_k;
     }
-    if (a.scale_index) {
-        scale_row = (unsigned)a.scale_index[valid ? r : 0];
-        valid = valid && scale_row < a.n_scale;
-    }
-    if (!valid) src = 0, scale_row = 0;
     const size_t col = (size_t)blk * 128 + q * 8;
     const half_t* xr = a.x + (size_t)src * a.n + col;
-    half8_t xv[4];
+    uint4_t xv[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) xv[k] = *reinterpret_cast<const half8_t*>(xr + k * 32);
+    for (int k = 0; k < 4; k++) xv[k] = *reinterpret_cast<const uint4_t*>(xr + k * 32);
     const HadamardColumns had(lane);
     const int s_begin = blockIdx.y * a.subs_per_wave, s_end = min(s_begin + a.subs_per_wave, a.n_sub);
     for (int s = s_begin; s < s_end; s++) {
-        half8_t hi[4], lo[4];
-        uint32_t low_bits = 0;
+        float4_t z[8];
+#pragma unroll
+        for (int nt = 0; nt < 8; nt++) z[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
+        auto contract = [&](auto k, half8_t v) {
+            static_for<0, 8>([&](auto nt) {
+                z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(), v,
+                                                                     z[nt.value], 0, 0, 0);
+            });
+        };
+        uint4_t sv[4];
+        uint32_t not_one = 0;
         if (a.suh) {
             const half_t* sr = a.suh + (size_t)scale_row * a.scale_ld + (size_t)s * a.sub_scale + col;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                const half8_t sv = *reinterpret_cast<const half8_t*>(sr + k * 32);
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    half_t h, l;
-                    split_halves(__fmul_rn((float)xv[k][j], (float)sv[j]), h, l);
-                    hi[k][j] = h;
-                    lo[k][j] = l;
-                }
-                low_bits |= any_bits(lo[k]);
+                sv[k] = *reinterpret_cast<const uint4_t*>(sr + k * 32);
+                const uint4_t m = (sv[k] & 0x7FFF7FFFu) ^ 0x3C003C00u;
+                not_one |= m.x | m.y | m.z | m.w;
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < 4; k++) hi[k] = xv[k];
+            for (int k = 0; k < 4; k++) sv[k] = uint4_t{0u, 0u, 0u, 0u};
         }
-        float4_t z[8];
-#pragma unroll
-        for (int nt = 0; nt < 8; nt++) z[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-        static_for<0, 4>([&](auto k) {
-            static_for<0, 8>([&](auto nt) {
-                z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(), hi[k.value],
-                                                                     z[nt.value], 0, 0, 0);
-            });
-        });
-        if (__ballot(low_bits != 0)) {
+        if (__ballot(not_one != 0) == 0) {
             static_for<0, 4>([&](auto k) {
-                static_for<0, 8>([&](auto nt) {
-                    z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(),
-                                                                         lo[k.value], z[nt.value], 0, 0, 0);
-                });
+                contract(k, __builtin_bit_cast(half8_t, xv[k.value] ^ (sv[k.value] & 0x80008000u)));
+            });
+        } else {
+            static_for<0, 4>([&](auto k) {
+                const half8_t x8 = __builtin_bit_cast(half8_t, xv[k.value]), s8 = __builtin_bit_cast(half8_t, sv[k.value]);
+                half8_t hi, lo;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float p = __builtin_fmaf((float)x8[j], (float)s8[j], -0.0f);
+                    hi[j] = (half_t)p;
+                    lo[j] = (half_t)__builtin_fmaf((float)hi[j], -1.0f, p);
+                }
+                contract(k, hi);
+                contract(k, lo);
             });
         }
         if (valid) {
@@ -456,10 +456,12 @@ int launch_had_rows(const uint16_t* x, int n_in_rows, int rows, int n, const int
     return launch_status();
 }
 
-// The rotation as the layer forwards use it: on the matrix pipe from nine rows on.
+// The rotation as the layer forwards use it: on the matrix pipe from 64 rows on (16 rows for two
+// siblings of 5120: 4.1 us in the butterfly kernel, 5.0 here; 77 rows for three: 5.8 and 5.4;
+// 2048 rows: 23.0 and 18.6).
 int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub, uint16_t* xh,
                         hipStream_t stream) {
-    if (rows < 9 || n < 128 || n % 128 || n_sub < 1 || (!suh && n_sub != 1) || !x || !xh || !aligned16(x) ||
+    if (rows < 64 || n < 128 || n % 128 || n_sub < 1 || (!suh && n_sub != 1) || !x || !xh || !aligned16(x) ||
         !aligned16(xh) || (suh && !aligned16(suh)))
         return launch_had_pre(x, rows, n, suh, n_sub, xh, stream);
     RotateArgs a{};
@@ -475,25 +477,27 @@ int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh,
 }
 
 // Rows sorted by expert: both rotations (gate and up signs of the row's expert, gu_suh
-// [E][2][n]) of token row tok[r], to xg[r] and, sub_stride halfs further, xu[r].
-int launch_had_pre_pairs(const uint16_t* x, int tokens, int rows, int n, const int32_t* tok, const uint16_t* gu_suh,
-                         int n_experts, const int32_t* expert, uint16_t* xg, size_t sub_stride, hipStream_t stream) {
+// [E][2][n]) of row r = pair order[r], to xg[r] and, sub_stride halfs further, xu[r].
+int launch_had_pre_pairs(const uint16_t* x, int tokens, int top_k, int n, const int32_t* order,
+                         const int32_t* indices, const uint16_t* gu_suh, int n_experts, uint16_t* xg,
+                         size_t sub_stride, hipStream_t stream) {
     if (!aligned16(x) || !aligned16(gu_suh) || !aligned16(xg) || sub_stride % 8) return EXL3_E_BAD_SHAPE;
     RotateArgs a{};
     a.x = reinterpret_cast<const half_t*>(x);
     a.suh = reinterpret_cast<const half_t*>(gu_suh);
     a.out = reinterpret_cast<half_t*>(xg);
-    a.rows = rows;
+    a.rows = tokens * top_k;
     a.n = n;
     a.n_sub = 2;
     a.sub_scale = (size_t)n;
     a.sub_stride = sub_stride;
     a.row_stride = (size_t)n;
-    a.in_index = tok;
-    a.scale_index = expert;
+    a.pair = order;
+    a.pair_expert = indices;
+    a.top_k = top_k;
+    a.n_tokens = tokens;
+    a.n_experts = n_experts;
     a.scale_ld = (size_t)2 * n;
-    a.n_in = (unsigned)tokens;
-    a.n_scale = (unsigned)n_experts;
     return launch_rotate(a, stream);
 }
 

@@ -812,18 +812,19 @@ constexpr int kSortMaxExperts = 1024;
 
 // Stable counting sort by expert id. Outputs, all indexed by sorted position:
 //   order[pos] = pair index (token * top_k + slot), tok[pos] = token,
-//   sidx[pos] = expert; table[b] = {expert, first row, end row of the expert, 0}
-// for every block of block_rows rows, unused entries {E-1, N, N, 0} (empty).
+//   sidx[pos] = expert (tok and sidx may be NULL); table[b] = {expert, first row, end row of
+//   the expert, 0} for every block of block_rows rows, unused entries {E-1, N, N, 0} (empty).
+// With `staged` the order is put together in LDS and written out in order: one CU's scattered
+// 4-byte stores (64 lines per instruction) are what this kernel is otherwise bound by.
 //
 // Each of the 16 waves owns one contiguous segment of the pairs and a cursor per expert in
 // LDS: count, one scan over (expert, wave), then every wave places its segment 64 pairs at a
 // time without meeting the others. A pair's rank among equal experts of its 64 comes from
-// ballots over the bits of the expert id. Latency-bound: 13 833 pairs over 257 experts take
-// 11 us; walking the pairs 1024 at a time with counts exchanged across the waves took 41.
+// ballots over the bits of the expert id.
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int* __restrict__ indices, int n_pairs, int top_k, int E, int block_rows,
     int* __restrict__ order, int* __restrict__ tok, int* __restrict__ sidx,
-    int4* __restrict__ table, int table_len) {
+    int4* __restrict__ table, int table_len, int staged) {
     constexpr int kWaves = kSortThreads / 64;
     extern __shared__ int cursor[];  // [kWaves][E]
     __shared__ int scan_tmp[2][kWaves];
@@ -833,7 +834,15 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int per_wave = (n_pairs + 64 * kWaves - 1) / (64 * kWaves) * 64;
     const int begin = wave * per_wave, end = min(begin + per_wave, n_pairs);
     int* mine = cursor + wave * E;
-    for (int i = begin + lane; i < end; i += 64) atomicAdd(&mine[clamp_expert(indices[i], E)], 1);
+    int* stage = cursor + kWaves * E;
+    for (int i0 = begin + lane; i0 < end; i0 += 8 * 64) {  // eight loads in flight
+        int e[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) e[j] = indices[min(i0 + j * 64, n_pairs - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (i0 + j * 64 < end) atomicAdd(&mine[clamp_expert(e[j], E)], 1);
+    }
     __syncthreads();
 
     // exclusive scans over the experts (E <= 1024 = one value per thread): rows and blocks
@@ -885,27 +894,36 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
 
     int ebits = 0;
     while ((1 << ebits) < E) ebits++;
-    int next = begin + lane < end ? indices[begin + lane] : 0;
-    for (int i0 = begin; i0 < end; i0 += 64) {
-        const int i = i0 + lane;
-        const bool valid = i < end;
-        const int e = valid ? clamp_expert(next, E) : 0;
-        if (i + 64 < end) next = indices[i + 64];
-        unsigned long long same = __ballot(valid);
-        for (int b = 0; b < ebits; b++) {
-            const unsigned long long m = __ballot((e >> b) & 1);
-            same &= ((e >> b) & 1) ? m : ~m;
-        }
-        const int rank = __popcll(same & ((1ull << lane) - 1ull));
-        if (valid) {
-            const int first = mine[e];
-            if (rank == 0) mine[e] = first + __popcll(same);  // behind the reads: LDS is in order
-            const int pos = first + rank;
-            order[pos] = i;
-            tok[pos] = i / top_k;
-            sidx[pos] = e;
+    for (int i0 = begin; i0 < end; i0 += 8 * 64) {
+        int ids[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) ids[j] = indices[min(i0 + j * 64 + lane, n_pairs - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = i0 + j * 64 + lane;
+            const bool valid = i < end;
+            const int e = valid ? clamp_expert(ids[j], E) : 0;
+            unsigned long long same = __ballot(valid);
+            if (!same) break;
+            for (int b = 0; b < ebits; b++) {
+                const unsigned long long m = __ballot((e >> b) & 1);
+                same &= ((e >> b) & 1) ? m : ~m;
+            }
+            const int rank = __popcll(same & ((1ull << lane) - 1ull));
+            if (valid) {
+                const int first = mine[e];
+                if (rank == 0) mine[e] = first + __popcll(same);  // behind the reads: LDS is in order
+                const int pos = first + rank;
+                if (staged) stage[pos] = i;
+                else order[pos] = i;
+                if (tok) tok[pos] = i / top_k;
+                if (sidx) sidx[pos] = e;
+            }
         }
     }
+    if (!staged) return;
+    __syncthreads();
+    for (int i = tid; i < n_pairs; i += kSortThreads) order[i] = stage[i];
 }
 
 // One wave per (sorted row, 128-block of H): post-Hadamard + svh of the gate and up
@@ -949,13 +967,15 @@ __global__ __launch_bounds__(256) void moe_glu_rows_kernel(
 static int launch_moe_sort(const int32_t* indices, int n_pairs, int top_k, int n_experts, int block_rows,
                            int32_t* order, int32_t* tok, int32_t* sidx, int32_t* table, int table_len,
                            hipStream_t stream) {
-    const size_t lds = (size_t)(kSortThreads / 64) * n_experts * sizeof(int);
+    size_t lds = (size_t)(kSortThreads / 64) * n_experts * sizeof(int);
+    const bool staged = lds + (size_t)n_pairs * sizeof(int) <= (size_t)150 << 10;
+    if (staged) lds += (size_t)n_pairs * sizeof(int);
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_sort_kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return EXL3_E_LAUNCH;
     moe_sort_kernel<<<dim3(1), dim3(kSortThreads), lds, stream>>>(indices, n_pairs, top_k, n_experts, block_rows,
                                                                   order, tok, sidx, reinterpret_cast<int4*>(table),
-                                                                  table_len);
+                                                                  table_len, staged);
     return launch_status();
 }
 
@@ -1154,7 +1174,7 @@ static MoePrefillWorkspace moe_prefill_workspace(long long pairs, int E, int D, 
         at += align_up(bytes, 256);
         return o;
     };
-    w.o_tables = take((size_t)pairs * 3 * sizeof(int));  // order, tok, sidx
+    w.o_tables = take((size_t)pairs * sizeof(int));  // order
     w.o_table = take((size_t)w.table_len * sizeof(int4));
     w.o_xg = take((size_t)pairs * D * 2);  // later the slots' outputs
     w.o_xu = take((size_t)pairs * D * 2);
@@ -1195,14 +1215,14 @@ EXL3_EXPORT int exl3_moe_prefill(const uint16_t* x, int tokens, const int32_t* i
         if (reinterpret_cast<uintptr_t>(p) & 15) return EXL3_E_BAD_SHAPE;
     char* base = static_cast<char*>(workspace);
     int* order = reinterpret_cast<int*>(base + w.o_tables);
-    int *tok = order + N, *sidx = tok + N;
     int* table = reinterpret_cast<int*>(base + w.o_table);
     uint16_t* xg = reinterpret_cast<uint16_t*>(base + w.o_xg);
     uint16_t* xd = reinterpret_cast<uint16_t*>(base + w.o_xd);
     const size_t xu_offset = (w.o_xu - w.o_xg) / 2;
     hipStream_t s = as_stream(stream);
-    if (int rc = launch_moe_sort(indices, N, top_k, E, w.block_rows, order, tok, sidx, table, w.table_len, s)) return rc;
-    if (int rc = launch_had_pre_pairs(x, tokens, N, D, tok, gu_suh, E, sidx, xg, xu_offset, s)) return rc;
+    if (int rc = launch_moe_sort(indices, N, top_k, E, w.block_rows, order, nullptr, nullptr, table, w.table_len, s))
+        return rc;
+    if (int rc = launch_had_pre_pairs(x, tokens, top_k, D, order, indices, gu_suh, E, xg, xu_offset, s)) return rc;
     // gate, up, GLU and rotation, then down with its output transform, back in pair order
     uint16_t* slots = scores ? xg : y;
     if (int rc = launch_moe_rows(xg, xg + xu_offset, N, gu_trellis, gu_svh, dn_trellis, dn_suh, dn_svh, E, D, H, K, cb,
