@@ -113,7 +113,10 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
     }
 
     // Prefill: rotation kernel, MFMA GEMM, output transform.
-    if (int rc = launch_rotate_layer(x, rows, in_features, suh, n_sub, xh, s)) return rc;
+    // (without counters the chain of the separate entry points, bit for bit)
+    if (int rc = counters ? launch_rotate_layer(x, rows, in_features, suh, n_sub, xh, s)
+                          : launch_had_pre(x, rows, in_features, suh, n_sub, xh, s))
+        return rc;
     if (counters && rows <= linear_mid_max_rows()) {
         // a few dozen rows: the decode still sets the pace; every weight is decoded
         // once and goes from registers into 16x16x32 MFMA; split reduction and output

@@ -312,7 +312,12 @@ __device__ __forceinline__ void wht128_lanes(float& a, float& b, int lane) {
 // strictly by the direct loads in between, never too weakly). The caller waits for the data
 // with s_waitcnt vmcnt. (m0 is reserved: the compiler sets it right where it needs it.)
 __device__ __forceinline__ void load_lds16(const void* base, uint32_t offset, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base)
+    // (scalar registers also where the compiler cannot tell that the values are uniform)
+    const uint64_t b = reinterpret_cast<uint64_t>(base);
+    const uint64_t sb = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32;
+    const int sl = __builtin_amdgcn_readfirstlane((int)lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(sl), "v"(offset), "s"(sb)
                  : "memory");
 }
 __device__ __forceinline__ uint32_t lds_byte_address(const void* p) {

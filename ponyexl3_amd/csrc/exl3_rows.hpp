@@ -91,10 +91,10 @@ __device__ __forceinline__ void rows_main(const uint32_t* w, size_t w_step, cons
     };
     using S0 = std::integral_constant<int, 0>;
     using S1 = std::integral_constant<int, 1>;
-    // Memory operations retire in order. A fill is followed by at least one trellis load of its
-    // step, the next step's fills and that step's trellis load: with no more than those
-    // outstanding it has landed.
-    constexpr int kAfterFill = LPW + 2;
+    // Memory operations retire in order. A fill is followed by the trellis loads of its step (K
+    // dwords: at least (K + 3) / 4), the next step's fills and that step's trellis loads: with
+    // no more than those outstanding it has landed.
+    constexpr int kAfterFill = LPW + 2 * ((K + 3) / 4);
     load_a(0, 0);
     load_w(0, S0{});
     load_a(1, 1);
@@ -175,6 +175,13 @@ struct HadamardColumns {
     __device__ __forceinline__ half8_t get() const {
         constexpr uint32_t uni = (__builtin_popcount((NT >> 1) & KS) & 1) ? 0x80008000u : 0u;
         constexpr uint32_t hi = uni ^ ((NT & 1) ? 0x80008000u : 0u);
+        return __builtin_bit_cast(half8_t, uint4_t{w0 ^ uni, w1 ^ uni, w0 ^ hi, w1 ^ hi});
+    }
+    // the same for column tile 2 a + ODD with a (uniform) not known at compile time
+    template <int ODD, int KS>
+    __device__ __forceinline__ half8_t get_part(int a) const {
+        const uint32_t uni = (__builtin_popcount(a & KS) & 1) ? 0x80008000u : 0u;
+        const uint32_t hi = uni ^ (ODD ? 0x80008000u : 0u);
         return __builtin_bit_cast(half8_t, uint4_t{w0 ^ uni, w1 ^ uni, w0 ^ hi, w1 ^ hi});
     }
 };

@@ -151,7 +151,10 @@ void linear_run(const LinearLayer& l, const at::Tensor& x, int64_t rows64, const
         if (l.member_out.size() != static_cast<size_t>(l.n_sub) || total != n_out)
             value_error("member_out must list the out_features of the stacked members");
         const at::Tensor xh = at::empty({rows64, l.n_sub, n_in}, x.options());
-        check_status(exl3_rotate(xp, rows, n_in, half_ptr(l.suh), l.n_sub, half_out(xh), ctx.stream), "exl3_rotate");
+        // (not fused: the chain of the separate entry points, bit for bit)
+        check_status((fused ? exl3_rotate : exl3_had128_pre)(xp, rows, n_in, half_ptr(l.suh), l.n_sub, half_out(xh),
+                                                             ctx.stream),
+                     "exl3_rotate");
         if (one_launch) {
             // one GEMM launch over all members, each block reading its member's rotation, then
             // the output transform
