@@ -389,6 +389,24 @@ int exl3_moe_forward(const uint16_t *x, int tokens, const int32_t *indices, int 
 size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
 
 /*
+ * A layer on up to 1024 already rotated rows: every weight is decoded once
+ * per up to 128 rows and goes from registers into the matrix pipe; output transform
+ * (Hadamard-128, svh, bias) included. Members of a sibling-fused layer may end on any
+ * 128-column block.
+ *   xh        fp16 [rows][n_sub][16*in_tiles], 16-byte aligned
+ *   group_sub i32 [out_tiles/8] member index of every 128-column block (required when n_sub > 1)
+ *   y         fp16 [rows][16*out_tiles]
+ *   workspace exl3_linear_rows_workspace_bytes(rows, in, out) bytes (may be 0), 16-byte aligned
+ * exl3_linear_rows_applies: whether it is the faster path for these sizes (and the trellis 16-byte
+ * aligned, which it requires); otherwise take exl3_linear_prefill.
+ */
+int exl3_linear_rows_applies(const uint16_t *trellis, int rows, int in_tiles, int out_tiles);
+size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, int out_features);
+int exl3_linear_rows(const uint16_t *xh, int rows, int n_sub, const uint16_t *trellis, int in_tiles, int out_tiles,
+                     int K, int cb, const int32_t *group_sub, const uint16_t *svh, const uint16_t *bias, uint16_t *y,
+                     void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Prefill of one layer on activations that exl3_had128_pre already rotated:
  * the MFMA trellis GEMM and the output transform (Hadamard-128, svh, bias), for a
  * plain layer (n_sub = 1) or a sibling-fused one whose members all have

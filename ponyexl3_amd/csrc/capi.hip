@@ -3,6 +3,7 @@
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace exl3 {
@@ -20,6 +21,9 @@ struct LinearWorkspace {
     size_t total() const { return xh_bytes + second_bytes + gemm_bytes; }
 };
 
+// The rows kernel copies trellis words 16 bytes at a time.
+static bool rows_aligned(const uint16_t* trellis) { return (reinterpret_cast<uintptr_t>(trellis) & 15) == 0; }
+
 static LinearWorkspace linear_workspace(int rows, int in_features, int out_features, int n_sub) {
     LinearWorkspace w{};
     w.xh_bytes = align_up((size_t)rows * n_sub * in_features * 2, 256);
@@ -34,6 +38,10 @@ static LinearWorkspace linear_workspace(int rows, int in_features, int out_featu
             const MidPlan m = plan_linear_mid(rows, in_features / 16, out_features / 128);
             const size_t mid = (size_t)m.n_splits * rows * out_features * sizeof(float);
             if (mid > w.second_bytes) w.second_bytes = mid;
+        }
+        if (linear_rows_applies(rows, in_features / 16, out_features / 16)) {
+            const size_t part = linear_rows_partial_bytes(rows, in_features / 16, out_features / 128);
+            if (part > w.second_bytes) w.second_bytes = part;
         }
         w.gemm_bytes = align_up(gemm_workspace_bytes(rows, in_features / 16, out_features / 16), 256);
     }
@@ -117,6 +125,12 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
     if (int rc = counters ? launch_rotate_layer(x, rows, in_features, suh, n_sub, xh, s)
                           : launch_had_pre(x, rows, in_features, suh, n_sub, xh, s))
         return rc;
+    if (counters && (n_sub == 1 || rows <= kLinearMidMaxRows) && rows_aligned(trellis) &&
+        rows > std::min(kLinearMidPreferredRows, linear_mid_max_rows()) &&
+        linear_rows_applies(rows, in_tiles, out_tiles))
+        return launch_linear_rows(xh, rows, (size_t)n_sub * in_features, (size_t)in_features, trellis, in_tiles,
+                                  out_tiles, K, cb, n_sub > 1 ? group_sub : nullptr, svh, bias, y,
+                                  reinterpret_cast<float*>(second), s);
     if (counters && rows <= linear_mid_max_rows()) {
         // a few dozen rows: the decode still sets the pace; every weight is decoded
         // once and goes from registers into 16x16x32 MFMA; split reduction and output
@@ -179,6 +193,33 @@ EXL3_EXPORT int exl3_linear_prefill(const uint16_t* xh, int rows, int n_sub, con
         return rc;
     if (post_done) return EXL3_OK;
     return launch_had_post(ytmp, 0, 1, 0, rows, out_features, svh, bias, y, s);
+}
+
+EXL3_EXPORT int exl3_linear_rows_applies(const uint16_t* trellis, int rows, int in_tiles, int out_tiles) {
+    return exl3::rows_aligned(trellis) && exl3::linear_rows_applies(rows, in_tiles, out_tiles);
+}
+
+EXL3_EXPORT size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, int out_features) {
+    if (rows < 1 || in_features < 128 || out_features < 128) return 0;
+    return exl3::linear_rows_partial_bytes(rows, in_features / 16, out_features / 128);
+}
+
+EXL3_EXPORT int exl3_linear_rows(const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis, int in_tiles,
+                                 int out_tiles, int K, int cb, const int32_t* group_sub, const uint16_t* svh,
+                                 const uint16_t* bias, uint16_t* y, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+    using namespace exl3;
+    if (int rc = check_k_cb(K, cb)) return rc;
+    if (!xh || !trellis || !y) return EXL3_E_NULL_POINTER;
+    if (rows < 1 || in_tiles < 8 || out_tiles < 8 || in_tiles % 8 || out_tiles % 8 || n_sub < 1)
+        return EXL3_E_BAD_SHAPE;
+    if (rows > kLinearRowsMaxRows) return EXL3_E_UNSUPPORTED;
+    if (n_sub > 1 && !group_sub) return EXL3_E_BAD_INDEX;
+    if (workspace_bytes < linear_rows_partial_bytes(rows, in_tiles, out_tiles / 8)) return EXL3_E_WORKSPACE;
+    const size_t in_features = (size_t)in_tiles * 16;
+    return launch_linear_rows(xh, rows, n_sub * in_features, in_features, trellis, in_tiles, out_tiles, K, cb,
+                              n_sub > 1 ? group_sub : nullptr, svh, bias, y, reinterpret_cast<float*>(workspace),
+                              as_stream(stream));
 }
 
 // ---------------------------------------------------------------------------

@@ -96,6 +96,10 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
 // [rows][n_sub][in]: weights decoded once and fed to 16x16x16 MFMA from registers;
 // partial: fp32 [plan.n_splits][rows][out]; counters as for launch_linear_small.
 constexpr int kLinearMidMaxRows = 32;
+// From here up the rows kernel (below) is faster where it can run (16-byte aligned trellis): 32
+// rows of 5120 -> 10240 26.2 -> 22.6 us, 17408 -> 5120 (K = 5) 42.6 -> 30.1; at 16 rows of 5120 ->
+// 10240 and 2048 -> 2048 it takes 22.7 and 13.1 us against 20.7 and 11.6 here.
+constexpr int kLinearMidPreferredRows = 16;
 struct MidPlan {
     int n_splits;          // workgroups per 128-column group
     int blocks_per_split;  // 128-row blocks of the reduction per workgroup
@@ -108,6 +112,22 @@ int launch_linear_mid(const uint16_t* xh, int rows, const uint16_t* trellis, int
                       int out_tiles, int K, int cb, int n_sub, const int32_t* group_sub,
                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial,
                       int* counters, MidPlan plan, hipStream_t stream);
+
+// Layer on rotated activations with up to kLinearRowsMaxRows rows (linear_rows.hip). Column group
+// g (128 columns) reads xh + group_sub[g] * sub_stride (group_sub may be NULL);
+// partial: linear_rows_partial_bytes(), 16-byte aligned.
+constexpr int kLinearRowsMaxRows = 1024;
+struct LinRowsPlan {
+    int n_row_blocks, block_rows, mr;  // mr: 32-row tiles of the kernel that holds block_rows
+    int n_splits, steps_per_split;     // ranges of the reduction, in 128-deep steps
+    double us;                         // estimate, without the input rotation
+};
+LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups);
+size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups);
+bool linear_rows_applies(int rows, int in_tiles, int out_tiles);
+int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
+                       int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
+                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream);
 
 int launch_had_pre(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub,
                    uint16_t* xh, hipStream_t stream);
@@ -129,6 +149,8 @@ struct GemmPlan {
     int split_runs, split_per, split_pitch, split_runs_per_tile;
 };
 GemmPlan plan_gemm(int rows, int in_tiles, int tn_count, bool allow_split);
+// Estimate of its time with the fix-up, against linear_rows_applies()' estimate.
+double gemm_estimate_us(int rows, int in_tiles, int tn_count);
 size_t gemm_workspace_bytes(int rows, int in_tiles, int tn_count);
 
 // Output transform the GEMM may fold into its fix-up pass: when every tile of the

@@ -47,103 +47,149 @@ __device__ __forceinline__ uint32_t rows_fill_offset(int f, int lane, int last_r
     return (uint32_t)((size_t)min(row, last_row) * ldx * 2 + chunk * 16);
 }
 
-template <int K, int CB, int CS>
-__device__ __forceinline__ void decode_column(const LaneWords<K>& lw, half2_t (&wp)[16]) {
-    static_for<0, 4>([&](auto i) {
-        constexpr int na = 4 * (2 * i.value + CS), nb = na + 2;
-        constexpr int ia = 8 * cw_col_sel(na) + (cw_row(na) >> 1);
-        constexpr int ib = 8 * cw_col_sel(nb) + (cw_row(nb) >> 1);
-        decode_pair2<CB>(lane_codeword<K, na>(lw), lane_codeword<K, na + 1>(lw), lane_codeword<K, nb>(lw),
-                         lane_codeword<K, nb + 1>(lw), wp[ia], wp[ib]);
-    });
+// Half H of quad I (0..3) of column tile pair CS: the quad is rows 2I, 2I + 1 and 2I + 8, 2I + 9
+// of the lane's column; its first half leaves two codewords scrambled in `x`.
+template <int K, int CB, int CS, int I, int H>
+__device__ __forceinline__ void decode_half_quad(const LaneWords<K>& lw, uint32_t (&x)[2], half2_t (&wp)[2][4]) {
+    constexpr int na = 4 * (2 * I + CS), nb = na + 2;
+    static_assert(cw_col_sel(na) == CS && cw_row(na) == 2 * I && cw_row(nb) == 2 * I + 8);
+    if constexpr (CB == CB_MUL1) {
+        wp[H][I].x = decode_mul1(lane_codeword<K, na + 2 * H>(lw));
+        wp[H][I].y = decode_mul1(lane_codeword<K, na + 2 * H + 1>(lw));
+    } else if constexpr (H == 0) {
+        x[0] = scramble<CB>(lane_codeword<K, na>(lw));
+        x[1] = scramble<CB>(lane_codeword<K, na + 1>(lw));
+    } else {
+        add_halves_pack2(x[0], x[1], scramble<CB>(lane_codeword<K, nb>(lw)), scramble<CB>(lane_codeword<K, nb + 1>(lw)),
+                         wp[0][I], wp[1][I]);
+    }
 }
+
+// Trellis words of a wave and step, in LDS as in memory: 64 lanes x K dwords.
+template <int K>
+struct RowsWords {
+    static constexpr int STAGE = 64 * K;                // dwords of one wave and stage
+    static constexpr int LOADS = (16 * K + 63) / 64;    // wave-wide direct loads of 16 bytes a lane
+};
 
 // acc[mr][cs] (+)= D of 32x32: column m (lane m of the decode: tile m >> 3, column (m & 7) +
 // 8 cs of it) x activation row 32 mr + n. A lane holds n = lane & 31 and m = 8 (i >> 2) +
 // 4 (lane >> 5) + (i & 3), i = 0..15.
-//   w       the lane's trellis words at step 0; w_step dwords further per step
-//   a       activation tile at step 0 (uniform); a_off: rows_fill_offset of the wave's LPW
-//           fills, which go to LDS bytes fill_to + 1024 i (fills: whether this wave has any)
-//   stages  the activation stages; read_off: the lane's first fragment, see rows_read_base
+//   w         the wave's trellis words at step 0 (uniform): four tiles of its first tile row;
+//             w_row dwords further the second; w_step dwords further per step
+//   a         activation tile at step 0 (uniform); a_off: rows_fill_offset of the wave's LPW
+//             fills, which go to LDS bytes fill_to + 1024 i (fills: whether this wave has any)
+//   stages    the activation stages; read_off: the lane's first fragment, see rows_read_base
+//   words     the wave's first word stage (16-byte aligned); word_stage dwords to its next
+//
+// Everything that comes from memory goes to LDS by direct loads, two steps and more ahead, so no
+// register waits for memory and the only wait is the counted one at the barrier: the compiler
+// cannot count the direct loads, and its waits for trellis words in registers drained them
+// to one step. One barrier in the middle of a step: before it the matrix pipe works on column
+// tile pair 0 while pair 1 is decoded, behind it on pair 1 while pair 0 of the next step is
+// decoded and that step's fragments are read, so that a wave keeps both pipes busy by itself
+// (decode of a pair: about 68 VALU instructions of 4 cycles between its 2 MR matrix
+// instructions of 32 cycles).
 template <int K, int CB, int MR, int NKS, int LPW>
-__device__ __forceinline__ void rows_main(const uint32_t* w, size_t w_step, const char* a,
+__device__ __forceinline__ void rows_main(const uint32_t* w, size_t w_row, size_t w_step, const char* a,
                                           const uint32_t (&a_off)[LPW], bool fills, uint32_t fill_to,
-                                          const half_t* stages, int read_off, int nsteps, int lane, float16_t (&acc)[MR][2]) {
+                                          const half_t* stages, int read_off, const uint32_t* words, int word_stage,
+                                          int nsteps, int lane, float16_t (&acc)[MR][2]) {
     using T = RowsTile<MR, NKS>;
+    using W = RowsWords<K>;
+    constexpr int kBatch = LPW + W::LOADS;
     const int last = nsteps - 1;
-    uint32_t words[2][K];
-    auto load_w = [&](int t, auto slot) {
-        constexpr int s = decltype(slot)::value;
-        const uint32_t* q = w + (size_t)min(t, last) * w_step;
-        // the origin of the address is hidden from the optimiser, which could otherwise move
-        // the load across the waits below that count it
-        asm volatile("" : "+v"(q));
-        const auto p = (const uint32_t __attribute__((address_space(1)))*)q;
+    uint32_t w_off[W::LOADS];
 #pragma unroll
-        for (int i = 0; i < K; i++) words[s][i] = __builtin_nontemporal_load(p + i);
-        __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < W::LOADS; i++) {
+        const int c = 64 * i + lane;  // 16-byte chunk
+        w_off[i] = c < 8 * K ? 16u * c : (uint32_t)w_row * 4u + 16u * (c - 8 * K);
+    }
+    const uint32_t words_to = lds_byte_address(words);
+    // direct load I of step t's batch
+    auto load_one = [&](int t, int stage, auto ic) {
+        constexpr int i = ic.value;
+        const int tc = min(t, last);
+        if constexpr (i < LPW) {
+            if (fills)
+                load_lds16(a + (size_t)tc * (T::BK * 2), a_off[i], fill_to + (uint32_t)(stage * T::STAGE + i * 512) * 2);
+        } else {
+            constexpr int j = i - LPW;
+            if (64 * (j + 1) <= 16 * K || lane < 16 * K - 64 * j)
+                load_lds16(w + (size_t)tc * w_step, w_off[j], words_to + (uint32_t)(stage * word_stage + j * 256) * 4);
+        }
     };
-    auto load_a = [&](int t, int stage) {
-        if (!fills) return;
-        const char* p = a + (size_t)min(t, last) * (T::BK * 2);
+    auto load_batch = [&](int t, int stage) { static_for<0, kBatch>([&](auto i) { load_one(t, stage, i); }); };
+    // All but the last `n` batches of this wave have landed, and all waves have got here.
+    auto arrive = [&](auto n) {
+        constexpr int b = decltype(n)::value;
+        if (fills) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(b * kBatch) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(b * W::LOADS) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    LaneWords<K> lw;
+    const int prev = ((lane & ~7) | ((lane + 7) & 7)) * K + K - 1;
+    auto read_words = [&](int stage) {
+        const uint32_t* q = words + stage * word_stage;
+        lw.w[0] = q[prev];
 #pragma unroll
-        for (int i = 0; i < LPW; i++) load_lds16(p, a_off[i], fill_to + (uint32_t)(stage * T::STAGE + i * 512) * 2);
+        for (int i = 0; i < K; i++) lw.w[i + 1] = q[lane * K + i];
     };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    // Memory operations retire in order. A fill is followed by the trellis loads of its step (K
-    // dwords: at least (K + 3) / 4), the next step's fills and that step's trellis loads: with
-    // no more than those outstanding it has landed.
-    constexpr int kAfterFill = LPW + 2 * ((K + 3) / 4);
-    load_a(0, 0);
-    load_w(0, S0{});
-    load_a(1, 1);
-    load_w(1, S1{});
-    barrier_with_loads_in_flight<kAfterFill>();
-    int s0 = 0, s2 = 2;  // stage of step t and of step t + 2
-    auto step = [&](int t, auto slot) {
-        const LaneWords<K> lw = finish_lane_words<K>(words[decltype(slot)::value], lane);
-        __builtin_amdgcn_sched_barrier(0);
-        load_a(t + 2, s2);
-        __builtin_amdgcn_sched_barrier(0);
-        const half_t* r = stages + s0 * T::STAGE;
-        half8_t af[MR][2];
+    half8_t af[MR][2];
+    auto read_a = [&](int stage, auto kh) {
+        const half_t* r = stages + stage * T::STAGE;
 #pragma unroll
         for (int mr = 0; mr < MR; mr++)
-#pragma unroll
-            for (int kh = 0; kh < 2; kh++)
-                af[mr][kh] = *reinterpret_cast<const half8_t*>(r + (read_off ^ (kh * 8)) + mr * 32 * T::BK);
-        half2_t wp[16];
-        auto contract = [&](auto csc) {
-            constexpr int cs = decltype(csc)::value;
-#pragma unroll
-            for (int kh = 0; kh < 2; kh++) {
-                const uint4_t q = {half2_to_bits(wp[8 * cs + 4 * kh]), half2_to_bits(wp[8 * cs + 4 * kh + 1]),
-                                   half2_to_bits(wp[8 * cs + 4 * kh + 2]), half2_to_bits(wp[8 * cs + 4 * kh + 3])};
-#pragma unroll
-                for (int mr = 0; mr < MR; mr++)
-                    acc[mr][cs] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, q), af[mr][kh],
-                                                                         acc[mr][cs], 0, 0, 0);
-            }
-        };
-        decode_column<K, CB, 0>(lw, wp);
-        contract(S0{});
-        decode_column<K, CB, 1>(lw, wp);
-        contract(S1{});
-        // behind the decode, so that the words can come back to the registers they left
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(t + 2, slot);
-        barrier_with_loads_in_flight<kAfterFill>();
-        s0 = s0 == 2 ? 0 : s0 + 1;
-        s2 = s2 == 2 ? 0 : s2 + 1;
+            af[mr][kh.value] = *reinterpret_cast<const half8_t*>(r + (read_off ^ (kh.value * 8)) + mr * 32 * T::BK);
     };
-    int t = 0;
-    for (; t + 1 < nsteps; t += 2) {
-        step(t, S0{});
-        step(t + 1, S1{});
+    half2_t wp[2][2][4];  // [cs][kh]
+    // 2 MR matrix instructions of pair cs; the eight half quads of pair ds, and whatever
+    // after(i) issues, go evenly between them
+    uint32_t x[2];
+    auto half_step = [&](auto csc, auto dsc, auto after) {
+        constexpr int cs = decltype(csc)::value, ds = decltype(dsc)::value;
+        static_for<0, 2 * MR>([&](auto ic) {
+            constexpr int i = ic.value, kh = i / MR, mr = i % MR;
+            const uint4_t q = {half2_to_bits(wp[cs][kh][0]), half2_to_bits(wp[cs][kh][1]),
+                               half2_to_bits(wp[cs][kh][2]), half2_to_bits(wp[cs][kh][3])};
+            acc[mr][cs] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, q), af[mr][kh],
+                                                                 acc[mr][cs], 0, 0, 0);
+            after(ic);
+            static_for<8 * i / (2 * MR), 8 * (i + 1) / (2 * MR)>(
+                [&](auto h) { decode_half_quad<K, CB, ds, h.value / 2, h.value % 2>(lw, x, wp[ds]); });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    using N0 = std::integral_constant<int, 0>;
+    using N1 = std::integral_constant<int, 1>;
+    using N2 = std::integral_constant<int, 2>;
+    load_batch(0, 0);
+    load_batch(1, 1);
+    load_batch(2, 2);
+    arrive(N2{});
+    read_words(0);
+    read_a(0, N0{});
+    read_a(0, N1{});
+    static_for<0, 8>([&](auto h) { decode_half_quad<K, CB, 0, h.value / 2, h.value % 2>(lw, x, wp[0]); });
+    // no scalar load is under way in the loop, so that waits there can count the LDS reads
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    int s0 = 0, s1 = 1;  // stages of step t and t + 1
+    for (int t = 0; t < nsteps; t++) {
+        half_step(N0{}, N1{}, [](auto) {});
+        arrive(N1{});  // step t + 1 is in LDS; stage s0 has been read by every wave
+        read_words(s1);
+        __builtin_amdgcn_sched_barrier(0);
+        half_step(N1{}, N0{}, [&](auto ic) {
+            constexpr int i = ic.value;
+            if constexpr (i == MR - 1) read_a(s1, N0{});
+            if constexpr (i == 2 * MR - 1) read_a(s1, N1{});
+            static_for<kBatch * i / (2 * MR), kBatch * (i + 1) / (2 * MR)>([&](auto j) { load_one(t + 3, s0, j); });
+        });
+        s0 = s1;
+        s1 = s1 == 2 ? 0 : s1 + 1;
     }
-    if (t < nsteps) step(t, S0{});
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no fill lands in LDS after this
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load lands in LDS after this
     __syncthreads();
 }
 

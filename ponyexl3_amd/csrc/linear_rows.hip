@@ -1,0 +1,301 @@
+// Layer on a few dozen to a few hundred rows (takes the lower end of the rows > 16 ladder of
+// ponyexl3/mlx/exl3_linear.py:137-161): the decode still costs more than the product, so every
+// weight is decoded once per up to 128 rows and goes from registers into 32x32x16 matrix
+// instructions (see exl3_rows.hpp for the contraction).
+//
+// Workgroup = one 128-column group (one block of the output Hadamard) x one row block of 32 MR
+// rows x one range of the reduction; its eight waves are two 64-column strips x four k-slices
+// of a 128-deep step. A whole reduction ends with the output transform
+// (ponyexl3/ref/forward.py:41-45) on the matrix pipe; ranges write fp32 partial rows that
+// the output transform kernel adds in range order.
+//
+// What bounds it: issue of the decode, and the matrix pipe next to it. 333 rows of 17408 -> 5120
+// (K = 4): VALU issue 42 % and matrix pipe 33 % of the SIMD cycles, which overlap only in part,
+// 26 % of the wave time in waits and barriers; the kernel 93 us where the GEMM took 102.
+// Half of a quad between two matrix instructions, rather than a whole quad between pairs of
+// them, and direct loads spread the same way gave 5 %.
+//
+// x is already rotated: fp16 [rows][n_sub][in].
+#include "exl3_device.hpp"
+#include "exl3_host.hpp"
+#include "exl3_rows.hpp"
+
+#pragma clang fp contract(off)
+
+namespace exl3 {
+
+constexpr int kLinRowsThreads = 512;
+constexpr int kLinRowsLd = 128 + 8;  // halfs: 16-byte reads of 16 tile rows hit all banks
+
+struct LinRowsArgs {
+    const uint32_t* trellis;
+    const half_t* xh;
+    const half_t* svh;
+    const half_t* bias;
+    half_t* y;
+    float* partial;
+    const int* group_sub;  // rotation of each column group, or NULL
+    size_t ldx, sub_stride;
+    int rows, block_rows, n_row_blocks, n_units, n_splits, steps_per_split, in_steps, out_tiles;
+};
+
+// Sums of the four k-slices of a strip. On return the wave of slice ks holds column tile pair
+// cs = ks >> 1 and, of each of its 32-row blocks, accumulators 8 (ks & 1) .. + 7 of sixteen:
+// two exchanges of half of what a wave holds, every wave busy in both.
+template <int MR>
+__device__ __forceinline__ void rows_add_slices4(float16_t (&acc)[MR][2], float4_t* ex, int wave, int lane,
+                                                 float (&sum)[MR][8]) {
+    const bool upper = wave & 2, odd = wave & 1;
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float4_t v;
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = upper ? acc[mr][0][4 * i + c] : acc[mr][1][4 * i + c];
+            ex[((wave ^ 2) * MR * 4 + mr * 4 + i) * 64 + lane] = v;
+        }
+    __syncthreads();
+    float half_sum[MR][16];
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4_t v = ex[(wave * MR * 4 + mr * 4 + i) * 64 + lane];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                half_sum[mr][4 * i + c] = __fadd_rn(upper ? acc[mr][1][4 * i + c] : acc[mr][0][4 * i + c], v[c]);
+        }
+    __syncthreads();
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            float4_t v;
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = odd ? half_sum[mr][4 * i + c] : half_sum[mr][8 + 4 * i + c];
+            ex[((wave ^ 1) * MR * 2 + mr * 2 + i) * 64 + lane] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const float4_t v = ex[(wave * MR * 2 + mr * 2 + i) * 64 + lane];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                sum[mr][4 * i + c] = __fadd_rn(odd ? half_sum[mr][8 + 4 * i + c] : half_sum[mr][4 * i + c], v[c]);
+        }
+    __syncthreads();
+}
+
+// Workgroups are dealt to the eight XCDs by index: the row blocks of one (column group, range)
+// unit u land on one XCD, whose L2 then reads their trellis words once.
+template <int K, int CB, int MR>
+__global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_kernel(LinRowsArgs p) {
+    using T = RowsTile<MR, 4>;
+    constexpr int LPW = T::FILLS / 8;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int set = blockIdx.x / (8 * p.n_row_blocks), in_set = blockIdx.x % (8 * p.n_row_blocks);
+    const int u = set * 8 + (in_set & 7), rb = in_set >> 3;
+    if (u >= p.n_units) return;
+    const int g = u / p.n_splits, split = u % p.n_splits;
+    const int k0 = split * p.steps_per_split;
+    const int nsteps = min(p.steps_per_split, p.in_steps - k0);
+    const int m0 = rb * p.block_rows;
+    const int valid = min(p.block_rows, p.rows - m0);
+
+    const int cq = wave >> 2, ks = wave & 3;
+    const size_t row_words = (size_t)p.out_tiles * (8 * K);
+    const uint32_t* w = p.trellis + ((size_t)k0 * 8 + 2 * ks) * row_words + (size_t)(g * 8 + cq * 4) * (8 * K);
+    const half_t* x = p.xh + (size_t)m0 * p.ldx + (size_t)k0 * 128;
+    if (p.group_sub) x += (size_t)p.group_sub[g] * p.sub_stride;
+    half_t* stages = reinterpret_cast<half_t*>(lds);
+    uint32_t a_off[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, 4>(wave * LPW + i, lane, valid - 1, p.ldx);
+    float16_t acc[MR][2];
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int cs = 0; cs < 2; cs++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
+    uint32_t* words = reinterpret_cast<uint32_t*>(stages + 3 * T::STAGE) + wave * RowsWords<K>::STAGE;
+    rows_main<K, CB, MR, 4, LPW>(w, row_words, 8 * row_words, reinterpret_cast<const char*>(x), a_off, true,
+                                 lds_byte_address(stages) + wave * LPW * 1024, stages, rows_read_base<MR, 4>(ks, lane),
+                                 words, 8 * RowsWords<K>::STAGE, nsteps, lane, acc);
+    float sum[MR][8];
+    rows_add_slices4<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
+
+    // lane: row lane & 31 of each 32-row block, columns col + 16 i + 0..3
+    const int col = cq * 64 + 32 * (ks & 1) + 8 * (ks >> 1) + 4 * (lane >> 5);
+    const size_t n = (size_t)p.out_tiles * 16;
+    if (p.n_splits > 1) {
+        float* dst = p.partial + ((size_t)split * p.rows + m0) * n + (size_t)g * 128 + col;
+#pragma unroll
+        for (int mr = 0; mr < MR; mr++) {
+            const int r = mr * 32 + (lane & 31);
+            if (r < valid) {
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    float4_t v;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) v[c] = sum[mr][4 * i + c];
+                    *reinterpret_cast<float4_t*>(dst + (size_t)r * n + 16 * i) = v;
+                }
+            }
+        }
+        return;
+    }
+    half_t* tile = reinterpret_cast<half_t*>(lds);  // [BM][kLinRowsLd]
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            half4_t o;
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] = (half_t)sum[mr][4 * i + c];
+            *reinterpret_cast<half4_t*>(tile + (mr * 32 + (lane & 31)) * kLinRowsLd + col + 16 * i) = o;
+        }
+    __syncthreads();
+    // output transform: 2 MR 16-row tiles x four 32-column parts, MR of them to a wave
+    const int fr = lane & 15, q = lane >> 4;
+    const HadamardColumns had(lane);
+#pragma unroll
+    for (int j = 0; j < MR; j++) {
+        const int id = wave + 8 * j, rt = id >> 2, a = id & 3;
+        const half_t* yrow = tile + (rt * 16 + fr) * kLinRowsLd + q * 8;
+        float4_t t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        static_for<0, 4>([&](auto k) {
+            const half8_t yv = *reinterpret_cast<const half8_t*>(yrow + k.value * 32);
+            t[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get_part<0, k.value>(a), yv, t[0], 0, 0, 0);
+            t[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get_part<1, k.value>(a), yv, t[1], 0, 0, 0);
+        });
+        const int r = rt * 16 + fr, c0 = g * 128 + a * 32 + q * 8;
+        if (r >= valid) continue;
+        half8_t o;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            float v = __fmul_rn(t[c >> 2][c & 3], kHadNorm);
+            if (p.svh) v = __fmul_rn(v, (float)p.svh[c0 + c]);
+            o[c] = (half_t)v;
+            if (p.bias) o[c] = o[c] + p.bias[c0 + c];
+        }
+        half_t* dst = p.y + (size_t)(m0 + r) * n + c0;
+        *reinterpret_cast<half4_t*>(dst) = half4_t{o[0], o[1], o[2], o[3]};
+        *reinterpret_cast<half4_t*>(dst + 4) = half4_t{o[4], o[5], o[6], o[7]};
+    }
+}
+
+// Microseconds of one 128-deep step of a workgroup, measured at 16..333 rows of 5120 x 10240,
+// 17408 x 5120, 5120 x 34816 (K = 4): a CU holds two workgroups of up to 64 rows or one of more.
+static double rows_step_us(int mr, bool pair) {
+    if (mr == 1) return pair ? 1.1 : 0.70;
+    if (mr == 2) return pair ? 1.27 : 0.73;
+    return mr == 3 ? 0.92 : 1.02;
+}
+constexpr double kRowsFillSteps = 5;      // pipeline fill and reduction of a workgroup
+constexpr double kRowsPostUs = 3;         // launch of the pass that adds the ranges
+constexpr double kRowsPartialRate = 8e6;  // bytes of partial rows written and read back per us
+
+LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups) {
+    LinRowsPlan p{};
+    p.n_row_blocks = (rows + 127) / 128;
+    p.block_rows = (rows + p.n_row_blocks - 1) / p.n_row_blocks;
+    p.mr = (p.block_rows + 31) / 32;
+    const int steps = in_tiles / 8;
+    p.n_splits = 1;
+    p.steps_per_split = steps;
+    p.us = 1e30;
+    for (int s = 1; s <= 16 && (s == 1 || steps / s >= 2); s++) {
+        const int per = (steps + s - 1) / s;
+        if ((steps + per - 1) / per != s) continue;  // some range would be empty
+        const long long n = (long long)p.n_row_blocks * n_groups * s;
+        double us;  // per step of all workgroups
+        if (p.mr <= 2)
+            us = n <= 256 ? rows_step_us(p.mr, false)
+                          : rows_step_us(p.mr, true) * (n <= 512 ? 1.0 : (double)n / 512 + 0.15);
+        else
+            us = rows_step_us(p.mr, false) * (double)((n + 255) / 256);
+        us *= per + kRowsFillSteps;
+        if (s > 1) us += kRowsPostUs + (double)s * rows * n_groups * 128 * 8 / kRowsPartialRate;
+        if (us < p.us) {
+            p.us = us;
+            p.n_splits = s;
+            p.steps_per_split = per;
+        }
+    }
+    return p;
+}
+
+// Whether the layer takes this kernel rather than the prefill GEMM, which has larger tiles (256
+// columns and up to 256 rows): estimated time against the GEMM's schedule. Measured (layer,
+// before -> now, us): 5120 -> 10240 at 77 rows 41.1 -> 28.8, 333 rows 80.9 -> 60.1; 17408 -> 5120
+// (K = 5) at 333 rows 115 -> 97; 2048 -> 2048 at 256 rows 34.3 -> 22.0. The GEMM keeps 5120 ->
+// 34816 at 128 rows (90 against 98) and 17408 -> 5120 at 512 (125 against 137).
+bool linear_rows_applies(int rows, int in_tiles, int out_tiles) {
+    static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
+    // fewer than four 128-deep steps do not fill the three stages of the pipeline
+    if (rows < 1 || rows > max_rows || in_tiles < 32 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8) return false;
+    // by a tenth, which is how far the two estimates are off
+    return rows <= kLinearMidMaxRows || plan_linear_rows(rows, in_tiles, out_tiles / 8).us <
+                                            0.9 * gemm_estimate_us(rows, in_tiles, out_tiles);
+}
+
+size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups) {
+    const LinRowsPlan p = plan_linear_rows(rows, in_tiles, n_groups);
+    return p.n_splits > 1 ? (size_t)p.n_splits * rows * n_groups * 128 * sizeof(float) : 0;
+}
+
+int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
+                       int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
+                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream) {
+    if (int rc = check_k_cb(K, cb)) return rc;
+    if (!xh || !trellis || !y) return EXL3_E_NULL_POINTER;
+    if (rows < 1 || in_tiles < 8 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8 || ldx % 8 ||
+        ldx < (size_t)in_tiles * 16 || ldx * 2 * 128 >= (1ull << 31))  // 32-bit row offsets inside a block
+        return EXL3_E_BAD_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(xh) & 15) || (reinterpret_cast<uintptr_t>(trellis) & 15) ||
+        (reinterpret_cast<uintptr_t>(y) & 7))
+        return EXL3_E_BAD_SHAPE;
+    const int n_groups = out_tiles / 8;
+    const LinRowsPlan plan = plan_linear_rows(rows, in_tiles, n_groups);
+    if (plan.n_splits > 1 && (!partial || (reinterpret_cast<uintptr_t>(partial) & 15))) return EXL3_E_WORKSPACE;
+    const long long units = (long long)n_groups * plan.n_splits;
+    const long long grid = (units + 7) / 8 * 8 * plan.n_row_blocks;
+    if (grid > 0x7FFFFFFFLL) return EXL3_E_BAD_SHAPE;
+    auto H_ = [](const uint16_t* q) { return reinterpret_cast<const half_t*>(q); };
+    const LinRowsArgs a{reinterpret_cast<const uint32_t*>(trellis), H_(xh), H_(svh), H_(bias),
+                        reinterpret_cast<half_t*>(y), partial, group_sub, ldx, sub_stride, rows,
+                        plan.block_rows, plan.n_row_blocks, (int)units, plan.n_splits, plan.steps_per_split,
+                        in_tiles / 8, out_tiles};
+    const int rc = dispatch_k_cb(K, cb, [&](auto k, auto c) {
+        auto go = [&](auto mrc) {
+            constexpr int MR = mrc.value;
+            constexpr size_t stages = (size_t)3 * (RowsTile<MR, 4>::STAGE * 2 + 8 * RowsWords<k.value>::STAGE * 4),
+                             exchange = (size_t)8 * MR * 4 * 64 * 16;
+            constexpr size_t bytes = stages > exchange ? stages : exchange;
+            static_assert(bytes >= (size_t)32 * MR * kLinRowsLd * 2, "the fp16 tile fits");
+            auto kernel = linear_rows_kernel<k.value, c.value, MR>;
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
+                return (int)EXL3_E_LAUNCH;
+            kernel<<<dim3((unsigned)grid), dim3(kLinRowsThreads), bytes, stream>>>(a);
+            return launch_status();
+        };
+        switch (plan.mr) {
+            case 1: return go(std::integral_constant<int, 1>{});
+            case 2: return go(std::integral_constant<int, 2>{});
+            case 3: return go(std::integral_constant<int, 3>{});
+            default: return go(std::integral_constant<int, 4>{});
+        }
+    });
+    if (rc != EXL3_OK || plan.n_splits == 1) return rc;
+    return launch_had_post(partial, 1, plan.n_splits, (size_t)rows * out_tiles * 16, rows, out_tiles * 16, svh, bias,
+                           y, stream);
+}
+
+}  // namespace exl3

@@ -1211,7 +1211,8 @@ EXL3_EXPORT int exl3_moe_prefill(const uint16_t* x, int tokens, const int32_t* i
     const MoePrefillWorkspace w = moe_prefill_workspace(N, E, D, H);
     if (workspace_bytes < w.total) return EXL3_E_WORKSPACE;
     for (const void* p : {(const void*)workspace, (const void*)y, (const void*)gu_svh, (const void*)dn_suh,
-                          (const void*)dn_svh, (const void*)x, (const void*)gu_suh})
+                          (const void*)dn_svh, (const void*)x, (const void*)gu_suh, (const void*)gu_trellis,
+                          (const void*)dn_trellis})
         if (reinterpret_cast<uintptr_t>(p) & 15) return EXL3_E_BAD_SHAPE;
     char* base = static_cast<char*>(workspace);
     int* order = reinterpret_cast<int*>(base + w.o_tables);

@@ -88,9 +88,8 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
 
     const int proj = wave >> 2, cq = (wave >> 1) & 1, ks = wave & 1;
     const size_t row_words = (size_t)E * 2 * (H >> 4) * (8 * K);
-    const uint32_t* w = trellis + (size_t)(2 * ks + (lane >> 5)) * row_words +
-                        ((size_t)(proj * E + e) * (H >> 4) + hg * 8 + cq * 4 + ((lane >> 3) & 3)) * (8 * K) +
-                        (lane & 7) * K;
+    const uint32_t* w = trellis + (size_t)(2 * ks) * row_words +
+                        ((size_t)(proj * E + e) * (H >> 4) + hg * 8 + cq * 4) * (8 * K);
     half_t* stages = reinterpret_cast<half_t*>(lds) + proj * 3 * T::STAGE;
     uint32_t a_off[LPW];
 #pragma unroll
@@ -102,9 +101,12 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
         for (int cs = 0; cs < 2; cs++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
-    rows_main<K, CB, MR, 2, LPW>(w, 4 * row_words, reinterpret_cast<const char*>((proj ? xu : xg) + (size_t)m0 * D),
-                                 a_off, true, lds_byte_address(stages) + (wave & 3) * LPW * 1024,
-                                 stages, rows_read_base<MR, 2>(ks, lane), D >> 6, lane, acc);
+    uint32_t* words = reinterpret_cast<uint32_t*>(reinterpret_cast<half_t*>(lds) + 2 * 3 * T::STAGE) +
+                      wave * RowsWords<K>::STAGE;
+    rows_main<K, CB, MR, 2, LPW>(w, row_words, 4 * row_words,
+                                 reinterpret_cast<const char*>((proj ? xu : xg) + (size_t)m0 * D), a_off, true,
+                                 lds_byte_address(stages) + (wave & 3) * LPW * 1024, stages,
+                                 rows_read_base<MR, 2>(ks, lane), words, 8 * RowsWords<K>::STAGE, D >> 6, lane, acc);
 
     float16_t sum[MR];
     rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
@@ -231,9 +233,8 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
 
     const int cq = wave >> 1, ks = wave & 1;
     const size_t row_words = (size_t)E * (D >> 4) * (8 * K);
-    const uint32_t* w = trellis + (size_t)(2 * ks + (lane >> 5)) * row_words +
-                        ((size_t)e * (D >> 4) + g * 16 + (full ? cq : cq & 1) * 4 + ((lane >> 3) & 3)) * (8 * K) +
-                        (lane & 7) * K;
+    const uint32_t* w = trellis + (size_t)(2 * ks) * row_words +
+                        ((size_t)e * (D >> 4) + g * 16 + (full ? cq : cq & 1) * 4) * (8 * K);
     half_t* stages = reinterpret_cast<half_t*>(lds);
     uint32_t a_off[LPW];
 #pragma unroll
@@ -245,9 +246,10 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
         for (int cs = 0; cs < 2; cs++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
-    rows_main<K, CB, MR, 2, LPW>(w, 4 * row_words, reinterpret_cast<const char*>(xd + (size_t)m0 * H), a_off,
-                                 wave * LPW < T::FILLS, lds_byte_address(stages) + wave * LPW * 1024,
-                                 stages, rows_read_base<MR, 2>(ks, lane), H >> 6, lane, acc);
+    uint32_t* words = reinterpret_cast<uint32_t*>(stages + 3 * T::STAGE) + wave * RowsWords<K>::STAGE;
+    rows_main<K, CB, MR, 2, LPW>(w, row_words, 4 * row_words, reinterpret_cast<const char*>(xd + (size_t)m0 * H),
+                                 a_off, wave * LPW < T::FILLS, lds_byte_address(stages) + wave * LPW * 1024, stages,
+                                 rows_read_base<MR, 2>(ks, lane), words, 8 * RowsWords<K>::STAGE, H >> 6, lane, acc);
     float16_t sum[MR];
     rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
     half_t* tile = reinterpret_cast<half_t*>(lds);  // [BM][kLd]
@@ -282,9 +284,9 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
     });
 }
 
-template <int MR>
+template <int K, int MR>
 static constexpr size_t rows_lds_bytes(int tiles, int tile_cols) {
-    const size_t stages = (size_t)tiles * 3 * RowsTile<MR, 2>::STAGE * 2;
+    const size_t stages = (size_t)3 * (tiles * RowsTile<MR, 2>::STAGE * 2 + 8 * RowsWords<K>::STAGE * 4);
     const size_t exchange = (size_t)8 * MR * 4 * 64 * 16;
     const size_t y = (size_t)tiles * RowsTile<MR, 2>::BM * (tile_cols + kYPad) * 2;
     return stages > exchange ? (stages > y ? stages : y) : (exchange > y ? exchange : y);
@@ -303,7 +305,7 @@ int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const ui
     return dispatch_k_cb(K, cb, [&](auto k, auto c) {
         auto go = [&](auto mrc) {
             constexpr int MR = mrc.value;
-            constexpr size_t gu_lds = rows_lds_bytes<MR>(2, 128), dn_lds = rows_lds_bytes<MR>(1, 256);
+            constexpr size_t gu_lds = rows_lds_bytes<k.value, MR>(2, 128), dn_lds = rows_lds_bytes<k.value, MR>(1, 256);
             auto gu = moe_gateup_rows_kernel<k.value, c.value, MR>;
             auto dn = moe_down_rows_kernel<k.value, c.value, MR>;
             if (hipFuncSetAttribute(reinterpret_cast<const void*>(gu), hipFuncAttributeMaxDynamicSharedMemorySize,

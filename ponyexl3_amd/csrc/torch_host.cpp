@@ -155,6 +155,15 @@ void linear_run(const LinearLayer& l, const at::Tensor& x, int64_t rows64, const
         check_status((fused ? exl3_rotate : exl3_had128_pre)(xp, rows, n_in, half_ptr(l.suh), l.n_sub, half_out(xh),
                                                              ctx.stream),
                      "exl3_rotate");
+        if (fused && l.group_sub.defined() && exl3_linear_rows_applies(tr, rows, l.in_tiles, l.out_tiles)) {
+            const size_t bytes = exl3_linear_rows_workspace_bytes(rows, n_in, n_out);
+            void* ws = bytes ? ctx.get(kWorkspace, bytes).mutable_data_ptr() : nullptr;
+            check_status(exl3_linear_rows(half_ptr(xh), rows, l.n_sub, tr, l.in_tiles, l.out_tiles, l.k, l.cb,
+                                          int_ptr(l.group_sub), half_ptr(l.svh), half_ptr(l.bias), yp, ws, bytes,
+                                          ctx.stream),
+                         "exl3_linear_rows");
+            return;
+        }
         if (one_launch) {
             // one GEMM launch over all members, each block reading its member's rotation, then
             // the output transform
@@ -327,7 +336,10 @@ void experts_run(const ExpertStack& m, const at::Tensor& x, const at::Tensor& in
     if (tokens * top_k > INT32_MAX) value_error("too many (token, slot) pairs");
     const int E = m.experts(), D = m.dim(), H = m.hidden(), kk = static_cast<int>(top_k);
     StreamContext ctx(x.device().index());
-    if (prefill) {
+    // (the prefill kernels copy trellis words 16 bytes at a time)
+    const bool aligned = !((reinterpret_cast<uintptr_t>(m.gu_trellis.const_data_ptr()) |
+                            reinterpret_cast<uintptr_t>(m.dn_trellis.const_data_ptr())) & 15);
+    if (prefill && aligned) {
         const int t = static_cast<int>(tokens);
         const at::Tensor& ws = ctx.get(kWorkspace, exl3_moe_prefill_workspace_bytes(t, kk, E, D, H));
         check_status(exl3_moe_prefill(half_ptr(x), t, int_ptr(indices), kk, half_ptr(m.gu_trellis), half_ptr(m.gu_suh),

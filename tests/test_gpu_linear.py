@@ -543,3 +543,46 @@ def test_two_streams_do_not_share_scratch(cuda):
     assert ws1 != ws2
     assert all(torch.equal(o, ref_a) for o in outs_a)
     assert all(torch.equal(o, ref_b) for o in outs_b)
+
+
+@pytest.mark.parametrize("rows,k,cb,n_in,outs", [
+    (1, 4, 0, 128, (128,)),              # one step, one column group
+    (32, 1, 1, 256, (128, 256)),         # a full 32-row tile; two rotations
+    (33, 2, 2, 512, (384, 128, 128)),    # members that end on odd 128-column blocks
+    (64, 3, 0, 1152, (1152,)),           # nine steps, nine groups: last set of eight ragged
+    (65, 5, 1, 2048, (256,)),            # split reduction, three tiles
+    (97, 6, 0, 1920, (128, 128)),        # fifteen steps, ranges of unequal length
+    (128, 7, 2, 640, (256,)),
+    (129, 8, 1, 512, (128,)),            # two row blocks of 65 and 64 rows
+    (300, 4, 1, 4096, (256, 256)),       # three row blocks, deep split
+    (1024, 4, 0, 256, (128,)),           # the most rows
+])
+def test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
+    """The kernel that takes a few dozen rows from registers into the matrix pipe: edges of its
+    row tiles, column groups, ranges and row blocks, every K, bias on and off. fp16 outputs of
+    fp16 rotated activations: the bar of the other layer tests."""
+    from ponyexl3_amd import _lib, make_exl3_layer, ops
+
+    lib = _lib.load()
+    layers = [make_exl3_layer(k=k, in_features=n_in, out_features=o, seed=700 + rows + i, mcg=cb == 1, mul1=cb == 2,
+                              bias=rows % 2 == 1) for i, o in enumerate(outs)]
+    tr = torch.cat([ops.as_trellis_tensor(l.trellis, cuda) for l in layers], dim=1).contiguous()
+    cat = lambda name: torch.cat([torch.from_numpy(getattr(l, name)).to(cuda) for l in layers])
+    suh = torch.stack([torch.from_numpy(l.suh).to(cuda) for l in layers])
+    svh, bias = cat("svh"), cat("bias") if layers[0].bias is not None else None
+    sub = torch.tensor([i for i, o in enumerate(outs) for _ in range(o // 128)], dtype=torch.int32, device=cuda)
+    x, xt = _x(np.random.default_rng(rows), (rows, n_in), cuda)
+    n_out = sum(outs)
+    xh = ops.had128_pre(xt, suh).contiguous()
+    need = lib.exl3_linear_rows_workspace_bytes(rows, n_in, n_out)
+    ws = torch.empty((max(need, 1),), dtype=torch.uint8, device=cuda)
+    y = torch.full((rows + 1, n_out), 7.0, dtype=torch.float16, device=cuda)
+    args = (ops._ptr(xh), rows, len(outs), ops._ptr(tr), n_in // 16, n_out // 16, k, cb, ops._ptr(sub), ops._ptr(svh),
+            ops._ptr(bias) if bias is not None else None, ops._ptr(y), ops._ptr(ws))
+    print(f"rows kernel rows={rows} k={k} cb={cb} {n_in}->{outs}", flush=True)
+    _lib.check(lib.exl3_linear_rows(*args, need, ops._stream()), "exl3_linear_rows")
+    assert bool((y[rows] == 7.0).all())
+    for l, part in zip(layers, torch.split(y[:rows], list(outs), dim=-1)):
+        assert rel_l2(part.cpu().numpy(), _oracle_forward(oracle, l, x)) <= TOL
+    if need:
+        assert lib.exl3_linear_rows(*args, need - 1, ops._stream()) == _lib.EXL3_E_WORKSPACE
