@@ -3,7 +3,6 @@
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 
-#include <algorithm>
 #include <mutex>
 
 namespace exl3 {
@@ -126,7 +125,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
                           : launch_had_pre(x, rows, in_features, suh, n_sub, xh, s))
         return rc;
     if (counters && (n_sub == 1 || rows <= kLinearMidMaxRows) && rows_aligned(trellis) &&
-        rows > std::min(kLinearMidPreferredRows, linear_mid_max_rows()) &&
+        (rows > linear_mid_max_rows() || linear_rows_before_mid(rows, K, in_tiles, out_tiles)) &&
         linear_rows_applies(rows, in_tiles, out_tiles))
         return launch_linear_rows(xh, rows, (size_t)n_sub * in_features, (size_t)in_features, trellis, in_tiles,
                                   out_tiles, K, cb, n_sub > 1 ? group_sub : nullptr, svh, bias, y,

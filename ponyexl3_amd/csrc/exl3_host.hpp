@@ -96,10 +96,16 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
 // [rows][n_sub][in]: weights decoded once and fed to 16x16x16 MFMA from registers;
 // partial: fp32 [plan.n_splits][rows][out]; counters as for launch_linear_small.
 constexpr int kLinearMidMaxRows = 32;
-// From here up the rows kernel (below) is faster where it can run (16-byte aligned trellis): 32
-// rows of 5120 -> 10240 26.2 -> 22.6 us, 17408 -> 5120 (K = 5) 42.6 -> 30.1; at 16 rows of 5120 ->
-// 10240 and 2048 -> 2048 it takes 22.7 and 13.1 us against 20.7 and 11.6 here.
-constexpr int kLinearMidPreferredRows = 16;
+// Whether the rows kernel (below) is faster, where it can run (16-byte aligned trellis). Above 16
+// rows always: 32 rows of 5120 -> 10240 26.2 -> 22.6 us (K = 4), 17408 -> 5120 42.6 -> 30.1 (K = 5).
+// Up to 16 rows from K = 5 on, where a lane of the medium-batch kernel needs three dwords for its
+// eight codewords (16 rows: 17408 -> 5120 at K = 6 36.3 -> 28.7, 5120 -> 34816 at K = 7 59.8 -> 52.1,
+// 14336 -> 4096 at K = 8 30.1 -> 25.8), and where few column groups share a long reduction (8192 ->
+// 2048 at K = 4 17.3 -> 14.1, 4096 -> 1024 at K = 3 13.3 -> 11.7); else not (5120 -> 34816 at K = 4
+// 42.6 against 46.5, 2048 -> 8192 13.3 against 14.6).
+inline bool linear_rows_before_mid(int rows, int K, int in_tiles, int out_tiles) {
+    return rows > 16 || K >= 5 || in_tiles >= 2 * out_tiles;
+}
 struct MidPlan {
     int n_splits;          // workgroups per 128-column group
     int blocks_per_split;  // 128-row blocks of the reduction per workgroup
