@@ -51,10 +51,11 @@ const char *exl3_status_string(int status);
 /* Largest row count the small-batch kernel (exl3_gemv) accepts per call. */
 int exl3_gemv_max_rows(void);
 
-/* Largest row count exl3_linear_forward serves with its small- and medium-batch
- * kernels when given counters (stacked suh included; above exl3_gemv_max_rows()
- * the input rotation runs as a launch of its own first). Beyond it the prefill
- * GEMM takes over. */
+/* Largest row count exl3_linear_forward serves with its small-batch, medium-batch and
+ * rows kernels for stacked suh too when given counters (above exl3_gemv_max_rows()
+ * the input rotation runs as a launch of its own first). Beyond it the rows kernel or
+ * the prefill GEMM takes plain layers, exl3_linear_rows and exl3_linear_prefill
+ * stacked ones. */
 int exl3_linear_small_max_rows(void);
 
 /*
@@ -270,7 +271,7 @@ size_t exl3_gemm_workspace_bytes(int rows, int in_tiles, int tn_count);
  *            and results are run-to-run deterministic. Above that and up to
  *            exl3_linear_small_max_rows() rows the array serves the medium-batch
  *            kernel as group counters (counters_len >= out/128; two launches: input
- *            rotation, then everything else). NULL selects the three-launch chain
+ *            rotation, then everything else), unless the rows kernel is faster. NULL selects the three-launch chain
  *            (exl3_had128_pre, exl3_gemv_partials, exl3_had128_post) resp. the
  *            prefill GEMM.
  *            Status word: when counters_len is at least two ints more than the call

@@ -126,10 +126,12 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
         return rc;
     if (counters && (n_sub == 1 || rows <= kLinearMidMaxRows) && rows_aligned(trellis) &&
         (rows > linear_mid_max_rows() || linear_rows_before_mid(rows, K, in_tiles, out_tiles)) &&
-        linear_rows_applies(rows, in_tiles, out_tiles))
+        linear_rows_applies(rows, in_tiles, out_tiles)) {
+        if (rows <= linear_mid_max_rows() && counters_len < (size_t)(out_tiles / 8)) return EXL3_E_WORKSPACE;
         return launch_linear_rows(xh, rows, (size_t)n_sub * in_features, (size_t)in_features, trellis, in_tiles,
                                   out_tiles, K, cb, n_sub > 1 ? group_sub : nullptr, svh, bias, y,
                                   reinterpret_cast<float*>(second), s);
+    }
     if (counters && rows <= linear_mid_max_rows()) {
         // a few dozen rows: the decode still sets the pace; every weight is decoded
         // once and goes from registers into 16x16x32 MFMA; split reduction and output

@@ -309,7 +309,8 @@ def gemv_max_rows() -> int:
 
 def linear_small_max_rows() -> int:
     """Rows up to which ``linear_forward(fused=True)`` uses the small- and
-    medium-batch kernels (stacked ``suh`` included); above it the prefill GEMM runs."""
+    medium-batch kernels (stacked ``suh`` included); above it the rows kernel or the prefill GEMM
+    runs."""
     return int(_lib.load().exl3_linear_small_max_rows())
 
 
@@ -579,8 +580,8 @@ def linear_forward(x2d, trellis, k, cb, suh=None, svh=None, bias=None, group_sub
     """Whole-layer forward on (rows, in) fp16 (``exl3_linear_forward``).
     ``fused=False`` selects the three-launch chain for small batches.
     ``member_out`` (out_features of each sibling, in order) is needed for a
-    sibling-fused group above ``linear_small_max_rows()`` rows: the prefill GEMM runs once
-    per member over its tile columns, each on its own rotated activations
+    sibling-fused group above ``linear_small_max_rows()`` rows where the rows kernel does not
+    apply: the prefill GEMM runs once per member over its tile columns, each on its own rotated activations
     (``FusedEXL3Group.forward_all``, ponyexl3/mlx/exl3_fused.py:136-202), or once
     over all members when each has ``out_features % 256 == 0`` (``block_sub``: the
     member index of every 256-column block, derived from ``group_sub`` if absent)."""
