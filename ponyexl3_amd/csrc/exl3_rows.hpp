@@ -1,6 +1,6 @@
 // Building blocks of the kernels that take a few dozen rows at a time: the weights go from
-// the trellis through registers straight into v_mfma_f32_32x32x16_f16, only the activations
-// pass through LDS.
+// the trellis through registers straight into v_mfma_f32_32x32x16_f16; activations and packed
+// words pass through LDS, decoded weights do not.
 //
 // Geometry. A wave decodes 64 columns x 32 reduction rows per step: lanes 0..31 hold four
 // tiles of one tile row, lanes 32..63 the same four tile columns of the next one, 32
