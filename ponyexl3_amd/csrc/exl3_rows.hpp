@@ -238,6 +238,52 @@ struct HadamardColumns {
 
 constexpr float kHadNorm = 0.088388347648318440550f;  // 1/sqrt(128)
 
+// Whether the scale values of all lanes are +-1, eight halfs at a time (packed sign words, the
+// usual case): a sign flip on fp16 bits is then all the product needs.
+template <int N>
+__device__ __forceinline__ bool all_plain_signs(const uint4_t (&s)[N]) {
+    uint32_t not_one = 0;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const uint4_t m = (s[k] & 0x7FFF7FFFu) ^ 0x3C003C00u;
+        not_one |= m.x | m.y | m.z | m.w;
+    }
+    return __ballot(not_one != 0) == 0;
+}
+
+// Unnormalised Hadamard-128 in fp32 on the layout of HadamardColumns: v[k][t] = element 32 k +
+// 8 (lane >> 4) + t of row lane & 15. Stages in the order of the element bits, a + b and a - b
+// each: the bits of wht128_lanes() and wht128_wide(). For rows whose scale vector is general: a
+// product of two halfs has 22 bits and reaches 2^32, which no pair of halfs holds (a high part
+// above 65504 is infinite, a low part below 2^-24 is lost).
+__device__ __forceinline__ void wht128_tile(float (&v)[4][8]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+#pragma unroll
+        for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+            for (int t = 0; t < 8; t++)
+                if ((t & h) == 0) butterfly_in_lane(v[k][t], v[k][t + h]);
+#pragma unroll
+        for (int t = 0; t < 8; t += 2) {
+            swap_rows16(v[k][t], v[k][t + 1]);
+            butterfly_in_lane(v[k][t], v[k][t + 1]);
+            swap_halves32(v[k][t], v[k][t + 1]);
+            butterfly_in_lane(v[k][t], v[k][t + 1]);
+            swap_halves32(v[k][t], v[k][t + 1]);
+            swap_rows16(v[k][t], v[k][t + 1]);
+        }
+    }
+#pragma unroll
+    for (int h = 1; h < 4; h <<= 1)
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if ((k & h) == 0) {
+#pragma unroll
+                for (int t = 0; t < 8; t++) butterfly_in_lane(v[k][t], v[k + h][t]);
+            }
+}
+
 // fp16 pair (hi, lo) with hi + lo = v up to the last bits of a 22-bit product
 __device__ __forceinline__ void split_halves(float v, half_t& hi, half_t& lo) {
     hi = (half_t)v;

@@ -111,12 +111,12 @@ __global__ __launch_bounds__(256) void had_pre_wide_kernel(const half_t* __restr
 }
 
 // Input side on the matrix pipe: a wave rotates 16 rows x one 128-wide block, for
-// subs_per_wave of the stacked siblings from one read of x, against entries +-1 with fp32 sums
-// (the fp32 butterfly's result up to the order of the additions). Plain signs (packed sign
-// words, the usual case) are applied to the fp16 bits of x; general scale vectors give
-// products of 22 bits, which enter exactly as a high and a low fp16 part. 32 (64) matrix
-// instructions of 16 cycles and 2 (6) VALU instructions per element replace about 18: the
-// butterfly form is bound by VALU issue.
+// subs_per_wave of the stacked siblings from one read of x. Plain signs (packed sign words, the
+// usual case) are applied to the fp16 bits of x and the block is contracted with entries +-1,
+// fp32 sums (the fp32 butterfly's result up to the order of the additions): 32 matrix
+// instructions of 16 cycles and 2 VALU instructions per element replace about 18, which the
+// butterfly form is bound by. With any other scale value among the wave's rows the products
+// need fp32: the butterfly then runs in this kernel, with the bits of the kernels above.
 // Row maps (MoE rows sorted by expert): row r is pair p = pair[r] of token p / top_k and
 // expert pair_expert[p], whose scales are scale_ld halfs from the next expert's; entries
 // outside the buffers are clamped.
@@ -160,43 +160,36 @@ __global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
         float4_t z[8];
 #pragma unroll
         for (int nt = 0; nt < 8; nt++) z[nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-        auto contract = [&](auto k, half8_t v) {
-            static_for<0, 8>([&](auto nt) {
-                z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(), v,
-                                                                     z[nt.value], 0, 0, 0);
-            });
-        };
         uint4_t sv[4];
-        uint32_t not_one = 0;
         if (a.suh) {
             const half_t* sr = a.suh + (size_t)scale_row * a.scale_ld + (size_t)s * a.sub_scale + col;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                sv[k] = *reinterpret_cast<const uint4_t*>(sr + k * 32);
-                const uint4_t m = (sv[k] & 0x7FFF7FFFu) ^ 0x3C003C00u;
-                not_one |= m.x | m.y | m.z | m.w;
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; k++) sv[k] = uint4_t{0u, 0u, 0u, 0u};
+            for (int k = 0; k < 4; k++) sv[k] = *reinterpret_cast<const uint4_t*>(sr + k * 32);
         }
-        if (__ballot(not_one != 0) == 0) {
+        if (!a.suh || all_plain_signs(sv)) {
             static_for<0, 4>([&](auto k) {
-                contract(k, __builtin_bit_cast(half8_t, xv[k.value] ^ (sv[k.value] & 0x80008000u)));
+                const uint4_t flip = a.suh ? sv[k.value] & 0x80008000u : uint4_t{0u, 0u, 0u, 0u};
+                const half8_t v = __builtin_bit_cast(half8_t, xv[k.value] ^ flip);
+                static_for<0, 8>([&](auto nt) {
+                    z[nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(had.template get<nt.value, k.value>(), v,
+                                                                         z[nt.value], 0, 0, 0);
+                });
             });
         } else {
-            static_for<0, 4>([&](auto k) {
-                const half8_t x8 = __builtin_bit_cast(half8_t, xv[k.value]), s8 = __builtin_bit_cast(half8_t, sv[k.value]);
-                half8_t hi, lo;
+            float v[4][8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float p = __builtin_fmaf((float)x8[j], (float)s8[j], -0.0f);
-                    hi[j] = (half_t)p;
-                    lo[j] = (half_t)__builtin_fmaf((float)hi[j], -1.0f, p);
-                }
-                contract(k, hi);
-                contract(k, lo);
-            });
+            for (int k = 0; k < 4; k++) {
+                float scale[8];
+                halfs_to_floats(xv[k], v[k]);
+                halfs_to_floats(sv[k], scale);
+#pragma unroll
+                for (int t = 0; t < 8; t++) v[k][t] = v[k][t] * scale[t];
+            }
+            wht128_tile(v);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int t = 0; t < 8; t++) z[2 * k + (t >> 2)][t & 3] = v[k][t];
         }
         if (valid) {
             half_t* o = a.out + (size_t)s * a.sub_stride + (size_t)r * a.row_stride + col;

@@ -82,6 +82,39 @@ def test_wide_and_narrow_kernels_give_the_same_bits(cuda, oracle):
     assert rel_l2(ops.had128_post(xt, vt).cpu().numpy(), ref) < 3e-4
 
 
+@pytest.mark.parametrize("rows,n,n_sub", [(64, 128, 1), (77, 640, 3), (256, 384, 2)])
+@pytest.mark.parametrize("scale,x_std", [(1.0, 1.0), (60.0, 3000.0), (1e-3, 1e-3)])
+def test_layer_rotation_with_general_scales(cuda, oracle, rows, n, n_sub, scale, x_std):
+    """The layer forwards rotate 64 rows and more on the matrix pipe; scale vectors that are not
+    +-1 take the fp32 butterfly there, so the bits are those of the separate entry point:
+    products past the fp16 range (6e4 * 60 and more), products of a few subnormals, infinite x."""
+    import ctypes
+
+    from ponyexl3_amd import _lib, ops
+
+    rng = np.random.default_rng(rows + n)
+    x = np.clip(rng.standard_normal((rows, n)) * x_std, -6e4, 6e4).astype(np.float16)
+    x[0, 3] = np.inf  # one per block at most: an output is the infinity with a sign
+    suh = (np.where(rng.random((n_sub, n)) > 0.5, -1, 1) * rng.uniform(0.5, 2, (n_sub, n)) * scale).astype(np.float16)
+    suh[:, 128 * (n // 256):128 * (n // 256) + 128] = np.sign(suh[:, :128])  # a block with plain signs
+    xt, st = _t(x, cuda), _t(suh, cuda)
+    got = torch.empty((rows, n_sub, n), dtype=torch.float16, device=cuda)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    print(f"rotate rows={rows} n={n} n_sub={n_sub} scale={scale}", flush=True)
+    _lib.check(_lib.load().exl3_rotate(p(xt), rows, n, p(st), n_sub, p(got), ops._stream()), "exl3_rotate")
+    ref = ops.had128_pre(xt, st)
+    assert not bool(torch.isnan(got).any())
+    plain = (st.abs() == 1).reshape(n_sub, n // 128, 128).all(-1).repeat_interleave(128, dim=-1).expand_as(got)
+    assert torch.equal(got[~plain].view(torch.int16), ref[~plain].view(torch.int16))
+    # plain signs: fp32 sums in another order, one fp16 rounding
+    d = (got - ref)[plain & torch.isfinite(ref)].double().norm()
+    assert not bool(plain.any()) or float(d) <= 3e-4 * float(ref[plain & torch.isfinite(ref)].double().norm())
+    with np.errstate(over="ignore"):
+        exact = oracle.had_r_128(x[1:].astype(np.float32), pre_scale=suh[0]).astype(np.float16)
+    ok = np.isfinite(exact)
+    assert rel_l2(got[1:, 0].cpu().numpy()[ok], exact[ok]) < 3e-4 or scale < 1e-2  # subnormal results
+
+
 def test_involution_at_scale(cuda):
     """Size-independent property at prefill size: H(H(x)) == x, norms preserved."""
     from ponyexl3_amd import ops
