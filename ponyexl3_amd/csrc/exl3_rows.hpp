@@ -256,24 +256,26 @@ __device__ __forceinline__ bool all_plain_signs(const uint4_t (&s)[N]) {
 // each: the bits of wht128_lanes() and wht128_wide(). For rows whose scale vector is general: a
 // product of two halfs has 22 bits and reaches 2^32, which no pair of halfs holds (a high part
 // above 65504 is infinite, a low part below 2^-24 is lost).
+// wht32_tile: element bits 0..4, one column part; wht128_tile: all seven.
+__device__ __forceinline__ void wht32_tile(float (&v)[8]) {
+#pragma unroll
+    for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+            if ((t & h) == 0) butterfly_in_lane(v[t], v[t + h]);
+#pragma unroll
+    for (int t = 0; t < 8; t += 2) {
+        swap_rows16(v[t], v[t + 1]);
+        butterfly_in_lane(v[t], v[t + 1]);
+        swap_halves32(v[t], v[t + 1]);
+        butterfly_in_lane(v[t], v[t + 1]);
+        swap_halves32(v[t], v[t + 1]);
+        swap_rows16(v[t], v[t + 1]);
+    }
+}
 __device__ __forceinline__ void wht128_tile(float (&v)[4][8]) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-#pragma unroll
-        for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-            for (int t = 0; t < 8; t++)
-                if ((t & h) == 0) butterfly_in_lane(v[k][t], v[k][t + h]);
-#pragma unroll
-        for (int t = 0; t < 8; t += 2) {
-            swap_rows16(v[k][t], v[k][t + 1]);
-            butterfly_in_lane(v[k][t], v[k][t + 1]);
-            swap_halves32(v[k][t], v[k][t + 1]);
-            butterfly_in_lane(v[k][t], v[k][t + 1]);
-            swap_halves32(v[k][t], v[k][t + 1]);
-            swap_rows16(v[k][t], v[k][t + 1]);
-        }
-    }
+    for (int k = 0; k < 4; k++) wht32_tile(v[k]);
 #pragma unroll
     for (int h = 1; h < 4; h <<= 1)
 #pragma unroll
@@ -282,18 +284,6 @@ __device__ __forceinline__ void wht128_tile(float (&v)[4][8]) {
 #pragma unroll
                 for (int t = 0; t < 8; t++) butterfly_in_lane(v[k][t], v[k + h][t]);
             }
-}
-
-// fp16 pair (hi, lo) with hi + lo = v up to the last bits of a 22-bit product
-__device__ __forceinline__ void split_halves(float v, half_t& hi, half_t& lo) {
-    hi = (half_t)v;
-    lo = (half_t)(v - (float)hi);
-}
-
-// Eight halfs of a column block as bits, for the "all zero" test of a low part.
-__device__ __forceinline__ uint32_t any_bits(half8_t v) {
-    const uint4_t u = __builtin_bit_cast(uint4_t, v) & 0x7FFF7FFFu;
-    return u.x | u.y | u.z | u.w;
 }
 
 }  // namespace exl3

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
                 static_for<0, MR>([&](auto i) { f(std::integral_constant<int, p.value * MR + i.value>{}, i); });
         });
     };
-    half8_t hi[MR], lo[MR];
+    half8_t h[MR];
     {
         half8_t yg[4], yu[4];
 #pragma unroll
@@ -149,8 +149,7 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
             const int col = hg * 128 + a.value * 32 + q * 8;
             const half8_t sg = *reinterpret_cast<const half8_t*>(gu_svh + (size_t)e * 2 * H + col);
             const half8_t su = *reinterpret_cast<const half8_t*>(gu_svh + (size_t)e * 2 * H + H + col);
-            const half8_t ds = *reinterpret_cast<const half8_t*>(dn_suh + (size_t)e * H + col);
-            float zg[8], zu[8], h[8];
+            float zg[8], zu[8];
             transform(yg, a, zg);
             transform(yu, a, zu);
 #pragma unroll
@@ -160,52 +159,67 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
             }
             if (activation == 1) {
 #pragma unroll
-                for (int c = 0; c < 8; c++) h[c] = glu_act(zg[c], zu[c], 1);
+                for (int c = 0; c < 8; c++) h[i.value][c] = (half_t)glu_act(zg[c], zu[c], 1);
             } else {
 #pragma unroll
-                for (int c = 0; c < 8; c++) h[c] = glu_act(zg[c], zu[c], 0);
-            }
-#pragma unroll
-            for (int c = 0; c < 8; c++) {
-                half_t h0, h1;
-                split_halves((float)(half_t)h[c] * (float)ds[c], h0, h1);
-                hi[i.value][c] = h0;
-                lo[i.value][c] = h1;
+                for (int c = 0; c < 8; c++) h[i.value][c] = (half_t)glu_act(zg[c], zu[c], 0);
             }
         });
     }
+    uint4_t ds[4];  // the expert's scales of the block, in the layout of a row
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        ds[k] = *reinterpret_cast<const uint4_t*>(dn_suh + (size_t)e * H + hg * 128 + k * 32 + q * 8);
     __syncthreads();
     for_parts([&](auto a, auto i) {
-        half_t* dst = tile + (rt * 16 + fr) * kLd + a.value * 32 + q * 8;
-        *reinterpret_cast<half8_t*>(dst) = hi[i.value];
-        *reinterpret_cast<half8_t*>(dst + T::BM * kLd) = lo[i.value];
+        *reinterpret_cast<half8_t*>(tile + (rt * 16 + fr) * kLd + a.value * 32 + q * 8) = h[i.value];
     });
     __syncthreads();
-    half8_t yh[4], yl[4];
-    uint32_t low_bits = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        yh[k] = *reinterpret_cast<const half8_t*>(yrow + k * 32);
-        yl[k] = *reinterpret_cast<const half8_t*>(yrow + T::BM * kLd + k * 32);
-        low_bits |= any_bits(yl[k]);
-    }
-    const bool has_low = __ballot(low_bits != 0) != 0;  // never with plain signs: the product is exact
     const bool store = rt * 16 + fr < valid;
     half_t* out = xd + (size_t)(m0 + rt * 16 + fr) * H + hg * 128 + q * 8;
-    for_parts([&](auto a, auto) {
-        float z[8];
-        transform(yh, a, z);
-        if (has_low) {
-            float zl[8];
-            transform(yl, a, zl);
-#pragma unroll
-            for (int c = 0; c < 8; c++) z[c] = __fadd_rn(z[c], zl[c]);
-        }
+    auto put = [&](auto a, const float (&z)[8]) {
         half8_t o;
 #pragma unroll
         for (int c = 0; c < 8; c++) o[c] = (half_t)(z[c] * kHadNorm);
         if (store) *reinterpret_cast<half8_t*>(out + a.value * 32) = o;
-    });
+    };
+    if (all_plain_signs(ds)) {
+        half8_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = __builtin_bit_cast(half8_t, *reinterpret_cast<const uint4_t*>(yrow + k * 32) ^ (ds[k] & 0x80008000u));
+        for_parts([&](auto a, auto) {
+            float z[8];
+            transform(v, a, z);
+            put(a, z);
+        });
+    } else {
+        // in fp32: column part k of the row up to element bit 4, twice over, then bits 5 and 6
+        // for the wave's own parts
+        auto five_stages = [&](int k, float (&v)[8]) {
+            float scale[8];
+            halfs_to_floats(*reinterpret_cast<const uint4_t*>(yrow + k * 32), v);
+            halfs_to_floats(ds[k], scale);
+#pragma unroll
+            for (int t = 0; t < 8; t++) v[t] = v[t] * scale[t];
+            wht32_tile(v);
+        };
+        float z[MR][8];
+#pragma unroll
+        for (int i = 0; i < MR; i++) {
+            const int a = part * MR + i;
+            float t[2][8], u[8];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                five_stages(2 * half, t[half]);
+                five_stages(2 * half + 1, u);
+#pragma unroll
+                for (int c = 0; c < 8; c++) t[half][c] = a & 1 ? __fsub_rn(t[half][c], u[c]) : __fadd_rn(t[half][c], u[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < 8; c++) z[i][c] = a & 2 ? __fsub_rn(t[0][c], t[1][c]) : __fadd_rn(t[0][c], t[1][c]);
+        }
+        for_parts([&](auto a, auto i) { put(a, z[i.value]); });
+    }
 }
 
 // unit = (row block b, 256-column block g of D), XCD order as above; rows go to out[order[r]].

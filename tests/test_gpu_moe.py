@@ -420,6 +420,52 @@ def test_pair_sort_kernel_equals_stable_argsort(cuda, tokens, top_k, E, block_ro
     assert torch.equal(o2, order) and torch.equal(tab2, table)
 
 
+@pytest.mark.parametrize("tokens,k", [(40, 4), (200, 8)])  # row blocks of 32 and of 64
+@pytest.mark.parametrize("kind", ["general", "spikes", "small"])
+def test_prefill_rotation_with_general_scales(cuda, tokens, k, kind):
+    """The gate/up kernel of the prefill chain rotates the GLU's output for the down projection;
+    scales that are not +-1 need fp32 products: past the fp16 range (a spike of 1.5e4 per block)
+    they are finite, small ones keep all bits. Its result, the last part of the workspace,
+    against the separate launches, fp16 roundings of the same values up to the order of the
+    sums in gate and up; the experts with plain signs in between keep theirs."""
+    from ponyexl3_amd import EXL3SwitchGLU, _lib, ops
+
+    E, D, H, kk = 7, 256, 384, 2
+    moe = EXL3SwitchGLU.from_layers(*_experts(E, D, H, k, True, 5100))
+    rng = np.random.default_rng(tokens)
+    sign = lambda *s: np.where(rng.random(s) > 0.5, -1.0, 1.0)
+    dn_suh = sign(E, H) * (rng.uniform(0.5, 2, (E, H)) if kind != "spikes" else 1.0)
+    if kind == "spikes":
+        dn_suh[:, ::128] *= 1.5e4
+    elif kind == "small":
+        dn_suh *= 1e-3
+    dn_suh[E // 2] = sign(H)
+    moe._dn_suh = torch.from_numpy(dn_suh.astype(np.float16)).to(cuda)
+    moe._gu_suh = torch.from_numpy((sign(E, 2, D) * rng.uniform(0.5, 2, (E, 2, D))).astype(np.float16)).to(cuda)
+    x = torch.from_numpy((rng.standard_normal((tokens, D)) * 0.05).astype(np.float16)).to(cuda)
+    idx = torch.from_numpy(np.stack([rng.permutation(E)[:kk] for _ in range(tokens)]).astype(np.int32)).to(cuda)
+    lib, n = _lib.load(), tokens * kk
+    total = lib.exl3_moe_prefill_workspace_bytes(tokens, kk, E, D, H)
+    ws = torch.zeros((total,), dtype=torch.uint8, device=cuda)
+    y = torch.empty((tokens, kk, D), dtype=torch.float16, device=cuda)
+    p = ops._ptr
+    print(f"prefill rotation tokens={tokens} k={k} {kind}", flush=True)
+    _lib.check(lib.exl3_moe_prefill(p(x), tokens, p(idx), kk, p(moe._gu_trellis), p(moe._gu_suh), p(moe._gu_svh),
+                                    p(moe._dn_trellis), p(moe._dn_suh), p(moe._dn_svh), E, D, H, k, moe._cb, 0, None,
+                                    p(y), p(ws), total, ops._stream()), "exl3_moe_prefill")
+    got = ws[total - (n * H * 2 + 255) // 256 * 256:][:n * H * 2].view(torch.float16).view(n, H)
+    order, tok, sidx, table = ops.moe_sort(idx, E, 64)
+    xg = ops.had128_rows(x, moe._gu_suh[:, 0], False, in_index=tok, scale_index=sidx)
+    xu = ops.had128_rows(x, moe._gu_suh[:, 1], False, in_index=tok, scale_index=sidx)
+    g = ops.gemm_grouped(xg, moe._gu_trellis, k, moe._cb, 0, H // 16, E, table, 64)
+    u = ops.gemm_grouped(xu, moe._gu_trellis, k, moe._cb, E * H // 16, H // 16, E, table, 64)
+    ref = ops.moe_glu_rows(g, u, sidx, moe._gu_svh, moe._dn_suh, 0)
+    assert bool(torch.isfinite(ref).all()) and bool(torch.isfinite(got).all())
+    if kind == "spikes":
+        assert float(ref.abs().max()) * 128 ** 0.5 > 65504  # products past the fp16 range did occur
+    assert rel_l2(got.float().cpu().numpy(), ref.float().cpu().numpy()) <= TOL
+
+
 @pytest.mark.parametrize("act", [0, 1])
 def test_glu_rows_kernel_equals_separate_launches(cuda, act):
     """Finish gate/up + GLU + down rotation in one launch against the per-row
