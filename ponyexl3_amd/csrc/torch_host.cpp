@@ -435,10 +435,21 @@ PyObject* experts_slots(PyObject* self, PyObject* args) {
 // module: its kernel is made for one round trip to memory, not for throughput.
 constexpr int64_t kGateMaxTokens = 32;
 
-// The weight of a plain bias-free fp16 torch.nn.Linear without hooks, as exl3_moe_gate
-// takes it; undefined if `gate` is anything else.
-at::Tensor plain_gate_weight(PyObject* gate, PyObject* linear_class, int D) {
-    if (reinterpret_cast<PyObject*>(Py_TYPE(gate)) != linear_class) return {};
+PyObject* linear_module_class() {
+    static PyObject* cls = [] {
+        PyObject* nn = PyImport_ImportModule("torch.nn");
+        PyObject* c = nn ? PyObject_GetAttrString(nn, "Linear") : nullptr;
+        Py_XDECREF(nn);
+        return c;
+    }();
+    if (!cls) throw python_error();
+    return cls;
+}
+
+// The weight of a plain bias-free fp16 torch.nn.Linear without hooks on the device of `x`, as
+// exl3_moe_gate takes it; undefined if `gate` is anything else.
+at::Tensor plain_gate_weight(PyObject* gate, const at::Tensor& x) {
+    if (reinterpret_cast<PyObject*>(Py_TYPE(gate)) != linear_module_class()) return {};
     PyObject** dict = _PyObject_GetDictPtr(gate);
     if (!dict || !*dict) return {};
     auto item = [&](const char* name) { return PyDict_GetItemString(*dict, name); };
@@ -453,21 +464,42 @@ at::Tensor plain_gate_weight(PyObject* gate, PyObject* linear_class, int D) {
     PyObject* weight = PyDict_GetItemString(params, "weight");
     if ((bias && bias != Py_None) || !weight || !THPVariable_Check(weight)) return {};
     const at::Tensor& w = THPVariable_Unpack(weight);
-    if (!w.is_cuda() || w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != D || !w.is_contiguous() ||
-        (reinterpret_cast<uintptr_t>(w.const_data_ptr()) & 15))
+    if (w.device() != x.device() || w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(-1) ||
+        !w.is_contiguous() || (reinterpret_cast<uintptr_t>(w.const_data_ptr()) & 15))
         return {};
     return w;
 }
 
-PyObject* linear_module_class() {
-    static PyObject* cls = [] {
-        PyObject* nn = PyImport_ImportModule("torch.nn");
-        PyObject* c = nn ? PyObject_GetAttrString(nn, "Linear") : nullptr;
-        Py_XDECREF(nn);
-        return c;
-    }();
-    if (!cls) throw python_error();
-    return cls;
+// Whether exl3_moe_route can read what a gate module returned for the tokens of `x`: `width`
+// logits per token, or any number if that is 0.
+bool usable_logits(PyObject* o, const at::Tensor& x, int64_t width) {
+    if (!THPVariable_Check(o)) return false;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    return t.device() == x.device() && !t.requires_grad() && t.dim() >= 1 && t.is_contiguous() &&
+           (t.scalar_type() == at::kHalf || t.scalar_type() == at::kFloat) &&
+           t.numel() == x.numel() / x.size(-1) * (width ? width : t.size(-1));
+}
+
+// The two tests above as the block applies them, for any device of x.
+PyObject* py_plain_gate_weight(PyObject*, PyObject* args) {
+    HANDLE_TH_ERRORS
+    PyObject *gate, *x;
+    if (!PyArg_ParseTuple(args, "OO", &gate, &x)) throw python_error();
+    if (!THPVariable_Check(x)) value_error("x must be a torch.Tensor");
+    const at::Tensor w = plain_gate_weight(gate, THPVariable_Unpack(x));
+    if (!w.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(w);
+    END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_usable_logits(PyObject*, PyObject* args) {
+    HANDLE_TH_ERRORS
+    PyObject *logits, *x;
+    long long width;
+    if (!PyArg_ParseTuple(args, "OOL", &logits, &x, &width)) throw python_error();
+    if (!THPVariable_Check(x)) value_error("x must be a torch.Tensor");
+    return PyBool_FromLong(usable_logits(logits, THPVariable_Unpack(x), width));
+    END_HANDLE_TH_ERRORS
 }
 
 // experts.block(x (..., D), gate, shared gate or None, top_k, norm, prefill) -> (..., D): the
@@ -496,8 +528,8 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
     at::Tensor logits, shared;
     const bool grad = at::GradMode::is_enabled();
     if (tokens <= kGateMaxTokens) {
-        const at::Tensor w = plain_gate_weight(gate, linear_module_class(), D);
-        const at::Tensor ws = has_shared ? plain_gate_weight(shared_gate, linear_module_class(), D) : at::Tensor();
+        const at::Tensor w = plain_gate_weight(gate, x);
+        const at::Tensor ws = has_shared ? plain_gate_weight(shared_gate, x) : at::Tensor();
         if (w.defined() && !(grad && w.requires_grad()) &&
             (!has_shared || (ws.defined() && ws.size(0) == 1 && !(grad && ws.requires_grad())))) {
             const int64_t E = w.size(0);
@@ -519,14 +551,8 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
             s = THPObjectPtr(PyObject_CallFunctionObjArgs(shared_gate, x3.get(), nullptr));
             if (!s) throw python_error();
         }
-        auto usable = [&](PyObject* o, int64_t numel_per_token) {
-            if (!THPVariable_Check(o)) return false;
-            const at::Tensor& t = THPVariable_Unpack(o);
-            return t.is_cuda() && !t.requires_grad() && t.dim() >= 1 && t.is_contiguous() &&
-                   (t.scalar_type() == at::kHalf || t.scalar_type() == at::kFloat) &&
-                   t.numel() == tokens * (numel_per_token ? numel_per_token : t.size(-1));
-        };
-        const bool ok = usable(l.get(), 0) && (!has_shared || (usable(s.get(), 1) && THPVariable_Unpack(s.get()).scalar_type() ==
+        const bool ok = usable_logits(l.get(), x, 0) &&
+                        (!has_shared || (usable_logits(s.get(), x, 1) && THPVariable_Unpack(s.get()).scalar_type() ==
                                                                              THPVariable_Unpack(l.get()).scalar_type()));
         if (!ok) return PyTuple_Pack(2, l.get(), has_shared ? s.get() : Py_None);
         logits = THPVariable_Unpack(l.get());
@@ -561,7 +587,10 @@ PyMethodDef experts_methods[] = {{"slots", experts_slots, METH_VARARGS, nullptr}
 
 PyTypeObject experts_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-PyMethodDef module_methods[] = {{"scratch", py_scratch, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef module_methods[] = {{"scratch", py_scratch, METH_VARARGS, nullptr},
+                                {"plain_gate_weight", py_plain_gate_weight, METH_VARARGS, nullptr},
+                                {"usable_logits", py_usable_logits, METH_VARARGS, nullptr},
+                                {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_exl3_host", nullptr, -1, module_methods};
 
