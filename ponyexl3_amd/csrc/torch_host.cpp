@@ -453,7 +453,7 @@ at::Tensor plain_gate_weight(PyObject* gate, const at::Tensor& x) {
     PyObject** dict = _PyObject_GetDictPtr(gate);
     if (!dict || !*dict) return {};
     auto item = [&](const char* name) { return PyDict_GetItemString(*dict, name); };
-    for (const char* hooks : {"_forward_hooks", "_forward_pre_hooks"}) {
+    for (const char* hooks : {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"}) {
         PyObject* h = item(hooks);
         if (!h || PyObject_Size(h) != 0) return {};
     }

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import numpy as np
 import torch
+from torch.nn.modules import module as _nn
 
 from . import _lib, ops
 from .layer import EXL3Layer, codebook_mode_from_flags, unpack_signs_or_pass
@@ -190,8 +191,9 @@ class EXL3MoEBlock(torch.nn.Module):
         self._shared_idx = switch.num_experts - 1
 
     def route(self, x: torch.Tensor):
+        logits = self.gate(x)
         shared = None if self.shared_expert_gate is None else self.shared_expert_gate(x)
-        return self._select(x, self.gate(x), shared)
+        return self._select(x, logits, shared)
 
     def _select(self, x, logits, shared_logits):
         inds, scores = route_topk(logits, self.top_k, self.norm_topk_prob)
@@ -204,13 +206,25 @@ class EXL3MoEBlock(torch.nn.Module):
             scores = torch.cat([scores, shared_w], dim=-1)
         return inds, scores
 
+    def _is_as_defined(self, switch) -> bool:
+        """Whether routing, experts and weighted sum are the ones defined in this file: the
+        native block may not pass by what a caller has put in their place or hooked."""
+        return (
+            type(self) is EXL3MoEBlock and type(switch) is EXL3SwitchGLU
+            and self.__dict__.keys().isdisjoint(_ROUTING) and "forward" not in switch.__dict__
+            and _replaceable() == _DEFINED
+            and not (switch._forward_hooks or switch._forward_pre_hooks
+                     or switch._backward_hooks or switch._backward_pre_hooks
+                     or _nn._global_forward_hooks or _nn._global_forward_pre_hooks
+                     or _nn._global_backward_hooks or _nn._global_backward_pre_hooks)
+        )
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         modules = self._modules  # plain dictionary: nn.Module's attribute lookup is slow
         gate, switch = modules.get("gate") or self.gate, modules["switch_mlp"]
         shared_gate = modules.get("shared_expert_gate")
         got = None
-        if (type(self) is EXL3MoEBlock and type(switch) is EXL3SwitchGLU
-                and not (switch._forward_hooks or switch._forward_pre_hooks)):
+        if self._is_as_defined(switch):
             # routing, experts and weighted sum in one native call
             dim = x.shape[-1]
             prefill = dim > 0 and switch._use_prefill(x.numel() // dim, self.top_k + (shared_gate is not None))
@@ -223,3 +237,15 @@ class EXL3MoEBlock(torch.nn.Module):
         inds, scores = self.route(x3) if got is None else self._select(x3, *got)
         y = switch(x3, inds)
         return combine_experts(y, scores).reshape(lead + (x.shape[-1],))
+
+
+_ROUTING = frozenset(("route", "_select"))
+
+
+def _replaceable():
+    """Functions that a caller may have replaced by name (the gates' own class among them)."""
+    return (EXL3MoEBlock.route, EXL3MoEBlock._select, EXL3SwitchGLU.forward, EXL3SwitchGLU.__call__,
+            torch.nn.Linear.forward, route_topk, combine_experts)
+
+
+_DEFINED = _replaceable()

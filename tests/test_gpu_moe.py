@@ -546,6 +546,34 @@ def test_moe_block_native_chain_equals_its_parts(cuda, tokens, shared):
     assert rel_l2(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
 
 
+@pytest.mark.parametrize("tokens", [2, 67])
+def test_moe_block_reaches_replaced_parts(cuda, tokens):
+    """A router replaced on the instance and hooks on all modules see the call, and the result
+    is that of the parts."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    E, D, H, kk = 5, 256, 128, 2
+    switch = EXL3SwitchGLU.from_layers(*_experts(E, D, H, 4, True, 4400))
+    lin = torch.nn.Linear(D, E, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin, None, switch, kk)
+    x = (torch.randn((1, tokens, D), generator=torch.Generator().manual_seed(tokens)) * 0.2).half().to(cuda)
+    y = block(x)
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: seen.append(type(m).__name__))
+    try:
+        y2 = block(x)
+    finally:
+        handle.remove()
+    assert seen == ["Linear", "EXL3SwitchGLU", "EXL3MoEBlock"]
+    assert rel_l2(y2.float().cpu().numpy(), y.float().cpu().numpy()) <= TOL
+    last = torch.tensor([E - 1, E - 2], dtype=torch.int32, device=cuda)
+    block.route = lambda x3: (last.expand(1, tokens, kk).contiguous(),
+                              torch.full((1, tokens, kk), 0.5, dtype=torch.float16, device=cuda))
+    y3 = block(x)
+    ref = switch(x, last.expand(1, tokens, kk).contiguous()).float().mean(dim=-2)
+    assert rel_l2(y3.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
+
+
 @pytest.mark.parametrize("tokens,E,D", [(1, 1, 128), (1, 256, 2048), (3, 15, 384), (16, 16, 1152), (17, 257, 640),
                                         (32, 33, 2176)])
 @pytest.mark.parametrize("shared", [False, True])

@@ -1,6 +1,7 @@
 """What the native MoE block takes in place of the modules' own operations, decided on the
 host: the tests run on CPU and meta tensors (no GPU needed)."""
 import pytest
+import pytest
 import torch
 
 from ponyexl3_amd import _lib
@@ -37,3 +38,75 @@ def test_logits_are_read_on_their_own_device_only():
     assert not host.usable_logits(ok.bfloat16(), _x(), 0)
     assert not host.usable_logits(ok[..., :5], _x(), 0)  # not contiguous
     assert not host.usable_logits(ok, _x(), 1)
+
+
+def _block(shared=False):
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    e, d, h, k = 3, 128, 128, 2
+    z = lambda *s: torch.zeros(s, dtype=torch.float16)
+    t = lambda *s: torch.zeros(s, dtype=torch.int16)
+    switch = EXL3SwitchGLU(gu_trellis=t(8, e * 2 * 8, 32), gu_suh=z(e, 2, d), gu_svh=z(e, 2 * h),
+                           dn_trellis=t(8, e * 8, 32), dn_suh=z(e, h), dn_svh=z(e, d), k=k, cb=0)
+    lin = lambda n: torch.nn.Linear(d, n, bias=False)
+    return EXL3MoEBlock(lin(e - shared), lin(1) if shared else None, switch, 1)
+
+
+def _hook(*args, **kw):
+    return None
+
+
+@pytest.mark.parametrize("change", [
+    lambda b, m: m.setattr(b, "route", b.route),
+    lambda b, m: m.setattr(b, "_select", b._select),
+    lambda b, m: m.setattr(b.switch_mlp, "forward", b.switch_mlp.forward),
+    lambda b, m: m.setattr(type(b), "route", lambda self, x: None),
+    lambda b, m: m.setattr(type(b.switch_mlp), "forward", lambda self, x, i: None),
+    lambda b, m: m.setattr("ponyexl3_amd.moe.route_topk", lambda *a: None),
+    lambda b, m: m.setattr("ponyexl3_amd.moe.combine_experts", lambda *a: None),
+    lambda b, m: m.setattr(torch.nn.Linear, "forward", lambda self, x: x),
+    lambda b, m: setattr(b.switch_mlp, "__class__", type("Sub", (type(b.switch_mlp),), {})),
+    lambda b, m: b.switch_mlp.register_forward_hook(_hook),
+    lambda b, m: b.switch_mlp.register_full_backward_hook(_hook),
+    lambda b, m: _nn().register_module_forward_hook(_hook),
+    lambda b, m: _nn().register_module_forward_pre_hook(_hook),
+    lambda b, m: _nn().register_module_full_backward_hook(_hook),
+])
+def test_block_does_not_pass_by_what_a_caller_changed(change, monkeypatch):
+    """Replaced methods and functions, hooks on the experts and hooks on all modules are
+    reached through the modules; without them the native block stands in."""
+    block = _block()
+    assert block._is_as_defined(block.switch_mlp)
+    handle = change(block, monkeypatch)
+    try:
+        assert not block._is_as_defined(block.switch_mlp)
+    finally:
+        if hasattr(handle, "remove"):
+            handle.remove()
+
+
+def _nn():
+    import torch.nn.modules.module as m
+
+    return m
+
+
+def test_gates_are_called_in_order():
+    """The router's gate first, then the shared expert's, as their side effects may show."""
+    block, seen = _block(shared=True), []
+    block.gate.register_forward_hook(lambda *a: seen.append("gate"))
+    block.shared_expert_gate.register_forward_hook(lambda *a: seen.append("shared"))
+    block.route(torch.zeros((1, 2, 128)))
+    assert seen == ["gate", "shared"]
+
+
+@pytest.mark.parametrize("hook", ["register_forward_hook", "register_forward_pre_hook",
+                                  "register_full_backward_hook", "register_full_backward_pre_hook"])
+def test_hooked_gate_is_called(hook):
+    gate = _gate()
+    handle = getattr(gate, hook)(_hook)
+    assert _lib.host().plain_gate_weight(gate, _x()) is None
+    handle.remove()
+    assert _lib.host().plain_gate_weight(gate, _x()) is not None
+    gate.forward = gate.forward
+    assert _lib.host().plain_gate_weight(gate, _x()) is None
