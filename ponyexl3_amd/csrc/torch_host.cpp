@@ -7,12 +7,18 @@
 // The module also owns the scratch buffers and counters of every (device, stream).
 // Everything runs under the GIL.
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
@@ -435,15 +441,39 @@ PyObject* experts_slots(PyObject* self, PyObject* args) {
 // module: its kernel is made for one round trip to memory, not for throughput.
 constexpr int64_t kGateMaxTokens = 32;
 
-PyObject* linear_module_class() {
-    static PyObject* cls = [] {
-        PyObject* nn = PyImport_ImportModule("torch.nn");
-        PyObject* c = nn ? PyObject_GetAttrString(nn, "Linear") : nullptr;
-        Py_XDECREF(nn);
-        return c;
-    }();
+PyObject* import_class(const char* module, const char* name) {
+    PyObject* mod = PyImport_ImportModule(module);
+    PyObject* cls = mod ? PyObject_GetAttrString(mod, name) : nullptr;
+    Py_XDECREF(mod);
     if (!cls) throw python_error();
     return cls;
+}
+PyObject* linear_module_class() {
+    static PyObject* cls = import_class("torch.nn", "Linear");
+    return cls;
+}
+
+// Whether something is to see or change the torch operations of a call: function modes (the one
+// behind torch.set_default_device only touches factory functions and is no reason), dispatch
+// modes, autocast, a function transform, tracing.
+bool operations_watched() {
+    const int64_t modes = at::impl::PythonTorchFunctionTLS::stack_len();
+    for (int64_t i = 0; i < modes; i++) {
+        static PyObject* device_mode = import_class("torch.utils._device", "DeviceContext");
+        PyObject* mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
+        if (reinterpret_cast<PyObject*>(Py_TYPE(mode)) != device_mode) return true;
+    }
+    return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::autocast::is_autocast_enabled(at::kCUDA) ||
+           c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+           at::tracer::impl::is_dispatch_enabled();
+}
+
+// A tensor that its memory describes: no subclass (whose data may live elsewhere and whose
+// operations may mean something else), no forward-mode tangent, no pending negation.
+bool plain_tensor(PyObject* o) {
+    if (!THPVariable_CheckExact(o)) return false;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    return !t._fw_grad(0).defined() && !t.is_neg();
 }
 
 // The weight of a plain bias-free fp16 torch.nn.Linear without hooks on the device of `x`, as
@@ -452,17 +482,23 @@ at::Tensor plain_gate_weight(PyObject* gate, const at::Tensor& x) {
     if (reinterpret_cast<PyObject*>(Py_TYPE(gate)) != linear_module_class()) return {};
     PyObject** dict = _PyObject_GetDictPtr(gate);
     if (!dict || !*dict) return {};
-    auto item = [&](const char* name) { return PyDict_GetItemString(*dict, name); };
-    for (const char* hooks : {"_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks"}) {
-        PyObject* h = item(hooks);
+    static PyObject* const hook_names[] = {
+        PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
+        PyUnicode_InternFromString("_backward_hooks"), PyUnicode_InternFromString("_backward_pre_hooks")};
+    static PyObject *const forward_name = PyUnicode_InternFromString("forward"),
+                    *const params_name = PyUnicode_InternFromString("_parameters"),
+                    *const bias_name = PyUnicode_InternFromString("bias"),
+                    *const weight_name = PyUnicode_InternFromString("weight");
+    for (PyObject* name : hook_names) {
+        PyObject* h = PyDict_GetItem(*dict, name);
         if (!h || PyObject_Size(h) != 0) return {};
     }
-    if (item("forward")) return {};  // replaced on the instance
-    PyObject* params = item("_parameters");
+    if (PyDict_GetItem(*dict, forward_name)) return {};  // replaced on the instance
+    PyObject* params = PyDict_GetItem(*dict, params_name);
     if (!params || !PyDict_Check(params)) return {};
-    PyObject* bias = PyDict_GetItemString(params, "bias");
-    PyObject* weight = PyDict_GetItemString(params, "weight");
-    if ((bias && bias != Py_None) || !weight || !THPVariable_Check(weight)) return {};
+    PyObject* bias = PyDict_GetItem(params, bias_name);
+    PyObject* weight = PyDict_GetItem(params, weight_name);
+    if ((bias && bias != Py_None) || !weight || !plain_tensor(weight)) return {};
     const at::Tensor& w = THPVariable_Unpack(weight);
     if (w.device() != x.device() || w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(-1) ||
         !w.is_contiguous() || (reinterpret_cast<uintptr_t>(w.const_data_ptr()) & 15))
@@ -473,14 +509,20 @@ at::Tensor plain_gate_weight(PyObject* gate, const at::Tensor& x) {
 // Whether exl3_moe_route can read what a gate module returned for the tokens of `x`: `width`
 // logits per token, or any number if that is 0.
 bool usable_logits(PyObject* o, const at::Tensor& x, int64_t width) {
-    if (!THPVariable_Check(o)) return false;
+    if (!plain_tensor(o)) return false;
     const at::Tensor& t = THPVariable_Unpack(o);
     return t.device() == x.device() && !t.requires_grad() && t.dim() >= 1 && t.is_contiguous() &&
            (t.scalar_type() == at::kHalf || t.scalar_type() == at::kFloat) &&
            t.numel() == x.numel() / x.size(-1) * (width ? width : t.size(-1));
 }
 
-// The two tests above as the block applies them, for any device of x.
+// The tests above as the block applies them, for any device of x.
+PyObject* py_operations_watched(PyObject*, PyObject*) {
+    HANDLE_TH_ERRORS
+    return PyBool_FromLong(operations_watched());
+    END_HANDLE_TH_ERRORS
+}
+
 PyObject* py_plain_gate_weight(PyObject*, PyObject* args) {
     HANDLE_TH_ERRORS
     PyObject *gate, *x;
@@ -505,7 +547,8 @@ PyObject* py_usable_logits(PyObject*, PyObject* args) {
 // experts.block(x (..., D), gate, shared gate or None, top_k, norm, prefill) -> (..., D): the
 // router (the gates are modules of the caller's; called, or if they are plain Linears and
 // there are few tokens, computed here), experts and weighted sum. Where the native route does
-// not apply (other types, sizes beyond its kernels, values that carry a gradient) it returns
+// not apply (other types, sizes beyond its kernels, values that carry a gradient or a tangent,
+// operations that a mode or transform is to see) it returns
 // (logits, shared logits or None) if the gates have been called, None if not.
 PyObject* experts_block(PyObject* self, PyObject* args) {
     HANDLE_TH_ERRORS
@@ -513,7 +556,7 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
     int top_k, norm, prefill;
     if (!PyArg_ParseTuple(args, "OOOipp", &x_arg, &gate, &shared_gate, &top_k, &norm, &prefill)) throw python_error();
     const ExpertStack& m = *reinterpret_cast<PyExperts*>(self)->stack;
-    if (!THPVariable_Check(x_arg)) Py_RETURN_NONE;
+    if (!THPVariable_Check(x_arg) || !plain_tensor(x_arg) || operations_watched()) Py_RETURN_NONE;
     at::Tensor x = THPVariable_Unpack(x_arg);
     const bool has_shared = shared_gate != Py_None;
     const int D = m.dim();
@@ -589,6 +632,7 @@ PyTypeObject experts_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 PyMethodDef module_methods[] = {{"scratch", py_scratch, METH_VARARGS, nullptr},
                                 {"plain_gate_weight", py_plain_gate_weight, METH_VARARGS, nullptr},
+                                {"operations_watched", py_operations_watched, METH_NOARGS, nullptr},
                                 {"usable_logits", py_usable_logits, METH_VARARGS, nullptr},
                                 {nullptr, nullptr, 0, nullptr}};
 

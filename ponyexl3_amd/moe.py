@@ -8,7 +8,8 @@ from __future__ import annotations
 
 import numpy as np
 import torch
-from torch.nn.modules import module as _nn
+from torch.nn.modules.module import (_global_backward_hooks, _global_backward_pre_hooks, _global_forward_hooks,
+                                     _global_forward_pre_hooks)
 
 from . import _lib, ops
 from .layer import EXL3Layer, codebook_mode_from_flags, unpack_signs_or_pass
@@ -209,14 +210,15 @@ class EXL3MoEBlock(torch.nn.Module):
     def _is_as_defined(self, switch) -> bool:
         """Whether routing, experts and weighted sum are the ones defined in this file: the
         native block may not pass by what a caller has put in their place or hooked."""
+        own, experts = self.__dict__, switch.__dict__
         return (
             type(self) is EXL3MoEBlock and type(switch) is EXL3SwitchGLU
-            and self.__dict__.keys().isdisjoint(_ROUTING) and "forward" not in switch.__dict__
+            and not ("route" in own or "_select" in own or "forward" in experts)
+            and not (experts["_forward_hooks"] or experts["_forward_pre_hooks"]
+                     or experts["_backward_hooks"] or experts["_backward_pre_hooks"]
+                     or _global_forward_hooks or _global_forward_pre_hooks
+                     or _global_backward_hooks or _global_backward_pre_hooks)
             and _replaceable() == _DEFINED
-            and not (switch._forward_hooks or switch._forward_pre_hooks
-                     or switch._backward_hooks or switch._backward_pre_hooks
-                     or _nn._global_forward_hooks or _nn._global_forward_pre_hooks
-                     or _nn._global_backward_hooks or _nn._global_backward_pre_hooks)
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -237,9 +239,6 @@ class EXL3MoEBlock(torch.nn.Module):
         inds, scores = self.route(x3) if got is None else self._select(x3, *got)
         y = switch(x3, inds)
         return combine_experts(y, scores).reshape(lead + (x.shape[-1],))
-
-
-_ROUTING = frozenset(("route", "_select"))
 
 
 def _replaceable():

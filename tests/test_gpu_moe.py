@@ -574,6 +574,40 @@ def test_moe_block_reaches_replaced_parts(cuda, tokens):
     assert rel_l2(y3.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
 
 
+def test_moe_block_under_autocast_and_with_tangents(cuda):
+    """The router's product, softmax and sum are torch's where something watches or changes
+    torch operations: bf16 logits and an fp32 sum under autocast, a tangent through the weights
+    of the sum in forward mode, a subclass of x that reaches the gate."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    E, D, H, kk, tokens = 5, 256, 128, 2, 3
+    switch = EXL3SwitchGLU.from_layers(*_experts(E, D, H, 4, True, 4500))
+    lin = torch.nn.Linear(D, E, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin, None, switch, kk)
+    x = (torch.randn((1, tokens, D), generator=torch.Generator().manual_seed(8)) * 0.2).half().to(cuda)
+
+    def parts():
+        inds, scores = block.route(x)
+        return (switch(x, inds) * scores[..., None]).sum(dim=-2)
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(block(x), parts()) and block(x).dtype == parts().dtype == torch.float32
+    with torch.autograd.forward_ad.dual_level():
+        out = block(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+        assert torch.autograd.forward_ad.unpack_dual(out).tangent is not None
+
+    class Sub(torch.Tensor):
+        seen = []
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            Sub.seen.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    block(x.as_subclass(Sub))
+    assert torch.nn.functional.linear in Sub.seen
+
+
 @pytest.mark.parametrize("tokens,E,D", [(1, 1, 128), (1, 256, 2048), (3, 15, 384), (16, 16, 1152), (17, 257, 640),
                                         (32, 33, 2176)])
 @pytest.mark.parametrize("shared", [False, True])

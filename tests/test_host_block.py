@@ -110,3 +110,61 @@ def test_hooked_gate_is_called(hook):
     assert _lib.host().plain_gate_weight(gate, _x()) is not None
     gate.forward = gate.forward
     assert _lib.host().plain_gate_weight(gate, _x()) is None
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+def _dual(t):
+    return torch.autograd.forward_ad.make_dual(t, torch.ones_like(t))
+
+
+def test_values_with_a_meaning_of_their_own_go_through_torch():
+    """Subclasses and forward-mode tangents: in the gate's weight and in logits."""
+    host = _lib.host()
+    gate = _gate()
+    logits = torch.zeros((1, TOKENS, E), dtype=torch.float16)
+    assert not host.usable_logits(logits.as_subclass(_Sub), _x(), 0)
+    assert not host.usable_logits(logits.clone().requires_grad_(), _x(), 0)
+    gate._parameters["weight"] = gate.weight.detach().as_subclass(_Sub)
+    assert host.plain_gate_weight(gate, _x()) is None
+    with torch.autograd.forward_ad.dual_level():
+        assert not host.usable_logits(_dual(logits), _x(), 0)
+        gate._parameters["weight"] = _dual(_gate().weight)
+        assert host.plain_gate_weight(gate, _x()) is None
+    assert host.usable_logits(logits, _x(), 0)
+
+
+def test_watched_operations():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    host = _lib.host()
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not host.operations_watched()
+    for mode in (Function(), Dispatch()):
+        with mode:
+            assert host.operations_watched()
+    torch.set_autocast_enabled("cuda", True)  # (the context manager needs a GPU)
+    try:
+        assert host.operations_watched()
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+    with torch.device("cpu"):  # only where new tensors go
+        assert not host.operations_watched()
+        with Function():
+            assert host.operations_watched()
+    inside = []
+    torch.func.vmap(lambda v: inside.append(host.operations_watched()) or v)(torch.zeros(2))
+    torch.jit.trace(lambda v: inside.append(host.operations_watched()) or v + 1, torch.zeros(2), check_trace=False)
+    assert inside == [True, True]
+    assert not host.operations_watched()
