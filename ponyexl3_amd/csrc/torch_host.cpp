@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <string>
@@ -55,6 +56,13 @@ const int32_t* int_ptr(const at::Tensor& t) {
     return t.defined() ? static_cast<const int32_t*>(t.const_data_ptr()) : nullptr;
 }
 uint16_t* half_out(const at::Tensor& t) { return static_cast<uint16_t*>(t.mutable_data_ptr()); }
+
+// (kernels that copy 16 bytes at a time)
+bool aligned16(std::initializer_list<const at::Tensor*> tensors) {
+    uintptr_t bits = 0;
+    for (const at::Tensor* t : tensors) bits |= reinterpret_cast<uintptr_t>(t->const_data_ptr());
+    return (bits & 15) == 0;
+}
 
 at::Tensor tensor_or_none(PyObject* o, const char* name) {
     if (o == Py_None) return {};
@@ -342,10 +350,8 @@ void experts_run(const ExpertStack& m, const at::Tensor& x, const at::Tensor& in
     if (tokens * top_k > INT32_MAX) value_error("too many (token, slot) pairs");
     const int E = m.experts(), D = m.dim(), H = m.hidden(), kk = static_cast<int>(top_k);
     StreamContext ctx(x.device().index());
-    // (the prefill kernels copy trellis words 16 bytes at a time)
-    const bool aligned = !((reinterpret_cast<uintptr_t>(m.gu_trellis.const_data_ptr()) |
-                            reinterpret_cast<uintptr_t>(m.dn_trellis.const_data_ptr())) & 15);
-    if (prefill && aligned) {
+    // the prefill kernels read everything 16 bytes at a time; the slot kernels take any address
+    if (prefill && aligned16({&x, &m.gu_trellis, &m.gu_suh, &m.gu_svh, &m.dn_trellis, &m.dn_suh, &m.dn_svh})) {
         const int t = static_cast<int>(tokens);
         const at::Tensor& ws = ctx.get(kWorkspace, exl3_moe_prefill_workspace_bytes(t, kk, E, D, H));
         check_status(exl3_moe_prefill(half_ptr(x), t, int_ptr(indices), kk, half_ptr(m.gu_trellis), half_ptr(m.gu_suh),
@@ -477,7 +483,7 @@ bool plain_tensor(PyObject* o) {
 }
 
 // The weight of a plain bias-free fp16 torch.nn.Linear without hooks on the device of `x`, as
-// exl3_moe_gate takes it; undefined if `gate` is anything else.
+// exl3_moe_gate takes it (both 16-byte aligned); undefined if `gate` is anything else.
 at::Tensor plain_gate_weight(PyObject* gate, const at::Tensor& x) {
     if (reinterpret_cast<PyObject*>(Py_TYPE(gate)) != linear_module_class()) return {};
     PyObject** dict = _PyObject_GetDictPtr(gate);
@@ -501,7 +507,7 @@ at::Tensor plain_gate_weight(PyObject* gate, const at::Tensor& x) {
     if ((bias && bias != Py_None) || !weight || !plain_tensor(weight)) return {};
     const at::Tensor& w = THPVariable_Unpack(weight);
     if (w.device() != x.device() || w.scalar_type() != at::kHalf || w.dim() != 2 || w.size(1) != x.size(-1) ||
-        !w.is_contiguous() || (reinterpret_cast<uintptr_t>(w.const_data_ptr()) & 15))
+        !w.is_contiguous() || !aligned16({&w, &x}))
         return {};
     return w;
 }

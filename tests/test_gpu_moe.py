@@ -574,6 +574,32 @@ def test_moe_block_reaches_replaced_parts(cuda, tokens):
     assert rel_l2(y3.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
 
 
+@pytest.mark.parametrize("tokens", [2, 67])
+def test_moe_block_takes_any_alignment(cuda, tokens):
+    """x, or a scale vector of the stack, as a contiguous view off the 16-byte grid: the gate's
+    product goes through the module and the experts through the slot kernels."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    E, D, H, kk = 5, 256, 128, 2
+    stack = _experts(E, D, H, 4, True, 4600)
+    lin = torch.nn.Linear(D, E, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin, None, EXL3SwitchGLU.from_layers(*stack), kk)
+    x = (torch.randn((1, tokens, D), generator=torch.Generator().manual_seed(tokens)) * 0.2).half().to(cuda)
+    ref = block(x).float().cpu().numpy()
+
+    def shifted(t):
+        s = torch.empty(t.numel() + 2, dtype=t.dtype, device=t.device)[2:].view(t.shape).copy_(t)
+        assert s.is_contiguous() and s.data_ptr() % 16
+        return s
+
+    print(f"block off the grid tokens={tokens}", flush=True)
+    assert rel_l2(block(shifted(x)).float().cpu().numpy(), ref) <= TOL
+    for name in ("_gu_svh", "_dn_suh"):
+        other = EXL3SwitchGLU.from_layers(*stack)
+        setattr(other, name, shifted(getattr(other, name)))
+        assert rel_l2(EXL3MoEBlock(lin, None, other, kk)(x).float().cpu().numpy(), ref) <= TOL
+
+
 def test_moe_block_under_autocast_and_with_tangents(cuda):
     """The router's product, softmax and sum are torch's where something watches or changes
     torch operations: bf16 logits and an fp32 sum under autocast, a tangent through the weights

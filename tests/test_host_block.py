@@ -24,6 +24,8 @@ def test_gate_weight_is_read_on_its_own_device_only():
     gate = _gate()
     assert host.plain_gate_weight(gate, _x()).data_ptr() == gate.weight.data_ptr()
     assert host.plain_gate_weight(gate, _x("meta")) is None
+    odd = torch.zeros(TOKENS * D + 8, dtype=torch.float16)[3:3 + TOKENS * D].view(1, TOKENS, D)
+    assert odd.is_contiguous() and host.plain_gate_weight(gate, odd) is None  # not 16-byte aligned
     assert host.plain_gate_weight(_gate("meta"), _x()) is None
     assert host.plain_gate_weight(_gate(dtype=torch.float32), _x()) is None
     assert host.plain_gate_weight(torch.nn.Linear(D, E, dtype=torch.float16), _x()) is None  # bias
