@@ -396,7 +396,7 @@ size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
  * 128-column block.
  *   xh        fp16 [rows][n_sub][16*in_tiles], 16-byte aligned
  *   group_sub i32 [out_tiles/8] member index of every 128-column block (required when n_sub > 1)
- *   y         fp16 [rows][16*out_tiles]
+ *   y         fp16 [rows][16*out_tiles], 8-byte aligned
  *   workspace exl3_linear_rows_workspace_bytes(rows, in, out) bytes (may be 0), 16-byte aligned
  * exl3_linear_rows_applies: whether it is the faster path for these sizes (and the trellis 16-byte
  * aligned, which it requires); otherwise take exl3_linear_prefill.

@@ -20,8 +20,13 @@ struct LinearWorkspace {
     size_t total() const { return xh_bytes + second_bytes + gemm_bytes; }
 };
 
-// The rows kernel copies trellis words 16 bytes at a time.
+// The rows kernel copies trellis words and activations 16 bytes at a time, writes partial rows 16
+// and results 8 at a time; the medium-batch kernel and the GEMM take what it cannot.
 static bool rows_aligned(const uint16_t* trellis) { return (reinterpret_cast<uintptr_t>(trellis) & 15) == 0; }
+static bool rows_aligned(const uint16_t* trellis, const void* workspace, const uint16_t* y) {
+    return rows_aligned(trellis) && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+           (reinterpret_cast<uintptr_t>(y) & 7) == 0;
+}
 
 static LinearWorkspace linear_workspace(int rows, int in_features, int out_features, int n_sub) {
     LinearWorkspace w{};
@@ -124,7 +129,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
     if (int rc = counters ? launch_rotate_layer(x, rows, in_features, suh, n_sub, xh, s)
                           : launch_had_pre(x, rows, in_features, suh, n_sub, xh, s))
         return rc;
-    if (counters && (n_sub == 1 || rows <= kLinearMidMaxRows) && rows_aligned(trellis) &&
+    if (counters && (n_sub == 1 || rows <= kLinearMidMaxRows) && rows_aligned(trellis, workspace, y) &&
         (rows > linear_mid_max_rows() || linear_rows_before_mid(rows, K, in_tiles, out_tiles)) &&
         linear_rows_applies(rows, in_tiles, out_tiles)) {
         if (rows <= linear_mid_max_rows() && counters_len < (size_t)(out_tiles / 8)) return EXL3_E_WORKSPACE;

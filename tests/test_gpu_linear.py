@@ -586,3 +586,30 @@ def test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
         assert rel_l2(part.cpu().numpy(), _oracle_forward(oracle, l, x)) <= TOL
     if need:
         assert lib.exl3_linear_rows(*args, need - 1, ops._stream()) == _lib.EXL3_E_WORKSPACE
+
+
+@pytest.mark.parametrize("rows,k,n_in,n_out", [(9, 5, 512, 256), (17, 4, 640, 384), (32, 6, 1024, 128),
+                                              (40, 4, 2048, 2048)])
+def test_layer_output_off_the_eight_byte_grid(cuda, oracle, rows, k, n_in, n_out):
+    """exl3_linear_forward states no alignment for y: where the rows kernel, which stores eight
+    bytes at a time, would be taken, a y on the 4-byte grid goes to the medium-batch kernel or the GEMM."""
+    from ponyexl3_amd import _lib, make_exl3_layer, ops
+
+    lib = _lib.load()
+    layer = make_exl3_layer(k=k, in_features=n_in, out_features=n_out, seed=rows)
+    tr = ops.as_trellis_tensor(layer.trellis, cuda)
+    suh, svh = torch.from_numpy(layer.suh).to(cuda), torch.from_numpy(layer.svh).to(cuda)
+    x, xt = _x(np.random.default_rng(rows), (rows, n_in), cuda)
+    need = lib.exl3_linear_workspace_bytes(rows, n_in, n_out, 1)
+    ws = torch.empty((need,), dtype=torch.uint8, device=cuda)
+    counters = torch.zeros((n_out // 128 + 2,), dtype=torch.int32, device=cuda)
+    p = ops._ptr
+    print(f"y off the grid rows={rows} k={k} {n_in}->{n_out}", flush=True)
+    for shift in (2, 0):
+        buf = torch.full((rows * n_out + 4,), 7.0, dtype=torch.float16, device=cuda)
+        y = buf[shift:shift + rows * n_out]
+        rc = lib.exl3_linear_forward(p(xt), rows, p(tr), n_in // 16, n_out // 16, k, 0, p(suh), 1, None, p(svh), None,
+                                     p(y), p(ws), need, p(counters), counters.numel(), ops._stream())
+        _lib.check(rc, "exl3_linear_forward")
+        assert rel_l2(y.view(rows, n_out).cpu().numpy(), _oracle_forward(oracle, layer, x)) <= TOL
+        assert bool((buf[shift + rows * n_out:] == 7.0).all()) and bool((counters == 0).all())
