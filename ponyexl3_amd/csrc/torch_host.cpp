@@ -353,7 +353,10 @@ void experts_run(const ExpertStack& m, const at::Tensor& x, const at::Tensor& in
     // the prefill kernels read everything 16 bytes at a time; the slot kernels take any address
     if (prefill && aligned16({&x, &m.gu_trellis, &m.gu_suh, &m.gu_svh, &m.dn_trellis, &m.dn_suh, &m.dn_svh})) {
         const int t = static_cast<int>(tokens);
-        const at::Tensor& ws = ctx.get(kWorkspace, exl3_moe_prefill_workspace_bytes(t, kk, E, D, H));
+        // 4 D + 2 H bytes per (token, slot): up to gigabytes, which go back to the allocator (it
+        // hands them out again in the order of this stream) and do not become the stream's scratch
+        const at::Tensor ws = at::empty({static_cast<int64_t>(exl3_moe_prefill_workspace_bytes(t, kk, E, D, H))},
+                                        x.options().dtype(at::kByte));
         check_status(exl3_moe_prefill(half_ptr(x), t, int_ptr(indices), kk, half_ptr(m.gu_trellis), half_ptr(m.gu_suh),
                                       half_ptr(m.gu_svh), half_ptr(m.dn_trellis), half_ptr(m.dn_suh),
                                       half_ptr(m.dn_svh), E, D, H, m.k, m.cb, m.activation, half_ptr(scores),

@@ -600,6 +600,29 @@ def test_moe_block_takes_any_alignment(cuda, tokens):
         assert rel_l2(EXL3MoEBlock(lin, None, other, kk)(x).float().cpu().numpy(), ref) <= TOL
 
 
+def test_prefill_keeps_no_memory(cuda):
+    """The sorted chain's rotated rows are gone when the call's result is: chunks of growing and
+    shrinking size leave what is allocated as it was, as do the experts called alone."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    E, D, H, kk = 5, 512, 128, 4
+    switch = EXL3SwitchGLU.from_layers(*_experts(E, D, H, 4, True, 4700))
+    lin = torch.nn.Linear(D, E, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin, None, switch, kk)
+    x = torch.randn((1, 1500, D), generator=torch.Generator().manual_seed(1)).half().to(cuda)
+    first = block(x[:, :30])  # router, scratch and library handles of this stream exist
+    del first
+    held = torch.cuda.memory_allocated()
+    for tokens in (200, 700, 1500, 400):
+        assert switch._use_prefill(tokens, kk)
+        print(f"prefill memory tokens={tokens}", flush=True)
+        y = block(x[:, :tokens])
+        inds, scores = block.route(x[:, :tokens])
+        z = switch(x[:, :tokens], inds)
+        del y, z, inds, scores
+        assert torch.cuda.memory_allocated() == held
+
+
 def test_moe_block_under_autocast_and_with_tangents(cuda):
     """The router's product, softmax and sum are torch's where something watches or changes
     torch operations: bf16 logits and an fp32 sum under autocast, a tangent through the weights
