@@ -910,9 +910,15 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
                 same &= ((e >> b) & 1) ? m : ~m;
             }
             const int rank = __popcll(same & ((1ull << lane) - 1ull));
+            // every lane reads its expert's cursor before the first of the equal ones moves it,
+            // and the next 64 pairs read behind that (e is 0 where there is no pair)
+            const int first = mine[e];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (valid && rank == 0) mine[e] = first + __popcll(same);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
             if (valid) {
-                const int first = mine[e];
-                if (rank == 0) mine[e] = first + __popcll(same);  // behind the reads: LDS is in order
                 const int pos = first + rank;
                 if (staged) stage[pos] = i;
                 else order[pos] = i;
