@@ -398,10 +398,12 @@ size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
  *   group_sub i32 [out_tiles/8] member index of every 128-column block (required when n_sub > 1)
  *   y         fp16 [rows][16*out_tiles], 8-byte aligned
  *   workspace exl3_linear_rows_workspace_bytes(rows, in, out) bytes (may be 0), 16-byte aligned
- * exl3_linear_rows_applies: whether it is the faster path for these sizes (and the trellis 16-byte
- * aligned, which it requires); otherwise take exl3_linear_prefill.
+ * exl3_linear_rows_faster: whether it is the faster path for these sizes, K and codebook (and the
+ * trellis 16-byte aligned, which it requires); otherwise take exl3_linear_prefill.
+ * exl3_linear_rows_applies: the same for K = 4 and 3INST weights.
  */
 int exl3_linear_rows_applies(const uint16_t *trellis, int rows, int in_tiles, int out_tiles);
+int exl3_linear_rows_faster(const uint16_t *trellis, int rows, int in_tiles, int out_tiles, int K, int cb);
 size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, int out_features);
 int exl3_linear_rows(const uint16_t *xh, int rows, int n_sub, const uint16_t *trellis, int in_tiles, int out_tiles,
                      int K, int cb, const int32_t *group_sub, const uint16_t *svh, const uint16_t *bias, uint16_t *y,

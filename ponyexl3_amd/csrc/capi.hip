@@ -43,7 +43,7 @@ static LinearWorkspace linear_workspace(int rows, int in_features, int out_featu
             const size_t mid = (size_t)m.n_splits * rows * out_features * sizeof(float);
             if (mid > w.second_bytes) w.second_bytes = mid;
         }
-        if (linear_rows_applies(rows, in_features / 16, out_features / 16)) {
+        if (linear_rows_ever_applies(rows, in_features / 16, out_features / 16)) {
             const size_t part = linear_rows_partial_bytes(rows, in_features / 16, out_features / 128);
             if (part > w.second_bytes) w.second_bytes = part;
         }
@@ -131,7 +131,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
         return rc;
     if (counters && (n_sub == 1 || rows <= kLinearMidMaxRows) && rows_aligned(trellis, workspace, y) &&
         (rows > linear_mid_max_rows() || linear_rows_before_mid(rows, K, in_tiles, out_tiles)) &&
-        linear_rows_applies(rows, in_tiles, out_tiles)) {
+        linear_rows_applies(rows, in_tiles, out_tiles, K, cb)) {
         if (rows <= linear_mid_max_rows() && counters_len < (size_t)(out_tiles / 8)) return EXL3_E_WORKSPACE;
         return launch_linear_rows(xh, rows, (size_t)n_sub * in_features, (size_t)in_features, trellis, in_tiles,
                                   out_tiles, K, cb, n_sub > 1 ? group_sub : nullptr, svh, bias, y,
@@ -202,7 +202,12 @@ EXL3_EXPORT int exl3_linear_prefill(const uint16_t* xh, int rows, int n_sub, con
 }
 
 EXL3_EXPORT int exl3_linear_rows_applies(const uint16_t* trellis, int rows, int in_tiles, int out_tiles) {
-    return exl3::rows_aligned(trellis) && exl3::linear_rows_applies(rows, in_tiles, out_tiles);
+    return exl3_linear_rows_faster(trellis, rows, in_tiles, out_tiles, 4, exl3::CB_3INST);
+}
+
+EXL3_EXPORT int exl3_linear_rows_faster(const uint16_t* trellis, int rows, int in_tiles, int out_tiles, int K, int cb) {
+    return exl3::check_k_cb(K, cb) == EXL3_OK && exl3::rows_aligned(trellis) &&
+           exl3::linear_rows_applies(rows, in_tiles, out_tiles, K, cb);
 }
 
 EXL3_EXPORT size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, int out_features) {

@@ -126,11 +126,12 @@ constexpr int kLinearRowsMaxRows = 1024;
 struct LinRowsPlan {
     int n_row_blocks, block_rows, mr;  // mr: 32-row tiles of the kernel that holds block_rows
     int n_splits, steps_per_split;     // ranges of the reduction, in 128-deep steps
-    double us;                         // estimate, without the input rotation
 };
 LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups);
 size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups);
-bool linear_rows_applies(int rows, int in_tiles, int out_tiles);
+bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb);
+// for some K and codebook
+bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles);
 int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
                        int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
                        const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream);
@@ -156,7 +157,7 @@ struct GemmPlan {
 };
 GemmPlan plan_gemm(int rows, int in_tiles, int tn_count, bool allow_split);
 // Estimate of its time with the fix-up, against linear_rows_applies()' estimate.
-double gemm_estimate_us(int rows, int in_tiles, int tn_count);
+double gemm_estimate_us(int rows, int in_tiles, int tn_count, int K, int cb);
 size_t gemm_workspace_bytes(int rows, int in_tiles, int tn_count);
 
 // Output transform the GEMM may fold into its fix-up pass: when every tile of the

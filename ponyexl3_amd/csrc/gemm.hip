@@ -739,19 +739,18 @@ GemmPlan plan_gemm(int rows, int in_tiles, int tn_count, bool allow_split) {
     return p;
 }
 
-// Measured per 64-deep step of a tile (5120 x 10240, 17408 x 5120, 5120 x 34816, K = 4): 1.1, 1.38
-// and 2.2 us at 64, 128 and 256 rows; a piece of a split tile costs 8 steps more, the fix-up 5 us.
-double gemm_estimate_us(int rows, int in_tiles, int tn_count) {
+// Against rows_estimate_us(), with which it was fitted (9 % rms): microseconds per 64-deep step of
+// a tile at 64, 128 and 256 rows, with what a bit from K = 5 on and MUL1 add; a piece of a split
+// tile costs 4.4 steps more, the fix-up 9 us, launch and fill 7.
+double gemm_estimate_us(int rows, int in_tiles, int tn_count, int K, int cb) {
+    static const double step[3] = {0.75, 1.07, 1.97}, per_bit[3] = {0.03, 0.02, 0.016}, mul1[3] = {1.23, 1.14, 1.0};
     const GemmPlan p = plan_gemm(rows, in_tiles, tn_count, true);
-    const int slots = gemm_slots();
+    const int slots = gemm_slots(), m = p.mi == 2 ? 0 : p.mi == 4 ? 1 : 2;
     double steps = (double)((p.full_tiles + slots - 1) / slots) * (in_tiles / 4);
-    double us = 0;
-    if (p.split_tiles) {
-        const double pieces = p.split_runs_per_tile ? 1 : 2;
-        steps += (double)((p.split_runs + slots - 1) / slots) * (p.split_per + 8 * pieces);
-        us = 5;
-    }
-    return us + steps * (p.mi == 2 ? 1.1 : p.mi == 4 ? 1.38 : 2.2);
+    if (p.split_tiles)
+        steps += (double)((p.split_runs + slots - 1) / slots) * (p.split_per + 4.4 * (p.split_runs_per_tile ? 1 : 2));
+    return steps * step[m] * (K > 4 ? 1 + per_bit[m] * (K - 4) : 1.0) * (cb == CB_MUL1 ? mul1[m] : 1.0) +
+           (p.split_tiles ? 16 : 7);
 }
 
 // fp32 partial tiles of the split region: slot = run + tile < runs + tiles

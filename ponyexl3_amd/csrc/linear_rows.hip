@@ -192,6 +192,8 @@ __global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_
 
 // Microseconds of one 128-deep step of a workgroup, measured at 16..333 rows of 5120 x 10240,
 // 17408 x 5120, 5120 x 34816 (K = 4): a CU holds two workgroups of up to 64 rows or one of more.
+// Only the number of ranges is chosen by it, the same at every K: pricing the one workgroup that a
+// CU holds at 33..64 rows from K = 6 on changed no choice among 1666 layers.
 static double rows_step_us(int mr, bool pair) {
     if (mr == 1) return pair ? 1.1 : 0.70;
     if (mr == 2) return pair ? 1.27 : 0.73;
@@ -209,7 +211,7 @@ LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups) {
     const int steps = in_tiles / 8;
     p.n_splits = 1;
     p.steps_per_split = steps;
-    p.us = 1e30;
+    double best = 1e30;
     for (int s = 1; s <= 16 && (s == 1 || steps / s >= 2); s++) {
         const int per = (steps + s - 1) / s;
         if ((steps + per - 1) / per != s) continue;  // some range would be empty
@@ -222,8 +224,8 @@ LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups) {
             us = rows_step_us(p.mr, false) * (double)((n + 255) / 256);
         us *= per + kRowsFillSteps;
         if (s > 1) us += kRowsPostUs + (double)s * rows * n_groups * 128 * 8 / kRowsPartialRate;
-        if (us < p.us) {
-            p.us = us;
+        if (us < best) {
+            best = us;
             p.n_splits = s;
             p.steps_per_split = per;
         }
@@ -231,18 +233,46 @@ LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups) {
     return p;
 }
 
+// Estimate of a plan's time for the choice between this kernel and the prefill GEMM, without the
+// input rotation. Alone on its CU, two to a CU, and in several rounds a workgroup's 128-deep step
+// takes: {65..96, 97..128 rows} 0.915 and 1.08 us alone, 0.93 and 1.19 in rounds; up to 64 rows
+// 0.765 alone, 1.40 for two, and 0.85 in rounds where LDS holds one (K = 6 and more: three stages
+// of activations and trellis words). Bit windows take more instructions from K = 5 on, and MUL1
+// decodes in more than the others, which more rows hide in part.
+static double rows_estimate_us(const LinRowsPlan& p, int rows, int n_groups, int K, int cb) {
+    static const double alone[3] = {0.765, 0.915, 1.08}, rounds[3] = {0.85, 0.93, 1.19}, mul1[3] = {1.28, 1.21, 1.12};
+    const int m = p.mr <= 2 ? 0 : p.mr - 2;
+    const long long n = (long long)p.n_row_blocks * n_groups * p.n_splits;
+    const size_t lds = 3 * ((size_t)p.mr * 32 * 128 * 2 + (size_t)8 * 64 * K * 4);
+    double us;
+    if (n <= 256) us = alone[m];
+    else if (p.mr <= 2 && 2 * lds <= (size_t)160 << 10) us = 1.40 * (n <= 512 ? 1.0 : (double)n / 512 + 0.15);
+    else us = rounds[m] * (double)((n + 255) / 256);
+    us *= (p.steps_per_split + kRowsFillSteps) * (K > 4 ? 1 + 0.014 * (K - 4) : 1.0) * (cb == CB_MUL1 ? mul1[m] : 1.0);
+    return us + (p.n_splits > 1 ? kRowsPostUs + (double)p.n_splits * rows * n_groups * 128 * 8 / kRowsPartialRate : 0);
+}
+
 // Whether the layer takes this kernel rather than the prefill GEMM, which has larger tiles (256
-// columns and up to 256 rows): estimated time against the GEMM's schedule. Measured (layer,
-// before -> now, us): 5120 -> 10240 at 77 rows 41.1 -> 28.8, 333 rows 80.9 -> 60.1; 17408 -> 5120
-// (K = 5) at 333 rows 115 -> 97; 2048 -> 2048 at 256 rows 34.3 -> 22.0. The GEMM keeps 5120 ->
-// 34816 at 128 rows (90 against 98) and 17408 -> 5120 at 512 (125 against 137).
-bool linear_rows_applies(int rows, int in_tiles, int out_tiles) {
+// columns and up to 256 rows). Both estimates were fitted to the choice over 2816 layers of 40 to
+// 1024 rows (in 1024..17408, out 1024..65536, K = 2..8, all codebooks): the layer is slower than
+// through the GEMM by more than 3 % in seven of them, 8 % at most, and 0.5 % slower than the
+// better of the two on average. Measured (layer, GEMM and this kernel, us): 5120 -> 10240 at 77
+// rows 41.1 and 28.8; 17408 -> 5120 (K = 5) at 333 rows 115 and 97; 5120 -> 34816 at 64 rows 63.7
+// and 59.3 at K = 4, but 69.0 and 73.0 at K = 6; 4096 -> 24576 at 256 rows 83.6 and 95.1 with MUL1.
+bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
     // fewer than four 128-deep steps do not fill the three stages of the pipeline
     if (rows < 1 || rows > max_rows || in_tiles < 32 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8) return false;
-    // by a tenth, which is how far the two estimates are off
-    return rows <= kLinearMidMaxRows || plan_linear_rows(rows, in_tiles, out_tiles / 8).us <
-                                            0.9 * gemm_estimate_us(rows, in_tiles, out_tiles);
+    if (rows <= kLinearMidMaxRows) return true;
+    const LinRowsPlan p = plan_linear_rows(rows, in_tiles, out_tiles / 8);
+    return rows_estimate_us(p, rows, out_tiles / 8, K, cb) < 0.95 * gemm_estimate_us(rows, in_tiles, out_tiles, K, cb);
+}
+
+bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles) {
+    for (int cb : {(int)CB_3INST, (int)CB_MUL1})
+        for (int K = 8; K >= 4; K--)  // (below it the estimates are those of K = 4)
+            if (linear_rows_applies(rows, in_tiles, out_tiles, K, cb)) return true;
+    return false;
 }
 
 size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups) {

@@ -169,7 +169,7 @@ void linear_run(const LinearLayer& l, const at::Tensor& x, int64_t rows64, const
         check_status((fused ? exl3_rotate : exl3_had128_pre)(xp, rows, n_in, half_ptr(l.suh), l.n_sub, half_out(xh),
                                                              ctx.stream),
                      "exl3_rotate");
-        if (fused && l.group_sub.defined() && exl3_linear_rows_applies(tr, rows, l.in_tiles, l.out_tiles)) {
+        if (fused && l.group_sub.defined() && exl3_linear_rows_faster(tr, rows, l.in_tiles, l.out_tiles, l.k, l.cb)) {
             const size_t bytes = exl3_linear_rows_workspace_bytes(rows, n_in, n_out);
             void* ws = bytes ? ctx.get(kWorkspace, bytes).mutable_data_ptr() : nullptr;
             check_status(exl3_linear_rows(half_ptr(xh), rows, l.n_sub, tr, l.in_tiles, l.out_tiles, l.k, l.cb,

@@ -146,6 +146,40 @@ def test_gemm_split_plan_sizes(lib, monkeypatch):
     assert int(lib.exl3_gemm_workspace_bytes(2048, 320, 2176)) == (256 + 64) * 256 * 256 * 4
 
 
+def test_rows_route_knows_the_weights(lib):
+    """The choice between the rows kernel and the prefill GEMM depends on K (one workgroup to a CU
+    at 33 to 64 rows from K = 6 on) and on the codebook's decode; layers measured on either side."""
+    aligned = ctypes.c_void_p(4096)
+    faster = lambda rows, n_in, n_out, k, cb: bool(
+        lib.exl3_linear_rows_faster(aligned, rows, n_in // 16, n_out // 16, k, cb))
+    assert faster(64, 5120, 34816, 4, 0) and faster(64, 5120, 34816, 5, 1)
+    assert not faster(34, 5120, 34816, 6, 1) and not faster(64, 5120, 34816, 8, 0)
+    assert not faster(200, 4096, 24576, 4, 2) and not faster(384, 5120, 34816, 2, 2)
+    for k in range(1, 9):
+        for cb in range(3):
+            assert faster(77, 5120, 10240, k, cb) and faster(32, 5120, 34816, k, cb)
+            assert not faster(1025, 5120, 10240, k, cb)
+    assert not lib.exl3_linear_rows_faster(ctypes.c_void_p(4104), 77, 320, 640, 4, 0)
+    assert not lib.exl3_linear_rows_faster(aligned, 77, 320, 640, 9, 0)
+    assert lib.exl3_linear_rows_applies(aligned, 77, 320, 640) == 1
+
+
+def test_layer_workspace_holds_the_rows_route(lib):
+    """exl3_linear_workspace_bytes does not know K: wherever the rows kernel may be taken for some
+    K and codebook, it holds the rotated activations and the partial rows."""
+    import random
+
+    rng = random.Random(5)
+    aligned = ctypes.c_void_p(4096)
+    for _ in range(400):
+        rows = rng.choice((rng.randint(9, 64), rng.randint(65, 1100)))
+        n_in, n_out, n_sub = 128 * rng.randint(1, 140), 128 * rng.randint(1, 300), rng.randint(1, 3)
+        total = lib.exl3_linear_workspace_bytes(rows, n_in, n_out, n_sub)
+        if any(lib.exl3_linear_rows_faster(aligned, rows, n_in // 16, n_out // 16, k, cb)
+               for k in range(1, 9) for cb in range(3)):
+            assert total >= rows * n_sub * n_in * 2 + lib.exl3_linear_rows_workspace_bytes(rows, n_in, n_out)
+
+
 def test_status_to_exception():
     from ponyexl3_amd import _lib
 
