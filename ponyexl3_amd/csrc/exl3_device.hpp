@@ -186,17 +186,6 @@ __host__ __device__ constexpr int cw_row(int n) {
     return 2 * ((n >> 3) & 3) + (n & 1) + 8 * ((n >> 1) & 1);
 }
 
-// Loads the K dwords of lane `lane` for the 8 tiles that start at dword
-// `base` (tile tn0 of row tk) and fetches the preceding dword from the
-// neighbouring lane (lane u-1 of the same tile, u = 0 wraps to u = 7).
-template <int K>
-__device__ __forceinline__ void load_lane_words(const uint32_t* __restrict__ base, int lane,
-                                                uint32_t (&own)[K]) {
-    const uint32_t* p = base + lane * K;
-#pragma unroll
-    for (int i = 0; i < K; i++) own[i] = p[i];
-}
-
 // The dword that precedes a lane's own K dwords: the last dword of lane u-1 of
 // the same tile (u = 0 wraps to u = 7, the stream is circular). One ds_bpermute.
 __device__ __forceinline__ uint32_t neighbour_word(uint32_t last_own, int lane) {
@@ -322,16 +311,6 @@ __device__ __forceinline__ void load_lds16(const void* base, uint32_t offset, ui
 }
 __device__ __forceinline__ uint32_t lds_byte_address(const void* p) {
     return (uint32_t)(uintptr_t)(const void __attribute__((address_space(3)))*)p;
-}
-
-// Workgroup barrier behind which this wave's LDS accesses are complete and all but its last
-// VM vector memory operations; __syncthreads() waits for every one of those, prefetches
-// included.
-template <int VM>
-__device__ __forceinline__ void barrier_with_loads_in_flight() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VM) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
 }
 
 // v[j] = element 8*(lane & 15) + j of the lane group's block, unnormalised WHT in place.

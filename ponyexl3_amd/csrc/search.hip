@@ -44,19 +44,6 @@ __device__ __forceinline__ float decode1_f32(uint32_t cw) {
     return v[0];
 }
 
-// if (err < best) { best = err; best_f = F; } with F an inline constant (0..64):
-// compare into VCC and two selects, nothing held in scalar registers.
-template <int F>
-__device__ __forceinline__ void take_if_less(float err, float& best, uint32_t& best_f) {
-    static_assert(F >= 0 && F <= 64, "inline integer constants end at 64");
-    asm("v_cmp_lt_f32_e32 vcc, %2, %0\n\t"
-        "v_cndmask_b32_e32 %0, %0, %2, vcc\n\t"
-        "v_cndmask_b32_e64 %1, %1, %3, vcc"
-        : "+v"(best), "+v"(best_f)
-        : "v"(err), "n"(F)
-        : "vcc");
-}
-
 // Where things sit for one K. A compressed state e (16-K bits) splits in two ways:
 //   as the target of a step   e = p << K | l      (p: 16-2K bits, l: K bits)
 //   as its source             e = f << P | p      (f: the K bits above, P = 16-2K)
