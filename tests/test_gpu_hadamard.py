@@ -96,7 +96,8 @@ def test_layer_rotation_with_general_scales(cuda, oracle, rows, n, n_sub, scale,
     x = np.clip(rng.standard_normal((rows, n)) * x_std, -6e4, 6e4).astype(np.float16)
     x[0, 3] = np.inf  # one per block at most: an output is the infinity with a sign
     suh = (np.where(rng.random((n_sub, n)) > 0.5, -1, 1) * rng.uniform(0.5, 2, (n_sub, n)) * scale).astype(np.float16)
-    suh[:, 128 * (n // 256):128 * (n // 256) + 128] = np.sign(suh[:, :128])  # a block with plain signs
+    if n > 128:
+        suh[:, 128:256] = np.sign(suh[:, 128:256])  # a block with plain signs
     xt, st = _t(x, cuda), _t(suh, cuda)
     got = torch.empty((rows, n_sub, n), dtype=torch.float16, device=cuda)
     p = lambda t: ctypes.c_void_p(t.data_ptr())

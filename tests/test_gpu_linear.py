@@ -613,3 +613,21 @@ def test_layer_output_off_the_eight_byte_grid(cuda, oracle, rows, k, n_in, n_out
         _lib.check(rc, "exl3_linear_forward")
         assert rel_l2(y.view(rows, n_out).cpu().numpy(), _oracle_forward(oracle, layer, x)) <= TOL
         assert bool((buf[shift + rows * n_out:] == 7.0).all()) and bool((counters == 0).all())
+
+
+@pytest.mark.parametrize("rows,k,n_in,n_out", [(64, 4, 640, 256), (130, 5, 512, 384), (300, 3, 256, 128)])
+def test_layer_with_general_scales(cuda, oracle, rows, k, n_in, n_out):
+    """Scale vectors that are not +-1, at row counts whose rotation runs on the matrix pipe; the
+    result does not depend on that."""
+    from ponyexl3_amd import EXL3Linear, make_exl3_layer
+
+    rng = np.random.default_rng(rows)
+    scale = lambda n, s: (np.where(rng.random(n) > 0.5, -1, 1) * rng.uniform(0.5, 2, n) * s).astype(np.float16)
+    layer = make_exl3_layer(k=k, in_features=n_in, out_features=n_out, seed=rows, suh=scale(n_in, 1.0),
+                            svh=scale(n_out, 0.05))
+    x, xt = _x(rng, (rows, n_in), cuda)
+    mod = EXL3Linear(layer)
+    y = mod(xt)
+    assert rel_l2(y.cpu().numpy(), _oracle_forward(oracle, layer, x)) <= TOL
+    few = torch.cat([mod(xt[r:r + 8]) for r in range(0, 32, 8)])
+    assert rel_l2(y[:32].float().cpu().numpy(), few.float().cpu().numpy()) <= TOL
