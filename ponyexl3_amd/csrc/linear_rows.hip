@@ -10,8 +10,8 @@
 // the output transform kernel adds in range order.
 //
 // What bounds it: issue of the decode, and the matrix pipe next to it. 333 rows of 17408 -> 5120
-// (K = 4): VALU issue 42 % and matrix pipe 33 % of the SIMD cycles, which overlap only in part,
-// 26 % of the wave time in waits and barriers; the kernel 93 us where the GEMM took 102.
+// (K = 4): VALU issue 49 % and matrix pipe 39 % of the SIMD cycles, which overlap only in part,
+// 30 % of the wave time in waits and barriers; the layer 88 us where the GEMM takes 108.
 // Half of a quad between two matrix instructions, rather than a whole quad between pairs of
 // them, and direct loads spread the same way gave 5 %.
 //

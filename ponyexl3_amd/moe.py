@@ -96,13 +96,16 @@ class EXL3SwitchGLU(torch.nn.Module):
 
     # The sorted, segmented prefill path replaces the slot kernels once the experts see
     # a few rows each (the reference switches at 9 tokens,
-    # ponyexl3/mlx/exl3_moe.py:770-787). Measured on 256 experts of 2048 x 512, top-8:
-    # the slot kernels, which share one pass over an expert's weights among up to four
-    # of its slots as long as the call has at most 512 slots, take 64 / 97 / 124 /
-    # 158 us at 16 / 32 / 48 / 64 tokens and 255 us at 72 (576 slots, every slot on
-    # its own); the prefill path takes 180-207 us from 40 to 96 tokens (every expert's
-    # weights are decoded once, eight launches). So: prefill above 512 slots, and
-    # below that from 2.5 rows per expert on (few experts, many rows each).
+    # ponyexl3/mlx/exl3_moe.py:770-787). The slot kernels share one pass over an expert's
+    # weights among up to four of its slots as long as the call has at most 512 slots; above
+    # that every slot is on its own. Measured (experts of one call, us, slot kernels and
+    # prefill): 256 experts of 2048 x 512, top-8, K = 4: 63 and 82 at 16 tokens, 99 and 112 at
+    # 32, 127 and 140 at 48, 150 and 151 at 64, 251 and 147 at 68 (544 slots). Fewer experts
+    # with more rows each: 64 of 2048 x 768, top-6, 82 and 72 at 28 tokens, 153 and 75 at 64; 128
+    # of 1024 x 768, top-8, 79 and 67 at 40. So: prefill above 512 slots, and below that from
+    # 2.5 rows per expert on. The lines were drawn with a slower prefill chain and are not where
+    # the two cross for every size: at K = 6 the 256 experts cross at 36 tokens (194 and 164 at
+    # 64), 8 experts with top-2 at 64 only (26 and 44 at 24).
     prefill_min_tokens = 24
     prefill_min_rows_per_expert = 2.5
     grouped_max_slots = 512
