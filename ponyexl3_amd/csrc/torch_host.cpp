@@ -548,7 +548,7 @@ PyObject* py_usable_logits(PyObject*, PyObject* args) {
     PyObject *logits, *x;
     long long width;
     if (!PyArg_ParseTuple(args, "OOL", &logits, &x, &width)) throw python_error();
-    if (!THPVariable_Check(x)) value_error("x must be a torch.Tensor");
+    if (!THPVariable_Check(x) || THPVariable_Unpack(x).numel() == 0) value_error("x must be a torch.Tensor with elements");
     return PyBool_FromLong(usable_logits(logits, THPVariable_Unpack(x), width));
     END_HANDLE_TH_ERRORS
 }

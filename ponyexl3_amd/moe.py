@@ -213,10 +213,11 @@ class EXL3MoEBlock(torch.nn.Module):
     def _is_as_defined(self, switch) -> bool:
         """Whether routing, experts and weighted sum are the ones defined in this file: the
         native block may not pass by what a caller has put in their place or hooked."""
+        if type(self) is not EXL3MoEBlock or type(switch) is not EXL3SwitchGLU:
+            return False
         own, experts = self.__dict__, switch.__dict__
         return (
-            type(self) is EXL3MoEBlock and type(switch) is EXL3SwitchGLU
-            and not ("route" in own or "_select" in own or "forward" in experts)
+            not ("route" in own or "_select" in own or "forward" in experts)
             and not (experts["_forward_hooks"] or experts["_forward_pre_hooks"]
                      or experts["_backward_hooks"] or experts["_backward_pre_hooks"]
                      or _global_forward_hooks or _global_forward_pre_hooks
@@ -225,9 +226,12 @@ class EXL3MoEBlock(torch.nn.Module):
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        modules = self._modules  # plain dictionary: nn.Module's attribute lookup is slow
-        gate, switch = modules.get("gate") or self.gate, modules["switch_mlp"]
-        shared_gate = modules.get("shared_expert_gate")
+        # (modules first: nn.Module's attribute lookup is slow; any callable may stand in for one)
+        modules = self._modules
+        gate, switch, shared_gate = modules.get("gate"), modules.get("switch_mlp"), modules.get("shared_expert_gate")
+        gate = self.gate if gate is None else gate
+        switch = self.switch_mlp if switch is None else switch
+        shared_gate = self.shared_expert_gate if shared_gate is None else shared_gate
         got = None
         if self._is_as_defined(switch):
             # routing, experts and weighted sum in one native call

@@ -575,6 +575,26 @@ def test_moe_block_reaches_replaced_parts(cuda, tokens):
 
 
 @pytest.mark.parametrize("tokens", [2, 67])
+def test_moe_block_with_callables_for_modules(cuda, tokens):
+    """Gates, the shared expert's included, and the experts may be any callables."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    E, D, H, kk = 5, 256, 128, 2
+    switch = EXL3SwitchGLU.from_layers(*_experts(E, D, H, 4, True, 4800))
+    lin = lambda n: torch.nn.Linear(D, n, bias=False).half().to(cuda).requires_grad_(False)
+    gate, shared = lin(E - 1), lin(1)
+    x = (torch.randn((1, tokens, D), generator=torch.Generator().manual_seed(tokens)) * 0.2).half().to(cuda)
+    ref = EXL3MoEBlock(gate, shared, switch, kk)(x).float().cpu().numpy()
+    call = lambda m: lambda *a: m(*a)
+    for g, s in ((gate, call(shared)), (call(gate), shared), (call(gate), call(shared))):
+        assert rel_l2(EXL3MoEBlock(g, s, switch, kk)(x).float().cpu().numpy(), ref) <= TOL
+    block = EXL3MoEBlock(gate, shared, switch, kk)
+    del block.switch_mlp
+    block.switch_mlp = call(switch)
+    assert rel_l2(block(x).float().cpu().numpy(), ref) <= TOL
+
+
+@pytest.mark.parametrize("tokens", [2, 67])
 def test_moe_block_takes_any_alignment(cuda, tokens):
     """x, or a scale vector of the stack, as a contiguous view off the 16-byte grid: the gate's
     product goes through the module and the experts through the slot kernels."""
