@@ -78,6 +78,11 @@ at::Tensor tensor_or_none(PyObject* o, const char* name) {
 // launches that point into it. Buffers grow by half at least, which bounds what is kept.
 struct Scratch {
     at::Tensor buf[3];
+    // Counters made while the stream was being captured: the fill that zeroes them is part of that
+    // graph and may not have run when another graph or an eager call uses them. Until an eager
+    // call has cleared them, every further capture records a fill of its own.
+    bool counters_unset = false;
+    unsigned long long cleared_in = 0;
 };
 enum { kWorkspace = 0, kGemmWorkspace = 1, kCounters = 2 };
 
@@ -112,8 +117,25 @@ struct StreamContext {
                                  .dtype(kind == kCounters ? at::kInt : at::kByte);
             t = kind == kCounters ? at::zeros({static_cast<int64_t>(want)}, opt)
                                   : at::empty({static_cast<int64_t>(want)}, opt);
+            if (kind == kCounters) scratch.counters_unset = capturing(&scratch.cleared_in);
+        } else if (kind == kCounters && scratch.counters_unset) {
+            unsigned long long id = 0;
+            if (!capturing(&id)) {
+                t.zero_();
+                scratch.counters_unset = false;
+            } else if (id != scratch.cleared_in) {
+                t.zero_();
+                scratch.cleared_in = id;
+            }
         }
         return t;
+    }
+
+    // whether the stream is being captured, and into which graph
+    bool capturing(unsigned long long* id) const {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        return hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, id) == hipSuccess &&
+               status == hipStreamCaptureStatusActive;
     }
 };
 
@@ -128,7 +150,7 @@ PyObject* py_scratch(PyObject*, PyObject* args) {
     StreamContext ctx(device);
     if (n < 0) {
         if (!ctx.scratch.buf[kind].defined()) Py_RETURN_NONE;
-        return THPVariable_Wrap(ctx.scratch.buf[kind]);
+        return THPVariable_Wrap(ctx.get(kind, 0));
     }
     return THPVariable_Wrap(ctx.get(kind, static_cast<size_t>(n)));
     END_HANDLE_TH_ERRORS

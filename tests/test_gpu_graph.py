@@ -75,3 +75,44 @@ def test_moe_replays(cuda, tokens):
 
     print(f"graph moe tokens={tokens}", flush=True)
     _replay_matches_eager(cuda, make_inputs, lambda x, idx: moe(x, idx))
+
+
+@pytest.mark.parametrize("rows", [1, 12])
+def test_counters_made_under_capture_are_zero_for_every_user(cuda, monkeypatch, rows):
+    """The first call of a stream may be a captured one; the fill that zeroes its counters is then
+    part of that graph. Whatever the memory holds, a second graph replayed before the first, the
+    first one and an eager call find zeros (accumulators at one row, group counters at twelve)."""
+    from ponyexl3_amd import EXL3Linear, _lib, make_exl3_layer
+
+    monkeypatch.setenv("EXL3_SPIN_LIMIT", str(1 << 16))
+    lin = EXL3Linear(make_exl3_layer(k=4, in_features=1024, out_features=512, seed=77))
+    x = torch.randn((rows, 1024), generator=torch.Generator().manual_seed(rows)).half().to(cuda)
+    ref = lin(x)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    graphs, outs = [], []
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            outs.append((lin(x), lin(x)))
+            counters = _lib.host().scratch(2, 0, 0)  # the capturing stream's
+        graphs.append(graph)
+    print(f"counters under capture rows={rows}", flush=True)
+
+    def dirty():
+        counters.fill_(0x5A5A5A5A)
+        torch.cuda.synchronize()
+
+    for i in (1, 0, 1):
+        dirty()
+        for _ in range(2):
+            graphs[i].replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, ref) for o in outs[i])
+    dirty()
+    with torch.cuda.stream(stream):
+        assert torch.equal(lin(x), ref)
+        torch.cuda.synchronize()
+        assert _lib.host().scratch(2, 0, -1).data_ptr() == counters.data_ptr()
+    assert bool((counters == 0).all())
