@@ -216,13 +216,16 @@ class EXL3MoEBlock(torch.nn.Module):
         if type(self) is not EXL3MoEBlock or type(switch) is not EXL3SwitchGLU:
             return False
         own, experts = self.__dict__, switch.__dict__
-        return (
-            not ("route" in own or "_select" in own or "forward" in experts)
-            and not (experts["_forward_hooks"] or experts["_forward_pre_hooks"]
-                     or experts["_backward_hooks"] or experts["_backward_pre_hooks"]
-                     or _global_forward_hooks or _global_forward_pre_hooks
-                     or _global_backward_hooks or _global_backward_pre_hooks)
-            and _replaceable() == _DEFINED
+        return not (
+            "route" in own or "_select" in own or "forward" in experts
+            or experts["_forward_hooks"] or experts["_forward_pre_hooks"]
+            or experts["_backward_hooks"] or experts["_backward_pre_hooks"]
+            or _global_forward_hooks or _global_forward_pre_hooks
+            or _global_backward_hooks or _global_backward_pre_hooks
+            # functions that a caller may have replaced by name, the gates' class among them
+            or EXL3MoEBlock.route is not _ROUTE or EXL3MoEBlock._select is not _SELECT
+            or EXL3SwitchGLU.forward is not _EXPERTS or EXL3SwitchGLU.__call__ is not _CALL
+            or _Linear.forward is not _PRODUCT or route_topk is not _TOPK or combine_experts is not _COMBINE
         )
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
@@ -235,8 +238,7 @@ class EXL3MoEBlock(torch.nn.Module):
         got = None
         if self._is_as_defined(switch):
             # routing, experts and weighted sum in one native call
-            dim = x.shape[-1]
-            prefill = dim > 0 and switch._use_prefill(x.numel() // dim, self.top_k + (shared_gate is not None))
+            prefill = switch._use_prefill(x.numel() // switch.input_dims, self.top_k + (shared_gate is not None))
             got = switch.native().block(x, gate, shared_gate, self.top_k, self.norm_topk_prob, prefill)
             if isinstance(got, torch.Tensor):
                 return got
@@ -248,10 +250,7 @@ class EXL3MoEBlock(torch.nn.Module):
         return combine_experts(y, scores).reshape(lead + (x.shape[-1],))
 
 
-def _replaceable():
-    """Functions that a caller may have replaced by name (the gates' own class among them)."""
-    return (EXL3MoEBlock.route, EXL3MoEBlock._select, EXL3SwitchGLU.forward, EXL3SwitchGLU.__call__,
-            torch.nn.Linear.forward, route_topk, combine_experts)
-
-
-_DEFINED = _replaceable()
+_Linear = torch.nn.Linear
+_ROUTE, _SELECT = EXL3MoEBlock.route, EXL3MoEBlock._select
+_EXPERTS, _CALL, _PRODUCT = EXL3SwitchGLU.forward, EXL3SwitchGLU.__call__, _Linear.forward
+_TOPK, _COMBINE = route_topk, combine_experts
