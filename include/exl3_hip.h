@@ -112,9 +112,9 @@ int exl3_had128_pre(const uint16_t *x, int rows, int n, const uint16_t *suh, int
                     uint16_t *xh, void *stream);
 
 /*
- * The same rotation as the layer forwards run it: from 64 rows on the Hadamard products
- * are on the matrix pipe (exact products, fp32 sums in another order, so single results can
- * round differently from exl3_had128_pre's).
+ * The same rotation as the layer forwards run it: from 64 rows on, blocks whose multipliers are
+ * all +-1 are transformed on the matrix pipe (fp32 sums in another order, so single results can
+ * round differently from exl3_had128_pre's); all others have exl3_had128_pre's bits.
  */
 int exl3_rotate(const uint16_t *x, int rows, int n, const uint16_t *suh, int n_sub, uint16_t *xh,
                 void *stream);
