@@ -479,8 +479,10 @@ PyObject* import_class(const char* module, const char* name) {
     if (!cls) throw python_error();
     return cls;
 }
+// (no guarded static: an import may hand the GIL to a thread that would wait for the guard with it)
 PyObject* linear_module_class() {
-    static PyObject* cls = import_class("torch.nn", "Linear");
+    static PyObject* cls = nullptr;
+    if (!cls) cls = import_class("torch.nn", "Linear");
     return cls;
 }
 
@@ -490,7 +492,8 @@ PyObject* linear_module_class() {
 bool operations_watched() {
     const int64_t modes = at::impl::PythonTorchFunctionTLS::stack_len();
     for (int64_t i = 0; i < modes; i++) {
-        static PyObject* device_mode = import_class("torch.utils._device", "DeviceContext");
+        static PyObject* device_mode = nullptr;
+        if (!device_mode) device_mode = import_class("torch.utils._device", "DeviceContext");
         PyObject* mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
         if (reinterpret_cast<PyObject*>(Py_TYPE(mode)) != device_mode) return true;
     }

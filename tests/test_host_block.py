@@ -170,3 +170,34 @@ def test_watched_operations():
     torch.jit.trace(lambda v: inside.append(host.operations_watched()) or v + 1, torch.zeros(2), check_trace=False)
     assert inside == [True, True]
     assert not host.operations_watched()
+
+
+def test_first_calls_of_two_threads_do_not_wait_for_each_other():
+    """The class of a plain gate is imported on the first call; the import lets other threads
+    run, which then make their first call."""
+    import subprocess
+    import sys
+    import textwrap
+
+    from conftest import ROOT
+
+    code = textwrap.dedent("""
+        import builtins, threading, time
+        import torch
+        from ponyexl3_amd import _lib
+        host, plain = _lib.host(), builtins.__import__
+        def slow(name, *a, **kw):
+            if name == "torch.nn":
+                time.sleep(0.3)
+            return plain(name, *a, **kw)
+        gate = torch.nn.Linear(64, 8, bias=False, dtype=torch.float16)
+        x, got = torch.zeros((1, 2, 64), dtype=torch.float16), []
+        builtins.__import__ = slow
+        threads = [threading.Thread(target=lambda: got.append(host.plain_gate_weight(gate, x))) for _ in range(3)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert len(got) == 3 and all(w is not None for w in got)
+    """)
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=60, cwd=ROOT)
