@@ -156,6 +156,19 @@ PyObject* py_scratch(PyObject*, PyObject* args) {
     END_HANDLE_TH_ERRORS
 }
 
+// Refuses what a kernel cannot read at a tensor's address; undefined tensors pass.
+void require(const at::Tensor& t, const char* name, std::initializer_list<at::ScalarType> types, int64_t numel,
+             const at::Tensor& like) {
+    if (!t.defined()) return;
+    const std::string n(name);
+    if (!t.is_cuda()) value_error(n + " must live on the GPU (got device " + t.device().str() + ")");
+    if (t.device() != like.device()) value_error(n + " must live on " + like.device().str());
+    if (!t.is_contiguous()) value_error(n + " must be contiguous");
+    if (std::find(types.begin(), types.end(), t.scalar_type()) == types.end())
+        value_error(n + " must not be " + c10::toString(t.scalar_type()));
+    if (t.numel() != numel) value_error(n + " has " + std::to_string(t.numel()) + " elements, not " + std::to_string(numel));
+}
+
 // ---------------------------------------------------------------------------
 // A linear layer or a sibling-fused group.
 struct LinearLayer {
@@ -283,6 +296,13 @@ int linear_init(PyObject* self, PyObject* args, PyObject*) {
         l->in_tiles = static_cast<int>(l->trellis.size(0));
         l->out_tiles = static_cast<int>(l->trellis.size(1));
         l->n_sub = l->suh.defined() && l->suh.dim() == 2 ? static_cast<int>(l->suh.size(0)) : 1;
+        if (k < 1 || k > 8 || l->trellis.size(2) != 16 * k) value_error("trellis must be 3D (in_tiles, out_tiles, 16*K)");
+        require(l->trellis, "trellis", {at::kShort, at::kUInt16}, l->trellis.numel(), l->trellis);
+        require(l->suh, "suh", {at::kHalf}, l->n_sub * l->in_features(), l->trellis);
+        require(l->svh, "svh", {at::kHalf}, l->out_features(), l->trellis);
+        require(l->bias, "bias", {at::kHalf}, l->out_features(), l->trellis);
+        require(l->group_sub, "group_sub", {at::kInt}, l->out_features() / 128, l->trellis);
+        require(l->block_sub, "block_sub", {at::kInt}, (l->out_features() + 255) / 256, l->trellis);
         if (members != Py_None) {
             PyObject* seq = PySequence_Fast(members, "member_out must be a sequence");
             if (!seq) return -1;
@@ -425,6 +445,14 @@ int experts_init(PyObject* self, PyObject* args, PyObject*) {
             if (!to[i]->defined() || !to[i]->is_cuda() || !to[i]->is_contiguous())
                 value_error("expert weights must be contiguous tensors on the GPU");
         }
+        if (m->gu_suh.dim() != 3 || m->dn_suh.dim() != 2 || k < 1 || k > 8) value_error("expert weights of unexpected shape");
+        const int64_t e = m->experts(), d = m->dim(), h = m->hidden();
+        require(m->gu_trellis, "gu_trellis", {at::kShort, at::kUInt16}, e * 2 * h * d / 16 * k, m->gu_trellis);
+        require(m->dn_trellis, "dn_trellis", {at::kShort, at::kUInt16}, e * h * d / 16 * k, m->gu_trellis);
+        require(m->gu_suh, "gu_suh", {at::kHalf}, e * 2 * d, m->gu_trellis);
+        require(m->gu_svh, "gu_svh", {at::kHalf}, e * 2 * h, m->gu_trellis);
+        require(m->dn_suh, "dn_suh", {at::kHalf}, e * h, m->gu_trellis);
+        require(m->dn_svh, "dn_svh", {at::kHalf}, e * d, m->gu_trellis);
         m->k = k;
         m->cb = cb;
         m->activation = activation;

@@ -643,6 +643,18 @@ def test_prefill_keeps_no_memory(cuda):
         assert torch.cuda.memory_allocated() == held
 
 
+@pytest.mark.parametrize("name", ["_gu_suh", "_gu_svh", "_dn_suh", "_dn_svh", "_gu_trellis"])
+def test_stack_of_another_type_is_refused(cuda, name):
+    """Before any launch: the kernels read fp16 scales and 16-bit words at these addresses."""
+    from ponyexl3_amd import EXL3SwitchGLU
+
+    switch = EXL3SwitchGLU.from_layers(*_experts(2, 128, 128, 4, True, 4900))
+    setattr(switch, name, getattr(switch, name).float())
+    with pytest.raises(ValueError):
+        switch(torch.zeros((1, 1, 128), dtype=torch.float16, device=cuda),
+               torch.zeros((1, 1, 1), dtype=torch.int32, device=cuda))
+
+
 def test_moe_block_under_autocast_and_with_tangents(cuda):
     """The router's product, softmax and sum are torch's where something watches or changes
     torch operations: bf16 logits and an fp32 sum under autocast, a tangent through the weights

@@ -172,6 +172,23 @@ def test_watched_operations():
     assert not host.operations_watched()
 
 
+def test_layers_and_experts_off_the_gpu_are_refused():
+    """A module whose weights are in host memory must not hand their address to a kernel,
+    whatever the input's device: the modules' calls say so before anything is launched."""
+    from ponyexl3_amd import EXL3Linear, FusedEXL3Group, make_exl3_layer
+
+    layers = [make_exl3_layer(k=4, in_features=128, out_features=128, seed=i, key=str(i)) for i in range(2)]
+    x = torch.zeros((1, 128), dtype=torch.float16)
+    with pytest.raises(ValueError, match="trellis must live on the GPU"):
+        EXL3Linear(layers[0], "cpu")(x)
+    with pytest.raises(ValueError, match="trellis must live on the GPU"):
+        FusedEXL3Group(layers, "cpu").forward_all(x)
+    with pytest.raises(ValueError, match="on the GPU"):
+        _block().switch_mlp(x.view(1, 1, 128), torch.zeros((1, 1, 1), dtype=torch.int32))
+    with pytest.raises(ValueError, match="16\\*K"):
+        _lib.host().Linear(torch.zeros((8, 8, 48), dtype=torch.int16), 4, 0, None, None, None, None, None, None)
+
+
 def test_first_calls_of_two_threads_do_not_wait_for_each_other():
     """The class of a plain gate is imported on the first call; the import lets other threads
     run, which then make their first call."""
