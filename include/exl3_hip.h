@@ -456,7 +456,9 @@ int exl3_moe_glu_rows(const uint16_t *g, const uint16_t *u, int n_rows, int H, c
  * as exl3_moe_forward; no limit of 4096 pairs, num_experts <= 1024.
  *   scores  fp16 [tokens][top_k]: y is fp16 [tokens][D], the weighted sum of a token's
  *           slots (exl3_moe.py:838-839); NULL: y is fp16 [tokens][top_k][D]
- *   workspace  at least exl3_moe_prefill_workspace_bytes(), 16-byte aligned
+ *   workspace  at least exl3_moe_prefill_workspace_bytes()
+ * All pointers but indices and scores 16-byte aligned (EXL3_E_BAD_SHAPE otherwise; exl3_moe_forward
+ * takes any).
  */
 size_t exl3_moe_prefill_workspace_bytes(int tokens, int top_k, int n_experts, int D, int H);
 int exl3_moe_prefill(const uint16_t *x, int tokens, const int32_t *indices, int top_k,
