@@ -38,15 +38,19 @@ __global__ __launch_bounds__(1024) void diag_decode_kernel(const uint32_t* __res
                                                            uint32_t rows_mask, int steps,
                                                            float* __restrict__ out) {
     // 64 tile rows of activations, each value stored twice as the layer kernels stage them
-    __shared__ __attribute__((aligned(16))) half_t xs[2048];
+    __shared__ __attribute__((aligned(16))) half_t xs[2048 + 32];  // and a tile row of zeros
     constexpr int kSlots = 4;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const half_t xval = (half_t)(float)((int)(threadIdx.x * 37 % 17) - 8);  // small integers, -8..8
     xs[2 * threadIdx.x] = xs[2 * threadIdx.x + 1] = xval;
+    if (threadIdx.x < 32) xs[2048 + threadIdx.x] = (half_t)0.f;
     __syncthreads();
     const uint32_t wave_global = blockIdx.x * 16 + wave;
     float4_t accv[2][1] = {{float4_t{0, 0, 0, 0}}, {float4_t{0, 0, 0, 0}}};
+    keep_in_agprs(accv[0][0]);
+    keep_in_agprs(accv[1][0]);
+    const bool own = (lane & 15) == 4 * (lane >> 4);  // see x_operand_row
     uint32_t w[kSlots][K];
     auto row_ptr = [&](int s) {
         const uint32_t r = (wave_global * (uint32_t)steps + (uint32_t)s) & rows_mask;
@@ -59,7 +63,7 @@ __global__ __launch_bounds__(1024) void diag_decode_kernel(const uint32_t* __res
 #pragma unroll
         for (int s = 0; s < kSlots; s++) {
             const uint32_t prev_next = neighbour_word(w[(s + 1) % kSlots][K - 1], lane);
-            const uint4_t* xp = reinterpret_cast<const uint4_t*>(xs + ((s0 + s) & 63) * 32);
+            const uint4_t* xp = reinterpret_cast<const uint4_t*>(xs + (own ? ((s0 + s) & 63) * 32 : 2048));
             __builtin_amdgcn_sched_barrier(0);
             dot_tile_row<K, CB, 1>(make_lane_words<K>(prev, w[s]), [&](int c) {
                 XChunk<1> t;

@@ -18,87 +18,99 @@ constexpr float kHadScaleF = 0.088388347648318440550f;  // 1/sqrt(128)
 // of in the same bank.
 constexpr int kXwLd = 264;
 
-// Activations of a tile row as the matrix pipe takes them, a quarter at a time: for each
-// group of four batch rows, lane i of every quad reads batch row 4q+i; chunk c = input
-// rows 4c..4c+3 of the tile row, each value twice (one ds_read_b128).
+// Rows of a wave's staging area: its MT batch rows and a row of zeros.
+template <int MT>
+constexpr int kXwRows = MT + 1;
+
+// The dot products of a tile row run on v_mfma_f32_16x16x32_f16 (A 16 x 32, B 32 x 16). A lane
+// supplies eight consecutive k-slots (group g = lane >> 4) of one row i = lane & 15 of A and of one
+// column of B, and receives D[4g..4g+3][lane & 15]. The weights a lane decodes belong to its own
+// two output columns, and the four lanes that share a column of B hold four different ones, so
+// A is block diagonal: row 4g + m holds the activations of batch row m in the k-slots of group g
+// and zeros elsewhere. D[4g + m] then is the dot product of the lane's own weights with batch row
+// m: no data crosses lanes and the VALU only extracts, multiplies and masks. One instruction does
+// the work of two v_mfma_f32_4x4x4_16b_f16 (sixteen blocks of four lanes) in the same time on
+// the matrix pipe and half the issue slots: the linears of two 5120-wide layers at K = 4, one row
+// 138.2 -> 133.6 us, five rows at K = 6 225.2 -> 222.3.
+//
+// Where lane `lane` reads its share of A for batch rows 4q..4q+3: the row of its own group, or
+// the zeros (also for rows past the batch).
+template <int MT>
+__device__ __forceinline__ const half_t* x_operand_row(half_t (*xw)[kXwLd], int lane, int q) {
+    const int i = lane & 15, m = 4 * q + (i & 3);
+    return xw[(i >> 2) == (lane >> 4) && m < MT ? m : MT];
+}
+
+// Activations of a tile row as the matrix pipe takes them, a part at a time: unsummed halves: chunk c
+// = input rows 4c..4c+3 of the tile row, each value twice; EXACT (weights rounded to fp16 before the
+// product, see dot_tile_row_exact): the block is staged once per value and chunk c = input rows
+// 8c..8c+7. One ds_read_b128 per group of four batch rows.
 template <int MT>
 struct XChunk {
     uint4_t v[(MT + 3) / 4];
 };
 
-// EXACT (weights rounded to fp16 before the product, see dot_tile_row_exact): the block is
-// staged once per value and chunk c = input rows 8c..8c+7 of the tile row.
 template <int MT, bool EXACT = false>
-__device__ __forceinline__ XChunk<MT> load_x_chunk(half_t (*xw)[kXwLd], int row_in_block, int xlane,
+__device__ __forceinline__ XChunk<MT> load_x_chunk(const half_t* const (&xr)[(MT + 3) / 4], int row_in_block,
                                                    int c) {
-    constexpr int NQ = (MT + 3) / 4;
     XChunk<MT> t;
 #pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        int m = 4 * q + xlane;
-        if (m > MT - 1) m = MT - 1;  // rows past the batch repeat a staged row; never used
-        t.v[q] = *reinterpret_cast<const uint4_t*>(
-            &xw[m][EXACT ? row_in_block * 16 + 8 * c : row_in_block * 32 + 8 * c]);
-    }
+    for (int q = 0; q < (MT + 3) / 4; q++)
+        t.v[q] = *reinterpret_cast<const uint4_t*>(xr[q] + (EXACT ? 16 : 32) * row_in_block + 8 * c);
     return t;
 }
 
-// The dot products of one tile row on the matrix pipe: v_mfma_f32_4x4x4_16b_f16
-// multiplies, in each of its 16 independent blocks of 4 lanes, a 4x4 A (lane i of the
-// block supplies row i) with a 4x4 B (lane j supplies column j) and leaves D[0..3][j] in
-// lane j. A row i = activations of batch row 4q+i, B column j = two consecutive weights
-// of lane j's own output column as their unsummed halves (lo, hi, lo', hi') against
-// (a, a, a', a'): every lane gets the dot products of its weights with four batch rows,
-// no data crosses lanes, and the VALU only extracts, multiplies and masks.
+// Weights enter as their unsummed halves (lo, hi, lo', hi', ...) against (a, a, a', a', ...), four
+// weights of a column to an instruction.
 //
-// Order of work: the sixteen codeword pairs of a lane are taken chunk by chunk of the
-// activations (input rows 0-3, 8-11, 4-7, 12-15 of the tile row, both columns each), so
-// that only two chunks are live at a time: the third and fourth are requested from LDS
-// when the first and second have been used up. The matrix instruction of a pair is
-// issued after the next pair has been decoded, so it never waits for the VALU result
-// it reads.
+// Order of work: the codewords of a lane are taken chunk by chunk of the activations (input rows
+// 0-3, 8-11, 4-7, 12-15 of the tile row, both columns each), so that only two chunks are live
+// at a time: the third and fourth are requested from LDS when the first and second have been
+// used up. The matrix instruction of a chunk and column is issued after half of the next one has been
+// decoded, so it never waits for the VALU result it reads.
+//
+// The sums have to live in accumulation registers (keep_in_agprs): the decode is inline assembly,
+// and the compiler does not see that its VALU writes must not follow a matrix instruction too
+// closely into registers that this one still reads as its third operand.
+__device__ __forceinline__ void keep_in_agprs(float4_t& v) { asm("" : "+a"(v)); }
+
 template <int K, int CB, int MT, class LoadChunk>
 __device__ __forceinline__ void dot_tile_row(const LaneWords<K>& lw, LoadChunk&& load_chunk,
                                              float4_t (&accv)[2][(MT + 3) / 4]) {
     constexpr int NQ = (MT + 3) / 4;
-    // pair t: column select cs = (t >> 1) & 1 ... see pair_n below
-    // t = 4*phase + 2*jj + cs with chunk(phase) = {0, 2, 1, 3}[phase], j = 2*chunk + jj
-    auto pair_j = [](int t) constexpr { return 2 * ((t >> 2) == 0 ? 0 : (t >> 2) == 1 ? 2 : (t >> 2) == 2 ? 1 : 3) + ((t >> 1) & 1); };
-    auto pair_cs = [](int t) constexpr { return t & 1; };
+    // step t = 2 * phase + cs takes chunk {0, 2, 1, 3}[phase] of column u + 8 * cs
+    auto step_chunk = [](int t) constexpr { return (t >> 1) == 0 ? 0 : (t >> 1) == 1 ? 2 : (t >> 1) == 2 ? 1 : 3; };
     // codewords n, n+1 hold input rows 2j, 2j+1 of column u + 8*cs (cw_row, cw_col_sel)
     auto pair_n = [](int j, int cs) constexpr { return 8 * (j & 3) + 4 * cs + 2 * (j >> 2); };
     XChunk<MT> xc[4];
     xc[0] = load_chunk(0);
     xc[2] = load_chunk(2);
-    uint2_t wb[16];
+    uint4_t wb[8];
     auto issue = [&](auto tc) {
-        constexpr int t = tc.value;
-        constexpr int j = pair_j(t), cs = pair_cs(t);
+        constexpr int t = tc.value, c = step_chunk(t), cs = t & 1;
 #pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            const uint4_t xv = xc[j >> 1].v[q];
-            const uint2_t xa = (j & 1) ? uint2_t{xv.z, xv.w} : uint2_t{xv.x, xv.y};
-            accv[cs][q] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, xa),
-                                                           __builtin_bit_cast(half4_t, wb[t]),
-                                                           accv[cs][q], 0, 0, 0);
-        }
+        for (int q = 0; q < NQ; q++)
+            accv[cs][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xc[c].v[q]),
+                                                                 __builtin_bit_cast(half8_t, wb[t]), accv[cs][q], 0, 0, 0);
     };
-    static_for<0, 16>([&](auto tc) {
-        constexpr int t = tc.value;
-        constexpr int n = pair_n(pair_j(t), pair_cs(t));
-        static_assert(cw_col_sel(n) == pair_cs(t) && (cw_row(n) >> 1) == pair_j(t), "pair order");
-        wb[t] = uint2_t{weight_halves<CB>(lane_codeword<K, n>(lw)),
-                        weight_halves<CB>(lane_codeword<K, n + 1>(lw))};
+    static_for<0, 8>([&](auto tc) {
+        constexpr int t = tc.value, c = step_chunk(t), cs = t & 1;
+        constexpr int n0 = pair_n(2 * c, cs), n1 = pair_n(2 * c + 1, cs);
+        static_assert(cw_col_sel(n0) == cs && cw_row(n0) == 4 * c && cw_row(n1) == 4 * c + 2, "pair order");
+        wb[t].x = weight_halves<CB>(lane_codeword<K, n0>(lw));
+        wb[t].y = weight_halves<CB>(lane_codeword<K, n0 + 1>(lw));
         if constexpr (t >= 1) issue(std::integral_constant<int, t - 1>{});
-        if constexpr (t == 4) xc[1] = load_chunk(1);   // chunk 0 has just been used up
-        if constexpr (t == 8) xc[3] = load_chunk(3);   // chunk 2 likewise
+        if constexpr (t == 2) xc[1] = load_chunk(1);  // chunk 0 has just been used up
+        if constexpr (t == 4) xc[3] = load_chunk(3);  // chunk 2 likewise
+        wb[t].z = weight_halves<CB>(lane_codeword<K, n1>(lw));
+        wb[t].w = weight_halves<CB>(lane_codeword<K, n1 + 1>(lw));
     });
-    issue(std::integral_constant<int, 15>{});
+    issue(std::integral_constant<int, 7>{});
 }
 
 // The same with the weights as the reference defines them, rounded to fp16 (the half add
-// of ponyexl3/ref/codebook.py:45-51) before they are multiplied: four weights per matrix
-// instruction against four activations. 32 more VALU instructions per tile row than the
+// of ponyexl3/ref/codebook.py:45-51) before they are multiplied: eight weights per matrix
+// instruction against eight activations. 32 more VALU instructions per tile row than the
 // unsummed form, whose products carry the exact sum of the two halves instead - a relative
 // difference of up to 2^-11 per weight, 4-5e-4 rel-L2 on a layer's output. Chains of
 // layers with a nonlinearity in between (the MoE experts) take this form for the
@@ -110,20 +122,17 @@ __device__ __forceinline__ void dot_tile_row_exact(const LaneWords<K>& lw, LoadC
     const XChunk<MT> xc[2] = {load_chunk(0), load_chunk(1)};
     half2_t wp[16];
     decode_lane<K, CB>(lw, wp);
-    // fresh-row groups outermost: consecutive MFMAs then write different accumulators
+    // column select innermost: consecutive instructions then write different accumulators
 #pragma unroll
-    for (int j4 = 0; j4 < 4; j4++) {  // input rows 4*j4 .. 4*j4+3 of the tile
+    for (int c = 0; c < 2; c++) {  // input rows 8c .. 8c+7 of the tile
 #pragma unroll
         for (int q = 0; q < NQ; q++) {
-            const uint4_t xv = xc[j4 >> 1].v[q];
-            const uint2_t xa = (j4 & 1) ? uint2_t{xv.z, xv.w} : uint2_t{xv.x, xv.y};
 #pragma unroll
             for (int cs = 0; cs < 2; cs++) {
-                const uint2_t wb = {half2_to_bits(wp[8 * cs + 2 * j4]),
-                                    half2_to_bits(wp[8 * cs + 2 * j4 + 1])};
-                accv[cs][q] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, xa),
-                                                               __builtin_bit_cast(half4_t, wb),
-                                                               accv[cs][q], 0, 0, 0);
+                const uint4_t wb = {half2_to_bits(wp[8 * cs + 4 * c]), half2_to_bits(wp[8 * cs + 4 * c + 1]),
+                                    half2_to_bits(wp[8 * cs + 4 * c + 2]), half2_to_bits(wp[8 * cs + 4 * c + 3])};
+                accv[cs][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, xc[c].v[q]),
+                                                                     __builtin_bit_cast(half8_t, wb), accv[cs][q], 0, 0, 0);
             }
         }
     }
@@ -150,7 +159,7 @@ __device__ __forceinline__ void load_lane_words_nt(global_words_t p, uint32_t (&
 // of the 8 tile columns that start at `base` (already offset by lane*K dwords)
 // and accumulates acc[m][0..1] += x[m][rows of the tile] . W[:, column u / u+8].
 //
-// Activations enter through the wave's own LDS slot xw[MT][kXwLd], one 128-wide
+// Activations enter through the wave's own LDS slot xw[kXwRows<MT>][kXwLd], one 128-wide
 // block (8 tile rows) at a time:
 //   ROTATE  xw = fp16(had128(x * suh) / sqrt(128))   (ponyexl3/ref/forward.py:32-34)
 //   else    xw = x                                   (x is already rotated)
@@ -229,10 +238,16 @@ __device__ __forceinline__ void stream_block_rows_at(const uint32_t* __restrict_
 #pragma unroll
     for (int cs = 0; cs < 2; cs++)
 #pragma unroll
-        for (int q = 0; q < NQ; q++) accv[cs][q] = float4_t{0.f, 0.f, 0.f, 0.f};
-    const int xlane = lane & 3;
+        for (int q = 0; q < NQ; q++) {
+            accv[cs][q] = float4_t{0.f, 0.f, 0.f, 0.f};
+            keep_in_agprs(accv[cs][q]);
+        }
+    *reinterpret_cast<uint2_t*>(&xw[MT][4 * lane]) = uint2_t{0u, 0u};
+    const half_t* xr[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) xr[q] = x_operand_row<MT>(xw, lane, q);
     auto consume = [&](const uint32_t (&words)[K], uint32_t prev, int row_in_block) {
-        auto chunk = [&](int c) { return load_x_chunk<MT, EXACT>(xw, row_in_block, xlane, c); };
+        auto chunk = [&](int c) { return load_x_chunk<MT, EXACT>(xr, row_in_block, c); };
         if constexpr (EXACT)
             dot_tile_row_exact<K, CB, MT>(make_lane_words<K>(prev, words), chunk, accv);
         else

@@ -199,10 +199,10 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(
     static_assert(NW == 4 || (NW == 8 && ATOMIC), "eight-wave workgroups use the accumulators");
     // the staged activations and, once every wave has left the streaming loop, the waves'
     // sums share one LDS buffer (at eight rows the two together would cost occupancy)
-    constexpr size_t kXsBytes = sizeof(half_t) * NW * MT * kXwLd;
+    constexpr size_t kXsBytes = sizeof(half_t) * NW * kXwRows<MT> * kXwLd;
     constexpr size_t kRedBytes = sizeof(float) * NW * MT * 128;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kXsBytes > kRedBytes ? kXsBytes : kRedBytes];
-    half_t (*xs)[MT][kXwLd] = reinterpret_cast<half_t (*)[MT][kXwLd]>(smem);
+    half_t (*xs)[kXwRows<MT>][kXwLd] = reinterpret_cast<half_t (*)[kXwRows<MT>][kXwLd]>(smem);
     float (*red)[MT][128] = reinterpret_cast<float (*)[MT][128]>(smem);
     const int g = blockIdx.x;
     const int lane = threadIdx.x & 63;

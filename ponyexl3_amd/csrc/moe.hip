@@ -234,7 +234,7 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_kernel(
     const int* __restrict__ indices, const half_t* __restrict__ gu_suh,
     const half_t* __restrict__ gu_svh, const half_t* __restrict__ dn_suh, half_t* xh_dn,
     float* part, int* counters, int top_k, int E, int D, int H, int activation) {
-    __shared__ __attribute__((aligned(16))) half_t xs[NW][1][kXwLd];
+    __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<1>][kXwLd];
     __shared__ float red[NW][128];
     __shared__ float up_val[128];
     __shared__ int last_flag;
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
     const half_t* __restrict__ gu_svh, const half_t* __restrict__ dn_suh, half_t* xh_dn,
     unsigned long long* sums, int top_k, int E, int D, int H, int activation, int* status,
     int spin_limit) {
-    __shared__ __attribute__((aligned(16))) half_t xs[8][1][kXwLd];
+    __shared__ __attribute__((aligned(16))) half_t xs[8][kXwRows<1>][kXwLd];
     __shared__ float red[8][128];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
     const uint32_t* __restrict__ dn_trellis, const half_t* __restrict__ xh_dn,
     const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* __restrict__ y,
     float* part, int* counters, int E, int D, int H) {
-    __shared__ __attribute__((aligned(16))) half_t xs[NW][1][kXwLd];
+    __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<1>][kXwLd];
     __shared__ float red[NW][128];
     __shared__ int last_flag;
     const int lane = threadIdx.x & 63;
@@ -583,7 +583,7 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
     const int* __restrict__ indices, const half_t* __restrict__ gu_suh,
     const half_t* __restrict__ gu_svh, const half_t* __restrict__ dn_suh, half_t* xh_dn,
     float* part, int* counters, int slots, int top_k, int E, int D, int H, int activation) {
-    __shared__ __attribute__((aligned(16))) half_t xs[NW][kGroupRows][kXwLd];
+    __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<kGroupRows>][kXwLd];
     __shared__ float red[NW][kGroupRows][128];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
     const uint32_t* __restrict__ dn_trellis, const half_t* __restrict__ xh_dn,
     const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* __restrict__ y,
     float* part, int* counters, int slots, int E, int D, int H) {
-    __shared__ __attribute__((aligned(16))) half_t xs[NW][kGroupRows][kXwLd];
+    __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<kGroupRows>][kXwLd];
     __shared__ float red[NW][kGroupRows][128];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
