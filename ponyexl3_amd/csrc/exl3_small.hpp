@@ -322,7 +322,7 @@ __device__ __forceinline__ void stream_block_rows(const uint32_t* __restrict__ b
 #pragma unroll
     for (int m = 0; m < MT; m++) xrow[m] = x + (size_t)(m < rows ? m : 0) * x_stride;
     uint32_t buf[kStreamSlots][K];
-    stream_block_rows_at<K, CB, MT, ROTATE, HALF, false, false, EXACT>(
+    stream_block_rows_at<K, CB, MT, ROTATE, HALF, (MT > 2), false, EXACT>(
         base, row_words, tk_begin, tk_end, xrow, rows, suh_row, xw, lane, acc, buf);
 }
 
