@@ -269,8 +269,9 @@ size_t exl3_gemm_workspace_bytes(int rows, int in_tiles, int tn_count);
  *            and is all zero again when the launch has finished, so a caller
  *            zeroes it once and reuses it (calls that overlap on one array race),
  *            and results are run-to-run deterministic. Above that and up to
- *            exl3_linear_small_max_rows() rows the array serves the medium-batch
- *            kernel as group counters (counters_len >= out/128; two launches: input
+ *            exl3_linear_small_max_rows() rows the array serves as group counters
+ *            (counters_len >= out/128): up to 16 rows of a layer that does not fill
+ *            the chip in one launch, else in the medium-batch kernel (two launches: input
  *            rotation, then everything else), unless the rows kernel is faster. NULL selects the three-launch chain
  *            (exl3_had128_pre, exl3_gemv_partials, exl3_had128_post) resp. the
  *            prefill GEMM.

@@ -22,7 +22,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(PKG_DIR, "libexl3_hip.so")
 
-SOURCES = ["decode.hip", "hadamard.hip", "gemv.hip", "linear_mid.hip", "linear_rows.hip", "gemm.hip", "moe.hip", "moe_route.hip", "moe_rows.hip", "search.hip", "capi.hip"]
+SOURCES = ["decode.hip", "hadamard.hip", "gemv.hip", "linear_batch.hip", "linear_mid.hip", "linear_rows.hip", "gemm.hip", "moe.hip", "moe_route.hip", "moe_rows.hip", "search.hip", "capi.hip"]
 # measurement probes (include/exl3_diag.h): a library of their own, kept out of the product ABI
 DIAG_SOURCES = ["diag.hip"]
 DIAG_LIB_PATH = os.path.join(PKG_DIR, "libexl3_diag.so")

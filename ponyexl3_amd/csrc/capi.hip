@@ -33,8 +33,8 @@ static LinearWorkspace linear_workspace(int rows, int in_features, int out_featu
     w.xh_bytes = align_up((size_t)rows * n_sub * in_features * 2, 256);
     if (rows <= kGemvMaxRows) {
         const GemvPlan a = plan_gemv(rows, in_features / 16, out_features / 128);
-        const GemvPlan b = plan_linear_small(rows, in_features / 16, out_features / 128);
-        const int n = a.n_partials() > b.n_partials() ? a.n_partials() : b.n_partials();
+        const int b = linear_small_max_partials(rows, in_features / 16, out_features / 128);
+        const int n = a.n_partials() > b ? a.n_partials() : b;
         w.second_bytes = (size_t)n * rows * out_features * sizeof(float);
     } else {
         w.second_bytes = (size_t)rows * out_features * 2;
@@ -43,6 +43,12 @@ static LinearWorkspace linear_workspace(int rows, int in_features, int out_featu
             const size_t mid = (size_t)m.n_splits * rows * out_features * sizeof(float);
             if (mid > w.second_bytes) w.second_bytes = mid;
         }
+        for (int K : {1, 8})
+            if (linear_batch_applies(rows, in_features / 16, out_features / 128, K)) {
+                const GemvPlan b = plan_linear_batch(rows, in_features / 16, out_features / 128);
+                const size_t part = (size_t)b.n_partials() * rows * out_features * sizeof(float);
+                if (part > w.second_bytes) w.second_bytes = part;
+            }
         if (linear_rows_ever_applies(rows, in_features / 16, out_features / 16)) {
             const size_t part = linear_rows_partial_bytes(rows, in_features / 16, out_features / 128);
             if (part > w.second_bytes) w.second_bytes = part;
@@ -124,6 +130,12 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
                                out_features, svh, bias, y, s);
     }
 
+    if (counters && rows <= linear_mid_max_rows() && linear_batch_applies(rows, in_tiles, out_tiles / 8, K)) {
+        if (counters_len < (size_t)(out_tiles / 8)) return EXL3_E_WORKSPACE;
+        return launch_linear_batch(x, rows, trellis, in_tiles, out_tiles, K, cb, suh, n_sub, group_sub, svh, bias, y,
+                                   reinterpret_cast<float*>(second), counters,
+                                   plan_linear_batch(rows, in_tiles, out_tiles / 8), s);
+    }
     // Prefill: rotation kernel, MFMA GEMM, output transform.
     // (without counters the chain of the separate entry points, bit for bit)
     if (int rc = counters ? launch_rotate_layer(x, rows, in_features, suh, n_sub, xh, s)
@@ -326,9 +338,9 @@ static StaticNeed static_need(int rows, int out_features, GemvPlan plan) {
 EXL3_EXPORT size_t exl3_linear_static_need_bytes(int rows, int in_features, int out_features) {
     using namespace exl3;
     if (rows < 1 || rows > kLinearSmallMaxRows || in_features < 128 || out_features < 128) return 0;
-    // the launch plan depends on K (deeper splits from K = 5 on): the larger of the two
+    // the launch plan depends on K: the largest of all
     size_t need = 0;
-    for (int K : {4, 8}) {
+    for (int K = 1; K <= 8; K++) {
         const GemvPlan plan = plan_linear_small_launch(rows, in_features / 16, out_features / 128, K);
         const size_t n = static_need(rows, out_features, plan).larger();
         if (n > need) need = n;

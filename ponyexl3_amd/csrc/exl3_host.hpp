@@ -56,7 +56,8 @@ constexpr int kGemvMaxRows = 8;
 struct GemvPlan {
     int n_splits;      // wave-level splits of the tile rows
     int tk_per_split;  // tile rows per split
-    int wg_waves = 4;  // waves per workgroup (4; the one-launch layer kernel also has 8)
+    int wg_waves = 4;  // waves per workgroup (4; the one-launch layer kernels also have 8)
+    bool batch = false;  // half blocks in linear_batch_kernel
     // the waves of a workgroup are summed in LDS: partial rows per group
     int n_partials() const { return (n_splits + wg_waves - 1) / wg_waves; }
 };
@@ -79,8 +80,11 @@ int launch_gemv_partials(const uint16_t* xh, int rows, int n_sub, const uint16_t
 constexpr int kLinearSmallMaxRows = kGemvMaxRows;
 bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan);
 // plan_linear_small with the reduction in mind: one row on a large layer takes
-// workgroups of eight waves when that brings the launch under the atomics limit.
-GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K = 4);
+// workgroups of eight waves when that brings the launch under the atomics limit; two rows and
+// more of a layer that does not fill the chip take linear_batch_kernel.
+GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K);
+// fp32 partial rows per output of the largest plan over K
+int linear_small_max_partials(int rows, int in_tiles, int n_groups);
 inline size_t linear_small_counter_ints(int rows, int out_features) {
     return 2 * (size_t)rows * out_features;  // >= out_features / 128
 }
@@ -91,6 +95,18 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
                         hipStream_t stream, int* status = nullptr);
 // `status` (device, may be NULL): set to non-zero by a finishing workgroup of the
 // accumulator reduction whose bounded wait for the other contributors ran out.
+
+// One-launch layer for 2..16 rows of layers that do not fill the chip (linear_batch.hip): counters and
+// partial rows as above (above 8 rows: partial rows and one counter per column group). Reached
+// through launch_linear_small() up to 8 rows (plan.batch).
+constexpr int kLinearBatchMaxRows = 16;
+bool linear_batch_applies(int rows, int in_tiles, int n_groups, int K);
+bool linear_batch_uses_atomics(int rows, int n_groups, GemvPlan plan);
+GemvPlan plan_linear_batch(int rows, int in_tiles, int n_groups);
+int launch_linear_batch(const uint16_t* x, int rows, const uint16_t* trellis, int in_tiles, int out_tiles, int K, int cb,
+                        const uint16_t* suh, int n_sub, const int32_t* group_sub, const uint16_t* svh,
+                        const uint16_t* bias, uint16_t* y, float* partial, int* counters, GemvPlan plan,
+                        hipStream_t stream, int* status = nullptr);
 
 // Medium-batch layer (rows <= kLinearMidMaxRows) on rotated activations xh, fp16
 // [rows][n_sub][in]: weights decoded once and fed to 16x16x16 MFMA from registers;

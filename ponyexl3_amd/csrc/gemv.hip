@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(
 // The counters array (accumulators uint64 [rows][out], or one int per column group)
 // must be zero on entry; it is zero again when the kernel ends.
 //
-// HALF (one and two rows only): splits are half blocks of four tile rows.
+// HALF (one row only): splits are half blocks of four tile rows.
 // ATOMIC: which of the two split reductions described at the end of the kernel runs.
 // NW: waves per workgroup, 4 or 8 (8 only with ATOMIC: half as many workgroups add
 // to a column group's accumulators).
@@ -477,8 +477,8 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
     // K = 6 43.3 -> 40.1 / 23.5 -> 22.2, K = 8 52.7 -> 47.5 / 29.0 -> 25.4 (K <= 4: no
     // gain or a loss).
     static const int kDeepFromK = env_int("EXL3_LINEAR_DEEP_FROM_K", 5, 1, 9);
-    // one and two rows: when even one block per wave leaves fewer than this many waves
-    // (four per SIMD), the waves take half blocks
+    // one row: when even one block per wave leaves fewer than this many waves (four per SIMD),
+    // the waves take half blocks
     static const int kHalfBelow = env_int("EXL3_LINEAR_HALF_BELOW", 4096, 0, 1 << 20);
     const int target_waves = 256 * 4 * kWavesPerSimd;
     const int n_blocks = in_tiles / 8;
@@ -490,7 +490,7 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
     // The accumulator reduction has to be able to take the partial sums (eight-bit
     // count, atomics limit); with partial rows, 100+ rows per column group would cost
     // the finishing workgroup more than the balance gains.
-    if (rows <= 2 && (long long)n_blocks * n_groups < kHalfBelow) {
+    if (rows == 1 && (long long)n_blocks * n_groups < kHalfBelow) {
         const long long whole = (long long)n_blocks * n_groups, n_simd = 1024;
         const long long cost_whole = ((whole + n_simd - 1) / n_simd) * (8 * 118 + 60);
         const long long cost_half = ((2 * whole + n_simd - 1) / n_simd) * (4 * 118 + 60);
@@ -520,6 +520,7 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
 // half blocks 327 k: 11.7 -> 11.2 us, gate+up 696 k: no loss; the step 83.0 -> 79.8 us);
 // at four rows neither limit gains (86.0 / 86.6 / 90.4 us at 300 k / 800 k / 1.6 M).
 bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
+    if (plan.batch) return linear_batch_uses_atomics(rows, n_groups, plan);
     static const int kMaxAtomics = env_int("EXL3_LINEAR_MAX_ATOMICS", 300000, 0, 1 << 30);
     if (plan.n_partials() > 255) return false;  // the count field has eight bits
     const long long limit = rows == 2 ? (long long)kMaxAtomics * 8 / 3 : kMaxAtomics;
@@ -527,6 +528,7 @@ bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
 }
 
 GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K) {
+    if (linear_batch_applies(rows, in_tiles, n_groups, K)) return plan_linear_batch(rows, in_tiles, n_groups);
     GemvPlan plan = plan_linear_small(rows, in_tiles, n_groups, K);
     if (rows == 1 && plan.tk_per_split >= 8 && !linear_small_uses_atomics(rows, n_groups, plan)) {
         GemvPlan wide = plan;
@@ -534,6 +536,15 @@ GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K) {
         if (linear_small_uses_atomics(rows, n_groups, wide)) plan = wide;
     }
     return plan;
+}
+
+int linear_small_max_partials(int rows, int in_tiles, int n_groups) {
+    int n = 0;
+    for (int K = 1; K <= 8; K++) {
+        const int p = plan_linear_small_launch(rows, in_tiles, n_groups, K).n_partials();
+        if (p > n) n = p;
+    }
+    return n;
 }
 
 int launch_gemv_partials(const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis,
@@ -574,6 +585,9 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
                         const int32_t* group_sub, const uint16_t* svh, const uint16_t* bias,
                         uint16_t* y, float* partial, int* counters, GemvPlan plan,
                         hipStream_t stream, int* status) {
+    if (plan.batch)
+        return launch_linear_batch(x, rows, trellis, in_tiles, out_tiles, K, cb, suh, n_sub, group_sub, svh, bias, y,
+                                   partial, counters, plan, stream, status);
     if (int rc = check_k_cb(K, cb)) return rc;
     if (!x || !trellis || !y || !counters) return EXL3_E_NULL_POINTER;
     const int spin_limit = reduction_spin_limit();
@@ -584,7 +598,7 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
         in_tiles % 8 || out_tiles % 8)
         return EXL3_E_BAD_SHAPE;
     if (n_sub > 1 && (!group_sub || !suh)) return EXL3_E_BAD_INDEX;
-    const bool half = plan.tk_per_split == 4 && rows <= 2;
+    const bool half = plan.tk_per_split == 4 && rows == 1;
     if (plan.n_splits < 1 || plan.n_splits > 4 * 65535 ||
         (!half && (plan.tk_per_split < 8 || plan.tk_per_split % 8)) ||
         (long long)plan.n_splits * plan.tk_per_split < in_tiles)
@@ -626,10 +640,7 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
                 if (half) go(std::integral_constant<int, 1>{}, T{});
                 else go(std::integral_constant<int, 1>{}, F{});
                 break;
-            case 2:
-                if (half) go(std::integral_constant<int, 2>{}, T{});
-                else go(std::integral_constant<int, 2>{}, F{});
-                break;
+            case 2: go(std::integral_constant<int, 2>{}, F{}); break;
             case 4: go(std::integral_constant<int, 4>{}, F{}); break;
             default: go(std::integral_constant<int, 8>{}, F{}); break;
         }

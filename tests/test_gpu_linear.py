@@ -58,6 +58,48 @@ def test_module_matches_oracle(cuda, oracle, rows, k, mcg):
     assert y.dtype == np.float16 and y.shape == (rows, 384)
     assert rel_l2(y, _oracle_forward(oracle, layer, x)) <= TOL
 
+@pytest.mark.parametrize("n_in,n_out", [(128, 128), (640, 384), (1152, 2048), (1664, 10240)])
+@pytest.mark.parametrize("rows", [2, 3, 4, 5, 8, 9, 15, 16])
+def test_half_block_batch_kernel_edges(cuda, oracle, rows, n_in, n_out):
+    """Layers that do not fill the chip, 2..16 rows: one workgroup with two busy waves, a last
+    workgroup that is not full, accumulators and partial rows, plain signs, general scales and none,
+    two members with rotations of their own, activations off any 4-byte grid; the call after it
+    finds the counters clean. The bound is the layer's: fp16 output and fp16 rotation, and up to 8
+    rows the exact sum of a weight's halves (4.8e-4 rel-L2 at most)."""
+    from ponyexl3_amd import make_exl3_layer, ops
+
+    rng = np.random.default_rng(rows * 7 + n_in)
+    k, cb = [(4, 0), (6, 1), (3, 2), (8, 0), (5, 1)][(rows + n_in // 128) % 5]
+    layer = make_exl3_layer(k=k, in_features=n_in, out_features=n_out, seed=rows, mcg=cb == 1, mul1=cb == 2, bias=True)
+    tr = ops.as_trellis_tensor(layer.trellis, cuda)
+    svh, bias = torch.from_numpy(layer.svh).to(cuda), torch.from_numpy(layer.bias).to(cuda)
+    xs = rng.standard_normal((rows, n_in)).astype(np.float16)
+    shifted = torch.empty(rows * n_in + 1, dtype=torch.float16, device=cuda)[1:].view(rows, n_in)
+    shifted.copy_(torch.from_numpy(xs))
+    signs = layer.suh.astype(np.float16)
+    general = (signs.astype(np.float32) * rng.uniform(0.5, 2.0, n_in)).astype(np.float16)
+    big = n_in * n_out > 1 << 22  # (the oracle's time)
+    for name, suh in (("signs", signs), ("general", general), ("none", None)):
+        if big and name != "general":
+            continue
+        st = None if suh is None else torch.from_numpy(suh).to(cuda)
+        print(f"batch rows={rows} {n_in}->{n_out} k={k} cb={cb} {name}", flush=True)
+        y = ops.linear_forward(shifted, tr, k, cb, st, svh, bias)
+        ref = oracle.linear_forward(layer.trellis, k, cb, np.ones(n_in, np.float16) if suh is None else suh, layer.svh,
+                                    xs, bias=layer.bias)
+        assert rel_l2(y.cpu().numpy(), ref) <= TOL
+        assert torch.equal(ops.linear_forward(shifted, tr, k, cb, st, svh, bias), y)
+    if n_out >= 256 and not big:
+        half = n_out // 256 * 128
+        sub = torch.zeros(n_out // 128, dtype=torch.int32, device=cuda)
+        sub[half // 128:] = 1
+        both = torch.from_numpy(np.stack([signs, general])).to(cuda)
+        y = ops.linear_forward(shifted, tr, k, cb, both, svh, bias, group_sub=sub, member_out=[half, n_out - half])
+        for cols, suh in ((slice(0, half), signs), (slice(half, n_out), general)):
+            ref = oracle.linear_forward(layer.trellis, k, cb, suh, layer.svh, xs, bias=layer.bias)
+            assert rel_l2(y.cpu().numpy()[:, cols], ref[:, cols]) <= TOL
+    ops.check_counters(cuda)
+
 
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("cb", [0, 1, 2])
