@@ -391,6 +391,31 @@ int exl3_moe_forward(const uint16_t *x, int tokens, const int32_t *indices, int 
 size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
 
 /*
+ * exl3_moe_route, exl3_moe_forward and exl3_moe_combine as one call (ponyexl3/mlx/exl3_moe.py:817-839)
+ * with the same results. A few slots (those whose gate and up reduce through accumulators, at
+ * most 256 experts to rank) take two launches: the experts' kernel ranks the logits of its token
+ * itself; the wave that stores the last slot of a token's column block adds the block's slots.
+ *   logits         fp16 [tokens][n_router]; shared_logits fp16 [tokens] or NULL, the shared
+ *                  expert being the last of num_experts (n_router = num_experts - 1)
+ *   indices, scores, slot_rows  scratch that ends up as the routing table, int32 and fp16
+ *                  [tokens][kk], and the slots' rows, fp16 [tokens][kk][D], kk = top_k plus the shared
+ *                  expert; slot_rows and out 16-byte aligned
+ *   out            fp16 [tokens][D]
+ *   workspace      at least exl3_moe_workspace_bytes(tokens, kk, D, H)
+ *   counters       int32 [counters_len], counters_len >= exl3_moe_decode_counters(tokens, kk, D, H),
+ *                  8-byte aligned, zero on entry and on exit; the last int is the status word
+ * tokens * kk <= 4096; the limits of exl3_moe_route.
+ */
+size_t exl3_moe_decode_counters(int tokens, int slots_per_token, int D, int H);
+int exl3_moe_decode(const uint16_t *x, int tokens, const uint16_t *logits,
+                    const uint16_t *shared_logits, int n_router, int top_k, int norm,
+                    const uint16_t *gu_trellis, const uint16_t *gu_suh, const uint16_t *gu_svh,
+                    const uint16_t *dn_trellis, const uint16_t *dn_suh, const uint16_t *dn_svh,
+                    int num_experts, int D, int H, int K, int cb, int activation, int32_t *indices,
+                    uint16_t *scores, uint16_t *slot_rows, uint16_t *out, void *workspace,
+                    size_t workspace_bytes, int32_t *counters, size_t counters_len, void *stream);
+
+/*
  * A layer on up to 1024 already rotated rows: every weight is decoded once
  * per up to 128 rows and goes from registers into the matrix pipe; output transform
  * (Hadamard-128, svh, bias) included. Members of a sibling-fused layer may end on any

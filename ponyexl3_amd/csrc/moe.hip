@@ -32,6 +32,7 @@
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 #include "exl3_glu.hpp"
+#include "exl3_route.hpp"
 #include "exl3_small.hpp"
 
 #include <algorithm>
@@ -224,6 +225,87 @@ __device__ __forceinline__ void moe_finish_block(float2_t sum, half2_t sv, int l
     o1 = (float)(half_t)(b * kHadScaleF * (float)sv.y);
 }
 
+// Routing by the expert kernel itself, from the router's logits: 3.4 us in front of the first weights
+// (8.0 -> 11.4 us) where a launch of its own in between takes 4.0 us and a gap of about 1, and 3.5 us of host time. Every wave finds the expert of its slot;
+// the first workgroup of a token writes the token's row of the routing table for the launch behind.
+// logits == nullptr: the table is there.
+constexpr int kInlineRouteExperts = 256;  // four per lane
+struct MoeRoute {
+    const half_t* logits;  // fp16 [tokens][n_experts]
+    const half_t* shared_logits;
+    int n_experts, norm;
+    half_t* scores;  // fp16 [tokens][top_k], top_k with the shared expert
+};
+
+__device__ __forceinline__ int moe_route_slot(const MoeRoute& r, int s, int top_k, int* indices, bool writes, int lane) {
+    const int t = s / top_k, j = s - t * top_k, ranked = top_k - (r.shared_logits != nullptr);
+    int key[kInlineRouteExperts / 64];
+    route_probabilities<half_t>(r.logits + (size_t)t * r.n_experts, r.n_experts, lane, key);
+    RouteChoice c{0.f, 0};
+    int e = r.n_experts;  // the shared expert
+    const int rounds = writes ? ranked : min(j + 1, ranked);
+    for (int i = 0; i < rounds; i++) {
+        const int chosen = route_next(key, lane, i, c);
+        if (i == j) e = chosen;
+    }
+    if (writes) route_write<half_t>(c, lane, t, r.n_experts, ranked, r.norm, r.shared_logits, indices, r.scores);
+    return e;
+}
+
+// Weighted sum over the slots of a token by the wave that stores the last of them: one 128-column block o of
+// slot s goes to y[s] through the level that the XCDs share, the wave that completes
+// (token, block) adds the token's slots in slot order (the arithmetic of moe_combine_kernel). A launch
+// of its own behind the experts takes 2.4 us and a gap, this 1.6. scores == nullptr: rows only. The
+// block at one token (2048 x 512, 8 of 256 experts): five launches 28.0 us, three 21.2.
+struct MoeCombine {
+    const half_t* scores;  // fp16 [tokens][top_k]
+    half_t* out;           // fp16 [tokens][D]
+    int* counters;         // int32 [tokens][D/128], zero on entry and exit
+    int top_k;
+};
+
+__device__ __forceinline__ void moe_store_row(const MoeCombine& c, half_t* y, int s, int og, int D, half2_t o, int lane) {
+    half_t* at = y + (size_t)s * D + og * 128 + 2 * lane;
+    if (!c.scores) {
+        *reinterpret_cast<half2_t*>(at) = o;
+        return;
+    }
+    __hip_atomic_store(reinterpret_cast<uint32_t*>(at), half2_to_bits(o), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int t = s / c.top_k;
+    int* counter = c.counters + (size_t)t * (D >> 7) + og;
+    int seen = 0;
+    if (lane == 0) seen = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__shfl(seen, 0, kWave) != c.top_k - 1) return;
+    asm volatile("" ::: "memory");
+    const half_t* row = y + (size_t)t * c.top_k * D + og * 128 + 2 * lane;
+    const half_t* score = c.scores + (size_t)t * c.top_k;
+    float a = 0.f, b = 0.f;
+    for (int j0 = 0; j0 < c.top_k; j0 += 8) {
+        uint32_t v[8];
+        float w[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int jj = min(j0 + j, c.top_k - 1);
+            v[j] = __hip_atomic_load(reinterpret_cast<const uint32_t*>(row + (size_t)jj * D), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+            w[j] = (float)score[jj];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (j0 + j < c.top_k) {
+                const half2_t h = bits_to_half2(v[j]);
+                a = __builtin_fmaf((float)h.x, w[j], a);
+                b = __builtin_fmaf((float)h.y, w[j], b);
+            }
+    }
+    half2_t sum;
+    sum.x = (half_t)a;
+    sum.y = (half_t)b;
+    *reinterpret_cast<half2_t*>(c.out + (size_t)t * D + og * 128 + 2 * lane) = sum;
+    if (lane == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // grid = (slots * 2 * H/128, ceil((D/128) / 4)); wave w of workgroup (gid, q) owns
 // the Hadamard block 4q + w of D for slot s = gid / (2*hblocks), projection
 // p = (gid / hblocks) & 1 and column block hg = gid % hblocks.
@@ -311,11 +393,10 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_kernel(
 // grid = (slots * H/128, chunks); sums: uint64 [slots][2][H], zero on entry and exit.
 template <int K, int CB, bool HALF>
 __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
-    const uint32_t* __restrict__ gu_trellis, const half_t* __restrict__ x,
-    const int* __restrict__ indices, const half_t* __restrict__ gu_suh,
-    const half_t* __restrict__ gu_svh, const half_t* __restrict__ dn_suh, half_t* xh_dn,
-    unsigned long long* sums, int top_k, int E, int D, int H, int activation, int* status,
-    int spin_limit) {
+    const uint32_t* __restrict__ gu_trellis, const half_t* __restrict__ x, int* indices, MoeRoute route,
+    const half_t* __restrict__ gu_suh, const half_t* __restrict__ gu_svh,
+    const half_t* __restrict__ dn_suh, half_t* xh_dn, unsigned long long* sums, int top_k, int E, int D, int H,
+    int activation, int* status, int spin_limit) {
     __shared__ __attribute__((aligned(16))) half_t xs[8][kXwRows<1>][kXwLd];
     __shared__ float red[8][128];
     const int lane = threadIdx.x & 63;
@@ -325,7 +406,10 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
     const int gid = blockIdx.x;
     const int hg = gid % hblocks, s = gid / hblocks;
     const int p = wave >> 2, j = wave & 3;
-    const int e = clamp_expert(indices[s], E);
+    const int e = clamp_expert(
+        route.logits ? moe_route_slot(route, s, top_k, indices, blockIdx.y == 0 && hg == 0 && wave == 0 && s % top_k == 0, lane)
+                     : indices[s],
+        E);
     const int blk = HALF ? blockIdx.y * 2 + (j >> 1) : blockIdx.y * 4 + j;
     const int tk0 = blk * 8 + (HALF ? (j & 1) * 4 : 0);
     float acc[1][2] = {{0.f, 0.f}};
@@ -407,8 +491,8 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
 template <int K, int CB, int NW>
 __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
     const uint32_t* __restrict__ dn_trellis, const half_t* __restrict__ xh_dn,
-    const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* __restrict__ y,
-    float* part, int* counters, int E, int D, int H) {
+    const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* y, float* part, int* counters,
+    MoeCombine combine, int E, int D, int H) {
     __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<1>][kXwLd];
     __shared__ float red[NW][128];
     __shared__ int last_flag;
@@ -454,7 +538,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
     half2_t o;
     o.x = (half_t)o0;
     o.y = (half_t)o1;
-    *reinterpret_cast<half2_t*>(y + (size_t)s * D + og * 128 + 2 * lane) = o;
+    moe_store_row(combine, y, s, og, D, o, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -685,8 +769,8 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
 template <int K, int CB, int NW>
 __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
     const uint32_t* __restrict__ dn_trellis, const half_t* __restrict__ xh_dn,
-    const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* __restrict__ y,
-    float* part, int* counters, int slots, int E, int D, int H) {
+    const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* y, float* part, int* counters,
+    MoeCombine combine, int slots, int E, int D, int H) {
     __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<kGroupRows>][kXwLd];
     __shared__ float red[NW][kGroupRows][128];
     const int lane = threadIdx.x & 63;
@@ -746,7 +830,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
     half2_t o;
     o.x = (half_t)o0;
     o.y = (half_t)o1;
-    *reinterpret_cast<half2_t*>(y + (size_t)sr * D + og * 128 + 2 * lane) = o;
+    moe_store_row(combine, y, sr, og, D, o, lane);
 }
 
 struct MoeWorkspace {
@@ -992,26 +1076,51 @@ EXL3_EXPORT size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H)
     return exl3::moe_workspace(tokens, top_k, D, H).total;
 }
 
-EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* indices, int top_k,
-                                 const uint16_t* gu_trellis, const uint16_t* gu_suh,
-                                 const uint16_t* gu_svh, const uint16_t* dn_trellis,
-                                 const uint16_t* dn_suh, const uint16_t* dn_svh, int num_experts,
-                                 int D, int H, int K, int cb, int activation, uint16_t* y,
-                                 void* workspace, size_t workspace_bytes, int32_t* counters,
-                                 size_t counters_len, void* stream) {
-    using namespace exl3;
+namespace exl3 {
+
+// What the two entry points below share. route.logits: the table `indices` and route.scores are outputs;
+// combine.out: y holds the slots' rows in between. `counters` for the combination: combine.counters.
+struct MoeCall {
+    const uint16_t* x;
+    int tokens;
+    int32_t* indices;
+    int top_k;
+    const uint16_t *gu_trellis, *gu_suh, *gu_svh, *dn_trellis, *dn_suh, *dn_svh;
+    int num_experts, D, H, K, cb, activation;
+    uint16_t* y;
+    void* workspace;
+    size_t workspace_bytes;
+    int32_t* counters;
+    size_t counters_len;
+    MoeRoute route;
+    MoeCombine combine;
+};
+
+static int moe_slots(const MoeCall& a, hipStream_t s) {
+    const uint16_t *x = a.x, *gu_trellis = a.gu_trellis, *gu_suh = a.gu_suh, *gu_svh = a.gu_svh,
+                   *dn_trellis = a.dn_trellis, *dn_suh = a.dn_suh, *dn_svh = a.dn_svh;
+    int32_t *indices = a.indices, *counters = a.counters;
+    const int tokens = a.tokens, top_k = a.top_k, num_experts = a.num_experts, D = a.D, H = a.H, K = a.K, cb = a.cb,
+              activation = a.activation;
+    const size_t counters_len = a.counters_len;
+    uint16_t* y = a.y;
     if (int rc = check_k_cb(K, cb)) return rc;
-    if (!x || !indices || !gu_trellis || !gu_suh || !gu_svh || !dn_trellis || !dn_suh || !dn_svh ||
-        !y || !workspace)
+    if (!x || !indices || !gu_trellis || !gu_suh || !gu_svh || !dn_trellis || !dn_suh || !dn_svh || !y || !a.workspace)
         return EXL3_E_NULL_POINTER;
     if (tokens < 1 || top_k < 1 || num_experts < 1 || D < 128 || H < 128 || D % 128 || H % 128 ||
         (long long)tokens * top_k > 4096)
         return EXL3_E_BAD_SHAPE;
     if (activation != 0 && activation != 1) return EXL3_E_UNSUPPORTED;
+    // the router in a launch of its own (unless the kernel of a few slots does it)
+    auto route_table = [&]() {
+        const MoeRoute& r = a.route;
+        if (!r.logits) return (int)EXL3_OK;
+        return exl3_moe_route(r.logits, 0, r.shared_logits, tokens, r.n_experts, top_k - (r.shared_logits != nullptr),
+                              r.norm, indices, reinterpret_cast<uint16_t*>(r.scores), s);
+    };
     const MoeWorkspace w = moe_workspace(tokens, top_k, D, H);
-    if (workspace_bytes < w.total) return EXL3_E_WORKSPACE;
-    hipStream_t s = as_stream(stream);
-    char* base = reinterpret_cast<char*>(workspace);
+    if (a.workspace_bytes < w.total) return EXL3_E_WORKSPACE;
+    char* base = reinterpret_cast<char*>(a.workspace);
     half_t* xh_gu = reinterpret_cast<half_t*>(base + w.o_xh_gu);
     half_t* xh_dn = reinterpret_cast<half_t*>(base + w.o_xh_dn);
     int* gu_sub = reinterpret_cast<int*>(base + w.o_tables);
@@ -1043,13 +1152,16 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
                           (long long)slots * 2 * H * pair_chunks <= moe_max_atomics() &&
                           counters_len >= pair_ints + (size_t)slots * dblocks &&
                           (reinterpret_cast<uintptr_t>(counters) & 7) == 0;
+        const bool routes = pair && a.route.n_experts <= kInlineRouteExperts;
+        if (!routes)
+            if (int rc = route_table()) return rc;
         auto chain = [&](auto k, auto c, auto nw) {
             constexpr int NW = nw.value;
             if (pair) {
                 moe_gateup_pair_kernel<k.value, c.value, NW == 8>
                     <<<dim3((unsigned)(slots * hblocks), (unsigned)pair_chunks), dim3(512), 0, s>>>(
                         reinterpret_cast<const uint32_t*>(gu_trellis),
-                        reinterpret_cast<const half_t*>(x), indices,
+                        reinterpret_cast<const half_t*>(x), indices, routes ? a.route : MoeRoute{},
                         reinterpret_cast<const half_t*>(gu_suh),
                         reinterpret_cast<const half_t*>(gu_svh),
                         reinterpret_cast<const half_t*>(dn_suh), xh_dn,
@@ -1064,7 +1176,7 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
                        dim3(NW * 64), 0, s>>>(reinterpret_cast<const uint32_t*>(dn_trellis), xh_dn,
                                               indices, reinterpret_cast<const half_t*>(dn_svh),
                                               reinterpret_cast<half_t*>(y), part_dn,
-                                              counters + pair_ints, num_experts, D, H);
+                                              counters + pair_ints, a.combine, num_experts, D, H);
                 return launch_status();
             }
             if (grouped) {
@@ -1083,7 +1195,7 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
                        dim3(NW * 64), 0, s>>>(reinterpret_cast<const uint32_t*>(dn_trellis), xh_dn,
                                               indices, reinterpret_cast<const half_t*>(dn_svh),
                                               reinterpret_cast<half_t*>(y), part_dn,
-                                              counters + (size_t)slots * hblocks, slots,
+                                              counters + (size_t)slots * hblocks, a.combine, slots,
                                               num_experts, D, H);
                 return launch_status();
             }
@@ -1100,7 +1212,7 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
                 <<<dim3((unsigned)(slots * dblocks), (unsigned)((hblocks + 3) / 4)), dim3(NW * 64),
                    0, s>>>(reinterpret_cast<const uint32_t*>(dn_trellis), xh_dn, indices,
                            reinterpret_cast<const half_t*>(dn_svh), reinterpret_cast<half_t*>(y),
-                           part_dn, counters + (size_t)slots * hblocks, num_experts, D, H);
+                           part_dn, counters + (size_t)slots * hblocks, a.combine, num_experts, D, H);
             return launch_status();
         };
         return dispatch_k_cb(K, cb, [&](auto k, auto c) {
@@ -1109,6 +1221,7 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
         });
     }
 
+    if (int rc = route_table()) return rc;
     {
         const int waves = slots * 2 * (D / 128);
         const int threads = waves * 64 > w.g_gu ? waves * 64 : w.g_gu;
@@ -1141,8 +1254,58 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
             part_dn, w.plan_dn.n_partials(), (size_t)w.g_dn * 128, indices,
             reinterpret_cast<const half_t*>(dn_svh), reinterpret_cast<half_t*>(y), slots, D,
             num_experts);
-        return launch_status();
+        if (int rc = launch_status()) return rc;
     }
+    if (!a.combine.scores) return EXL3_OK;
+    return exl3_moe_combine(y, reinterpret_cast<const uint16_t*>(a.combine.scores), tokens, top_k, D,
+                            reinterpret_cast<uint16_t*>(a.combine.out), s);
+}
+
+}  // namespace exl3
+
+EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* indices, int top_k,
+                                 const uint16_t* gu_trellis, const uint16_t* gu_suh,
+                                 const uint16_t* gu_svh, const uint16_t* dn_trellis,
+                                 const uint16_t* dn_suh, const uint16_t* dn_svh, int num_experts,
+                                 int D, int H, int K, int cb, int activation, uint16_t* y,
+                                 void* workspace, size_t workspace_bytes, int32_t* counters,
+                                 size_t counters_len, void* stream) {
+    using namespace exl3;
+    return moe_slots({x, tokens, const_cast<int32_t*>(indices), top_k, gu_trellis, gu_suh, gu_svh, dn_trellis, dn_suh,
+                      dn_svh, num_experts, D, H, K, cb, activation, y, workspace, workspace_bytes, counters,
+                      counters_len, {}, {}},
+                     as_stream(stream));
+}
+
+EXL3_EXPORT size_t exl3_moe_decode_counters(int tokens, int slots_per_token, int D, int H) {
+    if (tokens < 1 || slots_per_token < 1 || D < 128 || H < 128) return 0;
+    return (size_t)tokens * slots_per_token * ((size_t)4 * H + D / 128) + (size_t)tokens * (D / 128) + 2;
+}
+
+EXL3_EXPORT int exl3_moe_decode(const uint16_t* x, int tokens, const uint16_t* logits, const uint16_t* shared_logits,
+                                int n_router, int top_k, int norm, const uint16_t* gu_trellis, const uint16_t* gu_suh,
+                                const uint16_t* gu_svh, const uint16_t* dn_trellis, const uint16_t* dn_suh,
+                                const uint16_t* dn_svh, int num_experts, int D, int H, int K, int cb, int activation,
+                                int32_t* indices, uint16_t* scores, uint16_t* slot_rows, uint16_t* out,
+                                void* workspace, size_t workspace_bytes, int32_t* counters, size_t counters_len,
+                                void* stream) {
+    using namespace exl3;
+    if (!logits || !indices || !scores || !slot_rows || !out || !counters) return EXL3_E_NULL_POINTER;
+    if (tokens < 1 || n_router < 1 || top_k < 1 || top_k > n_router || D < 128 || H < 128 || D % 128 || H % 128 ||
+        n_router + (shared_logits != nullptr) > num_experts || (shared_logits && n_router != num_experts - 1))
+        return EXL3_E_BAD_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(slot_rows) & 15) || (reinterpret_cast<uintptr_t>(out) & 15)) return EXL3_E_BAD_SHAPE;
+    const int kk = top_k + (shared_logits != nullptr);
+    if (counters_len < exl3_moe_decode_counters(tokens, kk, D, H)) return EXL3_E_WORKSPACE;
+    // the combination's counters lie in front of the status word
+    const size_t own = (size_t)tokens * (D / 128);
+    int32_t* const combine = counters + counters_len - 2 - own;
+    const MoeRoute route{reinterpret_cast<const half_t*>(logits), reinterpret_cast<const half_t*>(shared_logits), n_router,
+                         norm, reinterpret_cast<half_t*>(scores)};
+    return moe_slots({x, tokens, indices, kk, gu_trellis, gu_suh, gu_svh, dn_trellis, dn_suh, dn_svh, num_experts, D, H, K,
+                      cb, activation, slot_rows, workspace, workspace_bytes, counters, counters_len, route,
+                      {reinterpret_cast<const half_t*>(scores), reinterpret_cast<half_t*>(out), combine, kk}},
+                     as_stream(stream));
 }
 
 EXL3_EXPORT int exl3_moe_sort(const int32_t* indices, int n_pairs, int top_k, int n_experts,

@@ -6,62 +6,15 @@
 // are one launch before the experts and one behind them.
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
+#include "exl3_route.hpp"
 
 namespace exl3 {
 
 constexpr int kRouteMaxExperts = 1024;  // 16 per lane
 constexpr int kRouteMaxTopK = 64;       // one per lane
 
-template <int CTRL>
-__device__ __forceinline__ int dpp_i32(int v) {
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
-}
-__device__ __forceinline__ void swap16_i32(int& a, int& b) {
-    float x = __builtin_bit_cast(float, a), y = __builtin_bit_cast(float, b);
-    swap_rows16(x, y);
-    a = __builtin_bit_cast(int, x);
-    b = __builtin_bit_cast(int, y);
-}
-__device__ __forceinline__ void swap32_i32(int& a, int& b) {
-    float x = __builtin_bit_cast(float, a), y = __builtin_bit_cast(float, b);
-    swap_halves32(x, y);
-    a = __builtin_bit_cast(int, x);
-    b = __builtin_bit_cast(int, y);
-}
-// op over the wave, the result in every lane: lanes 1, 2, 4, 8 apart through DPP operands
-// (quad permutations, mirrors), 16 and 32 apart by swapping registers
-template <typename Op>
-__device__ __forceinline__ int wave_all(int v, Op op) {
-    v = op(v, dpp_i32<0xB1>(v));
-    v = op(v, dpp_i32<0x4E>(v));
-    v = op(v, dpp_i32<0x141>(v));
-    v = op(v, dpp_i32<0x140>(v));
-    int a = v, b = v;
-    swap16_i32(a, b);
-    v = op(a, b);
-    a = v, b = v;
-    swap32_i32(a, b);
-    return op(a, b);
-}
-__device__ __forceinline__ int wave_max_i32(int v) {
-    return wave_all(v, [](int a, int b) { return a > b ? a : b; });
-}
-__device__ __forceinline__ float wave_max_f32(float v) {
-    return __builtin_bit_cast(float, wave_all(__builtin_bit_cast(int, v), [](int a, int b) {
-                                  return __builtin_bit_cast(int, __builtin_fmaxf(__builtin_bit_cast(float, a),
-                                                                                 __builtin_bit_cast(float, b)));
-                              }));
-}
-__device__ __forceinline__ float wave_sum_f32(float v) {
-    return __builtin_bit_cast(float, wave_all(__builtin_bit_cast(int, v), [](int a, int b) {
-                                  return __builtin_bit_cast(int, __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b));
-                              }));
-}
-
-// One wave per token; lane l holds experts l, l + 64, ..: softmax in fp32, then top_k rounds
-// of "largest probability, lowest expert among equals" (probabilities are non-negative, so
-// their bits order like they do; a taken or absent expert is -1). Lane j keeps choice j.
-// With a shared expert its index n_experts and sigmoid(shared logit) follow the top_k.
+// One wave per token, see route_probabilities() and route_next(). With a shared expert its index n_experts
+// and sigmoid(shared logit) follow the top_k.
 template <typename T, int EPL>
 __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ logits,
                                                         const T* __restrict__ shared_logits, int tokens,
@@ -70,57 +23,11 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const T* __restrict__ lo
     const int lane = threadIdx.x & 63;
     const long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t >= tokens) return;
-    const T* row = logits + t * n_experts;
-    float v[EPL], m = -__builtin_inff();
-#pragma unroll
-    for (int i = 0; i < EPL; i++) {
-        v[i] = i * 64 + lane < n_experts ? (float)row[i * 64 + lane] : -__builtin_inff();
-        m = __builtin_fmaxf(m, v[i]);
-    }
-    m = wave_max_f32(m);
-    float sum = 0.f;
-#pragma unroll
-    for (int i = 0; i < EPL; i++) {
-        v[i] = expf(v[i] - m);  // 0 where there is no expert
-        sum += v[i];
-    }
-    sum = wave_sum_f32(sum);
     int key[EPL];
-#pragma unroll
-    for (int i = 0; i < EPL; i++)
-        key[i] = i * 64 + lane < n_experts ? __builtin_bit_cast(int, v[i] / sum) & 0x7FFFFFFF : -1;
-    float chosen = 0.f;
-    int chosen_e = 0;
-    for (int j = 0; j < top_k; j++) {
-        int best = key[0];
-#pragma unroll
-        for (int i = 1; i < EPL; i++) best = key[i] > best ? key[i] : best;
-        best = __builtin_amdgcn_readfirstlane(wave_max_i32(best));
-        int e = 0;
-#pragma unroll
-        for (int i = EPL - 1; i >= 0; i--) {
-            const unsigned long long hit = __ballot(key[i] == best);
-            if (hit) e = i * 64 + (int)__builtin_ctzll(hit);
-        }
-#pragma unroll
-        for (int i = 0; i < EPL; i++)
-            if (e == i * 64 + lane) key[i] = -1;
-        if (lane == j) {
-            chosen = __builtin_bit_cast(float, best);
-            chosen_e = e;
-        }
-    }
-    if (norm) chosen = chosen / wave_sum_f32(chosen);
-    const int slots = top_k + (shared_logits != nullptr);
-    if (lane < top_k) {
-        indices[t * slots + lane] = chosen_e;
-        scores[t * slots + lane] = (half_t)chosen;
-    }
-    if (shared_logits && lane == 0) {
-        const float s = (float)shared_logits[t];
-        indices[t * slots + top_k] = n_experts;
-        scores[t * slots + top_k] = (half_t)(float)(T)(1.0f / (1.0f + expf(-s)));
-    }
+    route_probabilities<T, EPL>(logits + t * n_experts, n_experts, lane, key);
+    RouteChoice c{0.f, 0};
+    for (int j = 0; j < top_k; j++) route_next<EPL>(key, lane, j, c);
+    route_write<T>(c, lane, (int)t, n_experts, top_k, norm, shared_logits, indices, scores);
 }
 
 // Router logits of a few tokens: logits[t][e] = fp16(x[t] . w[e]), the shared gate's row (if

@@ -500,6 +500,48 @@ PyObject* experts_slots(PyObject* self, PyObject* args) {
 // module: its kernel is made for one round trip to memory, not for throughput.
 constexpr int64_t kGateMaxTokens = 32;
 
+// Router table, experts and weighted sum of a call on the slot kernels: one call, whose tables and slot
+// rows lie in the stream's scratch behind the kernels' workspace. x (tokens, D), logits fp16 (tokens,
+// n_router) and shared logits or null: device addresses; or w (and w_shared): the gate weights that they
+// are computed from. False where the slot kernels do not take the call at once.
+bool experts_decode(const ExpertStack& m, StreamContext& ctx, const at::Tensor& x, int64_t tokens, const uint16_t* logits,
+                    const uint16_t* shared, const at::Tensor& w, const at::Tensor& w_shared, int64_t n_router, int top_k,
+                    bool has_shared, int norm, const at::Tensor& y) {
+    const int E = m.experts(), D = m.dim(), H = m.hidden(), kk = top_k + has_shared;
+    if (n_router + has_shared > E || n_router > 1024 || (has_shared && n_router != E - 1) || top_k > n_router ||
+        tokens * kk > 4096 || !aligned16({&y}))
+        return false;
+    const int t = static_cast<int>(tokens);
+    size_t at = 0;
+    auto take = [&at](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    const size_t ws_bytes = exl3_moe_workspace_bytes(t, kk, D, H);
+    const size_t o_ws = take(ws_bytes), o_logits = take(w.defined() ? tokens * (n_router + has_shared) * 2 : 0),
+                 o_idx = take(tokens * kk * 4), o_scores = take(tokens * kk * 2), o_rows = take(tokens * kk * D * 2);
+    char* base = static_cast<char*>(ctx.get(kWorkspace, at).mutable_data_ptr());
+    const size_t n_cnt = exl3_moe_decode_counters(t, kk, D, H);
+    const at::Tensor& cnt = ctx.get(kCounters, n_cnt);
+    if (w.defined()) {
+        uint16_t* out = reinterpret_cast<uint16_t*>(base + o_logits);
+        check_status(exl3_moe_gate(half_ptr(x), t, D, half_ptr(w), static_cast<int>(n_router), half_ptr(w_shared), out,
+                                   has_shared ? out + tokens * n_router : nullptr, ctx.stream),
+                     "exl3_moe_gate");
+        logits = out;
+        shared = has_shared ? out + tokens * n_router : nullptr;
+    }
+    check_status(exl3_moe_decode(half_ptr(x), t, logits, shared, static_cast<int>(n_router), top_k, norm,
+                                 half_ptr(m.gu_trellis), half_ptr(m.gu_suh), half_ptr(m.gu_svh), half_ptr(m.dn_trellis),
+                                 half_ptr(m.dn_suh), half_ptr(m.dn_svh), E, D, H, m.k, m.cb, m.activation,
+                                 reinterpret_cast<int32_t*>(base + o_idx), reinterpret_cast<uint16_t*>(base + o_scores),
+                                 reinterpret_cast<uint16_t*>(base + o_rows), half_out(y), base + o_ws, ws_bytes,
+                                 static_cast<int32_t*>(cnt.mutable_data_ptr()), n_cnt, ctx.stream),
+                 "exl3_moe_decode");
+    return true;
+}
+
 PyObject* import_class(const char* module, const char* name) {
     PyObject* mod = PyImport_ImportModule(module);
     PyObject* cls = mod ? PyObject_GetAttrString(mod, name) : nullptr;
@@ -638,6 +680,11 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
         if (w.defined() && !(grad && w.requires_grad()) &&
             (!has_shared || (ws.defined() && ws.size(0) == 1 && !(grad && ws.requires_grad())))) {
             const int64_t E = w.size(0);
+            if (!prefill) {
+                at::Tensor y = at::empty(x.sizes(), x.options());
+                if (experts_decode(m, ctx, x, tokens, nullptr, nullptr, w, ws, E, top_k, has_shared, norm, y))
+                    return THPVariable_Wrap(std::move(y));
+            }
             const at::Tensor out = at::empty({tokens * (E + has_shared)}, x.options());
             logits = out.narrow(0, 0, tokens * E).view({tokens, E});
             if (has_shared) shared = out.narrow(0, tokens * E, tokens);
@@ -670,6 +717,10 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
         THPObjectPtr s(has_shared ? THPVariable_Wrap(shared.view({1, tokens, 1})) : Py_NewRef(Py_None));
         return PyTuple_Pack(2, l.get(), s.get());
     }
+    at::Tensor y = at::empty(x.sizes(), x.options());
+    if (!prefill && logits.scalar_type() == at::kHalf &&
+        experts_decode(m, ctx, x, tokens, half_ptr(logits), half_ptr(shared), {}, {}, n_experts, top_k, has_shared, norm, y))
+        return THPVariable_Wrap(std::move(y));
     const int64_t kk = top_k + has_shared;
     // indices and scores in one allocation
     const at::Tensor routing = at::empty({tokens * kk * 6}, x.options().dtype(at::kByte));
@@ -680,7 +731,6 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
                                 static_cast<int>(n_experts), top_k, norm, static_cast<int32_t*>(idx.mutable_data_ptr()),
                                 half_out(scores), ctx.stream),
                  "exl3_moe_route");
-    at::Tensor y = at::empty(x.sizes(), x.options());
     experts_run(m, x, idx, scores, prefill != 0, y);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS

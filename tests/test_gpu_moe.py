@@ -711,3 +711,57 @@ def test_gate_kernel_against_float64(cuda, tokens, E, D, shared):
     torch.testing.assert_close(logits.cpu().double(), ref[:, :E], rtol=6e-4, atol=1e-5)
     if shared:
         torch.testing.assert_close(sl.cpu().double(), ref[:, E], rtol=6e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("tokens,E,D,H,top_k", [(1, 1, 128, 128, 1), (1, 8, 256, 768, 8), (2, 64, 1152, 256, 5),
+                                                (3, 255, 2048, 512, 8), (5, 256, 640, 640, 7), (4, 300, 384, 256, 6),
+                                                (40, 16, 256, 384, 4), (9, 32, 256, 128, 4)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_decode_call_equals_its_parts(cuda, tokens, E, D, H, top_k, shared):
+    """exl3_moe_decode against exl3_moe_route, exl3_moe_forward and exl3_moe_combine, bit for bit, in every form
+    of the slot kernels (accumulators with the routing inside, more experts than it ranks there, grouped slots,
+    several partial rows of down), on coarse logits so that ties occur; twice, so that the counters
+    are shown to come back to zero."""
+    from ponyexl3_amd import _lib, ops
+
+    lib = _lib.load()
+    g = torch.Generator(device=cuda).manual_seed(E + D + tokens)
+    rnd = lambda *s: torch.randn(s, device=cuda, generator=g)
+    n = E + shared
+    k, cb = 4, E % 2
+    tr = lambda a, b: torch.randint(-32768, 32768, (a // 16, b // 16, 16 * k), dtype=torch.int16, device=cuda, generator=g)
+    gu, dn = tr(D, n * 2 * H), tr(H, n * D)
+    gu_suh, gu_svh = rnd(n, 2, D).sign().half(), (rnd(n, 2 * H).sign() / D ** 0.5).half()
+    dn_suh, dn_svh = rnd(n, H).sign().half(), (rnd(n, D).sign() / H ** 0.5).half()
+    x = rnd(tokens, D).half()
+    logits, sl = ((rnd(tokens, E) * 4).round() / 4).half(), rnd(tokens).half()
+    kk = top_k + shared
+    weights = [ops._ptr(t) for t in (gu, gu_suh, gu_svh, dn, dn_suh, dn_svh)]
+    idx, scores = torch.zeros((tokens, kk), dtype=torch.int32, device=cuda), torch.zeros((tokens, kk), device=cuda).half()
+    rows, out = torch.zeros((tokens, kk, D), device=cuda).half(), torch.zeros((tokens, D), device=cuda).half()
+    ws = torch.zeros(lib.exl3_moe_workspace_bytes(tokens, kk, D, H), dtype=torch.uint8, device=cuda)
+    n_cnt = lib.exl3_moe_decode_counters(tokens, kk, D, H)
+    cnt = torch.zeros(n_cnt, dtype=torch.int32, device=cuda)
+    sp = ops._ptr(sl) if shared else None
+    print(f"moe decode tokens={tokens} E={E} D={D} H={H} top_k={top_k} shared={shared}", flush=True)
+    _lib.check(lib.exl3_moe_route(ops._ptr(logits), 0, sp, tokens, E, top_k, 1, ops._ptr(idx), ops._ptr(scores),
+                                  ops._stream()), "route")
+    _lib.check(lib.exl3_moe_forward(ops._ptr(x), tokens, ops._ptr(idx), kk, *weights, n, D, H, k, cb, 0, ops._ptr(rows),
+                                    ops._ptr(ws), ws.numel(), ops._ptr(cnt), n_cnt, ops._stream()), "forward")
+    _lib.check(lib.exl3_moe_combine(ops._ptr(rows), ops._ptr(scores), tokens, kk, D, ops._ptr(out), ops._stream()),
+               "combine")
+    want = [t.clone() for t in (idx, scores, rows, out)]
+    for _ in range(2):
+        for t in (idx, scores, rows, out):
+            t.fill_(-1)
+        rc = lib.exl3_moe_decode(ops._ptr(x), tokens, ops._ptr(logits), sp, E, top_k, 1, *weights, n, D, H, k, cb, 0,
+                                 ops._ptr(idx), ops._ptr(scores), ops._ptr(rows), ops._ptr(out), ops._ptr(ws),
+                                 ws.numel(), ops._ptr(cnt), n_cnt, ops._stream())
+        _lib.check(rc, "decode")
+        for got, ref in zip((idx, scores, rows, out), want):
+            assert torch.equal(got, ref)
+        assert int(cnt.abs().sum()) == 0
+    assert not torch.isnan(out.float()).any()
+    assert lib.exl3_moe_decode(ops._ptr(x), tokens, ops._ptr(logits), sp, E, top_k, 1, *weights, n, D, H, k, cb, 0,
+                               ops._ptr(idx), ops._ptr(scores), ops._ptr(rows), ops._ptr(out), ops._ptr(ws),
+                               ws.numel(), ops._ptr(cnt), n_cnt - 1, ops._stream()) != 0
