@@ -13,13 +13,15 @@
 // One workgroup of 1024 lanes per CU evaluates all 65536 codewords of a step, 64 per
 // lane, and keeps only the minimum per state: which fresh value won matters for the 256
 // states on the final path alone, so the backtrack works it out again for those from the
-// cost rows of the pass (kept in the caller's workspace, 256 x 2^(16-K) halfs per tile)
+// cost rows of the pass (kept in the caller's workspace, fp16, all of them or every other one)
 // instead of every state paying for a select per candidate. A candidate then costs a
 // subtraction, an fma and half of a three-operand minimum. The backtrack of one tile is a
-// chain of 256 dependent loads; a workgroup keeps two tiles in flight and one of its waves
+// chain of dependent loads; a workgroup keeps two tiles in flight and one of its waves
 // walks the chain of one tile while all of them run the forward steps of the other.
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
+
+#include <type_traits>
 
 namespace exl3 {
 
@@ -61,18 +63,72 @@ struct SearchMap {
     static constexpr int S = K <= 6 ? 6 - K - G : 0;
     static constexpr int FS = K <= 6 ? 1 : 1 << (K - 6);
     static constexpr int NG = 1 << G, NS = 1 << S, NF = KK / FS;  // NG * NS * NF = 64
-    static constexpr int ROW_BYTES = 2 * EDGES;
-    // Byte offset of source (f, p) in a cost row. Rows of one p are 2^(K+1) bytes; the
-    // 16-byte units (8-byte at K = 2) are permuted by exclusive-or so that the lanes of a
-    // wave hit different LDS banks in both directions: consecutive p when they read, p
-    // that differ in bits K and up when they write.
+    // Costs are fp16 values. Up to K = 5 a lane uses a cost it has read for 2 (K = 2: 4) targets; there the
+    // fma gets it as fp32: with three plain registers it runs at the rate of the simple
+    // operations (2.5 cycles per wave and SIMD against 4 for the mixed one, where runs of them
+    // meet). K = 3..5: the rows in LDS hold fp32; K = 2, where a lane writes as many costs as it
+    // reads, they are converted when read. From K = 6 on every cost is used once.
+    static constexpr bool PLAIN_FMA = K <= 5, WIDE = K >= 3 && K <= 5;
+    // Rows go to the history by the lanes that make them, [lane][target][group], a store each, or (not
+    // DIRECT) as 16-byte pieces of the finished LDS row in the next step. K = 3, 4096 tiles: 9.05 ms against
+    // 9.29; K = 5 8.02 against 8.10; K = 2 10.9 against 10.6, K = 4 8.8 against 8.5.
+    static constexpr bool DIRECT = K == 3 || K == 5;
+    static constexpr int COST = WIDE ? 4 : 2, ROW_BYTES = COST * EDGES;  // row in LDS
+    static constexpr int HIST_BYTES = 2 * EDGES;                          // row in the history, fp16
+    typedef std::conditional_t<WIDE, float, half_t> cost_t;
+    // Steps that a move of the backtrack goes back. Two up to K = 3, where the 2^2K sources of the sources
+    // fit the lanes: only every other row is kept, and those rows are what the search writes most
+    // of (K = 2: 32 KB per step, at 256 CUs 6 TB/s). At K = 4 there are four to a lane, which cost more
+    // registers and time than the rows (64 tiles 604 -> 660 us).
+    static constexpr int BACK = K <= 3 ? 2 : 1;
+    // Byte offset of source (f, p) in a cost row. The 16-byte units are permuted by exclusive-or so
+    // that the lanes of a wave hit different LDS banks in both directions: consecutive p when
+    // they read, p that differ in bits K and up when they write. fp32: a plane of 2^P units for every
+    // four f; fp16: rows of one p together.
     static __device__ __forceinline__ uint32_t at(uint32_t p, uint32_t f) {
-        if constexpr (K == 2) return ((p ^ ((p >> 4) & 3)) << 3) + 2 * f;
-        else if constexpr (K == 3) return ((p ^ ((p >> 3) & 7)) << 4) + 2 * f;
-        else if constexpr (K == 4) return (((2 * p + (f >> 3)) ^ ((p >> 4) & 7)) << 4) + 2 * (f & 7);
-        else if constexpr (K == 5) return (((4 * p + (f >> 3)) ^ ((p >> 1) & 3)) << 4) + 2 * (f & 7);
-        else if constexpr (K == 6) return (((8 * p + (f >> 3)) ^ (p & 7)) << 4) + 2 * (f & 7);
-        else return (p << (K + 1)) + 2 * f;
+        if constexpr (WIDE) {
+            const uint32_t q = f >> 2;
+            uint32_t u;
+            if constexpr (K == 3) u = p ^ ((p >> 3) & 7) ^ (((p >> 6) & 1) << 3);
+            else if constexpr (K == 4) u = p ^ ((p >> 4) & 15);
+            else u = p ^ (q & 7) ^ (((p >> 5) & 1) << 3);
+            return (((q << P) + u) << 4) + 4 * (f & 3);
+        } else if constexpr (K == 2) {
+            return ((p ^ ((p >> 4) & 3)) << 3) + 2 * f;  // 8-byte units
+        } else if constexpr (K == 6) {
+            return (((8 * p + (f >> 3)) ^ (p & 7)) << 4) + 2 * (f & 7);
+        } else {
+            return (p << (K + 1)) + 2 * f;
+        }
+    }
+    // The same in a row of the history: 16-byte pieces of eight costs, piece i from hist_piece().
+    static __device__ __forceinline__ uint32_t hist_at(uint32_t p, uint32_t f) {
+        if constexpr (DIRECT) {  // the lane that made state (f, p)
+            const uint32_t e = (f << P) | p, ps = e >> K, l = e & (KK - 1);
+            constexpr int PL = P - K;
+            const uint32_t hi = ps >> PL, t = (ps & ((1u << PL) - 1)) | (hi >> G) << PL | (l >> S) << (P - G);
+            return (((t * NS + (l & (NS - 1))) * NG) + (hi & (NG - 1))) * 2;
+        } else if constexpr (WIDE) {
+            return ((((f >> 3) << P) + p) << 4) + 2 * (f & 7);
+        } else {
+            return at(p, f);
+        }
+    }
+    static __device__ __forceinline__ uint4_t hist_piece(const unsigned char* row, uint32_t i) {
+        if constexpr (!WIDE) {
+            return *reinterpret_cast<const uint4_t*>(row + 16 * i);
+        } else {
+            const uint32_t p = i & ((1u << P) - 1), f = (i >> P) * 8;
+            const float4_t a = *reinterpret_cast<const float4_t*>(row + at(p, f));
+            const float4_t b = *reinterpret_cast<const float4_t*>(row + at(p, f + 4));
+            half8_t h;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                h[c] = (half_t)a[c];  // exact
+                h[4 + c] = (half_t)b[c];
+            }
+            return __builtin_bit_cast(uint4_t, h);
+        }
     }
     // p of group g, l of target s and first fresh value of lane `tid`
     static __device__ __forceinline__ uint32_t lane_p(uint32_t tid, int g) {
@@ -149,24 +205,74 @@ __device__ __forceinline__ uint32_t search_predecessor(const half_t (&cost)[K > 
     return best < bound ? (f << M::P) | (edge >> K) : 0u;
 }
 
+// Minimum over all lanes of values that are equal within aligned groups of 2^K lanes (K = 2, 3).
+template <int K>
+__device__ __forceinline__ uint32_t groups_min(uint32_t v) {
+    if constexpr (K == 2) v = min_dpp<0x141>(v);
+    v = min_dpp<0x140>(v);
+    if constexpr (K == 3) {  // (K = 2: the sixteen lanes repeat)
+        float a = __builtin_bit_cast(float, v), b = a;
+        swap_rows16(a, b);
+        uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        v = x < y ? x : y;
+        a = __builtin_bit_cast(float, v), b = a;
+        swap_halves32(a, b);
+        x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+        v = x < y ? x : y;
+    }
+    return v;
+}
+
+// Two steps of the backtrack at once (K <= 3): lane (f1, f2), f2 the low K bits, has in `cost` the cost, two
+// steps back, of the source f2 of the source f1 of state `edge`. The costs in between are those of the
+// forward pass: minimum over f2, rounded to fp16. t1, t2: targets of the later and the earlier step.
+// Returns the state in between and sets `edge` to the one before; `fetch` gives the costs of the
+// sources of state 0, which stands in where no candidate stays under the bound.
+template <int K, int CB, class Fetch>
+__device__ __forceinline__ uint32_t search_two_back(half_t cost, uint32_t& edge, float t1, float t2, int lane,
+                                                    Fetch&& fetch) {
+    using M = SearchMap<K>;
+    constexpr uint32_t KK = M::KK;
+    const uint32_t bound = __builtin_bit_cast(uint32_t, kCostInf), p = edge >> K;
+    const uint32_t f2 = lane & (KK - 1), f1 = ((uint32_t)lane >> K) & (KK - 1);
+    const float d2 = decode1_f32<CB>((f2 << M::KR) | (f1 << M::P) | p) - t2;
+    const uint32_t err2 = __builtin_bit_cast(uint32_t, __builtin_fmaf(d2, d2, (float)cost));
+    const uint32_t best2 = wave_min<K>(err2);  // of the lane's group
+    const half_t between = (half_t)__builtin_fminf(kCostInf, __builtin_bit_cast(float, best2));
+    const float d1 = decode1_f32<CB>((f1 << M::KR) | edge) - t1;
+    const uint32_t err1 = __builtin_bit_cast(uint32_t, __builtin_fmaf(d1, d1, (float)between));
+    const uint32_t best1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)groups_min<K>(err1));
+    if (best1 >= bound) {
+        const half_t c[1] = {fetch()};
+        edge = search_predecessor<K, CB>(c, 0u, t2, lane);
+        return 0u;
+    }
+    // lowest f1 and, in its group, lowest f2 that attain the minima
+    const int first = (int)__builtin_ctzll(__ballot(err1 == best1)) & ~(int)(KK - 1);
+    const uint32_t mid = ((uint32_t)(first >> K) << M::P) | p;
+    const uint32_t best = (uint32_t)__builtin_amdgcn_readlane((int)best2, first);
+    const unsigned long long hit = __ballot(err2 == best) >> first;
+    edge = best < bound ? ((uint32_t)__builtin_ctzll(hit) << M::P) | (mid >> K) : 0u;
+    return mid;
+}
+
 // Workgroup b walks over tiles b, b + gridDim.x, .. in phases of 256 steps. With two
 // cost-history slots (b + gridDim.x < n_slots) phase n runs the forward steps of slot n & 1
 // (warm-up pass, two phases later the pinned pass) and the backtrack of what slot ~n & 1 did
 // in phase n - 1; with one slot the odd phases only backtrack. (A tile
 // alone on its CU takes 0.80 ms, of which the forward steps are 0.70.)
 //
-// The kernel is bound by VALU issue: 64 candidates per lane and step are 64 subtractions,
-// 64 mixed-precision fmas (the previous cost is read as fp16) and 32 v_min3; the lane's 64
-// decoded values stay in registers as fp32 for the whole launch. 16 waves of at most 128
-// registers fill the CU, so the whole of a step hides its own LDS latency; one barrier per
-// step. Rows are copied to the history in 16-byte stores from the finished LDS row of the
-// step before, by the upper eight waves: the wave that backtracks (0) has no stores in
-// flight that its loads would have to wait for.
-// Measured on 4096 tiles: 1.36 us per step (about 2600 of its 2900 cycles are issue slots),
-// 303 k (K = 2), 361 k (3), 364-368 k (4..6), 345 k tiles/s (7, 8) and 0.8 ms for up to 256
-// tiles at once. With a compare and two selects per candidate for the backpointer, 256 lanes
-// per tile and the backtrack at the end of each pass it was 141 k, 172 k, 189-225 k, 195-217 k
-// and 1.6-2.5 ms.
+// The kernel is bound by VALU issue: 64 subtractions, 64 fmas and 32 v_min3 per lane and step, plus
+// rounding and storing the 64 / NF results; the lane's 64 decoded values stay in registers as fp32 for
+// the whole phase. Add and fma on plain registers run at 2.5 cycles per wave and SIMD where waves
+// meet in runs of them, everything else (minima, conversions, the mixed fma) at 4; fp32 matrix
+// instructions occupy the same units (16x16x1: 32 cycles for 16 differences), which pays against the
+// subtraction only beside the mixed fma. 16 waves of at most 128 registers fill the CU, so the
+// whole of a step hides its own LDS latency; one barrier per step. The wave that backtracks (0) waits for
+// its loads of a step before it stores, and in the forms that copy finished rows it stores nothing.
+// Measured, 4096 tiles (MCG), ms, before (mixed fma, fp16 rows, every row kept) and now: K = 2 13.3 -> 10.6, 3 11.4
+// -> 9.05, 4 11.1 -> 8.5, 5 11.1 -> 8.0, 6 11.2 -> 9.9, 7 11.8 -> 10.7, 8 11.8 -> 10.7; up to 256 tiles at once 0.84 -> 0.73,
+// 0.81 -> 0.63, 0.81 -> 0.61, 0.82 -> 0.61, 0.79 -> 0.70, 0.83 -> 0.76, 0.87 -> 0.78.
 template <int K, int CB>
 __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
     const float* __restrict__ tiles, float* __restrict__ q_tiles, uint16_t* __restrict__ indices,
@@ -174,7 +280,8 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
     using M = SearchMap<K>;
     constexpr int EDGES = M::EDGES, KK = M::KK, NG = M::NG, NS = M::NS, NF = M::NF, FS = M::FS;
     constexpr int NB = K > 6 ? 1 << (K - 6) : 1;
-    constexpr size_t kSlotBytes = (size_t)256 * M::ROW_BYTES;
+    constexpr size_t kSlotBytes = (size_t)256 * M::HIST_BYTES;
+    using cost_t = typename M::cost_t;
     extern __shared__ __attribute__((aligned(16))) unsigned char rows_s[];  // [2][ROW_BYTES]
     __shared__ float target_s[2][256];
     __shared__ uint16_t state_s[256];
@@ -210,32 +317,44 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
         const uint32_t back_pin = back_pass == 1 ? pin_s[slot ^ 1] : 0;
         uint32_t edge = __builtin_amdgcn_readfirstlane((int)back_edge);
 
-        // one step of the pending backtrack in two halves: request the costs in front of
-        // it, later pick the predecessor
+        // one move of the pending backtrack (one step, two up to K = 3) in two halves: request the costs in
+        // front of it, later pick the predecessor. Costs of source (f, p) after step s (-1: in front of
+        // the pinned pass, nothing but the pin):
+        auto back_cost = [&](int s, uint32_t p, uint32_t f) {
+            if (s < 0) return ((f << M::P) | p) == back_pin ? (half_t)0.0f : bits_to_half(0x7C00);
+            return *reinterpret_cast<const half_t*>(back_hist + (size_t)(s / M::BACK) * M::HIST_BYTES + M::hist_at(p, f));
+        };
         half_t cost[NB];
         auto back_request = [&](int step) {
-            const uint32_t p = edge >> K;
+            if constexpr (M::BACK == 2) {
+                const uint32_t f1 = ((uint32_t)lane >> K) & (KK - 1);
+                cost[0] = back_cost(step - 2, ((f1 << M::P) | (edge >> K)) >> K, lane & (KK - 1));
+            } else {
 #pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const uint32_t f = (uint32_t)(lane + 64 * j) & (KK - 1);
-                if (step > 0) {
-                    cost[j] = *reinterpret_cast<const half_t*>(
-                        back_hist + (size_t)(step - 1) * M::ROW_BYTES + M::at(p, f));
-                } else {  // in front of the pinned pass: nothing but the pin
-                    cost[j] = ((f << M::P) | p) == back_pin ? (half_t)0.0f : bits_to_half(0x7C00);
-                }
+                for (int j = 0; j < NB; j++) cost[j] = back_cost(step - 1, edge >> K, (uint32_t)(lane + 64 * j) & (KK - 1));
             }
         };
         auto back_take = [&](int step) {
             const int ri = (step + back_roll) & 255;
-            const uint32_t prev = search_predecessor<K, CB>(cost, edge, target_s[slot ^ 1][ri], lane);
-            if (lane == 0) state_s[ri] = (uint16_t)((prev << K) | edge);
-            edge = prev;
+            if constexpr (M::BACK == 2) {
+                const int rj = (step - 1 + back_roll) & 255;
+                const uint32_t last = edge;
+                const uint32_t mid = search_two_back<K, CB>(cost[0], edge, target_s[slot ^ 1][ri], target_s[slot ^ 1][rj],
+                                                            lane, [&] { return back_cost(step - 2, 0u, lane & (KK - 1)); });
+                if (lane == 0) {
+                    state_s[ri] = (uint16_t)((mid << K) | last);
+                    state_s[rj] = (uint16_t)((edge << K) | mid);
+                }
+            } else {
+                const uint32_t prev = search_predecessor<K, CB>(cost, edge, target_s[slot ^ 1][ri], lane);
+                if (lane == 0) state_s[ri] = (uint16_t)((prev << K) | edge);
+                edge = prev;
+            }
         };
 
         if (tile < 0) {
             if (backs)
-                for (int step = 255; step >= back_end; step--) {
+                for (int step = 255; step >= back_end; step -= M::BACK) {
                     back_request(step);
                     back_take(step);
                 }
@@ -247,14 +366,14 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
             // everywhere but at the pin keeps every other predecessor from winning.
 #pragma unroll 1
             for (uint32_t e = tid; e < (uint32_t)EDGES; e += kSearchThreads) {
-                const half_t open = pass == 0 ? (half_t)0.0f : bits_to_half(0x7C00);
-                *reinterpret_cast<half_t*>(rows_s + M::ROW_BYTES + M::at(e & ((1u << M::P) - 1), e >> M::P)) =
-                    pass == 1 && e == pin ? (half_t)0.0f : open;
+                const cost_t open = pass == 0 ? (cost_t)0.0f : (cost_t)__builtin_inff();
+                *reinterpret_cast<cost_t*>(rows_s + M::ROW_BYTES + M::at(e & ((1u << M::P) - 1), e >> M::P)) =
+                    pass == 1 && e == pin ? (cost_t)0.0f : open;
             }
             // decoded values of the lane's codewords (f, p, l), f << KR | p << K | l, for the
             // steps of this phase (kept across phases they would be live next to the
             // backtrack's own code and spill)
-            float val[NG][NS][NF];
+            float16_t val[4];  // [group][target][fresh], flat
 #pragma unroll
             for (int g = 0; g < NG; g++)
 #pragma unroll
@@ -268,7 +387,7 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
                             asm volatile("" : "+v"(v[i]));  // decoded here, not again in every step
-                            val[g][s][f + i] = v[i];
+                            val[((g * NS + s) * NF + f) / 16][((g * NS + s) * NF + f) % 16 + i] = v[i];
                         }
                     }
                 }
@@ -278,19 +397,26 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
                 const unsigned char* prev_row = rows_s + ((step & 1) ^ 1) * M::ROW_BYTES;
                 unsigned char* row = rows_s + (step & 1) * M::ROW_BYTES;
                 const float target = target_s[slot][(step + roll) & 255];
-                const int back_step = 255 - step;
+                // (a move of two steps is requested in one forward step and made in the next)
+                const int back_step = 255 - step / M::BACK * M::BACK;
                 const bool back_now = backs && back_step >= back_end;
-                if (back_now) back_request(back_step);
-                // the row before this one goes to the history (what the backtrack of the
-                // warm-up pass never reads is left out)
-                if (step > (pass == 0 ? 127 : 0)) {
-                    unsigned char* dst = hist + (size_t)(step - 1) * M::ROW_BYTES;
+                if (back_now && step % M::BACK == 0) back_request(back_step);
+                // the row before this one goes to the history (what the backtrack never reads is
+                // left out: up to K = 3 every other row, in the warm-up pass those of the first half)
+                if (!M::DIRECT && step > (pass == 0 ? 127 : 0) && step % M::BACK == 0) {
+                    unsigned char* dst = hist + (size_t)((step - 1) / M::BACK) * M::HIST_BYTES;
                     if (tid >= kSearchThreads / 2)
-                        for (uint32_t o = (tid - kSearchThreads / 2) * 16; o < (uint32_t)M::ROW_BYTES;
-                             o += 8 * kSearchThreads)
-                            *reinterpret_cast<uint4_t*>(dst + o) = *reinterpret_cast<const uint4_t*>(prev_row + o);
+                        for (uint32_t i = tid - kSearchThreads / 2; i < (uint32_t)M::HIST_BYTES / 16;
+                             i += kSearchThreads / 2)
+                            *reinterpret_cast<uint4_t*>(dst + 16 * i) = M::hist_piece(prev_row, i);
                 }
                 half_t out[NG][NS];
+                const float minus_target = -target;
+                auto differences = [&](int j) {
+                    return __builtin_amdgcn_mfma_f32_16x16x1f32(1.0f, minus_target, val[j], 0, 0, 0);
+                };
+                float16_t diff, diff_next;
+                if constexpr (!M::PLAIN_FMA) diff_next = differences(0);
 #pragma unroll
                 for (int g = 0; g < NG; g++) {
                     const uint32_t p = M::lane_p(tid, g), f0 = M::lane_f(tid);
@@ -300,26 +426,58 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
 #pragma unroll
                     for (int fc = 0; fc < NF; fc += 8) {
                         constexpr int CH = NF < 8 ? NF : 8;
-                        uint32_t w[4];
-                        if constexpr (CH == 8) {
-                            const uint4_t q = *reinterpret_cast<const uint4_t*>(prev_row + M::at(p, f0 + fc));
-                            w[0] = q.x, w[1] = q.y, w[2] = q.z, w[3] = q.w;
+                        float pc[CH];
+                        if constexpr (M::WIDE) {
+#pragma unroll
+                            for (int i = 0; i < CH; i += 4) {
+                                const float4_t q = *reinterpret_cast<const float4_t*>(prev_row + M::at(p, f0 + fc + i));
+#pragma unroll
+                                for (int c = 0; c < 4; c++) pc[i + c] = q[c];
+                            }
+                        } else if constexpr (CH == 4) {
+                            const half4_t q = *reinterpret_cast<const half4_t*>(prev_row + M::at(p, f0 + fc));
+#pragma unroll
+                            for (int c = 0; c < 4; c++) {
+                                pc[c] = (float)q[c];
+                                asm("" : "+v"(pc[c]));  // converted here, not in every fma
+                            }
                         } else {
-                            const uint2_t q = *reinterpret_cast<const uint2_t*>(prev_row + M::at(p, f0 + fc));
-                            w[0] = q.x, w[1] = q.y, w[2] = w[3] = 0;
+                            const uint4_t q = *reinterpret_cast<const uint4_t*>(prev_row + M::at(p, f0 + fc));
+                            halfs_to_floats(q, pc);  // folded into the fma
+                        }
+                        // From K = 6 on sixteen differences at a time come from the matrix pipe (-target times one
+                        // on top of the values: one rounding, as the subtraction), a batch ahead.
+                        if constexpr (!M::PLAIN_FMA) {
+                            if (fc % 16 == 0) {
+                                diff = diff_next;
+                                if (fc + 16 < NF) diff_next = differences(fc / 16 + 1);
+                            }
+                        }
+                        // differences, fmas and minima in runs: the simple operations run at their higher
+                        // rate where waves meet in them
+                        float d[NS][CH];
+                        if constexpr (M::PLAIN_FMA) {
+#pragma unroll
+                            for (int s = 0; s < NS; s++)
+#pragma unroll
+                                for (int i = 0; i < CH; i++) d[s][i] = val[((g * NS + s) * NF + fc) / 16][((g * NS + s) * NF + fc) % 16 + i] - target;
+                            __builtin_amdgcn_sched_barrier(0);
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < CH; i++) d[0][i] = diff[fc % 16 + i];
                         }
 #pragma unroll
                         for (int s = 0; s < NS; s++)
 #pragma unroll
-                            for (int i = 0; i < CH; i += 2) {
-                                const half2_t pc = bits_to_half2(w[i >> 1]);
-                                const float d0 = val[g][s][fc + i] - target, d1 = val[g][s][fc + i + 1] - target;
-                                const float e0 = __builtin_fmaf(d0, d0, (float)pc.x);
-                                const float e1 = __builtin_fmaf(d1, d1, (float)pc.y);
+                            for (int i = 0; i < CH; i++) d[s][i] = __builtin_fmaf(d[s][i], d[s][i], pc[i]);
+                        if constexpr (M::PLAIN_FMA) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int s = 0; s < NS; s++)
+#pragma unroll
+                            for (int i = 0; i < CH; i += 2)
                                 // an error at or above the bound never wins, which is all the
                                 // reference's clamp to 65504 achieves
-                                best[s] = __builtin_fminf(__builtin_fminf(best[s], e0), e1);
-                            }
+                                best[s] = __builtin_fminf(__builtin_fminf(best[s], d[s][i]), d[s][i + 1]);
                     }
 #pragma unroll
                     for (int s = 0; s < NS; s++) {
@@ -332,17 +490,31 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
                 for (int s = 0; s < NS; s++) {
                     const uint32_t e = (M::lane_p(tid, 0) << K) | M::lane_l(tid, s);
                     unsigned char* dst = row + M::at(e & ((1u << M::P) - 1), e >> M::P);
-                    if constexpr (NG == 4) {
-                        const half4_t o = {out[0][s], out[1][s], out[2][s], out[3][s]};
-                        *reinterpret_cast<half4_t*>(dst) = o;
+                    if constexpr (NG == 4 && !M::WIDE) {
+                        *reinterpret_cast<half4_t*>(dst) = half4_t{out[0][s], out[1][s], out[2][s], out[3][s]};
+                    } else if constexpr (NG == 4) {
+                        *reinterpret_cast<float4_t*>(dst) =
+                            float4_t{(float)out[0][s], (float)out[1][s], (float)out[2][s], (float)out[3][s]};
                     } else if constexpr (NG == 2) {
-                        const half2_t o = {out[0][s], out[1][s]};
-                        *reinterpret_cast<half2_t*>(dst) = o;
+                        *reinterpret_cast<float2_t*>(dst) = float2_t{(float)out[0][s], (float)out[1][s]};
                     } else {
-                        if (FS == 1 || (tid & (FS - 1)) == 0) *reinterpret_cast<half_t*>(dst) = out[0][s];
+                        if (FS == 1 || (tid & (FS - 1)) == 0) *reinterpret_cast<cost_t*>(dst) = (cost_t)out[0][s];
                     }
                 }
-                if (back_now) back_take(back_step);
+                if (back_now && step % M::BACK == M::BACK - 1) back_take(back_step);
+                if constexpr (M::DIRECT) {
+                    if (step % M::BACK == M::BACK - 1 && step >= (pass == 0 ? 127 : 0)) {
+                        typedef half_t piece_t __attribute__((ext_vector_type(NG * NS < 8 ? NG * NS : 8)));
+                        constexpr int N = sizeof(piece_t) / 2;
+#pragma unroll
+                        for (int j = 0; j < NG * NS; j += N) {
+                            piece_t h;
+#pragma unroll
+                            for (int i = 0; i < N; i++) h[i] = out[(i + j) % NG][(i + j) / NG];
+                            *reinterpret_cast<piece_t*>(hist + (size_t)(step / M::BACK) * M::HIST_BYTES + (NG * NS * tid + j) * 2) = h;
+                        }
+                    }
+                }
                 __syncthreads();
             }
         }
@@ -352,8 +524,8 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
             uint32_t key = 0xFFFFFFFFu;
 #pragma unroll 1
             for (uint32_t e = tid; e < (uint32_t)EDGES; e += kSearchThreads) {
-                const uint32_t bits = *reinterpret_cast<const uint16_t*>(
-                    rows_s + M::ROW_BYTES + M::at(e & ((1u << M::P) - 1), e >> M::P));
+                const uint32_t bits = half_to_bits((half_t) * reinterpret_cast<const cost_t*>(
+                    rows_s + M::ROW_BYTES + M::at(e & ((1u << M::P) - 1), e >> M::P)));
                 const uint32_t cand = (bits << 16) | e;
                 key = cand < key ? cand : key;
             }
@@ -447,11 +619,11 @@ EXL3_EXPORT int exl3_quantize_tiles(const float* tiles, int n_tiles, int K, int 
     // one workgroup per CU; slots beyond the grid are the workgroups' second ones
     const size_t cus = (size_t)quantize_cus();
     const size_t grid = slots < cus ? slots : cus;
-    const size_t lds = 2 * (sizeof(uint16_t) << (16 - K));  // two cost rows
     return dispatch_k_cb(K, cb, [&](auto k, auto c) {
         if constexpr (k.value < 2) {
             return (int)EXL3_E_BAD_K;
         } else {
+            constexpr size_t lds = 2 * (size_t)SearchMap<k.value>::ROW_BYTES;  // two cost rows
             if (hipFuncSetAttribute(
                     reinterpret_cast<const void*>(quantize_tiles_kernel<k.value, c.value>),
                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)

@@ -36,6 +36,25 @@ def test_same_path_as_the_oracle_search(cuda, oracle, k, cb):
     np.testing.assert_array_equal(q, oracle.decode_table(cb)[idx].astype(np.float32))
 
 
+@pytest.mark.parametrize("k", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("cb", [DEFAULT, MCG, MUL1])
+def test_costs_at_the_bound(cuda, oracle, k, cb):
+    """Positions that no candidate can reach under the bound of 65504 (the backtrack then stands on state
+    0): single ones at odd and even places, two in a row, at both ends and at the middle where the warm-up
+    pass starts, and a tile whose costs add up to the bound halfway; next to plain tiles, so that
+    two tiles are in flight. Bit for bit the oracle's path."""
+    from ponyexl3_amd import search
+
+    tiles = _tiles(40 + k, 9)
+    for i, places in enumerate(([100], [101], [150, 151], [151, 152], [0], [255], [127, 128], range(0, 256, 3))):
+        tiles[i, list(places)] = 300.0 if i < 7 else 40.0
+    print(f"search bound k={k} cb={cb}", flush=True)
+    q, idx = search.quantize_tiles_np(tiles, k, cb, device=cuda)
+    q_ref, idx_ref = oracle.quantize_tiles_search(tiles, k, cb)
+    np.testing.assert_array_equal(idx, idx_ref)
+    np.testing.assert_array_equal(q.view(np.uint32), q_ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("k,cb", [(2, MCG), (3, MCG), (4, DEFAULT), (4, MCG), (4, MUL1)])
 def test_quality_against_the_exact_search(cuda, oracle, k, cb):
     """mse <= 1.10 x the exact float64 Viterbi (tests/test_convert_metal.py:44-71)."""
