@@ -181,25 +181,10 @@ def public_weight(trellis, k: int, cb: int, suh=None, svh=None, tn_offset: int =
                   tn_count: int | None = None, transposed: bool = False):
     """Public weight of a slice of tile columns, (in, 16*tn_count) or transposed, fp16 with
     the cast points of the forward (``exl3_public_weight``); ``svh`` belongs to the slice."""
-    in_tiles, out_tiles = _trellis_dims(trellis, k)
-    if tn_count is None:
-        tn_count = out_tiles - tn_offset
-    if tn_offset < 0 or tn_count < 0 or tn_offset + tn_count > out_tiles:
+    if tn_count is not None and tn_count < 0:
         raise ValueError("slice exceeds output features")
-    n_in, n_out = in_tiles * 16, tn_count * 16
-    if n_in % 128 or n_out % 128:
-        raise ValueError("in/out features must be multiples of 128 for the Hadamard transform")
-    for name, v, n in (("suh", suh, n_in), ("svh", svh, n_out)):
-        if v is not None and _half(v, name).numel() != n:
-            raise ValueError(f"{name} length does not match the feature dim")
-    w = torch.empty((n_out, n_in) if transposed else (n_in, n_out), dtype=torch.float16, device=trellis.device)
-    if w.numel() == 0:
-        return w
-    rc = _lib.load().exl3_public_weight(
-        _ptr(trellis), in_tiles, out_tiles, int(k), int(cb), _ptr(suh), _ptr(svh), int(tn_offset), int(tn_count),
-        int(bool(transposed)), _ptr(w), _stream())
-    _lib.check(rc, "exl3_public_weight")
-    return w
+    return _lib.host().public_weight(trellis, int(k), int(cb), suh, svh, int(tn_offset),
+                                     -1 if tn_count is None else int(tn_count), bool(transposed))
 
 
 def reconstruct_inner(trellis, k: int, cb: int, n_offset: int = 0, n_count: int | None = None):

@@ -83,3 +83,39 @@ def test_folded_linear_tracks_exact_layer(cuda, oracle, bias):
     ref = oracle.linear_forward(layer.trellis, 4, int(layer.codebook_mode), layer.suh, layer.svh, x,
                                 bias=layer.bias)
     assert rel_l2(y, ref) < 2e-3
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_folded_linear_is_a_whole_module(cuda, bias):
+    """The fold builds its Linear without Linear.__init__: the same attributes, parameters and state as a
+    module built the usual way, usable and copyable like one."""
+    import copy
+
+    from ponyexl3_amd import make_exl3_layer, native
+
+    layer = make_exl3_layer(k=4, in_features=256, out_features=128, seed=5, bias=bias)
+    lin = native.folded_linear_from_exl3(layer, device=cuda)
+    ref = torch.nn.Linear(256, 128, bias=bias, device=cuda, dtype=torch.float16)
+    assert type(lin) is torch.nn.Linear and set(lin.__dict__) == set(ref.__dict__) and repr(lin) == repr(ref)
+    assert [n for n, _ in lin.named_parameters()] == [n for n, _ in ref.named_parameters()]
+    ref.load_state_dict(lin.state_dict())
+    x = torch.randn((3, 256), device=cuda).half()
+    assert torch.equal(lin(x), ref(x)) and torch.equal(copy.deepcopy(lin)(x), ref(x))
+    assert not any(p.requires_grad for p in lin.parameters())
+
+
+def test_public_weight_argument_errors(cuda):
+    from ponyexl3_amd import make_exl3_layer, ops
+
+    layer = make_exl3_layer(k=4, in_features=128, out_features=256, seed=6)
+    tr = ops.as_trellis_tensor(layer.trellis, cuda)
+    suh, svh = torch.from_numpy(layer.suh).to(cuda), torch.from_numpy(layer.svh).to(cuda)
+    bad = [(tr, 9, 0), (tr, 3, 0), (tr.view(-1), 4, 0), (tr.cpu(), 4, 0), (tr.int(), 4, 0), ("x", 4, 0), (tr, 4, 7)]
+    for args in bad:
+        with pytest.raises(ValueError):
+            ops.public_weight(*args)
+    for kw in ({"suh": suh[:64]}, {"svh": suh}, {"suh": suh.float()}, {"svh": svh.cpu()}, {"tn_offset": -1},
+               {"tn_offset": 17}, {"tn_count": -1}, {"tn_count": 4}, {"tn_offset": 8, "tn_count": 16}, {"suh": [1.0]}):
+        with pytest.raises(ValueError):
+            ops.public_weight(tr, 4, 0, **kw)
+    assert ops.public_weight(tr, 4, 0, tn_offset=16).shape == (128, 0)
