@@ -893,6 +893,7 @@ static MoeWorkspace moe_workspace(int tokens, int top_k, int D, int H) {
 
 constexpr int kSortThreads = 1024;
 constexpr int kSortMaxExperts = 1024;
+constexpr int kSortMaxGroups = 32;
 
 // Stable counting sort by expert id. Outputs, all indexed by sorted position:
 //   order[pos] = pair index (token * top_k + slot), tok[pos] = token,
@@ -901,25 +902,38 @@ constexpr int kSortMaxExperts = 1024;
 // With `staged` the order is put together in LDS and written out in order: one CU's scattered
 // 4-byte stores (64 lines per instruction) are what this kernel is otherwise bound by.
 //
-// Each of the 16 waves owns one contiguous segment of the pairs and a cursor per expert in
-// LDS: count, one scan over (expert, wave), then every wave places its segment 64 pairs at a
-// time without meeting the others. A pair's rank among equal experts of its 64 comes from
-// ballots over the bits of the expert id.
+// Every workgroup owns a contiguous part of the pairs, each of its 16 waves a segment of that and a
+// cursor per expert in LDS: count, one scan over (expert, wave), then every wave places its segment 64
+// pairs at a time without meeting the others. A pair's rank among equal experts of its 64 comes from
+// ballots over the bits of the expert id. Where a part begins is known without an exchange:
+// every workgroup counts all pairs, those before and behind its own part in two counters per expert (13 833
+// pairs: 14 loads and LDS additions per lane). There one workgroup takes 21.5 us, 14 take 8.3; 6972 pairs
+// 12.3 and 7.3.
+__host__ __device__ constexpr int sort_pairs_per_wave(int n_pairs, int groups) {
+    const long long waves = (long long)groups * (kSortThreads / 64);
+    return (int)((n_pairs + 64 * waves - 1) / (64 * waves) * 64);
+}
+
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int* __restrict__ indices, int n_pairs, int top_k, int E, int block_rows,
     int* __restrict__ order, int* __restrict__ tok, int* __restrict__ sidx,
     int4* __restrict__ table, int table_len, int staged) {
     constexpr int kWaves = kSortThreads / 64;
-    extern __shared__ int cursor[];  // [kWaves][E]
+    extern __shared__ int cursor[];  // [kWaves][E], pairs before [E], behind [E], staging
     __shared__ int scan_tmp[2][kWaves];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < kWaves * E; i += kSortThreads) cursor[i] = 0;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int* const before = cursor + kWaves * E;
+    int* const behind = before + E;
+    int* const stage = behind + E;
+    for (int i = tid; i < (kWaves + 2) * E; i += kSortThreads) cursor[i] = 0;
     __syncthreads();
-    const int per_wave = (n_pairs + 64 * kWaves - 1) / (64 * kWaves) * 64;
-    const int begin = wave * per_wave, end = min(begin + per_wave, n_pairs);
+    const int groups = gridDim.x;
+    const int per_wave = sort_pairs_per_wave(n_pairs, groups);
+    const int part = blockIdx.x * kWaves * per_wave;
+    const int begin = min(part + wave * per_wave, n_pairs), end = min(begin + per_wave, n_pairs);
     int* mine = cursor + wave * E;
-    int* stage = cursor + kWaves * E;
-    for (int i0 = begin + lane; i0 < end; i0 += 8 * 64) {  // eight loads in flight
+    // eight loads in flight
+    for (int i0 = begin + lane; groups == 1 && i0 < end; i0 += 8 * 64) {
         int e[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) e[j] = indices[min(i0 + j * 64, n_pairs - 1)];
@@ -927,13 +941,25 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
         for (int j = 0; j < 8; j++)
             if (i0 + j * 64 < end) atomicAdd(&mine[clamp_expert(e[j], E)], 1);
     }
+    for (int i0 = wave * 64; groups > 1 && i0 < n_pairs; i0 += 8 * kSortThreads) {
+        int e[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) e[j] = indices[min(i0 + j * kSortThreads + lane, n_pairs - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int i = i0 + j * kSortThreads;  // 64 pairs of one segment
+            int* const count = i < part ? before
+                               : i >= part + kWaves * per_wave ? behind : cursor + (i - part) / per_wave * E;
+            if (i + lane < n_pairs) atomicAdd(&count[clamp_expert(e[j], E)], 1);
+        }
+    }
     __syncthreads();
 
     // exclusive scans over the experts (E <= 1024 = one value per thread): rows and blocks
     int c = 0;
     if (tid < E) {
 #pragma unroll
-        for (int w = 0; w < kWaves; w++) c += cursor[w * E + tid];
+        for (int w = 0; w < kWaves + 2; w++) c += cursor[w * E + tid];
     }
     const int nb = (c + block_rows - 1) / block_rows;
     int inc_rows = c, inc_blk = nb;
@@ -962,17 +988,18 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int row0 = base_rows + inc_rows - c;  // first sorted row of expert tid
     const int blk0 = base_blk + inc_blk - nb;
     if (tid < E) {
-        int at = row0;
+        int at = row0 + before[tid];
 #pragma unroll
         for (int w = 0; w < kWaves; w++) {
             const int n = cursor[w * E + tid];
             cursor[w * E + tid] = at;
             at += n;
         }
-        for (int b = 0; b < nb && blk0 + b < table_len; b++)
-            table[blk0 + b] = int4{tid, row0 + b * block_rows, row0 + c, 0};
+        if (blockIdx.x == 0)
+            for (int b = 0; b < nb && blk0 + b < table_len; b++)
+                table[blk0 + b] = int4{tid, row0 + b * block_rows, row0 + c, 0};
     }
-    for (int b = total_blk + tid; b < table_len; b += kSortThreads)
+    for (int b = total_blk + tid + blockIdx.x * kSortThreads; b < table_len; b += kSortThreads * groups)
         table[b] = int4{E - 1, n_pairs, n_pairs, 0};
     __syncthreads();
 
@@ -1057,13 +1084,17 @@ __global__ __launch_bounds__(256) void moe_glu_rows_kernel(
 static int launch_moe_sort(const int32_t* indices, int n_pairs, int top_k, int n_experts, int block_rows,
                            int32_t* order, int32_t* tok, int32_t* sidx, int32_t* table, int table_len,
                            hipStream_t stream) {
-    size_t lds = (size_t)(kSortThreads / 64) * n_experts * sizeof(int);
-    const bool staged = lds + (size_t)n_pairs * sizeof(int) <= (size_t)150 << 10;
+    size_t lds = (size_t)(kSortThreads / 64 + 2) * n_experts * sizeof(int);
+    // a workgroup per kSortThreads pairs (64 to a wave), up to kSortMaxGroups, from the size on where
+    // one alone takes longer (1025 pairs 5.6 and 6.4 us, 2436 7.3 and 6.7)
+    const int groups =
+        n_pairs <= 2 * kSortThreads ? 1 : std::min(kSortMaxGroups, (n_pairs + kSortThreads - 1) / kSortThreads);
+    const bool staged = groups == 1 && lds + (size_t)n_pairs * sizeof(int) <= (size_t)150 << 10;
     if (staged) lds += (size_t)n_pairs * sizeof(int);
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_sort_kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return EXL3_E_LAUNCH;
-    moe_sort_kernel<<<dim3(1), dim3(kSortThreads), lds, stream>>>(indices, n_pairs, top_k, n_experts, block_rows,
+    moe_sort_kernel<<<dim3((unsigned)groups), dim3(kSortThreads), lds, stream>>>(indices, n_pairs, top_k, n_experts, block_rows,
                                                                   order, tok, sidx, reinterpret_cast<int4*>(table),
                                                                   table_len, staged);
     return launch_status();

@@ -765,3 +765,11 @@ def test_decode_call_equals_its_parts(cuda, tokens, E, D, H, top_k, shared):
     assert lib.exl3_moe_decode(ops._ptr(x), tokens, ops._ptr(logits), sp, E, top_k, 1, *weights, n, D, H, k, cb, 0,
                                ops._ptr(idx), ops._ptr(scores), ops._ptr(rows), ops._ptr(out), ops._ptr(ws),
                                ws.numel(), ops._ptr(cnt), n_cnt - 1, ops._stream()) != 0
+
+
+@pytest.mark.parametrize("pairs,E", [(2048, 9), (2049, 1), (2049, 257), (3073, 1024), (32768, 3), (32769, 300),
+                                     (65600, 64)])
+def test_pair_sort_in_several_parts(cuda, pairs, E):
+    """Sizes at which the sort changes from one workgroup to several, with a last one that holds one pair, and
+    from one round of 64 pairs per wave to two."""
+    test_pair_sort_kernel_equals_stable_argsort(cuda, pairs, 1, E, 64)
