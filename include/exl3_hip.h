@@ -519,6 +519,12 @@ int exl3_moe_gate(const uint16_t *x, int tokens, int D, const uint16_t *w, int n
 int exl3_moe_route(const void *logits, int logits_fp32, const void *shared_logits, int tokens,
                    int n_experts, int top_k, int norm, int32_t *indices, uint16_t *scores,
                    void *stream);
+/* The same for fp16 logits with the shared expert's gate computed in the launch: shared logit of a
+ * token = fp16(x . w_shared), fp32 sums; x fp16 [tokens][D], w_shared fp16 [D], both 16-byte aligned,
+ * D % 8 == 0. */
+int exl3_moe_route_shared(const uint16_t *logits, const uint16_t *x, int D, const uint16_t *w_shared,
+                          int tokens, int n_experts, int top_k, int norm, int32_t *indices,
+                          uint16_t *scores, void *stream);
 int exl3_moe_combine(const uint16_t *y, const uint16_t *scores, int tokens, int slots, int D,
                      uint16_t *out, void *stream);
 

@@ -103,19 +103,20 @@ __device__ __forceinline__ int route_next(int (&key)[EPL], int lane, int j, Rout
     return e;
 }
 
-// Row t of the routing table after top_k choices.
+// Row t of the routing table after top_k choices, with a shared expert behind them whose gate's logit
+// is given.
 template <typename T>
 __device__ __forceinline__ void route_write(RouteChoice c, int lane, int t, int n_experts, int top_k, int norm,
-                                            const T* __restrict__ shared_logits, int* __restrict__ indices,
+                                            bool shared, T shared_logit, int* __restrict__ indices,
                                             half_t* __restrict__ scores) {
     if (norm) c.p = c.p / wave_sum_f32(c.p);
-    const int slots = top_k + (shared_logits != nullptr);
+    const int slots = top_k + shared;
     if (lane < top_k) {
         indices[(size_t)t * slots + lane] = c.e;
         scores[(size_t)t * slots + lane] = (half_t)c.p;
     }
-    if (shared_logits && lane == 0) {
-        const float s = (float)shared_logits[t];
+    if (shared && lane == 0) {
+        const float s = (float)shared_logit;
         indices[(size_t)t * slots + top_k] = n_experts;
         scores[(size_t)t * slots + top_k] = (half_t)(float)(T)(1.0f / (1.0f + expf(-s)));
     }

@@ -248,7 +248,8 @@ __device__ __forceinline__ int moe_route_slot(const MoeRoute& r, int s, int top_
         const int chosen = route_next(key, lane, i, c);
         if (i == j) e = chosen;
     }
-    if (writes) route_write<half_t>(c, lane, t, r.n_experts, ranked, r.norm, r.shared_logits, indices, r.scores);
+    if (writes) route_write<half_t>(c, lane, t, r.n_experts, ranked, r.norm, r.shared_logits != nullptr,
+                                     r.shared_logits ? r.shared_logits[t] : (half_t)0.f, indices, r.scores);
     return e;
 }
 

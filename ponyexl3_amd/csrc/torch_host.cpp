@@ -672,7 +672,7 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
     if (!x.is_contiguous()) x = x.contiguous();
     StreamContext ctx(x.device().index());
 
-    at::Tensor logits, shared;
+    at::Tensor logits, shared, w_shared;  // shared logits, or the weight that the router's kernel takes for them
     const bool grad = at::GradMode::is_enabled();
     if (tokens <= kGateMaxTokens) {
         const at::Tensor w = plain_gate_weight(gate, x);
@@ -698,17 +698,22 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
         THPObjectPtr x3(THPVariable_Wrap(x.view({1, tokens, D})));
         THPObjectPtr l(PyObject_CallFunctionObjArgs(gate, x3.get(), nullptr));
         if (!l) throw python_error();
+        bool ok = usable_logits(l.get(), x, 0);
+        if (has_shared && prefill && ok && THPVariable_Unpack(l.get()).scalar_type() == at::kHalf &&
+            THPVariable_Unpack(l.get()).size(-1) == m.experts() - 1 && top_k < m.experts()) {
+            w_shared = plain_gate_weight(shared_gate, x);
+            if (w_shared.defined() && (w_shared.size(0) != 1 || (grad && w_shared.requires_grad()))) w_shared = at::Tensor();
+        }
         THPObjectPtr s;
-        if (has_shared) {
+        if (has_shared && !w_shared.defined()) {
             s = THPObjectPtr(PyObject_CallFunctionObjArgs(shared_gate, x3.get(), nullptr));
             if (!s) throw python_error();
         }
-        const bool ok = usable_logits(l.get(), x, 0) &&
-                        (!has_shared || (usable_logits(s.get(), x, 1) && THPVariable_Unpack(s.get()).scalar_type() ==
+        ok = ok && (!s || (usable_logits(s.get(), x, 1) && THPVariable_Unpack(s.get()).scalar_type() ==
                                                                              THPVariable_Unpack(l.get()).scalar_type()));
         if (!ok) return PyTuple_Pack(2, l.get(), has_shared ? s.get() : Py_None);
         logits = THPVariable_Unpack(l.get());
-        if (has_shared) shared = THPVariable_Unpack(s.get());
+        if (s) shared = THPVariable_Unpack(s.get());
     }
     const int64_t n_experts = logits.size(-1);
     if (n_experts + has_shared > m.experts() || n_experts > 1024 || (has_shared && n_experts != m.experts() - 1) ||
@@ -726,11 +731,17 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
     const at::Tensor routing = at::empty({tokens * kk * 6}, x.options().dtype(at::kByte));
     const at::Tensor idx = routing.narrow(0, 0, tokens * kk * 4).view(at::kInt).view({tokens, kk});
     const at::Tensor scores = routing.narrow(0, tokens * kk * 4, tokens * kk * 2).view(at::kHalf).view({tokens, kk});
-    check_status(exl3_moe_route(logits.const_data_ptr(), logits.scalar_type() == at::kFloat,
-                                has_shared ? shared.const_data_ptr() : nullptr, static_cast<int>(tokens),
-                                static_cast<int>(n_experts), top_k, norm, static_cast<int32_t*>(idx.mutable_data_ptr()),
-                                half_out(scores), ctx.stream),
-                 "exl3_moe_route");
+    if (w_shared.defined())
+        check_status(exl3_moe_route_shared(half_ptr(logits), half_ptr(x), D, half_ptr(w_shared), static_cast<int>(tokens),
+                                           static_cast<int>(n_experts), top_k, norm,
+                                           static_cast<int32_t*>(idx.mutable_data_ptr()), half_out(scores), ctx.stream),
+                     "exl3_moe_route_shared");
+    else
+        check_status(exl3_moe_route(logits.const_data_ptr(), logits.scalar_type() == at::kFloat,
+                                    has_shared ? shared.const_data_ptr() : nullptr, static_cast<int>(tokens),
+                                    static_cast<int>(n_experts), top_k, norm,
+                                    static_cast<int32_t*>(idx.mutable_data_ptr()), half_out(scores), ctx.stream),
+                     "exl3_moe_route");
     experts_run(m, x, idx, scores, prefill != 0, y);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS

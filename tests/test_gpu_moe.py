@@ -1,4 +1,5 @@
 """Routed MoE expert chain against the oracle's unfused per-expert chain."""
+import ctypes
 import os
 
 import numpy as np
@@ -522,6 +523,37 @@ def test_route_kernel_against_torch(cuda, tokens, E, top_k, norm, fp32, shared):
         assert (idx[:, top_k] == E).all()
         torch.testing.assert_close(scores[:, top_k].cpu().double(), torch.sigmoid(sd.cpu().double())[:, 0],
                                    rtol=1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("tokens,E,top_k,D", [(1, 4, 4, 8), (5, 64, 2, 128), (33, 129, 8, 520), (70, 256, 8, 2048),
+                                              (9, 600, 64, 2056)])
+def test_route_kernel_with_the_shared_gate(cuda, tokens, E, top_k, D):
+    """exl3_moe_route_shared: the table of exl3_moe_route, and behind it sigmoid(fp16(x . w)). The logit's error
+    is that of an fp32 sum of D terms, in any order, and of its fp16 rounding; the sigmoid's slope is at most
+    1/4; expf and the quotient add a few units of 2^-23, the fp16 result half of 2^-10."""
+    from ponyexl3_amd import _lib, ops
+
+    g = torch.Generator().manual_seed(tokens + E)
+    logits = torch.randn((tokens, E), generator=g).half().to(cuda)
+    x, w = torch.randn((tokens, D), generator=g).half(), (torch.randn((D,), generator=g) * D**-0.5).half()
+    xd, wd = x.to(cuda), w.to(cuda)
+    idx = torch.full((tokens, top_k + 1), -1, dtype=torch.int32, device=cuda)
+    scores = torch.zeros((tokens, top_k + 1), dtype=torch.float16, device=cuda)
+    want_idx, want = torch.empty_like(idx[:, :top_k]).contiguous(), torch.empty_like(scores[:, :top_k]).contiguous()
+    lib = _lib.load()
+    print(f"route shared tokens={tokens} E={E} top_k={top_k} D={D}", flush=True)
+    _lib.check(lib.exl3_moe_route_shared(ops._ptr(logits), ops._ptr(xd), D, ops._ptr(wd), tokens, E, top_k, 1,
+                                         ops._ptr(idx), ops._ptr(scores), ops._stream()), "exl3_moe_route_shared")
+    _lib.check(lib.exl3_moe_route(ops._ptr(logits), 0, None, tokens, E, top_k, 1, ops._ptr(want_idx), ops._ptr(want),
+                                  ops._stream()), "exl3_moe_route")
+    assert torch.equal(idx[:, :top_k], want_idx) and torch.equal(scores[:, :top_k], want)
+    assert bool((idx[:, top_k] == E).all())
+    xw = x.double() * w.double()
+    exact, spread = xw.sum(-1), xw.abs().sum(-1)
+    bound = 0.25 * (D * 2.0**-24 * spread + 2.0**-11 * exact.abs() + 2.0**-25) + 2.0**-11 + 2.0**-21
+    assert bool(((scores[:, top_k].cpu().double() - torch.sigmoid(exact)).abs() <= bound).all())
+    assert lib.exl3_moe_route_shared(ops._ptr(logits), ctypes.c_void_p(xd.data_ptr() + 2), D, ops._ptr(wd), tokens, E, top_k, 1,
+                                     ops._ptr(idx), ops._ptr(scores), ops._stream()) == _lib.EXL3_E_BAD_SHAPE
 
 
 @pytest.mark.parametrize("tokens,shared", [(1, False), (9, True), (30, True), (67, False)])
