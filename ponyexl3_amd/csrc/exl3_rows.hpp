@@ -22,7 +22,7 @@
 // with more rows one has it to itself. 333 rows of 17408 -> 5120 (K = 5), whole layer: 115 us with
 // words in registers and the barrier at the step's end, 101 in this form, 97 with half quads and
 // direct loads one by one between the matrix instructions; the prefill GEMM 115. 1537 tokens
-// through 257 experts: gate/up 150 us, down 85 (2.2 rounds of workgroups).
+// through 257 experts: gate/up 150 us, down 87 with two k-slices, 73 with one.
 #pragma once
 
 #include "exl3_device.hpp"
@@ -31,13 +31,15 @@ namespace exl3 {
 
 template <int MR, int NKS>
 struct RowsTile {
-    static_assert(NKS == 2 || NKS == 4, "LDS rows of 128 or 256 bytes");
+    static_assert(NKS == 1 || NKS == 2 || NKS == 4, "LDS rows of 64, 128 or 256 bytes");
     static constexpr int BM = 32 * MR, BK = 32 * NKS, CHUNKS = BK / 8;
     static constexpr int STAGE = BM * BK;              // halfs per stage
     static constexpr int FILLS = STAGE * 2 / 1024;     // wave-wide direct loads per stage
     // 16-byte chunk c of row r is stored at chunk c ^ swizzle(r): a fragment read (32 rows,
     // one chunk) then touches every bank equally
-    static __device__ __forceinline__ int swizzle(int row) { return NKS == 2 ? (row >> 1) & 7 : row & 15; }
+    static __device__ __forceinline__ int swizzle(int row) {
+        return NKS == 1 ? (row >> 2) & 3 : NKS == 2 ? (row >> 1) & 7 : row & 15;
+    }
 };
 
 // Byte offset in the activation matrix of what lane `lane` of fill `f` of a stage copies

@@ -1,6 +1,11 @@
 // Routed experts of a prefill chunk: the (token, slot) rows are sorted by expert, a
 // workgroup takes up to 64 rows of one expert through 128 columns of gate AND up or 256
-// columns of down (see exl3_rows.hpp for the contraction).
+// columns of down (see exl3_rows.hpp for the contraction): 64-column strips times NKS k-slices.
+//
+// What bounds them: issue of the decode. 1537 tokens through 257 experts, NKS = 2: VALU issue 85 % and
+// 77 % (gate/up, down) of the time that CUs are busy, which is 81 and 84 % of the time (2.2 and 4.4
+// rounds of workgroups); 25 and 36 % of the VALU instructions stood outside the main loop. Looping
+// workgroups, one launch of as many as the chip holds, were slower (gate/up 158 -> 162 us, down 94 -> 103).
 //
 // moe_gateup_rows_kernel ends with everything that stands between the two products: output
 // transform of gate and up (ponyexl3/ref/forward.py:41-42), GLU, rotation for the down
@@ -16,7 +21,6 @@
 
 namespace exl3 {
 
-constexpr int kRowsThreads = 512;
 constexpr int kYPad = 8;  // halfs: 16-byte reads of 16 tile rows hit all banks
 
 // Sums of two k-slices: the wave of slice ks keeps columns cs = ks. `ex` holds MR*4 float4 per
@@ -63,16 +67,39 @@ __device__ __forceinline__ void rows_store_half(const float16_t (&sum)[MR], half
         }
 }
 
+// The products of a wave (64 columns from `col`) as fp16 in an LDS tile [32 MR][ld], after the sum of
+// two k-slices if there are (`ex`: LDS of the exchange, over which the tile may lie).
+template <int MR, int NKS>
+__device__ __forceinline__ void rows_to_tile(float16_t (&acc)[MR][2], void* ex, half_t* tile, int ld, int col, int wave,
+                                             int lane) {
+    if constexpr (NKS == 2) {
+        float16_t sum[MR];
+        rows_add_slices2<MR>(acc, static_cast<float4_t*>(ex), wave, lane, sum);
+        rows_store_half<MR>(sum, tile, ld, col, wave & 1, lane);
+    } else {
+#pragma unroll
+        for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                half4_t o;
+#pragma unroll
+                for (int c = 0; c < 4; c++) o[c] = (half_t)acc[mr][i & 1][4 * (i >> 1) + c];
+                *reinterpret_cast<half4_t*>(tile + (mr * 32 + (lane & 31)) * ld + col + 8 * i + 4 * (lane >> 5)) = o;
+            }
+    }
+}
+
 // grid: unit = (row block b, 128-column block hg of H), dealt so that the units of a row block
 // land on one XCD (they read the same activations): b = 8 (u / (8 hblocks)) + u % 8.
 // table[b] = {expert, first row, end row of the expert, 0}, empty if first >= end.
-template <int K, int CB, int MR>
-__global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
+template <int K, int CB, int MR, int NKS>
+__global__ __launch_bounds__(256 * NKS, 4) void moe_gateup_rows_kernel(
     const uint32_t* __restrict__ trellis, const half_t* __restrict__ xg, const half_t* __restrict__ xu,
     const int4* __restrict__ table, int n_blocks, const half_t* __restrict__ gu_svh,
     const half_t* __restrict__ dn_suh, half_t* __restrict__ xd, int n_rows, int E, int D, int H, int activation) {
-    using T = RowsTile<MR, 2>;
-    constexpr int kFillWaves = 4, LPW = T::FILLS / kFillWaves;
+    using T = RowsTile<MR, NKS>;
+    constexpr int kFillWaves = 2 * NKS, LPW = T::FILLS / kFillWaves;
+    constexpr int kParts = 2 * MR / NKS;  // of a wave, of the four 32-column parts of a row tile
     constexpr int kLd = 128 + kYPad;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
@@ -86,14 +113,14 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
     if (e < 0 || e >= E || m0 < 0 || m0 >= end) return;
     const int valid = min(end - m0, T::BM);
 
-    const int proj = wave >> 2, cq = (wave >> 1) & 1, ks = wave & 1;
+    const int proj = wave / (2 * NKS), cq = (wave / NKS) & 1, ks = wave % NKS;
     const size_t row_words = (size_t)E * 2 * (H >> 4) * (8 * K);
     const uint32_t* w = trellis + (size_t)(2 * ks) * row_words +
                         ((size_t)(proj * E + e) * (H >> 4) + hg * 8 + cq * 4) * (8 * K);
     half_t* stages = reinterpret_cast<half_t*>(lds) + proj * 3 * T::STAGE;
     uint32_t a_off[LPW];
 #pragma unroll
-    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, 2>((wave & 3) * LPW + i, lane, valid - 1, D);
+    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, NKS>(wave % kFillWaves * LPW + i, lane, valid - 1, D);
     float16_t acc[MR][2];
 #pragma unroll
     for (int mr = 0; mr < MR; mr++)
@@ -103,18 +130,17 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
             for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
     uint32_t* words = reinterpret_cast<uint32_t*>(reinterpret_cast<half_t*>(lds) + 2 * 3 * T::STAGE) +
                       wave * RowsWords<K>::STAGE;
-    rows_main<K, CB, MR, 2, LPW>(w, row_words, 4 * row_words,
-                                 reinterpret_cast<const char*>((proj ? xu : xg) + (size_t)m0 * D), a_off, true,
-                                 lds_byte_address(stages) + (wave & 3) * LPW * 1024, stages,
-                                 rows_read_base<MR, 2>(ks, lane), words, 8 * RowsWords<K>::STAGE, D >> 6, lane, acc);
+    rows_main<K, CB, MR, NKS, LPW>(w, row_words, 2 * NKS * row_words,
+                                   reinterpret_cast<const char*>((proj ? xu : xg) + (size_t)m0 * D), a_off, true,
+                                   lds_byte_address(stages) + wave % kFillWaves * LPW * 1024, stages,
+                                   rows_read_base<MR, NKS>(ks, lane), words, 4 * NKS * RowsWords<K>::STAGE,
+                                   D / (32 * NKS), lane, acc);
 
-    float16_t sum[MR];
-    rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
     half_t* tile = reinterpret_cast<half_t*>(lds);  // [gate | up][BM][kLd]
-    rows_store_half<MR>(sum, tile + proj * T::BM * kLd, kLd, cq * 64, ks, lane);
+    rows_to_tile<MR, NKS>(acc, lds, tile + proj * T::BM * kLd, kLd, cq * 64, wave, lane);
     __syncthreads();
 
-    // Output transform, GLU and rotation: a wave takes a 16-row tile and MR of the four
+    // Output transform, GLU and rotation: a wave takes a 16-row tile and kParts of the four
     // 32-column parts of the block.
     const int rt = wave % (2 * MR), part = wave / (2 * MR);
     const int fr = lane & 15, q = lane >> 4;
@@ -132,12 +158,12 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
     };
     // f(a) for the wave's parts a, which are compile-time values in each branch
     auto for_parts = [&](auto f) {
-        static_for<0, 4 / MR>([&](auto p) {
+        static_for<0, 4 / kParts>([&](auto p) {
             if (part == p.value)
-                static_for<0, MR>([&](auto i) { f(std::integral_constant<int, p.value * MR + i.value>{}, i); });
+                static_for<0, kParts>([&](auto i) { f(std::integral_constant<int, p.value * kParts + i.value>{}, i); });
         });
     };
-    half8_t h[MR];
+    half8_t h[kParts];
     {
         half8_t yg[4], yu[4];
 #pragma unroll
@@ -177,11 +203,11 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
     __syncthreads();
     const bool store = rt * 16 + fr < valid;
     half_t* out = xd + (size_t)(m0 + rt * 16 + fr) * H + hg * 128 + q * 8;
-    auto put = [&](auto a, const float (&z)[8]) {
+    auto put = [&](int a, const float (&z)[8]) {
         half8_t o;
 #pragma unroll
         for (int c = 0; c < 8; c++) o[c] = (half_t)(z[c] * kHadNorm);
-        if (store) *reinterpret_cast<half8_t*>(out + a.value * 32) = o;
+        if (store) *reinterpret_cast<half8_t*>(out + a * 32) = o;
     };
     if (all_plain_signs(ds)) {
         half8_t v[4];
@@ -203,11 +229,10 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
             for (int t = 0; t < 8; t++) v[t] = v[t] * scale[t];
             wht32_tile(v);
         };
-        float z[MR][8];
 #pragma unroll
-        for (int i = 0; i < MR; i++) {
-            const int a = part * MR + i;
-            float t[2][8], u[8];
+        for (int i = 0; i < kParts; i++) {
+            const int a = part * kParts + i;
+            float t[2][8], u[8], z[8];
 #pragma unroll
             for (int half = 0; half < 2; half++) {
                 five_stages(2 * half, t[half]);
@@ -216,20 +241,22 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_gateup_rows_kernel(
                 for (int c = 0; c < 8; c++) t[half][c] = a & 1 ? __fsub_rn(t[half][c], u[c]) : __fadd_rn(t[half][c], u[c]);
             }
 #pragma unroll
-            for (int c = 0; c < 8; c++) z[i][c] = a & 2 ? __fsub_rn(t[0][c], t[1][c]) : __fadd_rn(t[0][c], t[1][c]);
+            for (int c = 0; c < 8; c++) z[c] = a & 2 ? __fsub_rn(t[0][c], t[1][c]) : __fadd_rn(t[0][c], t[1][c]);
+            put(a, z);
         }
-        for_parts([&](auto a, auto i) { put(a, z[i.value]); });
     }
 }
 
 // unit = (row block b, 256-column block g of D), XCD order as above; rows go to out[order[r]].
-template <int K, int CB, int MR>
-__global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
+template <int K, int CB, int MR, int NKS>
+__global__ __launch_bounds__(256 * NKS, 4) void moe_down_rows_kernel(
     const uint32_t* __restrict__ trellis, const half_t* __restrict__ xd, const int4* __restrict__ table, int n_blocks,
     const half_t* __restrict__ dn_svh, const int* __restrict__ order, half_t* __restrict__ out, int n_rows, int E,
     int D, int H) {
-    using T = RowsTile<MR, 2>;
-    constexpr int LPW = (T::FILLS + 7) / 8;
+    using T = RowsTile<MR, NKS>;
+    constexpr int LPW = 1;
+    constexpr int kParts = 4 * MR / NKS;  // of a wave, of the eight 32-column parts of a row tile
+    static_assert(T::FILLS <= 4 * NKS, "a fill a wave");
     constexpr int kLd = 256 + kYPad;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
@@ -245,14 +272,14 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
     // a last block of 128 columns: its upper half repeats the lower half's and is not stored
     const bool full = g * 256 + 128 < D;
 
-    const int cq = wave >> 1, ks = wave & 1;
+    const int cq = wave / NKS, ks = wave % NKS;
     const size_t row_words = (size_t)E * (D >> 4) * (8 * K);
     const uint32_t* w = trellis + (size_t)(2 * ks) * row_words +
                         ((size_t)e * (D >> 4) + g * 16 + (full ? cq : cq & 1) * 4) * (8 * K);
     half_t* stages = reinterpret_cast<half_t*>(lds);
     uint32_t a_off[LPW];
 #pragma unroll
-    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, 2>(wave * LPW + i, lane, valid - 1, H);
+    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, NKS>(wave * LPW + i, lane, valid - 1, H);
     float16_t acc[MR][2];
 #pragma unroll
     for (int mr = 0; mr < MR; mr++)
@@ -261,25 +288,24 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
     uint32_t* words = reinterpret_cast<uint32_t*>(stages + 3 * T::STAGE) + wave * RowsWords<K>::STAGE;
-    rows_main<K, CB, MR, 2, LPW>(w, row_words, 4 * row_words, reinterpret_cast<const char*>(xd + (size_t)m0 * H),
-                                 a_off, wave * LPW < T::FILLS, lds_byte_address(stages) + wave * LPW * 1024, stages,
-                                 rows_read_base<MR, 2>(ks, lane), words, 8 * RowsWords<K>::STAGE, H >> 6, lane, acc);
-    float16_t sum[MR];
-    rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
+    rows_main<K, CB, MR, NKS, LPW>(w, row_words, 2 * NKS * row_words, reinterpret_cast<const char*>(xd + (size_t)m0 * H),
+                                   a_off, wave < T::FILLS, lds_byte_address(stages) + wave * LPW * 1024, stages,
+                                   rows_read_base<MR, NKS>(ks, lane), words, 4 * NKS * RowsWords<K>::STAGE,
+                                   H / (32 * NKS), lane, acc);
     half_t* tile = reinterpret_cast<half_t*>(lds);  // [BM][kLd]
-    rows_store_half<MR>(sum, tile, kLd, cq * 64, ks, lane);
+    rows_to_tile<MR, NKS>(acc, lds, tile, kLd, cq * 64, wave, lane);
     __syncthreads();
 
-    // output transform: a wave takes a 16-row tile and 2 MR of the eight 32-column parts
+    // output transform: a wave takes a 16-row tile and kParts of the eight 32-column parts
     const int rt = wave % (2 * MR), part = wave / (2 * MR);
     const int fr = lane & 15, q = lane >> 4;
     const HadamardColumns had(lane);
     const int r = rt * 16 + fr;
     const size_t dst_row = r < valid ? (size_t)order[m0 + r] : 0;
-    static_for<0, 4 / MR>([&](auto p) {
+    static_for<0, 8 / kParts>([&](auto p) {
         if (part != p.value) return;
-        static_for<0, 2 * MR>([&](auto i) {
-            constexpr int c = p.value * 2 * MR + i.value, half = c >> 2, a = c & 3;
+        static_for<0, kParts>([&](auto i) {
+            constexpr int c = p.value * kParts + i.value, half = c >> 2, a = c & 3;
             if (half && !full) return;
             const half_t* yrow = tile + (rt * 16 + fr) * kLd + half * 128 + q * 8;
             float4_t t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -298,13 +324,26 @@ __global__ __launch_bounds__(kRowsThreads, 4) void moe_down_rows_kernel(
     });
 }
 
-template <int K, int MR>
+template <int K, int MR, int NKS>
 static constexpr size_t rows_lds_bytes(int tiles, int tile_cols) {
-    const size_t stages = (size_t)3 * (tiles * RowsTile<MR, 2>::STAGE * 2 + 8 * RowsWords<K>::STAGE * 4);
-    const size_t exchange = (size_t)8 * MR * 4 * 64 * 16;
-    const size_t y = (size_t)tiles * RowsTile<MR, 2>::BM * (tile_cols + kYPad) * 2;
+    const size_t stages = (size_t)3 * (tiles * RowsTile<MR, NKS>::STAGE * 2 + 4 * NKS * RowsWords<K>::STAGE * 4);
+    const size_t exchange = NKS == 2 ? (size_t)8 * MR * 4 * 64 * 16 : 0;
+    const size_t y = (size_t)tiles * RowsTile<MR, NKS>::BM * (tile_cols + kYPad) * 2;
     return stages > exchange ? (stages > y ? stages : y) : (exchange > y ? exchange : y);
 }
+
+// Workgroups of four waves (NKS = 1) instead of eight: no exchange between k-slices, twice the steps
+// for a prologue and an epilogue, and four to a CU that are at different points of their work; but
+// half the waves where there are too few units to fill the chip. Over 48 shapes (33 to 1537 tokens,
+// 32 to 257 experts, D 1024..2048, H 256..768, K 2..8), whole prefill call:
+// down, from 800 units on (by the table's length, which is 1.1 to 1.8 times the units with rows): 1 to 10 us
+//   less of 45 to 320, none slower (2048 x 512, 257 experts, 9 a token: 1537 tokens K = 4 293.6 ->
+//   276.1); below 1.1 us less to 2.1 us more;
+// gate/up, where LDS holds one workgroup of eight waves on a CU (64 rows, K >= 6), from 400 units on:
+//   1000 tokens K = 6 312.1 -> 275.6, 820 tokens through 64 experts K = 7 137.7 -> 132.5, none slower;
+//   264 units 80.6 -> 84.9. Where it holds two, 8 us more to 7 us less.
+constexpr long long kDownNarrowUnits = 800, kGateUpNarrowUnits = 400;
+constexpr size_t kLdsBytes = (size_t)160 << 10;
 
 // block_rows: 32 or 64
 int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const uint16_t* gu_trellis,
@@ -317,26 +356,32 @@ int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const ui
     if (gu_grid > 0x7FFFFFFFLL || dn_grid > 0x7FFFFFFFLL) return EXL3_E_BAD_SHAPE;
     auto H_ = [](const uint16_t* p) { return reinterpret_cast<const half_t*>(p); };
     return dispatch_k_cb(K, cb, [&](auto k, auto c) {
-        auto go = [&](auto mrc) {
-            constexpr int MR = mrc.value;
-            constexpr size_t gu_lds = rows_lds_bytes<k.value, MR>(2, 128), dn_lds = rows_lds_bytes<k.value, MR>(1, 256);
-            auto gu = moe_gateup_rows_kernel<k.value, c.value, MR>;
-            auto dn = moe_down_rows_kernel<k.value, c.value, MR>;
+        auto go = [&](auto mrc, auto gnc, auto dnc) {
+            constexpr int MR = mrc.value, GN = gnc.value, DN = dnc.value;
+            constexpr size_t gu_lds = rows_lds_bytes<k.value, MR, GN>(2, 128), dn_lds = rows_lds_bytes<k.value, MR, DN>(1, 256);
+            auto gu = moe_gateup_rows_kernel<k.value, c.value, MR, GN>;
+            auto dn = moe_down_rows_kernel<k.value, c.value, MR, DN>;
             if (hipFuncSetAttribute(reinterpret_cast<const void*>(gu), hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)gu_lds) != hipSuccess ||
                 hipFuncSetAttribute(reinterpret_cast<const void*>(dn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)dn_lds) != hipSuccess)
                 return (int)EXL3_E_LAUNCH;
-            gu<<<dim3((unsigned)gu_grid), dim3(kRowsThreads), gu_lds, stream>>>(
+            gu<<<dim3((unsigned)gu_grid), dim3(256 * GN), gu_lds, stream>>>(
                 reinterpret_cast<const uint32_t*>(gu_trellis), H_(xg), H_(xu), reinterpret_cast<const int4*>(table),
                 n_blocks, H_(gu_svh), H_(dn_suh), reinterpret_cast<half_t*>(xd), n_rows, E, D, H, activation);
             if (int rc = launch_status()) return rc;
-            dn<<<dim3((unsigned)dn_grid), dim3(kRowsThreads), dn_lds, stream>>>(
+            dn<<<dim3((unsigned)dn_grid), dim3(256 * DN), dn_lds, stream>>>(
                 reinterpret_cast<const uint32_t*>(dn_trellis), H_(xd), reinterpret_cast<const int4*>(table), n_blocks,
                 H_(dn_svh), order, reinterpret_cast<half_t*>(out), n_rows, E, D, H);
             return launch_status();
         };
-        return block_rows == 32 ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 2>{});
+        using N1 = std::integral_constant<int, 1>;
+        using N2 = std::integral_constant<int, 2>;
+        const bool many_dn = dn_grid >= kDownNarrowUnits;
+        if (block_rows == 32) return many_dn ? go(N1{}, N2{}, N1{}) : go(N1{}, N2{}, N2{});
+        if constexpr (2 * rows_lds_bytes<k.value, 2, 2>(2, 128) > kLdsBytes)
+            if (gu_grid >= kGateUpNarrowUnits) return many_dn ? go(N2{}, N1{}, N1{}) : go(N2{}, N1{}, N2{});
+        return many_dn ? go(N2{}, N2{}, N1{}) : go(N2{}, N2{}, N2{});
     });
 }
 

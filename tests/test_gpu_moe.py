@@ -221,6 +221,40 @@ def test_prefill_path_matches_oracle_and_slot_kernels(cuda, oracle, tokens, act)
     assert rel_l2(y.cpu().numpy(), slots.cpu().numpy()) <= TOL
 
 
+@pytest.mark.parametrize("tokens,E,kk,D,H,K,cb,act,general", [
+    (40, 300, 3, 640, 128, 3, 2, 0, False),    # down in four waves, 32 rows; a last block of 128 columns
+    (590, 170, 8, 1152, 256, 6, 0, 1, True),   # both, 64 rows, blocks of one row and of 64; scales other than +-1
+    (300, 32, 8, 1024, 768, 8, 1, 0, False),   # gate/up in four waves, down in eight
+])
+def test_prefill_workgroups_of_four_waves(cuda, tokens, E, kk, D, H, K, cb, act, general):
+    """The prefill kernels at as many row blocks as they take in workgroups of four waves, against the slot
+    kernels on the same input (bar of the other prefill test)."""
+    from ponyexl3_amd import _lib, ops
+
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(tokens)
+    bits = lambda *s: torch.randint(-32768, 32768, s, generator=g, dtype=torch.int16).to(cuda)
+    def scale(size, *s):
+        v = torch.randint(0, 2, s, generator=g) * 2.0 - 1.0
+        return (v * size * (0.5 + torch.rand(s, generator=g) if general else 1)).half().to(cuda)
+    gu, dn = bits(D // 16, 2 * E * H // 16, 16 * K), bits(H // 16, E * D // 16, 16 * K)
+    gsu, gsv, dsu, dsv = scale(1, E, 2, D), scale(D**-0.5, E, 2, H), scale(1, E, H), scale(H**-0.5, E, D)
+    x = (torch.randn((tokens, D), generator=g) * 0.5).half().to(cuda)
+    # a few experts get most of the pairs, some one, some none
+    weight = torch.rand((tokens, E), generator=g) * torch.linspace(0.3, 1, E)
+    idx = weight.topk(kk, dim=1).indices.int().contiguous().to(cuda)
+    y = torch.full((tokens, kk, D), float("nan"), dtype=torch.float16, device=cuda)
+    need = lib.exl3_moe_prefill_workspace_bytes(tokens, kk, E, D, H)
+    ws = torch.empty((need,), dtype=torch.uint8, device=cuda)
+    p = ops._ptr
+    print(f"prefill four waves tokens={tokens} E={E} D={D} H={H} K={K}", flush=True)
+    _lib.check(lib.exl3_moe_prefill(p(x), tokens, p(idx), kk, p(gu), p(gsu), p(gsv), p(dn), p(dsu), p(dsv), E, D, H, K,
+                                    cb, act, None, p(y), p(ws), need, ops._stream()), "exl3_moe_prefill")
+    slots = torch.cat([ops.moe_forward(x[r:r + 8], idx[r:r + 8], gu, gsu, gsv, dn, dsu, dsv, K, cb, act)
+                       for r in range(0, tokens, 8)])
+    assert rel_l2(y.float().cpu().numpy(), slots.float().cpu().numpy()) <= TOL
+
+
 def test_moe_equals_linear_modules(cuda):
     """The stacked chain equals the same experts run as individual EXL3Linear
     modules (fused-vs-unfused, ponyexl3/tests/test_moe_activation.py:44-65)."""
