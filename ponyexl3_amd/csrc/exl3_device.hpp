@@ -260,10 +260,16 @@ __device__ __forceinline__ float butterfly_dpp(float v, uint32_t sign) {
 // stage is an add and a subtract inside the lane. swap_back restores the layout (both
 // swaps are involutions; undo them in reverse order).
 __device__ __forceinline__ void swap_rows16(float& a, float& b) {
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    const uint32_t x = r[0], y = r[1];  // (a bit_cast of an element takes element 0)
+    a = __builtin_bit_cast(float, x);
+    b = __builtin_bit_cast(float, y);
 }
 __device__ __forceinline__ void swap_halves32(float& a, float& b) {
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    const uint32_t x = r[0], y = r[1];  // (a bit_cast of an element takes element 0)
+    a = __builtin_bit_cast(float, x);
+    b = __builtin_bit_cast(float, y);
 }
 __device__ __forceinline__ void butterfly_in_lane(float& a, float& b) {
     const float s = __fadd_rn(a, b), d = __fsub_rn(a, b);
