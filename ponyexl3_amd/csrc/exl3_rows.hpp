@@ -208,6 +208,34 @@ __device__ __forceinline__ int rows_read_base(int ks, int lane) {
     return row * T::BK + (chunk ^ T::swizzle(row)) * 8;
 }
 
+// Sums of two k-slices: the wave of slice ks keeps columns cs = ks. `ex` holds MR*4 float4 per
+// lane and wave; every wave passes its other half to its partner (wave ^ 1).
+template <int MR>
+__device__ __forceinline__ void rows_add_slices2(float16_t (&acc)[MR][2], float4_t* ex, int wave, int lane,
+                                                 float16_t (&sum)[MR]) {
+    const bool second = wave & 1;
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float4_t v;
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = second ? acc[mr][0][4 * i + c] : acc[mr][1][4 * i + c];
+            ex[((wave ^ 1) * MR * 4 + mr * 4 + i) * 64 + lane] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4_t v = ex[(wave * MR * 4 + mr * 4 + i) * 64 + lane];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                sum[mr][4 * i + c] = __fadd_rn(second ? acc[mr][1][4 * i + c] : acc[mr][0][4 * i + c], v[c]);
+        }
+    __syncthreads();
+}
+
 // Hadamard-128 on the matrix pipe with outputs eight columns to a lane. Column tile nt of
 // block half a = nt >> 1 is laid out so that matrix row m stands for column 32 a + 8 (m >> 2)
 // + 4 (nt & 1) + (m & 3): after a pair of tiles a lane (q = lane >> 4, activation row lane &

@@ -4,8 +4,8 @@
 // instructions (see exl3_rows.hpp for the contraction).
 //
 // Workgroup = one 128-column group (one block of the output Hadamard) x one row block of 32 MR
-// rows x one range of the reduction; its eight waves are two 64-column strips x four k-slices
-// of a 128-deep step. A whole reduction ends with the output transform
+// rows x one range of the reduction; its waves are two 64-column strips x NKS (four or two) k-slices
+// of a 32 NKS deep step. A whole reduction ends with the output transform
 // (ponyexl3/ref/forward.py:41-45) on the matrix pipe; ranges write fp32 partial rows that
 // the output transform kernel adds in range order.
 //
@@ -24,7 +24,6 @@
 
 namespace exl3 {
 
-constexpr int kLinRowsThreads = 512;
 constexpr int kLinRowsLd = 128 + 8;  // halfs: 16-byte reads of 16 tile rows hit all banks
 
 struct LinRowsArgs {
@@ -91,10 +90,10 @@ __device__ __forceinline__ void rows_add_slices4(float16_t (&acc)[MR][2], float4
 
 // Workgroups are dealt to the eight XCDs by index: the row blocks of one (column group, range)
 // unit u land on one XCD, whose L2 then reads their trellis words once.
-template <int K, int CB, int MR>
-__global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_kernel(LinRowsArgs p) {
-    using T = RowsTile<MR, 4>;
-    constexpr int LPW = T::FILLS / 8;
+template <int K, int CB, int MR, int NKS>
+__global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 2) void linear_rows_kernel(LinRowsArgs p) {
+    using T = RowsTile<MR, NKS>;
+    constexpr int LPW = T::FILLS / (2 * NKS);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -107,7 +106,7 @@ __global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_
     const int m0 = rb * p.block_rows;
     const int valid = min(p.block_rows, p.rows - m0);
 
-    const int cq = wave >> 2, ks = wave & 3;
+    const int cq = wave / NKS, ks = wave % NKS;
     const size_t row_words = (size_t)p.out_tiles * (8 * K);
     const uint32_t* w = p.trellis + ((size_t)k0 * 8 + 2 * ks) * row_words + (size_t)(g * 8 + cq * 4) * (8 * K);
     const half_t* x = p.xh + (size_t)m0 * p.ldx + (size_t)k0 * 128;
@@ -115,7 +114,7 @@ __global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_
     half_t* stages = reinterpret_cast<half_t*>(lds);
     uint32_t a_off[LPW];
 #pragma unroll
-    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, 4>(wave * LPW + i, lane, valid - 1, p.ldx);
+    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, NKS>(wave * LPW + i, lane, valid - 1, p.ldx);
     float16_t acc[MR][2];
 #pragma unroll
     for (int mr = 0; mr < MR; mr++)
@@ -124,14 +123,16 @@ __global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
     uint32_t* words = reinterpret_cast<uint32_t*>(stages + 3 * T::STAGE) + wave * RowsWords<K>::STAGE;
-    rows_main<K, CB, MR, 4, LPW>(w, row_words, 8 * row_words, reinterpret_cast<const char*>(x), a_off, true,
-                                 lds_byte_address(stages) + wave * LPW * 1024, stages, rows_read_base<MR, 4>(ks, lane),
-                                 words, 8 * RowsWords<K>::STAGE, nsteps, lane, acc);
-    float sum[MR][8];
-    rows_add_slices4<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
-
-    // lane: row lane & 31 of each 32-row block, columns col + 16 i + 0..3
-    const int col = cq * 64 + 32 * (ks & 1) + 8 * (ks >> 1) + 4 * (lane >> 5);
+    rows_main<K, CB, MR, NKS, LPW>(w, row_words, 2 * NKS * row_words, reinterpret_cast<const char*>(x), a_off, true,
+                                   lds_byte_address(stages) + wave * LPW * 1024, stages,
+                                   rows_read_base<MR, NKS>(ks, lane), words, 2 * NKS * RowsWords<K>::STAGE,
+                                   nsteps * (4 / NKS), lane, acc);
+    // lane: row lane & 31 of each 32-row block, columns col + 16 i + 0..3, i < NI
+    constexpr int NI = 8 / NKS;
+    std::conditional_t<NKS == 4, float[MR][8], float16_t[MR]> sum;
+    if constexpr (NKS == 4) rows_add_slices4<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
+    else rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
+    const int col = cq * 64 + (NKS == 4 ? 32 * (ks & 1) + 8 * (ks >> 1) : 8 * ks) + 4 * (lane >> 5);
     const size_t n = (size_t)p.out_tiles * 16;
     if (p.n_splits > 1) {
         float* dst = p.partial + ((size_t)split * p.rows + m0) * n + (size_t)g * 128 + col;
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_
             const int r = mr * 32 + (lane & 31);
             if (r < valid) {
 #pragma unroll
-                for (int i = 0; i < 2; i++) {
+                for (int i = 0; i < NI; i++) {
                     float4_t v;
 #pragma unroll
                     for (int c = 0; c < 4; c++) v[c] = sum[mr][4 * i + c];
@@ -154,19 +155,19 @@ __global__ __launch_bounds__(kLinRowsThreads, MR <= 2 ? 4 : 2) void linear_rows_
 #pragma unroll
     for (int mr = 0; mr < MR; mr++)
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < NI; i++) {
             half4_t o;
 #pragma unroll
             for (int c = 0; c < 4; c++) o[c] = (half_t)sum[mr][4 * i + c];
             *reinterpret_cast<half4_t*>(tile + (mr * 32 + (lane & 31)) * kLinRowsLd + col + 16 * i) = o;
         }
     __syncthreads();
-    // output transform: 2 MR 16-row tiles x four 32-column parts, MR of them to a wave
+    // output transform: 2 MR 16-row tiles x four 32-column parts
     const int fr = lane & 15, q = lane >> 4;
     const HadamardColumns had(lane);
 #pragma unroll
-    for (int j = 0; j < MR; j++) {
-        const int id = wave + 8 * j, rt = id >> 2, a = id & 3;
+    for (int j = 0; j < 4 * MR / NKS; j++) {
+        const int id = wave + 2 * NKS * j, rt = id >> 2, a = id & 3;
         const half_t* yrow = tile + (rt * 16 + fr) * kLinRowsLd + q * 8;
         float4_t t[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
         static_for<0, 4>([&](auto k) {
@@ -233,6 +234,39 @@ LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups) {
     return p;
 }
 
+// Workgroups of four waves (two k-slices) instead of eight, where there are more of eight than the
+// chip holds at once: with half the registers and LDS to a workgroup a CU holds four of them up to 64
+// rows (three from K = 6 on), three (two from K = 6 on) up to 96, two above, where it held one of
+// eight waves from 65 rows on or at K = 6, two else: 12 waves where there were 8, and the last round is
+// of smaller pieces. 70 layers of 46 to 994 rows beyond that line, without the rotation: 18 % less at
+// 77 rows of 5120 -> 34816 (80.8 -> 66.1 us), 21 % at 64 rows with K = 6 (77.5 -> 60.9), 15 % at 700
+// rows of 2048 -> 6144 (50.9 -> 43.1), 11 % at the median, more (0.3 to 3 %) in three; below it
+// mostly slower (256 rows of 5120 -> 10240 46.7 and 58.1). Up to 32 rows a CU holds three of eight
+// waves, and the line is beyond the layers measured.
+static int rows_per_cu(int mr, int nks, int K) {
+    const int lds = 3 * (mr * 32 * nks * 32 * 2 + 2 * nks * 64 * K * 4), fit = (160 << 10) / lds;
+    const int waves = mr <= 2 ? 16 : nks == 2 && mr == 3 ? 12 : 8;  // of a CU, by registers
+    return std::min(fit, waves / (2 * nks));
+}
+static long long rows_workgroups(const LinRowsPlan& p, int n_groups) {
+    return (long long)p.n_row_blocks * n_groups * p.n_splits;
+}
+static bool rows_narrow(const LinRowsPlan& p, int n_groups, int K) {
+    return p.mr >= 2 && rows_workgroups(p, n_groups) > 256 * rows_per_cu(p.mr, 4, K);
+}
+
+// Time of a plan of more than 64 rows in workgroups of four waves, fitted to the same layers (4 %
+// root mean square): rounds of as many as the chip holds, a last one that costs between its share
+// and that of its fullest CU.
+static double rows_narrow_estimate_us(const LinRowsPlan& p, int n_groups, int K) {
+    static const double step[2] = {0.695, 0.817};
+    const int m = p.mr - 3, per_cu = rows_per_cu(p.mr, 2, K);
+    const long long n = rows_workgroups(p, n_groups), full = n / (256 * per_cu), rest = n % (256 * per_cu);
+    double load = full * (per_cu + 0.54);
+    if (rest) load += 0.66 * (double)((rest + 255) / 256) + 0.34 * (double)rest / 256 + 0.54;
+    return step[m] * (p.steps_per_split + 5) * load * (K > 4 ? 1 + 0.013 * (K - 4) : 1.0) + 4;
+}
+
 // Estimate of a plan's time for the choice between this kernel and the prefill GEMM, without the
 // input rotation. Alone on its CU, two to a CU, and in several rounds a workgroup's 128-deep step
 // takes: {65..96, 97..128 rows} 0.915 and 1.08 us alone, 0.93 and 1.19 in rounds; up to 64 rows
@@ -242,21 +276,27 @@ LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups) {
 static double rows_estimate_us(const LinRowsPlan& p, int rows, int n_groups, int K, int cb) {
     static const double alone[3] = {0.765, 0.915, 1.08}, rounds[3] = {0.85, 0.93, 1.19}, mul1[3] = {1.28, 1.21, 1.12};
     const int m = p.mr <= 2 ? 0 : p.mr - 2;
-    const long long n = (long long)p.n_row_blocks * n_groups * p.n_splits;
+    const long long n = rows_workgroups(p, n_groups);
+    const double split_us =
+        p.n_splits > 1 ? kRowsPostUs + (double)p.n_splits * rows * n_groups * 128 * 8 / kRowsPartialRate : 0;
+    if (p.mr >= 3 && cb != CB_MUL1 && rows_narrow(p, n_groups, K)) return rows_narrow_estimate_us(p, n_groups, K) + split_us;
     const size_t lds = 3 * ((size_t)p.mr * 32 * 128 * 2 + (size_t)8 * 64 * K * 4);
     double us;
     if (n <= 256) us = alone[m];
     else if (p.mr <= 2 && 2 * lds <= (size_t)160 << 10) us = 1.40 * (n <= 512 ? 1.0 : (double)n / 512 + 0.15);
     else us = rounds[m] * (double)((n + 255) / 256);
     us *= (p.steps_per_split + kRowsFillSteps) * (K > 4 ? 1 + 0.014 * (K - 4) : 1.0) * (cb == CB_MUL1 ? mul1[m] : 1.0);
-    return us + (p.n_splits > 1 ? kRowsPostUs + (double)p.n_splits * rows * n_groups * 128 * 8 / kRowsPartialRate : 0);
+    return us + split_us;
 }
 
 // Whether the layer takes this kernel rather than the prefill GEMM, which has larger tiles (256
 // columns and up to 256 rows). Both estimates were fitted to the choice over 2816 layers of 40 to
 // 1024 rows (in 1024..17408, out 1024..65536, K = 2..8, all codebooks): the layer is slower than
 // through the GEMM by more than 3 % in seven of them, 8 % at most, and 0.5 % slower than the
-// better of the two on average. Measured (layer, GEMM and this kernel, us): 5120 -> 10240 at 77
+// better of the two on average. (Since then workgroups of four waves have moved the line from 65 rows
+// on, see rows_narrow_estimate_us: of the 70 layers the choice costs 0.1 % on average, 4 % at most, where
+// the estimate of eight waves cost 3.8 %; up to 64 rows the line is where it was, and with MUL1, where the
+// GEMM keeps up: 200 rows of 4096 -> 24576 84.3 us, four waves 88.9.) Measured (layer, GEMM and this kernel, us): 5120 -> 10240 at 77
 // rows 41.1 and 28.8; 17408 -> 5120 (K = 5) at 333 rows 115 and 97; 5120 -> 34816 at 64 rows 63.7
 // and 59.3 at K = 4, but 69.0 and 73.0 at K = 6; 4096 -> 24576 at 256 rows 83.6 and 95.1 with MUL1.
 bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
@@ -303,24 +343,27 @@ int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stri
                         plan.block_rows, plan.n_row_blocks, (int)units, plan.n_splits, plan.steps_per_split,
                         in_tiles / 8, out_tiles};
     const int rc = dispatch_k_cb(K, cb, [&](auto k, auto c) {
-        auto go = [&](auto mrc) {
-            constexpr int MR = mrc.value;
-            constexpr size_t stages = (size_t)3 * (RowsTile<MR, 4>::STAGE * 2 + 8 * RowsWords<k.value>::STAGE * 4),
-                             exchange = (size_t)8 * MR * 4 * 64 * 16;
+        auto go = [&](auto mrc, auto nks) {
+            constexpr int MR = mrc.value, NKS = nks.value;
+            constexpr size_t stages = (size_t)3 * (RowsTile<MR, NKS>::STAGE * 2 + 2 * NKS * RowsWords<k.value>::STAGE * 4),
+                             exchange = (size_t)2 * NKS * MR * 4 * 64 * 16;
             constexpr size_t bytes = stages > exchange ? stages : exchange;
             static_assert(bytes >= (size_t)32 * MR * kLinRowsLd * 2, "the fp16 tile fits");
-            auto kernel = linear_rows_kernel<k.value, c.value, MR>;
+            auto kernel = linear_rows_kernel<k.value, c.value, MR, NKS>;
             if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess)
                 return (int)EXL3_E_LAUNCH;
-            kernel<<<dim3((unsigned)grid), dim3(kLinRowsThreads), bytes, stream>>>(a);
+            kernel<<<dim3((unsigned)grid), dim3(128 * NKS), bytes, stream>>>(a);
             return launch_status();
         };
+        using N2 = std::integral_constant<int, 2>;
+        using N4 = std::integral_constant<int, 4>;
+        const bool narrow = rows_narrow(plan, n_groups, k.value);
         switch (plan.mr) {
-            case 1: return go(std::integral_constant<int, 1>{});
-            case 2: return go(std::integral_constant<int, 2>{});
-            case 3: return go(std::integral_constant<int, 3>{});
-            default: return go(std::integral_constant<int, 4>{});
+            case 1: return go(std::integral_constant<int, 1>{}, N4{});
+            case 2: return narrow ? go(N2{}, N2{}) : go(N2{}, N4{});
+            case 3: return narrow ? go(std::integral_constant<int, 3>{}, N2{}) : go(std::integral_constant<int, 3>{}, N4{});
+            default: return narrow ? go(N4{}, N2{}) : go(N4{}, N4{});
         }
     });
     if (rc != EXL3_OK || plan.n_splits == 1) return rc;

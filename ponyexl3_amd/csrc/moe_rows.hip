@@ -23,34 +23,6 @@ namespace exl3 {
 
 constexpr int kYPad = 8;  // halfs: 16-byte reads of 16 tile rows hit all banks
 
-// Sums of two k-slices: the wave of slice ks keeps columns cs = ks. `ex` holds MR*4 float4 per
-// lane and wave; every wave passes its other half to its partner (wave ^ 1).
-template <int MR>
-__device__ __forceinline__ void rows_add_slices2(float16_t (&acc)[MR][2], float4_t* ex, int wave, int lane,
-                                                 float16_t (&sum)[MR]) {
-    const bool second = wave & 1;
-#pragma unroll
-    for (int mr = 0; mr < MR; mr++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            float4_t v;
-#pragma unroll
-            for (int c = 0; c < 4; c++) v[c] = second ? acc[mr][0][4 * i + c] : acc[mr][1][4 * i + c];
-            ex[((wave ^ 1) * MR * 4 + mr * 4 + i) * 64 + lane] = v;
-        }
-    __syncthreads();
-#pragma unroll
-    for (int mr = 0; mr < MR; mr++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float4_t v = ex[(wave * MR * 4 + mr * 4 + i) * 64 + lane];
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-                sum[mr][4 * i + c] = __fadd_rn(second ? acc[mr][1][4 * i + c] : acc[mr][0][4 * i + c], v[c]);
-        }
-    __syncthreads();
-}
-
 // The fp16 casts of the sums to an LDS tile [BM][ld], first column `col` of the wave's strip.
 template <int MR>
 __device__ __forceinline__ void rows_store_half(const float16_t (&sum)[MR], half_t* tile, int ld, int col, int cs,

@@ -630,6 +630,18 @@ def test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
         assert lib.exl3_linear_rows(*args, need - 1, ops._stream()) == _lib.EXL3_E_WORKSPACE
 
 
+@pytest.mark.parametrize("rows,k,cb,n_in,outs", [
+    (49, 4, 0, 256, (65792,)),           # 64 rows, more workgroups than two to a CU
+    (64, 6, 1, 256, (16384, 16640)),     # and than one (K >= 6)
+    (71, 8, 0, 384, (16512, 16512)),     # 96 rows
+    (96, 2, 2, 640, (33024,)),
+    (997, 3, 1, 640, (4352,)),           # 128 rows, eight row blocks
+])
+def test_rows_kernel_in_workgroups_of_four_waves(cuda, oracle, rows, k, cb, n_in, outs):
+    """The same where there are more workgroups of eight waves than the chip holds at once."""
+    test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs)
+
+
 @pytest.mark.parametrize("rows,k,n_in,n_out", [(9, 5, 512, 256), (17, 4, 640, 384), (32, 6, 1024, 128),
                                               (40, 4, 2048, 2048)])
 def test_layer_output_off_the_eight_byte_grid(cuda, oracle, rows, k, n_in, n_out):
