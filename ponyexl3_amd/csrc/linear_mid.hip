@@ -1,6 +1,6 @@
 // Medium-batch layer kernel (rows 9..32): the regime where every weight should
 // still be decoded exactly once per launch (the decode sets the pace) but the dot
-// products no longer fit the 4x4x4 matrix instruction of the small-batch kernel.
+// products, which in the small-batch kernel grow with every four batch rows, take whole 16-row operands.
 //
 // The trellis format was laid out for a 16x8x16 tensor-core fragment
 // (ponyexl3/ref/perm.py:8-25): "thread" t = 0..31 of a tile owns the eight

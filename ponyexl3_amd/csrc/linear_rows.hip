@@ -255,16 +255,16 @@ static bool rows_narrow(const LinRowsPlan& p, int n_groups, int K) {
     return p.mr >= 2 && rows_workgroups(p, n_groups) > 256 * rows_per_cu(p.mr, 4, K);
 }
 
-// Time of a plan of more than 64 rows in workgroups of four waves, fitted to the same layers (4 %
-// root mean square): rounds of as many as the chip holds, a last one that costs between its share
+// Time of a plan in workgroups of four waves, fitted to the same layers (4 % root mean square): rounds of as many as the chip holds, a last one that costs between its share
 // and that of its fullest CU.
-static double rows_narrow_estimate_us(const LinRowsPlan& p, int n_groups, int K) {
-    static const double step[2] = {0.695, 0.817};
-    const int m = p.mr - 3, per_cu = rows_per_cu(p.mr, 2, K);
+static double rows_narrow_estimate_us(const LinRowsPlan& p, int n_groups, int K, int cb) {
+    static const double step[3] = {0.615, 0.695, 0.817}, mul1[3] = {1.036, 1.149, 1.075};
+    const int m = p.mr - 2, per_cu = rows_per_cu(p.mr, 2, K);
     const long long n = rows_workgroups(p, n_groups), full = n / (256 * per_cu), rest = n % (256 * per_cu);
     double load = full * (per_cu + 0.54);
     if (rest) load += 0.66 * (double)((rest + 255) / 256) + 0.34 * (double)rest / 256 + 0.54;
-    return step[m] * (p.steps_per_split + 5) * load * (K > 4 ? 1 + 0.013 * (K - 4) : 1.0) + 4;
+    return step[m] * (p.steps_per_split + 5) * load * (K > 4 ? 1 + 0.013 * (K - 4) : 1.0) *
+               (cb == CB_MUL1 ? mul1[m] : 1.0) + 4;
 }
 
 // Estimate of a plan's time for the choice between this kernel and the prefill GEMM, without the
@@ -279,7 +279,7 @@ static double rows_estimate_us(const LinRowsPlan& p, int rows, int n_groups, int
     const long long n = rows_workgroups(p, n_groups);
     const double split_us =
         p.n_splits > 1 ? kRowsPostUs + (double)p.n_splits * rows * n_groups * 128 * 8 / kRowsPartialRate : 0;
-    if (p.mr >= 3 && cb != CB_MUL1 && rows_narrow(p, n_groups, K)) return rows_narrow_estimate_us(p, n_groups, K) + split_us;
+    if (rows_narrow(p, n_groups, K)) return rows_narrow_estimate_us(p, n_groups, K, cb) + split_us;
     const size_t lds = 3 * ((size_t)p.mr * 32 * 128 * 2 + (size_t)8 * 64 * K * 4);
     double us;
     if (n <= 256) us = alone[m];
@@ -293,11 +293,12 @@ static double rows_estimate_us(const LinRowsPlan& p, int rows, int n_groups, int
 // columns and up to 256 rows). Both estimates were fitted to the choice over 2816 layers of 40 to
 // 1024 rows (in 1024..17408, out 1024..65536, K = 2..8, all codebooks): the layer is slower than
 // through the GEMM by more than 3 % in seven of them, 8 % at most, and 0.5 % slower than the
-// better of the two on average. (Since then workgroups of four waves have moved the line from 65 rows
-// on, see rows_narrow_estimate_us: of the 70 layers the choice costs 0.1 % on average, 4 % at most, where
-// the estimate of eight waves cost 3.8 %; up to 64 rows the line is where it was, and with MUL1, where the
-// GEMM keeps up: 200 rows of 4096 -> 24576 84.3 us, four waves 88.9.) Measured (layer, GEMM and this kernel, us): 5120 -> 10240 at 77
-// rows 41.1 and 28.8; 17408 -> 5120 (K = 5) at 333 rows 115 and 97; 5120 -> 34816 at 64 rows 63.7
+// better of the two on average. Workgroups of four waves have lines of their own: over 140 layers that
+// take them (33 to 994 rows), where the line of the eight-wave estimate lost 1 % (96 rows), 3 % (128 rows,
+// and MUL1 from 65 on), 5 % (64 rows, K <= 5) and 14 % (64 rows, K >= 6) to the better of the two, these
+// lose 0.2, 1.9, 0.3, 0.1 and 3 %, and no layer goes to the slower one that did not before. Up to 64
+// rows the GEMM's estimate is 11 % low, and with K <= 5 it was faster in one of 17 layers, by 2 %.
+// Measured (layer, GEMM and this kernel, us): 5120 -> 10240 at 77 rows 41.1 and 28.8; 17408 -> 5120 (K = 5) at 333 rows 115 and 97; 5120 -> 34816 at 64 rows 63.7
 // and 59.3 at K = 4, but 69.0 and 73.0 at K = 6; 4096 -> 24576 at 256 rows 83.6 and 95.1 with MUL1.
 bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
@@ -305,7 +306,10 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     if (rows < 1 || rows > max_rows || in_tiles < 32 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8) return false;
     if (rows <= kLinearMidMaxRows) return true;
     const LinRowsPlan p = plan_linear_rows(rows, in_tiles, out_tiles / 8);
-    return rows_estimate_us(p, rows, out_tiles / 8, K, cb) < 0.95 * gemm_estimate_us(rows, in_tiles, out_tiles, K, cb);
+    const double us = rows_estimate_us(p, rows, out_tiles / 8, K, cb), gemm_us = gemm_estimate_us(rows, in_tiles, out_tiles, K, cb);
+    if (!rows_narrow(p, out_tiles / 8, K)) return us < 0.95 * gemm_us;
+    if (p.mr == 2) return K <= 5 || us < 1.05 * gemm_us;
+    return us < (cb == CB_MUL1 ? 0.92 : p.mr == 3 ? 1.0 : 0.9) * gemm_us;
 }
 
 bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles) {

@@ -547,7 +547,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
 // route to the same expert share one pass over its weights: the grid stays one
 // workgroup set per slot, every workgroup finds the slots of its own expert in the
 // routing table, and only the first of every four of them (in slot order) works, on up
-// to four batch rows (the 4x4x4 matrix instructions carry four rows at the price of
+// to four batch rows (the matrix instructions carry four rows at the price of
 // one). The others leave at once. Per row the arithmetic, the partial rows and the
 // counters are those of the kernels above, so the results are bit-identical.
 
