@@ -121,6 +121,12 @@ __global__ __launch_bounds__(256) void had_pre_wide_kernel(const half_t* __restr
 // expert pair_expert[p], whose scales are scale_ld halfs from the next expert's; entries
 // outside the buffers are clamped.
 // Results: out + s * sub_stride + r * row_stride.
+//
+// What bounds the large ones is the way of the results to memory. From the matrix pipe's layout the
+// sixteen lanes of a quarter wave touch sixteen rows, 16 bytes each, and what the L2 holds at the end is written
+// back then. STREAM turns the tile in LDS, rows and results alike, so that loads and stores cover four
+// rows of 256 bytes in lane order, and stores past the L2. 13 833 pairs of 2048 (113 MB) 38.8 -> 31.6 us (35.8
+// with the stores alone turned, 33.6 without the hint), 333 rows of 17408 7.4 -> 5.8. Same bits. Small results are better read back from the L2: see launch_rotate().
 struct RotateArgs {
     const half_t* x;
     const half_t* suh;
@@ -133,7 +139,18 @@ struct RotateArgs {
     size_t scale_ld;
 };
 
+constexpr int kRotateLd = 128 + 8;  // halfs: rows four LDS banks apart
+
+// The LDS tile belongs to one wave: order for the compiler, the hardware keeps it.
+__device__ __forceinline__ void rotate_tile_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <bool STREAM>
 __global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
+    __shared__ __attribute__((aligned(16))) half_t tiles[STREAM ? 4 : 1][STREAM ? 16 * kRotateLd : 8];
+    half_t* const tile = tiles[STREAM ? threadIdx.x >> 6 : 0];
     const int lane = threadIdx.x & 63;
     const int fr = lane & 15, q = lane >> 4;
     const int blocks = a.n >> 7;
@@ -141,7 +158,7 @@ __global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
     const int row_tiles = (a.rows + 15) >> 4;
     if (wid >= (long long)row_tiles * blocks) return;
     // consecutive waves take consecutive blocks of the same rows
-    const int blk = (int)(wid % blocks), r = (int)(wid / blocks) * 16 + fr;
+    const int blk = (int)(wid % blocks), r0 = (int)(wid / blocks) * 16, r = r0 + fr;
     const bool valid = r < a.rows;
     int src = valid ? r : 0, scale_row = 0;
     if (a.pair) {
@@ -150,10 +167,24 @@ __global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
         src = p / a.top_k;
     }
     const size_t col = (size_t)blk * 128 + q * 8;
-    const half_t* xr = a.x + (size_t)src * a.n + col;
     uint4_t xv[4];
+    if constexpr (STREAM) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) xv[k] = *reinterpret_cast<const uint4_t*>(xr + k * 32);
+        for (int i = 0; i < 4; i++) {
+            const size_t row = (size_t)__shfl(src, 4 * i + q, kWave);
+            xv[i] = *reinterpret_cast<const uint4_t*>(a.x + row * a.n + (size_t)blk * 128 + fr * 8);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) *reinterpret_cast<uint4_t*>(tile + (4 * i + q) * kRotateLd + fr * 8) = xv[i];
+        rotate_tile_order();
+#pragma unroll
+        for (int k = 0; k < 4; k++) xv[k] = *reinterpret_cast<const uint4_t*>(tile + fr * kRotateLd + k * 32 + q * 8);
+        rotate_tile_order();
+    } else {
+        const half_t* xr = a.x + (size_t)src * a.n + col;
+#pragma unroll
+        for (int k = 0; k < 4; k++) xv[k] = *reinterpret_cast<const uint4_t*>(xr + k * 32);
+    }
     const HadamardColumns had(lane);
     const int s_begin = blockIdx.y * a.subs_per_wave, s_end = min(s_begin + a.subs_per_wave, a.n_sub);
     for (int s = s_begin; s < s_end; s++) {
@@ -191,15 +222,26 @@ __global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
 #pragma unroll
                 for (int t = 0; t < 8; t++) z[2 * k + (t >> 2)][t & 3] = v[k][t];
         }
-        if (valid) {
-            half_t* o = a.out + (size_t)s * a.sub_stride + (size_t)r * a.row_stride + col;
+        half_t* const o = a.out + (size_t)s * a.sub_stride;
 #pragma unroll
-            for (int p = 0; p < 4; p++) {
-                half8_t v;
+        for (int p = 0; p < 4; p++) {
+            half8_t v;
 #pragma unroll
-                for (int c = 0; c < 8; c++) v[c] = (half_t)(z[2 * p + (c >> 2)][c & 3] * kHadScale);
-                *reinterpret_cast<half8_t*>(o + p * 32) = v;
+            for (int c = 0; c < 8; c++) v[c] = (half_t)(z[2 * p + (c >> 2)][c & 3] * kHadScale);
+            if constexpr (STREAM) *reinterpret_cast<half8_t*>(tile + fr * kRotateLd + p * 32 + q * 8) = v;
+            else if (valid) *reinterpret_cast<half8_t*>(o + (size_t)r * a.row_stride + col + p * 32) = v;
+        }
+        if constexpr (STREAM) {
+            rotate_tile_order();
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int ro = r0 + 4 * i + q;
+                const uint4_t v = *reinterpret_cast<const uint4_t*>(tile + (4 * i + q) * kRotateLd + fr * 8);
+                if (ro < a.rows)
+                    __builtin_nontemporal_store(
+                        v, reinterpret_cast<uint4_t*>(o + (size_t)ro * a.row_stride + (size_t)blk * 128 + fr * 8));
             }
+            rotate_tile_order();
         }
     }
 }
@@ -210,7 +252,14 @@ static int launch_rotate(RotateArgs a, hipStream_t stream) {
     a.subs_per_wave = waves * a.n_sub <= 4096 ? 1 : a.n_sub;
     const long long grid = (waves + 3) / 4, gy = (a.n_sub + a.subs_per_wave - 1) / a.subs_per_wave;
     if (grid > 0x7FFFFFFFLL || gy > 65535) return EXL3_E_BAD_SHAPE;
-    had_pre_mfma_kernel<<<dim3((unsigned)grid, (unsigned)gy), dim3(256), 0, stream>>>(a);
+    // Past the L2 from 8 MB of results on: whole layers of 77 rows x 3 x 5120 (2.4 MB) and 754 x 2304 (3.5 MB) are 0.5 %
+    // slower that way, 333 x 17408 (11.6 MB) 1 % faster, the experts of 1537 tokens (113 MB) 0.6 to 1.7 %. Not
+    // for more rows than the rows kernels take: the GEMM, which the matrix pipe's clock bounds, gives the time
+    // back (2048 x 5120 -> 34816 0.2 % slower).
+    const bool stream_results = (a.pair || a.rows <= kLinearRowsMaxRows) &&
+                                (size_t)a.rows * a.n * a.n_sub * sizeof(half_t) >= (size_t)8 << 20;
+    auto kernel = stream_results ? had_pre_mfma_kernel<true> : had_pre_mfma_kernel<false>;
+    kernel<<<dim3((unsigned)grid, (unsigned)gy), dim3(256), 0, stream>>>(a);
     return launch_status();
 }
 

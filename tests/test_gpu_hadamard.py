@@ -116,6 +116,31 @@ def test_layer_rotation_with_general_scales(cuda, oracle, rows, n, n_sub, scale,
     assert rel_l2(got[1:, 0].cpu().numpy()[ok], exact[ok]) < 3e-4 or scale < 1e-2  # subnormal results
 
 
+@pytest.mark.parametrize("rows,n,n_sub", [(1023, 4224, 1), (258, 17408, 1), (1015, 1408, 3), (1001, 128, 33)])
+def test_large_rotation_equals_its_parts(cuda, rows, n, n_sub):
+    """From 8 MB of results on, up to 1024 rows, the rotation turns its tiles in LDS and stores past the L2; rows are
+    independent, so the bits are those of calls on a few of them, and nothing behind the results changes."""
+    from ponyexl3_amd import _lib, ops
+
+    rng = np.random.default_rng(rows + n)
+    x = _t(rng.standard_normal((rows, n)).astype(np.float16), cuda)
+    suh = np.where(rng.random((n_sub, n)) > 0.5, -1, 1).astype(np.float16)
+    suh[-1, -128:] *= rng.uniform(0.5, 2, 128).astype(np.float16)  # one block with general scales
+    st, p = _t(suh, cuda), ops._ptr
+    assert rows * n * n_sub * 2 >= 8 << 20 and rows % 16
+
+    def rotate(part):
+        buf = torch.full((part.shape[0] * n_sub * n + 64,), 7.0, dtype=torch.float16, device=cuda)
+        _lib.check(_lib.load().exl3_rotate(p(part), part.shape[0], n, p(st), n_sub, p(buf), ops._stream()), "exl3_rotate")
+        assert bool((buf[-64:] == 7.0).all())
+        return buf[:-64].view(part.shape[0], n_sub, n)
+
+    print(f"large rotation rows={rows} n={n} n_sub={n_sub}", flush=True)
+    got = rotate(x)
+    for r in list(range(0, rows - 75, 500)) + [rows - 75]:  # (64 rows and more: below it another kernel)
+        assert torch.equal(got[r:r + 75].view(torch.int16), rotate(x[r:r + 75]).view(torch.int16))
+
+
 def test_involution_at_scale(cuda):
     """Size-independent property at prefill size: H(H(x)) == x, norms preserved."""
     from ponyexl3_amd import ops

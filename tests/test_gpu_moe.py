@@ -501,6 +501,39 @@ def test_prefill_rotation_with_general_scales(cuda, tokens, k, kind):
     assert rel_l2(got.float().cpu().numpy(), ref.float().cpu().numpy()) <= TOL
 
 
+@pytest.mark.parametrize("tokens,D", [(257, 2048), (251, 2176)])
+def test_large_prefill_equals_its_halves(cuda, tokens, D):
+    """Rotations of 8 MB of pair rows and more take another way to memory; each token's rows are those
+    of a call on half the tokens, up to the order of the sums (the row blocks may differ)."""
+    from ponyexl3_amd import EXL3SwitchGLU, _lib, ops
+
+    E, H, kk, k = 7, 128, 4, 4
+    moe = EXL3SwitchGLU.from_layers(*_experts(E, D, H, k, True, 5200))
+    rng = np.random.default_rng(tokens)
+    scale = moe._gu_suh.clone()
+    scale[E // 2, 1, 128:256] *= 1.5  # a block with general scales
+    x = torch.from_numpy((rng.standard_normal((tokens, D)) * 0.05).astype(np.float16)).to(cuda)
+    idx = torch.from_numpy(np.stack([rng.permutation(E)[:kk] for _ in range(tokens)]).astype(np.int32)).to(cuda)
+    lib, p = _lib.load(), ops._ptr
+    assert tokens * kk * D * 4 >= 8 << 20
+
+    def run(xs, ids):
+        t = xs.shape[0]
+        total = lib.exl3_moe_prefill_workspace_bytes(t, kk, E, D, H)
+        ws = torch.empty((total,), dtype=torch.uint8, device=cuda)
+        y = torch.empty((t, kk, D), dtype=torch.float16, device=cuda)
+        _lib.check(lib.exl3_moe_prefill(p(xs), t, p(ids), kk, p(moe._gu_trellis), p(scale), p(moe._gu_svh),
+                                        p(moe._dn_trellis), p(moe._dn_suh), p(moe._dn_svh), E, D, H, k, moe._cb, 0, None,
+                                        p(y), p(ws), total, ops._stream()), "exl3_moe_prefill")
+        return y
+
+    print(f"large prefill tokens={tokens} D={D}", flush=True)
+    got, half = run(x, idx), tokens // 2
+    ref = torch.cat([run(x[:half].contiguous(), idx[:half].contiguous()), run(x[half:].contiguous(), idx[half:].contiguous())])
+    for a, b in ((got[:half], ref[:half]), (got[half:], ref[half:])):
+        assert rel_l2(a.float().cpu().numpy(), b.float().cpu().numpy()) <= TOL
+
+
 @pytest.mark.parametrize("act", [0, 1])
 def test_glu_rows_kernel_equals_separate_launches(cuda, act):
     """Finish gate/up + GLU + down rotation in one launch against the per-row
