@@ -111,6 +111,7 @@ struct StreamContext {
         if (!t.defined() || static_cast<size_t>(t.numel()) < n) {
             size_t want = std::max(n, t.defined() ? static_cast<size_t>(t.numel()) * 3 / 2 : 0);
             want = std::max<size_t>(want, kind == kCounters ? 4096 : size_t(1) << 20);
+            if (kind == kCounters) want += want & 1;  // whole 64-bit accumulators
             if (t.defined()) retired().push_back(t);
             const auto opt = at::TensorOptions()
                                  .device(at::Device(at::kCUDA, static_cast<c10::DeviceIndex>(device)))
