@@ -232,8 +232,8 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(
     // returning 64-bit atomic adds, and the workgroup whose add completes the group
     // applies the output transform.
     //
-    // Accumulator word of one (batch row, column): count << 56 | sum, the sum a signed
-    // fixed-point number with 24 fraction bits. Integer addition is associative, so the
+    // Accumulator word of one (batch row, column): a count and a fixed-point sum in 64 bits, with
+    // 21 to 33 fraction bits by the number of partial rows (fix_word). Integer addition is associative, so the
     // total does not depend on the order in which workgroups arrive (run-to-run
     // deterministic), and the returned old value tells a lane both how many partial
     // rows are in and what they add up to: the usual chain of store, wait, counter,
@@ -262,6 +262,7 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(
         unsigned long long* sums = reinterpret_cast<unsigned long long*>(counters);
         const size_t out_total = (size_t)n_groups * 128;
         const int wg_splits = (n_splits + NW - 1) / NW;  // partial rows per group
+        const int bits = fix_count_bits(wg_splits);
         const size_t col = (size_t)g * 128 + 2 * lane;
         // requested now, needed only by the finishing workgroup: by then they are here
         half2_t sv, bv;
@@ -278,20 +279,20 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(
                     vx = __fadd_rn(vx, red[w][m][2 * lane]);
                     vy = __fadd_rn(vy, red[w][m][2 * lane + 1]);
                 }
-                const unsigned long long ax = fix_word(vx), ay = fix_word(vy);
+                const unsigned long long ax = fix_word(vx, bits), ay = fix_word(vy, bits);
                 unsigned long long* slot = sums + (size_t)m * out_total + col;
                 w0[m] = __hip_atomic_fetch_add(slot, ax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + ax;
                 w1[m] = __hip_atomic_fetch_add(slot + 1, ay, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + ay;
             }
         }
         // lane 0's first word is (row 0, first column of the group)
-        const int first_count = __builtin_amdgcn_readfirstlane(fix_count(w0[0]));
+        const int first_count = __builtin_amdgcn_readfirstlane(fix_count(w0[0], bits));
         if (first_count != wg_splits) return;
         auto all_complete = [&]() {
             bool ok = true;
 #pragma unroll
             for (int m = 0; m < MT; m++)
-                if (m < rows) ok = ok && fix_count(w0[m]) == wg_splits && fix_count(w1[m]) == wg_splits;
+                if (m < rows) ok = ok && fix_count(w0[m], bits) == wg_splits && fix_count(w1[m], bits) == wg_splits;
             return __ballot(ok) == ~0ull;
         };
         bool complete = all_complete();
@@ -328,8 +329,8 @@ __global__ __launch_bounds__(NW * 64) void linear_small_kernel(
                 __hip_atomic_store(slot + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 // the cast at ponyexl3/ref/forward.py:41, then the output Hadamard of this one
                 // 128-column block, svh and bias (forward.py:42-45)
-                float a = (float)(half_t)fix_value(w0[m]);
-                float b = (float)(half_t)fix_value(w1[m]);
+                float a = (float)(half_t)fix_value(w0[m], bits);
+                float b = (float)(half_t)fix_value(w1[m], bits);
                 wht128_lanes(a, b, lane);
                 a = __fmul_rn(a, kHadScaleF);
                 b = __fmul_rn(b, kHadScaleF);
@@ -522,7 +523,7 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
 bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
     if (plan.batch) return linear_batch_uses_atomics(rows, n_groups, plan);
     static const int kMaxAtomics = env_int("EXL3_LINEAR_MAX_ATOMICS", 300000, 0, 1 << 30);
-    if (plan.n_partials() > 255) return false;  // the count field has eight bits
+    if (plan.n_partials() > kFixMaxContributors) return false;
     const long long limit = rows == 2 ? (long long)kMaxAtomics * 8 / 3 : kMaxAtomics;
     return (long long)n_groups * plan.n_partials() * 128 * rows <= limit;
 }

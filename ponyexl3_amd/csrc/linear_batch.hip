@@ -363,13 +363,14 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
     half2_t o[MR];
     if constexpr (ATOMIC) {
         unsigned long long* sums = reinterpret_cast<unsigned long long*>(counters) + col;
+        const int bits = fix_count_bits(wg_splits);
         unsigned long long w0[MR], w1[MR];
 #pragma unroll
         for (int i = 0; i < MR; i++) {
             w0[i] = w1[i] = 0;
             const int m = wave + NW * i;
             if (m < rows) {
-                const unsigned long long ax = fix_word(va[i]), ay = fix_word(vb[i]);
+                const unsigned long long ax = fix_word(va[i], bits), ay = fix_word(vb[i], bits);
                 unsigned long long* slot = sums + (size_t)m * out_total;
                 w0[i] = __hip_atomic_fetch_add(slot, ax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + ax;
                 w1[i] = __hip_atomic_fetch_add(slot + 1, ay, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + ay;
@@ -380,7 +381,7 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
         // the same barrier: the polls wait for waves that run, not for one to be scheduled.
         __shared__ int finishes, gave_up;
         if (threadIdx.x == 0) {
-            finishes = fix_count(w0[0]) == wg_splits;
+            finishes = fix_count(w0[0], bits) == wg_splits;
             gave_up = 0;
         }
         __syncthreads();
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
             if (m >= rows) break;
             const unsigned long long* slot = sums + (size_t)m * out_total;
             auto complete = [&]() {
-                return __ballot(fix_count(w0[i]) == wg_splits && fix_count(w1[i]) == wg_splits) == ~0ull;
+                return __ballot(fix_count(w0[i], bits) == wg_splits && fix_count(w1[i], bits) == wg_splits) == ~0ull;
             };
             bool ok = complete();
             for (int spin = 0; !ok && spin < spin_limit; spin++) {
@@ -412,8 +413,8 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
                 __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(slot + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            va[i] = fix_value(w0[i]);
-            vb[i] = fix_value(w1[i]);
+            va[i] = fix_value(w0[i], bits);
+            vb[i] = fix_value(w1[i], bits);
         }
         batch_finish<MR>(va, vb, svh, bias, col, lane, o);
 #pragma unroll
@@ -485,9 +486,13 @@ static int batch_rows(int rows) { return rows <= 4 ? 4 : rows <= 8 ? 8 : 16; }
 // reload costs 1-2 us more than a returning atomic. Where the two met in a sweep of 2..8 rows, by
 // millions of weights: 10 180 k atomics, 17 200 k, 42 520 k, 52 660 k, 89 1500 k, 178 1750 k; at 3
 // rows of 8192 -> 5120 11.9 against 15.0 us, at 8 rows 22.0 against 17.0 (four waves per workgroup).
+// Launches that linear_small_kernel would reduce through fp32 partial rows (four whole blocks to each)
+// take accumulators only where these are as good: up to 31 contributors, 30 fraction bits.
 bool linear_batch_uses_atomics(int rows, int n_groups, GemvPlan plan) {
-    if (rows > 8 || plan.n_partials() > 255) return false;  // the count field has eight bits
+    if (rows > 8 || plan.n_partials() > kFixMaxContributors) return false;
     const long long weights = (long long)n_groups * 128 * plan.n_splits * 64;
+    const long long whole_blocks = (long long)n_groups * ((plan.n_splits + 7) / 8) * 128 * rows;
+    if (plan.n_partials() > kFixFineContributors && whole_blocks > (rows == 2 ? 800000 : 300000)) return false;
     return (long long)n_groups * plan.n_partials() * 128 * rows <= 60000 + weights / 100;
 }
 
@@ -500,11 +505,15 @@ bool linear_batch_uses_atomics(int rows, int n_groups, GemvPlan plan) {
 //              5 rows K = 4 21.7 -> 22.7, K = 6 25.5 -> 23.6
 //   9..16 rows 1664 -> 2560 16 rows 11.2 -> 9.1 (with the rotation's launch), 2560 -> 4096 12.5 -> 9.4, 8192 -> 5120
 //              21.2 -> 18.5; 5120 -> 10240 20.2 -> 21.7
+// Reductions too long for fine accumulators (linear_batch_uses_atomics) at 3..4 rows pay 3 us for their partial
+// rows and end earlier: 17408 -> 3328 (3536) K = 4 18.1 -> 17.9, 16384 -> 3456 (3456) K = 4 16.7 -> 17.2, 17408 ->
+// 4352 (4624) K = 6 22.7 -> 21.1, 17408 -> 5120 (5440) K = 6 22.7 -> 23.4, K = 8 26.7 -> 25.1.
 bool linear_batch_applies(int rows, int in_tiles, int n_groups, int K) {
     if (rows < 2 || rows > kLinearBatchMaxRows) return false;
     const long long units = (long long)(in_tiles / 8) * n_groups;
     if (rows > 8) return units <= 2700;
     if (rows > 4) return units <= (K >= 5 ? 5000 : 3300);
+    if (rows > 2 && in_tiles > 32 * kFixFineContributors) return units <= (K >= 7 ? 12000 : K == 6 ? 5000 : 3400);
     // (the top line keeps the partial rows of exl3_linear_forward_static within its array)
     return units <= (K >= 6 ? 12000 : K == 5 ? 5000 : 4096);
 }

@@ -428,6 +428,7 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
     red[wave][c0 + 8] = acc[0][1];
     __syncthreads();
     if (wave != 0) return;
+    const int bits = fix_count_bits(n_chunks);
     // word q of a lane: projection q >> 1, column 2*lane + (q & 1); wave order within a projection
     unsigned long long w[4];
     unsigned long long* slot[4];
@@ -438,14 +439,14 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
 #pragma unroll
         for (int i = 1; i < 4; i++) v = __fadd_rn(v, red[w0 + i][col]);
         slot[q] = sums + ((size_t)s * 2 + (q >> 1)) * H + hg * 128 + col;
-        const unsigned long long a = fix_word(v);
+        const unsigned long long a = fix_word(v, bits);
         w[q] = __hip_atomic_fetch_add(slot[q], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + a;
     }
-    if (__builtin_amdgcn_readfirstlane(fix_count(w[0])) != n_chunks) return;
+    if (__builtin_amdgcn_readfirstlane(fix_count(w[0], bits)) != n_chunks) return;
     auto all_complete = [&]() {
         bool ok = true;
 #pragma unroll
-        for (int q = 0; q < 4; q++) ok = ok && fix_count(w[q]) == n_chunks;
+        for (int q = 0; q < 4; q++) ok = ok && fix_count(w[q], bits) == n_chunks;
         return __ballot(ok) == ~0ull;
     };
     bool complete = all_complete();
@@ -471,9 +472,9 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
         __hip_atomic_store(slot[q], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
     float g0, g1, u0, u1;
-    moe_finish_block(float2_t{fix_value(w[0]), fix_value(w[1])},
+    moe_finish_block(float2_t{fix_value(w[0], bits), fix_value(w[1], bits)},
                      *reinterpret_cast<const half2_t*>(svh_e), lane, g0, g1);
-    moe_finish_block(float2_t{fix_value(w[2]), fix_value(w[3])},
+    moe_finish_block(float2_t{fix_value(w[2], bits), fix_value(w[3], bits)},
                      *reinterpret_cast<const half2_t*>(svh_e + H), lane, u0, u1);
     const float h0 = (float)(half_t)glu_act(g0, u0, activation);
     const float h1 = (float)(half_t)glu_act(g1, u1, activation);
@@ -1180,7 +1181,7 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
         // and up of a k-chunk in one workgroup, reduced through returning atomics
         const int pair_chunks = half ? (dblocks + 1) / 2 : (dblocks + 3) / 4;
         const size_t pair_ints = (size_t)slots * 2 * H * 2;
-        const bool pair = !grouped && pair_chunks <= 255 &&
+        const bool pair = !grouped && pair_chunks <= kFixMaxContributors &&
                           (long long)slots * 2 * H * pair_chunks <= moe_max_atomics() &&
                           counters_len >= pair_ints + (size_t)slots * dblocks &&
                           (reinterpret_cast<uintptr_t>(counters) & 7) == 0;

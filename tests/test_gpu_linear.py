@@ -685,3 +685,28 @@ def test_layer_with_general_scales(cuda, oracle, rows, k, n_in, n_out):
     assert rel_l2(y.cpu().numpy(), _oracle_forward(oracle, layer, x)) <= TOL
     few = torch.cat([mod(xt[r:r + 8]) for r in range(0, 32, 8)])
     assert rel_l2(y[:32].float().cpu().numpy(), few.float().cpu().numpy()) <= TOL
+
+
+@pytest.mark.parametrize("rows,n_in,n_out", [(6, 5120, 5120), (4, 8192, 5120), (3, 5120, 10240), (4, 17408, 2560),
+                                             (1, 5120, 1024), (2, 17408, 5120)])
+def test_one_launch_layer_at_small_activations(cuda, rows, n_in, n_out):
+    """Activations of 1e-5: the partial sums of the split reduction keep their bits, whichever way
+    they are added. The inner product in 64 bits on the same rotated activations; what is left is
+    the fp16 cast before and after the output transform (2^-11/sqrt(3) relative at most, 2.8e-4 each) and the
+    weights' unsummed halves (4-5e-4): 6.5e-4 together, so 1e-3. Sums on a grid of 2^-20 are off by 2e-3."""
+    from ponyexl3_amd import make_exl3_layer, ops
+
+    layer = make_exl3_layer(k=4, in_features=n_in, out_features=n_out, seed=n_in + rows)
+    tr = ops.as_trellis_tensor(layer.trellis, cuda)
+    suh, svh = torch.from_numpy(layer.suh).to(cuda), torch.from_numpy(layer.svh).to(cuda)
+    x = (torch.randn((rows, n_in), device=cuda, generator=torch.Generator(cuda).manual_seed(rows)) * 1e-5).half()
+    print("small activations", rows, n_in, n_out, flush=True)
+    got = ops.linear_forward(x, tr, 4, 0, suh, svh, fused=True).double()
+    h = torch.ones((1, 1), dtype=torch.float64, device=cuda)
+    for _ in range(7):
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    rotate = lambda v: (v.reshape(rows, -1, 128) @ h).reshape(rows, -1) / 128 ** 0.5
+    xh = rotate(x.double() * suh.double()).half()
+    inner = xh.double() @ ops.decode_full(tr, 4, 0).double()
+    ref = rotate(inner) * svh.double()
+    assert rel_l2(got.cpu().numpy(), ref.cpu().numpy()) <= 1e-3

@@ -93,3 +93,60 @@ def test_preseeded_count_never_completes(shim):
     for _ in range(5):
         w = (w + shim.shim_fix_word(1.0)) & MASK
     assert shim.shim_fix_count(w) == 4
+
+
+def _reduce(lib, partial):
+    partial = np.ascontiguousarray(partial, np.float32)
+    c, n = partial.shape
+    total, count = np.empty(n, np.float32), np.empty(n, np.int32)
+    as_p = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    lib.shim_fix_reduce(as_p(partial), c, n, as_p(total), as_p(count))
+    return total, count
+
+
+@pytest.mark.parametrize("contributors", [1, 2, 10, 15, 16, 20, 31])
+@pytest.mark.parametrize("scale", [30.0, 1.0, 1e-3, 1e-4, 1e-5, 1e-6])
+def test_words_of_few_contributors_lose_nothing_against_fp32_partial_rows(shim, contributors, scale):
+    """Totals of partial sums of 512 products at activations of `scale`, after the fp16 cast that
+    follows: as far from 64 bits as an fp32 sum in index order. Up to 31 contributors the words
+    have 30 fraction bits or more; their roundings (31 of 2^-30/sqrt(12) rms) are at most 1/11 of the
+    rms of the cast on fp16's finest grid, 2^-24/sqrt(12): 0.4 % of its error, tolerance 1 %."""
+    rng = np.random.default_rng(contributors)
+    partial = (rng.standard_normal((contributors, 1 << 15)) * (scale * 512 ** 0.5 * 1.24)).astype(np.float32)
+    exact = partial.astype(np.float64).sum(axis=0)
+    rows = partial[0].copy()
+    for p in partial[1:]:
+        rows += p
+    total, count = _reduce(shim, partial)
+    assert (count == contributors).all()
+    err = lambda v: float(np.linalg.norm(v.astype(np.float16).astype(np.float64) - exact))
+    assert np.isfinite(total).all()
+    assert err(total) <= 1.01 * err(rows) + 1e-12
+
+
+@pytest.mark.parametrize("contributors", [1, 15, 16, 31, 32, 63, 64, 127, 128, 255])
+def test_words_at_both_ends_of_every_count_width(shim, contributors):
+    """Extremes of the clamp, a single non-finite contributor and nothing but non-finite ones, at the
+    smallest and the largest number of contributors of each width of the count."""
+    c, big = contributors, 262144.0
+    cols = np.full((c, 6), big, np.float32)
+    cols[:, 1] = -big
+    cols[:, 2] = np.inf
+    cols[0, 3] = np.nan
+    cols[0, 4] = -np.inf
+    cols[:, 4][1:] = -big
+    cols[:, 5] = np.where(np.arange(c) % 2, -3.5, 3.5)
+    total, count = _reduce(shim, cols)
+    assert (count == c).all()
+    assert total[0] == c * big and total[1] == -c * big
+    assert np.isnan(total[2:5]).all()
+    assert total[5] == (3.5 if c % 2 else 0.0)
+    # a word that starts with the count's field full never reads as complete
+    lib, b = shim, shim.shim_fix_count_bits(c)
+    lib.shim_fix_word_bits.restype = ctypes.c_uint64
+    lib.shim_fix_word_bits.argtypes = [ctypes.c_float, ctypes.c_int]
+    lib.shim_fix_count_of.argtypes = [ctypes.c_uint64, ctypes.c_int]
+    w = 0xFF << 56
+    for _ in range(c):
+        w = (w + lib.shim_fix_word_bits(big, b)) & MASK
+    assert lib.shim_fix_count_of(w, b) == c - 1

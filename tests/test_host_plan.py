@@ -1,0 +1,36 @@
+"""Launch plans of the one-launch layer kernels as the library reports them (no GPU needed)."""
+import ctypes
+
+import pytest
+
+
+def _plan(lib, rows, n_in, n_out, k):
+    out = [ctypes.c_int() for _ in range(4)]
+    assert lib.exl3_linear_plan(rows, n_in // 16, n_out // 16, k, *[ctypes.byref(v) for v in out]) == 0
+    n_splits, tile_rows, waves, atomic = (v.value for v in out)
+    return -(-n_splits // waves), tile_rows, waves, bool(atomic)
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from ponyexl3_amd import _lib
+
+    return _lib.load()
+
+
+@pytest.mark.parametrize("rows", range(2, 9))
+def test_large_launches_reduce_in_fp32_or_in_words_as_good(lib, rows):
+    """A launch of more atomics than the whole-block kernel sends through its accumulators (300 k, 800 k at
+    two rows) takes fp32 partial rows, or words of at least 30 fraction bits: up to 31 partial rows."""
+    limit = 800000 if rows == 2 else 300000
+    seen = 0
+    for n_in in (1664, 2560, 5120, 6144, 8192, 14336, 15872, 16000, 16384, 17408):
+        for n_out in (1024, 2560, 5120, 5888, 10240, 12288, 34816):
+            for k in range(1, 9):
+                partials, tile_rows, waves, atomic = _plan(lib, rows, n_in, n_out, k)
+                # per column group: the same splits in partial rows of eight waves of half blocks
+                whole = n_out * rows * (-(-n_in // 512) if tile_rows == 4 else partials)
+                if atomic and whole > limit:
+                    seen += 1
+                    assert partials <= 31, (n_in, n_out, k)
+    assert seen or rows in (2, 7, 8)
