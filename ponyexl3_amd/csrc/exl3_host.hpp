@@ -243,6 +243,18 @@ inline bool exact_weights() {
     return v != 0;
 }
 
+// EXL3_LINEAR_MAX_ATOMICS: one-launch layers that would issue more atomics than this (8/3 of it at two
+// rows) reduce through partial rows, whichever kernel they take. Not set (-1): each kernel's own line.
+inline int linear_max_atomics_set() {
+    static const int v = env_int("EXL3_LINEAR_MAX_ATOMICS", -1, 0, 1 << 30);
+    return v;
+}
+// Line of linear_small_kernel.
+inline long long linear_small_max_atomics(int rows) {
+    const long long v = linear_max_atomics_set() < 0 ? 300000 : linear_max_atomics_set();
+    return rows == 2 ? v * 8 / 3 : v;
+}
+
 // Polls a finishing workgroup spends on accumulators whose counts are not complete yet
 // before it gives up (EXL3_SPIN_LIMIT; read at every launch so that a test can lower it).
 inline int reduction_spin_limit() { return env_int("EXL3_SPIN_LIMIT", 1 << 22, 1, 1 << 30); }

@@ -522,10 +522,8 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
 // at four rows neither limit gains (86.0 / 86.6 / 90.4 us at 300 k / 800 k / 1.6 M).
 bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
     if (plan.batch) return linear_batch_uses_atomics(rows, n_groups, plan);
-    static const int kMaxAtomics = env_int("EXL3_LINEAR_MAX_ATOMICS", 300000, 0, 1 << 30);
     if (plan.n_partials() > kFixMaxContributors) return false;
-    const long long limit = rows == 2 ? (long long)kMaxAtomics * 8 / 3 : kMaxAtomics;
-    return (long long)n_groups * plan.n_partials() * 128 * rows <= limit;
+    return (long long)n_groups * plan.n_partials() * 128 * rows <= linear_small_max_atomics(rows);
 }
 
 GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K) {

@@ -488,12 +488,15 @@ static int batch_rows(int rows) { return rows <= 4 ? 4 : rows <= 8 ? 8 : 16; }
 // rows of 8192 -> 5120 11.9 against 15.0 us, at 8 rows 22.0 against 17.0 (four waves per workgroup).
 // Launches that linear_small_kernel would reduce through fp32 partial rows (four whole blocks to each)
 // take accumulators only where these are as good: up to 31 contributors, 30 fraction bits.
+// EXL3_LINEAR_MAX_ATOMICS, where it is set, takes the place of both lines.
 bool linear_batch_uses_atomics(int rows, int n_groups, GemvPlan plan) {
     if (rows > 8 || plan.n_partials() > kFixMaxContributors) return false;
-    const long long weights = (long long)n_groups * 128 * plan.n_splits * 64;
+    const long long atomics = (long long)n_groups * plan.n_partials() * 128 * rows;
+    if (linear_max_atomics_set() >= 0) return atomics <= linear_small_max_atomics(rows);
     const long long whole_blocks = (long long)n_groups * ((plan.n_splits + 7) / 8) * 128 * rows;
-    if (plan.n_partials() > kFixFineContributors && whole_blocks > (rows == 2 ? 800000 : 300000)) return false;
-    return (long long)n_groups * plan.n_partials() * 128 * rows <= 60000 + weights / 100;
+    if (plan.n_partials() > kFixFineContributors && whole_blocks > linear_small_max_atomics(rows)) return false;
+    const long long weights = (long long)n_groups * 128 * plan.n_splits * 64;
+    return atomics <= 60000 + weights / 100;
 }
 
 // Half blocks double the waves and rotate 128 values for 64 rows of weights, which pays while the

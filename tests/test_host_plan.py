@@ -1,7 +1,12 @@
 """Launch plans of the one-launch layer kernels as the library reports them (no GPU needed)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
+
+from conftest import ROOT
 
 
 def _plan(lib, rows, n_in, n_out, k):
@@ -34,3 +39,31 @@ def test_large_launches_reduce_in_fp32_or_in_words_as_good(lib, rows):
                     seen += 1
                     assert partials <= 31, (n_in, n_out, k)
     assert seen or rows in (2, 7, 8)
+
+
+_PLANS = """
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+from ponyexl3_amd import _lib
+lib = _lib.load()
+for rows in range(1, 9):
+    for n_in, n_out in ((128, 128), (1664, 2560), (5120, 1024), (5120, 5120), (5120, 10240), (17408, 5120), (5120, 34816)):
+        for k in (2, 4, 6, 8):
+            out = [ctypes.c_int() for _ in range(4)]
+            assert lib.exl3_linear_plan(rows, n_in // 16, n_out // 16, k, *[ctypes.byref(v) for v in out]) == 0
+            n_splits, _, waves, atomic = (v.value for v in out)
+            partials = -(-n_splits // waves)
+            print(partials, partials * n_out * rows * 3 // (8 if rows == 2 else 3), atomic)
+"""
+
+
+@pytest.mark.parametrize("limit", [0, 50000, 300000, 1 << 30])
+def test_the_atomics_switch_reaches_every_one_launch_kernel(limit):
+    """EXL3_LINEAR_MAX_ATOMICS (read once per process): launches of more atomics reduce through partial rows,
+    launches of as many or fewer through accumulators, whether waves take whole or half blocks."""
+    env = dict(os.environ, EXL3_LINEAR_MAX_ATOMICS=str(limit))
+    run = subprocess.run([sys.executable, "-c", _PLANS, ROOT], env=env, capture_output=True, text=True, check=True)
+    rows = [tuple(map(int, line.split())) for line in run.stdout.splitlines()]
+    assert len(rows) == 8 * 7 * 4
+    for partials, atomics, atomic in rows:
+        assert atomic == (partials <= 255 and atomics <= limit)
