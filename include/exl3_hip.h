@@ -404,7 +404,8 @@ size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
  *   workspace      at least exl3_moe_workspace_bytes(tokens, kk, D, H)
  *   counters       int32 [counters_len], counters_len >= exl3_moe_decode_counters(tokens, kk, D, H),
  *                  8-byte aligned, zero on entry and on exit; the last int is the status word
- * tokens * kk <= 4096; the limits of exl3_moe_route.
+ * tokens * kk <= 4096; the limits of exl3_moe_route (top_k <= 64, n_router <= 1024, else
+ * EXL3_E_UNSUPPORTED), also where the experts' kernel ranks.
  */
 size_t exl3_moe_decode_counters(int tokens, int slots_per_token, int D, int H);
 int exl3_moe_decode(const uint16_t *x, int tokens, const uint16_t *logits,

@@ -6,6 +6,9 @@
 
 namespace exl3 {
 
+constexpr int kRouteMaxExperts = 1024;  // 16 per lane
+constexpr int kRouteMaxTopK = 64;       // one per lane
+
 template <int CTRL>
 __device__ __forceinline__ int dpp_i32(int v) {
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);

@@ -1327,6 +1327,8 @@ EXL3_EXPORT int exl3_moe_decode(const uint16_t* x, int tokens, const uint16_t* l
     if (tokens < 1 || n_router < 1 || top_k < 1 || top_k > n_router || D < 128 || H < 128 || D % 128 || H % 128 ||
         n_router + (shared_logits != nullptr) > num_experts || (shared_logits && n_router != num_experts - 1))
         return EXL3_E_BAD_SHAPE;
+    // whoever ranks, the router's kernel or the experts'
+    if (n_router > kRouteMaxExperts || top_k > kRouteMaxTopK) return EXL3_E_UNSUPPORTED;
     if ((reinterpret_cast<uintptr_t>(slot_rows) & 15) || (reinterpret_cast<uintptr_t>(out) & 15)) return EXL3_E_BAD_SHAPE;
     const int kk = top_k + (shared_logits != nullptr);
     if (counters_len < exl3_moe_decode_counters(tokens, kk, D, H)) return EXL3_E_WORKSPACE;

@@ -10,9 +10,6 @@
 
 namespace exl3 {
 
-constexpr int kRouteMaxExperts = 1024;  // 16 per lane
-constexpr int kRouteMaxTopK = 64;       // one per lane
-
 // fp16(x . w) over a wave, fp32 sums; n % 8 == 0
 __device__ __forceinline__ half_t wave_dot(const half_t* __restrict__ x, const half_t* __restrict__ w, int n, int lane) {
     float acc[8] = {};

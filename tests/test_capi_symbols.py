@@ -107,6 +107,29 @@ def test_argument_errors_before_launch(lib):
     assert lib.exl3_moe_forward(p, 1, p, 8, p, p, p, p, p, p, 4, 256, 128, 4, 0, 7, p, p, 1 << 20, None, 0, None) == _lib.EXL3_E_UNSUPPORTED
 
 
+def test_moe_decode_keeps_the_limits_of_the_router(lib):
+    """exl3_moe_decode ranks at most 64 choices (one per lane) of at most 1024 experts, as exl3_moe_route
+    does, also where the experts' kernel ranks them itself (up to 256 experts)."""
+    from ponyexl3_amd import _lib
+
+    p = ctypes.c_void_p(0x1000)  # never dereferenced: the checks below fail first
+
+    def decode(n_router, top_k, shared=False, experts=None, tokens=1):
+        experts = experts or n_router + shared
+        return lib.exl3_moe_decode(p, tokens, p, p if shared else None, n_router, top_k, 1, p, p, p, p, p, p, experts, 256,
+                                   128, 4, 0, 0, p, p, p, p, p, 0, p, 1 << 30, None)
+
+    fits = _lib.EXL3_E_WORKSPACE  # the next check: the workspace's length, which is 0 here
+    for shared in (False, True):
+        assert decode(128, 64, shared) == fits
+        assert decode(128, 65, shared) == _lib.EXL3_E_UNSUPPORTED
+        assert decode(256, 256, shared) == _lib.EXL3_E_UNSUPPORTED
+        assert decode(1024, 8, shared) == fits
+        assert decode(1025, 8, shared) == _lib.EXL3_E_UNSUPPORTED
+        assert decode(64, 65, shared) == _lib.EXL3_E_BAD_SHAPE
+    assert lib.exl3_moe_route(p, 0, None, 1, 128, 65, 1, p, p, None) == _lib.EXL3_E_UNSUPPORTED
+
+
 def test_workspace_sizes(lib):
     assert lib.exl3_gemv_workspace_bytes(1, 256, 32) >= 4096 * 4
     assert lib.exl3_gemv_workspace_bytes(0, 256, 32) == 0
