@@ -127,13 +127,15 @@ __global__ __launch_bounds__(256) void decode_full_t_kernel(const uint32_t* __re
 // over the rows of the block:
 //   Y[i][n] = fp16(sum_j +-q_i W[j][n]),   Z[i][m] = fp16(sum_n +-Y[i][n] / sqrt(128) * svh_m)
 // Both run on the matrix pipe (v_mfma_f32_16x16x32_f16, fp32 sums in the order of the
-// prefill GEMM), the fragments of H made from sign words each lane holds. 512 MFMAs
-// per block = 21 us for 5120 x 17408 and the decode 9 us, so the kernel is bound by writing
-// the result; it goes out through LDS in 256-byte row pieces, non-temporal (nobody reads it
-// soon; 65 -> 62 us). One 34 KiB LDS tile serves all three stages (each stage reads its
-// operands into registers before the next one writes), so several workgroups share a CU and
-// their phases overlap; four instead of three per CU (128 registers) is no faster.
-// Measured, 5120 x 17408 at K = 4, transposed: 62 us (3.6 TB/s of trellis and result); the
+// prefill GEMM), the fragments of H made from sign words each lane holds. For 5120 x 17408 at
+// K = 4 VALU issue (decode, signs, conversions) takes 35 us of a SIMD's time, the matrix pipe 18,
+// and a plain fill of the result would take 26: no unit is full. What the kernel waits for is its own
+// sequence, load, decode, transform, transform, store, with five barriers between and no load of the
+// next block in flight (waves wait half of their time). The result goes out through LDS in
+// 256-byte row pieces, non-temporal (nobody reads it soon; 65 -> 62 us). One 34 KiB LDS tile serves
+// all three stages (each stage reads its operands into registers before the next one writes), so four
+// workgroups share a CU and their phases overlap.
+// Measured, 5120 x 17408 at K = 4, transposed: 60 us (3.7 TB/s of trellis and result); the
 // identity through the prefill kernels, the concatenation of its column stripes and the
 // transposed copy took 1.42 ms.
 constexpr int kPubLd = 128 + kDecPad;  // halfs per row: 16-byte reads of 16 rows hit all banks

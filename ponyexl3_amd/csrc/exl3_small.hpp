@@ -69,9 +69,10 @@ __device__ __forceinline__ XChunk<MT> load_x_chunk(const half_t* const (&xr)[(MT
 // used up. The matrix instruction of a chunk and column is issued after half of the next one has been
 // decoded, so it never waits for the VALU result it reads.
 //
-// The sums have to live in accumulation registers (keep_in_agprs): the decode is inline assembly,
-// and the compiler does not see that its VALU writes must not follow a matrix instruction too
-// closely into registers that this one still reads as its third operand.
+// The sums live in accumulation registers (keep_in_agprs): the half adds of the rounded form below
+// are inline assembly, and the compiler does not see that their VALU writes must not follow a matrix
+// instruction too closely into registers that this one still reads as its third operand. The decode of
+// the unsummed form is plain code, which the compiler keeps apart by itself; it shares the declaration.
 __device__ __forceinline__ void keep_in_agprs(float4_t& v) { asm("" : "+a"(v)); }
 
 template <int K, int CB, int MT, class LoadChunk>

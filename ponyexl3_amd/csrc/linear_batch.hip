@@ -329,7 +329,7 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
         for (int i = 0; i < T::NQ; i++) {
 #pragma unroll
             for (int c = 0; c < (T::EXACT ? 16 : 4); c++) acc[cs].v[i][c] = 0.f;
-            if constexpr (!T::EXACT) asm("" : "+a"(acc[cs].v[i]));  // see keep_in_agprs()
+            if constexpr (!T::EXACT) asm("" : "+a"(acc[cs].v[i]));  // as keep_in_agprs()
         }
     if (split < n_splits)
         batch_main<K, CB, R>(trellis + (size_t)g * 8 * (8 * K) + lane * K, (size_t)out_tiles * (8 * K), split * 4, x,

@@ -67,19 +67,22 @@ struct SearchMap {
     // fma gets it as fp32: with three plain registers it runs at the rate of the simple
     // operations (2.5 cycles per wave and SIMD against 4 for the mixed one, where runs of them
     // meet). K = 3..5: the rows in LDS hold fp32; K = 2, where a lane writes as many costs as it
-    // reads, they are converted when read. From K = 6 on every cost is used once.
+    // reads, they are converted when read. From K = 6 on every cost is used once. With fp16 rows and the
+    // mixed fma instead, all else as it is, ms at 4096 / 64 tiles: K = 2 11.4 / 0.79 against 11.0 / 0.73,
+    // 3 11.0 / 0.77 against 9.4 / 0.62, 4 10.6 / 0.77 against 9.0 / 0.60, 5 10.5 / 0.78 against 8.4 / 0.61.
     static constexpr bool PLAIN_FMA = K <= 5, WIDE = K >= 3 && K <= 5;
     // Rows go to the history by the lanes that make them, [lane][target][group], a store each, or (not
-    // DIRECT) as 16-byte pieces of the finished LDS row in the next step. K = 3, 4096 tiles: 9.05 ms against
-    // 9.29; K = 5 8.02 against 8.10; K = 2 10.9 against 10.6, K = 4 8.8 against 8.5.
+    // DIRECT) as 16-byte pieces of the finished LDS row in the next step. K = 3, 4096 tiles: 9.36 ms against
+    // 9.67, 64 tiles 0.62 against 0.67; K = 5 8.37 against 8.39; K = 2 10.9 against 10.6, K = 4 8.8 against 8.5.
     static constexpr bool DIRECT = K == 3 || K == 5;
     static constexpr int COST = WIDE ? 4 : 2, ROW_BYTES = COST * EDGES;  // row in LDS
     static constexpr int HIST_BYTES = 2 * EDGES;                          // row in the history, fp16
     typedef std::conditional_t<WIDE, float, half_t> cost_t;
     // Steps that a move of the backtrack goes back. Two up to K = 3, where the 2^2K sources of the sources
     // fit the lanes: only every other row is kept, and those rows are what the search writes most
-    // of (K = 2: 32 KB per step, at 256 CUs 6 TB/s). At K = 4 there are four to a lane, which cost more
-    // registers and time than the rows (64 tiles 604 -> 660 us).
+    // of (K = 2: 32 KB per step, at 256 CUs 6 TB/s). One step at a time, ms at 4096 / 64 tiles: K = 2 13.0 / 0.77
+    // against 11.0 / 0.73, K = 3 10.3 / 0.66 against 9.4 / 0.62. At K = 4 there are four to a lane, which cost
+    // more registers and time than the rows (64 tiles 604 -> 660 us).
     static constexpr int BACK = K <= 3 ? 2 : 1;
     // Byte offset of source (f, p) in a cost row. The 16-byte units are permuted by exclusive-or so
     // that the lanes of a wave hit different LDS banks in both directions: consecutive p when
@@ -270,9 +273,10 @@ __device__ __forceinline__ uint32_t search_two_back(half_t cost, uint32_t& edge,
 // subtraction only beside the mixed fma. 16 waves of at most 128 registers fill the CU, so the
 // whole of a step hides its own LDS latency; one barrier per step. The wave that backtracks (0) waits for
 // its loads of a step before it stores, and in the forms that copy finished rows it stores nothing.
-// Measured, 4096 tiles (MCG), ms, before (mixed fma, fp16 rows, every row kept) and now: K = 2 13.3 -> 10.6, 3 11.4
-// -> 9.05, 4 11.1 -> 8.5, 5 11.1 -> 8.0, 6 11.2 -> 9.9, 7 11.8 -> 10.7, 8 11.8 -> 10.7; up to 256 tiles at once 0.84 -> 0.73,
-// 0.81 -> 0.63, 0.81 -> 0.61, 0.82 -> 0.61, 0.79 -> 0.70, 0.83 -> 0.76, 0.87 -> 0.78.
+// Measured, 4096 tiles (MCG), ms, before the four (mixed fma, fp16 rows, every row kept and copied, subtractions) and with
+// all of them: K = 2 13.3 -> 10.6, 3 11.4 -> 9.05, 4 11.1 -> 8.5, 5 11.1 -> 8.0, 6 11.2 -> 9.9, 7 11.8 -> 10.7, 8 11.8
+// -> 10.7; up to 256 tiles at once 0.84 -> 0.73, 0.81 -> 0.63, 0.81 -> 0.61, 0.82 -> 0.61, 0.79 -> 0.70, 0.83 -> 0.76, 0.87
+// -> 0.78. What each gives by itself is beside it (SearchMap, and the differences below).
 template <int K, int CB>
 __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
     const float* __restrict__ tiles, float* __restrict__ q_tiles, uint16_t* __restrict__ indices,
@@ -446,7 +450,9 @@ __global__ __launch_bounds__(kSearchThreads, 1) void quantize_tiles_kernel(
                             halfs_to_floats(q, pc);  // folded into the fma
                         }
                         // From K = 6 on sixteen differences at a time come from the matrix pipe (-target times one
-                        // on top of the values: one rounding, as the subtraction), a batch ahead.
+                        // on top of the values: one rounding, as the subtraction), a batch ahead. With the
+                        // subtraction, ms at 4096 / 64 tiles: K = 6 10.4 / 0.72 against 10.0 / 0.69, 7 11.1 / 0.77
+                        // against 10.7 / 0.75, 8 11.65 / 0.85 against 10.9 / 0.76.
                         if constexpr (!M::PLAIN_FMA) {
                             if (fc % 16 == 0) {
                                 diff = diff_next;
