@@ -475,7 +475,7 @@ def bench_ceilings(dev):
     """What this GPU delivers, measured in the same run: a streaming read of cold
     memory (the denominator next to the published 8 TB/s), and the small-batch
     kernels' inner loop on its own (wave-wide load, per-lane decode of 32 codewords,
-    16 matrix-pipe dot products; one workgroup of 16 waves per CU, 128 tile rows per
+    8 matrix instructions; one workgroup of 16 waves per CU, 128 tile rows per
     wave, no Hadamard, no reduction): the rate the VALU instruction sequence of the
     bit-exact decode allows before any layer structure is added. 'cold' walks over a
     2 GiB buffer so that every launch reads memory no earlier launch of the
