@@ -215,6 +215,12 @@ int launch_had_pre_pairs(const uint16_t* x, int tokens, int top_k, int n, const 
                          const int32_t* indices, const uint16_t* gu_suh, int n_experts, uint16_t* xg,
                          size_t sub_stride, hipStream_t stream);
 
+// exl3_moe_route with the list of slot groups behind it (exl3_groups.hpp): num_experts >= every index of
+// the table, at most kGroupMaxSlots slots; `arrived`: an int that is zero, and is again afterwards.
+int launch_moe_route_groups(const uint16_t* logits, const uint16_t* shared_logits, int tokens, int n_experts, int top_k,
+                            int norm, int32_t* indices, uint16_t* scores, int num_experts, int4* groups, int* arrived,
+                            hipStream_t stream);
+
 // Experts of rows sorted by expert (row-block table as exl3_moe_sort's, blocks of 32 or 64):
 // gate, up, GLU and rotation to xd [n_rows][H], down to out[order[r]] [..][D].
 int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const uint16_t* gu_trellis,

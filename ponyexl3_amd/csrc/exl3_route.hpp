@@ -107,20 +107,25 @@ __device__ __forceinline__ int route_next(int (&key)[EPL], int lane, int j, Rout
 }
 
 // Row t of the routing table after top_k choices, with a shared expert behind them whose gate's logit
-// is given.
-template <typename T>
+// is given. PUBLISH: indices through the level that the XCDs share, for a workgroup of the same launch.
+template <typename T, bool PUBLISH = false>
 __device__ __forceinline__ void route_write(RouteChoice c, int lane, int t, int n_experts, int top_k, int norm,
                                             bool shared, T shared_logit, int* __restrict__ indices,
                                             half_t* __restrict__ scores) {
     if (norm) c.p = c.p / wave_sum_f32(c.p);
     const int slots = top_k + shared;
+    auto put = [&](int j, int e) {
+        int* at = indices + (size_t)t * slots + j;
+        if constexpr (PUBLISH) __hip_atomic_store(at, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else *at = e;
+    };
     if (lane < top_k) {
-        indices[(size_t)t * slots + lane] = c.e;
+        put(lane, c.e);
         scores[(size_t)t * slots + lane] = (half_t)c.p;
     }
     if (shared && lane == 0) {
         const float s = (float)shared_logit;
-        indices[(size_t)t * slots + top_k] = n_experts;
+        put(top_k, n_experts);
         scores[(size_t)t * slots + top_k] = (half_t)(float)(T)(1.0f / (1.0f + expf(-s)));
     }
 }

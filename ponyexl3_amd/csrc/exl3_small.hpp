@@ -146,16 +146,6 @@ __device__ __forceinline__ void load_lane_words_nt(const uint32_t* __restrict__ 
     for (int i = 0; i < K; i++) own[i] = __builtin_nontemporal_load(p + i);
 }
 
-// The same through a pointer that is declared to be in global memory (for addresses
-// whose origin the compiler cannot see; it would otherwise emit flat loads).
-using global_words_t = const uint32_t __attribute__((address_space(1)))*;
-
-template <int K>
-__device__ __forceinline__ void load_lane_words_nt(global_words_t p, uint32_t (&own)[K]) {
-#pragma unroll
-    for (int i = 0; i < K; i++) own[i] = __builtin_nontemporal_load(p + i);
-}
-
 // One wave streams tile rows [tk_begin, tk_end) (both multiples of 8, non-empty)
 // of the 8 tile columns that start at `base` (already offset by lane*K dwords)
 // and accumulates acc[m][0..1] += x[m][rows of the tile] . W[:, column u / u+8].
@@ -175,12 +165,11 @@ __device__ __forceinline__ void load_lane_words_nt(global_words_t p, uint32_t (&
 // The batch rows are given by address (xrow[m], m < MT; entries past `rows` repeat a
 // valid row), so that a caller can gather them. GUARD: rows past `rows` are neither
 // loaded nor rotated (their LDS rows and sums are then meaningless and must not be
-// used). PRELOADED: the caller has already issued the first trellis loads into `buf`
-// with issue_first_rows (to overlap their latency with work of its own).
+// used).
 constexpr int kStreamSlots = 4;  // wave-wide loads in flight (divides the 8 steps of a block)
 
-template <int K, bool HALF, class Words>
-__device__ __forceinline__ void issue_first_rows(Words base, size_t row_words, int tk_begin,
+template <int K, bool HALF>
+__device__ __forceinline__ void issue_first_rows(const uint32_t* __restrict__ base, size_t row_words, int tk_begin,
                                                  int tk_end, uint32_t (&buf)[kStreamSlots][K]) {
 #pragma unroll
     for (int s = 0; s < kStreamSlots; s++) {
@@ -189,15 +178,14 @@ __device__ __forceinline__ void issue_first_rows(Words base, size_t row_words, i
     }
 }
 
-template <int K, int CB, int MT, bool ROTATE, bool HALF, bool GUARD, bool PRELOADED,
-          bool EXACT = false>
+template <int K, int CB, int MT, bool ROTATE, bool HALF, bool GUARD, bool EXACT = false>
 __device__ __forceinline__ void stream_block_rows_at(const uint32_t* __restrict__ base,
                                                      size_t row_words, int tk_begin, int tk_end,
                                                      const half_t* const (&xrow)[MT], int rows,
                                                      const half_t* __restrict__ suh_row,
                                                      half_t (*xw)[kXwLd], int lane,
-                                                     float (&acc)[MT][2],
-                                                     uint32_t (&buf)[kStreamSlots][K]) {
+                                                     float (&acc)[MT][2]) {
+    uint32_t buf[kStreamSlots][K];
     half2_t xraw[MT], sraw;
     auto fetch_block = [&](int blk) {
         const int off = blk * 128 + 2 * lane;
@@ -266,7 +254,7 @@ __device__ __forceinline__ void stream_block_rows_at(const uint32_t* __restrict_
     // order, so the rotation then only waits for the activations and the decode of the
     // first row only for that row, not for all kSlots rows.
     fetch_block(tk_begin >> 3);
-    if constexpr (!PRELOADED) issue_first_rows<K, HALF>(base, row_words, tk_begin, tk_end, buf);
+    issue_first_rows<K, HALF>(base, row_words, tk_begin, tk_end, buf);
     __builtin_amdgcn_sched_barrier(0);  // all of them in flight before the rotation starts
     if constexpr (HALF) {
         // all four loads up front, no refills
@@ -322,9 +310,8 @@ __device__ __forceinline__ void stream_block_rows(const uint32_t* __restrict__ b
     const half_t* xrow[MT];
 #pragma unroll
     for (int m = 0; m < MT; m++) xrow[m] = x + (size_t)(m < rows ? m : 0) * x_stride;
-    uint32_t buf[kStreamSlots][K];
-    stream_block_rows_at<K, CB, MT, ROTATE, HALF, (MT > 2), false, EXACT>(
-        base, row_words, tk_begin, tk_end, xrow, rows, suh_row, xw, lane, acc, buf);
+    stream_block_rows_at<K, CB, MT, ROTATE, HALF, (MT > 2), EXACT>(
+        base, row_words, tk_begin, tk_end, xrow, rows, suh_row, xw, lane, acc);
 }
 
 }  // namespace exl3

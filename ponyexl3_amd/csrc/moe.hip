@@ -32,10 +32,12 @@
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 #include "exl3_glu.hpp"
+#include "exl3_groups.hpp"
 #include "exl3_route.hpp"
 #include "exl3_small.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -545,105 +547,41 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
 
 // ---------------------------------------------------------------------------
 // The same chain with the slots grouped by expert. With several tokens, slots that
-// route to the same expert share one pass over its weights: the grid stays one
-// workgroup set per slot, every workgroup finds the slots of its own expert in the
-// routing table, and only the first of every four of them (in slot order) works, on up
-// to four batch rows (the matrix instructions carry four rows at the price of
-// one). The others leave at once. Per row the arithmetic, the partial rows and the
+// route to the same expert share one pass over its weights: a workgroup set per entry of the list
+// that make_slot_groups() has left, up to four batch rows each (the matrix instructions carry
+// four rows at the price of one). The grid holds as many sets as there could be groups (one per
+// slot); those past the list leave after one scalar load. Per row the arithmetic, the partial rows and the
 // counters are those of the kernels above, so the results are bit-identical.
 
-constexpr int kGroupRows = 4;       // batch rows one workgroup carries
-constexpr int kGroupMaxSlots = 512; // routing table entries a workgroup scans (8 per lane)
-
 struct SlotGroup {
-    int n;               // rows of this workgroup; 0 = another workgroup carries this slot
+    int n;               // rows; 0 = past the list
     int expert;
-    int s0, s1, s2, s3;  // the rows' slots, ascending; entries past n repeat s0
+    int s0, s1, s2, s3;  // the rows' slots; past n: s0
 };
 
-// Loads above stay above, work below stays below (in the optimiser, which would sink
-// loads to their first use, and in the instruction scheduler): the routing table is
-// requested first, the first trellis rows second, and the search of the table runs
-// while the trellis rows are in flight. Emits no instruction.
-__device__ __forceinline__ void pin_program_order() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// The same address with its origin hidden from the optimiser: loads through a kernel
-// argument that is declared free of aliases may otherwise move across pin_program_order.
-__device__ __forceinline__ global_words_t opaque_pointer(const uint32_t* p) {
-    asm volatile("" : "+v"(p));
-    return (global_words_t)p;
-}
-
-// A wave's copy of the routing table: lane l holds entries c*64 + l (the last entry
-// repeated past the end). Always the same number of loads, whatever `slots` is, so
-// that the wait for them can leave younger loads in flight.
-struct SlotTable {
-    int idx[kGroupMaxSlots / 64];
-};
-
-__device__ __forceinline__ SlotTable load_slot_table(const int* __restrict__ indices, int slots,
-                                                     int lane) {
-    SlotTable t;
-#pragma unroll
-    for (int c = 0; c < kGroupMaxSlots / 64; c++) t.idx[c] = indices[min(c * 64 + lane, slots - 1)];
-    return t;
-}
-
-// Nothing computed from the table may be placed above this point.
-__device__ __forceinline__ void use_table_from_here(SlotTable& t) {
-#pragma unroll
-    for (int c = 0; c < kGroupMaxSlots / 64; c++) asm volatile("" : "+v"(t.idx[c]));
-}
-
-// Every wave computes the same answer (wave-uniform values). Branch-free: the matches
-// of chunk c are a 64-bit ballot; the slots before s are counted, the first three
-// after s extracted.
-__device__ __forceinline__ SlotGroup find_slot_group(const SlotTable& t, int slots, int s,
-                                                     int expert, int E, int lane) {
-    constexpr int kChunks = kGroupMaxSlots / 64;
-    const int sc = s >> 6, sb = s & 63;
-    const uint64_t below = (1ull << sb) - 1ull;
-    uint64_t after[kChunks];
-    int before = 0;
-#pragma unroll
-    for (int c = 0; c < kChunks; c++) {
-        const uint64_t m =
-            __ballot(c * 64 + lane < slots && clamp_expert(t.idx[c], E) == expert);
-        before += __popcll(c < sc ? m : (c == sc ? m & below : 0ull));
-        after[c] = c < sc ? 0ull : (c == sc ? m & ~(below | (1ull << sb)) : m);
-    }
-    int n = 1, next[kGroupRows - 1];
-#pragma unroll
-    for (int take = 0; take < kGroupRows - 1; take++) {
-        int pos = -1;
-#pragma unroll
-        for (int c = kChunks - 1; c >= 0; c--)
-            if (after[c] != 0) pos = c;  // lowest chunk that still has a match
-#pragma unroll
-        for (int c = 0; c < kChunks; c++) {
-            if (pos == c) {
-                pos = c * 64 + (int)__builtin_ctzll(after[c]) + (1 << 20);
-                after[c] &= after[c] - 1;
-            }
-        }
-        next[take] = pos < 0 ? s : pos - (1 << 20);
-        n += pos >= 0;
-    }
+// (both entries are requested together)
+__device__ __forceinline__ SlotGroup load_slot_group(const int4* __restrict__ list, int i) {
+    const int count = list[0].x;
+    const int4 v = list[1 + i];
     SlotGroup g;
-    g.expert = expert;
-    g.n = __builtin_amdgcn_readfirstlane((before % kGroupRows) == 0 ? n : 0);
-    g.s0 = s;
-    g.s1 = __builtin_amdgcn_readfirstlane(next[0]);
-    g.s2 = __builtin_amdgcn_readfirstlane(next[1]);
-    g.s3 = __builtin_amdgcn_readfirstlane(next[2]);
+    g.n = i < count ? v.y : 0;
+    g.expert = v.x;
+    g.s0 = v.z & 0xFFFF;
+    g.s1 = g.n > 1 ? (int)((uint32_t)v.z >> 16) : g.s0;
+    g.s2 = g.n > 2 ? v.w & 0xFFFF : g.s0;
+    g.s3 = g.n > 3 ? (int)((uint32_t)v.w >> 16) : g.s0;
     return g;
 }
 
 __device__ __forceinline__ int group_slot(const SlotGroup& g, int r) {
     return r == 1 ? g.s1 : (r == 2 ? g.s2 : (r == 3 ? g.s3 : g.s0));
+}
+
+// The list for a routing table that is there already.
+__global__ __launch_bounds__(kGroupThreads) void moe_groups_kernel(const int* __restrict__ indices, int slots, int E,
+                                                                   int4* list) {
+    __shared__ GroupScratch scratch;
+    make_slot_groups([&](int s) { return clamp_expert(indices[s], E); }, slots, E, list, scratch);
 }
 
 // The NW waves' sums of batch row r, added in wave order.
@@ -659,16 +597,16 @@ __device__ __forceinline__ float2_t moe_row_sum(const float (*red)[kGroupRows][1
     return v;
 }
 
-// Same grid and arguments as moe_gateup_kernel (+ slots). Wave r of the working
+// Grid and arguments as moe_gateup_kernel, the list in place of the routing table. Wave r of a
 // workgroup takes batch row r through the split reduction and, as the last
 // contributor of (slot, column block), through gate finish, up finish, GLU and the
 // rotation for the down projection.
 template <int K, int CB, int NW>
 __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
     const uint32_t* __restrict__ gu_trellis, const half_t* __restrict__ x,
-    const int* __restrict__ indices, const half_t* __restrict__ gu_suh,
+    const int4* __restrict__ groups, const half_t* __restrict__ gu_suh,
     const half_t* __restrict__ gu_svh, const half_t* __restrict__ dn_suh, half_t* xh_dn,
-    float* part, int* counters, int slots, int top_k, int E, int D, int H, int activation) {
+    float* part, int* counters, int top_k, int E, int D, int H, int activation) {
     __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<kGroupRows>][kXwLd];
     __shared__ float red[NW][kGroupRows][128];
     const int lane = threadIdx.x & 63;
@@ -677,38 +615,27 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
     const int n_wg = gridDim.y;
     const int gid = blockIdx.x;
     const int hg = gid % hblocks, sp = gid / hblocks;
-    const int s = sp >> 1, p = sp & 1;
-    // the first trellis loads only need this slot's own expert: they are in flight
-    // while the routing table is searched; workgroups that carry nothing drop them
-    const int e = clamp_expert(indices[s], E);
+    const int p = sp & 1;
+    const SlotGroup grp = load_slot_group(groups, sp >> 1);
+    if (grp.n == 0) return;
+    const int e = grp.expert;
     constexpr bool kHalf = NW == 8;
     const int part_idx = blockIdx.y * NW + wave;
     const int blk = kHalf ? part_idx >> 1 : part_idx;
-    // (waves past the last block load the last block's rows and drop them, so that every
-    // wave has the same loads in flight behind the table's)
-    const int tk0 = min(blk, dblocks - 1) * 8 + (kHalf ? (part_idx & 1) * 4 : 0);
-    const int tk1 = tk0 + (kHalf ? 4 : 8);
-    const size_t row_words = (size_t)E * 2 * (H >> 4) * (8 * K);
-    const uint32_t* base =
-        gu_trellis + ((size_t)(p * E + e) * (H >> 4) + 8 * hg) * (8 * K) + lane * K;
-    SlotTable table = load_slot_table(indices, slots, lane);
-    uint32_t buf[kStreamSlots][K];
-    pin_program_order();
-    issue_first_rows<K, kHalf>(opaque_pointer(base), row_words, tk0, tk1, buf);
-    pin_program_order();
-    use_table_from_here(table);
-    const SlotGroup grp = find_slot_group(table, slots, s, e, E, lane);
-    if (grp.n == 0) return;
+    const int tk0 = blk * 8 + (kHalf ? (part_idx & 1) * 4 : 0);
     float acc[kGroupRows][2];
 #pragma unroll
     for (int m = 0; m < kGroupRows; m++) acc[m][0] = acc[m][1] = 0.f;
     if (blk < dblocks) {
+        const size_t row_words = (size_t)E * 2 * (H >> 4) * (8 * K);
+        const uint32_t* base =
+            gu_trellis + ((size_t)(p * E + e) * (H >> 4) + 8 * hg) * (8 * K) + lane * K;
         const half_t* xrow[kGroupRows];
 #pragma unroll
         for (int m = 0; m < kGroupRows; m++) xrow[m] = x + (size_t)(group_slot(grp, m) / top_k) * D;
-        stream_block_rows_at<K, CB, kGroupRows, true, kHalf, true, true, true>(
-            base, row_words, tk0, tk1, xrow, grp.n, gu_suh + ((size_t)e * 2 + p) * D, xs[wave],
-            lane, acc, buf);
+        stream_block_rows_at<K, CB, kGroupRows, true, kHalf, true, true>(
+            base, row_words, tk0, tk0 + (kHalf ? 4 : 8), xrow, grp.n, gu_suh + ((size_t)e * 2 + p) * D, xs[wave],
+            lane, acc);
     }
     const int c0 = (lane >> 3) * 16 + (lane & 7);
 #pragma unroll
@@ -767,12 +694,13 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
     if (lane == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Same grid and arguments as moe_down_kernel (+ slots); wave r finishes batch row r.
-template <int K, int CB, int NW>
+// Grid and arguments as moe_down_kernel, the list in place of the routing table; wave r finishes
+// batch row r. EXACT: weights rounded to fp16 before the product (moe_exact_down()).
+template <int K, int CB, int NW, bool EXACT>
 __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
     const uint32_t* __restrict__ dn_trellis, const half_t* __restrict__ xh_dn,
-    const int* __restrict__ indices, const half_t* __restrict__ dn_svh, half_t* y, float* part, int* counters,
-    MoeCombine combine, int slots, int E, int D, int H) {
+    const int4* __restrict__ groups, const half_t* __restrict__ dn_svh, half_t* y, float* part, int* counters,
+    MoeCombine combine, int E, int D, int H) {
     __shared__ __attribute__((aligned(16))) half_t xs[NW][kXwRows<kGroupRows>][kXwLd];
     __shared__ float red[NW][kGroupRows][128];
     const int lane = threadIdx.x & 63;
@@ -780,32 +708,25 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
     const int dblocks = D >> 7, hblocks = H >> 7;
     const int n_wg = gridDim.y;
     const int gid = blockIdx.x;
-    const int og = gid % dblocks, s = gid / dblocks;
-    const int e = clamp_expert(indices[s], E);
+    const int og = gid % dblocks;
+    const SlotGroup grp = load_slot_group(groups, gid / dblocks);
+    if (grp.n == 0) return;
+    const int e = grp.expert;
     constexpr bool kHalf = NW == 8;
     const int part_idx = blockIdx.y * NW + wave;
     const int blk = kHalf ? part_idx >> 1 : part_idx;
-    const int tk0 = min(blk, hblocks - 1) * 8 + (kHalf ? (part_idx & 1) * 4 : 0);
-    const int tk1 = tk0 + (kHalf ? 4 : 8);
-    const size_t row_words = (size_t)E * (D >> 4) * (8 * K);
-    const uint32_t* base = dn_trellis + ((size_t)e * (D >> 4) + 8 * og) * (8 * K) + lane * K;
-    SlotTable table = load_slot_table(indices, slots, lane);
-    uint32_t buf[kStreamSlots][K];
-    pin_program_order();
-    issue_first_rows<K, kHalf>(opaque_pointer(base), row_words, tk0, tk1, buf);
-    pin_program_order();
-    use_table_from_here(table);
-    const SlotGroup grp = find_slot_group(table, slots, s, e, E, lane);
-    if (grp.n == 0) return;
+    const int tk0 = blk * 8 + (kHalf ? (part_idx & 1) * 4 : 0);
     float acc[kGroupRows][2];
 #pragma unroll
     for (int m = 0; m < kGroupRows; m++) acc[m][0] = acc[m][1] = 0.f;
     if (blk < hblocks) {
+        const size_t row_words = (size_t)E * (D >> 4) * (8 * K);
+        const uint32_t* base = dn_trellis + ((size_t)e * (D >> 4) + 8 * og) * (8 * K) + lane * K;
         const half_t* xrow[kGroupRows];
 #pragma unroll
         for (int m = 0; m < kGroupRows; m++) xrow[m] = xh_dn + (size_t)group_slot(grp, m) * H;
-        stream_block_rows_at<K, CB, kGroupRows, false, kHalf, true, true>(
-            base, row_words, tk0, tk1, xrow, grp.n, nullptr, xs[wave], lane, acc, buf);
+        stream_block_rows_at<K, CB, kGroupRows, false, kHalf, true, EXACT>(
+            base, row_words, tk0, tk0 + (kHalf ? 4 : 8), xrow, grp.n, nullptr, xs[wave], lane, acc);
     }
     const int c0 = (lane >> 3) * 16 + (lane & 7);
 #pragma unroll
@@ -854,6 +775,28 @@ static int moe_half_below() {
 static bool moe_group_slots() {
     static const int v = env_int("EXL3_MOE_GROUP", 1, 0, 1);
     return v != 0;
+}
+
+// Whether the slots are grouped by expert: where that is expected to spare enough passes over an expert's
+// weights to pay for the list and for reducing through partial rows, a quarter of the slots and
+// 18 of them (router choices taken as independent and even; a shared expert has all tokens). Whole
+// block, us, every slot on its own -> grouped, passes spared of slots: 8 tokens through 256 experts of 2048 x 512, top-8
+// 6.6 of 64 46.3 -> 48.6; 14 tokens 20 of 112 65.8 -> 63.1; 24 with a shared expert 74 of 216 97 (the table searched
+// by every wave) -> 89; 5 tokens, 64 of 1792 x 512 5.3 of 25 26.8 -> 30.3; 10 tokens, 64 of 1408 x 384 20 of 60 36.1 -> 31.6;
+// 10 tokens, 64 of 1536 x 512 40 of 90 48.4 -> 40.7. Of 74 such calls one (17 of 42) ends up more than 3 % above the better.
+static bool moe_groups_apply(int tokens, int top_k, int num_experts, bool shared) {
+    const long long slots = (long long)tokens * top_k;
+    if (tokens < 2 || slots > kGroupMaxSlots || num_experts > kGroupMaxExperts || !moe_group_slots()) return false;
+    const double experts = num_experts - (shared && num_experts > 1), chosen = top_k - shared;
+    const double passes = experts * (1.0 - std::pow(1.0 - std::min(1.0, chosen / experts), tokens)) + (shared ? (tokens + 3) / 4 : 0);
+    return slots - passes >= std::max(18.0, 0.25 * slots);
+}
+
+// Calls of a size that the sorted prefill kernels also serve get the rounded weights of those in the down
+// projection too, so that the result is no further from the reference's arithmetic whichever is faster
+// (7.1e-4 of the output with unsummed halves, 6.8e-4 with rounded weights, against 64 bits).
+static bool moe_exact_down(int tokens, int slots, int num_experts) {
+    return tokens >= 24 && (slots > 512 || slots >= 2.5 * num_experts);
 }
 
 // Gate/up launches that would issue more atomics than this reduce through partial rows
@@ -1144,10 +1087,20 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
         (long long)tokens * top_k > 4096)
         return EXL3_E_BAD_SHAPE;
     if (activation != 0 && activation != 1) return EXL3_E_UNSUPPORTED;
-    // the router in a launch of its own (unless the kernel of a few slots does it)
-    auto route_table = [&]() {
+    // the router in a launch of its own (unless the kernel of a few slots does it), with the list of
+    // groups if one is wanted
+    auto route_table = [&](int4* groups = nullptr, int* arrived = nullptr) {
         const MoeRoute& r = a.route;
-        if (!r.logits) return (int)EXL3_OK;
+        if (!r.logits) {
+            if (!groups) return (int)EXL3_OK;
+            moe_groups_kernel<<<dim3(1), dim3(kGroupThreads), 0, s>>>(indices, tokens * top_k, num_experts, groups);
+            return launch_status();
+        }
+        if (groups)
+            return launch_moe_route_groups(reinterpret_cast<const uint16_t*>(r.logits),
+                                           reinterpret_cast<const uint16_t*>(r.shared_logits), tokens, r.n_experts,
+                                           top_k - (r.shared_logits != nullptr), r.norm, indices,
+                                           reinterpret_cast<uint16_t*>(r.scores), num_experts, groups, arrived, s);
         return exl3_moe_route(r.logits, 0, r.shared_logits, tokens, r.n_experts, top_k - (r.shared_logits != nullptr),
                               r.norm, indices, reinterpret_cast<uint16_t*>(r.scores), s);
     };
@@ -1171,11 +1124,7 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
         // few slots: eight waves per workgroup, each on half a block, so that the
         // chip holds twice the loads in flight (same workgroup count, same partial rows)
         const bool half = (size_t)slots * 2 * hblocks * dblocks < (size_t)moe_half_below();
-        // several tokens: slots of one expert share a pass over its weights, once enough
-        // of them coincide to pay for the table search (from one slot per two experts on:
-        // 16 tokens of top-8 over 256 experts, where ~20 % of the slots share an expert)
-        const bool grouped = tokens > 1 && slots <= kGroupMaxSlots && 2 * slots >= num_experts &&
-                             moe_group_slots();
+        const bool grouped = moe_groups_apply(tokens, top_k, num_experts, a.route.shared_logits != nullptr);
         // every slot on its own, few enough atomics, and counters large enough to hold
         // the accumulators (uint64 [slots][2][H], then the down launch's counters): gate
         // and up of a k-chunk in one workgroup, reduced through returning atomics
@@ -1186,8 +1135,11 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
                           counters_len >= pair_ints + (size_t)slots * dblocks &&
                           (reinterpret_cast<uintptr_t>(counters) & 7) == 0;
         const bool routes = pair && a.route.n_experts <= kInlineRouteExperts;
+        // the list takes the place of the chain's tables (2 (2 H + D) / 128 ints per slot: four per slot
+        // and four more from two slots on); the counter behind those of the two launches
+        int4* const groups = grouped ? reinterpret_cast<int4*>(base + w.o_tables) : nullptr;
         if (!routes)
-            if (int rc = route_table()) return rc;
+            if (int rc = route_table(groups, counters + (size_t)slots * (hblocks + dblocks))) return rc;
         auto chain = [&](auto k, auto c, auto nw) {
             constexpr int NW = nw.value;
             if (pair) {
@@ -1216,20 +1168,24 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
                 moe_gateup_grouped_kernel<k.value, c.value, NW>
                     <<<dim3((unsigned)(slots * 2 * hblocks), (unsigned)((dblocks + 3) / 4)),
                        dim3(NW * 64), 0, s>>>(reinterpret_cast<const uint32_t*>(gu_trellis),
-                                              reinterpret_cast<const half_t*>(x), indices,
+                                              reinterpret_cast<const half_t*>(x), groups,
                                               reinterpret_cast<const half_t*>(gu_suh),
                                               reinterpret_cast<const half_t*>(gu_svh),
                                               reinterpret_cast<const half_t*>(dn_suh), xh_dn,
-                                              part_gu, counters, slots, top_k, num_experts, D, H,
+                                              part_gu, counters, top_k, num_experts, D, H,
                                               activation);
                 if (int rc = launch_status()) return rc;
-                moe_down_grouped_kernel<k.value, c.value, NW>
-                    <<<dim3((unsigned)(slots * dblocks), (unsigned)((hblocks + 3) / 4)),
-                       dim3(NW * 64), 0, s>>>(reinterpret_cast<const uint32_t*>(dn_trellis), xh_dn,
-                                              indices, reinterpret_cast<const half_t*>(dn_svh),
-                                              reinterpret_cast<half_t*>(y), part_dn,
-                                              counters + (size_t)slots * hblocks, a.combine, slots,
-                                              num_experts, D, H);
+                auto down = [&](auto exact) {
+                    moe_down_grouped_kernel<k.value, c.value, NW, exact.value>
+                        <<<dim3((unsigned)(slots * dblocks), (unsigned)((hblocks + 3) / 4)),
+                           dim3(NW * 64), 0, s>>>(reinterpret_cast<const uint32_t*>(dn_trellis), xh_dn,
+                                                  groups, reinterpret_cast<const half_t*>(dn_svh),
+                                                  reinterpret_cast<half_t*>(y), part_dn,
+                                                  counters + (size_t)slots * hblocks, a.combine,
+                                                  num_experts, D, H);
+                };
+                if (moe_exact_down(tokens, slots, num_experts)) down(std::true_type{});
+                else down(std::false_type{});
                 return launch_status();
             }
             moe_gateup_kernel<k.value, c.value, NW>

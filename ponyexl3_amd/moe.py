@@ -6,6 +6,8 @@ router / weighted sum of ``EXL3MoEBlock`` (ponyexl3/mlx/exl3_moe.py:790-839).
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import torch
 from torch.nn.modules.module import (_global_backward_hooks, _global_backward_pre_hooks, _global_forward_hooks,
@@ -97,24 +99,32 @@ class EXL3SwitchGLU(torch.nn.Module):
     # The sorted, segmented prefill path replaces the slot kernels once the experts see
     # a few rows each (the reference switches at 9 tokens,
     # ponyexl3/mlx/exl3_moe.py:770-787). The slot kernels share one pass over an expert's
-    # weights among up to four of its slots as long as the call has at most 512 slots; above
-    # that every slot is on its own. Measured (experts of one call, us, slot kernels and
-    # prefill): 256 experts of 2048 x 512, top-8, K = 4: 63 and 82 at 16 tokens, 99 and 112 at
-    # 32, 127 and 140 at 48, 150 and 151 at 64, 251 and 147 at 68 (544 slots). Fewer experts
-    # with more rows each: 64 of 2048 x 768, top-6, 82 and 72 at 28 tokens, 153 and 75 at 64; 128
-    # of 1024 x 768, top-8, 79 and 67 at 40. So: prefill above 512 slots, and below that from
-    # 2.5 rows per expert on. The lines were drawn with a slower prefill chain and are not where
-    # the two cross for every size: at K = 6 the 256 experts cross at 36 tokens (194 and 164 at
-    # 64), 8 experts with top-2 at 64 only (26 and 44 at 24).
+    # weights among up to four of its slots as long as the call has at most 1024 slots; above
+    # that every slot is on its own. Below it both times grow with passes over an expert's weights: groups of
+    # four slots here, blocks of 32 rows and the rows themselves there, whose sort, rotation and
+    # combination cost more to begin with. With routing taken as even, in us for experts of 2^20 weights per
+    # projection: 28 + 0.50 groups against 42 + 0.51 blocks + 0.019 slots up to 5 bits, 24 + 0.68 groups against
+    # 45 + 0.61 blocks from 6 on, fitted to 58 calls of 10 to 161 tokens (5 us rms; one goes to the slower path by
+    # more than 1 %). Measured, slot kernels and prefill: 256 experts of 2048 x 512, top-8 and a shared one,
+    # K = 4: 142 and 169 at 56 tokens, 167 and 177 at 80, 187 and 179 at 100; 64 of 1152 x 256, top-8: 41 and 54 at 40;
+    # 32 of 1664 x 512, top-7 and a shared one, K = 6: 47 and 64 at 16; 128 of 1280 x 768, top-4 and a shared one,
+    # K = 6: 149 and 122 at 92.
     prefill_min_tokens = 24
-    prefill_min_rows_per_expert = 2.5
-    grouped_max_slots = 512
+    grouped_max_slots = 1024
 
     def _use_prefill(self, tokens: int, top_k: int) -> bool:
         slots = tokens * top_k
-        return tokens >= self.prefill_min_tokens and (
-            slots > self.grouped_max_slots
-            or slots >= self.prefill_min_rows_per_expert * self.num_experts)
+        if tokens < self.prefill_min_tokens or slots > self.grouped_max_slots:
+            return tokens >= self.prefill_min_tokens
+        rows = slots / self.num_experts
+        if rows > 6 or (slots > 512 and rows < 1):
+            return True  # beyond the fit; most slots would be on their own
+        groups = self.num_experts * (rows / 4 + 0.375 * (1 - math.exp(-2 * rows)))
+        blocks = self.num_experts * (1 - math.exp(-rows))
+        size = self.input_dims * self.hidden_dims / 2**20
+        if self._k <= 5:
+            return size * (0.50 * groups - 0.51 * blocks - 0.019 * slots) > 14
+        return size * (0.68 * groups - 0.61 * blocks) > 21
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         if indices.dim() != 3:
