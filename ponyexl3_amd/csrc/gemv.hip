@@ -27,6 +27,7 @@
 #include "exl3_host.hpp"
 #include "exl3_small.hpp"
 
+#include <algorithm>
 #include <stdlib.h>
 
 namespace exl3 {
@@ -467,6 +468,13 @@ GemvPlan plan_gemv(int rows, int in_tiles, int n_groups) {
     return GemvPlan{n_splits, tk_per_split};
 }
 
+// One row: when even one block per wave leaves fewer than this many waves (four per SIMD), the waves
+// take half blocks where the cost below says so; from here on one_row_half_blocks().
+static int linear_half_below() {
+    static const int v = env_int("EXL3_LINEAR_HALF_BELOW", 4096, 0, 1 << 20);
+    return v;
+}
+
 // Plan of the one-launch layer kernel: splits are whole Hadamard blocks (8 tile
 // rows) and every wave gets the same number of blocks where that divides.
 GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
@@ -478,9 +486,7 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
     // K = 6 43.3 -> 40.1 / 23.5 -> 22.2, K = 8 52.7 -> 47.5 / 29.0 -> 25.4 (K <= 4: no
     // gain or a loss).
     static const int kDeepFromK = env_int("EXL3_LINEAR_DEEP_FROM_K", 5, 1, 9);
-    // one row: when even one block per wave leaves fewer than this many waves (four per SIMD),
-    // the waves take half blocks
-    static const int kHalfBelow = env_int("EXL3_LINEAR_HALF_BELOW", 4096, 0, 1 << 20);
+    const int kHalfBelow = linear_half_below();
     const int target_waves = 256 * 4 * kWavesPerSimd;
     const int n_blocks = in_tiles / 8;
     // Half blocks double the waves, which evens out the load of the SIMDs when whole
@@ -523,16 +529,40 @@ GemvPlan plan_linear_small(int rows, int in_tiles, int n_groups, int K) {
 bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
     if (plan.batch) return linear_batch_uses_atomics(rows, n_groups, plan);
     if (plan.n_partials() > kFixMaxContributors) return false;
+    if (plan.tk_per_split == 4 && plan.wg_waves == 8 && linear_max_atomics_set() < 0) return true;  // see one_row_half_blocks()
     return (long long)n_groups * plan.n_partials() * 128 * rows <= linear_small_max_atomics(rows);
+}
+
+// One row of a layer that fills the chip: waves of half a Hadamard block as well, in workgroups of eight.
+// A wave's fixed part (rotation, sums, reduction) is 190 of 1000 VALU instructions with a whole block and
+// comes twice, but a SIMD that would draw five or six waves draws ten or eleven of half the length, all
+// four of their loads go out at once, and no wave waits for a refill: from K = 5 on, where words
+// are more of the time, 10 to 18 % less. Per weight the launch issues 1/512 atomics, 20 k per us
+// where the memory side retires 75 k, so their number is no limit. Layer, us, whole blocks -> half:
+//   5120 -> 34816 K = 2 / 4 / 5 / 6 / 8: 24.7 -> 24.8, 27.3 -> 26.2, 31.5 -> 28.8, 34.7 -> 29.9, 42.8 -> 36.7
+//   4096 -> 24576 K = 4 / 6 / 8: 16.4 -> 16.2, 19.6 -> 18.9, 24.2 -> 22.1; 6144 -> 16384 K = 8 26.4 -> 21.4
+//   7168 -> 36864 K = 4 / 6: 37.7 -> 37.7, 47.2 -> 43.4; 2048 -> 65536 K = 4 / 6: 20.9 -> 21.1, 25.7 -> 24.0
+// Workgroups of four waves spread the work better still where they are few: up to K = 4 within the line of the whole
+// blocks (3072 -> 24576 K = 4 13.8 -> 12.9, eight waves 13.4; K = 6 15.9 and 15.7).
+// Not where that means more contributors to a sum than before and more than 31, whose words have fewer
+// fraction bits than fp32 partial rows are good for.
+static GemvPlan one_row_half_blocks(int in_tiles, int n_groups, int K, GemvPlan whole) {
+    GemvPlan half{in_tiles / 4, 4};
+    if (K > 4 || half.n_partials() > kFixFineContributors || !linear_small_uses_atomics(1, n_groups, half)) half.wg_waves = 8;
+    const bool fine = half.n_partials() <= std::max(kFixFineContributors, whole.n_partials());
+    return fine && linear_small_uses_atomics(1, n_groups, half) ? half : whole;
 }
 
 GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K) {
     if (linear_batch_applies(rows, in_tiles, n_groups, K)) return plan_linear_batch(rows, in_tiles, n_groups);
     GemvPlan plan = plan_linear_small(rows, in_tiles, n_groups, K);
-    if (rows == 1 && plan.tk_per_split >= 8 && !linear_small_uses_atomics(rows, n_groups, plan)) {
-        GemvPlan wide = plan;
-        wide.wg_waves = 8;
-        if (linear_small_uses_atomics(rows, n_groups, wide)) plan = wide;
+    if (rows == 1 && plan.tk_per_split >= 8) {
+        if (!linear_small_uses_atomics(rows, n_groups, plan)) {
+            GemvPlan wide = plan;
+            wide.wg_waves = 8;
+            if (linear_small_uses_atomics(rows, n_groups, wide)) plan = wide;
+        }
+        if ((long long)(in_tiles / 8) * n_groups >= linear_half_below()) plan = one_row_half_blocks(in_tiles, n_groups, K, plan);
     }
     return plan;
 }
@@ -603,8 +633,7 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
         (long long)plan.n_splits * plan.tk_per_split < in_tiles)
         return EXL3_E_BAD_SHAPE;
     const int n_groups = out_tiles / 8;
-    if (plan.wg_waves != 4 && !(plan.wg_waves == 8 && rows == 1 && !half && atomic))
-        return EXL3_E_UNSUPPORTED;
+    if (plan.wg_waves != 4 && !(plan.wg_waves == 8 && rows == 1 && atomic)) return EXL3_E_UNSUPPORTED;
     const dim3 grid((unsigned)n_groups, (unsigned)plan.n_partials());
     const int mt = rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8;
     return dispatch_k_cb(K, cb, [&](auto k, auto c) {
@@ -622,14 +651,18 @@ int launch_linear_small(const uint16_t* x, int rows, const uint16_t* trellis, in
             if (atomic) launch(std::true_type{});
             else launch(std::false_type{});
         };
-        if (plan.wg_waves == 8) {  // one row, whole blocks, accumulators (checked above)
-            linear_small_kernel<k.value, c.value, 1, false, true, 8>
-                <<<grid, dim3(512), 0, stream>>>(
-                    reinterpret_cast<const uint32_t*>(trellis), reinterpret_cast<const half_t*>(x),
-                    reinterpret_cast<const half_t*>(suh), reinterpret_cast<const half_t*>(svh),
-                    reinterpret_cast<const half_t*>(bias), reinterpret_cast<half_t*>(y), partial,
-                    counters, group_sub, in_tiles, out_tiles, rows, n_groups, plan.tk_per_split,
-                    plan.n_splits, status, spin_limit);
+        if (plan.wg_waves == 8) {  // one row, accumulators (checked above)
+            auto wide = [&](auto halfc) {
+                linear_small_kernel<k.value, c.value, 1, halfc.value, true, 8>
+                    <<<grid, dim3(512), 0, stream>>>(
+                        reinterpret_cast<const uint32_t*>(trellis), reinterpret_cast<const half_t*>(x),
+                        reinterpret_cast<const half_t*>(suh), reinterpret_cast<const half_t*>(svh),
+                        reinterpret_cast<const half_t*>(bias), reinterpret_cast<half_t*>(y), partial,
+                        counters, group_sub, in_tiles, out_tiles, rows, n_groups, plan.tk_per_split,
+                        plan.n_splits, status, spin_limit);
+            };
+            if (half) wide(std::true_type{});
+            else wide(std::false_type{});
             return launch_status();
         }
         using T = std::true_type;
