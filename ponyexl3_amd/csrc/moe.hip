@@ -763,11 +763,19 @@ struct MoeWorkspace {
     int g_gu, g_dn;
 };
 
-// Two-launch chain: below this many whole-block waves in the gate/up launch the waves
-// take half blocks (4096 = four per SIMD).
-static int moe_half_below() {
-    static const int v = env_int("EXL3_MOE_HALF_BELOW", 4096, 0, 1 << 20);
-    return v;
+// Two-launch chain: whether the waves take half Hadamard blocks, eight to a workgroup, instead of whole
+// ones, four to a workgroup (same workgroups, same partial rows). Every slot on its own: where the gate/up launch
+// would have fewer than 3200 waves of whole blocks, three to a SIMD: twice the loads in flight then count for
+// more than a second rotation (block of 8 slots a token, 256 experts of 2048 x 512: 1 token 22.8 -> 21.1 us, 3 tokens 29.5 ->
+// 29.3; 192 of 1536 x 512, 35 slots 29.9 and 32.5, 42 slots 34.3 and 38.1). Grouped slots: below 4096, and from
+// K = 5 on always, where the four tile rows that a wave has in flight take 80 registers and more and whole blocks wait
+// for their refills (20 tokens of 7 slots, 129 experts of 1664 x 512 K = 4 / 5 / 6 / 8 58.5 -> 58.0, 60.8 -> 59.0, 65.8 ->
+// 61.9, 76.4 -> 66.6; 40 of 8 slots, 257 of 2048 x 512 K = 4 115 and 124, K = 8 175 -> 148). EXL3_MOE_HALF_BELOW,
+// where it is set, takes the place of both lines.
+static bool moe_half_blocks(long long whole_waves, bool grouped, int K) {
+    static const int set = env_int("EXL3_MOE_HALF_BELOW", -1, 0, 1 << 20);
+    if (set >= 0) return whole_waves < set;
+    return grouped ? K >= 5 || whole_waves < 4096 : whole_waves < 3200;
 }
 
 // Two-launch chain with several tokens: slots of the same expert in one workgroup (1) or
@@ -1121,10 +1129,8 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
         // two launches: gate/up + GLU + rotation, then down
         const int hblocks = H / 128, dblocks = D / 128;
         if (counters_len < (size_t)slots * (hblocks + dblocks)) return EXL3_E_WORKSPACE;
-        // few slots: eight waves per workgroup, each on half a block, so that the
-        // chip holds twice the loads in flight (same workgroup count, same partial rows)
-        const bool half = (size_t)slots * 2 * hblocks * dblocks < (size_t)moe_half_below();
         const bool grouped = moe_groups_apply(tokens, top_k, num_experts, a.route.shared_logits != nullptr);
+        const bool half = moe_half_blocks((long long)slots * 2 * hblocks * dblocks, grouped, K);
         // every slot on its own, few enough atomics, and counters large enough to hold
         // the accumulators (uint64 [slots][2][H], then the down launch's counters): gate
         // and up of a k-chunk in one workgroup, reduced through returning atomics
