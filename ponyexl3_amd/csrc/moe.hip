@@ -786,18 +786,21 @@ static bool moe_group_slots() {
 }
 
 // Whether the slots are grouped by expert: where that is expected to spare enough passes over an expert's
-// weights to pay for the list and for reducing through partial rows, a quarter of the slots and
-// 18 of them (router choices taken as independent and even; a shared expert has all tokens). Whole
-// block, us, every slot on its own -> grouped, passes spared of slots: 8 tokens through 256 experts of 2048 x 512, top-8
-// 6.6 of 64 46.3 -> 48.6; 14 tokens 20 of 112 65.8 -> 63.1; 24 with a shared expert 74 of 216 97 (the table searched
-// by every wave) -> 89; 5 tokens, 64 of 1792 x 512 5.3 of 25 26.8 -> 30.3; 10 tokens, 64 of 1408 x 384 20 of 60 36.1 -> 31.6;
-// 10 tokens, 64 of 1536 x 512 40 of 90 48.4 -> 40.7. Of 74 such calls one (17 of 42) ends up more than 3 % above the better.
+// weights to pay for the list and for reducing through partial rows, a fifth of the slots and
+// 18 of them (router choices taken as independent and even; a shared expert has all tokens). us,
+// every slot on its own -> grouped, passes spared of slots: 4 tokens through 192 experts of 1920 x 512, top-4 and a
+// shared one, K = 5 3.5 of 20 26.8 -> 30.6; 9 tokens, 192 of 1280 x 256, K = 6 10.4 of 54 27.6 -> 30.2; 13 tokens,
+// 192 of 2048 x 512, top-8, K = 5 22 of 104 64.7 -> 62.9; 13 tokens, 256 of 1664 x 512, K = 8 22 of 104 70.3 -> 64.9; 24
+// tokens, 74 of 216 97 (the table searched by every wave) -> 89; 19 tokens, 128 of 2048 x 512, K = 2 49 of 133 99 -> 76.
+// Of 64 calls of 3 to 22 tokens with 8 to 40 % spared two on the grouped side (20 and 22 of 55 and 63, experts of
+// 1664 x 256 and 1408 x 512) are 4 and 6 % above the other; six on the single side 8 to 14 % (large experts,
+// 7 to 18 spared).
 static bool moe_groups_apply(int tokens, int top_k, int num_experts, bool shared) {
     const long long slots = (long long)tokens * top_k;
     if (tokens < 2 || slots > kGroupMaxSlots || num_experts > kGroupMaxExperts || !moe_group_slots()) return false;
     const double experts = num_experts - (shared && num_experts > 1), chosen = top_k - shared;
     const double passes = experts * (1.0 - std::pow(1.0 - std::min(1.0, chosen / experts), tokens)) + (shared ? (tokens + 3) / 4 : 0);
-    return slots - passes >= std::max(18.0, 0.25 * slots);
+    return slots - passes >= std::max(18.0, 0.2 * slots);
 }
 
 // Calls of a size that the sorted prefill kernels also serve get the rounded weights of those in the down

@@ -100,31 +100,38 @@ class EXL3SwitchGLU(torch.nn.Module):
     # a few rows each (the reference switches at 9 tokens,
     # ponyexl3/mlx/exl3_moe.py:770-787). The slot kernels share one pass over an expert's
     # weights among up to four of its slots as long as the call has at most 1024 slots; above
-    # that every slot is on its own. Below it both times grow with passes over an expert's weights: groups of
-    # four slots here, blocks of 32 rows and the rows themselves there, whose sort, rotation and
-    # combination cost more to begin with. With routing taken as even, in us for experts of 2^20 weights per
-    # projection: 28 + 0.50 groups against 42 + 0.51 blocks + 0.019 slots up to 5 bits, 24 + 0.68 groups against
-    # 45 + 0.61 blocks from 6 on, fitted to 58 calls of 10 to 161 tokens (5 us rms; one goes to the slower path by
-    # more than 1 %). Measured, slot kernels and prefill: 256 experts of 2048 x 512, top-8 and a shared one,
-    # K = 4: 142 and 169 at 56 tokens, 167 and 177 at 80, 187 and 179 at 100; 64 of 1152 x 256, top-8: 41 and 54 at 40;
-    # 32 of 1664 x 512, top-7 and a shared one, K = 6: 47 and 64 at 16; 128 of 1280 x 768, top-4 and a shared one,
-    # K = 6: 149 and 122 at 92.
+    # that every slot is on its own. From 24 tokens on, and 512 slots or 2.5 per expert, the two are close: both
+    # grow with passes over an expert's weights, groups of four slots here, blocks of 32 rows and the rows
+    # themselves there, whose sort, rotation and combination cost more to begin with. us for experts of 2^20 weights
+    # a projection, routing taken as even, by bits per weight: (fixed, per group) and (fixed, per block, per slot),
+    # fitted to 129 calls of 10 to 163 tokens (4 to 5 us rms). Taken only 7 % below the prefill's: of 43 calls of
+    # those sizes none then ends on the slower path by more than 0.5 %, and they take 7 % less than through the prefill.
+    # Measured, slot kernels and prefill: 256 experts of 2048 x 512, top-8 and a shared one, K = 4: 142 and
+    # 169 at 56 tokens, 167 and 177 at 80, 187 and 179 at 100; 64 of 1152 x 256, top-8: 41 and 54 at 40; 128 of
+    # 1280 x 768, top-4 and a shared one, K = 5: 123 and 108 at 89.
     prefill_min_tokens = 24
-    grouped_max_slots = 1024
+    prefill_min_rows_per_expert = 2.5
+    grouped_max_slots = 512
+    _grouped_slots_limit = 1024
+    _grouped_us = ((30.5, 0.42), (28, 0.50), (28, 0.50), (26.4, 0.573), (24.5, 0.606), (23.4, 0.686), (27.8, 0.711))
+    _prefill_us = ((42, 0.51, 0.0), (42, 0.51, 0.019), (42, 0.51, 0.019), (43.4, 0.569, 0.008), (40.2, 0.608, 0.013),
+                   (40.4, 0.568, 0.039), (46.2, 0.586, 0.014))  # K = 2 (and 1) to 8
 
     def _use_prefill(self, tokens: int, top_k: int) -> bool:
         slots = tokens * top_k
-        if tokens < self.prefill_min_tokens or slots > self.grouped_max_slots:
-            return tokens >= self.prefill_min_tokens
+        if tokens < self.prefill_min_tokens or (
+                slots <= self.grouped_max_slots and slots < self.prefill_min_rows_per_expert * self.num_experts):
+            return False
         rows = slots / self.num_experts
-        if rows > 6 or (slots > 512 and rows < 1):
-            return True  # beyond the fit; most slots would be on their own
-        groups = self.num_experts * (rows / 4 + 0.375 * (1 - math.exp(-2 * rows)))
-        blocks = self.num_experts * (1 - math.exp(-rows))
+        # (beyond what was fitted; most slots on their own)
+        if slots > self._grouped_slots_limit or rows > 6 or (slots > self.grouped_max_slots and rows < 1):
+            return True
         size = self.input_dims * self.hidden_dims / 2**20
-        if self._k <= 5:
-            return size * (0.50 * groups - 0.51 * blocks - 0.019 * slots) > 14
-        return size * (0.68 * groups - 0.61 * blocks) > 21
+        fixed, group = self._grouped_us[max(self._k, 2) - 2]
+        grouped = fixed + size * group * self.num_experts * (rows / 4 + 0.375 * (1 - math.exp(-2 * rows)))
+        fixed, block, slot = self._prefill_us[max(self._k, 2) - 2]
+        prefill = fixed + size * (block * self.num_experts * (1 - math.exp(-rows)) + slot * slots)
+        return grouped > 0.93 * prefill
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         if indices.dim() != 3:
