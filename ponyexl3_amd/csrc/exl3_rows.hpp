@@ -78,7 +78,7 @@ struct RowsWords {
     static constexpr int LOADS = (16 * K + 63) / 64;    // wave-wide direct loads of 16 bytes a lane
 };
 
-// acc[mr][cs] (+)= D of 32x32: column m (lane m of the decode: tile m >> 3, column (m & 7) +
+// acc[mr][cs] = D of 32x32: column m (lane m of the decode: tile m >> 3, column (m & 7) +
 // 8 cs of it) x activation row 32 mr + n. A lane holds n = lane & 31 and m = 8 (i >> 2) +
 // 4 (lane >> 5) + (i & 3), i = 0..15.
 //   w         the wave's trellis words at step 0 (uniform): four tiles of its first tile row;
@@ -173,6 +173,13 @@ __device__ __forceinline__ void rows_main(const uint32_t* w, size_t w_row, size_
     load_batch(0, 0);
     load_batch(1, 1);
     load_batch(2, 2);
+    // zeros by the matrix pipe, which idles here: 2 MR instructions in place of 32 MR moves (twice that
+    // where the compiler joins a loop that may not run at all; nsteps >= 1)
+#pragma unroll
+    for (int mr = 0; mr < MR; mr++)
+#pragma unroll
+        for (int cs = 0; cs < 2; cs++)
+            acc[mr][cs] = __builtin_amdgcn_mfma_f32_32x32x16_f16(half8_t{}, half8_t{}, float16_t{}, 0, 0, 0);
     arrive(N2{});
     read_words(0);
     read_a(0, N0{});
@@ -181,7 +188,8 @@ __device__ __forceinline__ void rows_main(const uint32_t* w, size_t w_row, size_
     // no scalar load is under way in the loop, so that waits there can count the LDS reads
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     int s0 = 0, s1 = 1;  // stages of step t and t + 1
-    for (int t = 0; t < nsteps; t++) {
+    int t = 0;
+    do {
         half_step(N0{}, N1{}, [](auto) {});
         arrive(N1{});  // step t + 1 is in LDS; stage s0 has been read by every wave
         read_words(s1);
@@ -194,7 +202,7 @@ __device__ __forceinline__ void rows_main(const uint32_t* w, size_t w_row, size_
         });
         s0 = s1;
         s1 = s1 == 2 ? 0 : s1 + 1;
-    }
+    } while (++t < nsteps);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load lands in LDS after this
     __syncthreads();
 }

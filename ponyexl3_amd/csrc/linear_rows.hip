@@ -116,12 +116,6 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
 #pragma unroll
     for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, NKS>(wave * LPW + i, lane, valid - 1, p.ldx);
     float16_t acc[MR][2];
-#pragma unroll
-    for (int mr = 0; mr < MR; mr++)
-#pragma unroll
-        for (int cs = 0; cs < 2; cs++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[mr][cs][i] = 0.f;
     uint32_t* words = reinterpret_cast<uint32_t*>(stages + 3 * T::STAGE) + wave * RowsWords<K>::STAGE;
     rows_main<K, CB, MR, NKS, LPW>(w, row_words, 2 * NKS * row_words, reinterpret_cast<const char*>(x), a_off, true,
                                    lds_byte_address(stages) + wave * LPW * 1024, stages,

@@ -559,6 +559,35 @@ def test_glu_rows_kernel_equals_separate_launches(cuda, act):
         ops.moe_glu_rows(g, u[:, :256], sidx, gu_svh, dn_suh, act)
 
 
+def test_silu_over_the_range_of_halfs(cuda):
+    """SiLU where its power over- and underflows: gate values from 2^-12 to the fp16 limit and past it (infinite),
+    both signs, against float64. A block's rotation spreads an infinite or undefined value over the whole block; the
+    others are within two fp16 roundings (of h and of the result, 2^-11 each) of the largest h times sqrt(128)."""
+    from ponyexl3_amd import ops
+
+    rng = np.random.default_rng(23)
+    N, H, E = 192, 512, 5
+    g = torch.from_numpy(rng.standard_normal((N, H)).astype(np.float16)).to(cuda)
+    u = torch.from_numpy(rng.standard_normal((N, H)).astype(np.float16)).to(cuda)
+    sidx = torch.from_numpy(np.sort(rng.integers(0, E, size=N)).astype(np.int32)).to(cuda)
+    gu_svh = torch.ones((E, 2 * H), dtype=torch.float16)
+    size = 2.0 ** rng.uniform(-12, 15, (E, H // 128, 128))
+    size[:, 2:] = 2.0 ** rng.uniform(-3, 8, (E, H // 128 - 2, 128))  # (nothing infinite there)
+    gu_svh[:, :H] = torch.from_numpy(size.reshape(E, H).astype(np.float16))
+    gu_svh[:, H:] = 2.0 ** -9
+    gu_svh, dn_suh = gu_svh.to(cuda), torch.ones((E, H), dtype=torch.float16, device=cuda)
+    got = ops.moe_glu_rows(g, u, sidx, gu_svh, dn_suh, 0).double().cpu().view(N, -1, 128)
+    gf = ops.had128_rows(g, gu_svh[:, :H], True, scale_index=sidx).double().cpu()
+    uf = ops.had128_rows(u, gu_svh[:, H:], True, scale_index=sidx).double().cpu()
+    h = (gf / (1 + torch.exp(-gf)) * uf).view(N, -1, 128)
+    ref = ops.had128_rows(h.view(N, H).to(torch.float16).to(cuda), dn_suh, False, scale_index=sidx).double().cpu().view(N, -1, 128)
+    ok = torch.isfinite(h).all(-1)
+    assert (~ok).any() and ok[:, 2:].all() and float(gf[torch.isfinite(gf)].abs().max()) > 4e4
+    assert torch.equal(torch.isfinite(got).all(-1), ok) and not torch.isfinite(got[~ok]).any()
+    bound = 2 * 2.0 ** -11 * 128 ** 0.5 * h.abs().amax(-1, keepdim=True)
+    assert ((got - ref).abs() <= bound)[ok].all()
+
+
 @pytest.mark.parametrize("tokens,E,top_k,norm,fp32", [(1, 1, 1, True, False), (5, 63, 8, True, False),
                                                       (3, 64, 64, False, True), (130, 65, 4, True, True),
                                                       (7, 257, 6, False, False), (4, 1024, 16, True, False)])
