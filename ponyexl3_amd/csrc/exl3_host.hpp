@@ -211,9 +211,12 @@ int launch_had_rows(const uint16_t* x, int n_in_rows, int rows, int n, const int
 
 int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub, uint16_t* xh,
                         hipStream_t stream);
+// Rows of (token, slot) pairs rotated with their experts' scales: in the order `order`, or, without it, in that of the
+// pairs; then also sorted by the same launch (sort: groups and staged are set here).
+struct SortArgs;
 int launch_had_pre_pairs(const uint16_t* x, int tokens, int top_k, int n, const int32_t* order,
                          const int32_t* indices, const uint16_t* gu_suh, int n_experts, uint16_t* xg,
-                         size_t sub_stride, hipStream_t stream);
+                         size_t sub_stride, const SortArgs* sort, hipStream_t stream);
 
 // exl3_moe_route with the list of slot groups behind it (exl3_groups.hpp): num_experts >= every index of
 // the table, at most kGroupMaxSlots slots; `arrived`: an int that is zero, and is again afterwards.
@@ -222,12 +225,13 @@ int launch_moe_route_groups(const uint16_t* logits, const uint16_t* shared_logit
                             hipStream_t stream);
 
 // Experts of rows sorted by expert (row-block table as exl3_moe_sort's, blocks of 32 or 64):
-// gate, up, GLU and rotation to xd [n_rows][H], down to out[order[r]] [..][D].
+// gate, up, GLU and rotation to xd [n_rows][H], down to out[order[r]] [..][D]. gather: row r of xg and xu
+// is at order[r] (32-bit byte offsets).
 int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const uint16_t* gu_trellis,
                     const uint16_t* gu_svh, const uint16_t* dn_trellis, const uint16_t* dn_suh,
                     const uint16_t* dn_svh, int E, int D, int H, int K, int cb, int activation,
                     const int32_t* table, int n_blocks, int block_rows, const int32_t* order,
-                    uint16_t* xd, uint16_t* out, hipStream_t stream);
+                    bool gather, uint16_t* xd, uint16_t* out, hipStream_t stream);
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 

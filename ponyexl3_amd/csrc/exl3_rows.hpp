@@ -44,13 +44,17 @@ struct RowsTile {
 
 // Byte offset in the activation matrix of what lane `lane` of fill `f` of a stage copies
 // (relative to the tile's first row and the step's first column); rows past `last_row` repeat
-// it.
-template <int MR, int NKS>
-__device__ __forceinline__ uint32_t rows_fill_offset(int f, int lane, int last_row, size_t ldx) {
+// it. row_of: where in the matrix a row of the tile is.
+template <int MR, int NKS, typename RowOf>
+__device__ __forceinline__ uint32_t rows_fill_offset(int f, int lane, int last_row, size_t ldx, RowOf row_of) {
     using T = RowsTile<MR, NKS>;
     const int row = f * (64 / T::CHUNKS) + lane / T::CHUNKS;
     const int chunk = (lane % T::CHUNKS) ^ T::swizzle(row);
-    return (uint32_t)((size_t)min(row, last_row) * ldx * 2 + chunk * 16);
+    return (uint32_t)((size_t)row_of(min(row, last_row)) * ldx * 2 + chunk * 16);
+}
+template <int MR, int NKS>
+__device__ __forceinline__ uint32_t rows_fill_offset(int f, int lane, int last_row, size_t ldx) {
+    return rows_fill_offset<MR, NKS>(f, lane, last_row, ldx, [](int row) { return row; });
 }
 
 // Half H of quad I (0..3) of column tile pair CS: the quad is rows 2I, 2I + 1 and 2I + 8, 2I + 9

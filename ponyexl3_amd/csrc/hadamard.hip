@@ -17,6 +17,7 @@
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 #include "exl3_rows.hpp"
+#include "exl3_sort.hpp"
 
 #pragma clang fp contract(off)
 
@@ -117,8 +118,7 @@ __global__ __launch_bounds__(256) void had_pre_wide_kernel(const half_t* __restr
 // instructions of 16 cycles and 2 VALU instructions per element replace about 18, which the
 // butterfly form is bound by. With any other scale value among the wave's rows the products
 // need fp32: the butterfly then runs in this kernel, with the bits of the kernels above.
-// Row maps (MoE rows sorted by expert): row r is pair p = pair[r] of token p / top_k and
-// expert pair_expert[p], whose scales are scale_ld halfs from the next expert's; entries
+// Row maps (MoE): row r is pair p = pair[r] (r without pair) of token p / top_k and expert pair_expert[p], whose scales are scale_ld halfs from the next expert's; entries
 // outside the buffers are clamped.
 // Results: out + s * sub_stride + r * row_stride.
 //
@@ -147,22 +147,22 @@ __device__ __forceinline__ void rotate_tile_order() {
     __builtin_amdgcn_wave_barrier();
 }
 
+// Four waves from wave 4 `block` on; `tiles`: LDS, 16 x kRotateLd halfs to a wave (STREAM).
 template <bool STREAM>
-__global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
-    __shared__ __attribute__((aligned(16))) half_t tiles[STREAM ? 4 : 1][STREAM ? 16 * kRotateLd : 8];
-    half_t* const tile = tiles[STREAM ? threadIdx.x >> 6 : 0];
+__device__ __forceinline__ void rotate_waves(const RotateArgs& a, unsigned block, half_t* tiles) {
+    half_t* const tile = STREAM ? tiles + (threadIdx.x >> 6) * (16 * kRotateLd) : nullptr;
     const int lane = threadIdx.x & 63;
     const int fr = lane & 15, q = lane >> 4;
     const int blocks = a.n >> 7;
-    const long long wid = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const long long wid = (long long)block * 4 + (threadIdx.x >> 6);
     const int row_tiles = (a.rows + 15) >> 4;
     if (wid >= (long long)row_tiles * blocks) return;
     // consecutive waves take consecutive blocks of the same rows
     const int blk = (int)(wid % blocks), r0 = (int)(wid / blocks) * 16, r = r0 + fr;
     const bool valid = r < a.rows;
     int src = valid ? r : 0, scale_row = 0;
-    if (a.pair) {
-        const int p = min(max(a.pair[src], 0), a.n_tokens * a.top_k - 1);
+    if (a.pair_expert) {
+        const int p = a.pair ? min(max(a.pair[src], 0), a.n_tokens * a.top_k - 1) : src;
         scale_row = min(max(a.pair_expert[p], 0), a.n_experts - 1);
         src = p / a.top_k;
     }
@@ -246,20 +246,52 @@ __global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
     }
 }
 
-static int launch_rotate(RotateArgs a, hipStream_t stream) {
+constexpr size_t kRotateTileBytes = (size_t)4 * 16 * kRotateLd * sizeof(half_t);
+
+template <bool STREAM>
+__global__ __launch_bounds__(256, 4) void had_pre_mfma_kernel(RotateArgs a) {
+    __shared__ __attribute__((aligned(16))) half_t tiles[STREAM ? kRotateTileBytes / sizeof(half_t) : 8];
+    rotate_waves<STREAM>(a, blockIdx.x, tiles);
+}
+
+// Rotation of pairs in their own order and, by the first workgroups, their sort, which nothing in the rotation
+// needs: as a launch in front it takes 5 us up to 2000 pairs and 10 us at 13 833, here no more than the
+// rotation does. Whole prefill call with the sort in front and the rows in sorted order -> this way: 97 tokens, 194 pairs
+// 63.5 -> 58.5 us, 400 tokens, 2000 pairs 65.2 -> 60.5, 1537 tokens 289 -> 278; 58 shapes of 45 to 2048 tokens 4.5 %.
+constexpr int kRotateThreads = 256;
+template <bool STREAM>
+__global__ __launch_bounds__(kRotateThreads, 4) void moe_sort_rotate_kernel(RotateArgs a, SortArgs sort) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    if (blockIdx.x >= (unsigned)sort.groups) rotate_waves<STREAM>(a, blockIdx.x - sort.groups, reinterpret_cast<half_t*>(lds));
+    else if (blockIdx.y == 0) sort_pairs<kRotateThreads>(sort, blockIdx.x, reinterpret_cast<int*>(lds));
+}
+
+static int launch_rotate(RotateArgs a, const SortArgs* sort, hipStream_t stream) {
     const long long waves = (long long)((a.rows + 15) / 16) * (a.n / 128);
     // few rows: the siblings in parallel; else one read of x for all of them
     a.subs_per_wave = waves * a.n_sub <= 4096 ? 1 : a.n_sub;
     const long long grid = (waves + 3) / 4, gy = (a.n_sub + a.subs_per_wave - 1) / a.subs_per_wave;
-    if (grid > 0x7FFFFFFFLL || gy > 65535) return EXL3_E_BAD_SHAPE;
+    if (grid + (sort ? kSortMaxGroups : 0) > 0x7FFFFFFFLL || gy > 65535) return EXL3_E_BAD_SHAPE;
     // Past the L2 from 8 MB of results on: whole layers of 77 rows x 3 x 5120 (2.4 MB) and 754 x 2304 (3.5 MB) are 0.5 %
     // slower that way, 333 x 17408 (11.6 MB) 1 % faster, the experts of 1537 tokens (113 MB) 0.6 to 1.7 %. Not
     // for more rows than the rows kernels take: the GEMM, which the matrix pipe's clock bounds, gives the time
     // back (2048 x 5120 -> 34816 0.2 % slower).
-    const bool stream_results = (a.pair || a.rows <= kLinearRowsMaxRows) &&
+    const bool stream_results = (a.pair_expert || a.rows <= kLinearRowsMaxRows) &&
                                 (size_t)a.rows * a.n * a.n_sub * sizeof(half_t) >= (size_t)8 << 20;
-    auto kernel = stream_results ? had_pre_mfma_kernel<true> : had_pre_mfma_kernel<false>;
-    kernel<<<dim3((unsigned)grid, (unsigned)gy), dim3(256), 0, stream>>>(a);
+    if (!sort) {
+        auto kernel = stream_results ? had_pre_mfma_kernel<true> : had_pre_mfma_kernel<false>;
+        kernel<<<dim3((unsigned)grid, (unsigned)gy), dim3(256), 0, stream>>>(a);
+        return launch_status();
+    }
+    SortArgs so = *sort;
+    // a workgroup per 1024 pairs, up to kSortMaxGroups; in place of one alone for 2000 pairs two, where the
+    // rotation is as short as the sort: 400 tokens 62.3 -> 60.4 us, 273 tokens 59.1 -> 57.5
+    so.groups = std::min(kSortMaxGroups, (so.n_pairs + 1023) / 1024);
+    so.staged = so.groups == 1;
+    const size_t need = sort_lds_ints(kRotateThreads, so) * sizeof(int);
+    const size_t lds = stream_results ? std::max(need, kRotateTileBytes) : need;
+    auto kernel = stream_results ? moe_sort_rotate_kernel<true> : moe_sort_rotate_kernel<false>;
+    kernel<<<dim3((unsigned)(grid + so.groups), (unsigned)gy), dim3(kRotateThreads), lds, stream>>>(a, so);
     return launch_status();
 }
 
@@ -515,14 +547,14 @@ int launch_rotate_layer(const uint16_t* x, int rows, int n, const uint16_t* suh,
     a.n_sub = n_sub;
     a.sub_scale = a.sub_stride = (size_t)n;
     a.row_stride = (size_t)n_sub * n;
-    return launch_rotate(a, stream);
+    return launch_rotate(a, nullptr, stream);
 }
 
 // Rows sorted by expert: both rotations (gate and up signs of the row's expert, gu_suh
 // [E][2][n]) of row r = pair order[r], to xg[r] and, sub_stride halfs further, xu[r].
 int launch_had_pre_pairs(const uint16_t* x, int tokens, int top_k, int n, const int32_t* order,
                          const int32_t* indices, const uint16_t* gu_suh, int n_experts, uint16_t* xg,
-                         size_t sub_stride, hipStream_t stream) {
+                         size_t sub_stride, const SortArgs* sort, hipStream_t stream) {
     if (!aligned16(x) || !aligned16(gu_suh) || !aligned16(xg) || sub_stride % 8) return EXL3_E_BAD_SHAPE;
     RotateArgs a{};
     a.x = reinterpret_cast<const half_t*>(x);
@@ -540,7 +572,7 @@ int launch_had_pre_pairs(const uint16_t* x, int tokens, int top_k, int n, const 
     a.n_tokens = tokens;
     a.n_experts = n_experts;
     a.scale_ld = (size_t)2 * n;
-    return launch_rotate(a, stream);
+    return launch_rotate(a, sort, stream);
 }
 
 }  // namespace exl3

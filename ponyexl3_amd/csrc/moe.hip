@@ -32,6 +32,7 @@
 #include "exl3_device.hpp"
 #include "exl3_host.hpp"
 #include "exl3_glu.hpp"
+#include "exl3_sort.hpp"
 #include "exl3_groups.hpp"
 #include "exl3_route.hpp"
 #include "exl3_small.hpp"
@@ -43,10 +44,6 @@
 #pragma clang fp contract(off)
 
 namespace exl3 {
-
-// Routing indices come from the caller's device memory; an out-of-range value is
-// clamped so that it can never turn into an out-of-bounds read.
-__device__ __forceinline__ int clamp_expert(int e, int E) { return e < 0 ? 0 : (e >= E ? E - 1 : e); }
 
 // xh_gu[s][p][:] = fp16(had(x[t] * gu_suh[e][p])); also fills the group tables:
 //   gate/up GEMV group (s, p, hg): sub = 2s+p, tile = (p*E + e)*(H/16) + 8*hg
@@ -848,155 +845,10 @@ static MoeWorkspace moe_workspace(int tokens, int top_k, int D, int H) {
 // small: tokens * top_k), and finish gate/up + GLU + down rotation per sorted row.
 
 constexpr int kSortThreads = 1024;
-constexpr int kSortMaxExperts = 1024;
-constexpr int kSortMaxGroups = 32;
 
-// Stable counting sort by expert id. Outputs, all indexed by sorted position:
-//   order[pos] = pair index (token * top_k + slot), tok[pos] = token,
-//   sidx[pos] = expert (tok and sidx may be NULL); table[b] = {expert, first row, end row of
-//   the expert, 0} for every block of block_rows rows, unused entries {E-1, N, N, 0} (empty).
-// With `staged` the order is put together in LDS and written out in order: one CU's scattered
-// 4-byte stores (64 lines per instruction) are what this kernel is otherwise bound by.
-//
-// Every workgroup owns a contiguous part of the pairs, each of its 16 waves a segment of that and a
-// cursor per expert in LDS: count, one scan over (expert, wave), then every wave places its segment 64
-// pairs at a time without meeting the others. A pair's rank among equal experts of its 64 comes from
-// ballots over the bits of the expert id. Where a part begins is known without an exchange:
-// every workgroup counts all pairs, those before and behind its own part in two counters per expert (13 833
-// pairs: 14 loads and LDS additions per lane). There one workgroup takes 21.5 us, 14 take 8.3; 6972 pairs
-// 12.3 and 7.3.
-__host__ __device__ constexpr int sort_pairs_per_wave(int n_pairs, int groups) {
-    const long long waves = (long long)groups * (kSortThreads / 64);
-    return (int)((n_pairs + 64 * waves - 1) / (64 * waves) * 64);
-}
-
-__global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
-    const int* __restrict__ indices, int n_pairs, int top_k, int E, int block_rows,
-    int* __restrict__ order, int* __restrict__ tok, int* __restrict__ sidx,
-    int4* __restrict__ table, int table_len, int staged) {
-    constexpr int kWaves = kSortThreads / 64;
-    extern __shared__ int cursor[];  // [kWaves][E], pairs before [E], behind [E], staging
-    __shared__ int scan_tmp[2][kWaves];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int* const before = cursor + kWaves * E;
-    int* const behind = before + E;
-    int* const stage = behind + E;
-    for (int i = tid; i < (kWaves + 2) * E; i += kSortThreads) cursor[i] = 0;
-    __syncthreads();
-    const int groups = gridDim.x;
-    const int per_wave = sort_pairs_per_wave(n_pairs, groups);
-    const int part = blockIdx.x * kWaves * per_wave;
-    const int begin = min(part + wave * per_wave, n_pairs), end = min(begin + per_wave, n_pairs);
-    int* mine = cursor + wave * E;
-    // eight loads in flight
-    for (int i0 = begin + lane; groups == 1 && i0 < end; i0 += 8 * 64) {
-        int e[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) e[j] = indices[min(i0 + j * 64, n_pairs - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (i0 + j * 64 < end) atomicAdd(&mine[clamp_expert(e[j], E)], 1);
-    }
-    for (int i0 = wave * 64; groups > 1 && i0 < n_pairs; i0 += 8 * kSortThreads) {
-        int e[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) e[j] = indices[min(i0 + j * kSortThreads + lane, n_pairs - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int i = i0 + j * kSortThreads;  // 64 pairs of one segment
-            int* const count = i < part ? before
-                               : i >= part + kWaves * per_wave ? behind : cursor + (i - part) / per_wave * E;
-            if (i + lane < n_pairs) atomicAdd(&count[clamp_expert(e[j], E)], 1);
-        }
-    }
-    __syncthreads();
-
-    // exclusive scans over the experts (E <= 1024 = one value per thread): rows and blocks
-    int c = 0;
-    if (tid < E) {
-#pragma unroll
-        for (int w = 0; w < kWaves + 2; w++) c += cursor[w * E + tid];
-    }
-    const int nb = (c + block_rows - 1) / block_rows;
-    int inc_rows = c, inc_blk = nb;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int r = __shfl_up(inc_rows, off, kWave), b = __shfl_up(inc_blk, off, kWave);
-        if (lane >= off) {
-            inc_rows += r;
-            inc_blk += b;
-        }
-    }
-    if (lane == 63) {
-        scan_tmp[0][wave] = inc_rows;
-        scan_tmp[1][wave] = inc_blk;
-    }
-    __syncthreads();
-    int base_rows = 0, base_blk = 0, total_blk = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-        if (w < wave) {
-            base_rows += scan_tmp[0][w];
-            base_blk += scan_tmp[1][w];
-        }
-        total_blk += scan_tmp[1][w];
-    }
-    const int row0 = base_rows + inc_rows - c;  // first sorted row of expert tid
-    const int blk0 = base_blk + inc_blk - nb;
-    if (tid < E) {
-        int at = row0 + before[tid];
-#pragma unroll
-        for (int w = 0; w < kWaves; w++) {
-            const int n = cursor[w * E + tid];
-            cursor[w * E + tid] = at;
-            at += n;
-        }
-        if (blockIdx.x == 0)
-            for (int b = 0; b < nb && blk0 + b < table_len; b++)
-                table[blk0 + b] = int4{tid, row0 + b * block_rows, row0 + c, 0};
-    }
-    for (int b = total_blk + tid + blockIdx.x * kSortThreads; b < table_len; b += kSortThreads * groups)
-        table[b] = int4{E - 1, n_pairs, n_pairs, 0};
-    __syncthreads();
-
-    int ebits = 0;
-    while ((1 << ebits) < E) ebits++;
-    for (int i0 = begin; i0 < end; i0 += 8 * 64) {
-        int ids[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) ids[j] = indices[min(i0 + j * 64 + lane, n_pairs - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int i = i0 + j * 64 + lane;
-            const bool valid = i < end;
-            const int e = valid ? clamp_expert(ids[j], E) : 0;
-            unsigned long long same = __ballot(valid);
-            if (!same) break;
-            for (int b = 0; b < ebits; b++) {
-                const unsigned long long m = __ballot((e >> b) & 1);
-                same &= ((e >> b) & 1) ? m : ~m;
-            }
-            const int rank = __popcll(same & ((1ull << lane) - 1ull));
-            // every lane reads its expert's cursor before the first of the equal ones moves it,
-            // and the next 64 pairs read behind that (e is 0 where there is no pair)
-            const int first = mine[e];
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (valid && rank == 0) mine[e] = first + __popcll(same);
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (valid) {
-                const int pos = first + rank;
-                if (staged) stage[pos] = i;
-                else order[pos] = i;
-                if (tok) tok[pos] = i / top_k;
-                if (sidx) sidx[pos] = e;
-            }
-        }
-    }
-    if (!staged) return;
-    __syncthreads();
-    for (int i = tid; i < n_pairs; i += kSortThreads) order[i] = stage[i];
+__global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(SortArgs a) {
+    extern __shared__ int cursor[];
+    sort_pairs<kSortThreads>(a, blockIdx.x, cursor);
 }
 
 // One wave per (sorted row, 128-block of H): post-Hadamard + svh of the gate and up
@@ -1037,22 +889,17 @@ __global__ __launch_bounds__(256) void moe_glu_rows_kernel(
     *reinterpret_cast<half2_t*>(xh_dn + off) = o;
 }
 
-static int launch_moe_sort(const int32_t* indices, int n_pairs, int top_k, int n_experts, int block_rows,
-                           int32_t* order, int32_t* tok, int32_t* sidx, int32_t* table, int table_len,
-                           hipStream_t stream) {
-    size_t lds = (size_t)(kSortThreads / 64 + 2) * n_experts * sizeof(int);
+static int launch_moe_sort(SortArgs a, hipStream_t stream) {
     // a workgroup per kSortThreads pairs (64 to a wave), up to kSortMaxGroups, from the size on where
     // one alone takes longer (1025 pairs 5.6 and 6.4 us, 2436 7.3 and 6.7)
-    const int groups =
-        n_pairs <= 2 * kSortThreads ? 1 : std::min(kSortMaxGroups, (n_pairs + kSortThreads - 1) / kSortThreads);
-    const bool staged = groups == 1 && lds + (size_t)n_pairs * sizeof(int) <= (size_t)150 << 10;
-    if (staged) lds += (size_t)n_pairs * sizeof(int);
+    a.groups = a.n_pairs <= 2 * kSortThreads ? 1 : std::min(kSortMaxGroups, (a.n_pairs + kSortThreads - 1) / kSortThreads);
+    a.staged = 1;
+    a.staged = a.groups == 1 && sort_lds_ints(kSortThreads, a) * sizeof(int) <= (size_t)150 << 10;
+    const size_t lds = sort_lds_ints(kSortThreads, a) * sizeof(int);
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(moe_sort_kernel),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return EXL3_E_LAUNCH;
-    moe_sort_kernel<<<dim3((unsigned)groups), dim3(kSortThreads), lds, stream>>>(indices, n_pairs, top_k, n_experts, block_rows,
-                                                                  order, tok, sidx, reinterpret_cast<int4*>(table),
-                                                                  table_len, staged);
+    moe_sort_kernel<<<dim3((unsigned)a.groups), dim3(kSortThreads), lds, stream>>>(a);
     return launch_status();
 }
 
@@ -1318,7 +1165,8 @@ EXL3_EXPORT int exl3_moe_sort(const int32_t* indices, int n_pairs, int top_k, in
         return EXL3_E_BAD_SHAPE;
     if (n_experts > kSortMaxExperts) return EXL3_E_UNSUPPORTED;
     if (reinterpret_cast<uintptr_t>(table) & 15) return EXL3_E_BAD_SHAPE;
-    return launch_moe_sort(indices, n_pairs, top_k, n_experts, block_rows, order, tok, sidx, table, table_len,
+    return launch_moe_sort({indices, n_pairs, top_k, n_experts, block_rows, order, tok, sidx,
+                            reinterpret_cast<int4*>(table), table_len, 1, 0},
                            as_stream(stream));
 }
 
@@ -1390,13 +1238,19 @@ EXL3_EXPORT int exl3_moe_prefill(const uint16_t* x, int tokens, const int32_t* i
     uint16_t* xd = reinterpret_cast<uint16_t*>(base + w.o_xd);
     const size_t xu_offset = (w.o_xu - w.o_xg) / 2;
     hipStream_t s = as_stream(stream);
-    if (int rc = launch_moe_sort(indices, N, top_k, E, w.block_rows, order, nullptr, nullptr, table, w.table_len, s))
+    const SortArgs sort{indices, N, top_k, E, w.block_rows, order, nullptr, nullptr, reinterpret_cast<int4*>(table), w.table_len, 1, 0};
+    // The rotated rows stay in the order of the pairs, which one launch then rotates and sorts, and gate/up gathers
+    // them, at 32-bit offsets; beyond those they are put in sorted order, and the sort comes first.
+    const bool gather = (unsigned long long)N * D * 2 <= 0xFFFFFFFFull;
+    if (!gather)
+        if (int rc = launch_moe_sort(sort, s)) return rc;
+    if (int rc = launch_had_pre_pairs(x, tokens, top_k, D, gather ? nullptr : order, indices, gu_suh, E, xg, xu_offset,
+                                      gather ? &sort : nullptr, s))
         return rc;
-    if (int rc = launch_had_pre_pairs(x, tokens, top_k, D, order, indices, gu_suh, E, xg, xu_offset, s)) return rc;
     // gate, up, GLU and rotation, then down with its output transform, back in pair order
     uint16_t* slots = scores ? xg : y;
     if (int rc = launch_moe_rows(xg, xg + xu_offset, N, gu_trellis, gu_svh, dn_trellis, dn_suh, dn_svh, E, D, H, K, cb,
-                                 activation, table, w.table_len, w.block_rows, order, xd, slots, s))
+                                 activation, table, w.table_len, w.block_rows, order, gather, xd, slots, s))
         return rc;
     return scores ? exl3_moe_combine(slots, scores, tokens, top_k, D, y, stream) : EXL3_OK;
 }

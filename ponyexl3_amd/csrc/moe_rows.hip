@@ -65,12 +65,14 @@ __device__ __forceinline__ void rows_to_tile(float16_t (&acc)[MR][2], void* ex, 
 
 // grid: unit = (row block b, 128-column block hg of H), dealt so that the units of a row block
 // land on one XCD (they read the same activations): b = 8 (u / (8 hblocks)) + u % 8.
-// table[b] = {expert, first row, end row of the expert, 0}, empty if first >= end.
+// table[b] = {expert, first row, end row of the expert, 0}, empty if first >= end. gather: row r of xg and xu is
+// at gather[r] (or at r).
 template <int K, int CB, int MR, int NKS>
 __global__ __launch_bounds__(256 * NKS, 4) void moe_gateup_rows_kernel(
     const uint32_t* __restrict__ trellis, const half_t* __restrict__ xg, const half_t* __restrict__ xu,
     const int4* __restrict__ table, int n_blocks, const half_t* __restrict__ gu_svh,
-    const half_t* __restrict__ dn_suh, half_t* __restrict__ xd, int n_rows, int E, int D, int H, int activation) {
+    const half_t* __restrict__ dn_suh, const int* __restrict__ gather, half_t* __restrict__ xd, int n_rows, int E, int D,
+    int H, int activation) {
     using T = RowsTile<MR, NKS>;
     constexpr int kFillWaves = 2 * NKS, LPW = T::FILLS / kFillWaves;
     constexpr int kParts = 2 * MR / NKS;  // of a wave, of the four 32-column parts of a row tile
@@ -94,12 +96,14 @@ __global__ __launch_bounds__(256 * NKS, 4) void moe_gateup_rows_kernel(
     half_t* stages = reinterpret_cast<half_t*>(lds) + proj * 3 * T::STAGE;
     uint32_t a_off[LPW];
 #pragma unroll
-    for (int i = 0; i < LPW; i++) a_off[i] = rows_fill_offset<MR, NKS>(wave % kFillWaves * LPW + i, lane, valid - 1, D);
+    for (int i = 0; i < LPW; i++) 
+        a_off[i] = rows_fill_offset<MR, NKS>(wave % kFillWaves * LPW + i, lane, valid - 1, D,
+                                             [&](int row) { return gather ? gather[m0 + row] : row; });
     float16_t acc[MR][2];
     uint32_t* words = reinterpret_cast<uint32_t*>(reinterpret_cast<half_t*>(lds) + 2 * 3 * T::STAGE) +
                       wave * RowsWords<K>::STAGE;
     rows_main<K, CB, MR, NKS, LPW>(w, row_words, 2 * NKS * row_words,
-                                   reinterpret_cast<const char*>((proj ? xu : xg) + (size_t)m0 * D), a_off, true,
+                                   reinterpret_cast<const char*>((proj ? xu : xg) + (gather ? 0 : (size_t)m0 * D)), a_off, true,
                                    lds_byte_address(stages) + wave % kFillWaves * LPW * 1024, stages,
                                    rows_read_base<MR, NKS>(ks, lane), words, 4 * NKS * RowsWords<K>::STAGE,
                                    D / (32 * NKS), lane, acc);
@@ -311,7 +315,7 @@ constexpr size_t kLdsBytes = (size_t)160 << 10;
 int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const uint16_t* gu_trellis,
                     const uint16_t* gu_svh, const uint16_t* dn_trellis, const uint16_t* dn_suh,
                     const uint16_t* dn_svh, int E, int D, int H, int K, int cb, int activation,
-                    const int32_t* table, int n_blocks, int block_rows, const int32_t* order, uint16_t* xd,
+                    const int32_t* table, int n_blocks, int block_rows, const int32_t* order, bool gather, uint16_t* xd,
                     uint16_t* out, hipStream_t stream) {
     const long long sets = (n_blocks + 7) / 8;
     const long long gu_grid = sets * 8 * (H / 128), dn_grid = sets * 8 * ((D + 255) / 256);
@@ -330,7 +334,7 @@ int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const ui
                 return (int)EXL3_E_LAUNCH;
             gu<<<dim3((unsigned)gu_grid), dim3(256 * GN), gu_lds, stream>>>(
                 reinterpret_cast<const uint32_t*>(gu_trellis), H_(xg), H_(xu), reinterpret_cast<const int4*>(table),
-                n_blocks, H_(gu_svh), H_(dn_suh), reinterpret_cast<half_t*>(xd), n_rows, E, D, H, activation);
+                n_blocks, H_(gu_svh), H_(dn_suh), gather ? order : nullptr, reinterpret_cast<half_t*>(xd), n_rows, E, D, H, activation);
             if (int rc = launch_status()) return rc;
             dn<<<dim3((unsigned)dn_grid), dim3(256 * DN), dn_lds, stream>>>(
                 reinterpret_cast<const uint32_t*>(dn_trellis), H_(xd), reinterpret_cast<const int4*>(table), n_blocks,

@@ -6,8 +6,6 @@ router / weighted sum of ``EXL3MoEBlock`` (ponyexl3/mlx/exl3_moe.py:790-839).
 
 from __future__ import annotations
 
-import math
-
 import numpy as np
 import torch
 from torch.nn.modules.module import (_global_backward_hooks, _global_backward_pre_hooks, _global_forward_hooks,
@@ -99,39 +97,26 @@ class EXL3SwitchGLU(torch.nn.Module):
     # The sorted, segmented prefill path replaces the slot kernels once the experts see
     # a few rows each (the reference switches at 9 tokens,
     # ponyexl3/mlx/exl3_moe.py:770-787). The slot kernels share one pass over an expert's
-    # weights among up to four of its slots as long as the call has at most 1024 slots; above
-    # that every slot is on its own. From 24 tokens on, and 512 slots or 2.5 per expert, the two are close: both
-    # grow with passes over an expert's weights, groups of four slots here, blocks of 32 rows and the rows
-    # themselves there, whose sort, rotation and combination cost more to begin with. us for experts of 2^20 weights
-    # a projection, routing taken as even, by bits per weight: (fixed, per group) and (fixed, per block, per slot),
-    # fitted to 129 calls of 10 to 163 tokens (4 to 5 us rms). Taken only 7 % below the prefill's: of 43 calls of
-    # those sizes none then ends on the slower path by more than 0.5 %, and they take 7 % less than through the prefill.
-    # Measured, slot kernels and prefill: 256 experts of 2048 x 512, top-8 and a shared one, K = 4: 142 and
-    # 169 at 56 tokens, 167 and 177 at 80, 187 and 179 at 100; 64 of 1152 x 256, top-8: 41 and 54 at 40; 128 of
-    # 1280 x 768, top-4 and a shared one, K = 5: 123 and 108 at 89.
+    # weights among up to four of its slots; the prefill, with a rotation and a combination of its own, costs some 14 us more
+    # to begin with and less for every pass and slot. From 24 tokens on, and 512 slots or 2.5 per expert, it
+    # therefore depends on the work: up to 150 slots' worth of experts of 2^20 weights per projection, with
+    # at most 6 slots per expert, the slot kernels are the faster ones. Of 78 calls of those sizes none takes longer than
+    # through the prefill, and they take 2.7 % less; the better choice each time would be 1 % less again. us, slot
+    # kernels and prefill: 32 tokens, top-4 of 32 experts of 1792 x 256 35 and 48; 28 of 64 of 1536 x 512, top-6 and a
+    # shared one 63 and 69; 64 of 64 of 1664 x 512, top-4 and a shared one 76 and 76; 120 of 128 of
+    # 1408 x 512, top-3 92 and 88; 107 of 128 of 1152 x 768, top-5 and a shared one 157 and 120.
     prefill_min_tokens = 24
     prefill_min_rows_per_expert = 2.5
     grouped_max_slots = 512
-    _grouped_slots_limit = 1024
-    _grouped_us = ((30.5, 0.42), (28, 0.50), (28, 0.50), (26.4, 0.573), (24.5, 0.606), (23.4, 0.686), (27.8, 0.711))
-    _prefill_us = ((42, 0.51, 0.0), (42, 0.51, 0.019), (42, 0.51, 0.019), (43.4, 0.569, 0.008), (40.2, 0.608, 0.013),
-                   (40.4, 0.568, 0.039), (46.2, 0.586, 0.014))  # K = 2 (and 1) to 8
+    grouped_max_work = 150 << 20
 
     def _use_prefill(self, tokens: int, top_k: int) -> bool:
         slots = tokens * top_k
         if tokens < self.prefill_min_tokens or (
                 slots <= self.grouped_max_slots and slots < self.prefill_min_rows_per_expert * self.num_experts):
             return False
-        rows = slots / self.num_experts
-        # (beyond what was fitted; most slots on their own)
-        if slots > self._grouped_slots_limit or rows > 6 or (slots > self.grouped_max_slots and rows < 1):
-            return True
-        size = self.input_dims * self.hidden_dims / 2**20
-        fixed, group = self._grouped_us[max(self._k, 2) - 2]
-        grouped = fixed + size * group * self.num_experts * (rows / 4 + 0.375 * (1 - math.exp(-2 * rows)))
-        fixed, block, slot = self._prefill_us[max(self._k, 2) - 2]
-        prefill = fixed + size * (block * self.num_experts * (1 - math.exp(-rows)) + slot * slots)
-        return grouped > 0.93 * prefill
+        return (slots > self.grouped_max_slots or slots > 6 * self.num_experts
+                or slots * self.input_dims * self.hidden_dims > self.grouped_max_work)
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         if indices.dim() != 3:

@@ -455,6 +455,76 @@ def test_pair_sort_kernel_equals_stable_argsort(cuda, tokens, top_k, E, block_ro
     assert torch.equal(o2, order) and torch.equal(tab2, table)
 
 
+@pytest.mark.parametrize("tokens,kk,E", [(1, 1, 1), (9, 7, 3), (16, 4, 65), (65, 1, 1024), (512, 2, 7), (205, 5, 600),
+                                         (683, 3, 64), (4100, 8, 257), (4097, 8, 1024)])
+def test_prefill_sorts_as_the_sort_kernel(cuda, tokens, kk, E):
+    """The prefill chain sorts in the launch that rotates, 256 threads to a workgroup and one per 1024 pairs: order and
+    row-block table, at the front of its workspace, are those of the sort by itself (whole numbers, equal), clamped ids and
+    experts without pairs included."""
+    from ponyexl3_amd import _lib, ops
+
+    lib, p = _lib.load(), ops._ptr
+    D, H, K, n = 128, 128, 2, tokens * kk
+    rng = np.random.default_rng(n + E)
+    idx = rng.integers(0, E, size=(tokens, kk)).astype(np.int32)
+    if E > 4:
+        idx[idx == 3] = 2
+        idx[0, 0] = E + 5
+        idx[-1, -1] = -4
+    idx = torch.from_numpy(idx).to(cuda)
+    bits = lambda *s: torch.randint(-32768, 32768, s, dtype=torch.int16, device=cuda)
+    ones = lambda *s: torch.ones(s, dtype=torch.float16, device=cuda)
+    x = torch.randn((tokens, D), device=cuda).half() * 0.1
+    need = lib.exl3_moe_prefill_workspace_bytes(tokens, kk, E, D, H)
+    ws = torch.full((need,), 0xCC, dtype=torch.uint8, device=cuda)
+    y = torch.empty((tokens, kk, D), dtype=torch.float16, device=cuda)
+    w = [bits(D // 16, 2 * E * H // 16, 16 * K), ones(E, 2, D), ones(E, 2, H), bits(H // 16, E * D // 16, 16 * K), ones(E, H),
+         ones(E, D)]
+    print(f"prefill sort tokens={tokens} kk={kk} E={E}", flush=True)
+    _lib.check(lib.exl3_moe_prefill(p(x), tokens, p(idx), kk, *map(p, w), E, D, H, K, 0, 0, None, p(y), p(ws), need,
+                                    ops._stream()), "exl3_moe_prefill")
+    block_rows = 32 if n <= 24 * E else 64
+    order, _, _, table = ops.moe_sort(idx, E, block_rows)
+    assert torch.equal(ws[:4 * n].view(torch.int32), order)
+    at = (4 * n + 255) // 256 * 256
+    assert torch.equal(ws[at:at + 16 * table.shape[0]].view(torch.int32).view(-1, 4), table.view(-1, 4))
+
+
+def test_prefill_past_32_bit_offsets(cuda):
+    """From 4 GiB of rotated rows on they are put in sorted order, behind a sort of its own, instead of gathered: the
+    last tokens' rows are those of a call on them alone, up to the order of the sums (the row blocks differ)."""
+    from ponyexl3_amd import _lib, ops
+
+    if torch.cuda.mem_get_info()[0] < 40 << 30:
+        pytest.skip("needs 40 GB of memory")
+    lib, p = _lib.load(), ops._ptr
+    tokens, kk, E, D, H, K = 32800, 4, 8, 16384, 128, 2
+    assert tokens * kk * D * 2 > 0xFFFFFFFF
+    g = torch.Generator(device=cuda).manual_seed(5)
+    bits = lambda *s: torch.randint(-32768, 32768, s, dtype=torch.int16, device=cuda, generator=g)
+    sign = lambda size, *s: ((torch.randint(0, 2, s, device=cuda, generator=g) * 2.0 - 1.0) * size).half()
+    w = [bits(D // 16, 2 * E * H // 16, 16 * K), sign(1, E, 2, D), sign(D**-0.5, E, 2, H), bits(H // 16, E * D // 16, 16 * K),
+         sign(1, E, H), sign(H**-0.5, E, D)]
+    x = torch.randn((tokens, D), device=cuda, generator=g, dtype=torch.float16) * 0.5
+    idx = torch.rand((tokens, E), device=cuda, generator=g).topk(kk, dim=1).indices.int().contiguous()
+
+    def run(xs, ids):
+        t = xs.shape[0]
+        need = lib.exl3_moe_prefill_workspace_bytes(t, kk, E, D, H)
+        ws = torch.empty((need,), dtype=torch.uint8, device=cuda)
+        y = torch.full((t, kk, D), float("nan"), dtype=torch.float16, device=cuda)
+        _lib.check(lib.exl3_moe_prefill(p(xs), t, p(ids), kk, *map(p, w), E, D, H, K, 0, 0, None, p(y), p(ws), need,
+                                        ops._stream()), "exl3_moe_prefill")
+        return y
+
+    print("prefill past 32-bit offsets", flush=True)
+    got = run(x, idx)
+    for part in (slice(0, 100), slice(tokens - 100, tokens)):
+        ref = run(x[part].contiguous(), idx[part].contiguous())
+        assert rel_l2(got[part].float().cpu().numpy(), ref.float().cpu().numpy()) <= TOL
+    assert bool(torch.isfinite(got).all())
+
+
 @pytest.mark.parametrize("tokens,k", [(40, 4), (200, 8)])  # row blocks of 32 and of 64
 @pytest.mark.parametrize("kind", ["general", "spikes", "small"])
 def test_prefill_rotation_with_general_scales(cuda, tokens, k, kind):
