@@ -307,8 +307,11 @@ static constexpr size_t rows_lds_bytes(int tiles, int tile_cols) {
 //   276.1); below 1.1 us less to 2.1 us more;
 // gate/up, where LDS holds one workgroup of eight waves on a CU (64 rows, K >= 6), from 400 units on:
 //   1000 tokens K = 6 312.1 -> 275.6, 820 tokens through 64 experts K = 7 137.7 -> 132.5, none slower;
-//   264 units 80.6 -> 84.9. Where it holds two, 8 us more to 7 us less.
-constexpr long long kDownNarrowUnits = 800, kGateUpNarrowUnits = 400;
+//   264 units 80.6 -> 84.9;
+// gate/up, where it holds two, from 1300 units on: 1.3 % less of whole calls (1600 tokens, top-8 of 128 experts of
+//   1152 x 768 271 -> 263, 1536 of 256 of 1024 x 384 146 -> 141; two of 13 slower, 219 -> 223 at most); below, 4 to 14 % more
+//   up to 400 units and 2 % less to 2 % more on from there (1104 units 148 -> 145, 1152 158 -> 162).
+constexpr long long kDownNarrowUnits = 800, kGateUpNarrowUnits = 400, kGateUpManyUnits = 1300;
 constexpr size_t kLdsBytes = (size_t)160 << 10;
 
 // block_rows: 32 or 64
@@ -345,8 +348,9 @@ int launch_moe_rows(const uint16_t* xg, const uint16_t* xu, int n_rows, const ui
         using N2 = std::integral_constant<int, 2>;
         const bool many_dn = dn_grid >= kDownNarrowUnits;
         if (block_rows == 32) return many_dn ? go(N1{}, N2{}, N1{}) : go(N1{}, N2{}, N2{});
-        if constexpr (2 * rows_lds_bytes<k.value, 2, 2>(2, 128) > kLdsBytes)
-            if (gu_grid >= kGateUpNarrowUnits) return many_dn ? go(N2{}, N1{}, N1{}) : go(N2{}, N1{}, N2{});
+        constexpr bool one_per_cu = 2 * rows_lds_bytes<k.value, 2, 2>(2, 128) > kLdsBytes;
+        if (gu_grid >= (one_per_cu ? kGateUpNarrowUnits : kGateUpManyUnits))
+            return many_dn ? go(N2{}, N1{}, N1{}) : go(N2{}, N1{}, N2{});
         return many_dn ? go(N2{}, N2{}, N1{}) : go(N2{}, N2{}, N2{});
     });
 }

@@ -225,6 +225,7 @@ def test_prefill_path_matches_oracle_and_slot_kernels(cuda, oracle, tokens, act)
     (40, 300, 3, 640, 128, 3, 2, 0, False),    # down in four waves, 32 rows; a last block of 128 columns
     (590, 170, 8, 1152, 256, 6, 0, 1, True),   # both, 64 rows, blocks of one row and of 64; scales other than +-1
     (300, 32, 8, 1024, 768, 8, 1, 0, False),   # gate/up in four waves, down in eight
+    (590, 170, 8, 640, 768, 4, 0, 0, False),   # both, with LDS for two of eight waves
 ])
 def test_prefill_workgroups_of_four_waves(cuda, tokens, E, kk, D, H, K, cb, act, general):
     """The prefill kernels at as many row blocks as they take in workgroups of four waves, against the slot
