@@ -782,6 +782,13 @@ static bool moe_group_slots() {
     return v != 0;
 }
 
+// Calls of a size that the sorted prefill kernels also serve get the rounded weights of those in the down
+// projection too, so that the result is no further from the reference's arithmetic whichever is faster
+// (7.1e-4 of the output with unsummed halves, 6.8e-4 with rounded weights, against 64 bits).
+static bool moe_exact_down(int tokens, int slots, int num_experts) {
+    return tokens >= 24 && (slots > 512 || slots >= 2.5 * num_experts);
+}
+
 // Whether the slots are grouped by expert: where that is expected to spare enough passes over an expert's
 // weights to pay for the list and for reducing through partial rows, a fifth of the slots and
 // 18 of them (router choices taken as independent and even; a shared expert has all tokens). us,
@@ -791,20 +798,15 @@ static bool moe_group_slots() {
 // tokens, 74 of 216 97 (the table searched by every wave) -> 89; 19 tokens, 128 of 2048 x 512, K = 2 49 of 133 99 -> 76.
 // Of 64 calls of 3 to 22 tokens with 8 to 40 % spared two on the grouped side (20 and 22 of 55 and 63, experts of
 // 1664 x 256 and 1408 x 512) are 4 and 6 % above the other; six on the single side 8 to 14 % (large experts,
-// 7 to 18 spared).
+// 7 to 18 spared). Calls that are to have rounded weights in the down projection, which the grouped kernel has, are
+// grouped where fewer are spared, too (24 slots of 8 experts: 16).
 static bool moe_groups_apply(int tokens, int top_k, int num_experts, bool shared) {
     const long long slots = (long long)tokens * top_k;
     if (tokens < 2 || slots > kGroupMaxSlots || num_experts > kGroupMaxExperts || !moe_group_slots()) return false;
     const double experts = num_experts - (shared && num_experts > 1), chosen = top_k - shared;
     const double passes = experts * (1.0 - std::pow(1.0 - std::min(1.0, chosen / experts), tokens)) + (shared ? (tokens + 3) / 4 : 0);
-    return slots - passes >= std::max(18.0, 0.2 * slots);
-}
-
-// Calls of a size that the sorted prefill kernels also serve get the rounded weights of those in the down
-// projection too, so that the result is no further from the reference's arithmetic whichever is faster
-// (7.1e-4 of the output with unsummed halves, 6.8e-4 with rounded weights, against 64 bits).
-static bool moe_exact_down(int tokens, int slots, int num_experts) {
-    return tokens >= 24 && (slots > 512 || slots >= 2.5 * num_experts);
+    return slots - passes >= std::max(18.0, 0.2 * slots) ||
+           (moe_exact_down(tokens, (int)slots, num_experts) && slots >= 2.5 * num_experts);
 }
 
 // Gate/up launches that would issue more atomics than this reduce through partial rows
