@@ -117,11 +117,9 @@ constexpr int kLinearMidMaxRows = 32;
 // Up to 16 rows from K = 5 on, where a lane of the medium-batch kernel needs three dwords for its
 // eight codewords (16 rows: 17408 -> 5120 at K = 6 36.3 -> 28.7, 5120 -> 34816 at K = 7 59.8 -> 52.1,
 // 14336 -> 4096 at K = 8 30.1 -> 25.8), and where few column groups share a long reduction (8192 ->
-// 2048 at K = 4 17.3 -> 14.1, 4096 -> 1024 at K = 3 13.3 -> 11.7); else not (5120 -> 34816 at K = 4
-// 42.6 against 46.5, 2048 -> 8192 13.3 against 14.6).
-inline bool linear_rows_before_mid(int rows, int K, int in_tiles, int out_tiles) {
-    return rows > 16 || K >= 5 || in_tiles >= 2 * out_tiles;
-}
+// 2048 at K = 4 17.3 -> 14.1, 4096 -> 1024 at K = 3 13.3 -> 11.7); else by how evenly the two fill the chip, see
+// there (5120 -> 34816 at K = 4 stays: 41.0 against 46.5).
+bool linear_rows_before_mid(int rows, int K, int in_tiles, int out_tiles);
 struct MidPlan {
     int n_splits;          // workgroups per 128-column group
     int blocks_per_split;  // 128-row blocks of the reduction per workgroup

@@ -306,6 +306,27 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     return us < (cb == CB_MUL1 ? 0.92 : p.mr == 3 ? 1.0 : 0.9) * gemm_us;
 }
 
+// Up to 16 rows the rows kernel spends twice the matrix work and half the publishing of the medium-batch kernel, and
+// which one is faster hangs on how evenly each fills 256 CUs: the rows kernel with whole reductions as one
+// workgroup for every CU or two, nearly, or with few steps; with ranges where nearly two workgroups to a CU have 10 to 20 steps each
+// (30 below K = 4, where the decode is shorter) and the medium-batch kernel's workgroups leave 7 % and more
+// of their last round empty. Layer, medium-batch -> rows kernel, us: 15 rows of 1536 -> 64896 26.6 -> 21.7, 15 of 1024 -> 61568
+// 22.5 -> 17.3, 15 of 2560 -> 29440 24.3 -> 20.1, 14 of 9216 -> 5248 22.3 -> 19.0, 12 of 12288 -> 10368 34.6 -> 29.4. Beyond the lines: 11 rows of
+// 2560 -> 43008 (336 workgroups of 20 steps) 35.8 and 40.7, 10 of 8192 -> 21632 (507 of 22) 34.8 and 36.5, 14 of 4096 -> 19072 (447) 22.8
+// and 24.0, 12 of 7168 -> 12288 (768 medium-batch workgroups, three to a CU) 22.8
+// and 24.9. Over 245 layers of 9 to 16
+// rows 3.5 % less, none more than 2 % slower.
+bool linear_rows_before_mid(int rows, int K, int in_tiles, int out_tiles) {
+    if (rows > 16 || K >= 5 || in_tiles >= 2 * out_tiles) return true;
+    const int n_groups = out_tiles / 8;
+    const LinRowsPlan p = plan_linear_rows(rows, in_tiles, n_groups);
+    const long long n = rows_workgroups(p, n_groups);
+    if (n > 512) return false;
+    if (p.n_splits == 1) return n >= 430 || (n >= 340 && p.steps_per_split <= 14) || (n <= 256 && (n >= 200 || p.steps_per_split <= 16));
+    const int mid = n_groups * plan_linear_mid(rows, in_tiles, n_groups).n_splits, rounds = (mid + 255) / 256;
+    return n >= 450 && p.steps_per_split >= 10 && p.steps_per_split <= (K == 4 ? 20 : 30) && mid < 0.93 * 256 * rounds;
+}
+
 bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles) {
     for (int cb : {(int)CB_3INST, (int)CB_MUL1})
         for (int K = 8; K >= 4; K--)  // (below it the estimates are those of K = 4)
