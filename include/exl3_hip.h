@@ -377,8 +377,8 @@ int exl3_linear_forward_static(const uint16_t *x, int rows, const uint16_t *trel
  *               Two more ints than that make the last int the status word of
  *               exl3_counters_status.
  * Only the selected experts' trellis blocks are read. In the two-launch chain, with
- * 2 <= tokens, at most 1024 slots and 1024 experts, and where an even routing would spare a fifth
- * of the slots and 18 of them their own pass, the slots that route to one expert share a pass over
+ * 2 <= tokens, at most 1024 slots and 1024 experts, and where an even routing would spare 15 %
+ * of the slots and 15 of them their own pass, the slots that route to one expert share a pass over
  * its weights (four batch rows per pass; same arithmetic per row, bit-identical results; one small
  * launch more); EXL3_MOE_GROUP=0 switches that off. From 24 tokens on, with more than 512 slots or 2.5 per
  * expert, those calls round the down projection's weights to fp16 like the prefill chain.

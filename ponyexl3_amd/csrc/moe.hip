@@ -790,22 +790,21 @@ static bool moe_exact_down(int tokens, int slots, int num_experts) {
 }
 
 // Whether the slots are grouped by expert: where that is expected to spare enough passes over an expert's
-// weights to pay for the list and for reducing through partial rows, a fifth of the slots and
-// 18 of them (router choices taken as independent and even; a shared expert has all tokens). us,
-// every slot on its own -> grouped, passes spared of slots: 4 tokens through 192 experts of 1920 x 512, top-4 and a
-// shared one, K = 5 3.5 of 20 26.8 -> 30.6; 9 tokens, 192 of 1280 x 256, K = 6 10.4 of 54 27.6 -> 30.2; 13 tokens,
-// 192 of 2048 x 512, top-8, K = 5 22 of 104 64.7 -> 62.9; 13 tokens, 256 of 1664 x 512, K = 8 22 of 104 70.3 -> 64.9; 24
-// tokens, 74 of 216 97 (the table searched by every wave) -> 89; 19 tokens, 128 of 2048 x 512, K = 2 49 of 133 99 -> 76.
-// Of 64 calls of 3 to 22 tokens with 8 to 40 % spared two on the grouped side (20 and 22 of 55 and 63, experts of
-// 1664 x 256 and 1408 x 512) are 4 and 6 % above the other; six on the single side 8 to 14 % (large experts,
-// 7 to 18 spared). Calls that are to have rounded weights in the down projection, which the grouped kernel has, are
-// grouped where fewer are spared, too (24 slots of 8 experts: 16).
-static bool moe_groups_apply(int tokens, int top_k, int num_experts, bool shared) {
+// weights to pay for the list and for reducing through partial rows, 15 % of the slots and
+// 15 of them (choices taken as independent and even). From what every entry point knows, so that the block and its parts
+// take the same way: that one of the experts may be a shared one, which all tokens have, is not asked.
+// us, every slot on its own -> grouped, passes spared of slots: 11 tokens through 257 experts of 2048 x 512 with 9 slots a token, K = 4
+// 15.6 of 99 63.2 -> 59.6, 14 tokens 25 of 126 72.5 -> 67.1; 24, 68 of 216 97 -> 86; 17 tokens, 3 of 64 experts of 1024 x 768,
+// K = 5 15.3 of 51 38.3 -> 34.7; 10 tokens, 7 of 192 of 1280 x 768, K = 3 8.0 of 70 48.5 -> 51.0; 9 tokens, 8 of 256 of
+// 1024 x 384 8.4 of 72 30.7 -> 33.9. Of 90 calls of 2 to 26 tokens with 11 to 30 % spared the 46 on the grouped side
+// take 6 % less, four of them (few weights: 256 and 384 wide) 2 to 8 % more; of the 44 on the single side ten would
+// take 6 to 15 % less grouped (wide experts, MUL1), as many 5 to 11 % more. Calls that are to have rounded weights in the down
+// projection, which the grouped kernel has, are grouped where fewer are spared, too (24 slots of 8 experts: 16).
+static bool moe_groups_apply(int tokens, int top_k, int num_experts) {
     const long long slots = (long long)tokens * top_k;
     if (tokens < 2 || slots > kGroupMaxSlots || num_experts > kGroupMaxExperts || !moe_group_slots()) return false;
-    const double experts = num_experts - (shared && num_experts > 1), chosen = top_k - shared;
-    const double passes = experts * (1.0 - std::pow(1.0 - std::min(1.0, chosen / experts), tokens)) + (shared ? (tokens + 3) / 4 : 0);
-    return slots - passes >= std::max(18.0, 0.2 * slots) ||
+    const double passes = num_experts * (1.0 - std::pow(1.0 - std::min(1.0, (double)top_k / num_experts), tokens));
+    return slots - passes >= std::max(15.0, 0.15 * slots) ||
            (moe_exact_down(tokens, (int)slots, num_experts) && slots >= 2.5 * num_experts);
 }
 
@@ -981,7 +980,7 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
         // two launches: gate/up + GLU + rotation, then down
         const int hblocks = H / 128, dblocks = D / 128;
         if (counters_len < (size_t)slots * (hblocks + dblocks)) return EXL3_E_WORKSPACE;
-        const bool grouped = moe_groups_apply(tokens, top_k, num_experts, a.route.shared_logits != nullptr);
+        const bool grouped = moe_groups_apply(tokens, top_k, num_experts);
         const bool half = moe_half_blocks((long long)slots * 2 * hblocks * dblocks, grouped, K);
         // every slot on its own, few enough atomics, and counters large enough to hold
         // the accumulators (uint64 [slots][2][H], then the down launch's counters): gate

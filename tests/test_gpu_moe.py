@@ -917,6 +917,19 @@ def test_gate_kernel_against_float64(cuda, tokens, E, D, shared):
                                                 (40, 16, 256, 384, 4), (9, 32, 256, 128, 4)])
 @pytest.mark.parametrize("shared", [False, True])
 def test_decode_call_equals_its_parts(cuda, tokens, E, D, H, top_k, shared):
+    _decode_call_and_parts(cuda, tokens, E, D, H, top_k, shared, 4)
+
+
+# around the line between single and grouped slots, where that one expert of the table is a shared one (which only the one call
+# knows) must not choose the kernels: accumulators against partial rows, and from K = 5 on half blocks against whole ones
+@pytest.mark.parametrize("tokens,E,D,H,top_k,k", [(8, 64, 1024, 256, 6, 4), (8, 128, 640, 256, 8, 6), (10, 256, 1024, 256, 8, 6),
+                                                  (11, 256, 1024, 256, 8, 4), (12, 256, 1024, 256, 8, 6), (14, 256, 1024, 256, 8, 4),
+                                                  (13, 256, 1152, 512, 8, 8)])
+def test_decode_call_equals_its_parts_beside_the_grouping_line(cuda, tokens, E, D, H, top_k, k):
+    _decode_call_and_parts(cuda, tokens, E, D, H, top_k, True, k)
+
+
+def _decode_call_and_parts(cuda, tokens, E, D, H, top_k, shared, k):
     """exl3_moe_decode against exl3_moe_route, exl3_moe_forward and exl3_moe_combine, bit for bit, in every form
     of the slot kernels (accumulators with the routing inside, more experts than it ranks there, grouped slots,
     several partial rows of down), on coarse logits so that ties occur; twice, so that the counters
@@ -927,7 +940,7 @@ def test_decode_call_equals_its_parts(cuda, tokens, E, D, H, top_k, shared):
     g = torch.Generator(device=cuda).manual_seed(E + D + tokens)
     rnd = lambda *s: torch.randn(s, device=cuda, generator=g)
     n = E + shared
-    k, cb = 4, E % 2
+    cb = E % 2
     tr = lambda a, b: torch.randint(-32768, 32768, (a // 16, b // 16, 16 * k), dtype=torch.int16, device=cuda, generator=g)
     gu, dn = tr(D, n * 2 * H), tr(H, n * D)
     gu_suh, gu_svh = rnd(n, 2, D).sign().half(), (rnd(n, 2 * H).sign() / D ** 0.5).half()
