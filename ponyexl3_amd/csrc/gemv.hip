@@ -544,13 +544,20 @@ bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
 //   7168 -> 36864 K = 4 / 6: 37.7 -> 37.7, 47.2 -> 43.4; 2048 -> 65536 K = 4 / 6: 20.9 -> 21.1, 25.7 -> 24.0
 // Workgroups of four waves spread the work better still where they are few: up to K = 4 within the line of the whole
 // blocks (3072 -> 24576 K = 4 13.8 -> 12.9, eight waves 13.4; K = 6 15.9 and 15.7).
-// Not where that means more contributors to a sum than before and more than 31, whose words have fewer
-// fraction bits than fp32 partial rows are good for.
+// Only where the whole blocks meet in accumulators too, and in words of no more fraction bits: half blocks are twice
+// the contributors where whole ones come two to a wave (from K = 5 on) or eight waves to a workgroup, and past 15 of them a word has
+// 30 bits in place of 33 (11904 -> 14848 K = 6 stays at 35.3, half blocks 30.6; workgroups of sixteen waves, which
+// would keep the bits, take up to 13 % more than whole blocks where they are few or decode MUL1).
 static GemvPlan one_row_half_blocks(int in_tiles, int n_groups, int K, GemvPlan whole) {
-    GemvPlan half{in_tiles / 4, 4};
-    if (K > 4 || half.n_partials() > kFixFineContributors || !linear_small_uses_atomics(1, n_groups, half)) half.wg_waves = 8;
-    const bool fine = half.n_partials() <= std::max(kFixFineContributors, whole.n_partials());
-    return fine && linear_small_uses_atomics(1, n_groups, half) ? half : whole;
+    if (!linear_small_uses_atomics(1, n_groups, whole)) return whole;
+    for (const int waves : {4, 8}) {
+        if (waves == 4 && K > 4) continue;
+        const GemvPlan half{in_tiles / 4, 4, waves};
+        if (fix_count_bits(half.n_partials()) <= fix_count_bits(whole.n_partials()) &&
+            linear_small_uses_atomics(1, n_groups, half))
+            return half;
+    }
+    return whole;
 }
 
 GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K) {

@@ -19,14 +19,16 @@ def _plan(k, n_in, n_out):
     return tuple(v.value for v in out)  # splits, tile rows, waves, accumulators
 
 
-# (tile rows of a wave, waves of a workgroup) that the layer is to take: a last workgroup with waves to spare
-# (33 and 65 blocks), 31 partial rows and the first count beyond them, one block, eight and four waves
-@pytest.mark.parametrize("k,cb,n_in,n_out,tile_rows,waves", [
-    (4, 0, 4224, 24576, 4, 8), (6, 1, 8320, 8192, 4, 8), (8, 2, 15872, 4352, 4, 8), (5, 0, 17408, 5120, 16, 4),
-    (4, 0, 17408, 10240, 8, 8), (3, 1, 3072, 24576, 4, 4), (7, 0, 128, 524288, 4, 8), (2, 0, 1024, 65536, 4, 4)])
-def test_half_block_waves_of_a_full_chip(cuda, k, cb, n_in, n_out, tile_rows, waves):
+# (tile rows of a wave, waves of a workgroup, accumulators or partial rows) that the layer is to take: a last workgroup with
+# waves to spare (33 blocks), 15 contributors in half blocks and the first count beyond them, whose words would be coarser than those
+# of whole blocks, 31 where whole blocks have 16, two blocks, one block in partial rows, four waves up to 15 contributors and eight beyond
+@pytest.mark.parametrize("k,cb,n_in,n_out,tile_rows,waves,atomics", [
+    (4, 0, 4224, 24576, 4, 8, 1), (6, 1, 7680, 9216, 4, 8, 1), (6, 1, 8320, 8192, 16, 4, 1), (8, 2, 15872, 4352, 4, 8, 1),
+    (5, 0, 17408, 5120, 16, 4, 1), (4, 0, 17408, 10240, 8, 8, 1), (3, 1, 3072, 24576, 4, 4, 1), (7, 0, 256, 262144, 4, 8, 1),
+    (7, 0, 128, 524288, 8, 4, 0), (2, 0, 1024, 65536, 4, 4, 1), (4, 1, 3840, 17536, 4, 4, 1), (4, 1, 4096, 16896, 4, 8, 1)])
+def test_half_block_waves_of_a_full_chip(cuda, k, cb, n_in, n_out, tile_rows, waves, atomics):
     splits, rows_of_wave, wg_waves, atomic = _plan(k, n_in, n_out)
-    assert (rows_of_wave, wg_waves, atomic) == (tile_rows, waves, 1)
+    assert (rows_of_wave, wg_waves, atomic) == (tile_rows, waves, atomics)
     g = torch.Generator(device=cuda).manual_seed(n_in + k)
     tr = torch.randint(-32768, 32768, (n_in // 16, n_out // 16, 16 * k), dtype=torch.int16, device=cuda, generator=g)
     sign = lambda n: (torch.randint(0, 2, (n,), device=cuda, generator=g) * 2 - 1).half()

@@ -41,6 +41,43 @@ def test_large_launches_reduce_in_fp32_or_in_words_as_good(lib, rows):
     assert seen or rows in (2, 7, 8)
 
 
+def _whole_block_contributors(n_in, n_out, k):
+    """Contributors per sum of one row's launch in whole blocks (0: fp32 partial rows): up to twelve waves per
+    SIMD, two blocks to a wave from K = 5 on where that leaves two, and workgroups of eight waves where those of four would
+    issue more than 300 k atomics."""
+    blocks, groups = n_in // 128, n_out // 128
+    splits = min(max(12288 // groups, 1), blocks)
+    per = -(-blocks // splits)
+    if k >= 5 and per == 1 and blocks >= 2 and groups * ((blocks + 1) // 2) >= 2048:
+        per = 2
+    splits = -(-blocks // per)
+    for waves in (4, 8):
+        n = -(-splits // waves)
+        if n <= 255 and groups * n * 128 <= 300000:
+            return n
+    return 0
+
+
+def test_one_row_of_a_full_chip_keeps_the_fraction_bits_of_whole_blocks(lib):
+    """Where 4096 waves of whole blocks and more would run, one row takes half blocks only if its sums stay as fine:
+    accumulators where whole blocks have them, in words of no fewer fraction bits (33 up to 15 contributors, 30 up
+    to 31, ...); else the plan of whole blocks."""
+    halves = 0
+    for n_in in range(1024, 17409, 128):
+        for n_out in list(range(1024, 65537, 1664)) + [34816, 151936, 303872]:
+            if n_in // 128 * (n_out // 128) < 4096:
+                continue
+            for k in range(1, 9):
+                n, tile_rows, waves, atomic = _plan(lib, 1, n_in, n_out, k)
+                whole = _whole_block_contributors(n_in, n_out, k)
+                if tile_rows == 4:
+                    halves += 1
+                    assert whole and atomic and max(n.bit_length(), 4) <= max(whole.bit_length(), 4), (n_in, n_out, k)
+                else:
+                    assert atomic == (whole > 0) and (not whole or n == whole), (n_in, n_out, k)
+    assert halves > 1000
+
+
 _PLANS = """
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
