@@ -548,8 +548,14 @@ bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
 // the contributors where whole ones come two to a wave (from K = 5 on) or eight waves to a workgroup, and past 15 of them a word has
 // 30 bits in place of 33 (11904 -> 14848 K = 6 stays at 35.3, half blocks 30.6; workgroups of sixteen waves, which
 // would keep the bits, take up to 13 % more than whole blocks where they are few or decode MUL1).
+// Nor up to K = 2 where at most 24 blocks are to be added, and six to eight whole blocks to a SIMD come out even: there is
+// little to even out and little to decode, and the second rotation shows (K = 2, whole -> half: 2048 -> 65536 20.0 -> 20.6, 2048 -> 57344 17.5 ->
+// 18.0, 3072 -> 32000 15.0 -> 15.7; but 2816 -> 51840, 8.7 to a SIMD, 22.3 -> 21.2 and 6144 -> 16384 15.3 -> 14.8). Of 78 layers of
+// 4 to 10 whole blocks a SIMD, K = 2 to 4, the others are 2.8 % faster in half blocks, the slowest 2 % slower.
 static GemvPlan one_row_half_blocks(int in_tiles, int n_groups, int K, GemvPlan whole) {
     if (!linear_small_uses_atomics(1, n_groups, whole)) return whole;
+    const long long units = (long long)(in_tiles / 8) * n_groups, rounds = (units + 1023) / 1024;
+    if (K <= 2 && in_tiles <= 24 * 8 && rounds >= 6 && rounds <= 8 && units >= 0.95 * 1024 * rounds) return whole;
     for (const int waves : {4, 8}) {
         if (waves == 4 && K > 4) continue;
         const GemvPlan half{in_tiles / 4, 4, waves};

@@ -78,6 +78,16 @@ def test_one_row_of_a_full_chip_keeps_the_fraction_bits_of_whole_blocks(lib):
     assert halves > 1000
 
 
+@pytest.mark.parametrize("k,n_in,n_out,half", [
+    (2, 2048, 65536, False), (1, 2048, 65536, False), (3, 2048, 65536, True), (2, 3072, 32000, False), (2, 3072, 31104, True),
+    (2, 3200, 31360, True), (2, 2816, 51840, True), (2, 1280, 52480, True), (2, 2560, 32768, True)])
+def test_one_row_of_light_layers_that_come_out_even_takes_whole_blocks(lib, k, n_in, n_out, half):
+    """Up to K = 2, up to 24 blocks deep, six to eight whole blocks to a SIMD that leave less than a twentieth of the last
+    round idle: both sides of each of the lines."""
+    _, tile_rows, _, _ = _plan(lib, 1, n_in, n_out, k)
+    assert (tile_rows == 4) == half
+
+
 _PLANS = """
 import ctypes, sys
 sys.path.insert(0, sys.argv[1])
