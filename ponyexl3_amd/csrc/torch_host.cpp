@@ -700,13 +700,21 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
         THPObjectPtr l(PyObject_CallFunctionObjArgs(gate, x3.get(), nullptr));
         if (!l) throw python_error();
         bool ok = usable_logits(l.get(), x, 0);
-        if (has_shared && prefill && ok && THPVariable_Unpack(l.get()).scalar_type() == at::kHalf &&
+        if (has_shared && ok && THPVariable_Unpack(l.get()).scalar_type() == at::kHalf &&
             THPVariable_Unpack(l.get()).size(-1) == m.experts() - 1 && top_k < m.experts()) {
             w_shared = plain_gate_weight(shared_gate, x);
             if (w_shared.defined() && (w_shared.size(0) != 1 || (grad && w_shared.requires_grad()))) w_shared = at::Tensor();
         }
         THPObjectPtr s;
-        if (has_shared && !w_shared.defined()) {
+        if (w_shared.defined() && !prefill) {
+            // the slot kernels' router takes logits: one row of the gate's kernel, where the module's product is a library
+            // call that takes 2 to 5 us more in front of the experts (55 x 1280 15 us more: block 54.3 -> 38.9)
+            shared = at::empty({tokens}, x.options());
+            check_status(exl3_moe_gate(half_ptr(x), static_cast<int>(tokens), D, half_ptr(w_shared), 1, nullptr,
+                                       half_out(shared), nullptr, ctx.stream),
+                         "exl3_moe_gate");
+            w_shared = at::Tensor();
+        } else if (has_shared && !w_shared.defined()) {
             s = THPObjectPtr(PyObject_CallFunctionObjArgs(shared_gate, x3.get(), nullptr));
             if (!s) throw python_error();
         }

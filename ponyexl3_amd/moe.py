@@ -100,11 +100,12 @@ class EXL3SwitchGLU(torch.nn.Module):
     # weights among up to four of its slots; the prefill, with a rotation and a combination of its own, costs some 14 us more
     # to begin with and less for every pass and slot. From 24 tokens on, and 512 slots or 2.5 per expert, it
     # therefore depends on the work: up to 150 slots' worth of experts of 2^20 weights per projection, with
-    # at most 6 slots per expert, the slot kernels are the faster ones. Of 78 calls of those sizes none takes longer than
-    # through the prefill, and they take 2.7 % less; the better choice each time would be 1 % less again. us, slot
-    # kernels and prefill: 32 tokens, top-4 of 32 experts of 1792 x 256 35 and 48; 28 of 64 of 1536 x 512, top-6 and a
-    # shared one 63 and 69; 64 of 64 of 1664 x 512, top-4 and a shared one 76 and 76; 120 of 128 of
-    # 1408 x 512, top-3 92 and 88; 107 of 128 of 1152 x 768, top-5 and a shared one 157 and 120.
+    # at most 6 slots per expert, the slot kernels are the faster ones, on the whole: 179 such calls (K = 2 to 8, all codebooks) take
+    # 14 % less than through the prefill, seven of them 2 to 6 % more and three 9 to 11 % (33 tokens, top-4 of 32 experts of
+    # 1152 x 768 and a shared one 54 and 49; MUL1, 109 tokens, top-3 of 128 of 1408 x 256 and a shared one 72 and 66). Of 81 calls
+    # beyond the lines (up to 200 and 7) 42 would be faster in the slot kernels, by 7 % at the median. us, slot
+    # kernels and prefill: 26 tokens, top-2 of 16 experts of 1408 x 384 32 and 51; 49 of 64 of 1152 x 384, top-6 48 and 50; 71 of 32 of 2048 x
+    # 512, top-2 54 and 63; 65 of 32 of 1280 x 768, top-2 and a shared one 62 and 51.
     prefill_min_tokens = 24
     prefill_min_rows_per_expert = 2.5
     grouped_max_slots = 512

@@ -745,6 +745,29 @@ def test_moe_block_native_chain_equals_its_parts(cuda, tokens, shared):
     assert rel_l2(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
 
 
+@pytest.mark.parametrize("tokens,E,kk,prefill", [(33, 30, 2, False), (120, 40, 1, False), (40, 6, 4, True)])
+def test_shared_gate_is_computed_here_for_many_tokens(cuda, monkeypatch, tokens, E, kk, prefill):
+    """Past the tokens of the router's kernel the router's product is its module's; the shared gate's single column is not, on
+    the slot kernels either: one linear product is called, and the result is that of the parts."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+    from ponyexl3_amd.moe import combine_experts
+
+    D, H = 256, 128
+    switch = EXL3SwitchGLU.from_layers(*_experts(E + 1, D, H, 4, True, 4600))
+    assert switch._use_prefill(tokens, kk + 1) == prefill
+    lin = lambda n: torch.nn.Linear(D, n, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin(E), lin(1), switch, kk)
+    x = torch.randn((1, tokens, D), generator=torch.Generator().manual_seed(tokens)).half().to(cuda)
+    linear, widths = torch.nn.functional.linear, []
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda a, w, *r: (widths.append(w.shape[0]), linear(a, w, *r))[1])
+    print(f"shared gate tokens={tokens}", flush=True)
+    y = block(x)
+    assert widths == [E]
+    inds, scores = block.route(x)
+    ref = combine_experts(switch(x, inds).float(), scores)
+    assert rel_l2(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
+
+
 @pytest.mark.parametrize("tokens", [2, 67])
 def test_moe_block_reaches_replaced_parts(cuda, tokens):
     """A router replaced on the instance and hooks on all modules see the call, and the result
