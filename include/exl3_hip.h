@@ -393,6 +393,14 @@ int exl3_moe_forward(const uint16_t *x, int tokens, const int32_t *indices, int 
 size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
 
 /*
+ * 1 if exl3_moe_forward and exl3_moe_decode, given counters, group the slots of such a call by expert and round the
+ * down projection's weights as exl3_moe_prefill does (top_k slots a token, a shared expert among them; EXL3_MOE_GROUP
+ * and EXL3_EXACT_WEIGHTS as set), else 0: for a caller that chooses between the two by time, so that the result is no
+ * coarser either way.
+ */
+int exl3_moe_groups_rounded(int tokens, int top_k, int num_experts);
+
+/*
  * exl3_moe_route, exl3_moe_forward and exl3_moe_combine as one call (ponyexl3/mlx/exl3_moe.py:817-839)
  * with the same results. A few slots (those whose gate and up reduce through accumulators, at
  * most 256 experts to rank) take two launches: the experts' kernel ranks the logits of its token

@@ -784,7 +784,8 @@ static bool moe_group_slots() {
 
 // Calls of a size that the sorted prefill kernels also serve get the rounded weights of those in the down
 // projection too, so that the result is no further from the reference's arithmetic whichever is faster
-// (7.1e-4 of the output with unsummed halves, 6.8e-4 with rounded weights, against 64 bits).
+// (7.1e-4 of the output with unsummed halves, 6.8e-4 with rounded weights, against 64 bits). The sizes from which on callers
+// turn to the prefill are their own (EXL3SwitchGLU starts out with these); exl3_moe_groups_rounded tells them what holds here.
 static bool moe_exact_down(int tokens, int slots, int num_experts) {
     return tokens >= 24 && (slots > 512 || slots >= 2.5 * num_experts);
 }
@@ -1121,6 +1122,12 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
                       dn_svh, num_experts, D, H, K, cb, activation, y, workspace, workspace_bytes, counters,
                       counters_len, {}, {}},
                      as_stream(stream));
+}
+
+EXL3_EXPORT int exl3_moe_groups_rounded(int tokens, int top_k, int num_experts) {
+    using namespace exl3;
+    return tokens > 0 && top_k > 0 && num_experts > 0 && !exact_weights() && moe_groups_apply(tokens, top_k, num_experts) &&
+           moe_exact_down(tokens, tokens * top_k, num_experts);
 }
 
 EXL3_EXPORT size_t exl3_moe_decode_counters(int tokens, int slots_per_token, int D, int H) {

@@ -116,8 +116,11 @@ class EXL3SwitchGLU(torch.nn.Module):
         if tokens < self.prefill_min_tokens or (
                 slots <= self.grouped_max_slots and slots < self.prefill_min_rows_per_expert * self.num_experts):
             return False
+        # (and the slot kernels only where the library says that they round what the prefill rounds: the lines above may be
+        # set by the caller, grouping switched off)
         return (slots > self.grouped_max_slots or slots > 6 * self.num_experts
-                or slots * self.input_dims * self.hidden_dims > self.grouped_max_work)
+                or slots * self.input_dims * self.hidden_dims > self.grouped_max_work
+                or not _lib.load().exl3_moe_groups_rounded(tokens, top_k, self.num_experts))
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         if indices.dim() != 3:
