@@ -377,8 +377,8 @@ int exl3_linear_forward_static(const uint16_t *x, int rows, const uint16_t *trel
  *               Two more ints than that make the last int the status word of
  *               exl3_counters_status.
  * Only the selected experts' trellis blocks are read. In the two-launch chain, with
- * 2 <= tokens, at most 1024 slots and 1024 experts, and where an even routing would spare 15 %
- * of the slots and 15 of them their own pass, the slots that route to one expert share a pass over
+ * 2 <= tokens, at most 1024 slots and 1024 experts, and where an even routing would spare a fifth
+ * of the slots and 18 of them (15 % where that is 11 * 2^20 weights per projection) their own pass, the slots that route to one expert share a pass over
  * its weights (four batch rows per pass; same arithmetic per row, bit-identical results; one small
  * launch more); EXL3_MOE_GROUP=0 switches that off. From 24 tokens on, with more than 512 slots or 2.5 per
  * expert, those calls round the down projection's weights to fp16 like the prefill chain.
@@ -398,7 +398,7 @@ size_t exl3_moe_workspace_bytes(int tokens, int top_k, int D, int H);
  * and EXL3_EXACT_WEIGHTS as set), else 0: for a caller that chooses between the two by time, so that the result is no
  * coarser either way.
  */
-int exl3_moe_groups_rounded(int tokens, int top_k, int num_experts);
+int exl3_moe_groups_rounded(int tokens, int top_k, int num_experts, int D, int H);
 
 /*
  * exl3_moe_route, exl3_moe_forward and exl3_moe_combine as one call (ponyexl3/mlx/exl3_moe.py:817-839)

@@ -52,7 +52,7 @@ PROTOTYPES = {
     ),
     "exl3_moe_gate": (_i, [_vp, _i, _i, _vp, _i, _vp, _vp, _vp, _vp]),
     "exl3_moe_decode_counters": (_sz, [_i] * 4),
-    "exl3_moe_groups_rounded": (_i, [_i] * 3),
+    "exl3_moe_groups_rounded": (_i, [_i] * 5),
     "exl3_moe_decode": (_i, [_vp, _i, _vp, _vp, _i, _i, _i] + [_vp] * 6 + [_i] * 6 + [_vp] * 5 + [_sz, _vp, _sz, _vp]),
     "exl3_moe_route": (_i, [_vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),
     "exl3_moe_route_shared": (_i, [_vp, _vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),

@@ -791,21 +791,23 @@ static bool moe_exact_down(int tokens, int slots, int num_experts) {
 }
 
 // Whether the slots are grouped by expert: where that is expected to spare enough passes over an expert's
-// weights to pay for the list and for reducing through partial rows, 15 % of the slots and
-// 15 of them (choices taken as independent and even). From what every entry point knows, so that the block and its parts
-// take the same way: that one of the experts may be a shared one, which all tokens have, is not asked.
-// us, every slot on its own -> grouped, passes spared of slots: 11 tokens through 257 experts of 2048 x 512 with 9 slots a token, K = 4
-// 15.6 of 99 63.2 -> 59.6, 14 tokens 25 of 126 72.5 -> 67.1; 24, 68 of 216 97 -> 86; 17 tokens, 3 of 64 experts of 1024 x 768,
+// weights to pay for the list and for reducing through partial rows (3 us and more): a fifth of the slots and 18 of them, or 15 %
+// and the passes over 11 experts of 2^20 weights per projection (choices taken as independent and even). From what every entry
+// point knows, so that the block and its parts take the same way: that one of the experts may be a shared one, which all tokens have,
+// is not asked. us, every slot on its own -> grouped, passes spared of slots: 11 tokens through 257 experts of 2048 x 512 with 9 slots a
+// token, K = 4 15.6 of 99 63.2 -> 59.6, 14 tokens 25 of 126 72.5 -> 67.1; 24, 68 of 216 97 -> 86; 17 tokens, 3 of 64 experts of 1024 x 768,
 // K = 5 15.3 of 51 38.3 -> 34.7; 10 tokens, 7 of 192 of 1280 x 768, K = 3 8.0 of 70 48.5 -> 51.0; 9 tokens, 8 of 256 of
-// 1024 x 384 8.4 of 72 30.7 -> 33.9. Of 90 calls of 2 to 26 tokens with 11 to 30 % spared the 46 on the grouped side
-// take 6 % less, four of them (few weights: 256 and 384 wide) 2 to 8 % more; of the 44 on the single side ten would
-// take 6 to 15 % less grouped (wide experts, MUL1), as many 5 to 11 % more. Calls that are to have rounded weights in the down
+// 1024 x 384 8.4 of 72 30.7 -> 33.9; 7 tokens, 6 of 33 of 1280 x 256 17 of 42 23.2 -> 26.5. Of 90 calls of 2 to 26 tokens with 11 to 30 % spared
+// the 47 on the grouped side take 6 % less, four of them 2 to 8 % more; of the 43 on the single side fourteen would take 4 to 13 % less
+// grouped (wide experts, MUL1), as many 3 to 11 % more. Calls that are to have rounded weights in the down
 // projection, which the grouped kernel has, are grouped where fewer are spared, too (24 slots of 8 experts: 16).
-static bool moe_groups_apply(int tokens, int top_k, int num_experts) {
+static bool moe_groups_apply(int tokens, int top_k, int num_experts, int D, int H) {
     const long long slots = (long long)tokens * top_k;
     if (tokens < 2 || slots > kGroupMaxSlots || num_experts > kGroupMaxExperts || !moe_group_slots()) return false;
     const double passes = num_experts * (1.0 - std::pow(1.0 - std::min(1.0, (double)top_k / num_experts), tokens));
-    return slots - passes >= std::max(15.0, 0.15 * slots) ||
+    const double spared = slots - passes;
+    return spared >= std::max(18.0, 0.2 * slots) ||
+           (spared >= std::max(11.0, 0.15 * slots) && spared * D * H >= 11.0 * (1 << 20)) ||
            (moe_exact_down(tokens, (int)slots, num_experts) && slots >= 2.5 * num_experts);
 }
 
@@ -981,7 +983,7 @@ static int moe_slots(const MoeCall& a, hipStream_t s) {
         // two launches: gate/up + GLU + rotation, then down
         const int hblocks = H / 128, dblocks = D / 128;
         if (counters_len < (size_t)slots * (hblocks + dblocks)) return EXL3_E_WORKSPACE;
-        const bool grouped = moe_groups_apply(tokens, top_k, num_experts);
+        const bool grouped = moe_groups_apply(tokens, top_k, num_experts, D, H);
         const bool half = moe_half_blocks((long long)slots * 2 * hblocks * dblocks, grouped, K);
         // every slot on its own, few enough atomics, and counters large enough to hold
         // the accumulators (uint64 [slots][2][H], then the down launch's counters): gate
@@ -1124,10 +1126,10 @@ EXL3_EXPORT int exl3_moe_forward(const uint16_t* x, int tokens, const int32_t* i
                      as_stream(stream));
 }
 
-EXL3_EXPORT int exl3_moe_groups_rounded(int tokens, int top_k, int num_experts) {
+EXL3_EXPORT int exl3_moe_groups_rounded(int tokens, int top_k, int num_experts, int D, int H) {
     using namespace exl3;
-    return tokens > 0 && top_k > 0 && num_experts > 0 && !exact_weights() && moe_groups_apply(tokens, top_k, num_experts) &&
-           moe_exact_down(tokens, tokens * top_k, num_experts);
+    return tokens > 0 && top_k > 0 && num_experts > 0 && !exact_weights() &&
+           moe_groups_apply(tokens, top_k, num_experts, D, H) && moe_exact_down(tokens, tokens * top_k, num_experts);
 }
 
 EXL3_EXPORT size_t exl3_moe_decode_counters(int tokens, int slots_per_token, int D, int H) {

@@ -120,7 +120,8 @@ class EXL3SwitchGLU(torch.nn.Module):
         # set by the caller, grouping switched off)
         return (slots > self.grouped_max_slots or slots > 6 * self.num_experts
                 or slots * self.input_dims * self.hidden_dims > self.grouped_max_work
-                or not _lib.load().exl3_moe_groups_rounded(tokens, top_k, self.num_experts))
+                or not _lib.load().exl3_moe_groups_rounded(tokens, top_k, self.num_experts, self.input_dims,
+                                                               self.hidden_dims))
 
     def forward(self, x: torch.Tensor, indices: torch.Tensor) -> torch.Tensor:
         if indices.dim() != 3:

@@ -947,7 +947,7 @@ def test_decode_call_equals_its_parts(cuda, tokens, E, D, H, top_k, shared):
 # knows) must not choose the kernels: accumulators against partial rows, and from K = 5 on half blocks against whole ones
 @pytest.mark.parametrize("tokens,E,D,H,top_k,k", [(8, 64, 1024, 256, 6, 4), (8, 128, 640, 256, 8, 6), (10, 256, 1024, 256, 8, 6),
                                                   (11, 256, 1024, 256, 8, 4), (12, 256, 1024, 256, 8, 6), (14, 256, 1024, 256, 8, 4),
-                                                  (13, 256, 1152, 512, 8, 8)])
+                                                  (13, 256, 1152, 512, 8, 8), (11, 256, 2048, 512, 8, 4)])
 def test_decode_call_equals_its_parts_beside_the_grouping_line(cuda, tokens, E, D, H, top_k, k):
     _decode_call_and_parts(cuda, tokens, E, D, H, top_k, True, k)
 
