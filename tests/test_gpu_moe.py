@@ -23,6 +23,12 @@ def _experts(E, D, H, k, mcg, seed):
     return gate, up, down
 
 
+def _switch(E, D, H, k):
+    from ponyexl3_amd import EXL3SwitchGLU
+
+    return EXL3SwitchGLU.from_layers(*_experts(E, D, H, k, False, 1300))
+
+
 def _oracle_chain(oracle, gate, up, down, x, idx, act):
     experts = [{"gate": (g.trellis, g.suh, g.svh), "up": (u.trellis, u.suh, u.svh),
                 "down": (d.trellis, d.suh, d.svh)} for g, u, d in zip(gate, up, down)]
@@ -79,42 +85,79 @@ def test_two_launch_and_five_launch_chains(cuda, oracle, tokens):
     assert rel_l2(y1.cpu().numpy(), y5.cpu().numpy()) <= TOL
 
 
-@pytest.mark.parametrize("tokens,top_k,E", [(2, 2, 2), (5, 2, 3), (9, 3, 4), (32, 2, 40), (256, 2, 3)])
-def test_slots_grouped_by_expert_equal_ungrouped(cuda, tokens, top_k, E):
-    """With several tokens the slots of one expert share a pass over its weights, four
-    rows at a time (here up to 171 slots per expert, i.e. many leaders per expert, and
-    the routing table scanned in up to eight chunks). The arithmetic per row is that of
-    the per-slot kernels, so the result is bit-identical to runs that do not group: one
-    token at a time (a token's experts are distinct), and, for the 512-slot case, whose
-    waves take whole Hadamard blocks where a single token's take half blocks, the same
-    tokens inside a 514-slot call, which is past the grouped kernels' routing table."""
-    from ponyexl3_amd import EXL3SwitchGLU, ops
+def _groups_of(ws, slots, D, H):
+    """Number of groups in the list that a grouped call leaves in its workspace (behind the two buffers of rotated rows)."""
+    at = sum((n * 2 + 255) // 256 * 256 for n in (slots * 2 * D, slots * H))
+    return int(ws[at:at + 4].view(torch.int32)[0])
 
-    D, H, k = 384, 256, 4
-    gate, up, down = _experts(E, D, H, k, False, 1300)
-    moe = EXL3SwitchGLU.from_layers(gate, up, down)
+
+def _moe_forward(x, idx, moe, k, D, H):
+    """exl3_moe_forward as ops.moe_forward with accumulators=False calls it, with a workspace that can be looked at."""
+    from ponyexl3_amd import _lib, ops
+
+    lib, p, (tokens, top_k) = _lib.load(), ops._ptr, idx.shape
+    need = lib.exl3_moe_workspace_bytes(tokens, top_k, D, H)
+    ws = torch.full((need,), 0xCC, dtype=torch.uint8, device=x.device)
+    y = torch.empty((tokens, top_k, D), dtype=torch.float16, device=x.device)
+    n = tokens * top_k * (H // 128 + D // 128)
+    cnt = ops.sync_counters(x.device, n)
+    _lib.check(lib.exl3_moe_forward(p(x), tokens, p(idx), top_k, p(moe._gu_trellis), p(moe._gu_suh), p(moe._gu_svh),
+                                    p(moe._dn_trellis), p(moe._dn_suh), p(moe._dn_svh), moe.num_experts, D, H, k, moe._cb, 0,
+                                    p(y), p(ws), need, p(cnt), n + 2, ops._stream()), "exl3_moe_forward")
+    assert int(cnt.abs().sum()) == 0
+    return y, ws
+
+
+# few and many experts, groups of one to four rows and up to 20 of one expert, one and two workgroups a reduction; up to
+# K = 4 half blocks below 4096 waves of whole ones and whole blocks from there on, from K = 5 on half blocks throughout
+@pytest.mark.parametrize("tokens,top_k,E,D,H,k,whole", [
+    (9, 3, 4, 384, 256, 4, False), (32, 2, 40, 384, 256, 4, False), (12, 3, 6, 640, 128, 6, False), (23, 7, 12, 256, 640, 8, False),
+    (20, 8, 16, 640, 384, 4, True), (23, 7, 30, 640, 640, 3, True)])
+def test_slots_grouped_by_expert_equal_ungrouped(cuda, tokens, top_k, E, D, H, k, whole):
+    """With several tokens the slots of one expert share a pass over its weights, four rows at a time. Below the
+    prefill's sizes the arithmetic per row is that of the per-slot kernels, so the result is bit-identical to runs that do
+    not group, take the same blocks and reduce through partial rows too: one token at a time where waves take half
+    blocks, and where they take whole ones the same tokens among more than 1024 slots, which no list holds."""
+    moe = _switch(E, D, H, k)
+    many = 1024 // top_k + 1
     rng = np.random.default_rng(tokens * 7 + E)
-    x = (rng.standard_normal((tokens + 1, D)) * 0.5).astype(np.float16)
-    idx = np.stack([rng.permutation(E)[:top_k] for _ in range(tokens + 1)]).astype(np.int32)
-    xt, it = torch.from_numpy(x).to(cuda), torch.from_numpy(idx).to(cuda)
-    args = (moe._gu_trellis, moe._gu_suh, moe._gu_svh, moe._dn_trellis, moe._dn_suh, moe._dn_svh, k, moe._cb)
-    print(f"moe grouped tokens={tokens} top_k={top_k} E={E}", flush=True)
-    y = ops.moe_forward(xt[:tokens], it[:tokens], *args)
-    y_again = ops.moe_forward(xt[:tokens], it[:tokens], *args)
-    assert torch.equal(y, y_again)
-    assert int(ops.sync_counters(cuda, 1).abs().sum()) == 0
-    # the runs that do not group reduce through partial rows like the grouped kernels
-    # (accumulators=False); the accumulator reduction rounds the sum differently
-    if tokens * top_k == 512:
-        wide = ops.moe_forward(xt, it, *args, accumulators=False)
+    x = torch.from_numpy((rng.standard_normal((many, D)) * 0.5).astype(np.float16)).to(cuda)
+    idx = torch.from_numpy(np.stack([rng.permutation(E)[:top_k] for _ in range(many)]).astype(np.int32)).to(cuda)
+    slots = tokens * top_k
+    assert (slots * 2 * (D // 128) * (H // 128) >= 4096) == whole and (tokens < 24 or slots < 2.5 * E)
+    print(f"moe grouped tokens={tokens} top_k={top_k} E={E} k={k}", flush=True)
+    y, ws = _moe_forward(x[:tokens], idx[:tokens], moe, k, D, H)
+    count = torch.bincount(idx[:tokens].flatten().long(), minlength=E)
+    assert _groups_of(ws, slots, D, H) == int(((count + 3) // 4).sum()) < slots
+    assert torch.equal(y, _moe_forward(x[:tokens], idx[:tokens], moe, k, D, H)[0])
+    if whole:
+        wide, ws = _moe_forward(x, idx, moe, k, D, H)
+        assert _groups_of(ws, many * top_k, D, H) == -0x33333334  # 0xCCCCCCCC: no list
         assert torch.equal(y, wide[:tokens])
-    step = max(1, tokens // 16)
-    for t in list(range(0, tokens, step)) + [tokens - 1]:
-        one = ops.moe_forward(xt[t:t + 1], it[t:t + 1], *args, accumulators=False)
-        if tokens * top_k == 512:
-            assert rel_l2(y[t].float().cpu().numpy(), one[0].float().cpu().numpy()) <= TOL
-        else:
-            assert torch.equal(y[t], one[0]), f"token {t}"
+    else:
+        for t in range(tokens):
+            assert torch.equal(y[t], _moe_forward(x[t:t + 1], idx[t:t + 1], moe, k, D, H)[0][0]), f"token {t}"
+
+
+@pytest.mark.parametrize("tokens,top_k,E,D,H,k", [(256, 2, 3, 384, 256, 4), (256, 2, 3, 384, 256, 6), (24, 2, 16, 384, 256, 4),
+                                                  (171, 3, 257, 256, 128, 5)])
+def test_rows_of_a_group_do_not_touch_each_other(cuda, tokens, top_k, E, D, H, k):
+    """From the prefill's sizes on grouped calls round the down projection's weights, which no ungrouped one does: a slot's
+    result is bit for bit that of a call of the same size in which the other tokens have other inputs and other experts, so
+    that it sits in another group among other rows (the values themselves: test_down_weights_are_rounded_...)."""
+    from ponyexl3_amd import _lib
+
+    assert _lib.load().exl3_moe_groups_rounded(tokens, top_k, E, D, H)
+    moe = _switch(E, D, H, k)
+    rng = np.random.default_rng(tokens + E)
+    draw = lambda: (torch.from_numpy((rng.standard_normal((tokens, D)) * 0.5).astype(np.float16)).to(cuda),
+                    torch.from_numpy(np.stack([rng.permutation(E)[:top_k] for _ in range(tokens)]).astype(np.int32)).to(cuda))
+    (x, idx), (x2, idx2) = draw(), draw()
+    print(f"moe rounded groups tokens={tokens} top_k={top_k} E={E} k={k}", flush=True)
+    y, _ = _moe_forward(x, idx, moe, k, D, H)
+    kept = torch.from_numpy(rng.permutation(tokens)[:tokens // 3]).to(cuda)
+    x2[kept], idx2[kept] = x[kept], idx[kept]
+    assert torch.equal(_moe_forward(x2, idx2, moe, k, D, H)[0][kept], y[kept])
 
 
 @pytest.mark.parametrize("tokens,top_k,E,D,H,act", [(1, 2, 4, 640, 640, 0), (1, 8, 64, 2048, 512, 0),
@@ -491,16 +534,18 @@ def test_prefill_sorts_as_the_sort_kernel(cuda, tokens, kk, E):
     assert torch.equal(ws[at:at + 16 * table.shape[0]].view(torch.int32).view(-1, 4), table.view(-1, 4))
 
 
-def test_prefill_past_32_bit_offsets(cuda):
-    """From 4 GiB of rotated rows on they are put in sorted order, behind a sort of its own, instead of gathered: the
+@pytest.mark.parametrize("tokens", [16400, 32767, 32800])
+def test_prefill_past_31_and_32_bit_offsets(cuda, tokens):
+    """Rotated rows are gathered at 32-bit byte offsets, the last ones past 2^31 (16400 tokens) and up to the last row that
+    such an offset reaches (32767); from 4 GiB on (32800) they are put in sorted order, behind a sort of its own, instead. The
     last tokens' rows are those of a call on them alone, up to the order of the sums (the row blocks differ)."""
     from ponyexl3_amd import _lib, ops
 
     if torch.cuda.mem_get_info()[0] < 40 << 30:
         pytest.skip("needs 40 GB of memory")
     lib, p = _lib.load(), ops._ptr
-    tokens, kk, E, D, H, K = 32800, 4, 8, 16384, 128, 2
-    assert tokens * kk * D * 2 > 0xFFFFFFFF
+    kk, E, D, H, K = 4, 8, 16384, 128, 2
+    assert tokens * kk * D * 2 > 1 << 31 and (tokens * kk * D * 2 > 0xFFFFFFFF) == (tokens > 32767)
     g = torch.Generator(device=cuda).manual_seed(5)
     bits = lambda *s: torch.randint(-32768, 32768, s, dtype=torch.int16, device=cuda, generator=g)
     sign = lambda size, *s: ((torch.randint(0, 2, s, device=cuda, generator=g) * 2.0 - 1.0) * size).half()
@@ -518,7 +563,7 @@ def test_prefill_past_32_bit_offsets(cuda):
                                         ops._stream()), "exl3_moe_prefill")
         return y
 
-    print("prefill past 32-bit offsets", flush=True)
+    print(f"prefill past 31-bit offsets tokens={tokens}", flush=True)
     got = run(x, idx)
     for part in (slice(0, 100), slice(tokens - 100, tokens)):
         ref = run(x[part].contiguous(), idx[part].contiguous())
