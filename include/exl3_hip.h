@@ -378,10 +378,14 @@ int exl3_linear_forward_static(const uint16_t *x, int rows, const uint16_t *trel
  *               exl3_counters_status.
  * Only the selected experts' trellis blocks are read. In the two-launch chain, with
  * 2 <= tokens, at most 1024 slots and 1024 experts, and where an even routing would spare a fifth
- * of the slots and 18 of them (15 % where that is 11 * 2^20 weights per projection) their own pass, the slots that route to one expert share a pass over
- * its weights (four batch rows per pass; same arithmetic per row, bit-identical results; one small
- * launch more); EXL3_MOE_GROUP=0 switches that off. From 24 tokens on, with more than 512 slots or 2.5 per
- * expert, those calls round the down projection's weights to fp16 like the prefill chain.
+ * of the slots and 18 of them (15 % where that is 11 * 2^20 weights per projection) their own pass, the slots that route to
+ * one expert share a pass over its weights (four batch rows per pass; one small launch more); EXL3_MOE_GROUP=0 switches
+ * that off. A slot's result does not depend on the slots that it shares a pass with. It is bit for bit that of an ungrouped
+ * call if that reduces through partial rows (counters_len below the accumulators' size) and takes the same blocks (half
+ * Hadamard blocks: ungrouped below 3200 waves of whole ones in gate/up, grouped below 4096 and from K = 5 on always), else it
+ * differs by the order and the rounding of fp32 sums, an fp16 ulp or two. From 24 tokens on, with more than 512 slots or
+ * 2.5 per expert, grouped calls round the down projection's weights to fp16 like the prefill chain: 4e-4 and more (relative
+ * 2-norm) from the unsummed halves of ungrouped ones.
  */
 int exl3_moe_forward(const uint16_t *x, int tokens, const int32_t *indices, int top_k,
                      const uint16_t *gu_trellis, const uint16_t *gu_suh, const uint16_t *gu_svh,

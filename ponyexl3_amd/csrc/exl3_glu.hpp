@@ -5,12 +5,13 @@
 
 namespace exl3 {
 
-// g / (1 + exp(-g)) in 16 instructions, where expf() and the division take 26: the quotient, corrected once by its
-// remainder, needs no scaling (its divisor is 1 and more), and the power no clamping. exp(-g) = 2^n 2^f with n + f =
-// -g log2(e), n whole and f at most 1/2. Rounded to a half the result is that of the other form for all 65536 halfs g, and
-// over 2^22 normal g of deviation 4 the fp32 errors are the same (2.02 ulp at most, 0.472 rms). So are
-// zeros, infinities and NaNs: -g goes in between -100, where 1 + exp(-g) is 1, and 200, where exp(-g) is
-// infinite, and v_div_fixup gives what an infinite g or divisor makes of a quotient.
+// g / (1 + exp(-g)). The exponential by reduction to a power of two, the product with log2(e) in two parts as in Cody and
+// Waite's: exp(-g) = 2^n 2^f with n + f = -g log2(e), n whole and f at most 1/2, where the second part of log2(e)
+// keeps the bits below the first product; 2^f by v_exp_f32. The quotient by v_rcp_f32 and one Newton correction with the
+// remainder; it needs no scaling, as its divisor is 1 and more. Rounded to a half the result is that of
+// g / (1.0f + expf(-g)) for all 65536 halfs g, and over 2^22 normal g of deviation 4 the fp32 errors are the same (2.02 ulp at most,
+// 0.472 rms). So are zeros, infinities and NaNs: -g goes in between -100, where 1 + exp(-g) is 1, and 200, where
+// exp(-g) is infinite, and v_div_fixup gives what an infinite g or divisor makes of a quotient.
 __device__ __forceinline__ float silu(float g) {
 #pragma clang fp contract(off)
     const float t = __builtin_amdgcn_fmed3f(-g, -100.f, 200.f);

@@ -314,8 +314,8 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
 // 22.5 -> 17.3, 15 of 2560 -> 29440 24.3 -> 20.1, 14 of 9216 -> 5248 22.3 -> 19.0, 12 of 12288 -> 10368 34.6 -> 29.4. Beyond the lines: 11 rows of
 // 2560 -> 43008 (336 workgroups of 20 steps) 35.8 and 40.7, 10 of 8192 -> 21632 (507 of 22) 34.8 and 36.5, 14 of 4096 -> 19072 (447) 22.8
 // and 24.0, 12 of 7168 -> 12288 (768 medium-batch workgroups, three to a CU) 22.8
-// and 24.9. Over 245 layers of 9 to 16
-// rows 3.5 % less, none more than 2 % slower.
+// and 24.9. Of 225 layers of 9 to 16 rows on both sides of the lines the 71 that changed from the medium-batch kernel take 8.3 %
+// less, one of them 1.7 % more (12 rows of 1024 -> 49152 21.6 and 22.0); the others, same kernel, repeat within 4 %.
 bool linear_rows_before_mid(int rows, int K, int in_tiles, int out_tiles) {
     if (rows > 16 || K >= 5 || in_tiles >= 2 * out_tiles) return true;
     const int n_groups = out_tiles / 8;

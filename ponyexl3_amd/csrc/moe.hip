@@ -548,7 +548,8 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
 // that make_slot_groups() has left, up to four batch rows each (the matrix instructions carry
 // four rows at the price of one). The grid holds as many sets as there could be groups (one per
 // slot); those past the list leave after one scalar load. Per row the arithmetic, the partial rows and the
-// counters are those of the kernels above, so the results are bit-identical.
+// counters are those of the kernels above with partial rows, so the results are bit-identical to theirs where both take
+// half blocks, or both whole ones (moe_half_blocks()), and the down weights are not rounded (moe_exact_down()).
 
 struct SlotGroup {
     int n;               // rows; 0 = past the list

@@ -4,8 +4,8 @@
 //
 // What bounds them: issue of the decode. 1537 tokens through 257 experts, NKS = 2: VALU issue 85 % and
 // 77 % (gate/up, down) of the time that CUs are busy, which is 81 and 84 % of the time (2.2 and 4.4
-// rounds of workgroups); 25 and 36 % of the VALU instructions stood outside the main loop. SiLU in 16 instructions in
-// place of 26 and accumulators that the matrix pipe clears, whole call: 1537 tokens 309 -> 301 us, 400 through 65
+// rounds of workgroups); 25 and 36 % of the VALU instructions stood outside the main loop. SiLU without the
+// scaling that its range does not need and accumulators that the matrix pipe clears, whole call: 1537 tokens 309 -> 301 us, 400 through 65
 // experts of 1024 x 256 67.9 -> 65.2; over 58 shapes of 45 to 2048 tokens 2 %. Looping
 // workgroups, one launch of as many as the chip holds, were slower (gate/up 158 -> 162 us, down 94 -> 103).
 //
