@@ -45,7 +45,7 @@ CB = 0
 # rocprofv3 --pmc runs of this script (FETCH_SIZE, then WRITE_SIZE), each scaled
 # by what the same counter reads for a plain copy of known size; see
 # profiles/linear_small_k4_config2_pmc.txt.
-TRAFFIC_BYTES_PER_STEP = 200_702_566
+TRAFFIC_BYTES_PER_STEP = 198_074_418
 
 # (name, in, [member out sizes]) of the config-2 layer; several members = sibling-fused
 LAYER_FUSED_QKV = [
