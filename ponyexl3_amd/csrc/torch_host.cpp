@@ -500,6 +500,7 @@ PyObject* experts_slots(PyObject* self, PyObject* args) {
 // Up to this many tokens the router's product runs in exl3_moe_gate, above it in the gate
 // module: its kernel is made for one round trip to memory, not for throughput.
 constexpr int64_t kGateMaxTokens = 32;
+constexpr int64_t kGateGridTokens = 16 * 65535;
 
 // Router table, experts and weighted sum of a call on the slot kernels: one call, whose tables and slot
 // rows lie in the stream's scratch behind the kernels' workspace. x (tokens, D), logits fp16 (tokens,
@@ -700,7 +701,8 @@ PyObject* experts_block(PyObject* self, PyObject* args) {
         THPObjectPtr l(PyObject_CallFunctionObjArgs(gate, x3.get(), nullptr));
         if (!l) throw python_error();
         bool ok = usable_logits(l.get(), x, 0);
-        if (has_shared && ok && THPVariable_Unpack(l.get()).scalar_type() == at::kHalf &&
+        // (a grid of exl3_moe_gate holds kGateGridTokens; more reach the slot kernels where the caller has moved the line)
+        if (has_shared && ok && (prefill || tokens <= kGateGridTokens) && THPVariable_Unpack(l.get()).scalar_type() == at::kHalf &&
             THPVariable_Unpack(l.get()).size(-1) == m.experts() - 1 && top_k < m.experts()) {
             w_shared = plain_gate_weight(shared_gate, x);
             if (w_shared.defined() && (w_shared.size(0) != 1 || (grad && w_shared.requires_grad()))) w_shared = at::Tensor();

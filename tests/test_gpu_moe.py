@@ -813,6 +813,25 @@ def test_shared_gate_is_computed_here_for_many_tokens(cuda, monkeypatch, tokens,
     assert rel_l2(y.float().cpu().numpy(), ref.cpu().numpy()) <= TOL
 
 
+def test_slot_kernels_take_more_tokens_than_a_gate_grid(cuda):
+    """One token more than a launch of the gate's kernel holds, kept off the prefill by a line that the caller moved: the
+    shared gate's column goes through its module and every token has the result of a small call."""
+    from ponyexl3_amd import EXL3MoEBlock, EXL3SwitchGLU
+
+    D, tokens = 128, 16 * 65535 + 1
+    switch = EXL3SwitchGLU.from_layers(*_experts(2, D, 128, 4, True, 4650))
+    switch.prefill_min_tokens = 1 << 30
+    lin = lambda n: torch.nn.Linear(D, n, bias=False).half().to(cuda).requires_grad_(False)
+    block = EXL3MoEBlock(lin(1), lin(1), switch, 1)
+    base = torch.randn((1021, D), generator=torch.Generator().manual_seed(4)).half().to(cuda)
+    print(f"slot kernels tokens={tokens}", flush=True)
+    ref = block(base).float()
+    y = block(base.repeat(-(-tokens // 1021), 1)[:tokens])
+    for part in y.split(1021):
+        want = ref[: len(part)]
+        assert (part.float() - want).norm() <= TOL * want.norm()
+
+
 @pytest.mark.parametrize("tokens", [2, 67])
 def test_moe_block_reaches_replaced_parts(cuda, tokens):
     """A router replaced on the instance and hooks on all modules see the call, and the result
