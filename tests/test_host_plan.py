@@ -78,12 +78,16 @@ def test_one_row_of_a_full_chip_keeps_the_fraction_bits_of_whole_blocks(lib):
     assert halves > 1000
 
 
+# none left over by workgroups of four; one and two; the same in as many rounds; three; whole blocks eight to a workgroup: none left over by
+# the fours in as many rounds and in fewer, one, three in as many and in fewer; K = 3 on both sides, K = 4
 @pytest.mark.parametrize("k,n_in,n_out,half", [
-    (2, 2048, 65536, False), (1, 2048, 65536, False), (3, 2048, 65536, True), (2, 3072, 32000, False), (2, 3072, 31104, True),
-    (2, 3200, 31360, True), (2, 2816, 51840, True), (2, 1280, 52480, True), (2, 2560, 32768, True)])
-def test_one_row_of_light_layers_that_come_out_even_takes_whole_blocks(lib, k, n_in, n_out, half):
-    """Up to K = 2, up to 24 blocks deep, six to eight whole blocks to a SIMD that leave less than a twentieth of the last
-    round idle: both sides of each of the lines."""
+    (2, 2048, 65536, False), (1, 2048, 65536, False), (2, 3072, 31104, False), (1, 9728, 13824, False),
+    (2, 3200, 31360, True), (2, 2816, 51840, True), (2, 1280, 52480, True), (2, 4864, 15232, True),
+    (2, 4736, 19328, False), (1, 9472, 8320, False), (2, 1408, 61952, False),
+    (1, 2560, 63104, False), (2, 6144, 30336, False), (2, 4608, 34176, True), (2, 6656, 27392, True), (2, 2688, 56064, True),
+    (2, 3456, 47232, False), (1, 2944, 55296, True), (3, 2048, 65536, False), (3, 3840, 33792, True), (4, 2048, 65536, True), (4, 9728, 13824, True)])
+def test_one_row_of_light_layers_takes_half_blocks_where_they_balance(lib, k, n_in, n_out, half):
+    """Up to K = 3 half blocks come in workgroups of eight only where they fill the chip in fewer rounds than the whole ones."""
     _, tile_rows, _, _ = _plan(lib, 1, n_in, n_out, k)
     assert (tile_rows == 4) == half
 
