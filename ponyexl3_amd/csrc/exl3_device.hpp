@@ -64,9 +64,8 @@ enum : int { CB_3INST = 0, CB_MCG = 1, CB_MUL1 = 2 };
 // result is the fp16 sum of the two halves of x (one rounding).
 //
 // MUL1: x = cw*0x83DCD12D; h = 1024 + (sum of the four bytes of x);
-// result = fp16(h * K_INV + K_BIAS). h*K_INV + K_BIAS is an integer multiple of
-// 2^-18 below 2^4, hence exact in fp32, so the single fp32->fp16 conversion is
-// the only rounding (the reference rounds once from double).
+// result = fp16(h * K_INV + K_BIAS), rounded once (the reference rounds once from
+// double): h, K_INV and K_BIAS are fp16 values and v_pk_fma_f16 rounds the exact result.
 //
 // Instruction choice follows measured gfx950 issue rates: v_mul_lo_u32 and
 // v_mad_u64_u32 run at the full 16 lanes/clk/SIMD, v_bitop3_b32 at the faster
@@ -123,11 +122,15 @@ __device__ __forceinline__ void add_halves_pack2(uint32_t x0, uint32_t x1, uint3
     rb = bits_to_half2(b);
 }
 
-__device__ __forceinline__ half_t decode_mul1(uint32_t cw) {
-    const uint32_t x = cw * 0x83DCD12Du;
-    const uint32_t s = __builtin_amdgcn_sad_u8(x, 0u, 1024u);
-    const float v = __builtin_fmaf((float)s, 0.00676727294921875f, -10.3828125f);
-    return (half_t)v;
+// Two MUL1 codewords -> a packed pair. v_sad_u8 adds the four bytes of a product onto the fp16
+// bits of 1024 (0x6400: steps of one up to 2047) in the lower half, v_sad_hi_u8 in the upper one, and one
+// packed fma rounds once: 2.5 instructions a weight after the bit window. Through 32 bits (byte sum,
+// conversion, fma, conversion, packing) it was 5.5.
+__device__ __forceinline__ half2_t decode_mul1_pair(uint32_t cw0, uint32_t cw1) {
+    const uint32_t s = __builtin_amdgcn_sad_u8(cw0 * 0x83DCD12Du, 0u, 0x64006400u);
+    const half2_t h = bits_to_half2(__builtin_amdgcn_sad_hi_u8(cw1 * 0x83DCD12Du, 0u, s));
+    return __builtin_elementwise_fma(h, half2_t{(half_t)0.00676727294921875f, (half_t)0.00676727294921875f},
+                                     half2_t{(half_t)-10.3828125f, (half_t)-10.3828125f});
 }
 
 // Four codewords -> two packed pairs of fp16 weights (cw0, cw1) and (cw2, cw3).
@@ -135,26 +138,22 @@ template <int CB>
 __device__ __forceinline__ void decode_pair2(uint32_t cw0, uint32_t cw1, uint32_t cw2,
                                              uint32_t cw3, half2_t& ra, half2_t& rb) {
     if constexpr (CB == CB_MUL1) {
-        ra.x = decode_mul1(cw0);
-        ra.y = decode_mul1(cw1);
-        rb.x = decode_mul1(cw2);
-        rb.y = decode_mul1(cw3);
+        ra = decode_mul1_pair(cw0, cw1);
+        rb = decode_mul1_pair(cw2, cw3);
     } else {
         add_halves_pack2(scramble<CB>(cw0), scramble<CB>(cw1), scramble<CB>(cw2),
                          scramble<CB>(cw3), ra, rb);
     }
 }
 
-// One codeword -> the dword whose two fp16 halves add up to the weight (3INST / MCG:
-// the scrambled word itself; MUL1: the weight and a zero). A dot product is linear, so
-// a kernel that feeds both halves to the matrix pipe as two k-slots against the same
-// activation gets a * lo + a * hi in fp32 - the product with the exact sum of the two
-// halves, which the fp16 weight is the rounding of - and saves the half add.
+// One codeword of 3INST or MCG -> the dword whose two fp16 halves add up to the weight, i.e. the
+// scrambled word itself. A dot product is linear, so a kernel that feeds both halves to the matrix
+// pipe as two k-slots against the same activation gets a * lo + a * hi in fp32 - the product with
+// the exact sum of the two halves, which the fp16 weight is the rounding of - and saves the half
+// add. MUL1 has no halves: its weight comes rounded from the packed fma, and every kernel takes
+// it as such.
 template <int CB>
-__device__ __forceinline__ uint32_t weight_halves(uint32_t cw) {
-    if constexpr (CB == CB_MUL1) return (uint32_t)half_to_bits(decode_mul1(cw));
-    else return scramble<CB>(cw);
-}
+constexpr bool kHasHalves = CB != CB_MUL1;
 
 // The K+1 dwords a lane needs for its 32 codewords: w[0] is the dword that
 // precedes the lane's own K dwords (already wrapped), w[1..K] are its own.

@@ -64,8 +64,7 @@ __device__ __forceinline__ void decode_half_quad(const LaneWords<K>& lw, uint32_
     constexpr int na = 4 * (2 * I + CS), nb = na + 2;
     static_assert(cw_col_sel(na) == CS && cw_row(na) == 2 * I && cw_row(nb) == 2 * I + 8);
     if constexpr (CB == CB_MUL1) {
-        wp[H][I].x = decode_mul1(lane_codeword<K, na + 2 * H>(lw));
-        wp[H][I].y = decode_mul1(lane_codeword<K, na + 2 * H + 1>(lw));
+        wp[H][I] = decode_mul1_pair(lane_codeword<K, na + 2 * H>(lw), lane_codeword<K, na + 2 * H + 1>(lw));
     } else if constexpr (H == 0) {
         x[0] = scramble<CB>(lane_codeword<K, na>(lw));
         x[1] = scramble<CB>(lane_codeword<K, na + 1>(lw));

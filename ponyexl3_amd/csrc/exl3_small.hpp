@@ -98,13 +98,13 @@ __device__ __forceinline__ void dot_tile_row(const LaneWords<K>& lw, LoadChunk&&
         constexpr int t = tc.value, c = step_chunk(t), cs = t & 1;
         constexpr int n0 = pair_n(2 * c, cs), n1 = pair_n(2 * c + 1, cs);
         static_assert(cw_col_sel(n0) == cs && cw_row(n0) == 4 * c && cw_row(n1) == 4 * c + 2, "pair order");
-        wb[t].x = weight_halves<CB>(lane_codeword<K, n0>(lw));
-        wb[t].y = weight_halves<CB>(lane_codeword<K, n0 + 1>(lw));
+        wb[t].x = scramble<CB>(lane_codeword<K, n0>(lw));
+        wb[t].y = scramble<CB>(lane_codeword<K, n0 + 1>(lw));
         if constexpr (t >= 1) issue(std::integral_constant<int, t - 1>{});
         if constexpr (t == 2) xc[1] = load_chunk(1);  // chunk 0 has just been used up
         if constexpr (t == 4) xc[3] = load_chunk(3);  // chunk 2 likewise
-        wb[t].z = weight_halves<CB>(lane_codeword<K, n1>(lw));
-        wb[t].w = weight_halves<CB>(lane_codeword<K, n1 + 1>(lw));
+        wb[t].z = scramble<CB>(lane_codeword<K, n1>(lw));
+        wb[t].w = scramble<CB>(lane_codeword<K, n1 + 1>(lw));
     });
     issue(std::integral_constant<int, 7>{});
 }
@@ -178,13 +178,14 @@ __device__ __forceinline__ void issue_first_rows(const uint32_t* __restrict__ ba
     }
 }
 
-template <int K, int CB, int MT, bool ROTATE, bool HALF, bool GUARD, bool EXACT = false>
+template <int K, int CB, int MT, bool ROTATE, bool HALF, bool GUARD, bool ROUNDED = false>
 __device__ __forceinline__ void stream_block_rows_at(const uint32_t* __restrict__ base,
                                                      size_t row_words, int tk_begin, int tk_end,
                                                      const half_t* const (&xrow)[MT], int rows,
                                                      const half_t* __restrict__ suh_row,
                                                      half_t (*xw)[kXwLd], int lane,
                                                      float (&acc)[MT][2]) {
+    constexpr bool EXACT = ROUNDED || !kHasHalves<CB>;
     uint32_t buf[kStreamSlots][K];
     half2_t xraw[MT], sraw;
     auto fetch_block = [&](int blk) {

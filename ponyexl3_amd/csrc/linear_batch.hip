@@ -28,17 +28,18 @@
 
 namespace exl3 {
 
-// R: batch rows that the kernel stages (4, 8 or 16); they take unsummed halves (4, 8) or rounded weights.
-template <int R>
+// R: batch rows that the kernel stages (4, 8 or 16); up to 8 take unsummed halves where the codebook has them.
+template <int R, int CB>
 struct BatchTile {
-    static constexpr bool EXACT = R > 8;
+    static constexpr bool EXACT = R > 8 || !kHasHalves<CB>;
     // Up to 8 rows v_mfma_f32_16x16x32_f16, four rows each; above v_mfma_f32_32x32x16_f16, whose 32
     // A rows serve 16 rows in both lane halves.
-    static constexpr int NQ = EXACT ? 1 : R / 4;
-    typedef float vec_t __attribute__((ext_vector_type(EXACT ? 16 : 4)));
+    static constexpr bool WIDE = R > 8;
+    static constexpr int NQ = WIDE ? 1 : R / 4;
+    typedef float vec_t __attribute__((ext_vector_type(WIDE ? 16 : 4)));
     struct acc_t {  // batch row m of a column
         vec_t v[NQ];
-        __device__ __forceinline__ float row(int m) const { return EXACT ? v[0][m] : v[m >> 2][m & 3]; }
+        __device__ __forceinline__ float row(int m) const { return WIDE ? v[0][m] : v[m >> 2][m & 3]; }
     };
     // halfs per staged row: the 64 values of a half block (unsummed: each twice) and 16 bytes, so that
     // consecutive rows start four LDS banks apart
@@ -46,7 +47,7 @@ struct BatchTile {
     // Where lane `lane` reads its share of A: k-slots of group (lane >> 4 or >> 5) in A row i hold the
     // batch row whose sums land in that group's lanes, zeros (row R) elsewhere.
     static __device__ __forceinline__ int operand_row(int lane, int part) {
-        if constexpr (!EXACT) {
+        if constexpr (!WIDE) {
             const int i = lane & 15, m = 4 * part + (i & 3);
             return (i >> 2) == (lane >> 4) ? m : R;
         } else {
@@ -57,7 +58,7 @@ struct BatchTile {
     static __device__ __forceinline__ void mfma(const uint4_t (&a)[NQ], uint4_t b, acc_t& c) {
 #pragma unroll
         for (int i = 0; i < NQ; i++) {
-            if constexpr (!EXACT)
+            if constexpr (!WIDE)
                 c.v[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[i]),
                                                                 __builtin_bit_cast(half8_t, b), c.v[i], 0, 0, 0);
             else
@@ -76,8 +77,8 @@ template <int K, int CB, int R>
 __device__ __forceinline__ void batch_main(const uint32_t* __restrict__ base, size_t row_words, int tk,
                                            const half_t* __restrict__ x, int in_features, int rows,
                                            const half_t* __restrict__ suh, half_t* xw, int lane,
-                                           typename BatchTile<R>::acc_t (&acc)[2]) {
-    using T = BatchTile<R>;
+                                           typename BatchTile<R, CB>::acc_t (&acc)[2]) {
+    using T = BatchTile<R, CB>;
     constexpr bool EXACT = T::EXACT;
     const int blk = (tk >> 3) * 128, upper = (tk >> 2) & 1;
     constexpr int kSlots = kStreamSlots;
@@ -100,7 +101,7 @@ __device__ __forceinline__ void batch_main(const uint32_t* __restrict__ base, si
     };
     // xw rows = this half of fp16(had128(x * suh) / sqrt(128))   (ponyexl3/ref/forward.py:32-34).
     // Activations are requested first: loads return in issue order (see stream_block_rows_at).
-    if constexpr (!EXACT) {
+    if constexpr (R <= 8) {
         // lane = (row fr, elements E q .. E q + E - 1)
         constexpr int E = 2 * R;
         const int fr = lane & (R - 1), q = lane / R;
@@ -259,13 +260,13 @@ __device__ __forceinline__ void batch_main(const uint32_t* __restrict__ base, si
                 constexpr int t = tc.value, c = step_chunk(t), cs = t & 1;
                 constexpr int n0 = pair_n(2 * c, cs), n1 = pair_n(2 * c + 1, cs);
                 static_assert(cw_col_sel(n0) == cs && cw_row(n0) == 4 * c && cw_row(n1) == 4 * c + 2);
-                wb[t].x = weight_halves<CB>(lane_codeword<K, n0>(lw));
-                wb[t].y = weight_halves<CB>(lane_codeword<K, n0 + 1>(lw));
+                wb[t].x = scramble<CB>(lane_codeword<K, n0>(lw));
+                wb[t].y = scramble<CB>(lane_codeword<K, n0 + 1>(lw));
                 if constexpr (t >= 1) issue(std::integral_constant<int, t - 1>{});
                 if constexpr (t == 2) xc[1] = chunk(s, 1);
                 if constexpr (t == 4) xc[3] = chunk(s, 3);
-                wb[t].z = weight_halves<CB>(lane_codeword<K, n1>(lw));
-                wb[t].w = weight_halves<CB>(lane_codeword<K, n1 + 1>(lw));
+                wb[t].z = scramble<CB>(lane_codeword<K, n1>(lw));
+                wb[t].w = scramble<CB>(lane_codeword<K, n1 + 1>(lw));
             });
             issue(std::integral_constant<int, 7>{});
         }
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
     const half_t* __restrict__ svh, const half_t* __restrict__ bias, half_t* __restrict__ y, float* partial,
     int* counters, const int* __restrict__ group_sub, int in_tiles, int out_tiles, int rows, int n_groups,
     int* status, int spin_limit) {
-    using T = BatchTile<R>;
+    using T = BatchTile<R, CB>;
     constexpr int MR = (R + NW - 1) / NW;  // batch rows per wave in the reduction: wave, wave + NW, ...
     constexpr size_t kXsBytes = sizeof(half_t) * NW * (R + 1) * T::LD;
     constexpr size_t kRedBytes = sizeof(float) * NW * R * 128;
@@ -328,8 +329,8 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
 #pragma unroll
         for (int i = 0; i < T::NQ; i++) {
 #pragma unroll
-            for (int c = 0; c < (T::EXACT ? 16 : 4); c++) acc[cs].v[i][c] = 0.f;
-            if constexpr (!T::EXACT) asm("" : "+a"(acc[cs].v[i]));  // as keep_in_agprs()
+            for (int c = 0; c < (T::WIDE ? 16 : 4); c++) acc[cs].v[i][c] = 0.f;
+            if constexpr (!T::WIDE) asm("" : "+a"(acc[cs].v[i]));  // as keep_in_agprs()
         }
     if (split < n_splits)
         batch_main<K, CB, R>(trellis + (size_t)g * 8 * (8 * K) + lane * K, (size_t)out_tiles * (8 * K), split * 4, x,

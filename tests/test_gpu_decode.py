@@ -34,6 +34,18 @@ def test_random_trellis_bit_exact(cuda, oracle, k, cb):
     np.testing.assert_array_equal(w.view(np.uint16), oracle.decode_trellis(tr, k, cb).view(np.uint16))
 
 
+@pytest.mark.parametrize("cb", [0, 1, 2])
+def test_every_codeword_bit_exact(cuda, oracle, cb):
+    """All 65 536 codewords, in both halves of the packed pairs that the kernels decode: at K = 8 a
+    codeword is two neighbouring bytes, and tiles i, 0, i, 1, ... hold every pair in either order."""
+    j = np.arange(256).reshape(2, 128)
+    encoded = np.stack([np.stack([np.full_like(j, i), j], axis=-1).reshape(2, 256) for i in range(256)])
+    tr = oracle.pack_trellis(encoded.reshape(16, 32, 256).astype(np.uint16), 8)
+    assert len(np.unique(oracle.unpack_trellis(tr, 8))) == 65536
+    w = _decode(tr, 8, cb, cuda)
+    np.testing.assert_array_equal(w.view(np.uint16), oracle.decode_trellis(tr, 8, cb).view(np.uint16))
+
+
 def test_column_slices(cuda, oracle):
     rng = np.random.default_rng(5)
     tr = rng.integers(0, 65536, size=(4, 19, 80), dtype=np.uint16)
