@@ -127,17 +127,24 @@ __global__ __launch_bounds__(256) void decode_full_t_kernel(const uint32_t* __re
 // over the rows of the block:
 //   Y[i][n] = fp16(sum_j +-q_i W[j][n]),   Z[i][m] = fp16(sum_n +-Y[i][n] / sqrt(128) * svh_m)
 // Both run on the matrix pipe (v_mfma_f32_16x16x32_f16, fp32 sums in the order of the
-// prefill GEMM), the fragments of H made from sign words each lane holds. For 5120 x 17408 at
-// K = 4 VALU issue (decode, signs, conversions) takes 35 us of a SIMD's time, the matrix pipe 18,
-// and a plain fill of the result would take 26: no unit is full. What the kernel waits for is its own
-// sequence, load, decode, transform, transform, store, with five barriers between and no load of the
-// next block in flight (waves wait half of their time). The result goes out through LDS in
-// 256-byte row pieces, non-temporal (nobody reads it soon; 65 -> 62 us). One 34 KiB LDS tile serves
-// all three stages (each stage reads its operands into registers before the next one writes), so four
-// workgroups share a CU and their phases overlap.
-// Measured, 5120 x 17408 at K = 4, transposed: 60 us (3.7 TB/s of trellis and result); the
-// identity through the prefill kernels, the concatenation of its column stripes and the
-// transposed copy took 1.42 ms.
+// prefill GEMM), the fragments of H made from sign words each lane holds. The decoded weights are
+// operands of the first product without a trip through LDS: a wave takes 32 columns over all 128 rows, its
+// loads put neighbouring pairs of tile rows on lane bits 4 and 5, and one exchange of 16-lane rows a
+// register brings rows 0..7 and 8..15 of a tile into the lanes that the operand wants them in.
+// For 5120 x 17408 at K = 4 VALU issue (decode, signs, conversions: 730 instructions a wave) takes 30 us of a SIMD's
+// time, the matrix pipe 18, and a plain fill of the result would take 26: no unit is full; what is left are the phases of
+// a workgroup, of which four share a CU (one 34 KiB LDS tile, 128 registers): decode and first product, second
+// product, store, with three barriers between. The result goes out through LDS in 256-byte row pieces,
+// non-temporal (nobody reads it soon).
+// Measured, us, transposed: decoded weights through LDS (five barriers, scales loaded where they are used, a wait
+// each) -> operands from registers, scales in front -> words of the next block requested ahead:
+//   5120 x 17408 K = 2 / 4 / 8: 63.5 / 65.5 / 71.6 -> 56.3 / 56.5 / 63.1 -> 54.0 / 52.8 / 55.6 (4.2 TB/s of trellis and
+//   result at K = 4), not transposed K = 4 69.7 -> 58.5 -> 54.2; 2048 x 2048 7.4 -> 5.7 -> 5.8.
+// The identity through the prefill kernels, the concatenation of its column stripes and the transposed copy took 1420.
+//
+// Workgroups that start together: 256 CUs of four. The one this many places on gets the place of this one, and as a
+// multiple of eight on the same XCD, whose L2 then has its words.
+constexpr unsigned kPubAhead = 1024;
 constexpr int kPubLd = 128 + kDecPad;  // halfs per row: 16-byte reads of 16 rows hit all banks
 
 // Signs of a fragment of H128 for rows / columns 16 nt + fr and k = 32 ks + 8 q + 0..7: entry
@@ -167,104 +174,119 @@ struct HadamardFragments {
 };
 
 template <int K, int CB, bool T>
-__global__ __launch_bounds__(256, 3) void public_weight_kernel(
+__global__ __launch_bounds__(256, 4) void public_weight_kernel(
     const uint32_t* __restrict__ trellis, const half_t* __restrict__ suh,
     const half_t* __restrict__ svh, half_t* __restrict__ w_out, int out_tiles, int tn_offset,
     int blocks_fast, size_t ldw) {
     constexpr float kScale = 0.088388347648318440550f;  // 1/sqrt(128)
     __shared__ __attribute__((aligned(16))) half_t tile[128 * kPubLd];
+    __shared__ __attribute__((aligned(16))) float sv_s[128];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int fr = lane & 15, q = lane >> 4;
     // consecutive workgroups write consecutive pieces of the same output rows
     const int fast = blockIdx.x % blocks_fast, slow = blockIdx.x / blocks_fast;
     const int bi = T ? fast : slow, bn = T ? slow : fast;
 
-    // decode: wave w takes tile rows 2w, 2w + 1; a lane's two columns go to tile[n][j], 16
-    // consecutive j (pairs {2cs + hh + 4t, t = 0..3} are rows 8hh..8hh+7 of column cs)
-    {
-        uint32_t own[2][K];
+    // Wave w takes columns 32w .. 32w + 31, i.e. two tile columns (lane bit 3) of all eight tile rows: 4r + 2 (lane
+    // bit 4) + (lane bit 5) in load r.
+    uint32_t own[2][K];
 #pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const uint32_t* p = trellis + ((size_t)(bi * 8 + 2 * wave + r) * out_tiles + tn_offset + bn * 8) * (8 * K) +
-                                lane * K;
+    for (int r = 0; r < 2; r++) {
+        const uint32_t* p = trellis +
+                            ((size_t)(bi * 8 + 4 * r + (lane >> 3 & 2) + (lane >> 5)) * out_tiles + tn_offset + bn * 8 + 2 * wave +
+                             (lane >> 3 & 1)) * (8 * K) + (lane & 7) * K;
 #pragma unroll
-            for (int i = 0; i < K; i++) own[r][i] = __builtin_nontemporal_load(p + i);
-        }
-        const int n0 = (lane >> 3) * 16 + (lane & 7);
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const LaneWords<K> lw = finish_lane_words<K>(own[r], lane);
-            half2_t wp[16];
-            decode_lane<K, CB>(lw, wp);
-#pragma unroll
-            for (int cs = 0; cs < 2; cs++)
-#pragma unroll
-                for (int hh = 0; hh < 2; hh++) {
-                    const half2_t* c = wp + 8 * cs + 4 * hh;
-                    *reinterpret_cast<uint4_t*>(tile + (n0 + 8 * cs) * kPubLd + (2 * wave + r) * 16 + 8 * hh) =
-                        uint4_t{half2_to_bits(c[0]), half2_to_bits(c[1]), half2_to_bits(c[2]), half2_to_bits(c[3])};
-                }
-        }
+        for (int i = 0; i < K; i++) own[r][i] = __builtin_nontemporal_load(p + i);
     }
-    __syncthreads();
+    // one dword of each 128-byte line of the words of the block ahead
+    uint32_t ahead = 0;
+    {
+        const unsigned nb = blockIdx.x + kPubAhead;
+        const int nfast = nb % blocks_fast, nslow = nb / blocks_fast;
+        const int ni = T ? nfast : nslow, nn = T ? nslow : nfast;
+        constexpr int kLines = 2 * K;  // of a tile row
+        if (nb < gridDim.x && lane < 2 * kLines)
+            ahead = trellis[((size_t)(ni * 8 + 2 * wave + lane / kLines) * out_tiles + tn_offset + nn * 8) * (8 * K) +
+                            lane % kLines * 32];
+    }
+    // scales: one branch and one wait each, in front of everything that needs them
+    half_t su[8];
+    if (suh) {
+#pragma unroll
+        for (int nt = 0; nt < 8; nt++) su[nt] = suh[bi * 128 + nt * 16 + fr];
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < 8; nt++) su[nt] = (half_t)1.0f;
+    }
+    if (threadIdx.x < 128) sv_s[threadIdx.x] = svh ? (float)svh[bn * 128 + threadIdx.x] : 1.0f;
     const HadamardFragments had(lane);
-    half8_t op[2][4];
-    float4_t acc[2][8];
-    auto read_operands = [&] {  // rows 32 wave .. + 31 of the tile, all 128 k
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++)
-#pragma unroll
-            for (int ks = 0; ks < 4; ks++)
-                op[rt][ks] = *reinterpret_cast<const half8_t*>(tile + (wave * 32 + rt * 16 + fr) * kPubLd + ks * 32 + q * 8);
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++)
-#pragma unroll
-            for (int nt = 0; nt < 8; nt++) acc[rt][nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-    };
 
+    // A lane has rows 0..7 and 8..15 of its tile; the exchange of 16-lane rows makes of the two tile rows that lane
+    // bit 4 tells apart two operands of 32 rows, k = 8 q + t (column u + 8 cs of tile column lane >> 3 & 1 in
+    // operand row lane & 15).
+    half8_t w[4][2];  // [32-row step][cs]
+    static_for<0, 2>([&](auto r) {
+        const LaneWords<K> lw = finish_lane_words<K>(own[r.value], lane);
+        half2_t wp[16];
+        decode_lane<K, CB>(lw, wp);
+#pragma unroll
+        for (int cs = 0; cs < 2; cs++) {
+            uint4_t lo, hi;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const auto x = __builtin_amdgcn_permlane16_swap(half2_to_bits(wp[8 * cs + i]), half2_to_bits(wp[8 * cs + 4 + i]), false, false);
+                lo[i] = x[0];
+                hi[i] = x[1];
+            }
+            w[2 * r.value][cs] = __builtin_bit_cast(half8_t, lo);
+            w[2 * r.value + 1][cs] = __builtin_bit_cast(half8_t, hi);
+        }
+    });
     // Y^T[n][i] = sum_j W^T[n][j] H[j][i]: a lane gets four consecutive n of one i
-    read_operands();
-    __syncthreads();
     static_for<0, 8>([&](auto nt) {
-        const float su = suh ? (float)suh[bi * 128 + nt.value * 16 + fr] : 1.0f;
-        const uint32_t qi = half_to_bits((half_t)__fmul_rn(su, kScale)) * 0x10001u;
+        const uint32_t qi = half_to_bits((half_t)__fmul_rn((float)su[nt.value], kScale)) * 0x10001u;
+        float4_t y[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
         static_for<0, 4>([&](auto ks) {
             const half8_t h = had.template get<nt.value, ks.value>(qi);
 #pragma unroll
-            for (int rt = 0; rt < 2; rt++)
-                acc[rt][nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(op[rt][ks.value], h,
-                                                                           acc[rt][nt.value], 0, 0, 0);
+            for (int cs = 0; cs < 2; cs++)
+                y[cs] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[ks.value][cs], h, y[cs], 0, 0, 0);
         });
 #pragma unroll
-        for (int rt = 0; rt < 2; rt++) {
+        for (int cs = 0; cs < 2; cs++) {
             half4_t o;
 #pragma unroll
-            for (int c = 0; c < 4; c++) o[c] = (half_t)acc[rt][nt.value][c];
-            *reinterpret_cast<half4_t*>(tile + (nt.value * 16 + fr) * kPubLd + wave * 32 + rt * 16 + q * 4) = o;
+            for (int c = 0; c < 4; c++) o[c] = (half_t)y[cs][c];
+            *reinterpret_cast<half4_t*>(tile + (nt.value * 16 + fr) * kPubLd + wave * 32 + (q >> 1) * 16 + cs * 8 + (q & 1) * 4) = o;
         }
     });
+    asm volatile("" ::"v"(ahead));  // (its wait: long there)
     __syncthreads();
 
     // Z: a lane gets four consecutive i of one m (T) or four consecutive m of one i
-    read_operands();
+    half8_t op[2][4];  // rows 32 wave .. + 31 of the tile, all 128 k
+#pragma unroll
+    for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+            op[rt][ks] = *reinterpret_cast<const half8_t*>(tile + (wave * 32 + rt * 16 + fr) * kPubLd + ks * 32 + q * 8);
     __syncthreads();
+    float4_t acc[2][8];
     static_for<0, 4>([&](auto ks) {
         static_for<0, 8>([&](auto nt) {
             const half8_t h = had.template get<nt.value, ks.value>(0x3C003C00u);
 #pragma unroll
             for (int rt = 0; rt < 2; rt++)
                 acc[rt][nt.value] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                    T ? op[rt][ks.value] : h, T ? h : op[rt][ks.value], acc[rt][nt.value], 0, 0, 0);
+                    T ? op[rt][ks.value] : h, T ? h : op[rt][ks.value],
+                    ks.value == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : acc[rt][nt.value], 0, 0, 0);
         });
     });
-    const half_t* sv = svh ? svh + bn * 128 : nullptr;
 #pragma unroll
     for (int nt = 0; nt < 8; nt++) {
-        float s[4] = {1.f, 1.f, 1.f, 1.f};
-        if (sv) {
+        float s[4];
 #pragma unroll
-            for (int c = 0; c < 4; c++) s[c] = (float)(T ? sv[nt * 16 + fr] : sv[nt * 16 + q * 4 + c]);
-        }
+        for (int c = 0; c < 4; c++) s[c] = sv_s[T ? nt * 16 + fr : nt * 16 + q * 4 + c];
 #pragma unroll
         for (int rt = 0; rt < 2; rt++) {
             half4_t o;

@@ -69,6 +69,34 @@ def test_public_weight_slices_and_transpose(cuda, oracle, k, cb, n_in, n_out):
     assert rel_l2(plain.cpu().numpy(), oracle.reconstruct_public_weights(tr, one_in, one_out, k, cb)) < 1e-3
 
 
+@pytest.mark.parametrize("cb", [0, 1, 2])
+@pytest.mark.parametrize("k", range(1, 9))
+def test_public_weight_against_decoded_weights(cuda, k, cb):
+    """One block, and more blocks than start together (each asks for the words of one 1024 places on): the
+    bit-exact decoded weights under both transforms in 64 bits, with the two fp16 casts. A sum of 128 in fp32 is off by
+    up to 2^-20, which moves fewer than one cast in a hundred by a step of 2^-11: 2^-14 of the norm; 2^-13 asked."""
+    from ponyexl3_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(8 * cb + k)
+    i = torch.arange(128, device=cuda)
+    parity = (i[:, None] & i[None, :]).cpu().apply_(lambda v: bin(v).count("1") & 1).to(cuda)
+    had = (1 - 2 * parity).double()
+    for n_in, n_out in ((128, 128), (384, 128 * 345)):
+        print(f"public weight k={k} cb={cb} {n_in}x{n_out}", flush=True)
+        tr = torch.randint(-32768, 32768, (n_in // 16, n_out // 16, 16 * k), dtype=torch.int16, device=cuda, generator=g)
+        suh = torch.randn(n_in, device=cuda, generator=g).half()
+        svh = (0.02 * torch.randn(n_out, device=cuda, generator=g)).half()
+        w = ops.decode_full(tr, k, cb).double().view(n_in // 128, 128, n_out // 128, 128).transpose(1, 2)
+        q = (suh.float() * 0.08838834764831845).half().double().view(n_in // 128, 1, 128, 1)
+        y = (q * had.matmul(w)).half().double()
+        z = (y.matmul(had) * 0.08838834764831845 * svh.double().view(1, n_out // 128, 1, 128)).half()
+        ref = z.transpose(1, 2).reshape(n_in, n_out).double()
+        for transposed in (False, True):
+            got = ops.public_weight(tr, k, cb, suh, svh, transposed=transposed).double()
+            got = got.T if transposed else got
+            assert float((got - ref).norm() / ref.norm()) < 2.0 ** -13
+
+
 @pytest.mark.parametrize("bias", [False, True])
 def test_folded_linear_tracks_exact_layer(cuda, oracle, bias):
     from ponyexl3_amd import make_exl3_layer, native
