@@ -278,11 +278,8 @@ __device__ __forceinline__ void batch_main(const uint32_t* __restrict__ base, si
 // Output transform of MR rows of a 128-column block, two columns per lane: the fp16 cast at
 // ponyexl3/ref/forward.py:41, Hadamard, svh, bias (forward.py:42-45).
 template <int MR>
-__device__ __forceinline__ void batch_finish(float (&a)[MR], float (&b)[MR], const half_t* svh, const half_t* bias,
-                                             size_t col, int lane, half2_t (&o)[MR]) {
-    half2_t sv, bv;
-    if (svh) sv = half2_t{svh[col], svh[col + 1]};
-    if (bias) bv = half2_t{bias[col], bias[col + 1]};
+__device__ __forceinline__ void batch_finish(float (&a)[MR], float (&b)[MR], bool svh, half2_t sv, bool bias, half2_t bv,
+                                             int lane, half2_t (&o)[MR]) {
 #pragma unroll
     for (int i = 0; i < MR; i++) {
         a[i] = (float)(half_t)a[i];
@@ -336,6 +333,11 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
         batch_main<K, CB, R>(trellis + (size_t)g * 8 * (8 * K) + lane * K, (size_t)out_tiles * (8 * K), split * 4, x,
                              in_features, rows, suh ? suh + (size_t)sub * in_features : nullptr,
                              reinterpret_cast<half_t*>(smem) + wave * (R + 1) * T::LD, lane, acc);
+    // requested now, needed only by the finishing workgroup: by then they are here
+    const size_t col = (size_t)g * 128 + 2 * lane;
+    half2_t sv, bv;
+    if (svh) sv = half2_t{svh[col], svh[col + 1]};
+    if (bias) bv = half2_t{bias[col], bias[col + 1]};
     const int c0 = (lane >> 3) * 16 + (lane & 7);
     __syncthreads();  // nobody reads staged activations any more
 #pragma unroll
@@ -345,7 +347,6 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
     }
     __syncthreads();
     const size_t out_total = (size_t)n_groups * 128;
-    const size_t col = (size_t)g * 128 + 2 * lane;
     const int wg_splits = (n_splits + NW - 1) / NW;  // partial rows per group
     float va[MR], vb[MR];
 #pragma unroll
@@ -417,7 +418,7 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
             va[i] = fix_value(w0[i], bits);
             vb[i] = fix_value(w1[i], bits);
         }
-        batch_finish<MR>(va, vb, svh, bias, col, lane, o);
+        batch_finish<MR>(va, vb, svh, sv, bias, bv, lane, o);
 #pragma unroll
         for (int i = 0; i < MR; i++) {
             if (bad) o[i].x = o[i].y = bits_to_half(0x7E00);
@@ -469,7 +470,7 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
                     }
                 }
         }
-        batch_finish<MR>(va, vb, svh, bias, col, lane, o);
+        batch_finish<MR>(va, vb, svh, sv, bias, bv, lane, o);
 #pragma unroll
         for (int i = 0; i < MR; i++) {
             const int m = wave + NW * i;

@@ -225,8 +225,7 @@ __device__ __forceinline__ void moe_finish_block(float2_t sum, half2_t sv, int l
 }
 
 // Routing by the expert kernel itself, from the router's logits: 3.4 us in front of the first weights
-// (8.0 -> 11.4 us) where a launch of its own in between takes 4.0 us and a gap of about 1, and 3.5 us of host time. Every wave finds the expert of its slot;
-// the first workgroup of a token writes the token's row of the routing table for the launch behind.
+// (8.0 -> 11.4 us) where a launch of its own in between takes 4.0 us and a gap of about 1, and 3.5 us of host time. Every wave finds the expert of its slot.
 // logits == nullptr: the table is there.
 constexpr int kInlineRouteExperts = 256;  // four per lane
 struct MoeRoute {
@@ -236,20 +235,25 @@ struct MoeRoute {
     half_t* scores;  // fp16 [tokens][top_k], top_k with the shared expert
 };
 
-__device__ __forceinline__ int moe_route_slot(const MoeRoute& r, int s, int top_k, int* indices, bool writes, int lane) {
+__device__ __forceinline__ int moe_route_slot(const MoeRoute& r, int s, int top_k, bool writes, int lane, RouteChoice& c) {
     const int t = s / top_k, j = s - t * top_k, ranked = top_k - (r.shared_logits != nullptr);
+    if (j == ranked && !writes) return r.n_experts;  // the shared expert
     int key[kInlineRouteExperts / 64];
     route_probabilities<half_t>(r.logits + (size_t)t * r.n_experts, r.n_experts, lane, key);
-    RouteChoice c{0.f, 0};
-    int e = r.n_experts;  // the shared expert
-    const int rounds = writes ? ranked : min(j + 1, ranked);
+    int e = r.n_experts;
+    const int rounds = writes ? ranked : j + 1;
     for (int i = 0; i < rounds; i++) {
         const int chosen = route_next(key, lane, i, c);
         if (i == j) e = chosen;
     }
-    if (writes) route_write<half_t>(c, lane, t, r.n_experts, ranked, r.norm, r.shared_logits != nullptr,
-                                     r.shared_logits ? r.shared_logits[t] : (half_t)0.f, indices, r.scores);
     return e;
+}
+
+// The token's row of the table, for the launch behind: by the first workgroup of its last slot, which has chosen them all.
+__device__ __forceinline__ void moe_route_write(const MoeRoute& r, RouteChoice c, int t, int top_k, int* indices, int lane) {
+    const bool shared = r.shared_logits != nullptr;
+    route_write<half_t>(c, lane, t, r.n_experts, top_k - shared, r.norm, shared, shared ? r.shared_logits[t] : (half_t)0.f,
+                        indices, r.scores);
 }
 
 // Weighted sum over the slots of a token by the wave that stores the last of them: one 128-column block o of
@@ -406,10 +410,19 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
     const int gid = blockIdx.x;
     const int hg = gid % hblocks, s = gid / hblocks;
     const int p = wave >> 2, j = wave & 3;
-    const int e = clamp_expert(
-        route.logits ? moe_route_slot(route, s, top_k, indices, blockIdx.y == 0 && hg == 0 && wave == 0 && s % top_k == 0, lane)
-                     : indices[s],
-        E);
+    const bool writes = route.logits && blockIdx.y == 0 && hg == 0 && wave == 0 && s % top_k == top_k - 1;
+    RouteChoice choice{0.f, 0};
+    const int e = clamp_expert(route.logits ? moe_route_slot(route, s, top_k, writes, lane, choice) : indices[s], E);
+    // scales of what follows the reduction, requested now: behind it each would be a trip to memory that nothing hides.
+    // (block of 8 of 256 experts of 2048 x 512, with those of the down projection and the table's row written behind the weights: 1 token 21.5 -> 20.9
+    // us, with a shared expert 24.5 -> 24.2)
+    half2_t svg, svu, ds;
+    if (wave == 0) {
+        const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
+        svg = *reinterpret_cast<const half2_t*>(svh_e);
+        svu = *reinterpret_cast<const half2_t*>(svh_e + H);
+        ds = *reinterpret_cast<const half2_t*>(dn_suh + (size_t)e * H + hg * 128 + 2 * lane);
+    }
     const int blk = HALF ? blockIdx.y * 2 + (j >> 1) : blockIdx.y * 4 + j;
     const int tk0 = blk * 8 + (HALF ? (j & 1) * 4 : 0);
     float acc[1][2] = {{0.f, 0.f}};
@@ -427,6 +440,7 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
     red[wave][c0 + 8] = acc[0][1];
     __syncthreads();
     if (wave != 0) return;
+    if (writes) moe_route_write(route, choice, s / top_k, top_k, indices, lane);
     const int bits = fix_count_bits(n_chunks);
     // word q of a lane: projection q >> 1, column 2*lane + (q & 1); wave order within a projection
     unsigned long long w[4];
@@ -469,16 +483,11 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
 #pragma unroll
     for (int q = 0; q < 4; q++)
         __hip_atomic_store(slot[q], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
     float g0, g1, u0, u1;
-    moe_finish_block(float2_t{fix_value(w[0], bits), fix_value(w[1], bits)},
-                     *reinterpret_cast<const half2_t*>(svh_e), lane, g0, g1);
-    moe_finish_block(float2_t{fix_value(w[2], bits), fix_value(w[3], bits)},
-                     *reinterpret_cast<const half2_t*>(svh_e + H), lane, u0, u1);
+    moe_finish_block(float2_t{fix_value(w[0], bits), fix_value(w[1], bits)}, svg, lane, g0, g1);
+    moe_finish_block(float2_t{fix_value(w[2], bits), fix_value(w[3], bits)}, svu, lane, u0, u1);
     const float h0 = (float)(half_t)glu_act(g0, u0, activation);
     const float h1 = (float)(half_t)glu_act(g1, u1, activation);
-    const half2_t ds =
-        *reinterpret_cast<const half2_t*>(dn_suh + (size_t)e * H + hg * 128 + 2 * lane);
     float a = h0 * (float)ds.x, b = h1 * (float)ds.y;
     wht128_lanes(a, b, lane);
     half2_t o;
@@ -504,6 +513,8 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
     const int gid = blockIdx.x;
     const int og = gid % dblocks, s = gid / dblocks;
     const int e = clamp_expert(indices[s], E);
+    half2_t sv;  // (requested now, as in moe_gateup_pair_kernel)
+    if (wave == 0) sv = *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);
     constexpr bool kHalf = NW == 8;
     const int part_idx = blockIdx.y * NW + wave;
     const int blk = kHalf ? part_idx >> 1 : part_idx;
@@ -532,8 +543,6 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
     } else if (wave != 0) {
         return;
     }
-    const half2_t sv =
-        *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);
     float o0, o1;
     moe_finish_block(v, sv, lane, o0, o1);
     half2_t o;
@@ -649,7 +658,10 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
     const size_t gid_r = ((size_t)sr * 2 + p) * hblocks + hg;
     if (!moe_publish(part + (gid_r * n_wg + blockIdx.y) * 128, v, counter, 2 * n_wg, lane)) return;
     asm volatile("" ::: "memory");
-    // both projections' partial rows in flight together
+    // both projections' partial rows in flight together, and the scales
+    const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
+    const half2_t svg = *reinterpret_cast<const half2_t*>(svh_e), svu = *reinterpret_cast<const half2_t*>(svh_e + H);
+    const half2_t ds = *reinterpret_cast<const half2_t*>(dn_suh + (size_t)e * H + hg * 128 + 2 * lane);
     const float* rows_g = part + (((size_t)sr * 2) * hblocks + hg) * n_wg * 128;
     const float* rows_u = part + (((size_t)sr * 2 + 1) * hblocks + hg) * n_wg * 128;
     float2_t sg{0.f, 0.f}, su{0.f, 0.f};
@@ -675,14 +687,11 @@ __global__ __launch_bounds__(NW * 64) void moe_gateup_grouped_kernel(
             }
         }
     }
-    const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
     float g0, g1, u0, u1;
-    moe_finish_block(sg, *reinterpret_cast<const half2_t*>(svh_e), lane, g0, g1);
-    moe_finish_block(su, *reinterpret_cast<const half2_t*>(svh_e + H), lane, u0, u1);
+    moe_finish_block(sg, svg, lane, g0, g1);
+    moe_finish_block(su, svu, lane, u0, u1);
     const float h0 = (float)(half_t)glu_act(g0, u0, activation);
     const float h1 = (float)(half_t)glu_act(g1, u1, activation);
-    const half2_t ds =
-        *reinterpret_cast<const half2_t*>(dn_suh + (size_t)e * H + hg * 128 + 2 * lane);
     float a = h0 * (float)ds.x, b = h1 * (float)ds.y;
     wht128_lanes(a, b, lane);
     half2_t o;
@@ -726,6 +735,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
         stream_block_rows_at<K, CB, kGroupRows, false, kHalf, true, EXACT>(
             base, row_words, tk0, tk0 + (kHalf ? 4 : 8), xrow, grp.n, nullptr, xs[wave], lane, acc);
     }
+    const half2_t sv = *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);  // here after the sums
     const int c0 = (lane >> 3) * 16 + (lane & 7);
 #pragma unroll
     for (int m = 0; m < kGroupRows; m++) {
@@ -744,8 +754,6 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
         v = moe_sum_rows(part + gid_r * n_wg * 128, n_wg, lane);
         if (lane == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    const half2_t sv =
-        *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);
     float o0, o1;
     moe_finish_block(v, sv, lane, o0, o1);
     half2_t o;

@@ -642,6 +642,37 @@ def test_rows_kernel_in_workgroups_of_four_waves(cuda, oracle, rows, k, cb, n_in
     test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs)
 
 
+@pytest.mark.parametrize("rows,n_in,n_out", [(17, 512, 256), (33, 512, 384), (77, 256, 65536), (100, 512, 128)])
+@pytest.mark.parametrize("shift", [1, 2, 4])
+def test_rows_kernel_scales_off_the_sixteen_byte_grid(cuda, rows, n_in, n_out, shift):
+    """svh and bias anywhere on the two-byte grid: the same bits as where eight of them are one load
+    (one to four 32-row tiles, workgroups of eight and of four waves)."""
+    from ponyexl3_amd import _lib, ops
+
+    lib = _lib.load()
+    g = torch.Generator(device=cuda).manual_seed(rows)
+    tr = torch.randint(-32768, 32768, (n_in // 16, n_out // 16, 64), dtype=torch.int16, device=cuda, generator=g)
+    xh = torch.randn(rows, n_in, device=cuda, generator=g).half()
+    scales = 0.05 * torch.randn(2, n_out, device=cuda, generator=g)
+    need = lib.exl3_linear_rows_workspace_bytes(rows, n_in, n_out)
+    assert need == 0  # one range: the output transform inside the kernel
+    out = []
+    for off in (0, shift):
+        sv, bv = (torch.zeros(n_out + 8, dtype=torch.float16, device=cuda)[off:off + n_out] for _ in range(2))
+        sv.copy_(scales[0])
+        bv.copy_(scales[1])
+        assert sv.data_ptr() % 16 == 2 * off and bv.data_ptr() % 16 == 2 * off
+        y = torch.empty((rows, n_out), dtype=torch.float16, device=cuda)
+        ws = torch.empty((16,), dtype=torch.uint8, device=cuda)
+        print(f"rows kernel rows={rows} {n_in}->{n_out} offset {off}", flush=True)
+        _lib.check(lib.exl3_linear_rows(ops._ptr(xh), rows, 1, ops._ptr(tr), n_in // 16, n_out // 16, 4, 0, None,
+                                        ops._ptr(sv), ops._ptr(bv), ops._ptr(y), ops._ptr(ws), 0, ops._stream()),
+                   "exl3_linear_rows")
+        out.append(y)
+    assert bool(out[0].isfinite().all()) and float(out[0].float().std()) > 0.1
+    assert torch.equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("rows,k,n_in,n_out", [(9, 5, 512, 256), (17, 4, 640, 384), (32, 6, 1024, 128),
                                               (40, 4, 2048, 2048)])
 def test_layer_output_off_the_eight_byte_grid(cuda, oracle, rows, k, n_in, n_out):
