@@ -159,6 +159,10 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
                                  svh, bias, y, reinterpret_cast<float*>(second), counters,
                                  plan_linear_mid(rows, in_tiles, n_groups), s);
     }
+    if (counters && n_sub == 1 && rows_aligned(trellis, workspace, y) &&
+        linear_rows_long_applies(rows, in_tiles, out_tiles, K, ws.second_bytes + ws.gemm_bytes))
+        return launch_linear_rows(xh, rows, (size_t)in_features, (size_t)in_features, trellis, in_tiles, out_tiles, K, cb,
+                                  nullptr, svh, bias, y, reinterpret_cast<float*>(second), s);
     uint16_t* ytmp = reinterpret_cast<uint16_t*>(second);
     if (n_sub == 1) {
         const GemmPost post{svh, bias, y, (size_t)out_features};
@@ -176,7 +180,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
 
 // Prefill of a layer whose activations are already rotated: MFMA GEMM over
 // xh [rows][n_sub][in] (block_sub picks the rotation of every 256-column block when
-// n_sub > 1), then the output transform, folded into the GEMM's fix-up pass where
+// n_sub > 1; small layers of up to 2048 rows through the rows kernel), then the output transform, folded into the GEMM's fix-up pass where
 // every tile is split.
 EXL3_EXPORT size_t exl3_linear_prefill_workspace_bytes(int rows, int in_features, int out_features) {
     if (rows < 1 || in_features < 64 || out_features < 128) return 0;
@@ -201,6 +205,10 @@ EXL3_EXPORT int exl3_linear_prefill(const uint16_t* xh, int rows, int n_sub, con
     const size_t g_bytes = align_up(gemm_workspace_bytes(rows, in_tiles, out_tiles), 256);
     if (workspace_bytes < y_bytes + g_bytes) return EXL3_E_WORKSPACE;
     hipStream_t s = as_stream(stream);
+    if (rows_aligned(trellis, workspace, y) && linear_rows_long_applies(rows, in_tiles, out_tiles, K, y_bytes + g_bytes))
+        return launch_linear_rows(xh, rows, (size_t)n_sub * in_features, (size_t)in_features, trellis, in_tiles, out_tiles,
+                                  K, cb, n_sub > 1 ? block_sub : nullptr, svh, bias, y, reinterpret_cast<float*>(workspace), s,
+                                  1);
     uint16_t* ytmp = reinterpret_cast<uint16_t*>(workspace);
     const GemmPost post{svh, bias, y, (size_t)out_features};
     bool post_done = false;

@@ -33,9 +33,9 @@ struct LinRowsArgs {
     const half_t* bias;
     half_t* y;
     float* partial;
-    const int* group_sub;  // rotation of each column group, or NULL
+    const int* group_sub;  // rotation of each column group (sub_shift 1: of each pair of groups), or NULL
     size_t ldx, sub_stride;
-    int rows, block_rows, n_row_blocks, n_units, n_splits, steps_per_split, in_steps, out_tiles;
+    int rows, block_rows, n_row_blocks, n_units, n_splits, steps_per_split, in_steps, out_tiles, sub_shift, xcd_chunk;
 };
 
 // Sums of the four k-slices of a strip. On return the wave of slice ks holds column tile pair
@@ -89,7 +89,9 @@ __device__ __forceinline__ void rows_add_slices4(float16_t (&acc)[MR][2], float4
 }
 
 // Workgroups are dealt to the eight XCDs by index: the row blocks of one (column group, range)
-// unit u land on one XCD, whose L2 then reads their trellis words once.
+// unit u land on one XCD, whose L2 then reads their trellis words once. Whole units in turn (xcd_chunk = 0) can leave one
+// XCD with more workgroups than another; else each gets xcd_chunk, an eighth of them, neighbours, so that the row blocks of seven units at most
+// lie across a border, and units of one range are neighbours too. See rows_deal_evenly().
 template <int K, int CB, int MR, int NKS>
 __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 2) void linear_rows_kernel(LinRowsArgs p) {
     using T = RowsTile<MR, NKS>;
@@ -97,10 +99,11 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int set = blockIdx.x / (8 * p.n_row_blocks), in_set = blockIdx.x % (8 * p.n_row_blocks);
-    const int u = set * 8 + (in_set & 7), rb = in_set >> 3;
+    const unsigned xcd = blockIdx.x & 7, id = (blockIdx.x >> 3) + xcd * p.xcd_chunk, t = id / (unsigned)p.n_row_blocks;
+    const int rb = id % (unsigned)p.n_row_blocks, u = p.xcd_chunk ? t : t * 8 + xcd;
     if (u >= p.n_units) return;
-    const int g = u / p.n_splits, split = u % p.n_splits;
+    const int fast = p.xcd_chunk ? p.out_tiles >> 3 : p.n_splits, q0 = u / fast, q1 = u % fast;
+    const int g = p.xcd_chunk ? q1 : q0, split = p.xcd_chunk ? q0 : q1;
     const int k0 = split * p.steps_per_split;
     const int nsteps = min(p.steps_per_split, p.in_steps - k0);
     const int m0 = rb * p.block_rows;
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
     const size_t row_words = (size_t)p.out_tiles * (8 * K);
     const uint32_t* w = p.trellis + ((size_t)k0 * 8 + 2 * ks) * row_words + (size_t)(g * 8 + cq * 4) * (8 * K);
     const half_t* x = p.xh + (size_t)m0 * p.ldx + (size_t)k0 * 128;
-    if (p.group_sub) x += (size_t)p.group_sub[g] * p.sub_stride;
+    if (p.group_sub) x += (size_t)p.group_sub[g >> p.sub_shift] * p.sub_stride;
     half_t* stages = reinterpret_cast<half_t*>(lds);
     uint32_t a_off[LPW];
 #pragma unroll
@@ -145,9 +148,9 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
     if constexpr (NKS == 4) rows_add_slices4<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
     else rows_add_slices2<MR>(acc, reinterpret_cast<float4_t*>(lds), wave, lane, sum);
     const int col = cq * 64 + (NKS == 4 ? 32 * (ks & 1) + 8 * (ks >> 1) : 8 * ks) + 4 * (lane >> 5);
-    const size_t n = (size_t)p.out_tiles * 16;
+    const size_t n_out = (size_t)p.out_tiles * 16;
     if (p.n_splits > 1) {
-        float* dst = p.partial + ((size_t)split * p.rows + m0) * n + (size_t)g * 128 + col;
+        float* dst = p.partial + ((size_t)split * p.rows + m0) * n_out + (size_t)g * 128 + col;
 #pragma unroll
         for (int mr = 0; mr < MR; mr++) {
             const int r = mr * 32 + (lane & 31);
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
                     float4_t v;
 #pragma unroll
                     for (int c = 0; c < 4; c++) v[c] = sum[mr][4 * i + c];
-                    *reinterpret_cast<float4_t*>(dst + (size_t)r * n + 16 * i) = v;
+                    *reinterpret_cast<float4_t*>(dst + (size_t)r * n_out + 16 * i) = v;
                 }
             }
         }
@@ -196,7 +199,7 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
             o[c] = (half_t)v;
             if (p.bias) o[c] = o[c] + bv[c];
         }
-        half_t* dst = p.y + (size_t)(m0 + r) * n + c0;
+        half_t* dst = p.y + (size_t)(m0 + r) * n_out + c0;
         *reinterpret_cast<half4_t*>(dst) = half4_t{o[0], o[1], o[2], o[3]};
         *reinterpret_cast<half4_t*>(dst + 4) = half4_t{o[4], o[5], o[6], o[7]};
     }
@@ -266,6 +269,17 @@ static bool rows_narrow(const LinRowsPlan& p, int n_groups, int K) {
     return p.mr >= 2 && rows_workgroups(p, n_groups) > 256 * rows_per_cu(p.mr, 4, K);
 }
 
+// Whether the workgroups are dealt to the XCDs one by one and not in whole units: where an XCD gets more of them than its 32 CUs hold
+// at once, and fewer that way (12 row blocks of 19 units: 36 on three XCDs, 24 on the others, one to a CU; evenly 29). Layers,
+// whole units -> evenly, us: 514 rows of 13184 -> 6272 (K = 6) 206 -> 126, 788 of 6912 -> 1536 62.5 -> 40.7, 1309 of 2688 -> 2176
+// 59.5 -> 35.6. Of 700 layers of 33 to 2048 rows 37 in workgroups of eight waves take 33 % less that way, 167 of four waves 4 %. Where all are resident at once whole units, which
+// spread neighbouring trellis words over the XCDs, are as good or better (224 rows of 4992 -> 3072 28.6 and 29.9,
+// 333 of 17408 -> 5120 92.3 and 93.2, 300 of 5120 -> 8192 48.3 and 48.7).
+static bool rows_deal_evenly(const LinRowsPlan& p, int n_groups, int K) {
+    const long long units = (long long)n_groups * p.n_splits, most = (units + 7) / 8 * p.n_row_blocks;
+    return most > 32 * rows_per_cu(p.mr, rows_narrow(p, n_groups, K) ? 2 : 4, K) && most > (units * p.n_row_blocks + 7) / 8;
+}
+
 // Time of a plan in workgroups of four waves, fitted to the same layers (4 % root mean square): rounds of as many as the chip holds, a last one that costs between its share
 // and that of its fullest CU.
 static double rows_narrow_estimate_us(const LinRowsPlan& p, int n_groups, int K, int cb) {
@@ -323,6 +337,23 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     return us < (cb == CB_MUL1 ? 0.92 : p.mr == 3 ? 1.0 : 0.9) * gemm_us;
 }
 
+// Whether a layer of more rows than kLinearRowsMaxRows, which the prefill GEMM takes, goes to this kernel all the same; `room`: bytes
+// for partial rows. Layers too small to fill the GEMM's 256 x 256 tiles, or with few steps to a tile. Over 350 of 1025
+// to 2048 rows (in 1024..17408, out 1024..34816, K = 2..8, all codebooks; MUL1 needs no factors here) 197 lie on this
+// side of the line and take 19 % less, one in a hundred 2 to 4 % more; the layers as they are routed take 1.1 % more than the better
+// kernel each time, all of them through the GEMM 13.6 %. GEMM -> this kernel, us: 1167 rows of 1024 -> 3072 38.1 -> 22.1,
+// 1623 of 5376 -> 2176 73.1 -> 61.2, 1118 of 3456 -> 6656 98.8 -> 74.2; beyond the line 1446 of 7168 -> 10624 230
+// and 275, 1920 of 8064 -> 8320 (K = 7) 290 and 310. From 150 us of the GEMM on its estimate is the higher one, and the line lower.
+bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K, size_t room) {
+    static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
+    if (rows <= kLinearRowsMaxRows || rows > kLinearRowsLongMaxRows || max_rows < kLinearRowsMaxRows || in_tiles < 32 ||
+        in_tiles % 8 || out_tiles < 8 || out_tiles % 8 || linear_rows_partial_bytes(rows, in_tiles, out_tiles / 8) > room)
+        return false;
+    const double gemm_us = gemm_estimate_us(rows, in_tiles, out_tiles, K, CB_3INST);
+    return rows_estimate_us(plan_linear_rows(rows, in_tiles, out_tiles / 8), rows, out_tiles / 8, K, CB_3INST) <
+           (gemm_us < 150 ? 1.05 : 0.94) * gemm_us;
+}
+
 // Up to 16 rows the rows kernel spends twice the matrix work and half the publishing of the medium-batch kernel, and
 // which one is faster hangs on how evenly each fills 256 CUs: the rows kernel with whole reductions as one
 // workgroup for every CU or two, nearly, or with few steps; with ranges where nearly two workgroups to a CU have 10 to 20 steps each
@@ -358,7 +389,8 @@ size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups) {
 
 int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
                        int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
-                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream) {
+                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream,
+                       int sub_shift) {
     if (int rc = check_k_cb(K, cb)) return rc;
     if (!xh || !trellis || !y) return EXL3_E_NULL_POINTER;
     if (rows < 1 || in_tiles < 8 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8 || ldx % 8 ||
@@ -371,13 +403,14 @@ int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stri
     const LinRowsPlan plan = plan_linear_rows(rows, in_tiles, n_groups);
     if (plan.n_splits > 1 && (!partial || (reinterpret_cast<uintptr_t>(partial) & 15))) return EXL3_E_WORKSPACE;
     const long long units = (long long)n_groups * plan.n_splits;
-    const long long grid = (units + 7) / 8 * 8 * plan.n_row_blocks;
+    const long long chunk = rows_deal_evenly(plan, n_groups, K) ? (units * plan.n_row_blocks + 7) / 8 : 0;
+    const long long grid = chunk ? 8 * chunk : (units + 7) / 8 * 8 * plan.n_row_blocks;
     if (grid > 0x7FFFFFFFLL) return EXL3_E_BAD_SHAPE;
     auto H_ = [](const uint16_t* q) { return reinterpret_cast<const half_t*>(q); };
     const LinRowsArgs a{reinterpret_cast<const uint32_t*>(trellis), H_(xh), H_(svh), H_(bias),
                         reinterpret_cast<half_t*>(y), partial, group_sub, ldx, sub_stride, rows,
                         plan.block_rows, plan.n_row_blocks, (int)units, plan.n_splits, plan.steps_per_split,
-                        in_tiles / 8, out_tiles};
+                        in_tiles / 8, out_tiles, sub_shift, (int)chunk};
     const int rc = dispatch_k_cb(K, cb, [&](auto k, auto c) {
         auto go = [&](auto mrc, auto nks) {
             constexpr int MR = mrc.value, NKS = nks.value;

@@ -642,6 +642,28 @@ def test_rows_kernel_in_workgroups_of_four_waves(cuda, oracle, rows, k, cb, n_in
     test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs)
 
 
+@pytest.mark.parametrize("rows,k,cb,n_in,outs", [
+    (1025, 4, 0, 512, (128,)),            # the first row count past the rows kernel's own limit
+    (1111, 8, 2, 640, (384,)),            # nine row blocks of unequal length
+    (2048, 3, 1, 512, (256, 256)),        # the last; two rotations, one for every 256 columns
+    (1500, 6, 0, 3328, (1024,)),          # ranges: partial rows in the GEMM's workspace
+    (1300, 4, 1, 1024, (512, 1280, 256)),
+    (2049, 4, 0, 512, (256,)),            # past it: the GEMM
+])
+def test_long_layers_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
+    """Layers of more than 1024 rows that are too small for the GEMM's tiles go to the rows kernel inside the
+    layer calls; without counters, and past 2048 rows, they stay with the GEMM."""
+    from ponyexl3_amd import EXL3Linear, FusedEXL3Group, make_exl3_layer
+
+    layers = [make_exl3_layer(k=k, in_features=n_in, out_features=o, seed=900 + i, mcg=cb == 1, mul1=cb == 2,
+                              bias=len(outs) == 1 and rows % 2 == 1) for i, o in enumerate(outs)]
+    x, xt = _x(np.random.default_rng(rows), (rows, n_in), cuda)
+    print(f"long layer rows={rows} k={k} cb={cb} {n_in}->{outs}", flush=True)
+    parts = (EXL3Linear(layers[0], cuda)(xt),) if len(outs) == 1 else FusedEXL3Group(layers, cuda).forward_all(xt)
+    for l, part in zip(layers, parts):
+        assert rel_l2(part.cpu().numpy(), _oracle_forward(oracle, l, x)) <= TOL
+
+
 @pytest.mark.parametrize("rows,n_in,n_out", [(17, 512, 256), (33, 512, 384), (77, 256, 65536), (100, 512, 128)])
 @pytest.mark.parametrize("shift", [1, 2, 4])
 def test_rows_kernel_scales_off_the_sixteen_byte_grid(cuda, rows, n_in, n_out, shift):
