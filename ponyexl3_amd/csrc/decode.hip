@@ -231,10 +231,19 @@ __global__ __launch_bounds__(256, 4) void public_weight_kernel(
         decode_lane<K, CB>(lw, wp);
 #pragma unroll
         for (int cs = 0; cs < 2; cs++) {
+            uint32_t a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                a[i] = half2_to_bits(wp[8 * cs + i]);
+                b[i] = half2_to_bits(wp[8 * cs + 4 + i]);
+            }
+            // the exchange wants two wait states behind a VALU write of its registers; the compiler does not see
+            // those of the asm in add_halves_pack2()
+            asm("s_nop 1" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]));
             uint4_t lo, hi;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const auto x = __builtin_amdgcn_permlane16_swap(half2_to_bits(wp[8 * cs + i]), half2_to_bits(wp[8 * cs + 4 + i]), false, false);
+                const auto x = __builtin_amdgcn_permlane16_swap(a[i], b[i], false, false);
                 lo[i] = x[0];
                 hi[i] = x[1];
             }
