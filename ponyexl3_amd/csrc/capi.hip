@@ -119,7 +119,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
             if (counters_len < need) return EXL3_E_WORKSPACE;
             return launch_linear_small(x, rows, trellis, in_tiles, out_tiles, K, cb, suh, n_sub,
                                        group_sub, svh, bias, y, partial, counters,
-                                       plan_linear_small_launch(rows, in_tiles, n_groups, K, cb), s,
+                                       plan_linear_small_launch(rows, in_tiles, n_groups, K), s,
                                        counters_status_word(counters, counters_len, need));
         }
         if (int rc = launch_had_pre(x, rows, in_features, suh, n_sub, xh, s)) return rc;
@@ -349,7 +349,7 @@ EXL3_EXPORT size_t exl3_linear_static_need_bytes(int rows, int in_features, int 
     // the launch plan depends on K: the largest of all (plans that the codebook decides between need the same)
     size_t need = 0;
     for (int K = 1; K <= 8; K++) {
-        const GemvPlan plan = plan_linear_small_launch(rows, in_features / 16, out_features / 128, K, CB_3INST);
+        const GemvPlan plan = plan_linear_small_launch(rows, in_features / 16, out_features / 128, K);
         const size_t n = static_need(rows, out_features, plan).larger();
         if (n > need) need = n;
     }
@@ -370,7 +370,7 @@ EXL3_EXPORT int exl3_linear_forward_static(const uint16_t* x, int rows, const ui
     if (exact_weights()) return EXL3_E_UNSUPPORTED;  // the chain that rounds the weights needs a workspace
     if (n_sub > 1 && (!group_sub || !suh)) return EXL3_E_BAD_INDEX;
     const int n_groups = out_tiles / 8;
-    const GemvPlan plan = plan_linear_small_launch(rows, in_tiles, n_groups, K, cb);
+    const GemvPlan plan = plan_linear_small_launch(rows, in_tiles, n_groups, K);
     const StaticNeed need = static_need(rows, out_tiles * 16, plan);
     if (need.partial_bytes > kStaticPartialBytes || need.counter_bytes > kStaticCounterBytes - 8)
         return EXL3_E_STATIC_LIMIT;

@@ -82,7 +82,7 @@ bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan);
 // plan_linear_small with the reduction in mind: one row on a large layer takes
 // workgroups of eight waves when that brings the launch under the atomics limit; two rows and
 // more of a layer that does not fill the chip take linear_batch_kernel.
-GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K, int cb);
+GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K);
 // fp32 partial rows per output of the largest plan over K
 int linear_small_max_partials(int rows, int in_tiles, int n_groups);
 inline size_t linear_small_counter_ints(int rows, int out_features) {

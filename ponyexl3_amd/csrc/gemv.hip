@@ -548,16 +548,17 @@ bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
 // the contributors where whole ones come two to a wave (from K = 5 on) or eight waves to a workgroup, and past 15 of them a word has
 // 30 bits in place of 33 (11904 -> 14848 K = 6 stays at 35.3, half blocks 30.6; workgroups of sixteen waves, which
 // would keep the bits, take up to 13 % more than whole blocks where they are few or decode MUL1).
-// Where decoding is light (K <= 3), and with MUL1 at K = 4, whose decode hides the loads, only what balances pays for the second
+// Where decoding is light (K <= 3) only what balances pays for the second
 // rotation. A workgroup of eight half blocks puts two on every SIMD, as one of four whole blocks puts one: a SIMD's share
 // changes only by the last workgroup of a column group, where one or two whole blocks left over take a SIMD each and their halves
 // twice as many, and where the whole blocks come eight to a workgroup. half_blocks_balance() compares the rounds of the
 // 256 CUs, in whole blocks to a SIMD; a last workgroup of eight that is not full counts for its share. On its near side 78 measurements
-// give 4.1 % less in half blocks, the slowest 1.6 % more (whole -> half: K = 1 3200 -> 26112 13.4 -> 12.8, K = 2 5376 -> 19456 15.5 -> 15.0, MUL1
-// K = 2 2688 -> 56064 41.5 -> 38.3, K = 4 6912 -> 16512 31.1 -> 30.0; K = 2 7552 -> 21888 22.4 -> 22.8); on the far side 109 give
+// give 4.1 % less in half blocks, the slowest 1.6 % more (whole -> half: K = 1 3200 -> 26112 13.4 -> 12.8, K = 2 5376 -> 19456 15.5 -> 15.0;
+// K = 2 7552 -> 21888 22.4 -> 22.8); on the far side 109 give
 // 0.8 % more, the best 1.8 % less, the worst 3.5 % more (K = 1 9728 -> 13824 18.3 -> 18.9, K = 2 2048 -> 65536 20.0 -> 20.6, 3072 -> 32000
-// 15.0 -> 15.7, K = 3 3584 -> 31744 16.2 -> 16.4, MUL1 K = 4 12032 -> 11904 34.8 -> 35.8). 3INST and MCG at K = 4 take half
-// blocks on both sides: beyond the line 25 measurements give 2.3 % less, none more.
+// 15.0 -> 15.7, K = 3 3584 -> 31744 16.2 -> 16.4). At K = 4 half
+// blocks on both sides: beyond the line 25 measurements of 3INST and MCG give 2.3 % less, none more, and 14 of MUL1 on
+// either side 0.5 to 5.8 % (12032 -> 11904 23.6 -> 22.4, 5120 -> 34816 27.7 -> 27.0, 2048 -> 65536 22.3 -> 21.3).
 static bool half_blocks_balance(int n_blocks, int n_groups, int whole_waves) {
     const int full = n_blocks / 4, rest = n_blocks % 4, fours = (n_blocks + 3) / 4, eights = (n_blocks + 7) / 8;
     auto rounds = [n_groups](int per_group) { return ((long long)n_groups * per_group + 255) / 256; };
@@ -565,12 +566,12 @@ static bool half_blocks_balance(int n_blocks, int n_groups, int whole_waves) {
            (whole_waves == 8 && rounds(fours) * eights < rounds(eights) * fours);
 }
 
-static GemvPlan one_row_half_blocks(int in_tiles, int n_groups, int K, int cb, GemvPlan whole) {
+static GemvPlan one_row_half_blocks(int in_tiles, int n_groups, int K, GemvPlan whole) {
     if (!linear_small_uses_atomics(1, n_groups, whole)) return whole;
     for (const int waves : {4, 8}) {
         if (waves == 4 && K > 4) continue;
         const GemvPlan half{in_tiles / 4, 4, waves};
-        if (waves == 8 && (K <= 3 || (K == 4 && cb == CB_MUL1)) && !half_blocks_balance(in_tiles / 8, n_groups, whole.wg_waves)) break;
+        if (waves == 8 && K <= 3 && !half_blocks_balance(in_tiles / 8, n_groups, whole.wg_waves)) break;
         if (fix_count_bits(half.n_partials()) <= fix_count_bits(whole.n_partials()) &&
             linear_small_uses_atomics(1, n_groups, half))
             return half;
@@ -578,7 +579,7 @@ static GemvPlan one_row_half_blocks(int in_tiles, int n_groups, int K, int cb, G
     return whole;
 }
 
-GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K, int cb) {
+GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K) {
     if (linear_batch_applies(rows, in_tiles, n_groups, K)) return plan_linear_batch(rows, in_tiles, n_groups);
     GemvPlan plan = plan_linear_small(rows, in_tiles, n_groups, K);
     if (rows == 1 && plan.tk_per_split >= 8) {
@@ -587,7 +588,7 @@ GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K, i
             wide.wg_waves = 8;
             if (linear_small_uses_atomics(rows, n_groups, wide)) plan = wide;
         }
-        if ((long long)(in_tiles / 8) * n_groups >= linear_half_below()) plan = one_row_half_blocks(in_tiles, n_groups, K, cb, plan);
+        if ((long long)(in_tiles / 8) * n_groups >= linear_half_below()) plan = one_row_half_blocks(in_tiles, n_groups, K, plan);
     }
     return plan;
 }
@@ -595,8 +596,7 @@ GemvPlan plan_linear_small_launch(int rows, int in_tiles, int n_groups, int K, i
 int linear_small_max_partials(int rows, int in_tiles, int n_groups) {
     int n = 0;
     for (int K = 1; K <= 8; K++) {
-        // (the codebook decides between plans of as many partial rows)
-        const int p = plan_linear_small_launch(rows, in_tiles, n_groups, K, CB_3INST).n_partials();
+        const int p = plan_linear_small_launch(rows, in_tiles, n_groups, K).n_partials();
         if (p > n) n = p;
     }
     return n;
@@ -738,7 +738,7 @@ EXL3_EXPORT int exl3_linear_plan(int rows, int in_tiles, int out_tiles, int K, i
     if (rows < 1 || rows > kLinearSmallMaxRows || in_tiles < 8 || out_tiles < 8 || in_tiles % 8 ||
         out_tiles % 8 || K < 1 || K > 8)
         return EXL3_E_BAD_SHAPE;
-    const GemvPlan plan = plan_linear_small_launch(rows, in_tiles, out_tiles / 8, K, CB_3INST);
+    const GemvPlan plan = plan_linear_small_launch(rows, in_tiles, out_tiles / 8, K);
     if (n_splits) *n_splits = plan.n_splits;
     if (tile_rows_per_split) *tile_rows_per_split = plan.tk_per_split;
     if (waves_per_workgroup) *waves_per_workgroup = plan.wg_waves;
