@@ -54,8 +54,8 @@ int exl3_gemv_max_rows(void);
 /* Largest row count exl3_linear_forward serves with its small-batch, medium-batch and
  * rows kernels for stacked suh too when given counters (above exl3_gemv_max_rows()
  * the input rotation runs as a launch of its own first). Beyond it the rows kernel or
- * the prefill GEMM takes plain layers, exl3_linear_rows and exl3_linear_prefill
- * stacked ones. */
+ * the prefill GEMM takes plain layers; exl3_linear_rows, exl3_linear_rows_long and
+ * exl3_linear_prefill stacked ones. */
 int exl3_linear_small_max_rows(void);
 
 /*
@@ -443,13 +443,20 @@ int exl3_moe_decode(const uint16_t *x, int tokens, const uint16_t *logits,
  * exl3_linear_rows_faster: whether it is the faster path for these sizes, K and codebook (and the
  * trellis 16-byte aligned, which it requires); otherwise take exl3_linear_prefill.
  * exl3_linear_rows_applies: the same for K = 4 and 3INST weights.
+ * exl3_linear_rows_long, exl3_linear_rows_long_faster: the same for 1025 to 2048 rows, where the kernel is the faster
+ * one for layers too small to fill the GEMM's tiles. The workspace is then no larger than
+ * exl3_linear_prefill_workspace_bytes().
  */
 int exl3_linear_rows_applies(const uint16_t *trellis, int rows, int in_tiles, int out_tiles);
 int exl3_linear_rows_faster(const uint16_t *trellis, int rows, int in_tiles, int out_tiles, int K, int cb);
+int exl3_linear_rows_long_faster(const uint16_t *trellis, int rows, int in_tiles, int out_tiles, int K, int cb);
 size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, int out_features);
 int exl3_linear_rows(const uint16_t *xh, int rows, int n_sub, const uint16_t *trellis, int in_tiles, int out_tiles,
                      int K, int cb, const int32_t *group_sub, const uint16_t *svh, const uint16_t *bias, uint16_t *y,
                      void *workspace, size_t workspace_bytes, void *stream);
+int exl3_linear_rows_long(const uint16_t *xh, int rows, int n_sub, const uint16_t *trellis, int in_tiles, int out_tiles,
+                          int K, int cb, const int32_t *group_sub, const uint16_t *svh, const uint16_t *bias, uint16_t *y,
+                          void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * Prefill of one layer on activations that exl3_had128_pre already rotated:

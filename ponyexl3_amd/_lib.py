@@ -41,8 +41,10 @@ PROTOTYPES = {
     "exl3_linear_prefill_workspace_bytes": (_sz, [_i, _i, _i]),
     "exl3_linear_rows_applies": (_i, [_vp, _i, _i, _i]),
     "exl3_linear_rows_faster": (_i, [_vp, _i, _i, _i, _i, _i]),
+    "exl3_linear_rows_long_faster": (_i, [_vp, _i, _i, _i, _i, _i]),
     "exl3_linear_rows_workspace_bytes": (_sz, [_i, _i, _i]),
     "exl3_linear_rows": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "exl3_linear_rows_long": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "exl3_linear_prefill": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "exl3_moe_sort": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),
     "exl3_moe_glu_rows": (_i, [_vp, _vp, _i, _i, _vp, _vp, _vp, _i, _i, _vp, _vp]),

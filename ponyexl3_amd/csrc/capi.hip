@@ -160,7 +160,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
                                  plan_linear_mid(rows, in_tiles, n_groups), s);
     }
     if (counters && n_sub == 1 && rows_aligned(trellis, workspace, y) &&
-        linear_rows_long_applies(rows, in_tiles, out_tiles, K, ws.second_bytes + ws.gemm_bytes))
+        linear_rows_long_applies(rows, in_tiles, out_tiles, K))
         return launch_linear_rows(xh, rows, (size_t)in_features, (size_t)in_features, trellis, in_tiles, out_tiles, K, cb,
                                   nullptr, svh, bias, y, reinterpret_cast<float*>(second), s);
     uint16_t* ytmp = reinterpret_cast<uint16_t*>(second);
@@ -180,7 +180,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
 
 // Prefill of a layer whose activations are already rotated: MFMA GEMM over
 // xh [rows][n_sub][in] (block_sub picks the rotation of every 256-column block when
-// n_sub > 1; small layers of up to 2048 rows through the rows kernel), then the output transform, folded into the GEMM's fix-up pass where
+// n_sub > 1), then the output transform, folded into the GEMM's fix-up pass where
 // every tile is split.
 EXL3_EXPORT size_t exl3_linear_prefill_workspace_bytes(int rows, int in_features, int out_features) {
     if (rows < 1 || in_features < 64 || out_features < 128) return 0;
@@ -205,10 +205,6 @@ EXL3_EXPORT int exl3_linear_prefill(const uint16_t* xh, int rows, int n_sub, con
     const size_t g_bytes = align_up(gemm_workspace_bytes(rows, in_tiles, out_tiles), 256);
     if (workspace_bytes < y_bytes + g_bytes) return EXL3_E_WORKSPACE;
     hipStream_t s = as_stream(stream);
-    if (rows_aligned(trellis, workspace, y) && linear_rows_long_applies(rows, in_tiles, out_tiles, K, y_bytes + g_bytes))
-        return launch_linear_rows(xh, rows, (size_t)n_sub * in_features, (size_t)in_features, trellis, in_tiles, out_tiles,
-                                  K, cb, n_sub > 1 ? block_sub : nullptr, svh, bias, y, reinterpret_cast<float*>(workspace), s,
-                                  1);
     uint16_t* ytmp = reinterpret_cast<uint16_t*>(workspace);
     const GemmPost post{svh, bias, y, (size_t)out_features};
     bool post_done = false;
@@ -235,22 +231,42 @@ EXL3_EXPORT size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, i
     return exl3::linear_rows_partial_bytes(rows, in_features / 16, out_features / 128);
 }
 
-EXL3_EXPORT int exl3_linear_rows(const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis, int in_tiles,
-                                 int out_tiles, int K, int cb, const int32_t* group_sub, const uint16_t* svh,
-                                 const uint16_t* bias, uint16_t* y, void* workspace, size_t workspace_bytes,
-                                 void* stream) {
+EXL3_EXPORT int exl3_linear_rows_long_faster(const uint16_t* trellis, int rows, int in_tiles, int out_tiles, int K, int cb) {
+    return exl3::check_k_cb(K, cb) == EXL3_OK && exl3::rows_aligned(trellis) &&
+           exl3::linear_rows_long_applies(rows, in_tiles, out_tiles, K);
+}
+
+static int linear_rows_between(int min_rows, int max_rows, const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis,
+                               int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub, const uint16_t* svh,
+                               const uint16_t* bias, uint16_t* y, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace exl3;
     if (int rc = check_k_cb(K, cb)) return rc;
     if (!xh || !trellis || !y) return EXL3_E_NULL_POINTER;
     if (rows < 1 || in_tiles < 8 || out_tiles < 8 || in_tiles % 8 || out_tiles % 8 || n_sub < 1)
         return EXL3_E_BAD_SHAPE;
-    if (rows > kLinearRowsMaxRows) return EXL3_E_UNSUPPORTED;
+    if (rows < min_rows || rows > max_rows) return EXL3_E_UNSUPPORTED;
     if (n_sub > 1 && !group_sub) return EXL3_E_BAD_INDEX;
     if (workspace_bytes < linear_rows_partial_bytes(rows, in_tiles, out_tiles / 8)) return EXL3_E_WORKSPACE;
     const size_t in_features = (size_t)in_tiles * 16;
     return launch_linear_rows(xh, rows, n_sub * in_features, in_features, trellis, in_tiles, out_tiles, K, cb,
                               n_sub > 1 ? group_sub : nullptr, svh, bias, y, reinterpret_cast<float*>(workspace),
                               as_stream(stream));
+}
+
+EXL3_EXPORT int exl3_linear_rows(const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis, int in_tiles,
+                                 int out_tiles, int K, int cb, const int32_t* group_sub, const uint16_t* svh,
+                                 const uint16_t* bias, uint16_t* y, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+    return linear_rows_between(1, exl3::kLinearRowsMaxRows, xh, rows, n_sub, trellis, in_tiles, out_tiles, K, cb, group_sub,
+                               svh, bias, y, workspace, workspace_bytes, stream);
+}
+
+EXL3_EXPORT int exl3_linear_rows_long(const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis, int in_tiles,
+                                      int out_tiles, int K, int cb, const int32_t* group_sub, const uint16_t* svh,
+                                      const uint16_t* bias, uint16_t* y, void* workspace, size_t workspace_bytes,
+                                      void* stream) {
+    return linear_rows_between(exl3::kLinearRowsMaxRows + 1, exl3::kLinearRowsLongMaxRows, xh, rows, n_sub, trellis, in_tiles,
+                               out_tiles, K, cb, group_sub, svh, bias, y, workspace, workspace_bytes, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -137,7 +137,7 @@ int launch_linear_mid(const uint16_t* xh, int rows, const uint16_t* trellis, int
 // g (128 columns) reads xh + group_sub[g] * sub_stride (group_sub may be NULL);
 // partial: linear_rows_partial_bytes(), 16-byte aligned.
 constexpr int kLinearRowsMaxRows = 1024;
-constexpr int kLinearRowsLongMaxRows = 2048;  // inside the layer calls, see linear_rows_long_applies()
+constexpr int kLinearRowsLongMaxRows = 2048;  // inside the fused layer calls, see linear_rows_long_applies()
 struct LinRowsPlan {
     int n_row_blocks, block_rows, mr;  // mr: 32-row tiles of the kernel that holds block_rows
     int n_splits, steps_per_split;     // ranges of the reduction, in 128-deep steps
@@ -149,8 +149,8 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb);
 bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles);
 int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
                        int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
-                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream, int sub_shift = 0);
-bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K, size_t room);
+                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream);
+bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K);
 
 int launch_had_pre(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub,
                    uint16_t* xh, hipStream_t stream);

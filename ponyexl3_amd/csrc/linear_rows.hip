@@ -33,9 +33,9 @@ struct LinRowsArgs {
     const half_t* bias;
     half_t* y;
     float* partial;
-    const int* group_sub;  // rotation of each column group (sub_shift 1: of each pair of groups), or NULL
+    const int* group_sub;  // rotation of each column group, or NULL
     size_t ldx, sub_stride;
-    int rows, block_rows, n_row_blocks, n_units, n_splits, steps_per_split, in_steps, out_tiles, sub_shift, xcd_chunk;
+    int rows, block_rows, n_row_blocks, n_units, n_splits, steps_per_split, in_steps, out_tiles, xcd_chunk;
 };
 
 // Sums of the four k-slices of a strip. On return the wave of slice ks holds column tile pair
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
     const size_t row_words = (size_t)p.out_tiles * (8 * K);
     const uint32_t* w = p.trellis + ((size_t)k0 * 8 + 2 * ks) * row_words + (size_t)(g * 8 + cq * 4) * (8 * K);
     const half_t* x = p.xh + (size_t)m0 * p.ldx + (size_t)k0 * 128;
-    if (p.group_sub) x += (size_t)p.group_sub[g >> p.sub_shift] * p.sub_stride;
+    if (p.group_sub) x += (size_t)p.group_sub[g] * p.sub_stride;
     half_t* stages = reinterpret_cast<half_t*>(lds);
     uint32_t a_off[LPW];
 #pragma unroll
@@ -337,17 +337,18 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     return us < (cb == CB_MUL1 ? 0.92 : p.mr == 3 ? 1.0 : 0.9) * gemm_us;
 }
 
-// Whether a layer of more rows than kLinearRowsMaxRows, which the prefill GEMM takes, goes to this kernel all the same; `room`: bytes
-// for partial rows. Layers too small to fill the GEMM's 256 x 256 tiles, or with few steps to a tile. Over 350 of 1025
+// Whether a layer of more rows than kLinearRowsMaxRows, which the prefill GEMM takes, goes to this kernel all the same, where its
+// partial rows fit what the call's workspace holds for the GEMM. Layers too small to fill the GEMM's 256 x 256 tiles, or with few steps to a tile. Over 350 of 1025
 // to 2048 rows (in 1024..17408, out 1024..34816, K = 2..8, all codebooks; MUL1 needs no factors here) 197 lie on this
 // side of the line and take 19 % less, one in a hundred 2 to 4 % more; the layers as they are routed take 1.1 % more than the better
 // kernel each time, all of them through the GEMM 13.6 %. GEMM -> this kernel, us: 1167 rows of 1024 -> 3072 38.1 -> 22.1,
 // 1623 of 5376 -> 2176 73.1 -> 61.2, 1118 of 3456 -> 6656 98.8 -> 74.2; beyond the line 1446 of 7168 -> 10624 230
 // and 275, 1920 of 8064 -> 8320 (K = 7) 290 and 310. From 150 us of the GEMM on its estimate is the higher one, and the line lower.
-bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K, size_t room) {
+bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K) {
     static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
     if (rows <= kLinearRowsMaxRows || rows > kLinearRowsLongMaxRows || max_rows < kLinearRowsMaxRows || in_tiles < 32 ||
-        in_tiles % 8 || out_tiles < 8 || out_tiles % 8 || linear_rows_partial_bytes(rows, in_tiles, out_tiles / 8) > room)
+        in_tiles % 8 || out_tiles < 8 || out_tiles % 8 ||
+        linear_rows_partial_bytes(rows, in_tiles, out_tiles / 8) > (size_t)rows * out_tiles * 32 + gemm_workspace_bytes(rows, in_tiles, out_tiles))
         return false;
     const double gemm_us = gemm_estimate_us(rows, in_tiles, out_tiles, K, CB_3INST);
     return rows_estimate_us(plan_linear_rows(rows, in_tiles, out_tiles / 8), rows, out_tiles / 8, K, CB_3INST) <
@@ -389,8 +390,7 @@ size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups) {
 
 int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
                        int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
-                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream,
-                       int sub_shift) {
+                       const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream) {
     if (int rc = check_k_cb(K, cb)) return rc;
     if (!xh || !trellis || !y) return EXL3_E_NULL_POINTER;
     if (rows < 1 || in_tiles < 8 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8 || ldx % 8 ||
@@ -410,7 +410,7 @@ int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stri
     const LinRowsArgs a{reinterpret_cast<const uint32_t*>(trellis), H_(xh), H_(svh), H_(bias),
                         reinterpret_cast<half_t*>(y), partial, group_sub, ldx, sub_stride, rows,
                         plan.block_rows, plan.n_row_blocks, (int)units, plan.n_splits, plan.steps_per_split,
-                        in_tiles / 8, out_tiles, sub_shift, (int)chunk};
+                        in_tiles / 8, out_tiles, (int)chunk};
     const int rc = dispatch_k_cb(K, cb, [&](auto k, auto c) {
         auto go = [&](auto mrc, auto nks) {
             constexpr int MR = mrc.value, NKS = nks.value;

@@ -205,12 +205,17 @@ void linear_run(const LinearLayer& l, const at::Tensor& x, int64_t rows64, const
         check_status((fused ? exl3_rotate : exl3_had128_pre)(xp, rows, n_in, half_ptr(l.suh), l.n_sub, half_out(xh),
                                                              ctx.stream),
                      "exl3_rotate");
-        if (fused && l.group_sub.defined() && exl3_linear_rows_faster(tr, rows, l.in_tiles, l.out_tiles, l.k, l.cb)) {
+        // (past exl3_linear_rows()' rows the members of a stack that takes the rows kernel end on 256-column blocks, the ones
+        // it was measured against the GEMM with)
+        const bool fits = fused && l.group_sub.defined() && exl3_linear_rows_faster(tr, rows, l.in_tiles, l.out_tiles, l.k, l.cb);
+        const bool fits_long = fused && l.group_sub.defined() && one_launch &&
+                               exl3_linear_rows_long_faster(tr, rows, l.in_tiles, l.out_tiles, l.k, l.cb);
+        if (fits || fits_long) {
             const size_t bytes = exl3_linear_rows_workspace_bytes(rows, n_in, n_out);
             void* ws = bytes ? ctx.get(kWorkspace, bytes).mutable_data_ptr() : nullptr;
-            check_status(exl3_linear_rows(half_ptr(xh), rows, l.n_sub, tr, l.in_tiles, l.out_tiles, l.k, l.cb,
-                                          int_ptr(l.group_sub), half_ptr(l.svh), half_ptr(l.bias), yp, ws, bytes,
-                                          ctx.stream),
+            check_status((fits ? exl3_linear_rows : exl3_linear_rows_long)(
+                             half_ptr(xh), rows, l.n_sub, tr, l.in_tiles, l.out_tiles, l.k, l.cb, int_ptr(l.group_sub),
+                             half_ptr(l.svh), half_ptr(l.bias), yp, ws, bytes, ctx.stream),
                          "exl3_linear_rows");
             return;
         }

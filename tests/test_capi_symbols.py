@@ -83,6 +83,9 @@ def test_argument_errors_before_launch(lib):
     assert lib.exl3_linear_prefill(p, 4, 1, p, 8, 16, 4, 0, None, p, None, p, p, 16, None) == _lib.EXL3_E_WORKSPACE
     assert lib.exl3_linear_prefill(p, 4, 1, p, 7, 16, 4, 0, None, p, None, p, p, 1 << 30, None) == _lib.EXL3_E_BAD_SHAPE
     assert lib.exl3_linear_prefill_workspace_bytes(4, 128, 256) >= 4 * 256 * 2
+    for entry, rows in ((lib.exl3_linear_rows, 1025), (lib.exl3_linear_rows_long, 1024), (lib.exl3_linear_rows_long, 2049)):
+        assert entry(p, rows, 1, p, 32, 16, 4, 0, None, p, None, p, p, 1 << 30, None) == _lib.EXL3_E_UNSUPPORTED
+    assert lib.exl3_linear_rows_long(p, 1025, 2, p, 32, 16, 4, 0, None, p, None, p, p, 1 << 30, None) == _lib.EXL3_E_BAD_INDEX
     assert lib.exl3_moe_sort(p, 8, 2, 4, 64, p, p, p, p, 3, None) == _lib.EXL3_E_BAD_SHAPE  # table too short
     assert lib.exl3_moe_sort(p, 8, 2, 2000, 64, p, p, p, p, 4000, None) == _lib.EXL3_E_UNSUPPORTED
     assert lib.exl3_moe_sort(p, 8, 2, 4, 64, p, p, None, p, 8, None) == _lib.EXL3_E_NULL_POINTER
@@ -201,6 +204,12 @@ def test_layer_workspace_holds_the_rows_route(lib):
         if any(lib.exl3_linear_rows_faster(aligned, rows, n_in // 16, n_out // 16, k, cb)
                for k in range(1, 9) for cb in range(3)):
             assert total >= rows * n_sub * n_in * 2 + lib.exl3_linear_rows_workspace_bytes(rows, n_in, n_out)
+        rows = rng.randint(1025, 2048)
+        if any(lib.exl3_linear_rows_long_faster(aligned, rows, n_in // 16, n_out // 16, k, cb)
+               for k in range(1, 9) for cb in range(3)):
+            partial = lib.exl3_linear_rows_workspace_bytes(rows, n_in, n_out)
+            assert lib.exl3_linear_workspace_bytes(rows, n_in, n_out, 1) >= rows * n_in * 2 + partial
+            assert lib.exl3_linear_prefill_workspace_bytes(rows, n_in, n_out) >= partial
 
 
 def test_status_to_exception():

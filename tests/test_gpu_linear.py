@@ -664,6 +664,32 @@ def test_long_layers_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
         assert rel_l2(part.cpu().numpy(), _oracle_forward(oracle, l, x)) <= TOL
 
 
+@pytest.mark.parametrize("rows,k,cb,n_in,n_out", [(1025, 4, 0, 512, 512), (1500, 6, 0, 3328, 1024), (2048, 3, 1, 512, 512)])
+def test_prefill_entry_point_is_the_gemm(cuda, rows, k, cb, n_in, n_out):
+    """exl3_linear_prefill, and a stacked layer that is not fused, run the GEMM as a layer call without counters does, bit
+    for bit, also where a fused call of as many rows takes the rows kernel. The stack: two members with the same sign
+    vectors, i.e. one layer."""
+    from ponyexl3_amd import _lib, make_exl3_layer, ops
+
+    lib = _lib.load()
+    layer = make_exl3_layer(k=k, in_features=n_in, out_features=n_out, seed=rows, mcg=cb == 1, mul1=cb == 2)
+    tr, suh, svh = ops.as_trellis_tensor(layer.trellis, cuda), torch.from_numpy(layer.suh).to(cuda), torch.from_numpy(layer.svh).to(cuda)
+    _, xt = _x(np.random.default_rng(rows), (rows, n_in), cuda)
+    print(f"prefill rows={rows} k={k} cb={cb} {n_in}->{n_out}", flush=True)
+    assert lib.exl3_linear_rows_long_faster(ops._ptr(tr), rows, n_in // 16, n_out // 16, k, cb)
+    xh = ops.had128_pre(xt, suh).contiguous()
+    ref = ops.linear_forward(xt, tr, k, cb, suh, svh, fused=False)
+    ws = torch.empty((lib.exl3_linear_prefill_workspace_bytes(rows, n_in, n_out),), dtype=torch.uint8, device=cuda)
+    y = torch.empty((rows, n_out), dtype=torch.float16, device=cuda)
+    _lib.check(lib.exl3_linear_prefill(ops._ptr(xh), rows, 1, ops._ptr(tr), n_in // 16, n_out // 16, k, cb, None, ops._ptr(svh),
+                                       None, ops._ptr(y), ops._ptr(ws), ws.numel(), ops._stream()), "exl3_linear_prefill")
+    assert torch.equal(y, ref)
+    sub = (torch.arange(n_out // 128, device=cuda) >= n_out // 256).to(torch.int32)
+    stack = ops.linear_forward(xt, tr, k, cb, torch.stack([suh, suh]), svh, group_sub=sub, fused=False,
+                               member_out=[n_out // 2, n_out // 2])
+    assert torch.equal(stack, ref)
+
+
 @pytest.mark.parametrize("rows,n_in,n_out", [(17, 512, 256), (33, 512, 384), (77, 256, 65536), (100, 512, 128)])
 @pytest.mark.parametrize("shift", [1, 2, 4])
 def test_rows_kernel_scales_off_the_sixteen_byte_grid(cuda, rows, n_in, n_out, shift):
