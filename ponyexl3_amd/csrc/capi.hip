@@ -160,7 +160,7 @@ EXL3_EXPORT int exl3_linear_forward(const uint16_t* x, int rows, const uint16_t*
                                  plan_linear_mid(rows, in_tiles, n_groups), s);
     }
     if (counters && n_sub == 1 && rows_aligned(trellis, workspace, y) &&
-        linear_rows_long_applies(rows, in_tiles, out_tiles, K))
+        linear_rows_long_applies(rows, in_tiles, out_tiles, K, cb))
         return launch_linear_rows(xh, rows, (size_t)in_features, (size_t)in_features, trellis, in_tiles, out_tiles, K, cb,
                                   nullptr, svh, bias, y, reinterpret_cast<float*>(second), s);
     uint16_t* ytmp = reinterpret_cast<uint16_t*>(second);
@@ -233,7 +233,7 @@ EXL3_EXPORT size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, i
 
 EXL3_EXPORT int exl3_linear_rows_long_faster(const uint16_t* trellis, int rows, int in_tiles, int out_tiles, int K, int cb) {
     return exl3::check_k_cb(K, cb) == EXL3_OK && exl3::rows_aligned(trellis) &&
-           exl3::linear_rows_long_applies(rows, in_tiles, out_tiles, K);
+           exl3::linear_rows_long_applies(rows, in_tiles, out_tiles, K, cb);
 }
 
 static int linear_rows_between(int min_rows, int max_rows, const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis,

@@ -150,7 +150,7 @@ bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles);
 int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
                        int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
                        const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream);
-bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K);
+bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K, int cb);
 
 int launch_had_pre(const uint16_t* x, int rows, int n, const uint16_t* suh, int n_sub,
                    uint16_t* xh, hipStream_t stream);

@@ -338,21 +338,33 @@ bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
 }
 
 // Whether a layer of more rows than kLinearRowsMaxRows, which the prefill GEMM takes, goes to this kernel all the same, where its
-// partial rows fit what the call's workspace holds for the GEMM. Layers too small to fill the GEMM's 256 x 256 tiles, or with few steps to a tile. Over 350 of 1025
-// to 2048 rows (in 1024..17408, out 1024..34816, K = 2..8, all codebooks; MUL1 needs no factors here) 197 lie on this
-// side of the line and take 19 % less, one in a hundred 2 to 4 % more; the layers as they are routed take 1.1 % more than the better
-// kernel each time, all of them through the GEMM 13.6 %. GEMM -> this kernel, us: 1167 rows of 1024 -> 3072 38.1 -> 22.1,
-// 1623 of 5376 -> 2176 73.1 -> 61.2, 1118 of 3456 -> 6656 98.8 -> 74.2; beyond the line 1446 of 7168 -> 10624 230
-// and 275, 1920 of 8064 -> 8320 (K = 7) 290 and 310. From 150 us of the GEMM on its estimate is the higher one, and the line lower.
-bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K) {
+// partial rows fit what the call's workspace holds for the GEMM. Layers too small to fill the GEMM's 256 x 256 tiles, or with few
+// steps to a tile. The estimates are those for 3INST, which was fitted up to 1024 rows; past them
+//  * reductions of 24 steps and more take longer than estimated the more rows there are (every XCD reads all of them: 1.0 times at 1300
+//    rows, 1.2 at 2000), and the GEMM, whose pieces of such a reduction are long ones, is as fast as estimated;
+//  * ranges in workgroups of four waves were 1 % slower than the GEMM on average, some by 14 % (50 layers of 3INST and MCG);
+//  * the GEMM's estimate is low for MUL1, high from 150 us on and, below K = 4, where both are those of K = 4, 4 % high.
+// 609 layers that the estimates alone would send here (in 1024..17408, out 1024..34816, K = 2..8, all codebooks), the two kernels in turn on one
+// GPU: 40 of them are more than 2 % slower than through the GEMM, by up to 14 %. Of the 432 left two are, by 2.3 %; what the others gained
+// is 1.1 % of the whole.
+// GEMM -> this kernel, us: 1167 rows of 1024 -> 3072 38.1 -> 22.1, 1388 of 10880 -> 2944 143 -> 114, 1118 of 3456 -> 6656 98.8 -> 74.2,
+// 1659 of 7552 -> 2176 89.1 -> 78.3; beyond the line 1097 of 16512 -> 2048 (K = 7) 117 and 136, 1907 of 12928 -> 1792 127 and 135,
+// 2014 of 6656 -> 3584 127 and 136, 1257 of 13568 -> 1920 (K = 7) 105 and 117.
+bool linear_rows_long_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
     if (rows <= kLinearRowsMaxRows || rows > kLinearRowsLongMaxRows || max_rows < kLinearRowsMaxRows || in_tiles < 32 ||
         in_tiles % 8 || out_tiles < 8 || out_tiles % 8 ||
         linear_rows_partial_bytes(rows, in_tiles, out_tiles / 8) > (size_t)rows * out_tiles * 32 + gemm_workspace_bytes(rows, in_tiles, out_tiles))
         return false;
+    const LinRowsPlan p = plan_linear_rows(rows, in_tiles, out_tiles / 8);
     const double gemm_us = gemm_estimate_us(rows, in_tiles, out_tiles, K, CB_3INST);
-    return rows_estimate_us(plan_linear_rows(rows, in_tiles, out_tiles / 8), rows, out_tiles / 8, K, CB_3INST) <
-           (gemm_us < 150 ? 1.05 : 0.94) * gemm_us;
+    double us = rows_estimate_us(p, rows, out_tiles / 8, K, CB_3INST) * (K < 4 ? 1.04 : 1.0);
+    const bool mul1 = cb == CB_MUL1;
+    if (us >= (gemm_us >= 150 ? 0.94 : mul1 ? 1.05 : 1.02) * gemm_us) return false;
+    if (!mul1 && p.n_splits > 1 && rows_narrow(p, out_tiles / 8, K)) return false;
+    if (p.steps_per_split < 24) return true;
+    if (rows > 1300) us *= 1 + 0.2 * (rows - 1300) / 700;
+    return us < (mul1 ? 1.04 : 0.96) * gemm_us;
 }
 
 // Up to 16 rows the rows kernel spends twice the matrix work and half the publishing of the medium-batch kernel, and

@@ -190,6 +190,23 @@ def test_rows_route_knows_the_weights(lib):
     assert lib.exl3_linear_rows_applies(aligned, 77, 320, 640) == 1
 
 
+@pytest.mark.parametrize("rows,n_in,n_out,k,cb,rows_kernel", [
+    # (us through the GEMM and through the rows kernel, in turn on one GPU)
+    (1167, 1024, 3072, 4, 0, True), (1659, 7552, 2176, 4, 1, True),     # 38.1 and 22.1, 89.1 and 78.3
+    (1917, 7808, 2176, 4, 2, True), (1388, 10880, 2944, 4, 1, True),    # 109.8 and 87.5, 142.6 and 113.8
+    (1097, 16512, 2048, 7, 0, False), (1257, 13568, 1920, 7, 0, False),  # four waves, ranges: 117 and 136, 105 and 117
+    (1175, 8320, 2048, 4, 0, False), (2043, 15360, 1152, 3, 0, False),   # 71 and 77, 116 and 132
+    (1907, 12928, 1792, 4, 0, False), (2014, 6656, 3584, 4, 1, False),   # long reductions of many rows: 127 and 135, 127 and 136
+    (1942, 14976, 1664, 7, 2, False), (1425, 3712, 2944, 8, 0, False),   # 152 and 160, 67 and 70
+    (2018, 3840, 6016, 3, 0, False),                                     # K < 4: 114 and 124
+    (2049, 512, 256, 4, 0, False), (1024, 512, 256, 4, 0, False),
+])
+def test_long_layers_take_the_faster_kernel(lib, rows, n_in, n_out, k, cb, rows_kernel):
+    """1025 to 2048 rows: layers measured on either side of the line between the GEMM and the rows kernel."""
+    faster = lib.exl3_linear_rows_long_faster(ctypes.c_void_p(4096), rows, n_in // 16, n_out // 16, k, cb)
+    assert bool(faster) == rows_kernel
+
+
 def test_layer_workspace_holds_the_rows_route(lib):
     """exl3_linear_workspace_bytes does not know K: wherever the rows kernel may be taken for some
     K and codebook, it holds the rotated activations and the partial rows."""
