@@ -225,7 +225,8 @@ __device__ __forceinline__ void moe_finish_block(float2_t sum, half2_t sv, int l
 }
 
 // Routing by the expert kernel itself, from the router's logits: 3.4 us in front of the first weights
-// (8.0 -> 11.4 us) where a launch of its own in between takes 4.0 us and a gap of about 1, and 3.5 us of host time. Every wave finds the expert of its slot.
+// (8.0 -> 11.4 us) where a launch of its own in between takes 4.0 us and a gap of about 1, and 3.5 us of host time. Every wave finds the expert of its slot;
+// one workgroup a token writes the token's row of the routing table for the launch behind.
 // logits == nullptr: the table is there.
 constexpr int kInlineRouteExperts = 256;  // four per lane
 struct MoeRoute {
@@ -235,25 +236,22 @@ struct MoeRoute {
     half_t* scores;  // fp16 [tokens][top_k], top_k with the shared expert
 };
 
-__device__ __forceinline__ int moe_route_slot(const MoeRoute& r, int s, int top_k, bool writes, int lane, RouteChoice& c) {
+// writes: by the first workgroup of a token's last slot, which chooses them all anyway.
+__device__ __forceinline__ int moe_route_slot(const MoeRoute& r, int s, int top_k, int* indices, bool writes, int lane) {
     const int t = s / top_k, j = s - t * top_k, ranked = top_k - (r.shared_logits != nullptr);
     if (j == ranked && !writes) return r.n_experts;  // the shared expert
     int key[kInlineRouteExperts / 64];
     route_probabilities<half_t>(r.logits + (size_t)t * r.n_experts, r.n_experts, lane, key);
+    RouteChoice c{0.f, 0};
     int e = r.n_experts;
     const int rounds = writes ? ranked : j + 1;
     for (int i = 0; i < rounds; i++) {
         const int chosen = route_next(key, lane, i, c);
         if (i == j) e = chosen;
     }
+    if (writes) route_write<half_t>(c, lane, t, r.n_experts, ranked, r.norm, r.shared_logits != nullptr,
+                                     r.shared_logits ? r.shared_logits[t] : (half_t)0.f, indices, r.scores);
     return e;
-}
-
-// The token's row of the table, for the launch behind: by the first workgroup of its last slot, which has chosen them all.
-__device__ __forceinline__ void moe_route_write(const MoeRoute& r, RouteChoice c, int t, int top_k, int* indices, int lane) {
-    const bool shared = r.shared_logits != nullptr;
-    route_write<half_t>(c, lane, t, r.n_experts, top_k - shared, r.norm, shared, shared ? r.shared_logits[t] : (half_t)0.f,
-                        indices, r.scores);
 }
 
 // Weighted sum over the slots of a token by the wave that stores the last of them: one 128-column block o of
@@ -410,19 +408,8 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
     const int gid = blockIdx.x;
     const int hg = gid % hblocks, s = gid / hblocks;
     const int p = wave >> 2, j = wave & 3;
-    const bool writes = route.logits && blockIdx.y == 0 && hg == 0 && wave == 0 && s % top_k == top_k - 1;
-    RouteChoice choice{0.f, 0};
-    const int e = clamp_expert(route.logits ? moe_route_slot(route, s, top_k, writes, lane, choice) : indices[s], E);
-    // scales of what follows the reduction, requested now: behind it each would be a trip to memory that nothing hides.
-    // (block of 8 of 256 experts of 2048 x 512, with those of the down projection and the table's row written behind the weights: 1 token 21.5 -> 20.9
-    // us, with a shared expert 24.5 -> 24.2)
-    half2_t svg, svu, ds;
-    if (wave == 0) {
-        const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
-        svg = *reinterpret_cast<const half2_t*>(svh_e);
-        svu = *reinterpret_cast<const half2_t*>(svh_e + H);
-        ds = *reinterpret_cast<const half2_t*>(dn_suh + (size_t)e * H + hg * 128 + 2 * lane);
-    }
+    const bool writes = blockIdx.y == 0 && hg == 0 && wave == 0 && s % top_k == top_k - 1;
+    const int e = clamp_expert(route.logits ? moe_route_slot(route, s, top_k, indices, writes, lane) : indices[s], E);
     const int blk = HALF ? blockIdx.y * 2 + (j >> 1) : blockIdx.y * 4 + j;
     const int tk0 = blk * 8 + (HALF ? (j & 1) * 4 : 0);
     float acc[1][2] = {{0.f, 0.f}};
@@ -435,12 +422,23 @@ __global__ __launch_bounds__(512) void moe_gateup_pair_kernel(
                                                 gu_suh + ((size_t)e * 2 + p) * D, xs[wave], lane,
                                                 acc);
     }
+    // Scales of what follows the reduction, requested in front of it: its round trip hides theirs (behind it a shared-expert
+    // block of 8 of 256 experts of 2048 x 512 takes 24.5 us a token, so 24.2; without a shared expert there is no difference). In front of
+    // the weights they, and the choices of a table's row that is written behind them, cost five registers a lane: at K = 6 and 7 a
+    // CU then holds two workgroups in place of three (MCG: three of four), and 7 tokens of 6 slots, 257 experts of 1792 x 512, take 38.9 us in
+    // place of 36.8 at K = 6, 6 tokens of 5 slots of 2048 x 384 30.1 in place of 28.3 at K = 7.
+    half2_t svg, svu, ds;
+    if (wave == 0) {
+        const half_t* svh_e = gu_svh + (size_t)e * 2 * H + hg * 128 + 2 * lane;
+        svg = *reinterpret_cast<const half2_t*>(svh_e);
+        svu = *reinterpret_cast<const half2_t*>(svh_e + H);
+        ds = *reinterpret_cast<const half2_t*>(dn_suh + (size_t)e * H + hg * 128 + 2 * lane);
+    }
     const int c0 = (lane >> 3) * 16 + (lane & 7);
     red[wave][c0] = acc[0][0];
     red[wave][c0 + 8] = acc[0][1];
     __syncthreads();
     if (wave != 0) return;
-    if (writes) moe_route_write(route, choice, s / top_k, top_k, indices, lane);
     const int bits = fix_count_bits(n_chunks);
     // word q of a lane: projection q >> 1, column 2*lane + (q & 1); wave order within a projection
     unsigned long long w[4];
@@ -513,8 +511,6 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
     const int gid = blockIdx.x;
     const int og = gid % dblocks, s = gid / dblocks;
     const int e = clamp_expert(indices[s], E);
-    half2_t sv;  // (requested now, as in moe_gateup_pair_kernel)
-    if (wave == 0) sv = *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);
     constexpr bool kHalf = NW == 8;
     const int part_idx = blockIdx.y * NW + wave;
     const int blk = kHalf ? part_idx >> 1 : part_idx;
@@ -527,6 +523,8 @@ __global__ __launch_bounds__(NW * 64) void moe_down_kernel(
                                                   xh_dn + (size_t)s * H, (size_t)H, 1, nullptr,
                                                   xs[wave], lane, acc);
     }
+    half2_t sv;  // (requested behind the weights, as in moe_gateup_pair_kernel)
+    if (wave == 0) sv = *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);
     float2_t v = moe_wg_sum<NW>(red, acc, lane, wave);
     if (n_wg > 1) {
         int* counter = counters + gid;
@@ -735,7 +733,6 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
         stream_block_rows_at<K, CB, kGroupRows, false, kHalf, true, EXACT>(
             base, row_words, tk0, tk0 + (kHalf ? 4 : 8), xrow, grp.n, nullptr, xs[wave], lane, acc);
     }
-    const half2_t sv = *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);  // here after the sums
     const int c0 = (lane >> 3) * 16 + (lane & 7);
 #pragma unroll
     for (int m = 0; m < kGroupRows; m++) {
@@ -745,6 +742,7 @@ __global__ __launch_bounds__(NW * 64) void moe_down_grouped_kernel(
     __syncthreads();
     if (wave >= grp.n) return;
     const int sr = group_slot(grp, wave);
+    const half2_t sv = *reinterpret_cast<const half2_t*>(dn_svh + (size_t)e * D + og * 128 + 2 * lane);  // (behind the early exit: eight waves of K = 8 stay at 64 registers)
     float2_t v = moe_row_sum<NW>(red, wave, lane);
     if (n_wg > 1) {
         const size_t gid_r = (size_t)sr * dblocks + og;
