@@ -91,19 +91,33 @@ __device__ __forceinline__ void rows_add_slices4(float16_t (&acc)[MR][2], float4
 // Workgroups are dealt to the eight XCDs by index: the row blocks of one (column group, range)
 // unit u land on one XCD, whose L2 then reads their trellis words once. Whole units in turn (xcd_chunk = 0) can leave one
 // XCD with more workgroups than another; else each gets xcd_chunk, an eighth of them, neighbours, so that the row blocks of seven units at most
-// lie across a border, and units of one range are neighbours too. See rows_deal_evenly().
+// lie across a border, and units of one range are neighbours too. See rows_deal_evenly(). Each has its own way to the unit: one for both made the
+// kernel of short layers up to 7 % slower that are not dealt evenly (27 rows of 4992 -> 28672, MCG at K = 2, 33.3 and 36.5 us).
+// Up to 32 rows three workgroups fit on a CU by their LDS, and the register bound keeps them to that: 87 registers in place of 72 at K = 4 made
+// it two (17 rows of 4736 -> 22400 32.8 and 34.0 us).
 template <int K, int CB, int MR, int NKS>
-__global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 2) void linear_rows_kernel(LinRowsArgs p) {
+__global__ __launch_bounds__(128 * NKS, MR == 1 ? 6 : MR == 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 2) void linear_rows_kernel(LinRowsArgs p) {
     using T = RowsTile<MR, NKS>;
     constexpr int LPW = T::FILLS / (2 * NKS);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const unsigned xcd = blockIdx.x & 7, id = (blockIdx.x >> 3) + xcd * p.xcd_chunk, t = id / (unsigned)p.n_row_blocks;
-    const int rb = id % (unsigned)p.n_row_blocks, u = p.xcd_chunk ? t : t * 8 + xcd;
-    if (u >= p.n_units) return;
-    const int fast = p.xcd_chunk ? p.out_tiles >> 3 : p.n_splits, q0 = u / fast, q1 = u % fast;
-    const int g = p.xcd_chunk ? q1 : q0, split = p.xcd_chunk ? q0 : q1;
+    int g, split, rb;
+    if (p.xcd_chunk) {
+        const unsigned id = (blockIdx.x >> 3) + (blockIdx.x & 7) * p.xcd_chunk;
+        const int u = id / (unsigned)p.n_row_blocks, n_groups = p.out_tiles >> 3;
+        rb = id % (unsigned)p.n_row_blocks;
+        if (u >= p.n_units) return;
+        split = u / n_groups;
+        g = u % n_groups;
+    } else {
+        const int set = blockIdx.x / (8 * p.n_row_blocks), in_set = blockIdx.x % (8 * p.n_row_blocks);
+        const int u = set * 8 + (in_set & 7);
+        rb = in_set >> 3;
+        if (u >= p.n_units) return;
+        g = u / p.n_splits;
+        split = u % p.n_splits;
+    }
     const int k0 = split * p.steps_per_split;
     const int nsteps = min(p.steps_per_split, p.in_steps - k0);
     const int m0 = rb * p.block_rows;
@@ -124,24 +138,6 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
                                    lds_byte_address(stages) + wave * LPW * 1024, stages,
                                    rows_read_base<MR, NKS>(ks, lane), words, 2 * NKS * RowsWords<K>::STAGE,
                                    nsteps * (4 / NKS), lane, acc);
-    // Scales of the output transform: of the lane's columns, which are the same in all row tiles of a wave. Requested
-    // in front of the exchanges, and eight as one load where the vector allows it: as eight loads of two bytes for every row tile behind
-    // them they were up to a tenth of a layer. Us, before -> now: 100 rows of 4096 -> 24576 with bias 44.8 -> 40.8, 40 of
-    // 1536 -> 17408 19.0 -> 17.8, 306 of 2944 -> 11776 (K = 6) 57.7 -> 54.2, 700 of 2048 -> 6144 48.4 -> 48.4.
-    static_assert(2 * NKS % 4 == 0);
-    const int fr = lane & 15, q = lane >> 4, part = wave & 3, c0 = g * 128 + part * 32 + q * 8;
-    half8_t sv, bv;
-    auto eight = [](const half_t* v) {
-        if ((reinterpret_cast<uintptr_t>(v) & 15) == 0) return *reinterpret_cast<const half8_t*>(v);  // (the same for all lanes)
-        half8_t r;
-#pragma unroll
-        for (int c = 0; c < 8; c++) r[c] = v[c];
-        return r;
-    };
-    if (p.n_splits == 1) {
-        if (p.svh) sv = eight(p.svh + c0);
-        if (p.bias) bv = eight(p.bias + c0);
-    }
     // lane: row lane & 31 of each 32-row block, columns col + 16 i + 0..3, i < NI
     constexpr int NI = 8 / NKS;
     std::conditional_t<NKS == 4, float[MR][8], float16_t[MR]> sum;
@@ -166,6 +162,23 @@ __global__ __launch_bounds__(128 * NKS, MR <= 2 ? 4 : NKS == 2 && MR == 3 ? 3 : 
         }
         return;
     }
+    // Scales of the output transform: of the lane's columns, which are the same in all row tiles of a wave. Requested
+    // in front of the barrier, and eight as one load where the vector allows it: as eight loads of two bytes for every row tile behind
+    // it they were up to a tenth of a layer. Us, before -> now: 100 rows of 4096 -> 24576 with bias 45.3 -> 41.1, 40 of
+    // 1536 -> 17408 19.0 -> 17.2, 306 of 2944 -> 11776 (K = 6) 57.4 -> 54.4, 700 of 2048 -> 6144 48.4 -> 48.4. (In front of the exchanges, and with
+    // it on the way of the ranges too, these took 41.3, 17.6 and 54.2, and layers of ranges 1 % more than without.)
+    static_assert(2 * NKS % 4 == 0);
+    const int fr = lane & 15, q = lane >> 4, part = wave & 3, c0 = g * 128 + part * 32 + q * 8;
+    half8_t sv, bv;
+    auto eight = [](const half_t* v) {
+        if ((reinterpret_cast<uintptr_t>(v) & 15) == 0) return *reinterpret_cast<const half8_t*>(v);  // (the same for all lanes)
+        half8_t r;
+#pragma unroll
+        for (int c = 0; c < 8; c++) r[c] = v[c];
+        return r;
+    };
+    if (p.svh) sv = eight(p.svh + c0);
+    if (p.bias) bv = eight(p.bias + c0);
     half_t* tile = reinterpret_cast<half_t*>(lds);  // [BM][kLinRowsLd]
 #pragma unroll
     for (int mr = 0; mr < MR; mr++)

@@ -1,5 +1,5 @@
-"""Registers of the MoE slot kernels, from the metadata of the built library: how many workgroups a CU
-holds of the kernels whose waves wait for weights."""
+"""Registers of kernels whose waves wait for weights, from the metadata of the built library: how many
+workgroups a CU holds."""
 import os
 import re
 import struct
@@ -52,3 +52,10 @@ def test_moe_gate_up_workgroups_of_a_cu(registers, k, cb, half):
 def test_moe_grouped_down_workgroups_of_a_cu(registers, k):
     """20 tokens of 9 slots, 65 experts of 2048 x 512 at K = 8: 71.4 us with four workgroups to a CU, 73.2 with three."""
     assert _workgroups_of_eight(registers, "moe_down_grouped_kernel", k, 0, 8, 0) >= 4
+
+
+@pytest.mark.parametrize("cb", [0, 1, 2])
+@pytest.mark.parametrize("k", range(1, 9))
+def test_rows_kernel_workgroups_of_a_cu(registers, k, cb):
+    """Up to 32 rows: three, which is what their LDS allows up to K = 4."""
+    assert _workgroups_of_eight(registers, "linear_rows_kernel", k, cb, 1, 4) >= 3
