@@ -454,6 +454,11 @@ size_t exl3_linear_rows_workspace_bytes(int rows, int in_features, int out_featu
 int exl3_linear_rows(const uint16_t *xh, int rows, int n_sub, const uint16_t *trellis, int in_tiles, int out_tiles,
                      int K, int cb, const int32_t *group_sub, const uint16_t *svh, const uint16_t *bias, uint16_t *y,
                      void *workspace, size_t workspace_bytes, void *stream);
+/* The launch plan of exl3_linear_rows and exl3_linear_rows_long for a shape: row blocks, ranges of the reduction, waves
+ * of a workgroup (8 or 4), and whether workgroups go to the XCDs one by one (1) or in whole units, a column group and range
+ * with all its row blocks (0). Any output pointer may be NULL. */
+int exl3_linear_rows_plan(int rows, int in_tiles, int out_tiles, int K, int *n_row_blocks, int *n_ranges,
+                          int *waves_per_workgroup, int *dealt_evenly);
 int exl3_linear_rows_long(const uint16_t *xh, int rows, int n_sub, const uint16_t *trellis, int in_tiles, int out_tiles,
                           int K, int cb, const int32_t *group_sub, const uint16_t *svh, const uint16_t *bias, uint16_t *y,
                           void *workspace, size_t workspace_bytes, void *stream);

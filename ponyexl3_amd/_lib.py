@@ -44,6 +44,7 @@ PROTOTYPES = {
     "exl3_linear_rows_long_faster": (_i, [_vp, _i, _i, _i, _i, _i]),
     "exl3_linear_rows_workspace_bytes": (_sz, [_i, _i, _i]),
     "exl3_linear_rows": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
+    "exl3_linear_rows_plan": (_i, [_i, _i, _i, _i] + [ctypes.POINTER(_i)] * 4),
     "exl3_linear_rows_long": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "exl3_linear_prefill": (_i, [_vp, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "exl3_moe_sort": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),

@@ -236,6 +236,19 @@ EXL3_EXPORT int exl3_linear_rows_long_faster(const uint16_t* trellis, int rows, 
            exl3::linear_rows_long_applies(rows, in_tiles, out_tiles, K, cb);
 }
 
+EXL3_EXPORT int exl3_linear_rows_plan(int rows, int in_tiles, int out_tiles, int K, int* n_row_blocks, int* n_ranges,
+                                      int* waves_per_workgroup, int* dealt_evenly) {
+    using namespace exl3;
+    if (rows < 1 || rows > kLinearRowsLongMaxRows || in_tiles < 8 || in_tiles % 8 || out_tiles < 8 || out_tiles % 8 || K < 1 || K > 8)
+        return EXL3_E_BAD_SHAPE;
+    const LinRowsShape s = linear_rows_shape(rows, in_tiles, out_tiles / 8, K);
+    if (n_row_blocks) *n_row_blocks = s.n_row_blocks;
+    if (n_ranges) *n_ranges = s.n_splits;
+    if (waves_per_workgroup) *waves_per_workgroup = s.wg_waves;
+    if (dealt_evenly) *dealt_evenly = s.dealt_evenly;
+    return EXL3_OK;
+}
+
 static int linear_rows_between(int min_rows, int max_rows, const uint16_t* xh, int rows, int n_sub, const uint16_t* trellis,
                                int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub, const uint16_t* svh,
                                const uint16_t* bias, uint16_t* y, void* workspace, size_t workspace_bytes, void* stream) {

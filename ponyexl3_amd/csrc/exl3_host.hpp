@@ -144,6 +144,11 @@ struct LinRowsPlan {
 };
 LinRowsPlan plan_linear_rows(int rows, int in_tiles, int n_groups);
 size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups);
+struct LinRowsShape {
+    int n_row_blocks, n_splits, wg_waves;
+    bool dealt_evenly;  // workgroups to the XCDs one by one, not in whole units
+};
+LinRowsShape linear_rows_shape(int rows, int in_tiles, int n_groups, int K);
 bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb);
 // for some K and codebook
 bool linear_rows_ever_applies(int rows, int in_tiles, int out_tiles);

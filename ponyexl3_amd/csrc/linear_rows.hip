@@ -413,6 +413,11 @@ size_t linear_rows_partial_bytes(int rows, int in_tiles, int n_groups) {
     return p.n_splits > 1 ? (size_t)p.n_splits * rows * n_groups * 128 * sizeof(float) : 0;
 }
 
+LinRowsShape linear_rows_shape(int rows, int in_tiles, int n_groups, int K) {
+    const LinRowsPlan p = plan_linear_rows(rows, in_tiles, n_groups);
+    return {p.n_row_blocks, p.n_splits, rows_narrow(p, n_groups, K) ? 4 : 8, rows_deal_evenly(p, n_groups, K)};
+}
+
 int launch_linear_rows(const uint16_t* xh, int rows, size_t ldx, size_t sub_stride, const uint16_t* trellis,
                        int in_tiles, int out_tiles, int K, int cb, const int32_t* group_sub,
                        const uint16_t* svh, const uint16_t* bias, uint16_t* y, float* partial, hipStream_t stream) {

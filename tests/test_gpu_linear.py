@@ -622,12 +622,13 @@ def test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
     args = (ops._ptr(xh), rows, len(outs), ops._ptr(tr), n_in // 16, n_out // 16, k, cb, ops._ptr(sub), ops._ptr(svh),
             ops._ptr(bias) if bias is not None else None, ops._ptr(y), ops._ptr(ws))
     print(f"rows kernel rows={rows} k={k} cb={cb} {n_in}->{outs}", flush=True)
-    _lib.check(lib.exl3_linear_rows(*args, need, ops._stream()), "exl3_linear_rows")
+    entry = lib.exl3_linear_rows if rows <= 1024 else lib.exl3_linear_rows_long
+    _lib.check(entry(*args, need, ops._stream()), "exl3_linear_rows")
     assert bool((y[rows] == 7.0).all())
     for l, part in zip(layers, torch.split(y[:rows], list(outs), dim=-1)):
         assert rel_l2(part.cpu().numpy(), _oracle_forward(oracle, l, x)) <= TOL
     if need:
-        assert lib.exl3_linear_rows(*args, need - 1, ops._stream()) == _lib.EXL3_E_WORKSPACE
+        assert entry(*args, need - 1, ops._stream()) == _lib.EXL3_E_WORKSPACE
 
 
 @pytest.mark.parametrize("rows,k,cb,n_in,outs", [
@@ -642,6 +643,61 @@ def test_rows_kernel_in_workgroups_of_four_waves(cuda, oracle, rows, k, cb, n_in
     test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs)
 
 
+def _rows_plan(rows, n_in, n_out, k):
+    """Row blocks, ranges, waves of a workgroup, dealt to the XCDs one by one."""
+    import ctypes
+
+    from ponyexl3_amd import _lib
+
+    out = [ctypes.c_int() for _ in range(4)]
+    _lib.check(_lib.load().exl3_linear_rows_plan(rows, n_in // 16, n_out // 16, k, *[ctypes.byref(v) for v in out]), "plan")
+    return tuple(v.value for v in out)
+
+
+@pytest.mark.parametrize("rows,k,cb,n_in,outs,ranges,waves", [
+    (259, 4, 0, 128, (10368,), 1, 8),        # 81 units: the last XCD's share is short
+    (274, 8, 1, 1792, (768, 768), 7, 8),     # partial rows; a rotation for each half of the groups
+    (514, 4, 2, 128, (6272, 6144), 1, 4),    # members that end on odd 128-column blocks
+    (1281, 3, 0, 128, (2176,), 1, 8),        # past 1024 rows
+    (1281, 6, 1, 1536, (384,), 6, 8),
+    (1537, 4, 0, 128, (4224,), 1, 4),
+])
+def test_rows_kernel_dealt_evenly(cuda, oracle, rows, k, cb, n_in, outs, ranges, waves):
+    """Layers whose workgroups go to the XCDs one by one: another order of units, range-major, another grid and
+    ends inside a unit."""
+    plan = _rows_plan(rows, n_in, sum(outs), k)
+    assert plan[1:] == (ranges, waves, 1), plan
+    test_rows_kernel_against_oracle(cuda, oracle, rows, k, cb, n_in, outs)
+
+
+def test_rows_kernel_dealt_evenly_in_ranges_of_four_waves(cuda):
+    """The smallest such layer, too large for the oracle: against the GEMM and the output transform, member by member
+    (fp32 sums in other orders, fp16 results: the bar of the other layer tests)."""
+    from ponyexl3_amd import _lib, make_exl3_layer, ops
+
+    rows, k, n_in, outs = 129, 4, 4992, (8192, 8320)
+    n_out = sum(outs)
+    assert _rows_plan(rows, n_in, n_out, k) == (2, 3, 4, 1)
+    lib = _lib.load()
+    layers = [make_exl3_layer(k=k, in_features=n_in, out_features=o, seed=i) for i, o in enumerate(outs)]
+    trellis = [ops.as_trellis_tensor(l.trellis, cuda) for l in layers]
+    tr = torch.cat(trellis, dim=1).contiguous()
+    suh = torch.stack([torch.from_numpy(l.suh).to(cuda) for l in layers])
+    svh = torch.cat([torch.from_numpy(l.svh).to(cuda) for l in layers])
+    sub = torch.tensor([i for i, o in enumerate(outs) for _ in range(o // 128)], dtype=torch.int32, device=cuda)
+    _, xt = _x(np.random.default_rng(rows), (rows, n_in), cuda)
+    print(f"rows kernel, four waves and ranges, rows={rows} {n_in}->{outs}", flush=True)
+    xh = ops.had128_pre(xt, suh).contiguous()
+    ws = torch.empty((lib.exl3_linear_rows_workspace_bytes(rows, n_in, n_out),), dtype=torch.uint8, device=cuda)
+    y = torch.empty((rows, n_out), dtype=torch.float16, device=cuda)
+    _lib.check(lib.exl3_linear_rows(ops._ptr(xh), rows, 2, ops._ptr(tr), n_in // 16, n_out // 16, k, layers[0].codebook_mode,
+                                    ops._ptr(sub), ops._ptr(svh), None, ops._ptr(y), ops._ptr(ws), ws.numel(), ops._stream()),
+               "exl3_linear_rows")
+    for i, (l, part) in enumerate(zip(layers, torch.split(y, list(outs), dim=-1))):
+        ref = ops.had128_post(ops.inner_gemm(xh[:, i].contiguous(), trellis[i], k, l.codebook_mode), torch.from_numpy(l.svh).to(cuda))
+        assert float((part.float() - ref.float()).norm() / ref.float().norm()) <= TOL
+
+
 @pytest.mark.parametrize("rows,k,cb,n_in,outs", [
     (1025, 4, 0, 512, (128,)),            # the first row count past the rows kernel's own limit
     (1111, 8, 2, 640, (384,)),            # nine row blocks of unequal length
@@ -652,8 +708,8 @@ def test_rows_kernel_in_workgroups_of_four_waves(cuda, oracle, rows, k, cb, n_in
 ])
 def test_long_layers_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
     """Layers of more than 1024 rows that are too small for the GEMM's tiles go to the rows kernel inside the
-    layer calls; without counters, and past 2048 rows, they stay with the GEMM."""
-    from ponyexl3_amd import EXL3Linear, FusedEXL3Group, make_exl3_layer
+    fused layer calls; past 2048 rows they stay with the GEMM (without counters too: test_prefill_entry_point_is_the_gemm)."""
+    from ponyexl3_amd import EXL3Linear, FusedEXL3Group, _lib, make_exl3_layer, ops
 
     layers = [make_exl3_layer(k=k, in_features=n_in, out_features=o, seed=900 + i, mcg=cb == 1, mul1=cb == 2,
                               bias=len(outs) == 1 and rows % 2 == 1) for i, o in enumerate(outs)]
@@ -662,6 +718,23 @@ def test_long_layers_against_oracle(cuda, oracle, rows, k, cb, n_in, outs):
     parts = (EXL3Linear(layers[0], cuda)(xt),) if len(outs) == 1 else FusedEXL3Group(layers, cuda).forward_all(xt)
     for l, part in zip(layers, parts):
         assert rel_l2(part.cpu().numpy(), _oracle_forward(oracle, l, x)) <= TOL
+    # which kernel ran: the same bits as from its own entry point
+    lib, n_out, n_sub = _lib.load(), sum(outs), len(outs)
+    cat = lambda name: torch.cat([torch.from_numpy(getattr(l, name)).to(cuda) for l in layers])
+    tr = torch.cat([ops.as_trellis_tensor(l.trellis, cuda) for l in layers], dim=1).contiguous()
+    suh, svh, bias = cat("suh"), cat("svh"), cat("bias") if layers[0].bias is not None else None
+    sub = torch.tensor([i for i, o in enumerate(outs) for _ in range(o // 128)], dtype=torch.int32, device=cuda)
+    long = rows <= 2048
+    assert bool(lib.exl3_linear_rows_long_faster(ops._ptr(tr), rows, n_in // 16, n_out // 16, k, cb)) == long
+    xh = torch.empty((rows, n_sub, n_in), dtype=torch.float16, device=cuda)
+    _lib.check(lib.exl3_rotate(ops._ptr(xt), rows, n_in, ops._ptr(suh), n_sub, ops._ptr(xh), ops._stream()), "exl3_rotate")
+    ws = torch.empty((lib.exl3_linear_prefill_workspace_bytes(rows, n_in, n_out),), dtype=torch.uint8, device=cuda)
+    y = torch.empty((rows, n_out), dtype=torch.float16, device=cuda)
+    entry = lib.exl3_linear_rows_long if long else lib.exl3_linear_prefill
+    _lib.check(entry(ops._ptr(xh), rows, n_sub, ops._ptr(tr), n_in // 16, n_out // 16, k, cb,
+                     ops._ptr(sub) if n_sub > 1 else None, ops._ptr(svh), ops._ptr(bias) if bias is not None else None,
+                     ops._ptr(y), ops._ptr(ws), ws.numel(), ops._stream()), "long layer")
+    assert torch.equal(torch.cat(parts, dim=-1), y)
 
 
 @pytest.mark.parametrize("rows,k,cb,n_in,n_out", [(1025, 4, 0, 512, 512), (1500, 6, 0, 3328, 1024), (2048, 3, 1, 512, 512)])
