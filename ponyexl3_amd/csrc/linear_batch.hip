@@ -335,7 +335,9 @@ __global__ __launch_bounds__(NW * 64, R > 8 ? 4 : 1) void linear_batch_kernel(
                              reinterpret_cast<half_t*>(smem) + wave * (R + 1) * T::LD, lane, acc);
     // requested now, needed only by the finishing workgroup: by then they are here
     const size_t col = (size_t)g * 128 + 2 * lane;
-    half2_t sv, bv;
+    // (zeros where there are none: batch_finish() takes them by value, and an undefined argument would let the compiler
+    // conclude that both pointers are there)
+    half2_t sv{(half_t)0.f, (half_t)0.f}, bv = sv;
     if (svh) sv = half2_t{svh[col], svh[col + 1]};
     if (bias) bv = half2_t{bias[col], bias[col + 1]};
     const int c0 = (lane >> 3) * 16 + (lane & 7);

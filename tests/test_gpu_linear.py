@@ -587,6 +587,29 @@ def test_two_streams_do_not_share_scratch(cuda):
     assert all(torch.equal(o, ref_b) for o in outs_b)
 
 
+@pytest.mark.parametrize("rows", [1, 2, 4, 5, 8, 12, 16, 24])
+@pytest.mark.parametrize("k,cb,n_in,n_out", [(4, 0, 1024, 1024), (6, 1, 2048, 512), (3, 2, 640, 2304)])
+def test_absent_scales_and_bias_are_ones_and_zeros(cuda, rows, k, cb, n_in, n_out):
+    """A missing svh is a factor of one and a missing bias an addend of zero, bit for bit: a kernel that forgets that either
+    may be NULL reads near address 0 or multiplies by what a register holds."""
+    from ponyexl3_amd import ops
+
+    g = torch.Generator(device=cuda).manual_seed(rows)
+    tr = torch.randint(-32768, 32768, (n_in // 16, n_out // 16, 16 * k), dtype=torch.int16, device=cuda, generator=g)
+    x = torch.randn(rows, n_in, device=cuda, generator=g).half()
+    suh = (2 * torch.randint(0, 2, (n_in,), device=cuda, generator=g) - 1).half() / 64
+    ones, zeros = torch.ones(n_out, dtype=torch.float16, device=cuda), torch.zeros(n_out, dtype=torch.float16, device=cuda)
+    scale = torch.randn(n_out, device=cuda, generator=g).half()
+    print(f"absent scales rows={rows} k={k} cb={cb} {n_in}->{n_out}", flush=True)
+    ref = ops.linear_forward(x, tr, k, cb, suh, ones, zeros)
+    assert bool(ref.isfinite().all()) and float(ref.float().std()) > 0.1
+    assert torch.equal(ops.linear_forward(x, tr, k, cb, suh, None, None), ref)
+    assert torch.equal(ops.linear_forward(x, tr, k, cb, suh, ones, None), ref)
+    assert torch.equal(ops.linear_forward(x, tr, k, cb, suh, None, zeros), ref)
+    assert torch.equal(ops.linear_forward(x, tr, k, cb, suh, scale, None), ops.linear_forward(x, tr, k, cb, suh, scale, zeros))
+    assert torch.equal(ops.linear_forward(x, tr, k, cb, suh, None, scale), ops.linear_forward(x, tr, k, cb, suh, ones, scale))
+
+
 @pytest.mark.parametrize("rows,k,cb,n_in,outs", [
     (1, 4, 0, 128, (128,)),              # one step, one column group
     (32, 1, 1, 256, (128, 256)),         # a full 32-row tile; two rotations
