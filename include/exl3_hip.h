@@ -294,7 +294,6 @@ size_t exl3_linear_workspace_bytes(int rows, int in_features, int out_features, 
  * waves per workgroup (4 or 8) and whether the split reduction goes through the 64-bit
  * accumulators (1) or through partial rows (0). The counterpart of the reference's
  * split chooser (ponyexl3/mlx/gemv_metal.py:1405-1414). Any output pointer may be NULL.
- * One row of a large layer with MUL1 at K = 4 may take whole blocks where the plan says half ones.
  */
 int exl3_linear_plan(int rows, int in_tiles, int out_tiles, int K, int *n_splits,
                      int *tile_rows_per_split, int *waves_per_workgroup, int *atomic);

@@ -375,7 +375,7 @@ static StaticNeed static_need(int rows, int out_features, GemvPlan plan) {
 EXL3_EXPORT size_t exl3_linear_static_need_bytes(int rows, int in_features, int out_features) {
     using namespace exl3;
     if (rows < 1 || rows > kLinearSmallMaxRows || in_features < 128 || out_features < 128) return 0;
-    // the launch plan depends on K: the largest of all (plans that the codebook decides between need the same)
+    // the launch plan depends on K: the largest of all
     size_t need = 0;
     for (int K = 1; K <= 8; K++) {
         const GemvPlan plan = plan_linear_small_launch(rows, in_features / 16, out_features / 128, K);

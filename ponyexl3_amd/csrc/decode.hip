@@ -131,15 +131,17 @@ __global__ __launch_bounds__(256) void decode_full_t_kernel(const uint32_t* __re
 // operands of the first product without a trip through LDS: a wave takes 32 columns over all 128 rows, its
 // loads put neighbouring pairs of tile rows on lane bits 4 and 5, and one exchange of 16-lane rows a
 // register brings rows 0..7 and 8..15 of a tile into the lanes that the operand wants them in.
-// For 5120 x 17408 at K = 4 VALU issue (decode, signs, conversions: 730 instructions a wave) takes 30 us of a SIMD's
-// time, the matrix pipe 18, and a plain fill of the result would take 26: no unit is full; what is left are the phases of
-// a workgroup, of which four share a CU (one 34 KiB LDS tile, 128 registers): decode and first product, second
-// product, store, with three barriers between. The result goes out through LDS in 256-byte row pieces,
+// For 5120 x 17408 at K = 4 VALU issue (decode, signs, conversions: 730 instructions a wave, and 108 of the matrix pipe) is busy for
+// 82 % of the time that the CUs are, the matrix pipe for 41 %, and waves wait 25 % of theirs; a plain fill of the result would take
+// 26 us. What is left are the phases of a workgroup, of which four share a CU (one 34 KiB LDS tile, 128 registers): decode and first
+// product, second product, store, with three barriers between. The result goes out through LDS in 256-byte row pieces,
 // non-temporal (nobody reads it soon).
 // Measured, us, transposed: decoded weights through LDS (five barriers, scales loaded where they are used, a wait
 // each) -> operands from registers, scales in front -> words of the next block requested ahead:
-//   5120 x 17408 K = 2 / 4 / 8: 63.5 / 65.5 / 71.6 -> 56.3 / 56.5 / 63.1 -> 54.0 / 52.8 / 55.6 (4.2 TB/s of trellis and
-//   result at K = 4), not transposed K = 4 69.7 -> 58.5 -> 54.2; 2048 x 2048 7.4 -> 5.7 -> 5.8.
+//   5120 x 17408 K = 2 / 4 / 8: 63.5 / 65.5 / 71.6 -> 56.3 / 56.5 / 63.1 -> 54.0 / 52.8 / 55.6,
+//   not transposed K = 4 69.7 -> 58.5 -> 54.2; 2048 x 2048 7.4 -> 5.7 -> 5.8.
+// On other boxes 50.9 to 55 at K = 4 (4.1 to 4.4 TB/s of trellis and result). That is one layer again and again, whose words the last-level
+// cache can keep. Twelve layers in turn, each one's words from memory, first -> last of these forms: 60 / 62 / 72 -> 48.5 / 53.7 / 57.5.
 // The identity through the prefill kernels, the concatenation of its column stripes and the transposed copy took 1420.
 //
 // Workgroups that start together: 256 CUs of four. The one this many places on gets the place of this one, and as a

@@ -740,7 +740,7 @@ GemmPlan plan_gemm(int rows, int in_tiles, int tn_count, bool allow_split) {
 }
 
 // Against rows_estimate_us(), with which it was fitted (9 % rms): microseconds per 64-deep step of
-// a tile at 64, 128 and 256 rows, with what a bit from K = 5 on and MUL1 add; a piece of a split
+// a tile at 64, 128 and 256 rows, with what a bit from K = 5 on and MUL1 (its decode before that in pairs) add; a piece of a split
 // tile costs 4.4 steps more, the fix-up 9 us, launch and fill 7.
 double gemm_estimate_us(int rows, int in_tiles, int tn_count, int K, int cb) {
     static const double step[3] = {0.75, 1.07, 1.97}, per_bit[3] = {0.03, 0.02, 0.016}, mul1[3] = {1.23, 1.14, 1.0};

@@ -552,10 +552,10 @@ bool linear_small_uses_atomics(int rows, int n_groups, GemvPlan plan) {
 // rotation. A workgroup of eight half blocks puts two on every SIMD, as one of four whole blocks puts one: a SIMD's share
 // changes only by the last workgroup of a column group, where one or two whole blocks left over take a SIMD each and their halves
 // twice as many, and where the whole blocks come eight to a workgroup. half_blocks_balance() compares the rounds of the
-// 256 CUs, in whole blocks to a SIMD; a last workgroup of eight that is not full counts for its share. On its near side 78 measurements
-// give 4.1 % less in half blocks, the slowest 1.6 % more (whole -> half: K = 1 3200 -> 26112 13.4 -> 12.8, K = 2 5376 -> 19456 15.5 -> 15.0;
-// K = 2 7552 -> 21888 22.4 -> 22.8); on the far side 109 give
-// 0.8 % more, the best 1.8 % less, the worst 3.5 % more (K = 1 9728 -> 13824 18.3 -> 18.9, K = 2 2048 -> 65536 20.0 -> 20.6, 3072 -> 32000
+// 256 CUs, in whole blocks to a SIMD; a last workgroup of eight that is not full counts for its share. On its near side 45 measurements
+// of 3INST and MCG give 3.6 % less in half blocks, the slowest 1.6 % more (whole -> half: K = 1 3200 -> 26112 13.4 -> 12.8, K = 2 5376 -> 19456
+// 15.5 -> 15.0; K = 2 7552 -> 21888 22.4 -> 22.8), 21 of MUL1 2.8 % less, the slowest 2.4 % more; on the far side 62 and 30 give
+// 0.9 and 1.3 % more, the best 1.8 % less, the worst 3.4 and 5.6 % more (K = 1 9728 -> 13824 18.3 -> 18.9, K = 2 2048 -> 65536 20.0 -> 20.6, 3072 -> 32000
 // 15.0 -> 15.7, K = 3 3584 -> 31744 16.2 -> 16.4). At K = 4 half
 // blocks on both sides: beyond the line 25 measurements of 3INST and MCG give 2.3 % less, none more, and 14 of MUL1 on
 // either side 0.5 to 5.8 % (12032 -> 11904 23.6 -> 22.4, 5120 -> 34816 27.7 -> 27.0, 2048 -> 65536 22.3 -> 21.3).

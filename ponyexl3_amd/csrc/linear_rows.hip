@@ -309,8 +309,8 @@ static double rows_narrow_estimate_us(const LinRowsPlan& p, int n_groups, int K,
 // input rotation. Alone on its CU, two to a CU, and in several rounds a workgroup's 128-deep step
 // takes: {65..96, 97..128 rows} 0.915 and 1.08 us alone, 0.93 and 1.19 in rounds; up to 64 rows
 // 0.765 alone, 1.40 for two, and 0.85 in rounds where LDS holds one (K = 6 and more: three stages
-// of activations and trellis words). Bit windows take more instructions from K = 5 on, and MUL1
-// decodes in more than the others, which more rows hide in part.
+// of activations and trellis words). Bit windows take more instructions from K = 5 on. MUL1's factors, here, above and in
+// gemm_estimate_us(), are those of a decode of 5.5 instructions a weight in place of decode_mul1_pair()'s 2.5: see linear_rows_applies().
 static double rows_estimate_us(const LinRowsPlan& p, int rows, int n_groups, int K, int cb) {
     static const double alone[3] = {0.765, 0.915, 1.08}, rounds[3] = {0.85, 0.93, 1.19}, mul1[3] = {1.28, 1.21, 1.12};
     const int m = p.mr <= 2 ? 0 : p.mr - 2;
@@ -329,15 +329,19 @@ static double rows_estimate_us(const LinRowsPlan& p, int rows, int n_groups, int
 
 // Whether the layer takes this kernel rather than the prefill GEMM, which has larger tiles (256
 // columns and up to 256 rows). Both estimates were fitted to the choice over 2816 layers of 40 to
-// 1024 rows (in 1024..17408, out 1024..65536, K = 2..8, all codebooks): the layer is slower than
+// 1024 rows (in 1024..17408, out 1024..65536, K = 2..8, all codebooks), before MUL1 was decoded in pairs and before this kernel's shorter
+// epilogue and even dealing: as they were then the layer was slower than
 // through the GEMM by more than 3 % in seven of them, 8 % at most, and 0.5 % slower than the
-// better of the two on average. Workgroups of four waves have lines of their own: over 140 layers that
+// better of the two on average. As they are now the line errs to the GEMM: of 129 MUL1 layers drawn from 33 to 1024 rows ten take more than
+// 5 % more than through this kernel, 1.1 % on average (GEMM and this kernel, us: 405 rows of 1792 -> 8960 45.2 and 32.4, 200 of 4096 -> 24576
+// 75.8 and 67.1, 384 of 5120 -> 34816 at K = 2 187 and 170), of 65 3INST and MCG layers six, 1.3 % (830 of 1152 -> 22528 at K = 8 89.9 and 69.6);
+// none that comes here takes more than through the GEMM. Workgroups of four waves have lines of their own: over 140 layers that
 // take them (33 to 994 rows), where the line of the eight-wave estimate lost 1 % (96 rows), 3 % (128 rows,
 // and MUL1 from 65 on), 5 % (64 rows, K <= 5) and 14 % (64 rows, K >= 6) to the better of the two, these
-// lose 0.2, 1.9, 0.3, 0.1 and 3 %, and no layer goes to the slower one that did not before. Up to 64
+// lost 0.2, 1.9, 0.3, 0.1 and 3 %, and no layer went to the slower one that did not before. Up to 64
 // rows the GEMM's estimate is 11 % low, and with K <= 5 it was faster in one of 17 layers, by 2 %.
 // Measured (layer, GEMM and this kernel, us): 5120 -> 10240 at 77 rows 41.1 and 28.8; 17408 -> 5120 (K = 5) at 333 rows 115 and 97; 5120 -> 34816 at 64 rows 63.7
-// and 59.3 at K = 4, but 69.0 and 73.0 at K = 6; 4096 -> 24576 at 256 rows 83.6 and 95.1 with MUL1.
+// and 59.3 at K = 4, but 69.0 and 73.0 at K = 6.
 bool linear_rows_applies(int rows, int in_tiles, int out_tiles, int K, int cb) {
     static const int max_rows = env_int("EXL3_LINEAR_ROWS_MAX_ROWS", kLinearRowsMaxRows, 0, kLinearRowsMaxRows);
     // fewer than four 128-deep steps do not fill the three stages of the pipeline

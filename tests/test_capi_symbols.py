@@ -174,7 +174,9 @@ def test_gemm_split_plan_sizes(lib, monkeypatch):
 
 def test_rows_route_knows_the_weights(lib):
     """The choice between the rows kernel and the prefill GEMM depends on K (one workgroup to a CU
-    at 33 to 64 rows from K = 6 on) and on the codebook's decode; layers measured on either side."""
+    at 33 to 64 rows from K = 6 on) and on the codebook's decode. The layers of 3INST and MCG were measured on either side;
+    the two of MUL1 lie on the GEMM's side of a line that was fitted to an earlier decode (with today's they take 75.8 us there and
+    67.1 through the rows kernel, 187 and 170)."""
     aligned = ctypes.c_void_p(4096)
     faster = lambda rows, n_in, n_out, k, cb: bool(
         lib.exl3_linear_rows_faster(aligned, rows, n_in // 16, n_out // 16, k, cb))
