@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void decode_full_t_kernel(const uint32_t* __re
 // each) -> operands from registers, scales in front -> words of the next block requested ahead:
 //   5120 x 17408 K = 2 / 4 / 8: 63.5 / 65.5 / 71.6 -> 56.3 / 56.5 / 63.1 -> 54.0 / 52.8 / 55.6,
 //   not transposed K = 4 69.7 -> 58.5 -> 54.2; 2048 x 2048 7.4 -> 5.7 -> 5.8.
-// On other boxes 50.9 to 55 at K = 4 (4.1 to 4.4 TB/s of trellis and result). That is one layer again and again, whose words the last-level
+// On other GPUs of the kind 50.9 to 55 at K = 4 (4.1 to 4.4 TB/s of trellis and result). That is one layer again and again, whose words the last-level
 // cache can keep. Twelve layers in turn, each one's words from memory, first -> last of these forms: 60 / 62 / 72 -> 48.5 / 53.7 / 57.5.
 // The identity through the prefill kernels, the concatenation of its column stripes and the transposed copy took 1420.
 //
